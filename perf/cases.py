@@ -42,10 +42,10 @@ def listed():
     return [
         # an assistant's answer, 32 of its tokens behind a filled context: what a user waits
         # for most of the time
-        {"name": "decode, context 1024", "path": "qwen2_decode", "context": 1024, "steps": 32,
+        {"name": "decode at 1024", "path": "qwen2_decode", "context": 1024, "steps": 32,
          "qkv": "int8"},
         # the same about a long document, with the f32 q|k|v of the reference's shipped graph
-        {"name": "decode, context 12000", "path": "qwen2_decode", "context": 12000, "steps": 12,
+        {"name": "decode at 12000", "path": "qwen2_decode", "context": 12000, "steps": 12,
          "qkv": "f32"},
         # a short question
         {"name": "prompt of 27", "path": "qwen2_prefill", "tokens": 27, "context": 0, "qkv": "int8",
@@ -60,21 +60,21 @@ def listed():
         {"name": "prompt of 1931", "path": "qwen2_prefill", "tokens": 1931, "context": 0,
          "qkv": "int8", "precision": "digits"},
         # a document through latent and lightning attention and routed experts
-        {"name": "nukopel, prompt of 2048", "path": "nukopel", "tokens": 2048, "new": 0,
+        {"name": "nukopel prompt of 2048", "path": "nukopel", "tokens": 2048, "new": 0,
          "dtype": "bfloat16"},
         # a turn of a chat with it
-        {"name": "nukopel, 45 and 24 new", "path": "nukopel", "tokens": 45, "new": 24,
+        {"name": "nukopel 45 and 24 new", "path": "nukopel", "tokens": 45, "new": 24,
          "dtype": "bfloat16"},
         # a prompt through attention with a sink, differential attention and the delta rule
-        {"name": "lirulix, prompt of 777", "path": "lirulix", "tokens": 777, "new": 0,
+        {"name": "lirulix prompt of 777", "path": "lirulix", "tokens": 777, "new": 0,
          "dtype": "bfloat16"},
         # a turn of a chat with it where every activation stays 32-bit
-        {"name": "lirulix f32, 300 and 16 new", "path": "lirulix", "tokens": 300, "new": 16,
+        {"name": "lirulix f32 300 and 16 new", "path": "lirulix", "tokens": 300, "new": 16,
          "dtype": "float32"},
         # one decoder block for a batch of decoding requests
-        {"name": "mlp block, 12 rows", "path": "mlp", "rows": 12, "hidden": 1536, "inter": 8960},
+        {"name": "mlp block of 12 rows", "path": "mlp", "rows": 12, "hidden": 1536, "inter": 8960},
         # a matrix of the int8-activation variant on a prompt
-        {"name": "w8a8, 512 rows", "path": "w8a8", "rows": 512, "k": 1536, "n": 8960},
+        {"name": "w8a8 of 512 rows", "path": "w8a8", "rows": 512, "k": 1536, "n": 8960},
     ]
 
 
