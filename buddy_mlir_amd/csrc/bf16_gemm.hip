@@ -1,12 +1,11 @@
 // bf16_gemm.hip -- many activation rows times resident bfloat16 matrices on the
 // matrix cores: the matrix products of a prompt, plain and per expert.
 //
-// A workgroup of four wavefronts computes 16*RT rows x 64*GT channels.  Weights go
-// from memory to registers as they lie (a tile is the A operand: 16 channels x 32
-// k), each wavefront its own channels; the activation rows are the B operand and
-// are shared through LDS, 128 bytes of every row per step.  Both are requested
-// kStages - 1 steps ahead.  With f32 activations the same tiles are widened and
-// multiplied by v_mfma_f32_16x16x4_f32, so nothing is rounded below 32 bits.
+// Weights go from memory to registers as they lie, each of the four wavefronts of a
+// workgroup its own channels; the activation rows are the B operand and are shared
+// through LDS.  Both are requested three steps ahead.  Up to 16 rows a tile of 16
+// channels x 32 k is the A operand as it lies, and f32 activations are multiplied by
+// v_mfma_f32_16x16x4_f32; above that see rows_gemm_wide_kernel.
 #include "bf16_linear.h"
 #include "bf16_dev.h"
 
@@ -66,16 +65,52 @@ template <> __device__ __forceinline__ void store4<bf16_bits>(bf16_bits *p, f32x
 
 // Workgroups go to the eight dies in turn, each with an L2 of its own.  A die takes a run
 // of tiles, in panels of kPanel column blocks by all row blocks: the workgroups that it
-// runs at the same time share rows and channels.
+// runs at the same time share rows and channels.  Of experts' tiles the die takes a run of
+// row blocks too, so that an expert's weights come to one or two L2s and not to all eight.
 constexpr int kDies = 8, kPanel = 4;
-__device__ __forceinline__ void place_tile(int &bx, int &by) {
-  const int gx = gridDim.x, gy = gridDim.y, total = gx * gy, id = blockIdx.y * gx + blockIdx.x;
+__device__ __forceinline__ void place_tile(int gy, int &bx, int &by) {
+  const int gx = gridDim.x, total = gx * gy, id = blockIdx.y * gx + blockIdx.x;
   const int die = id % kDies, q = total / kDies, r = total % kDies;
   const int t = die * q + min(die, r) + id / kDies;
   const int panel = t / (kPanel * gy), rest = t - panel * kPanel * gy;
   const int width = min(kPanel, gx - panel * kPanel);
   by = rest / width;
   bx = panel * kPanel + rest - by * width;
+}
+
+// row blocks of all experts together
+__device__ __forceinline__ int count_blocks(const int *counts, int experts, int rows, int lane) {
+  int n = 0;
+  for (int i = lane; i < experts; i += 64)
+    n += (counts[i] + rows - 1) / rows;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1)
+    n += __shfl_xor(n, o, 64);
+  return __builtin_amdgcn_readfirstlane(n);
+}
+// the expert that a row block counted over all experts belongs to; `block` becomes the one
+// within it
+__device__ __forceinline__ int find_expert(const int *counts, int experts, int rows, int lane,
+                                           int &block) {
+  for (int base = 0; base < experts; base += 64) {
+    const int i = base + lane;
+    const int nb = i < experts ? (counts[i] + rows - 1) / rows : 0;
+    int incl = nb;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(incl, o, 64);
+      if (lane >= o)
+        incl += v;
+    }
+    const unsigned long long past = __ballot(incl > block);
+    if (past) {
+      const int l = __builtin_ctzll(past);
+      block -= __builtin_amdgcn_readlane(incl - nb, l);
+      return __builtin_amdgcn_readfirstlane(base + l);
+    }
+    block -= __builtin_amdgcn_readlane(incl, 63);
+  }
+  return -1;
 }
 
 template <typename T, int RT, int GT, int OUT, bool GROUPED>
@@ -93,34 +128,15 @@ rows_gemm_kernel(const uint4 *__restrict__ W, int ktiles, int steps, GemmDev a) 
 
   int bx = blockIdx.x, by = blockIdx.y;
   if constexpr (!GROUPED)
-    place_tile(bx, by);
+    place_tile(gridDim.y, bx, by);
   int row0 = by * kRows, rows = a.rows;
   const int *list = nullptr;
   if constexpr (GROUPED) {
-    // blockIdx.y counts the row blocks of all experts: find this one's expert
-    int block = blockIdx.y, e = -1;
-    for (int base = 0; base < a.experts; base += 64) {
-      const int i = base + lane;
-      const int nb = i < a.experts ? (a.counts[i] + kRows - 1) / kRows : 0;
-      int incl = nb;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int v = __shfl_up(incl, o, 64);
-        if (lane >= o)
-          incl += v;
-      }
-      const unsigned long long past = __ballot(incl > block);
-      if (past) {
-        const int l = __builtin_ctzll(past);
-        block -= __builtin_amdgcn_readlane(incl - nb, l);
-        e = base + l;
-        break;
-      }
-      block -= __builtin_amdgcn_readlane(incl, 63);
-    }
+    // blockIdx.y counts the row blocks of all experts
+    int block = blockIdx.y;
+    const int e = find_expert(a.counts, a.experts, kRows, lane, block);
     if (e < 0)
       return; // more workgroups than row blocks
-    e = __builtin_amdgcn_readfirstlane(e);
     row0 = block * kRows;
     rows = a.counts[e];
     list = a.lists + (int64_t)e * a.list_cap;
@@ -268,8 +284,274 @@ rows_gemm_kernel(const uint4 *__restrict__ W, int ktiles, int steps, GemmDev a) 
   }
 }
 
+// ---- tiles of 32 rows and more -----------------------------------------------------
+// The same product on v_mfma_f32_32x32x16_bf16.  A wavefront that has its SIMD to itself
+// issues 16 x 16 x 32 at 22 cycles apiece (1.2 PFLOP/s of the chip), 32 x 32 x 16 at its
+// 32 (1.9), with half the operand reads per product.  The A operand is 32 channels x 16 k:
+// the lanes take it from the tiles of two channel groups, 512 contiguous bytes of each.
+//
+// f32 activations are cut into three bfloat16 terms of 8 bits each as they enter LDS,
+// which is every bit of them; the weights are bfloat16 as they are.  All products are
+// exact, the sums f32: three matrix instructions at sixteen times the rate of the f32
+// ones.
+//
+// What bounds it: a step of 128 rows x 256 channels is 1024 cycles of matrix instructions
+// and takes 1725 at 2.0 GHz, with the loads of the rows and their way into LDS in the
+// wavefront's one stream of instructions, and the clock falls with the power the matrix
+// cores draw (2.4 to 1.9 GHz).  Against 16 x 16 tiles (us, rows x K x channels):
+//   bfloat16  2048 x 4096 x 4096   82.0 -> 75.2    f32   523 -> 216
+//             2048 x 1536 x 7168   72.4 -> 66.7          341 -> 154
+//              777 x 8960 x 1536   60.4 -> 41.3          307 -> 115
+//              777 x 1536 x 1536   13.8 -> 10.7           57 ->  23
+// The f32 sums are also nearer to 64 bits (4.2e-7 against 7.0e-7 at K = 1536).
+
+// four consecutive f32 values as three runs of bfloat16; the terms behind an infinity are
+// zero, those of a NaN are NaN
+__device__ __forceinline__ void split3(uint4 v, uint2 (&out)[3]) {
+  const unsigned u[4] = {v.x, v.y, v.z, v.w};
+  unsigned t[3][4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const float x = __uint_as_float(u[j]);
+    const unsigned hi = u[j] & 0xffff0000u;
+    const float r = __builtin_isinf(x) ? 0.f : x - __uint_as_float(hi);
+    const unsigned mid = __float_as_uint(r) & 0xffff0000u;
+    t[0][j] = u[j];
+    t[1][j] = __float_as_uint(r);
+    t[2][j] = __float_as_uint(r - __uint_as_float(mid));
+  }
+#pragma unroll
+  for (int p = 0; p < 3; ++p) // the upper halves of two words
+    out[p] = uint2{__builtin_amdgcn_perm(t[p][1], t[p][0], 0x07060302u),
+                   __builtin_amdgcn_perm(t[p][3], t[p][2], 0x07060302u)};
+}
+
+__device__ __forceinline__ f32x16 mfma_bf16_wide(uint4 a, uint4 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                 __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+constexpr int kWideK = 64; // k per step
+
 template <typename T, int RT, int GT, int OUT, bool GROUPED>
-int launch_variant(const RowsGemm &a, hipStream_t stream) {
+__global__ void __launch_bounds__(kGemmThreads)
+rows_gemm_wide_kernel(const uint4 *__restrict__ W, int ktiles, int steps, GemmDev a) {
+  constexpr bool kPair = OUT == kOutExpertAct;
+  constexpr int kTilesOut = kPair ? GT / 2 : GT; // 32-channel tiles of the result per wavefront
+  constexpr int kTerms = sizeof(T) == 4 ? 3 : 1;
+  constexpr int kRows = 32 * RT;
+  constexpr int kRunElems = 16 / (int)sizeof(T);
+  constexpr int kRowRuns = kWideK / kRunElems;
+  constexpr int kLoads = kRows * kRowRuns / kGemmThreads;
+  constexpr int kPlane = kRows * kLdsRow, kBuf = kTerms * kPlane;
+  static_assert(kRows * kRowRuns % kGemmThreads == 0, "every thread moves the same number of runs");
+  __shared__ __attribute__((aligned(16))) unsigned char lds[3 * kBuf];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  int bx = blockIdx.x, by = blockIdx.y;
+  if constexpr (!GROUPED)
+    place_tile(gridDim.y, bx, by);
+  int row0 = by * kRows, rows = a.rows;
+  const int *list = nullptr;
+  if constexpr (GROUPED) {
+    const int blocks = count_blocks(a.counts, a.experts, kRows, lane);
+    if ((int)(blockIdx.y * gridDim.x + blockIdx.x) >= blocks * (int)gridDim.x)
+      return; // more workgroups than tiles
+    place_tile(blocks, bx, by);
+    const int e = find_expert(a.counts, a.experts, kRows, lane, by);
+    if (e < 0)
+      return;
+    row0 = by * kRows;
+    rows = a.counts[e];
+    list = a.lists + (int64_t)e * a.list_cap;
+    W += (int64_t)e * a.expert_tiles * 64;
+  }
+
+  // the runs this thread moves: fixed rows, k advancing by the step
+  const T *src[kLoads];
+  int lds_at[kLoads];
+  const int run_k = tid % kRowRuns * kRunElems;
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) {
+    const int r = (i * kGemmThreads + tid) / kRowRuns;
+    lds_at[i] = r * kLdsRow + run_k * 2;
+    // a row past the end repeats the last one: its column of the result is not stored
+    const int lr = min(row0 + r, rows - 1);
+    int pr;
+    if constexpr (GROUPED)
+      pr = list[lr] / a.list_div;
+    else
+      pr = (a.ring_base + lr) & a.ring_mask;
+    src[i] = static_cast<const T *>(a.A) + (int64_t)pr * a.lda;
+  }
+
+  const int ch0 = (bx * 4 + wave) * kTilesOut * 2; // first channel group of this wavefront
+  const uint4 *wp[GT];
+#pragma unroll
+  for (int g = 0; g < GT; ++g) {
+    const int mat = kPair ? g / kTilesOut : 0;
+    const int gg = min(ch0 + 2 * (kPair ? g % kTilesOut : g) + ((lane >> 4) & 1), a.groups - 1);
+    wp[g] = W + ((int64_t)(mat * a.groups + gg) * ktiles) * 64 + (lane >> 5) * 16 + (lane & 15);
+  }
+
+  uint4 wr[4][GT * 4], xr[4][kLoads];
+  const int last_run = (a.K - 1) / kRunElems * kRunElems;
+  const bool ragged = a.K % kWideK != 0; // the last step reaches past K
+  auto fetch_w = [&](int s, uint4 (&w)[GT * 4]) {
+    const int t = min(s, steps - 1) * 2;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int g = 0; g < GT; ++g)
+        w[g * 4 + u] = wp[g][(int64_t)(t + u / 2) * 64 + (u & 1) * 32];
+  };
+  auto fetch_x = [&](int s, uint4 (&x)[kLoads]) {
+    const int k = min(min(s, steps - 1) * kWideK + run_k, last_run);
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i)
+      x[i] = *reinterpret_cast<const uint4 *>(src[i] + k);
+  };
+  auto put_x = [&](int s, uint4 (&x)[kLoads], unsigned char *buf) {
+    if (ragged && s == steps - 1) {
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i)
+        x[i] = keep_run<T>(x[i], a.K - s * kWideK - run_k);
+    }
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      if constexpr (kTerms == 1) {
+        *reinterpret_cast<uint4 *>(buf + lds_at[i]) = x[i];
+      } else {
+        uint2 t[3];
+        split3(x[i], t);
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+          *reinterpret_cast<uint2 *>(buf + p * kPlane + lds_at[i]) = t[p];
+      }
+    }
+  };
+
+  f32x16 acc[GT][RT];
+#pragma unroll
+  for (int g = 0; g < GT; ++g)
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+      acc[g][r] = f32x16{};
+
+  const int frag_at = (lane & 31) * kLdsRow + (lane >> 5) * 16;
+  uint4 frag[2][kTerms][RT];
+  auto load_frag = [&](const unsigned char *buf, int u, uint4 (&f)[kTerms][RT]) {
+#pragma unroll
+    for (int p = 0; p < kTerms; ++p)
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+        f[p][r] = *reinterpret_cast<const uint4 *>(buf + p * kPlane + frag_at + r * 32 * kLdsRow + u * 32);
+  };
+
+  // Step s multiplies buffer s % 3, whose first fragments were read during step s - 1, and
+  // fills buffer (s + 2) % 3, last read before the previous barrier.
+  unsigned char *cur = lds, *next = lds + kBuf, *fill = lds + 2 * kBuf;
+  fetch_x(0, xr[0]);
+  fetch_x(1, xr[1]);
+  fetch_w(0, wr[0]);
+  fetch_x(2, xr[2]);
+  fetch_w(1, wr[1]);
+  fetch_x(3, xr[3]);
+  fetch_w(2, wr[2]);
+  put_x(0, xr[0], cur);
+  put_x(1, xr[1], next);
+  fetch_x(4, xr[0]);
+  __syncthreads();
+  load_frag(cur, 0, frag[0]);
+  auto step = [&](int s, uint4 (&w)[GT * 4], uint4 (&w_new)[GT * 4], uint4 (&x)[kLoads],
+                  uint4 (&x_new)[kLoads]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      // the next fragments are asked for ahead of the products that cover their way, and
+      // stay there: left to itself the scheduler moves them to their use
+      load_frag(u < 3 ? cur : next, (u + 1) & 3, frag[(u + 1) & 1]);
+      if (u == 0)
+        fetch_w(s + 3, w_new);
+      if (u == 1)
+        put_x(s + 2, x, fill);
+      if (u == 2)
+        fetch_x(s + 5, x_new);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int p = kTerms - 1; p >= 0; --p)
+#pragma unroll
+        for (int g = 0; g < GT; ++g)
+#pragma unroll
+          for (int r = 0; r < RT; ++r)
+            acc[g][r] = mfma_bf16_wide(w[g * 4 + u], frag[u & 1][p][r], acc[g][r]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();
+    unsigned char *t = cur;
+    cur = next;
+    next = fill;
+    fill = t;
+  };
+  int s = 0;
+  for (; s + 4 <= steps; s += 4) {
+    step(s, wr[0], wr[3], xr[2], xr[1]);
+    step(s + 1, wr[1], wr[0], xr[3], xr[2]);
+    step(s + 2, wr[2], wr[1], xr[0], xr[3]);
+    step(s + 3, wr[3], wr[2], xr[1], xr[0]);
+  }
+  if (s < steps)
+    step(s, wr[0], wr[3], xr[2], xr[1]);
+  if (s + 1 < steps)
+    step(s + 1, wr[1], wr[0], xr[3], xr[2]);
+  if (s + 2 < steps)
+    step(s + 2, wr[2], wr[1], xr[0], xr[3]);
+
+  // a lane holds channels 8 j + (lane / 32) * 4 + 0..3, j = 0..3, of row lane % 32 of every tile
+#pragma unroll
+  for (int r = 0; r < RT; ++r) {
+    const int lr = row0 + r * 32 + (lane & 31);
+    if (lr >= rows)
+      continue;
+    int orow = lr;
+    if constexpr (GROUPED)
+      orow = list[lr];
+#pragma unroll
+    for (int g = 0; g < kTilesOut; ++g) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int ch = (ch0 + 2 * g) * 16 + 8 * j + (lane >> 5) * 4;
+        if (ch >= a.groups * 16)
+          continue;
+        f32x4 v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          v[i] = acc[g][r][4 * j + i];
+        if constexpr (OUT == kOutExpertAct) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            v[i] = gated_act(a.act, v[i], acc[g + kTilesOut][r][4 * j + i], a.limit);
+          store4<T>(static_cast<T *>(a.C) + (int64_t)orow * a.ldc + ch, v);
+        } else if constexpr (OUT == kOutF32) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (ch + i < a.silu_channels)
+              v[i] = silu_f(v[i]);
+          store4<float>(static_cast<float *>(a.C) + (int64_t)orow * a.ldc + ch, v);
+        } else if constexpr (OUT == kOutAct) {
+          store4<T>(static_cast<T *>(a.C) + (int64_t)orow * a.ldc + ch, v);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            store_act<T>(static_cast<T *>(a.C) + (int64_t)(ch + i) * a.ldc + orow, v[i]);
+        }
+      }
+    }
+  }
+}
+
+template <typename T, int ROWS, int CHANNELS, int OUT, bool GROUPED, typename F>
+int launch_tiles(F kernel, int elems, const RowsGemm &a, hipStream_t stream) {
   GemmDev d{};
   d.A = a.A;
   d.C = a.C;
@@ -289,43 +571,72 @@ int launch_variant(const RowsGemm &a, hipStream_t stream) {
   d.list_cap = a.list_cap;
   d.list_div = a.list_div;
   d.expert_tiles = a.expert_tiles;
-  constexpr int per = 4 * (OUT == kOutExpertAct ? GT / 2 : GT);
-  const int64_t blocks = GROUPED ? std::min<int64_t>(ceil_div(a.list_total, 16 * RT) + a.experts,
+  const int64_t blocks = GROUPED ? std::min<int64_t>(ceil_div(a.list_total, ROWS) + a.experts,
                                                      a.list_total)
-                                 : ceil_div(a.rows, 16 * RT);
+                                 : ceil_div(a.rows, ROWS);
   BH_REQUIRE(blocks <= 65535, "rows_gemm: %lld row blocks", (long long)blocks);
-  hipLaunchKernelGGL((rows_gemm_kernel<T, RT, GT, OUT, GROUPED>),
-                     dim3((unsigned)ceil_div(d.groups, per), (unsigned)blocks), dim3(kGemmThreads),
-                     0, stream, a.W.tiles, a.W.ktiles, (int)ceil_div(a.W.K, ActTraits<T>::kElems), d);
+  hipLaunchKernelGGL(kernel,
+                     dim3((unsigned)ceil_div(d.groups * 16, CHANNELS), (unsigned)blocks), dim3(kGemmThreads),
+                     0, stream, a.W.tiles, a.W.ktiles, (int)ceil_div(a.W.K, elems), d);
   BH_CHECK_HIP(hipGetLastError());
   return BUDDY_HIP_OK;
 }
 
-// rows and channels of a workgroup: tall tiles when there are rows for them, wide
-// ones when the launch still fills the 256 compute units
+// RT tiles of 16 rows, GT channel groups per wavefront (pairs count twice)
+template <typename T, int RT, int GT, int OUT, bool GROUPED>
+int launch_variant(const RowsGemm &a, hipStream_t stream) {
+  return launch_tiles<T, 16 * RT, 64 * (OUT == kOutExpertAct ? GT / 2 : GT), OUT, GROUPED>(
+      rows_gemm_kernel<T, RT, GT, OUT, GROUPED>, ActTraits<T>::kElems, a, stream);
+}
+// RT tiles of 32 rows, GT tiles of 32 channels per wavefront
+template <typename T, int RT, int GT, int OUT, bool GROUPED>
+int launch_wide(const RowsGemm &a, hipStream_t stream) {
+  return launch_tiles<T, 32 * RT, 128 * (OUT == kOutExpertAct ? GT / 2 : GT), OUT, GROUPED>(
+      rows_gemm_wide_kernel<T, RT, GT, OUT, GROUPED>, kWideK, a, stream);
+}
+
+// Up to 16 rows the product is bound by the weights: 16-row tiles, wide ones where they
+// still fill the 256 compute units.  Above that the tile with the lowest estimate: tiles
+// per compute unit x steps of 64 k x what a step of such a tile takes (us, measured with
+// K of 1536 to 8960 on full and on partly filled chips), plus what a tile takes to
+// begin and to store.
 template <typename T, int OUT, bool GROUPED>
 int launch_shape(const RowsGemm &a, hipStream_t stream) {
   const int64_t rows = GROUPED ? ceil_div(a.list_total, a.experts) : a.rows;
   const int64_t all_blocks = GROUPED ? std::min<int64_t>(a.experts, a.list_total) : 1;
-  constexpr int P = OUT == kOutExpertAct ? 2 : 1; // groups come in pairs
-  auto workgroups = [&](int rt, int gt) {
-    return ceil_div(a.W.groups(), 4 * gt / P) * ceil_div(rows, 16 * rt) * all_blocks;
+  constexpr bool kPair = OUT == kOutExpertAct;
+  constexpr int P = kPair ? 2 : 1; // groups come in pairs
+  auto workgroups = [&](int rt, int ch) {
+    return ceil_div(a.W.N, ch) * ceil_div(rows, rt) * all_blocks;
   };
   if (rows <= 16)
-    return workgroups(1, 2 * P) >= 256 ? launch_variant<T, 1, 2 * P, OUT, GROUPED>(a, stream)
-                                       : launch_variant<T, 1, P, OUT, GROUPED>(a, stream);
-  if (rows <= 32)
-    return workgroups(2, 2 * P) >= 256 ? launch_variant<T, 2, 2 * P, OUT, GROUPED>(a, stream)
-                                       : launch_variant<T, 2, P, OUT, GROUPED>(a, stream);
-  // what a workgroup fetches per product shrinks with both sides of its tile
-  if constexpr (sizeof(T) == 2) {
-    // -- but one such workgroup fills a compute unit: whole rounds of 256 pay
-    const int64_t w = workgroups(8, 4);
-    if (rows > 64 && w >= 240 && w * 5 >= round_up(w, 256) * 4)
-      return launch_variant<T, 8, 4, OUT, GROUPED>(a, stream);
+    return workgroups(16, 128) >= 256 ? launch_variant<T, 1, 2 * P, OUT, GROUPED>(a, stream)
+                                      : launch_variant<T, 1, P, OUT, GROUPED>(a, stream);
+  const double steps = (double)ceil_div(a.W.K, kWideK);
+  auto cost = [&](int rt, int ch, double step_us, double fixed_us) {
+    return (double)ceil_div(workgroups(rt, ch / P), 256) * steps * step_us + fixed_us;
+  };
+  if constexpr (sizeof(T) == 4) {
+    if constexpr (!kPair)
+      if (cost(32, 128, 0.46, 4.0) <= cost(32, 256, 0.80, 4.5))
+        return launch_wide<T, 1, 1, OUT, GROUPED>(a, stream);
+    return launch_wide<T, 1, 2, OUT, GROUPED>(a, stream);
+  } else {
+    const double tall = cost(128, 256, 1.02, 7.0);
+    if constexpr (kPair) {
+      const double half = cost(64, 256, 0.60, 5.0), low = cost(32, 256, 0.40, 4.0);
+      if (tall <= std::min(half, low))
+        return launch_wide<T, 4, 2, OUT, GROUPED>(a, stream);
+      return half <= low ? launch_wide<T, 2, 2, OUT, GROUPED>(a, stream)
+                         : launch_wide<T, 1, 2, OUT, GROUPED>(a, stream);
+    } else {
+      const double half = cost(64, 128, 0.29, 4.5), low = cost(32, 128, 0.21, 4.0);
+      if (tall <= std::min(half, low))
+        return launch_wide<T, 4, 2, OUT, GROUPED>(a, stream);
+      return half <= low ? launch_wide<T, 2, 1, OUT, GROUPED>(a, stream)
+                         : launch_wide<T, 1, 1, OUT, GROUPED>(a, stream);
+    }
   }
-  return workgroups(4, 2 * P) >= 256 ? launch_variant<T, 4, 2 * P, OUT, GROUPED>(a, stream)
-                                     : launch_variant<T, 4, P, OUT, GROUPED>(a, stream);
 }
 
 template <typename T> int launch_typed(const RowsGemm &a, hipStream_t stream) {

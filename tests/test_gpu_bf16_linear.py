@@ -71,6 +71,81 @@ def test_many_rows(bh, M, K, Nout, dtype):
     assert (got[:, (Nout + 15) // 16 * 16:] == 7.0).all()      # nothing past the padding
 
 
+def sums64(a, w):
+    """float64 sums, on the GPU where the CPU would take seconds."""
+    d = torch.from_numpy(np.asarray(a, np.float64)).cuda() @ torch.from_numpy(w).cuda().T
+    return d.cpu().numpy()
+
+
+# tiles of 32 x 128, 32 x 256 (f32), 64 x 128 and 128 x 256 with a remainder in rows, in
+# pairs of channel groups and in K: below, at and beyond a step, and fewer steps than the
+# kernel asks for ahead
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("M,K,Nout", [
+    (17, 63, 33), (31, 64, 16), (33, 65, 48), (32, 129, 130), (65, 193, 144), (97, 1000, 8200),
+    (129, 260, 40016), (2000, 1200, 4080), (1921, 1161, 4096)])
+def test_wide_tiles(bh, M, K, Nout, dtype):
+    w, tiles = make(bh, K, Nout, M + K)
+    a = np.random.default_rng(M).standard_normal((M, K)).astype(np.float32)
+    if dtype == 0:
+        a = N.bf16(a)
+    lda, ldc = (K + 7) // 8 * 8, (Nout + 15) // 16 * 16 + 4
+    if dtype == 0:
+        buf = np.full((M, lda), 0x7FC0, np.uint16)
+        buf[:, :K] = N.to_bf16_bits(a)
+        A = torch.from_numpy(buf.view(np.int16)).cuda()
+    else:
+        buf = np.full((M, lda), np.nan, np.float32)
+        buf[:, :K] = a
+        A = torch.from_numpy(buf).cuda()
+    C = torch.full((M, ldc), 7.0, device="cuda")
+    torch.cuda.synchronize()
+    assert bh.buddy_hip_gemm_bf16(A.data_ptr(), lda, dtype, tiles.data_ptr(), C.data_ptr(), ldc,
+                                  M, K, Nout, None) == 0
+    torch.cuda.synchronize()
+    got, want = C.cpu().numpy(), sums64(a, w)
+    err = np.abs(got[:, :Nout] - want).max()
+    assert err < 3e-6 * max(1.0, np.abs(want).max()), err
+    assert (got[:, (Nout + 15) // 16 * 16:] == 7.0).all()
+
+
+def test_f32_rows_keep_every_bit_and_their_infinities(bh):
+    """f32 rows go through three bfloat16 terms: a row times one weight of 1 per channel is
+    the row itself, whatever its size; an infinity or a NaN reaches its own row alone."""
+    M, K = 40, 96
+    w = np.eye(K)
+    dev = torch.from_numpy(N.to_bf16_bits(w).view(np.int16)).cuda()
+    tiles = torch.empty(bh.buddy_hip_bf16_tiles_bytes(K, K), dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    assert bh.buddy_hip_pack_bf16_tiles(dev.data_ptr(), K, K, tiles.data_ptr(), None) == 0
+    rng = np.random.default_rng(4)
+    a = (rng.standard_normal((M, K)) * 10.0 ** rng.uniform(-25, 25, (M, K))).astype(np.float32)
+    a[3, 5], a[3, 6] = np.float32(3.4028235e38), np.float32(-3.4028235e38)
+    w2 = rng.standard_normal((K, K))
+    for weights, bad in ((w, None), (w2, np.inf), (w2, -np.inf), (w2, np.nan)):
+        x = a if bad is None else rng.standard_normal((M, K)).astype(np.float32)
+        if bad is not None:
+            x[7, 30] = bad
+        b = N.bf16(weights)
+        dev = torch.from_numpy(N.to_bf16_bits(b).view(np.int16)).cuda()
+        A, C = torch.from_numpy(x).cuda(), torch.empty((M, K), device="cuda")
+        torch.cuda.synchronize()
+        assert bh.buddy_hip_pack_bf16_tiles(dev.data_ptr(), K, K, tiles.data_ptr(), None) == 0
+        assert bh.buddy_hip_gemm_bf16(A.data_ptr(), K, 1, tiles.data_ptr(), C.data_ptr(), K,
+                                      M, K, K, None) == 0
+        torch.cuda.synchronize()
+        got = C.cpu().numpy()
+        if bad is None:
+            np.testing.assert_array_equal(got, x)
+            continue
+        rest = np.arange(M) != 7
+        assert np.isfinite(got[rest]).all()
+        if np.isnan(bad):
+            assert np.isnan(got[7]).all()
+        else:
+            np.testing.assert_array_equal(got[7], bad * np.sign(b[:, 30]))
+
+
 @pytest.mark.parametrize("K,Nout", [(64, 16), (1, 3), (37, 50), (2048, 96), (2052, 70), (4100, 33),
                                     (8200, 17), (9001, 20), (1536, 40000), (300, 4100)])
 def test_one_row(bh, K, Nout):
