@@ -1,0 +1,111 @@
+// attn_fold.h -- partial results of a prompt's attention and their sum.
+//
+// The attention of a block of prompt tokens (attn_prompt.hip) takes the query heads of a
+// KV head together: row r of a KV head is query r / group, head r % group of its group,
+// and 256 consecutive rows are a block.  A block whose keys went to several workgroups
+// leaves one partial result per workgroup in slots of a workspace.
+#pragma once
+
+#include "common.h"
+
+#include <type_traits>
+
+namespace bh {
+
+constexpr int kPromptRows = 256;       // rows of a block
+constexpr int kPromptD = 128;          // head size
+constexpr int kPromptWorkgroups = 256; // at most, each with up to two partial results
+constexpr size_t kPromptSlots = 2 * kPromptWorkgroups;
+
+// Where the parts of a block lie: part 0 in slot `first`, part j > 0 in slot
+// 2 * (owner + j).  parts == 0: the finished rows are in the output already.
+struct PromptBlock {
+  int first, owner, parts, pad;
+};
+struct PromptFold {
+  const float *out = nullptr;   // [tokens, heads, 128], finished rows of whole blocks
+  const float *acc = nullptr;   // [slots][256 rows][128], sums of weight * value
+  const float *ml = nullptr;    // [slots][256 rows][2]: max (of the scores times log2 e), sum of the weights
+  const PromptBlock *blocks = nullptr; // [kv_heads][blocks]
+  int group = 0, nblk = 0;
+};
+
+// Short prompts at the start of a sequence are quicker with attn_prefill.hip, which needs
+// no partial results: 256 tokens take 18.3 us there and 18.8 here, 512 tokens 27.5 and 27.1
+// (a whole prompt of 512 4.83 ms there and 4.89 here), 1024 tokens 63 and 52; with 200
+// positions before 8 tokens 15.9 and 13.4, with 120 before 3 tokens 11.8 and 12.3.
+inline bool attn_prompt_pays(int q_len, int q_offset) { return q_len > 640 || q_offset >= 128; }
+
+// Attention of a session's prompt tokens (no mask), on a workspace of
+// attn_prompt_workspace_bytes; what it leaves is described by `fold`.
+struct AttnPrefillArgs;
+size_t attn_prompt_workspace_bytes(int q_len, int heads, int kv_heads);
+int launch_attn_prompt(const AttnPrefillArgs &a, void *workspace, PromptFold &fold, hipStream_t stream);
+// the finished rows [tokens, heads, 128] in place ...
+int launch_attn_fold_rows(const PromptFold &fold, float *out, int64_t o_stride, int heads, int tokens,
+                          hipStream_t stream);
+// ... or as the digit planes of the matmul behind the attention (gemm_w8_i8.hip)
+int launch_attn_fold_to_digits(const PromptFold &fold, int64_t o_stride, int heads, int tokens, int digits,
+                               void *staged, hipStream_t stream);
+
+#if defined(__HIPCC__)
+// four values d .. d + 3 of query head h at token t
+__device__ __forceinline__ void folded4(const PromptFold &f, int64_t out_stride, int t, int h, int d,
+                                        float (&v)[4]) {
+  const int kvh = h / f.group, row = t * f.group + (h - kvh * f.group);
+  const PromptBlock b = f.blocks[kvh * f.nblk + row / kPromptRows];
+  if (b.parts == 0) {
+    const float4 q = *reinterpret_cast<const float4 *>(f.out + (int64_t)t * out_stride +
+                                                       (int64_t)h * kPromptD + d);
+    v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+    return;
+  }
+  const int r = row % kPromptRows;
+  auto slot = [&](int j) { return (size_t)(j ? 2 * (b.owner + j) : b.first) * kPromptRows + r; };
+  float m = -INFINITY, l = 0.f, s[4] = {0.f, 0.f, 0.f, 0.f};
+  // several parts in one trip to memory; past the last one it is asked for again and has
+  // no weight
+  auto add = [&](int j0, auto width) {
+    constexpr int kWidth = decltype(width)::value;
+    float2 ml[kWidth];
+    float4 q[kWidth];
+#pragma unroll
+    for (int i = 0; i < kWidth; ++i) {
+      const size_t at = slot(j0 + i < b.parts ? j0 + i : b.parts - 1);
+      ml[i] = *reinterpret_cast<const float2 *>(f.ml + 2 * at);
+      q[i] = *reinterpret_cast<const float4 *>(f.acc + at * kPromptD + d);
+    }
+    float mx = m;
+#pragma unroll
+    for (int i = 0; i < kWidth; ++i)
+      mx = fmaxf(mx, ml[i].x);
+    const float old = __builtin_amdgcn_exp2f(m - mx); // 0 the first time
+    m = mx;
+    l *= old;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      s[e] *= old;
+#pragma unroll
+    for (int i = 0; i < kWidth; ++i) {
+      const float w = j0 + i < b.parts ? __builtin_amdgcn_exp2f(ml[i].x - m) : 0.f;
+      l = fmaf(ml[i].y, w, l);
+      s[0] = fmaf(q[i].x, w, s[0]);
+      s[1] = fmaf(q[i].y, w, s[1]);
+      s[2] = fmaf(q[i].z, w, s[2]);
+      s[3] = fmaf(q[i].w, w, s[3]);
+    }
+  };
+  if (b.parts <= 8)
+    for (int j = 0; j < b.parts; j += 4)
+      add(j, std::integral_constant<int, 4>{});
+  else
+    for (int j = 0; j < b.parts; j += 16)
+      add(j, std::integral_constant<int, 16>{});
+  const float inv = 1.0f / l;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    v[e] = s[e] * inv;
+}
+#endif
+
+} // namespace bh

@@ -30,6 +30,7 @@
 // Two workgroup shapes, as for bf16: 64 rows x 64 channels with K split over the
 // four wavefronts (narrow matrices), and 64 or 48 rows x 256 or 320 channels with
 // the activation fragments shared through LDS (wide matrices).
+#include "attn_fold.h"
 #include "gemm.h"
 
 #include <algorithm>
@@ -99,6 +100,17 @@ struct SiluMulRow { // silu(g) * u
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       v[e] = silu_times(gv[e], uv[e]);
+  }
+};
+
+struct FoldedRow { // the attention's output at one token, added up from its parts
+  const PromptFold &f;
+  int64_t o_stride;
+  int t, n;
+  __device__ __forceinline__ void operator()(int k0, float (&v)[4]) const {
+    v[0] = v[1] = v[2] = v[3] = 0.f;
+    if (k0 < n)
+      folded4(f, o_stride, t, k0 / kPromptD, k0 % kPromptD, v);
   }
 };
 
@@ -177,6 +189,14 @@ __device__ __forceinline__ void row_to_digits(const F &f, int n, int row, int D,
   }
 }
 
+__device__ __forceinline__ void padding_to_digits(int row, int D, int Mp, int Kp, int8_t *planes) {
+  for (int j = 0; j < D; ++j)
+    for (int k0 = threadIdx.x * 4; k0 < Kp; k0 += kRowThreads * 4)
+      *reinterpret_cast<unsigned *>(planes + ((size_t)j * Mp + row) * Kp + k0) = 0u;
+  if (threadIdx.x == 0)
+    reinterpret_cast<float *>(planes + (size_t)D * Mp * Kp)[row] = 1.0f;
+}
+
 __global__ void __launch_bounds__(kRowThreads)
 activations_to_digits_kernel(const float *__restrict__ A, int64_t lda, int M, int K, int D,
                              int Mp, int Kp, int8_t *__restrict__ planes) {
@@ -184,15 +204,24 @@ activations_to_digits_kernel(const float *__restrict__ A, int64_t lda, int M, in
   extern __shared__ __attribute__((aligned(16))) float row_cache[];
   const int row = blockIdx.x;
   if (row >= M) { // padding rows: zero digits, step 1
-    for (int j = 0; j < D; ++j)
-      for (int k0 = threadIdx.x * 4; k0 < Kp; k0 += kRowThreads * 4)
-        *reinterpret_cast<unsigned *>(planes + ((size_t)j * Mp + row) * Kp + k0) = 0u;
-    if (threadIdx.x == 0)
-      reinterpret_cast<float *>(planes + (size_t)D * Mp * Kp)[row] = 1.0f;
+    padding_to_digits(row, D, Mp, Kp, planes);
     return;
   }
   row_to_digits(PlainRow{A + (int64_t)row * lda, K}, K, row, D, Mp, Kp, planes, red,
                 row_cache);
+}
+
+__global__ void __launch_bounds__(kRowThreads)
+attn_fold_to_digits_kernel(PromptFold f, int64_t o_stride, int M, int K, int D, int Mp, int Kp,
+                           int8_t *__restrict__ planes) {
+  __shared__ float red[kRowThreads / 64];
+  extern __shared__ __attribute__((aligned(16))) float row_cache[];
+  const int row = blockIdx.x;
+  if (row >= M) {
+    padding_to_digits(row, D, Mp, Kp, planes);
+    return;
+  }
+  row_to_digits(FoldedRow{f, o_stride, row, K}, K, row, D, Mp, Kp, planes, red, row_cache);
 }
 
 __global__ void __launch_bounds__(kRowThreads)
@@ -1051,6 +1080,19 @@ int launch_activations_to_digits(const float *A, int64_t lda, int64_t M, int64_t
   hipLaunchKernelGGL(activations_to_digits_kernel, dim3((unsigned)l.rows_padded), dim3(kRowThreads),
                      row_cache_bytes(l.cols_padded), stream, A, lda, (int)M, (int)K, digits, l.rows_padded,
                      l.cols_padded, static_cast<int8_t *>(staged));
+  BH_CHECK_HIP(hipGetLastError());
+  return BUDDY_HIP_OK;
+}
+
+int launch_attn_fold_to_digits(const PromptFold &fold, int64_t o_stride, int heads, int tokens, int digits,
+                               void *staged, hipStream_t stream) {
+  const int64_t K = (int64_t)heads * kPromptD;
+  BH_REQUIRE(fold.blocks && staged && tokens > 0 && (digits == 2 || digits == 3),
+             "attn_fold_to_digits: bad argument");
+  const GemmStagingLayout l = gemm_staging_layout(tokens, K);
+  hipLaunchKernelGGL(attn_fold_to_digits_kernel, dim3((unsigned)l.rows_padded), dim3(kRowThreads),
+                     row_cache_bytes(l.cols_padded), stream, fold, o_stride, tokens, (int)K, digits,
+                     l.rows_padded, l.cols_padded, static_cast<int8_t *>(staged));
   BH_CHECK_HIP(hipGetLastError());
   return BUDDY_HIP_OK;
 }

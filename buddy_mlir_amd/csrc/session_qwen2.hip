@@ -18,6 +18,7 @@
 // feeds the argmax straight into the next step's embedding gather without a
 // host round trip.
 #include "attn.h"
+#include "attn_fold.h"
 #include "elementwise.h"
 #include "gemm.h"
 #include "gemv_w8a32.h"
@@ -106,6 +107,7 @@ struct Qwen2Session : Session {
   float *kv_rows = nullptr; // staging of get_kv_rows, grown on demand
   size_t kv_rows_cap = 0;
   unsigned short *pf_xn_bf = nullptr, *pf_g_bf = nullptr; // bf16 matmul inputs
+  void *pf_attn_ws = nullptr;          // partial results of the attention
   unsigned short *pf_att_dg = nullptr; // digit planes of the attention output (o_proj's input)
   int gemm_terms = 3; // bf16 terms per activation in the prefill matmuls (3 = exact)
   int gemm_digits = 3; // int8 digit planes instead of bf16 terms when not 0
@@ -314,6 +316,10 @@ struct Qwen2Session : Session {
       (void)hipFree(pf_tokens);
       pf_tokens = nullptr;
     }
+    if (pf_attn_ws) {
+      (void)hipFree(pf_attn_ws);
+      pf_attn_ws = nullptr;
+    }
     for (unsigned short **p : {&pf_xn_bf, &pf_g_bf, &pf_att_dg})
       if (*p) {
         (void)hipFree(*p);
@@ -335,6 +341,7 @@ struct Qwen2Session : Session {
     BH_CHECK_HIP(hipMalloc((void **)&pf_xn_bf, std::max(lx.bytes(3), lx.bytes_digits(3))));
     BH_CHECK_HIP(hipMalloc((void **)&pf_g_bf, std::max(lg.bytes(3), lg.bytes_digits(3))));
     BH_CHECK_HIP(hipMalloc((void **)&pf_att_dg, gemm_staging_layout(rows, QN).bytes_digits(3)));
+    BH_CHECK_HIP(hipMalloc(&pf_attn_ws, attn_prompt_workspace_bytes(rows, S.heads, S.kv_heads)));
     pf_rows = rows;
     return BUDDY_HIP_OK;
   }
@@ -449,20 +456,25 @@ struct Qwen2Session : Session {
       a.q_len = n;
       a.k_len = start_pos + n;
       a.scale = scale;
-      if ((rc = launch_attn_prefill(a, stream)))
+      PromptFold fold;
+      const bool folded = attn_prompt_pays(n, start_pos);
+      if ((rc = folded ? launch_attn_prompt(a, pf_attn_ws, fold, stream) : launch_attn_prefill(a, stream)))
         return rc;
       if (gemm_digits) {
         // o_proj's finished rows go on as the normed input of gate and up: where
         // the matmul splits K over workgroups, the kernel that adds the slices
         // holds whole rows and writes those digit planes itself
-        if ((rc = launch_activations_to_digits(pf_att, (int64_t)S.heads * S.head_dim, n,
-                                               (int64_t)S.heads * S.head_dim, gemm_digits,
-                                               pf_att_dg, stream)))
+        if ((rc = folded ? launch_attn_fold_to_digits(fold, a.o_stride, S.heads, n, gemm_digits,
+                                                      pf_att_dg, stream)
+                         : launch_activations_to_digits(pf_att, a.o_stride, n, a.o_stride, gemm_digits,
+                                                        pf_att_dg, stream)))
           return rc;
         if ((rc = gemm_staged(reinterpret_cast<const unsigned short *>(pf_att_dg), L.o, pf_x, n,
                               true, 0, L.ln2, pf_xn_bf)))
           return rc;
       } else {
+        if (folded && (rc = launch_attn_fold_rows(fold, pf_att, a.o_stride, S.heads, n, stream)))
+          return rc;
         if ((rc = gemm(pf_att, L.o, pf_x, n, true)))
           return rc;
         if ((rc = norm_to_staging(pf_x, L.ln2, n, pf_xn_bf)))
@@ -601,7 +613,7 @@ struct Qwen2Session : Session {
       (void)hipStreamSynchronize(stream);
     for (void *p : {(void *)pf_x, (void *)pf_xn, (void *)pf_qkv, (void *)pf_att, (void *)pf_g,
                     (void *)pf_tokens, (void *)kv_rows, (void *)pf_xn_bf, (void *)pf_g_bf,
-                    (void *)pf_att_dg})
+                    (void *)pf_att_dg, pf_attn_ws})
       if (p)
         (void)hipFree(p);
     release_gemm_staging(stream);

@@ -394,6 +394,60 @@ def test_prefill_in_two_blocks_and_after_decode_steps(oracle):
     sess.close()
 
 
+# the attention that shares out key tiles: row blocks of 256 rows (42.67 tokens of six heads)
+# and tiles of 32 keys at, below and beyond their edges, one and several KV heads, groups of
+# one to eight heads, one row behind a long context, more blocks than workgroups take whole
+@pytest.mark.parametrize("heads,kv_heads,before,n", [
+    (6, 1, 128, 1), (6, 1, 159, 1), (6, 1, 160, 43), (6, 1, 0, 641), (6, 1, 0, 683), (6, 1, 700, 130),
+    (2, 2, 130, 255), (2, 2, 0, 769), (8, 1, 129, 32), (8, 1, 0, 673), (3, 1, 1000, 86),
+    (4, 2, 300, 127), (12, 2, 0, 650)])
+def test_prompt_attention_equals_token_by_token(heads, kv_heads, before, n):
+    """A prompt as one block against the same tokens through the decode step, whose
+    attention is another kernel: logits of the last row and the second layer's cache rows,
+    which hold what the first layer's attention gave."""
+    shape = Shape(layers=2, hidden=256, heads=heads, kv_heads=kv_heads, head_dim=128, inter=256,
+                  vocab=320, max_len=before + n + 8)
+    toks = synthetic.first_tokens(shape, n, seed=before + n).astype(np.int32)
+    for precision in ("digits", "exact"):
+        sess, _ = synthetic.build_session(shape, context=before, ln_jitter=0.1)
+        _, got = sess.prefill(toks, before, precision=precision)
+        rows = [sess.get_kv(j)[:, before:before + n] for j in (2, 3)]
+        sess.close()
+        sess, _ = synthetic.build_session(shape, context=before, ln_jitter=0.1)
+        for i, t in enumerate(toks):
+            _, want = sess.decode(int(t), before + i, want_logits=i + 1 == n)
+        check_close(got, want)
+        for j in (2, 3):
+            check_close(rows[j - 2], sess.get_kv(j)[:, before:before + n])
+        sess.close()
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_prompt_attention_keeps_non_finite_tokens_from_earlier_rows(bad):
+    """A token in the middle of a long prompt whose embedding is not finite, and a cache row
+    whose values are not: rows that do not see them are what they are without, bit for bit;
+    rows that do are NaN."""
+    shape = Shape(layers=2, hidden=256, heads=6, kv_heads=1, head_dim=128, inter=256, vocab=320,
+                  max_len=720)
+    toks = (synthetic.first_tokens(shape, 700, seed=1) % 300).astype(np.int32)
+    at = 450
+    toks[at] = 310
+    sess, _ = synthetic.build_session(shape, context=0, ln_jitter=0.1)
+    embed = sess._globals["embed"]
+
+    def rows():
+        sess.prefill(toks, 0)
+        return [sess.get_kv(j)[0, :700].copy() for j in (2, 3)]
+
+    clean = rows()
+    embed[310, 7] = bad
+    torch.cuda.synchronize()
+    for got, want in zip(rows(), clean):
+        np.testing.assert_array_equal(got[:at], want[:at])
+        assert np.isnan(got[at:]).any(axis=1).all()
+    sess.close()
+
+
 def test_wide_hidden_size_through_the_slice_adding_norm_kernel(oracle):
     """hidden = 9216: the kernel that adds the K slices of o_proj / down and
     writes the next RMSNorm's digit planes keeps two copies of a row in LDS,
