@@ -4,8 +4,8 @@
 // Same contract as the bf16 kernels of gemm_w8_mfma.hip (the BLIS-style kernel
 // of midend/lib/Conversion/MatMulOptimization/MatMulBlisVectorization.cpp:351-360,
 // 398-986), another way to carry the f32 activations.  The int8 weights are used
-// as they lie: a lane's 16 bytes of a packed 16 x 64 tile are one operand of
-// v_mfma_i32_16x16x64_i8, so nothing is converted in the loop (the bf16 kernels
+// as they lie: a lane's 16 bytes of a packed 16 x 64 tile are an operand of
+// v_mfma_i32_32x32x32_i8, so nothing is converted in the loop (the bf16 kernels
 // spend more VALU time turning int8 into bf16 than the matrix cores spend on the
 // products).  The activations become fixed point for that:
 //   per row m a power-of-two step s[m] with |A[m,k]| / s[m] < 2^(8D-2),
@@ -27,9 +27,8 @@
 // padded, followed by the row steps (f32 [rows_padded]).  A lane's operand is 16
 // contiguous bytes of a plane row.
 //
-// Two workgroup shapes, as for bf16: 64 rows x 64 channels with K split over the
-// four wavefronts (narrow matrices), and 64 or 48 rows x 256 or 320 channels with
-// the activation fragments shared through LDS (wide matrices).
+// Workgroups take 32 rows x 128 or 256 channels, with the activation fragments shared
+// through LDS.
 #include "attn_fold.h"
 #include "gemm.h"
 
@@ -41,7 +40,7 @@
 namespace bh {
 namespace {
 
-constexpr int kSlices = 4;        // wavefronts per workgroup
+constexpr int kSlices = 4;    // wavefronts per workgroup
 
 typedef int v4i32 __attribute__((ext_vector_type(4)));
 
@@ -269,25 +268,19 @@ struct GemmI8Args {
   int64_t ldc;
   int M, N, Mp, Kp, groups, chunks;
   int ncols;       // column tiles
-  int cols_padded; // ids per row tile: column tiles x slices, padded to the XCD count
+  // the row tiles are shared out over bands of band_rows; ids_padded workgroup ids per row
+  // of a band: column tiles x slices x bands, padded to the XCD count
+  int ids_padded, band_rows, row_tiles;
+  int span;      // channels per wavefront, where K is split
+  int tile_rows; // rows per workgroup, where K is split
   // K split over `slices` workgroups per tile, chunks_per_slice chunks each
   // (the last may hold fewer, never none); partial is only used when slices > 1
   int slices, chunks_per_slice;
-  float *partial;     // [tile][slice][wavefront][row block][16][16 GPW]
+  float *partial;     // [tile][slice][wavefront][row][channel]
   int accumulate;
   int32_t *sums;      // one plane only: the int32 sums themselves, dense [M, N], or null
   int int_partials;   // one plane, K split: the slices leave their int32 sums as they are
 };
-
-// sum_j 256^j acc_j as f32 (each int32 sum is exact; the conversions round to 24
-// bits, like an f32 accumulator would)
-template <int D> __device__ __forceinline__ float combine(const v4i32 (&acc)[D], int r) {
-  float v = (float)acc[D - 1][r];
-#pragma unroll
-  for (int j = D - 2; j >= 0; --j)
-    v = fmaf(v, 256.0f, (float)acc[j][r]);
-  return v;
-}
 
 // The finished value of one output.  One plane is the w8a8 matmul, whose result
 // is f32(sum) * (s_a * s_w[n]) in exactly that order (linalg.py:12833-12845).
@@ -295,184 +288,19 @@ template <int D> __device__ __forceinline__ float scaled(float v, float step, fl
   return D == 1 ? v * (step * s) : (v * step) * s;
 }
 
-constexpr int kSplitGroups = 4; // channel groups of 16 per workgroup of the split kernel
-
-// lane holds channels n..n+3 of row m: C = step[m] * scale[n] * v (+ bias | + C)
-__device__ __forceinline__ void store_row(const GemmI8Args &a, int m, int n, float step,
-                                          const float (&v)[4], const float (&s)[4],
-                                          const float (&b)[4], bool vec) {
-  float o[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r)
-    o[r] = (v[r] * step) * s[r];
-  float *c = a.C + (int64_t)m * a.ldc + n;
-  if (vec) {
-    float4 q = make_float4(o[0], o[1], o[2], o[3]);
-    if (a.accumulate) {
-      const float4 p = *reinterpret_cast<const float4 *>(c);
-      q = make_float4(p.x + q.x, p.y + q.y, p.z + q.z, p.w + q.w);
-    } else {
-      q = make_float4(b[0] + q.x, b[1] + q.y, b[2] + q.z, b[3] + q.w);
-    }
-    *reinterpret_cast<float4 *>(c) = q;
-  } else {
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (n + r < a.N)
-        c[r] = a.accumulate ? c[r] + o[r] : b[r] + o[r];
-  }
-}
-
-template <int D> struct ChunkOperands {
-  v4i32 w[kSplitGroups];
-  v4i32 a[D][4]; // [digit][row block]
-};
-
-template <int D>
-__device__ __forceinline__ void load_chunk(const v4i32 *const (&wp)[kSplitGroups],
-                                           const int8_t *ap, size_t plane, size_t rb_stride,
-                                           int c, ChunkOperands<D> &o) {
-#pragma unroll
-  for (int g = 0; g < kSplitGroups; ++g)
-    o.w[g] = wp[g][(size_t)c * 64];
-#pragma unroll
-  for (int j = 0; j < D; ++j)
-#pragma unroll
-    for (int rb = 0; rb < 4; ++rb)
-      o.a[j][rb] = *reinterpret_cast<const v4i32 *>(ap + j * plane + rb * rb_stride +
-                                                    (size_t)c * kTileK);
-}
-
-// 64 rows x 64 channels per workgroup; the four wavefronts split K and meet in
-// LDS in slice order.
-template <int D>
-__global__ void __launch_bounds__(kSlices *kWave) gemm_w8_i8_kernel(
-    const int8_t *p_planes, const int4 *p_W, int p_Mp, int p_Kp, int p_groups, int p_chunks,
-    int p_ncols, int p_cols_padded, int p_slices, int p_chunks_per_slice, GemmI8Args rest) {
-  // what a wavefront needs before its first fetch arrives in SGPRs (this file is
-  // built with -amdgpu-kernarg-preload-count); the rest is loaded behind the fetch
-  GemmI8Args a = rest;
-  a.planes = p_planes;
-  a.W = p_W;
-  a.Mp = p_Mp;
-  a.Kp = p_Kp;
-  a.groups = p_groups;
-  a.chunks = p_chunks;
-  a.ncols = p_ncols;
-  a.cols_padded = p_cols_padded;
-  a.slices = p_slices;
-  a.chunks_per_slice = p_chunks_per_slice;
-  extern __shared__ __attribute__((aligned(16))) float red[]; // [slice][64][lane]
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int col = blockIdx.x % a.cols_padded, rbk = blockIdx.x / a.cols_padded;
-  if (col >= a.ncols)
-    return; // padding id
-  const int m0 = rbk * 64, g0 = col * kSplitGroups;
-  const int per = (a.chunks + kSlices - 1) / kSlices;
-  const int c0 = min(wave * per, a.chunks), c1 = min(c0 + per, a.chunks);
-
-  v4i32 acc[kSplitGroups][4][D];
-#pragma unroll
-  for (int g = 0; g < kSplitGroups; ++g)
-#pragma unroll
-    for (int rb = 0; rb < 4; ++rb)
-#pragma unroll
-      for (int j = 0; j < D; ++j)
-        acc[g][rb][j] = v4i32{0, 0, 0, 0};
-
-  const v4i32 *wp[kSplitGroups];
-#pragma unroll
-  for (int g = 0; g < kSplitGroups; ++g) // groups past the end repeat the last one
-    wp[g] = reinterpret_cast<const v4i32 *>(a.W) +
-            ((size_t)min(g0 + g, a.groups - 1) * a.chunks) * 64 + lane;
-  const size_t plane = (size_t)a.Mp * a.Kp, rb_stride = (size_t)16 * a.Kp;
-  const int8_t *ap = a.planes + (size_t)(m0 + (lane & 15)) * a.Kp + (lane >> 4) * 16;
-
-  ChunkOperands<D> cur, nxt;
-  if (c0 < c1)
-    load_chunk<D>(wp, ap, plane, rb_stride, c0, cur);
-  for (int c = c0; c < c1; ++c) {
-    if (c + 1 < c1)
-      load_chunk<D>(wp, ap, plane, rb_stride, c + 1, nxt);
-#pragma unroll
-    for (int j = 0; j < D; ++j)
-#pragma unroll
-      for (int rb = 0; rb < 4; ++rb)
-#pragma unroll
-        for (int g = 0; g < kSplitGroups; ++g)
-          acc[g][rb][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(cur.w[g], cur.a[j][rb],
-                                                                acc[g][rb][j], 0, 0, 0);
-    if (c + 1 < c1)
-      cur = nxt;
-  }
-
-  // wavefront w finishes channel group w: its scales, bias and the steps of the
-  // rows are asked for here, ahead of the meeting in LDS, not at their use
-  const int g = wave;
-  const int n = (g0 + g) * kTileN + (lane >> 4) * 4;
-  float s[4], b[4], row_step[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    s[r] = n + r < a.N ? a.scale[n + r] : 0.f;
-    b[r] = (a.bias && n + r < a.N) ? a.bias[n + r] : 0.f;
-  }
-#pragma unroll
-  for (int rb = 0; rb < 4; ++rb) {
-    const int m = m0 + rb * 16 + (lane & 15);
-    row_step[rb] = m < a.M ? a.steps[m] : 0.f;
-  }
-  float *mine = red + (size_t)wave * 64 * kWave;
-#pragma unroll
-  for (int gg = 0; gg < kSplitGroups; ++gg)
-#pragma unroll
-    for (int rb = 0; rb < 4; ++rb)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        mine[((gg * 4 + rb) * 4 + r) * kWave + lane] = combine<D>(acc[gg][rb], r);
-  __syncthreads();
-  if (g0 + g >= a.groups)
-    return;
-  const bool vec = n + 3 < a.N && (a.ldc & 3) == 0 &&
-                   (reinterpret_cast<uintptr_t>(a.C) & 15) == 0;
-#pragma unroll
-  for (int rb = 0; rb < 4; ++rb) {
-    const int m = m0 + rb * 16 + (lane & 15);
-    float v[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float sum = 0.f;
-#pragma unroll
-      for (int sl = 0; sl < kSlices; ++sl)
-        sum += red[((size_t)sl * 64 + (g * 4 + rb) * 4 + r) * kWave + lane];
-      v[r] = sum;
-    }
-    if (m >= a.M)
-      continue;
-    store_row(a, m, n, row_step[rb], v, s, b, vec);
-  }
-}
-
-// Wide matrices: 16 RB rows x 64 GPW channels per workgroup (GPW channel groups
-// per wavefront), every wavefront runs the whole K.  Wavefront w fetches the
-// digit fragments of row block w for everyone and leaves them in LDS in fragment
-// order (lane l at 16 l: conflict-free).  Weights go from global memory to
-// registers to the matrix core.
+// A tile: 32 RB rows x 128 GP channels per workgroup (GP tiles of 32 channels per
+// wavefront), every wavefront runs the whole K on v_mfma_i32_32x32x32_i8.  A wavefront
+// that has its SIMD to itself issues that instruction at its full rate, the 16 x 16 x 64
+// one at two thirds of it, and it reads half as many operands per product.  Its A operand
+// is 32 channels x 32 k: the lanes take it from the tiles of two channel groups.  What
+// bounds it: 1931 rows of gate | up run at 1.73 P operations/s (16 x 16 x 64: 1.57), half
+// of what the instruction alone reaches; twice the rows per weight give no more (below).
 //
-// The loop is a pipeline of three stages so that the matrix cores never wait:
-//  * global loads run kRing - 2 chunks ahead.  The compiler sinks ordinary loads
-//    down to their first use (and then waits for them there), so they are issued
-//    by hand and waited for by hand: a fetch is GPW + D loads in a fixed order,
-//    vmcnt counts them in order, and each wait names the registers it releases
-//    so that nothing reads them earlier.  The ring registers must never be
-//    spilled (a reload would read a register while its load is in flight): the
-//    build refuses scratch use in this file;
-//  * the fragments of chunk c + 2 go to LDS at the top of chunk c (three
-//    buffers), so the barrier that closes chunk c publishes them a whole chunk
-//    before they are wanted;
-//  * the fragments of the next digit plane (or of the next chunk's first one)
-//    are read from LDS into the second half of a two-slot register buffer while
-//    the matrix instructions of the current plane run.
+// The digit planes' rows go through LDS, shared by the wavefronts; weights go from memory
+// to registers to the matrix core.  Weights are asked for three chunks of 64 k
+// ahead, rows five (two in LDS: step c multiplies buffer c % 3, whose first fragments were
+// read during step c - 1, and fills buffer (c + 2) % 3, last read before the previous
+// barrier).
 //
 // Matrices too narrow to fill the chip with such tiles split K over several
 // workgroups per tile instead of shrinking the tile (a 64 x 64 tile reads its
@@ -482,402 +310,352 @@ __global__ void __launch_bounds__(kSlices *kWave) gemm_w8_i8_kernel(
 // (Finishing a tile inside the kernel, by the workgroup that arrives last at a
 // counter, needs device-scope fences; on this chip they write back and
 // invalidate a whole L2 each time and slowed the running workgroups threefold.)
-template <int GPW> struct RingDepth { static constexpr int value = GPW > 4 ? 4 : 5; };
-
-// LDS of the wide kernel: three fragment buffers in the loop, four output tiles in
-// the epilogue (and with PAIR the values that cross from wavefronts 2 and 3 to 0
-// and 1); behind them, with PAIR, the scales of the workgroup's channels of both
-// matrices and the steps of its rows, fetched once as the launch starts (loaded
-// at their use, every one of them was an L2 round trip the epilogue waited out).
-template <int D, int RB, int GPW, bool PAIR> constexpr size_t wide_main_lds_bytes() {
-  const size_t loop = sizeof(v4i32) * 3 * D * RB * kWave;
-  const size_t epi = sizeof(float) * kSlices * 16 * (GPW * 16 + 4) +
-                     (PAIR ? sizeof(float4) * kSlices * ((RB + 1) / 2) * GPW * kWave : 0);
-  return loop > epi ? loop : epi;
-}
-template <int RB, int GPW> constexpr int wide_epi_scales() { return 2 * 2 * GPW * 16; }
-template <int D, int RB, int GPW, bool PAIR> constexpr size_t wide_lds_bytes() {
-  return wide_main_lds_bytes<D, RB, GPW, PAIR>() +
-         (PAIR ? sizeof(float) * (wide_epi_scales<RB, GPW>() + RB * 16) : 0);
-}
-
-__device__ __forceinline__ void issue_load(v4i32 &dst, const void *p) {
-  asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(dst) : "v"(p) : "memory");
-}
-__device__ __forceinline__ void issue_load_f32(float &dst, const void *p) {
-  asm volatile("global_load_dword %0, %1, off" : "=v"(dst) : "v"(p) : "memory");
-}
-template <int D, int GPW> struct FetchRegs {
-  v4i32 w[GPW];
-  v4i32 a[D];
-};
-// Waits until at most N loads are in flight; the registers of `f` are only valid
-// after it.
-template <int N, int D, int GPW>
-__device__ __forceinline__ void wait_loads(FetchRegs<D, GPW> &f) {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-#pragma unroll
-  for (int g = 0; g < GPW; ++g)
-    asm volatile("" : "+v"(f.w[g])::"memory");
-#pragma unroll
-  for (int j = 0; j < D; ++j)
-    asm volatile("" : "+v"(f.a[j])::"memory");
-}
-
+//
 // PAIR: W holds two matrices of a.groups / 2 channel groups each, one behind the
-// other; wavefronts 0 and 1 of a workgroup take 32 GPW channels of the first,
-// wavefronts 2 and 3 the same channels of the second, and the result is
-// SiLU(first) * second ([M, N / 2]): the two exchange halves of their tiles
-// through LDS in the epilogue, so only half as much is stored and no launch
-// reads both results again.
-template <int D, int RB, int GPW, bool PAIR>
-__global__ void __launch_bounds__(kSlices *kWave) gemm_w8_i8_wide_kernel(
-    const int8_t *p_planes, const int4 *p_W, int p_Mp, int p_Kp, int p_groups, int p_chunks,
-    int p_ncols, int p_cols_padded, int p_slices, int p_chunks_per_slice, GemmI8Args rest) {
-  // what a wavefront needs before its first fetch arrives in SGPRs (this file is
-  // built with -amdgpu-kernarg-preload-count); the rest is loaded behind the fetch
-  GemmI8Args a = rest;
-  a.planes = p_planes;
-  a.W = p_W;
-  a.Mp = p_Mp;
-  a.Kp = p_Kp;
-  a.groups = p_groups;
-  a.chunks = p_chunks;
-  a.ncols = p_ncols;
-  a.cols_padded = p_cols_padded;
-  a.slices = p_slices;
-  a.chunks_per_slice = p_chunks_per_slice;
-  constexpr int kRing = RingDepth<GPW>::value;
-  constexpr int L = GPW + D; // loads per fetch
-  // chunks per unrolled pass: a multiple of the ring, and an even number of
-  // digit steps so that the two-slot fragment buffer is back where it started
-  constexpr int kPass = (kRing * D) % 2 == 0 ? kRing : 2 * kRing;
-  extern __shared__ __attribute__((aligned(16))) v4i32 frag_s[]; // [3][D][RB][64]
-  const int tid = threadIdx.x, lane = tid & 63;
+// other; a tile is a group of the first and the same group of the second, so that a lane
+// holds matching channels of both, and the result is SiLU(first) * second ([M, N / 2]).
+typedef int v16i32 __attribute__((ext_vector_type(16)));
+// Blocks of 32 rows per workgroup: the weights of 256 channels are used for three layers of
+// 32 rows or more (one plane of one block: 512 rows, 1536 -> 8960, 31.2 us; of three 18.6).
+constexpr int row_blocks(int D, int gp) { return D == 1 && gp == 2 ? 3 : 1; }
+constexpr int kWideRow = kTileK + 16; // bytes of a row in LDS: fragment reads meet every bank once
+
+// sum_j 256^j acc_j as f32 (each int32 sum is exact; the conversions round to 24
+// bits, like an f32 accumulator would)
+template <int D> __device__ __forceinline__ float combine(const v16i32 (&acc)[D], int r) {
+  float v = (float)acc[D - 1][r];
+#pragma unroll
+  for (int j = D - 2; j >= 0; --j)
+    v = fmaf(v, 256.0f, (float)acc[j][r]);
+  return v;
+}
+
+// sums 4 q .. 4 q + 3 as they are, carried as float bit patterns
+__device__ __forceinline__ float4 int_bits(const v16i32 &acc, int q) {
+  return make_float4(__int_as_float(acc[4 * q]), __int_as_float(acc[4 * q + 1]),
+                     __int_as_float(acc[4 * q + 2]), __int_as_float(acc[4 * q + 3]));
+}
+
+template <int D, int RB, int GP, bool PAIR>
+__device__ __forceinline__ void multiply_tile(const GemmI8Args &a) {
+  constexpr int kWidth = PAIR ? 16 : 32;    // channels of the result per tile
+  constexpr int kSpan = kWidth * GP;        // ... and per wavefront
+  constexpr int kRows = 32 * RB;            // rows of the tile
+  constexpr int L = D * RB;                 // layers of 32 rows: plane l % D of row block l / D
+  constexpr int kRuns = L * 32 * 4;         // 16-byte runs of a chunk's rows
+  constexpr int kThreads = kSlices * kWave;
+  constexpr int kLoads = (kRuns + kThreads - 1) / kThreads;
+  constexpr int kBuf = L * 32 * kWideRow;
+  constexpr int kTurn = kSpan + 4;          // floats of a row of the epilogue's tile
+  constexpr int kTurned = kSlices * 32 * kTurn * 4;
+  constexpr int kLds = 3 * kBuf > kTurned ? 3 * kBuf : kTurned;
+  constexpr int kScales = kSlices * 32 * GP;
+  // chunks of weights and of rows in registers
+  constexpr int kRing = 4;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[kLds];
+  // the epilogue's operands, asked for as the launch starts: scales (PAIR: of both
+  // matrices), bias, row steps
+  __shared__ __attribute__((aligned(16))) float scale_s[kScales], bias_s[PAIR ? 4 : kScales];
+  __shared__ float step_s[kRows];
+  const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, up = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // ids equal modulo 8 run on the same XCD: the row tiles of one (column tile,
-  // K slice) pair do, and share its weights in that XCD's L2
-  const int unit = blockIdx.x % a.cols_padded, rbk = blockIdx.x / a.cols_padded;
-  if (unit >= a.ncols * a.slices)
-    return; // padding id
-  const int col = unit % a.ncols, slice = unit / a.ncols;
-  const int m0 = rbk * RB * 16;
+  // ids equal modulo 8 run on the same XCD: the row tiles of one (column tile, K slice,
+  // band) do, and share its weights in that XCD's L2
+  const int id = blockIdx.x % a.ids_padded, units = a.ncols * a.slices;
+  const int unit = id % units, rbk = id / units * a.band_rows + blockIdx.x / a.ids_padded;
+  if (rbk >= a.row_tiles)
+    return; // padding id, or a last band with fewer rows
+  const int ctile = unit % a.ncols, slice = unit / a.ncols;
+  const int m0 = rbk * kRows;
   const int half_groups = a.groups / 2; // PAIR only
-  // first channel group of this wavefront; with PAIR, within its matrix
-  const int g0 = PAIR ? (col * 2 + (wave & 1)) * GPW : (col * kSlices + wave) * GPW;
-  const int gbase = PAIR ? (wave >> 1) * half_groups : 0;
   const int glast = PAIR ? half_groups - 1 : a.groups - 1;
+  const int g0 = (ctile * kSlices + wave) * (kSpan / 16); // first channel group of this wavefront
   const int cb = slice * a.chunks_per_slice;
   const int nch = min(a.chunks_per_slice, a.chunks - cb); // chunks of this slice, >= 1
 
-  v4i32 acc[GPW][RB][D];
+  const v4i32 *wp[GP];
 #pragma unroll
-  for (int g = 0; g < GPW; ++g)
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-      for (int j = 0; j < D; ++j)
-        acc[g][rb][j] = v4i32{0, 0, 0, 0};
-
-  const v4i32 *wp[GPW];
-#pragma unroll
-  for (int g = 0; g < GPW; ++g) // groups past the end repeat the last one
-    wp[g] = reinterpret_cast<const v4i32 *>(a.W) +
-            ((size_t)(gbase + min(g0 + g, glast)) * a.chunks + cb) * 64 + lane;
-  const size_t plane = (size_t)a.Mp * a.Kp;
-  // this wavefront fetches row block `wave` of the activation tile (with three
-  // row blocks the fourth wavefront repeats the third's loads and stages nothing)
-  const int my_rb = min(wave, RB - 1);
-  const int8_t *ap = a.planes + (size_t)(m0 + my_rb * 16 + (lane & 15)) * a.Kp +
-                     (size_t)cb * kTileK + (lane >> 4) * 16;
-
-  FetchRegs<D, GPW> ring[kRing];
-  // chunks past the end are fetched again from the last chunk (never used):
-  // every fetch is exactly L loads, which is what keeps the counts below exact
-  auto fetch = [&](int c, FetchRegs<D, GPW> &f) {
-    const int cc = min(c, nch - 1);
-#pragma unroll
-    for (int g = 0; g < GPW; ++g)
-      issue_load(f.w[g], wp[g] + (size_t)cc * 64);
-#pragma unroll
-    for (int j = 0; j < D; ++j)
-      issue_load(f.a[j], ap + j * plane + (size_t)cc * kTileK);
-  };
-  auto stage = [&](const FetchRegs<D, GPW> &f, int buf) { // own row block -> LDS
-    if (wave >= RB)
-      return;
-#pragma unroll
-    for (int j = 0; j < D; ++j)
-      frag_s[(((size_t)buf * D + j) * RB + wave) * kWave + lane] = f.a[j];
-  };
-  auto read_frags = [&](v4i32(&dst)[RB], int buf, int j) {
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-      dst[rb] = frag_s[(((size_t)buf * D + j) * RB + rb) * kWave + lane];
-  };
-  // PAIR: the epilogue's scales (both matrices, this workgroup's 64 GPW channels)
-  // and row steps, two per thread, requested ahead of the stream (so the counted
-  // waits below cover them) and parked in LDS for the epilogue
-  constexpr int kEpiScales = wide_epi_scales<RB, GPW>(); // [matrix][32 GPW channels]
-  float *epi_s = reinterpret_cast<float *>(frag_s) +
-                 wide_main_lds_bytes<D, RB, GPW, PAIR>() / sizeof(float);
-  float epi_v[2] = {0.f, 0.f};
-  bool epi_ok[2] = {false, false};
-  if constexpr (PAIR) {
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int idx = tid + u * kSlices * kWave;
-      const float *src = a.scale; // a valid address for the slots past the end
-      if (idx < kEpiScales) {
-        const int mtx = idx / (kEpiScales / 2), ch = idx % (kEpiScales / 2);
-        const int n = col * (kEpiScales / 2) + ch;
-        epi_ok[u] = n < a.N;
-        if (epi_ok[u])
-          src = a.scale + (size_t)mtx * a.N + n;
-      } else if (idx < kEpiScales + RB * 16) {
-        const int mr = m0 + idx - kEpiScales;
-        epi_ok[u] = mr < a.M;
-        if (epi_ok[u])
-          src = a.steps + mr;
-      }
-      issue_load_f32(epi_v[u], src);
-    }
+  for (int g = 0; g < GP; ++g) { // groups past the end repeat the last one
+    const int second = (lane >> 4) & 1; // group of the tile
+    const int gg =
+        PAIR ? min(g0 + g, glast) + second * half_groups : min(g0 + 2 * g + second, glast);
+    wp[g] = reinterpret_cast<const v4i32 *>(a.W) + ((size_t)gg * a.chunks + cb) * 64 + up * 16 +
+            (lane & 15);
   }
+  const int8_t *src[kLoads];
+  int lds_at[kLoads];
+  bool mine[kLoads];
 #pragma unroll
-  for (int u = 0; u < kRing; ++u)
-    fetch(u, ring[u]);
-  wait_loads<(kRing - 1) * L, D, GPW>(ring[0]); // chunk 0 has arrived
-  if constexpr (PAIR) {
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      asm volatile("" : "+v"(epi_v[u])::"memory"); // older than chunk 0: landed
-      const int idx = tid + u * kSlices * kWave;
-      if (idx < kEpiScales + RB * 16)
-        epi_s[idx] = epi_ok[u] ? epi_v[u] : 0.f;
-    }
+  for (int i = 0; i < kLoads; ++i) {
+    const int idx = i * kThreads + tid, l = min(idx / 128, L - 1);
+    const int r = idx / 4 % 32, q = idx & 3;
+    mine[i] = idx < kRuns;
+    src[i] = a.planes +
+             ((size_t)(l % D) * a.Mp + min(m0 + l / D * 32 + r, a.Mp - 1)) * a.Kp +
+             (size_t)cb * kTileK + q * 16;
+    lds_at[i] = (l * 32 + r) * kWideRow + q * 16;
   }
-  stage(ring[0], 0);
-  wait_loads<(kRing - 2) * L, D, GPW>(ring[1]);
-  stage(ring[1], 1);
+  v4i32 wr[kRing][GP * 2], xr[kRing][kLoads];
+  auto fetch_w = [&](int c, v4i32 (&w)[GP * 2]) {
+    const size_t cc = (size_t)min(c, nch - 1) * 64;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int g = 0; g < GP; ++g)
+        w[g * 2 + h] = wp[g][cc + h * 32];
+  };
+  auto fetch_x = [&](int c, v4i32 (&x)[kLoads]) {
+    const size_t cc = (size_t)min(c, nch - 1) * kTileK;
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i)
+      x[i] = *reinterpret_cast<const v4i32 *>(src[i] + cc);
+  };
+  auto put_x = [&](const v4i32 (&x)[kLoads], unsigned char *buf) {
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i)
+      if (kRuns % kThreads == 0 || mine[i])
+        *reinterpret_cast<v4i32 *>(buf + lds_at[i]) = x[i];
+  };
+  fetch_x(0, xr[0]);
+  fetch_x(1, xr[1]);
+#pragma unroll
+  for (int u = 0; u < kRing - 1; ++u) {
+    fetch_w(u, wr[u]);
+    if (u + 2 < kRing)
+      fetch_x(u + 2, xr[u + 2]);
+  }
+  if (a.slices == 1) {
+    const int n0 = ctile * kSlices * kSpan;
+    for (int i = tid; i < kScales; i += kThreads) {
+      const int mtx = PAIR ? i / (kScales / 2) : 0, n = n0 + (PAIR ? i % (kScales / 2) : i);
+      scale_s[i] = n < a.N ? a.scale[(size_t)mtx * a.N + n] : 0.f;
+      if constexpr (!PAIR)
+        bias_s[i] = a.bias && n < a.N ? a.bias[n] : 0.f;
+    }
+    for (int i = tid; i < kRows; i += kThreads)
+      step_s[i] = m0 + i < a.M ? a.steps[m0 + i] : 0.f;
+  }
+
+  v16i32 acc[GP][RB][D];
+#pragma unroll
+  for (int g = 0; g < GP; ++g)
+#pragma unroll
+    for (int l = 0; l < L; ++l)
+      acc[g][l / D][l % D] = v16i32{};
+
+  unsigned char *cur = lds, *next = lds + kBuf, *fill = lds + 2 * kBuf;
+  put_x(xr[0], cur);
+  put_x(xr[1], next);
+  fetch_x(kRing, xr[0]);
   __syncthreads();
-  v4i32 af[2][RB];
-  read_frags(af[0], 0, 0);
-  int buf = 0; // LDS buffer of chunk c: c % 3
-  for (int c0 = 0; c0 < nch; c0 += kPass) {
+  const int frag_at = col * kWideRow + up * 16;
+  v4i32 frag[4];
+  // sub-step u of a chunk: layer u % L, k half u / L
+  auto load_frag = [&](const unsigned char *buf, int u, v4i32 &f) {
+    f = *reinterpret_cast<const v4i32 *>(buf + frag_at + u % L * 32 * kWideRow + u / L * 32);
+  };
+  load_frag(cur, 0, frag[0]);
+  load_frag(cur, 1, frag[1]);
+  // f: the slot of sub-step 0's fragments
+  auto step = [&](int c, int f, v4i32 (&w)[GP * 2], v4i32 (&w_new)[GP * 2], v4i32 (&x)[kLoads],
+                  v4i32 (&x_new)[kLoads]) {
 #pragma unroll
-    for (int u = 0; u < kPass; ++u) {
-      const int c = c0 + u;
-      if (c < nch) {
-        FetchRegs<D, GPW> &cur = ring[u % kRing];
-        FetchRegs<D, GPW> &ahead = ring[(u + 2) % kRing];
-        const int buf1 = buf == 2 ? 0 : buf + 1, buf2 = buf1 == 2 ? 0 : buf1 + 1;
-        // in flight: chunks c+2 .. c+kRing-1.  Release chunk c+2 and put its row
-        // block into the buffer that held chunk c-1, whose readers passed the
-        // barrier that closed chunk c-1.
-        wait_loads<(kRing - 3) * L, D, GPW>(ahead);
-        stage(ahead, buf2);
+    for (int u = 0; u < 2 * L; ++u) {
+      // fragments are asked for two sub-steps ahead of their products (one takes less than
+      // the way through LDS), and stay there: left to itself the scheduler moves them to
+      // their use
+      load_frag(u + 2 < 2 * L ? cur : next, (u + 2) % (2 * L), frag[(f + u + 2) & 3]);
+      if (u == 0)
+        fetch_w(c + kRing - 1, w_new);
+      if (u == 1)
+        put_x(x, fill);
+      if (u == (L > 1 ? 2 : 1))
+        fetch_x(c + kRing + 1, x_new);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < D; ++j) {
-          const int p = (u * D + j) & 1; // slot of this digit step's fragments
-          if (j + 1 < D)
-            read_frags(af[p ^ 1], buf, j + 1);
-          else
-            read_frags(af[p ^ 1], buf1, 0);
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-            for (int g = 0; g < GPW; ++g)
-              acc[g][rb][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(cur.w[g], af[p][rb],
-                                                                    acc[g][rb][j], 0, 0, 0);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        // the matrix cores have read the registers of chunk c when the next
-        // instruction issues: fetch the chunk kRing further on into them
-        fetch(c + kRing, cur);
-        __syncthreads();
-        buf = buf1;
-      }
+      for (int g = 0; g < GP; ++g)
+        acc[g][u % L / D][u % D] = __builtin_amdgcn_mfma_i32_32x32x32_i8(
+            w[g * 2 + u / L], frag[(f + u) & 3], acc[g][u % L / D][u % D], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
     }
-  }
-  // loads of the repeated last chunk may still be in flight: their registers
-  // stay allocated until the wait is over
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    unsigned char *t = cur;
+    cur = next;
+    next = fill;
+    fill = t;
+  };
+  // step c: weights from slot c, new ones into slot c - 1; rows c + 2 go to LDS, new ones
+  // into slot c + 1 (all modulo kRing)
+  for (int c0 = 0; c0 < nch; c0 += kRing) {
 #pragma unroll
-  for (int u = 0; u < kRing; ++u)
-    wait_loads<0, D, GPW>(ring[u]);
+    for (int u = 0; u < kRing; ++u)
+      if (c0 + u < nch)
+        step(c0 + u, (u * 2 * L) & 3, wr[u], wr[(u + kRing - 1) % kRing], xr[(u + 2) % kRing],
+             xr[(u + 1) % kRing]);
+  }
 
   // ---- epilogue ---------------------------------------------------------
-  // A lane's accumulator registers are 4 channels of one row: stored as they are,
-  // a store instruction would write 64-byte pieces of 16 rows.  Each wavefront
-  // turns its 16 x (16 GPW) tile around in its own part of LDS (free now: every
-  // wavefront is past the last barrier of the loop) and writes whole row
-  // segments, 64 GPW bytes each.
-  constexpr int kPad = GPW * 16 + 4; // floats per tile row in LDS
-  float *tile = reinterpret_cast<float *>(frag_s) + wave * (16 * kPad);
+  // A lane holds channels 8 q + 4 up + 0..3, q = 0..3, of row `col` of every tile: stored
+  // as they are, a store instruction would write 32-byte pieces of 32 rows.  Each
+  // wavefront turns its 32 rows around in its own part of LDS (free now: every wavefront
+  // is past the last barrier of the loop) and writes whole row segments.
+  float *tile = reinterpret_cast<float *>(lds) + wave * (32 * kTurn);
   const int n0 = g0 * kTileN;
-  const bool vec = (a.ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(a.C) & 15) == 0;
+  auto turn_in = [&](int g, int q, float4 v) {
+    *reinterpret_cast<float4 *>(tile + col * kTurn + g * kWidth + 8 * q + 4 * up) = v;
+  };
+  constexpr int kQuads = kSpan / 4; // float4 of a row
   if (a.slices > 1) {
-    // unscaled sums of this slice; reduce_slices_kernel finishes the tile
-    constexpr int kSub = 16 * GPW * 16; // floats of one wavefront's row block
-    const int tile_id = rbk * a.ncols + col;
-    float *mine = a.partial +
-                  ((((size_t)tile_id * a.slices + slice) * kSlices + wave) * RB) * kSub;
+    // unscaled sums of this slice, [wavefront][row][channel]; the kernel that adds the
+    // slices finishes the tile
+    const size_t at = ((size_t)(rbk * a.ncols + ctile) * a.slices + slice) * kSlices + wave;
+    float *part = a.partial + at * kRows * kSpan;
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
 #pragma unroll
-      for (int g = 0; g < GPW; ++g) {
-        float4 o = make_float4(combine<D>(acc[g][rb], 0), combine<D>(acc[g][rb], 1),
-                               combine<D>(acc[g][rb], 2), combine<D>(acc[g][rb], 3));
-        if constexpr (D == 1) {
-          if (a.int_partials) // exact beyond 2^24: the bits travel as they are
-            o = make_float4(__int_as_float(acc[g][rb][0][0]), __int_as_float(acc[g][rb][0][1]),
-                            __int_as_float(acc[g][rb][0][2]), __int_as_float(acc[g][rb][0][3]));
-        }
-        *reinterpret_cast<float4 *>(tile + (lane & 15) * kPad + g * 16 + (lane >> 4) * 4) = o;
-      }
+      for (int g = 0; g < GP; ++g)
 #pragma unroll
-      for (int i = 0; i < GPW; ++i) {
-        const int idx = lane + 64 * i;
-        const int row = idx / (GPW * 4), c4 = idx % (GPW * 4);
-        *reinterpret_cast<float4 *>(mine + (size_t)rb * kSub + idx * 4) =
-            *reinterpret_cast<const float4 *>(tile + row * kPad + c4 * 4);
+        for (int q = 0; q < 4; ++q) {
+          const v16i32(&t)[D] = acc[g][rb];
+          float4 o = make_float4(combine<D>(t, 4 * q), combine<D>(t, 4 * q + 1),
+                                 combine<D>(t, 4 * q + 2), combine<D>(t, 4 * q + 3));
+          if constexpr (D == 1) {
+            if (a.int_partials) // exact beyond 2^24: the bits travel as they are
+              o = int_bits(t[0], q);
+          }
+          turn_in(g, q, o);
+        }
+#pragma unroll
+      for (int i = 0; i < kQuads / 2; ++i) {
+        const int idx = lane + 64 * i, row = idx / kQuads, c4 = idx % kQuads;
+        *reinterpret_cast<float4 *>(part + (size_t)(rb * 32 + row) * kSpan + c4 * 4) =
+            *reinterpret_cast<const float4 *>(tile + row * kTurn + c4 * 4);
       }
     }
     return;
   }
-  // without PAIR the scales and the bias stay in registers over the row blocks;
-  // with it there is no register left for them, and each use loads them again
-  float s[PAIR ? 1 : GPW][4], b[PAIR ? 1 : GPW][4];
-  if constexpr (!PAIR) {
-#pragma unroll
-    for (int g = 0; g < GPW; ++g) {
-      const int n = (g0 + g) * kTileN + (lane >> 4) * 4;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        s[g][r] = n + r < a.N ? a.scale[n + r] : 0.f;
-        b[g][r] = (a.bias && n + r < a.N) ? a.bias[n + r] : 0.f;
-      }
-    }
-  }
-  // finished values of channel group g, row block rb (PAIR: the scales of the
-  // second matrix follow those of the first; a.N is a multiple of 16)
-  auto finished = [&](int g, int rb, float step) {
-    float4 o;
-    if constexpr (PAIR) {
-      const float4 sc = *reinterpret_cast<const float4 *>(
-          epi_s + (wave >> 1) * (kEpiScales / 2) + ((wave & 1) * GPW + g) * kTileN +
-          (lane >> 4) * 4);
-      o.x = scaled<D>(combine<D>(acc[g][rb], 0), step, sc.x);
-      o.y = scaled<D>(combine<D>(acc[g][rb], 1), step, sc.y);
-      o.z = scaled<D>(combine<D>(acc[g][rb], 2), step, sc.z);
-      o.w = scaled<D>(combine<D>(acc[g][rb], 3), step, sc.w);
-    } else {
-      o.x = b[g][0] + scaled<D>(combine<D>(acc[g][rb], 0), step, s[g][0]);
-      o.y = b[g][1] + scaled<D>(combine<D>(acc[g][rb], 1), step, s[g][1]);
-      o.z = b[g][2] + scaled<D>(combine<D>(acc[g][rb], 2), step, s[g][2]);
-      o.w = b[g][3] + scaled<D>(combine<D>(acc[g][rb], 3), step, s[g][3]);
-    }
-    return o;
-  };
-  // PAIR: the wavefronts of the first matrix finish the upper row blocks of the
-  // tile, those of the second the lower ones (each stores half as much as an
-  // unpaired wavefront): what a wavefront computed of the other's row blocks
-  // crosses over through LDS, same lane, same registers
-  constexpr int kUpper = (RB + 1) / 2;
-  const bool second = PAIR && wave >= 2;
-  float4 *cross = reinterpret_cast<float4 *>(reinterpret_cast<float *>(frag_s) +
-                                             kSlices * 16 * kPad);
-  if constexpr (PAIR) {
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-      if (second ? rb >= kUpper : rb < kUpper)
-        continue; // stays here
-      const float step = epi_s[kEpiScales + rb * 16 + (lane & 15)];
-      const int slot = rb < kUpper ? rb : rb - kUpper;
-#pragma unroll
-      for (int g = 0; g < GPW; ++g)
-        cross[((wave * kUpper + slot) * GPW + g) * kWave + lane] = finished(g, rb, step);
-    }
-    __syncthreads();
-  }
+  const bool vec = (a.ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(a.C) & 15) == 0;
+  const float *scales = scale_s + wave * kSpan;
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
-    if (PAIR && (second ? rb < kUpper : rb >= kUpper))
-      continue; // the partner wavefront finishes this row block
-    const int mr = m0 + rb * 16 + (lane & 15);
-    float step;
-    if constexpr (PAIR)
-      step = epi_s[kEpiScales + rb * 16 + (lane & 15)];
-    else
-      step = mr < a.M ? a.steps[mr] : 0.f;
+    const float row_step = step_s[rb * 32 + col];
 #pragma unroll
-    for (int g = 0; g < GPW; ++g) {
-      float4 o = finished(g, rb, step);
-      if constexpr (PAIR) {
-        const int slot = rb < kUpper ? rb : rb - kUpper;
-        const float4 p = cross[(((wave ^ 2) * kUpper + slot) * GPW + g) * kWave + lane];
-        const float4 gate = second ? p : o, up = second ? o : p;
-        o = make_float4(silu_times(gate.x, up.x), silu_times(gate.y, up.y),
-                        silu_times(gate.z, up.z), silu_times(gate.w, up.w));
+    for (int g = 0; g < GP; ++g)
+#pragma unroll
+      for (int q = 0; q < kWidth / 8; ++q) {
+        const int ch = g * kWidth + 8 * q + 4 * up;
+        const v16i32(&t)[D] = acc[g][rb];
+        const float4 sc = *reinterpret_cast<const float4 *>(scales + ch);
+        const float s[4] = {sc.x, sc.y, sc.z, sc.w};
+        float o[4];
+        if constexpr (PAIR) {
+          const float4 su = *reinterpret_cast<const float4 *>(scales + kScales / 2 + ch);
+          const float s2[4] = {su.x, su.y, su.z, su.w};
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            o[i] = silu_times(scaled<D>(combine<D>(t, 4 * q + i), row_step, s[i]),
+                              scaled<D>(combine<D>(t, 4 * q + 8 + i), row_step, s2[i]));
+        } else {
+          const float4 bb = *reinterpret_cast<const float4 *>(bias_s + wave * kSpan + ch);
+          const float b[4] = {bb.x, bb.y, bb.z, bb.w};
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            o[i] = b[i] + scaled<D>(combine<D>(t, 4 * q + i), row_step, s[i]);
+        }
+        turn_in(g, q, make_float4(o[0], o[1], o[2], o[3]));
       }
-      *reinterpret_cast<float4 *>(tile + (lane & 15) * kPad + g * 16 + (lane >> 4) * 4) = o;
-    }
 #pragma unroll
-    for (int i = 0; i < GPW; ++i) { // 16 rows x 4 GPW float4 = 64 GPW lanes' worth
-      const int idx = lane + 64 * i;
-      const int row = idx / (GPW * 4), c4 = idx % (GPW * 4);
-      const float4 o = *reinterpret_cast<const float4 *>(tile + row * kPad + c4 * 4);
-      const int m = m0 + rb * 16 + row, n = n0 + c4 * 4;
+    for (int i = 0; i < kQuads / 2; ++i) {
+      const int idx = lane + 64 * i, row = idx / kQuads, c4 = idx % kQuads;
+      const float4 o = *reinterpret_cast<const float4 *>(tile + row * kTurn + c4 * 4);
+      const int m = m0 + rb * 32 + row, n = n0 + c4 * 4;
       if (m >= a.M || n >= a.N)
         continue;
-      float *c = a.C + (int64_t)m * a.ldc + n;
+      float *cp = a.C + (int64_t)m * a.ldc + n;
       if (vec && n + 3 < a.N) {
         float4 q = o;
         if (a.accumulate) {
-          const float4 p = *reinterpret_cast<const float4 *>(c);
+          const float4 p = *reinterpret_cast<const float4 *>(cp);
           q = make_float4(p.x + q.x, p.y + q.y, p.z + q.z, p.w + q.w);
         }
-        *reinterpret_cast<float4 *>(c) = q;
+        *reinterpret_cast<float4 *>(cp) = q;
       } else {
         const float v[4] = {o.x, o.y, o.z, o.w};
 #pragma unroll
         for (int r = 0; r < 4; ++r)
           if (n + r < a.N)
-            c[r] = a.accumulate ? c[r] + v[r] : v[r];
+            cp[r] = a.accumulate ? cp[r] + v[r] : v[r];
       }
     }
     if constexpr (D == 1) {
       if (a.sums) { // the same turn for the integer sums, carried as float bit patterns
 #pragma unroll
-        for (int g = 0; g < GPW; ++g)
-          *reinterpret_cast<float4 *>(tile + (lane & 15) * kPad + g * 16 + (lane >> 4) * 4) =
-              make_float4(__int_as_float(acc[g][rb][0][0]), __int_as_float(acc[g][rb][0][1]),
-                          __int_as_float(acc[g][rb][0][2]), __int_as_float(acc[g][rb][0][3]));
+        for (int g = 0; g < GP; ++g)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            turn_in(g, q, int_bits(acc[g][rb][0], q));
         const bool ivec = (a.N & 3) == 0 && (reinterpret_cast<uintptr_t>(a.sums) & 15) == 0;
 #pragma unroll
-        for (int i = 0; i < GPW; ++i) {
-          const int idx = lane + 64 * i;
-          const int row = idx / (GPW * 4), c4 = idx % (GPW * 4);
-          const float4 q = *reinterpret_cast<const float4 *>(tile + row * kPad + c4 * 4);
+        for (int i = 0; i < kQuads / 2; ++i) {
+          const int idx = lane + 64 * i, row = idx / kQuads, c4 = idx % kQuads;
+          const float4 q = *reinterpret_cast<const float4 *>(tile + row * kTurn + c4 * 4);
           const v4i32 o = {__float_as_int(q.x), __float_as_int(q.y), __float_as_int(q.z),
                            __float_as_int(q.w)};
-          const int m = m0 + rb * 16 + row, n = n0 + c4 * 4;
+          const int m = m0 + rb * 32 + row, n = n0 + c4 * 4;
           if (m >= a.M || n >= a.N)
             continue;
-          int32_t *c = a.sums + (int64_t)m * a.N + n;
+          int32_t *cp = a.sums + (int64_t)m * a.N + n;
           if (ivec) {
-            *reinterpret_cast<v4i32 *>(c) = o;
+            *reinterpret_cast<v4i32 *>(cp) = o;
           } else {
 #pragma unroll
             for (int r = 0; r < 4; ++r)
               if (n + r < a.N)
-                c[r] = o[r];
+                cp[r] = o[r];
           }
         }
       }
     }
   }
+}
+
+// What a wavefront needs before its first fetch arrives in SGPRs (this file is built
+// with -amdgpu-kernarg-preload-count); the rest is loaded behind the fetch.
+#define BH_I8_LEADING                                                                              \
+  const int8_t *planes, const int4 *W, int Mp, int Kp, int groups, int chunks, int ncols,          \
+      int slices, int chunks_per_slice, int ids_padded, int band_rows, int row_tiles, GemmI8Args a
+#define BH_I8_TAKE                                                                                 \
+  a.planes = planes;                                                                               \
+  a.W = W;                                                                                         \
+  a.Mp = Mp;                                                                                       \
+  a.Kp = Kp;                                                                                       \
+  a.groups = groups;                                                                               \
+  a.chunks = chunks;                                                                               \
+  a.ncols = ncols;                                                                                 \
+  a.slices = slices;                                                                               \
+  a.chunks_per_slice = chunks_per_slice;                                                           \
+  a.ids_padded = ids_padded;                                                                       \
+  a.band_rows = band_rows;                                                                         \
+  a.row_tiles = row_tiles;
+
+// 128 channels per workgroup, and 256
+template <int D>
+__global__ void __launch_bounds__(kSlices *kWave) gemm_w8_i8_kernel(BH_I8_LEADING) {
+  BH_I8_TAKE
+  multiply_tile<D, 1, 1, false>(a);
+}
+template <int D, bool PAIR>
+__global__ void __launch_bounds__(kSlices *kWave) gemm_w8_i8_wide_kernel(BH_I8_LEADING) {
+  BH_I8_TAKE
+  multiply_tile<D, row_blocks(D, 2), 2, PAIR>(a);
+}
+
+// Where the sums of row m, channels n.. of the first K slice lie.
+__device__ __forceinline__ const float *first_slice(const GemmI8Args &a, int m, int n) {
+  const int tile = m / a.tile_rows * a.ncols + n / (kSlices * a.span), wave = n / a.span % kSlices;
+  const size_t row =
+      ((size_t)tile * a.slices * kSlices + wave) * a.tile_rows + m % a.tile_rows;
+  return a.partial + row * a.span + n % a.span;
 }
 
 // Sum of a float4 over the K slices, in slice order, four loads in flight at a
@@ -919,19 +697,14 @@ __device__ __forceinline__ FinishOperands load_finish_operands(const GemmI8Args 
 
 // C (+)= step[m] * scale[n] * sum over slices of the unscaled sums, slice order.
 __global__ void __launch_bounds__(256)
-reduce_slices_kernel(GemmI8Args a, int rb_per_tile, int gpw) {
+reduce_slices_kernel(GemmI8Args a) {
   const int n4 = (a.N + 3) / 4;
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= (int64_t)a.M * n4)
     return;
   const int m = (int)(i / n4), n = (int)(i % n4) * 4;
-  const int span = 16 * gpw; // channels per wavefront
-  const int rbk = m / (16 * rb_per_tile), rb = (m / 16) % rb_per_tile, row = m % 16;
-  const int col = n / (kSlices * span), wave = (n / span) % kSlices, ch = n % span;
-  const int sub = 16 * span;
-  const size_t slice_stride = (size_t)kSlices * rb_per_tile * sub;
-  const float *p = a.partial + ((size_t)(rbk * a.ncols + col) * a.slices) * slice_stride +
-                   ((size_t)wave * rb_per_tile + rb) * sub + row * span + ch;
+  const size_t slice_stride = (size_t)kSlices * a.tile_rows * a.span;
+  const float *p = first_slice(a, m, n);
   const float step = a.steps[m];
   float *c = a.C + (int64_t)m * a.ldc + n;
   const FinishOperands f = load_finish_operands(a, c, n);
@@ -949,19 +722,14 @@ reduce_slices_kernel(GemmI8Args a, int rb_per_tile, int gpw) {
 // C = f32(sum) * (step * scale[n]) in that order (linalg.py:12833-12845), and the
 // sums themselves where the caller asked for them.
 __global__ void __launch_bounds__(256)
-reduce_slices_i32_kernel(GemmI8Args a, int rb_per_tile, int gpw) {
+reduce_slices_i32_kernel(GemmI8Args a) {
   const int n4 = (a.N + 3) / 4;
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= (int64_t)a.M * n4)
     return;
   const int m = (int)(i / n4), n = (int)(i % n4) * 4;
-  const int span = 16 * gpw;
-  const int rbk = m / (16 * rb_per_tile), rb = (m / 16) % rb_per_tile, row = m % 16;
-  const int col = n / (kSlices * span), wave = (n / span) % kSlices, ch = n % span;
-  const int sub = 16 * span;
-  const size_t slice_stride = (size_t)kSlices * rb_per_tile * sub;
-  const float *p = a.partial + ((size_t)(rbk * a.ncols + col) * a.slices) * slice_stride +
-                   ((size_t)wave * rb_per_tile + rb) * sub + row * span + ch;
+  const size_t slice_stride = (size_t)kSlices * a.tile_rows * a.span;
+  const float *p = first_slice(a, m, n);
   int v[4] = {0, 0, 0, 0};
   for (int sl = 0; sl < a.slices; sl += 4) {
     v4i32 q[4];
@@ -990,7 +758,7 @@ reduce_slices_i32_kernel(GemmI8Args a, int rb_per_tile, int gpw) {
 // row_to_digits, then [Kp2] the row.
 __global__ void __launch_bounds__(kRowThreads)
 reduce_slices_norm_kernel(const float *p_partial, const float *p_steps, int p_N, int p_ncols,
-                          int p_slices, int rb_per_tile, int gpw, GemmI8Args rest,
+                          int p_slices, int p_span, int p_tile_rows, GemmI8Args rest,
                           const float *__restrict__ norm_w, float inv_n, float eps, int D,
                           int Mp2, int Kp2, int8_t *__restrict__ planes) {
   GemmI8Args a = rest; // the leading parameters arrive in SGPRs, ahead of the first load
@@ -999,21 +767,18 @@ reduce_slices_norm_kernel(const float *p_partial, const float *p_steps, int p_N,
   a.N = p_N;
   a.ncols = p_ncols;
   a.slices = p_slices;
+  a.span = p_span;
+  a.tile_rows = p_tile_rows;
   __shared__ float red[kRowThreads / 64];
   extern __shared__ __attribute__((aligned(16))) float row_lds[];
   float *xrow = row_lds + Kp2;
   const int m = blockIdx.x;
   const int n4 = (a.N + 3) / 4;
-  const int span = 16 * gpw;
-  const int rbk = m / (16 * rb_per_tile), rb = (m / 16) % rb_per_tile, row = m % 16;
-  const int sub = 16 * span;
-  const size_t slice_stride = (size_t)kSlices * rb_per_tile * sub;
+  const size_t slice_stride = (size_t)kSlices * a.tile_rows * a.span;
   const float step = a.steps[m];
   for (int q4 = threadIdx.x; q4 < n4; q4 += kRowThreads) {
     const int n = q4 * 4;
-    const int col = n / (kSlices * span), wave = (n / span) % kSlices, ch = n % span;
-    const float *p = a.partial + ((size_t)(rbk * a.ncols + col) * a.slices) * slice_stride +
-                     ((size_t)wave * rb_per_tile + rb) * sub + row * span + ch;
+      const float *p = first_slice(a, m, n);
     float *c = a.C + (int64_t)m * a.ldc + n;
     const FinishOperands f = load_finish_operands(a, c, n);
     float v[4];
@@ -1045,23 +810,26 @@ reduce_slices_norm_kernel(const float *p_partial, const float *p_steps, int p_N,
 }
 
 BH_VARIANT_FAMILY(WideFamily, "gemm_w8_i8_wide_kernel");
-BH_VARIANT_FAMILY(SplitFamily, "gemm_w8_i8_kernel");
+BH_VARIANT_FAMILY(NarrowFamily, "gemm_w8_i8_kernel");
 
-template <int D, int RB, int GPW, bool PAIR = false>
-int launch_wide(const GemmI8Args &a, unsigned blocks, hipStream_t stream) {
-  constexpr size_t lds = wide_lds_bytes<D, RB, GPW, PAIR>();
-  auto kernel = gemm_w8_i8_wide_kernel<D, RB, GPW, PAIR>;
-  if (lds > 48 * 1024) {
-    static DynLdsOnce dyn_lds;
-    BH_CHECK_HIP(ensure_dyn_lds(dyn_lds, reinterpret_cast<const void *>(kernel),
-                                (int)lds));
-  }
-  BH_NOTE_VARIANT(WideFamily, D, RB, GPW, (int)PAIR);
-  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kSlices * kWave), lds, stream, a.planes, a.W, a.Mp,
-                     a.Kp, a.groups, a.chunks, a.ncols, a.cols_padded, a.slices, a.chunks_per_slice,
-                     a);
+template <class Kernel>
+int launch_tiles(Kernel kernel, const GemmI8Args &a, unsigned blocks, hipStream_t stream) {
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kSlices * kWave), 0, stream, a.planes, a.W, a.Mp,
+                     a.Kp, a.groups, a.chunks, a.ncols, a.slices, a.chunks_per_slice,
+                     a.ids_padded, a.band_rows, a.row_tiles, a);
   BH_CHECK_HIP(hipGetLastError());
   return BUDDY_HIP_OK;
+}
+
+template <int D, bool PAIR>
+int launch_wide(const GemmI8Args &a, unsigned blocks, hipStream_t stream) {
+  BH_NOTE_VARIANT(WideFamily, D, (int)PAIR);
+  return launch_tiles(gemm_w8_i8_wide_kernel<D, PAIR>, a, blocks, stream);
+}
+
+template <int D> int launch_narrow(const GemmI8Args &a, unsigned blocks, hipStream_t stream) {
+  BH_NOTE_VARIANT(NarrowFamily, D);
+  return launch_tiles(gemm_w8_i8_kernel<D>, a, blocks, stream);
 }
 
 } // namespace
@@ -1078,14 +846,14 @@ int launch_activations_to_digits(const float *A, int64_t lda, int64_t M, int64_t
              "activations_to_digits: bad argument");
   const GemmStagingLayout l = gemm_staging_layout(M, K);
   hipLaunchKernelGGL(activations_to_digits_kernel, dim3((unsigned)l.rows_padded), dim3(kRowThreads),
-                     row_cache_bytes(l.cols_padded), stream, A, lda, (int)M, (int)K, digits, l.rows_padded,
-                     l.cols_padded, static_cast<int8_t *>(staged));
+                     row_cache_bytes(l.cols_padded), stream, A, lda, (int)M, (int)K, digits,
+                     l.rows_padded, l.cols_padded, static_cast<int8_t *>(staged));
   BH_CHECK_HIP(hipGetLastError());
   return BUDDY_HIP_OK;
 }
 
-int launch_attn_fold_to_digits(const PromptFold &fold, int64_t o_stride, int heads, int tokens, int digits,
-                               void *staged, hipStream_t stream) {
+int launch_attn_fold_to_digits(const PromptFold &fold, int64_t o_stride, int heads, int tokens,
+                               int digits, void *staged, hipStream_t stream) {
   const int64_t K = (int64_t)heads * kPromptD;
   BH_REQUIRE(fold.blocks && staged && tokens > 0 && (digits == 2 || digits == 3),
              "attn_fold_to_digits: bad argument");
@@ -1150,28 +918,97 @@ int workspace_for(hipStream_t stream, size_t bytes, char **out) {
   return BUDDY_HIP_OK;
 }
 
-template <int D> int launch_split(const GemmI8Args &a, unsigned blocks, hipStream_t stream) {
-  constexpr size_t lds = sizeof(float) * kSlices * 64 * kWave;
-  auto kernel = gemm_w8_i8_kernel<D>;
-  static DynLdsOnce dyn_lds;
-  BH_CHECK_HIP(ensure_dyn_lds(dyn_lds, reinterpret_cast<const void *>(kernel),
-                              (int)lds));
-  BH_NOTE_VARIANT(SplitFamily, D);
-  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kSlices * kWave), lds, stream, a.planes, a.W, a.Mp,
-                     a.Kp, a.groups, a.chunks, a.ncols, a.cols_padded, a.slices, a.chunks_per_slice,
-                     a);
-  BH_CHECK_HIP(hipGetLastError());
-  return BUDDY_HIP_OK;
+// Channel tiles per wavefront, K slices and bands of rows for a launch, by an estimate of
+// its time in microseconds.  An XCD (32 compute units) works on 64 workgroups at a time, two
+// to a compute unit.  A chunk of 64 k on L layers of 32 rows (planes, blocks of rows) takes
+// a compute unit with two workgroups 0.18 + 0.16 L us, one that has its compute unit to
+// itself 0.15 + 0.08 L us (with one channel tile 0.2 + 0.085 L and 0.06 + 0.07 L, at least
+// 0.21: the way through LDS); a last round that fills less than half runs at the latter.
+// Fitted to these, microseconds (three planes; two; in brackets 16 x 16 x 64 instructions
+// on tiles of 32 or 64 rows x 128 or 256 channels):
+//   gate | up, 1536 -> 2 x 8960: 27 rows 13.7 [18.4]; 12.1 [15.0], 256: 32.6 [30.6]; 27.3
+//     [23.3], 512: 52.3 [58.8]; 42.7 [44.3], 1931: 180 [201]; 141 [150]
+//   down, 8960 -> 1536, with the adding of its slices: 27 rows 12.7 [16.9]; 11.1 [15.1],
+//     512: 34 [36]; 29 [28], 1931: 96 [112]; 77 [95]
+//   q|k|v, 1536 -> 2048: 100 rows 10.0 [13.3]; 8.2 [12.6], 512: 12.5 [15.8]; 9.9 [11.8],
+//     1024: 17.2 [30.4]; 14.4 [22.7]
+//   one plane: 1536 -> 8960: 512 rows 18.6 [21.2], 2048: 52 [69]
+// (A tile of 64 rows x 256 channels, one workgroup to a compute unit, takes as long per
+// row; its rounds are coarser: gate | up at 512 rows 61.8, at 256 rows 40.6.)
+// The (column tile, slice) pairs of an XCD keep their row tiles together; where their number
+// is a poor multiple of 8 the rows are cut into bands, which share the XCDs more evenly and
+// read the weights once per band (4096 rows, 512 -> 512: 9.0 us, in one band 25.5).
+struct TilePlan {
+  int gp = 0, slices = 1, bands = 1;
+  double us = 0;
+};
+template <int D, bool PAIR>
+TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, bool may_split, double norm_us,
+                    int64_t sum_wgs) {
+  TilePlan best;
+  constexpr int64_t kRoom = 64;
+  for (int gp = PAIR ? 2 : 1; gp <= 2; ++gp) {
+    const int64_t ncols = ceil_div(channels, kSlices * gp * (PAIR ? 16 : 32));
+    const int layers = D * row_blocks(D, gp);
+    const int64_t rows = ceil_div(M, 32 * row_blocks(D, gp));
+    const double alone = gp == 2 ? 0.15 + 0.08 * layers : std::max(0.21, 0.06 + 0.07 * layers);
+    const double full = gp == 2 ? 0.18 + 0.16 * layers : 0.2 + 0.085 * layers;
+    for (int s = 1; s <= (may_split ? 16 : 1); ++s) {
+      int bands = 1;
+      int64_t per_xcd = ceil_div(ncols * s, 8) * rows;
+      for (int b = 2; b <= 8; b *= 2) {
+        const int64_t share = ceil_div(ncols * s * b, 8) * ceil_div(rows, b);
+        if (10 * share < 9 * per_xcd) {
+          per_xcd = share;
+          bands = b;
+        }
+      }
+      if (s > 1 && per_xcd > 4 * kRoom)
+        break;
+      const int64_t cps = ceil_div(chunks, s);
+      if (ceil_div(chunks, cps) != s)
+        continue; // the last slice would be empty
+      const double store = s > 1 ? 2.0 : 0.0; // of the partial sums
+      const double full_us = full * (double)cps + (gp == 2 ? 4.0 : 4.5) + store;
+      const double alone_us = alone * (double)cps + (gp == 2 ? 5.0 : 4.5) + store;
+      const int64_t left = per_xcd % kRoom;
+      const double last_us = left == 0 ? 0.0 : 2 * left <= kRoom ? alone_us : full_us;
+      double us = (double)(per_xcd / kRoom) * full_us + last_us;
+      if (s > 1) // the kernel that adds the slices: 3 us and its bytes
+        us += 3.0 + 4.0 * (double)(M * s) * (double)(ncols * 128 * gp) / 5e6 +
+              0.002 * (double)sum_wgs;
+      else
+        us += norm_us;
+      if (!best.gp || us < best.us - 1e-9)
+        best = {gp, s, bands, us};
+    }
+  }
+  return best;
 }
 
-template <int D, bool PAIR = false>
-int launch_shape(int rb, int gpw, const GemmI8Args &a, unsigned blocks, hipStream_t stream) {
-  switch (rb * 10 + gpw) {
-  case 34: return launch_wide<D, 3, 4, PAIR>(a, blocks, stream);
-  case 35: return launch_wide<D, 3, 5, PAIR>(a, blocks, stream);
-  case 44: return launch_wide<D, 4, 4, PAIR>(a, blocks, stream);
-  default: return launch_wide<D, 4, 5, PAIR>(a, blocks, stream);
+template <int D, bool PAIR>
+int launch_plan(const TilePlan &plan, GemmI8Args &a, hipStream_t stream) {
+  a.ncols = (int)ceil_div(a.N, kSlices * (PAIR ? 16 : 32) * plan.gp);
+  a.tile_rows = 32 * row_blocks(D, plan.gp);
+  a.span = 32 * plan.gp;
+  a.row_tiles = (int)ceil_div(a.M, a.tile_rows);
+  a.band_rows = (int)ceil_div(a.row_tiles, plan.bands);
+  a.slices = plan.slices;
+  a.chunks_per_slice = (int)ceil_div(a.chunks, plan.slices);
+  a.ids_padded = (int)round_up((int64_t)a.ncols * a.slices * plan.bands, 8);
+  if (plan.slices > 1) {
+    const size_t tile_floats = (size_t)a.tile_rows * kSlices * a.span;
+    const size_t bytes = sizeof(float) * tile_floats * plan.slices * (size_t)a.ncols * a.row_tiles;
+    char *ws = nullptr;
+    if (int rc = workspace_for(stream, bytes, &ws))
+      return rc;
+    a.partial = reinterpret_cast<float *>(ws);
   }
+  const unsigned blocks = (unsigned)(a.ids_padded * a.band_rows);
+  if constexpr (!PAIR)
+    if (plan.gp == 1)
+      return launch_narrow<D>(a, blocks, stream);
+  return launch_wide<D, PAIR>(a, blocks, stream);
 }
 
 } // namespace
@@ -1214,84 +1051,19 @@ int launch_gemm_w8_digits_d(const GemmW8Args &in, const void *planes, hipStream_
   a.int_partials = 0;
   a.slices = 1;
   if (in.silu_pair) {
-    // two matrices of N / 2 channels, result SiLU(first) * second: wide tiles of
-    // 32 GPW channels of both, whole K per workgroup
+    // two matrices of N / 2 channels, result SiLU(first) * second: whole K per workgroup
     BH_REQUIRE(!in.then_norm_w, "gemm_w8: no norm after the SiLU pair");
     BH_REQUIRE(in.N % (2 * kTileN) == 0 && !in.accumulate && !in.bias,
                "gemm_w8: the SiLU pair needs two matrices of a multiple of 16 channels, no "
                "bias, no accumulation");
     a.N = (int)(in.N / 2);
-    a.chunks_per_slice = a.chunks;
-    const int half_groups = a.groups / 2;
-    int best_gpw = 0, best_rb = 0;
-    double best_cost = 0;
-    for (int gpw : {5, 4})
-      for (int rb : {4, 3}) {
-        const int64_t ncols = ceil_div(half_groups, 2 * gpw), rows = ceil_div(in.M, 16 * rb);
-        const int64_t per_xcd = ceil_div(ncols, 8) * rows;
-        const double wg = 0.0125 * (double)(a.chunks * gpw * rb * in.digits) + 7.0;
-        const double cost = (double)ceil_div(per_xcd, 32) * wg;
-        if (!best_gpw || cost < best_cost - 1e-9) {
-          best_gpw = gpw;
-          best_rb = rb;
-          best_cost = cost;
-        }
-      }
-    a.ncols = (int)ceil_div(half_groups, 2 * best_gpw);
-    a.cols_padded = (int)round_up((int64_t)a.ncols, 8);
-    const int row_tiles = (int)ceil_div(in.M, 16 * best_rb);
-    return launch_shape<D, true>(best_rb, best_gpw, a, (unsigned)(a.cols_padded * row_tiles),
-                                 stream);
+    return launch_plan<D, true>(plan_tiles<D, true>(in.M, a.N, a.chunks, false, 0.0, 0), a, stream);
   }
-  // Three schemes, chosen by a model of their cost in microseconds (fitted to
-  // measurements at the Qwen2-1.5B shapes and M = 512):
-  //  * wide tiles, whole K per workgroup: the chip runs 256 workgroups at a time
-  //    (one wavefront per SIMD); a workgroup costs its matrix instructions
-  //    (12.5 ns each per SIMD, sustained) plus about 7 us of pipeline fill, drain
-  //    and stores; a launch costs rounds x that;
-  //  * wide tiles with K split over s workgroups: 2 us more per workgroup for the
-  //    partial sums, and the second kernel (3 us + its bytes at 3 TB/s);
-  //  * 64 x 64 tiles, K split over the wavefronts: bound by L2 -> CU traffic,
-  //    16 KiB per workgroup and chunk at about 6 TB/s.
   // A norm that is to follow (then_norm_w) costs a launch of its own, about
   // 5 us, unless the kernel that adds K slices writes its planes (it holds whole
   // rows, up to kRowCache columns).
   const double pending_norm = in.then_norm_w ? 5.0 : 0.0;
   const bool slices_fuse_norm = gemm_staging_layout(in.M, in.N).cols_padded <= kRowCache;
-  int best_gpw = 0, best_rb = 0, best_s = 0;
-  double best_cost = 0;
-  for (int gpw : {5, 4})
-    for (int rb : {4, 3}) {
-      const int64_t ncols = ceil_div(a.groups, gpw * kSlices), rows = ceil_div(in.M, 16 * rb);
-      for (int s = 1; s <= 16; ++s) {
-        // workgroups of the busiest XCD (32 CUs each): the (column tile, slice)
-        // pairs are dealt round robin, each with all its row tiles
-        const int64_t per_xcd = ceil_div(ncols * s, 8) * rows;
-        if (s > 1 && per_xcd > 32)
-          break;
-        const int64_t cps = ceil_div(a.chunks, s);
-        if (ceil_div(a.chunks, cps) != s)
-          continue; // the last slice would be empty
-        // (with the whole K in one workgroup a chunk of the pipelined loop takes
-        // 0.55 us however few matrix instructions it holds -- its barrier, staging
-        // and waits: 512 x 1536 x 2048 on two planes as 88 tiles of 48 x 256 took
-        // 19.4 us where 24 x 0.3 + 7 would be 14.2)
-        const double chunk_us =
-            std::max(0.0125 * (double)(gpw * rb * in.digits), s == 1 ? 0.55 : 0.0);
-        const double wg = chunk_us * (double)cps + 7.0 + (s > 1 ? 2.0 : 0.0);
-        double cost = (double)ceil_div(per_xcd, 32) * wg;
-        if (s > 1)
-          cost += 3.0 + 4.0 * (double)(ncols * rows * s) * (kSlices * rb * 16 * gpw * 16) / 3e6;
-        if (s == 1 || !slices_fuse_norm)
-          cost += pending_norm;
-        if (!best_gpw || cost < best_cost - 1e-9) {
-          best_gpw = gpw;
-          best_rb = rb;
-          best_s = s;
-          best_cost = cost;
-        }
-      }
-    }
   // the RMSNorm of the finished rows into digit planes, where the caller asked
   // for it and no kernel of the matmul holds whole rows
   auto then_norm = [&]() -> int {
@@ -1300,41 +1072,10 @@ int launch_gemm_w8_digits_d(const GemmW8Args &in, const void *planes, hipStream_
     return launch_rmsnorm_to_digits(in.C, in.ldc, in.then_norm_w, (int)in.M, (int)in.N,
                                     in.then_norm_eps, in.digits, in.then_norm_staged, stream);
   };
-  // The 64 x 64 kernel: two workgroups fit a compute unit, and a workgroup takes
-  // about 6 us for its first chunk per wavefront and 2 us for every further one
-  // (measured: 17.3 us for q|k|v, 18.6 us for o_proj at 512 rows, 72 us for
-  // down).  Neither it nor the unsplit wide kernel holds whole rows, so a norm
-  // that is to follow costs them a launch of its own.
-  const int64_t split_wgs = ceil_div(a.groups, kSplitGroups) * (a.Mp / 64);
-  const double split_cost =
-      1.0 + (double)ceil_div(split_wgs, 512) * (6.2 + 2.0 * (double)(ceil_div(a.chunks, kSlices) - 1)) +
-      pending_norm;
-  if (split_cost < best_cost) {
-    a.ncols = (int)ceil_div(a.groups, kSplitGroups);
-    a.cols_padded = (int)round_up(a.ncols, 8);
-    const unsigned blocks = (unsigned)(a.cols_padded * (a.Mp / 64));
-    if (int rc = launch_split<D>(a, blocks, stream))
-      return rc;
-    return then_norm();
-  }
-  a.ncols = (int)ceil_div(a.groups, best_gpw * kSlices);
-  a.cols_padded = (int)round_up((int64_t)a.ncols * best_s, 8);
-  const int row_tiles = (int)ceil_div(in.M, 16 * best_rb);
-  a.slices = best_s;
-  a.chunks_per_slice = (int)ceil_div(a.chunks, best_s);
-  if (best_s > 1) {
-    const size_t tile_floats = (size_t)kSlices * best_rb * 16 * best_gpw * 16;
-    const size_t bytes = sizeof(float) * tile_floats * best_s * (size_t)a.ncols * row_tiles;
-    char *ws = nullptr;
-    if (int rc = workspace_for(stream, bytes, &ws))
-      return rc;
-    a.partial = reinterpret_cast<float *>(ws);
-  }
-  const unsigned blocks = (unsigned)(a.cols_padded * row_tiles);
-  int rc = launch_shape<D>(best_rb, best_gpw, a, blocks, stream);
-  if (rc)
+  const TilePlan plan = plan_tiles<D, false>(in.M, in.N, a.chunks, true, pending_norm, 0);
+  if (int rc = launch_plan<D, false>(plan, a, stream))
     return rc;
-  if (best_s == 1)
+  if (plan.slices == 1)
     return then_norm();
   const GemmStagingLayout next = gemm_staging_layout(in.M, in.N);
   if (in.then_norm_w && slices_fuse_norm) {
@@ -1347,8 +1088,8 @@ int launch_gemm_w8_digits_d(const GemmW8Args &in, const void *planes, hipStream_
                                   (int)(2 * sizeof(float) * kRowCache)));
     }
     hipLaunchKernelGGL(reduce_slices_norm_kernel, dim3((unsigned)a.M), dim3(kRowThreads),
-                       row_lds, stream, a.partial, a.steps, a.N, a.ncols, a.slices, best_rb,
-                       best_gpw, a, in.then_norm_w, 1.0f / (float)in.N, in.then_norm_eps,
+                       row_lds, stream, a.partial, a.steps, a.N, a.ncols, a.slices, a.span,
+                       a.tile_rows, a, in.then_norm_w, 1.0f / (float)in.N, in.then_norm_eps,
                        in.digits, next.rows_padded, next.cols_padded,
                        static_cast<int8_t *>(in.then_norm_staged));
     BH_CHECK_HIP(hipGetLastError());
@@ -1356,7 +1097,7 @@ int launch_gemm_w8_digits_d(const GemmW8Args &in, const void *planes, hipStream_
   }
   const int64_t threads = (int64_t)a.M * ((a.N + 3) / 4);
   hipLaunchKernelGGL(reduce_slices_kernel, dim3((unsigned)ceil_div(threads, 256)), dim3(256), 0,
-                     stream, a, best_rb, best_gpw);
+                     stream, a);
   BH_CHECK_HIP(hipGetLastError());
   return then_norm();
 }
@@ -1398,52 +1139,14 @@ int launch_gemm_w8a8_plane(const void *plane, const int8_t *W, const float *wsca
   // the cost model of the digit-plane launch with one plane; K slices leave int32
   // sums in the workspace (f32 ones would round above 2^24) and a second kernel
   // adds them exactly
-  int best_gpw = 0, best_rb = 0, best_s = 0;
-  double best_cost = 0;
   const int64_t reduce_wgs = ceil_div(M * ceil_div(N, 4), 256);
-  for (int gpw : {5, 4})
-    for (int rb : {4, 3}) {
-      const int64_t ncols = ceil_div(a.groups, gpw * kSlices), rows = ceil_div(M, 16 * rb);
-      for (int s = 1; s <= 16; ++s) {
-        const int64_t per_xcd = ceil_div(ncols * s, 8) * rows;
-        if (s > 1 && per_xcd > 32)
-          break;
-        const int64_t cps = ceil_div(a.chunks, s);
-        if (ceil_div(a.chunks, cps) != s)
-          continue; // the last slice would be empty
-        const double chunk_us = std::max(0.0125 * (double)(gpw * rb), s == 1 ? 0.55 : 0.0);
-        const double wg = chunk_us * (double)cps + 7.0 + (s > 1 ? 2.0 : 0.0);
-        double cost = (double)ceil_div(per_xcd, 32) * wg;
-        if (s > 1)
-          cost += 3.0 + 4.0 * (double)(ncols * rows * s) * (kSlices * rb * 16 * gpw * 16) / 3e6 +
-                  0.002 * (double)reduce_wgs;
-        if (!best_gpw || cost < best_cost - 1e-9) {
-          best_gpw = gpw;
-          best_rb = rb;
-          best_s = s;
-          best_cost = cost;
-        }
-      }
-    }
-  a.ncols = (int)ceil_div(a.groups, best_gpw * kSlices);
-  a.cols_padded = (int)round_up((int64_t)a.ncols * best_s, 8);
-  const int row_tiles = (int)ceil_div(M, 16 * best_rb);
-  a.slices = best_s;
-  a.chunks_per_slice = (int)ceil_div(a.chunks, best_s);
-  if (best_s > 1) {
-    const size_t tile_floats = (size_t)kSlices * best_rb * 16 * best_gpw * 16;
-    const size_t bytes = sizeof(float) * tile_floats * best_s * (size_t)a.ncols * row_tiles;
-    char *ws = nullptr;
-    if (int rc = workspace_for(stream, bytes, &ws))
-      return rc;
-    a.partial = reinterpret_cast<float *>(ws);
-    a.int_partials = 1;
-  }
-  if (int rc = launch_shape<1>(best_rb, best_gpw, a, (unsigned)(a.cols_padded * row_tiles), stream))
+  const TilePlan plan = plan_tiles<1, false>(M, N, a.chunks, true, 0.0, reduce_wgs);
+  a.int_partials = plan.slices > 1;
+  if (int rc = launch_plan<1, false>(plan, a, stream))
     return rc;
-  if (best_s > 1) {
-    hipLaunchKernelGGL(reduce_slices_i32_kernel, dim3((unsigned)reduce_wgs), dim3(256), 0, stream, a,
-                       best_rb, best_gpw);
+  if (plan.slices > 1) {
+    hipLaunchKernelGGL(reduce_slices_i32_kernel, dim3((unsigned)reduce_wgs), dim3(256), 0, stream,
+                       a);
     BH_CHECK_HIP(hipGetLastError());
   }
   return BUDDY_HIP_OK;

@@ -246,6 +246,35 @@ def test_every_int8_prefill_matmul_variant(bh, oracle):
         assert launched(bh, fam) == compiled(bh, fam), compiled(bh, fam) - launched(bh, fam)
 
 
+@pytest.mark.parametrize("M,K,N", [
+    (17, 64, 1), (31, 65, 127),       # less than a tile of rows, of channels; one and two chunks
+    (32, 128, 128), (33, 192, 129),   # a tile, and one row and one channel more
+    (64, 257, 255), (65, 320, 257),   # the same of the 256-channel tile, five chunks
+    (100, 1000, 31), (17, 5000, 48),  # K over several workgroups, the last with fewer chunks
+    (97, 8960, 513), (300, 4100, 1100)])
+def test_int8_matmul_tile_edges(bh, oracle, M, K, N):
+    """Digit planes and exact integer sums: against the sums in 64 bits."""
+    w8a8_case(bh, oracle, M, K, N)  # bit for bit
+    q, s = synthetic.quantized_linear(K, N, M + K + N)
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn((M, K), generator=g, device="cuda")
+    c0 = torch.randn((M, N), generator=g, device="cuda")
+    qh, sh = q.cpu().numpy().astype(np.float64), s.cpu().numpy().astype(np.float64)
+    for digits in (3, 2):
+        rounded, step = fixed_point_round(x.cpu().numpy(), digits=digits)
+        # Each plane's sum is rounded once (2^-24 of it), as is every step that joins
+        # planes, slices (up to 16), scales and the old values: 24 roundings of at most
+        # the sum of |digit| 256^j |q|, and the digits of X below the last sum to < 2^16.
+        size = (np.abs(rounded) + step * 2.0**16) @ np.abs(qh) * sh + np.abs(c0.cpu().numpy())
+        want = rounded.astype(np.float64) @ qh * sh
+        packed = ops.pack_w8(q)
+        got = ops.gemm_w8a32(x, packed, s, K, N, digits=digits)
+        more = c0.clone()
+        ops.gemm_w8a32(x, packed, s, K, N, out=more, accumulate=True, digits=digits)
+        for have, expect in ((got, want), (more, want + c0.cpu().numpy())):
+            assert (np.abs(have.cpu().numpy() - expect) <= 24 * 2.0**-24 * size).all()
+
+
 def test_every_bf16_prefill_matmul_variant(bh, oracle):
     bh.buddy_hip_variant_reset()
     for M, K, N in GEMM_BF16_SHAPES:
