@@ -341,7 +341,6 @@ struct Qwen2Session : Session {
     BH_CHECK_HIP(hipMalloc((void **)&pf_xn_bf, std::max(lx.bytes(3), lx.bytes_digits(3))));
     BH_CHECK_HIP(hipMalloc((void **)&pf_g_bf, std::max(lg.bytes(3), lg.bytes_digits(3))));
     BH_CHECK_HIP(hipMalloc((void **)&pf_att_dg, gemm_staging_layout(rows, QN).bytes_digits(3)));
-    BH_CHECK_HIP(hipMalloc(&pf_attn_ws, attn_prompt_workspace_bytes(rows, S.heads, S.kv_heads)));
     pf_rows = rows;
     return BUDDY_HIP_OK;
   }
@@ -416,6 +415,9 @@ struct Qwen2Session : Session {
                        pf_tokens, (int64_t)S.hidden, (int64_t)S.vocab, pf_x);
     BH_CHECK_HIP(hipGetLastError());
     int rc;
+    const bool folded = attn_prompt_pays(n, start_pos);
+    if (folded && !pf_attn_ws) // for as many rows as the other buffers have
+      BH_CHECK_HIP(hipMalloc(&pf_attn_ws, attn_prompt_workspace_bytes(pf_rows, S.heads, S.kv_heads)));
     bool normed_ahead = false; // pf_xn_bf already holds this layer's normed input
     for (int i = 0; i < S.layers; ++i) {
       Layer &L = layers[(size_t)i];
@@ -457,7 +459,6 @@ struct Qwen2Session : Session {
       a.k_len = start_pos + n;
       a.scale = scale;
       PromptFold fold;
-      const bool folded = attn_prompt_pays(n, start_pos);
       if ((rc = folded ? launch_attn_prompt(a, pf_attn_ws, fold, stream) : launch_attn_prefill(a, stream)))
         return rc;
       if (gemm_digits) {
