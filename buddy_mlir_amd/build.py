@@ -46,8 +46,9 @@ COMMON = [
 # load is issued: if it spilled one of those registers it would store garbage
 # and hand the register to something else while the load is still in flight.
 # Their kernels must therefore use no scratch at all; the build checks it.
-# (gemm_w8_i8.hip leaves the waiting to the compiler; there a spilled register's
-# reload would wait for every load in flight, which is what its rings avoid.)
+# (gemm_w8_i8.hip and gemm_w8_mfma.hip leave the waiting to the compiler; there a
+# spilled register's reload would wait for every load in flight, which is what
+# their rings avoid.)
 NO_SCRATCH = {"gemm_w8_mfma.hip", "gemv_w8a32_mfma.hip", "gemv_w8a32_i8.hip", "gemm_w8_i8.hip",
               "attn_prefill.hip"}
 

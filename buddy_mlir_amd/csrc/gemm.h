@@ -80,7 +80,9 @@ int launch_gemm_w8a8_plane(const void *plane, const int8_t *W, const float *wsca
                            int32_t *sums, int64_t M, int64_t K, int64_t N,
                            hipStream_t stream);
 
-// split-K workspace of the int8 matmul (dropped together with the staging)
+// split-K workspace of the int8 and bf16 matmuls, one grow-only buffer per stream (dropped
+// together with the staging)
+int gemm_slices_workspace(hipStream_t stream, size_t bytes, char **out);
 void release_gemm_i8_workspace(hipStream_t stream);
 
 // The matmul keeps a bf16 copy of its activations in a grow-only device buffer

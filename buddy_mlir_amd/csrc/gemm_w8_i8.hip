@@ -901,7 +901,9 @@ struct Workspace {
 std::mutex g_workspace_mutex;
 std::map<hipStream_t, Workspace> g_workspace;
 
-int workspace_for(hipStream_t stream, size_t bytes, char **out) {
+} // namespace
+
+int gemm_slices_workspace(hipStream_t stream, size_t bytes, char **out) {
   std::lock_guard<std::mutex> lock(g_workspace_mutex);
   Workspace &w = g_workspace[stream];
   if (w.bytes < bytes) {
@@ -917,6 +919,8 @@ int workspace_for(hipStream_t stream, size_t bytes, char **out) {
   *out = w.ptr;
   return BUDDY_HIP_OK;
 }
+
+namespace {
 
 // Channel tiles per wavefront, K slices and bands of rows for a launch, by an estimate of
 // its time in microseconds.  An XCD (32 compute units) works on 64 workgroups at a time, two
@@ -1000,7 +1004,7 @@ int launch_plan(const TilePlan &plan, GemmI8Args &a, hipStream_t stream) {
     const size_t tile_floats = (size_t)a.tile_rows * kSlices * a.span;
     const size_t bytes = sizeof(float) * tile_floats * plan.slices * (size_t)a.ncols * a.row_tiles;
     char *ws = nullptr;
-    if (int rc = workspace_for(stream, bytes, &ws))
+    if (int rc = gemm_slices_workspace(stream, bytes, &ws))
       return rc;
     a.partial = reinterpret_cast<float *>(ws);
   }

@@ -7,19 +7,17 @@
 //
 // Shape of the kernel:
 //  * the weights are read from the same wave-tile packed copy the decode GEMV
-//    streams (one resident copy serves prefill and decode).  A lane's 16 bytes
-//    of a 16 x 64 tile are, as they lie, two 8-wide operand fragments of
-//    v_mfma_f32_16x16x32_bf16 (rows = the tile's 16 channels): they go from
-//    global memory to registers, are converted to bf16 (|q| <= 128 is exact)
-//    and fed to the matrix core.  No LDS on the way;
+//    streams (one resident copy serves prefill and decode).  A lane takes the runs of 16
+//    k of one channel that make up its operands of v_mfma_f32_32x32x16_bf16 (32 channels
+//    = two tiles): they go from global memory to registers, are converted to bf16
+//    (|q| <= 128 is exact) and fed to the matrix core.  No LDS on the way;
 //  * the activations are converted once per call to bf16 terms (one term =
 //    "activations cast to bf16"; three terms carry all 24 significand bits of
-//    the f32 input) in a [term][row][k] buffer.  A lane's fragment of the other
-//    operand (columns = 16 activation rows) is 32 contiguous bytes of that
-//    buffer, so it is loaded straight from L2 as well;
-//  * a wavefront owns 64 rows x 64 channels of C (4 x 4 accumulators); the four
-//    wavefronts of a workgroup split K and meet in LDS, in slice order;
-//  * workgroup ids are laid out so that the row blocks of one column tile run
+//    the f32 input) in a [term][row][k] buffer, whose rows the wavefronts of a
+//    workgroup share through LDS;
+//  * workgroups take 32 or 64 rows x 128 or 256 channels, and K is split over
+//    several of them where a matrix is too narrow to fill the chip;
+//  * workgroup ids are laid out so that the row tiles of one column tile run
 //    on the same XCD (ids equal modulo 8) and share the weight tiles in its L2;
 //  * the per-channel scale is applied once to the f32 accumulators, where the
 //    reference multiplies every element before the FMA.
@@ -32,13 +30,12 @@
 namespace bh {
 namespace {
 
-constexpr int kRowsPerWave = 64;   // 4 row blocks of 16
-constexpr int kGroupsPerWave = 4;  // 4 channel groups of 16
-constexpr int kSlices = 4;         // k-slices = wavefronts per workgroup
+constexpr int kWaves = 4; // wavefronts per workgroup
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned short u16;
+typedef int v4i32 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ u16 bf16_rne(float x) {
   unsigned u = __float_as_uint(x);
@@ -55,7 +52,7 @@ __device__ __forceinline__ unsigned pack2(u16 lo, u16 hi) {
 __device__ __forceinline__ unsigned q2_to_bf16x2(int v, int j) {
   const float a = (float)(signed char)(v >> (8 * j));
   const float b = (float)(signed char)(v >> (8 * j + 8));
-  return (__float_as_uint(a) >> 16) | (__float_as_uint(b) & 0xffff0000u);
+  return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
 }
 __device__ __forceinline__ bf16x8 frag_from(int lo, int hi) {
   union {
@@ -66,15 +63,6 @@ __device__ __forceinline__ bf16x8 frag_from(int lo, int hi) {
                    q2_to_bf16x2(hi, 2));
   return x.v;
 }
-__device__ __forceinline__ bf16x8 as_frag(const uint4 &u) {
-  union {
-    uint4 u;
-    bf16x8 v;
-  } x;
-  x.u = u;
-  return x.v;
-}
-
 // A[M, K] f32 -> terms x [Mp, Kp] bf16, zero padded; term t holds the bf16
 // rounding of what the terms before it left over.
 __global__ void __launch_bounds__(256)
@@ -185,333 +173,302 @@ struct GemmArgs {
   float *C;
   int64_t ldc;
   int M, N, Mp, Kp, groups, chunks;
-  int ncols, cols_padded; // column tiles of 64 channels; padded to the XCD count
+  int ncols; // column tiles
+  // K split over `slices` workgroups per tile, chunks_per_slice chunks of 64 each (the last
+  // may hold fewer, never none)
+  int slices, chunks_per_slice;
+  int ids_padded, row_tiles; // ids per row tile: ncols x slices, padded to the XCD count
+  float *partial;            // [tile][slice][wavefront][row][channel], where K is split
+  int span, tile_rows;       // channels per wavefront, rows per workgroup
   int accumulate;
 };
 
-template <int TERMS> struct ChunkOperands {
-  int4 w[kGroupsPerWave];
-  uint4 a[TERMS][4][2]; // [term][row block][k half]
-};
-
-template <int TERMS>
-__device__ __forceinline__ void load_chunk(const int4 *const (&wp)[kGroupsPerWave],
-                                           const u16 *ap, size_t term_stride,
-                                           size_t rb_stride, int c,
-                                           ChunkOperands<TERMS> &o) {
-#pragma unroll
-  for (int g = 0; g < kGroupsPerWave; ++g)
-    o.w[g] = wp[g][(size_t)c * 64];
-#pragma unroll
-  for (int t = 0; t < TERMS; ++t)
-#pragma unroll
-    for (int rb = 0; rb < 4; ++rb) {
-      const uint4 *src = reinterpret_cast<const uint4 *>(
-          ap + t * term_stride + rb * rb_stride + (size_t)c * kTileK);
-      o.a[t][rb][0] = src[0];
-      o.a[t][rb][1] = src[1];
-    }
-}
-
-template <int TERMS>
-__global__ void __launch_bounds__(kSlices *kWave) gemm_w8_bf16_kernel(GemmArgs a) {
-  extern __shared__ __attribute__((aligned(16))) float red[]; // [slice][64][lane]
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int col = blockIdx.x % a.cols_padded, rbk = blockIdx.x / a.cols_padded;
-  if (col >= a.ncols)
-    return; // padding id
-  const int m0 = rbk * kRowsPerWave, g0 = col * kGroupsPerWave;
-  const int per = (a.chunks + kSlices - 1) / kSlices;
-  const int c0 = min(wave * per, a.chunks), c1 = min(c0 + per, a.chunks);
-
-  f32x4 acc[kGroupsPerWave][4];
-#pragma unroll
-  for (int g = 0; g < kGroupsPerWave; ++g)
-#pragma unroll
-    for (int rb = 0; rb < 4; ++rb)
-      acc[g][rb] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const int4 *wp[kGroupsPerWave];
-#pragma unroll
-  for (int g = 0; g < kGroupsPerWave; ++g) // groups past the end repeat the last one
-    wp[g] = a.W + ((size_t)min(g0 + g, a.groups - 1) * a.chunks) * 64 + lane;
-  const size_t term_stride = (size_t)a.Mp * a.Kp, rb_stride = (size_t)16 * a.Kp;
-  const u16 *ap = a.Abf + (size_t)(m0 + (lane & 15)) * a.Kp + (lane >> 4) * 16;
-
-  ChunkOperands<TERMS> cur, nxt;
-  if (c0 < c1)
-    load_chunk<TERMS>(wp, ap, term_stride, rb_stride, c0, cur);
-  for (int c = c0; c < c1; ++c) {
-    if (c + 1 < c1)
-      load_chunk<TERMS>(wp, ap, term_stride, rb_stride, c + 1, nxt);
-#pragma unroll
-    for (int g = 0; g < kGroupsPerWave; ++g) {
-      const bf16x8 w0 = frag_from(cur.w[g].x, cur.w[g].y);
-      const bf16x8 w1 = frag_from(cur.w[g].z, cur.w[g].w);
-#pragma unroll
-      for (int t = 0; t < TERMS; ++t)
-#pragma unroll
-        for (int rb = 0; rb < 4; ++rb) {
-          acc[g][rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              w0, as_frag(cur.a[t][rb][0]), acc[g][rb], 0, 0, 0);
-          acc[g][rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              w1, as_frag(cur.a[t][rb][1]), acc[g][rb], 0, 0, 0);
-        }
-    }
-    if (c + 1 < c1)
-      cur = nxt;
-  }
-
-  // ---- the k-slices meet in LDS; wavefront w finishes channel group w ------
-  float *mine = red + (size_t)wave * 64 * kWave;
-#pragma unroll
-  for (int g = 0; g < kGroupsPerWave; ++g)
-#pragma unroll
-    for (int rb = 0; rb < 4; ++rb)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        mine[((g * 4 + rb) * 4 + r) * kWave + lane] = acc[g][rb][r];
-  __syncthreads();
-  const int g = wave;
-  if (g0 + g >= a.groups)
-    return;
-  // lane holds channels n..n+3 of row m for each row block
-  const int n = (g0 + g) * kTileN + (lane >> 4) * 4;
-  float s[4], b[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    s[r] = n + r < a.N ? a.scale[n + r] : 0.f;
-    b[r] = (a.bias && n + r < a.N) ? a.bias[n + r] : 0.f;
-  }
-  const bool vec = n + 3 < a.N && (a.ldc & 3) == 0 &&
-                   (reinterpret_cast<uintptr_t>(a.C) & 15) == 0;
-#pragma unroll
-  for (int rb = 0; rb < 4; ++rb) {
-    const int m = m0 + rb * 16 + (lane & 15);
-    float v[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float sum = 0.f;
-#pragma unroll
-      for (int sl = 0; sl < kSlices; ++sl)
-        sum += red[((size_t)sl * 64 + (g * 4 + rb) * 4 + r) * kWave + lane];
-      v[r] = sum * s[r];
-    }
-    if (m >= a.M)
-      continue;
-    float *c = a.C + (int64_t)m * a.ldc + n;
-    if (vec) {
-      float4 o = make_float4(v[0], v[1], v[2], v[3]);
-      if (a.accumulate) {
-        const float4 p = *reinterpret_cast<const float4 *>(c);
-        o = make_float4(p.x + o.x, p.y + o.y, p.z + o.z, p.w + o.w);
-      } else {
-        o = make_float4(b[0] + o.x, b[1] + o.y, b[2] + o.z, b[3] + o.w);
-      }
-      *reinterpret_cast<float4 *>(c) = o;
-    } else {
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (n + r < a.N)
-          c[r] = a.accumulate ? c[r] + v[r] : b[r] + v[r];
-    }
-  }
-}
-
-// Wide matrices (enough column tiles to fill the chip without splitting K):
-// a workgroup owns 64 rows x 256 channels, one 64-channel span per wavefront,
-// every wavefront runs the whole K.  The activation fragments of a chunk are the
-// same for the four wavefronts: wavefront w fetches row block w for everyone
-// and leaves it in LDS in fragment order (lane l of fragment f at f*1 KiB +
-// 16 l: conflict-free by construction), so the fragments cross L2 -> CU once per
-// workgroup.  Weights stay on the register path.
+// A tile of 32 RB rows x 128 GP channels, on v_mfma_f32_32x32x16_bf16 (GP tiles of 32 channels per wavefront); every
+// wavefront runs the workgroup's whole share of K.  What bounds it: 1931 rows of 1536 -> 17920
+// run at 0.84 PFLOP/s, half of what the instruction alone reaches, with the conversion of the
+// weights and the way of the rows through LDS in the wavefronts' stream of instructions.
 //
-// Global loads run kRing - 2 chunks ahead of the matrix cores.  The compiler
-// sinks ordinary loads down to their first use (and then waits for them there),
-// so the loads of this loop are issued by hand and waited for by hand: a fetch
-// is kFetchLoads loads in a fixed order, vmcnt counts them in order, and each
-// wait names the registers it releases so that nothing reads them earlier.
-constexpr int kRing = 5;
+// Rows go through LDS, weights from memory to registers.  Weights are asked for three
+// chunks of 64 k ahead, rows five (two of them in LDS: step c multiplies buffer c % 3, whose
+// first fragments were read during step c - 1, and fills buffer (c + 2) % 3, last read before
+// the previous barrier).  The weights of a quarter of a chunk are converted while the
+// quarter before it is multiplied.
+constexpr int kRing = 4;               // chunks in registers
+constexpr int kRowBytes = 2 * kTileK + 16; // of a row in LDS: reads meet every bank once
 
-typedef int v4i32 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ void issue_load(v4i32 &dst, const void *p) {
-  asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(dst) : "v"(p) : "memory");
-}
-template <int TERMS> struct FetchRegs {
-  v4i32 w[kGroupsPerWave];
-  v4i32 a[TERMS][2];
-};
-// Waits until at most N loads are in flight; the registers of `f` are only
-// valid after it.
-template <int N, int TERMS> __device__ __forceinline__ void wait_loads(FetchRegs<TERMS> &f) {
-  static_assert(kGroupsPerWave == 4, "operand list below");
-  asm volatile("s_waitcnt vmcnt(%4)"
-               : "+v"(f.w[0]), "+v"(f.w[1]), "+v"(f.w[2]), "+v"(f.w[3])
-               : "n"(N)
-               : "memory");
-#pragma unroll
-  for (int t = 0; t < TERMS; ++t)
-    asm volatile("" : "+v"(f.a[t][0]), "+v"(f.a[t][1])::"memory");
-}
-__device__ __forceinline__ bf16x8 frag_from_v(int lo, int hi) { return frag_from(lo, hi); }
-
-// RB = row blocks of 16 per workgroup (4 or 3: whichever leaves the shorter last
-// round of workgroups on the chip).
-template <int TERMS, int RB>
-__global__ void __launch_bounds__(kSlices *kWave) gemm_w8_bf16_wide_kernel(GemmArgs a) {
-  constexpr int L = kGroupsPerWave + 2 * TERMS; // loads per fetch
-  extern __shared__ __attribute__((aligned(16))) v4i32 frag_s[]; // [2][TERMS][2 RB][64]
-  const int tid = threadIdx.x, lane = tid & 63;
+template <int TERMS, int RB, int GP>
+__device__ __forceinline__ void multiply_tile(const GemmArgs &a) {
+  constexpr int L = TERMS * RB; // layers of 32 rows: term l % TERMS of row block l / TERMS
+  constexpr int kRows = 32 * RB, kSpan = 32 * GP, kThreads = kWaves * kWave;
+  constexpr int kBuf = L * 32 * kRowBytes;
+  constexpr int kTurn = kSpan + 4; // floats of a row of the epilogue's tile
+  constexpr int kTurned = kWaves * 32 * kTurn * 4;
+  constexpr int kLds = 3 * kBuf > kTurned ? 3 * kBuf : kTurned;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[kLds];
+  __shared__ __attribute__((aligned(16))) float scale_s[kWaves * kSpan], bias_s[kWaves * kSpan];
+  const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, up = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int col = blockIdx.x % a.cols_padded, rbk = blockIdx.x / a.cols_padded;
-  if (col >= a.ncols)
+  // ids equal modulo 8 run on the same XCD: the row tiles of one (column tile, K slice) do,
+  // and share its weights in that XCD's L2
+  const int unit = blockIdx.x % a.ids_padded, rbk = blockIdx.x / a.ids_padded;
+  if (unit >= a.ncols * a.slices)
     return; // padding id
-  const int m0 = rbk * RB * 16;
-  const int g0 = (col * kSlices + wave) * kGroupsPerWave;
+  const int ctile = unit % a.ncols, slice = unit / a.ncols;
+  const int m0 = rbk * kRows;
+  const int g0 = (ctile * kWaves + wave) * (kSpan / 16); // first channel group of this wavefront
+  const int cb = slice * a.chunks_per_slice;
+  const int nch = min(a.chunks_per_slice, a.chunks - cb); // chunks of this slice, >= 1
 
-  f32x4 acc[kGroupsPerWave][RB];
+  const v4i32 *wp[GP];
 #pragma unroll
-  for (int g = 0; g < kGroupsPerWave; ++g)
+  for (int g = 0; g < GP; ++g) { // groups past the end repeat the last one
+    const int gg = min(g0 + 2 * g + ((lane >> 4) & 1), a.groups - 1);
+    wp[g] = reinterpret_cast<const v4i32 *>(a.W) + ((size_t)gg * a.chunks + cb) * 64 + up * 16 +
+            (lane & 15);
+  }
+  const u16 *src[L];
+#pragma unroll
+  for (int l = 0; l < L; ++l) // 8 threads per row, 32 rows per layer
+    src[l] = a.Abf +
+             ((size_t)(l % TERMS) * a.Mp + min(m0 + l / TERMS * 32 + tid / 8, a.Mp - 1)) * a.Kp +
+             (size_t)cb * kTileK + (tid & 7) * 8;
+  const int lds_at = tid / 8 * kRowBytes + (tid & 7) * 16;
+  v4i32 wr[kRing][GP * 2], xr[kRing][L];
+  auto fetch_w = [&](int c, v4i32 (&w)[GP * 2]) {
+    const size_t cc = (size_t)min(c, nch - 1) * 64;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int g = 0; g < GP; ++g)
+        w[g * 2 + h] = wp[g][cc + h * 32];
+  };
+  auto fetch_x = [&](int c, v4i32 (&x)[L]) {
+    const size_t cc = (size_t)min(c, nch - 1) * kTileK;
+#pragma unroll
+    for (int l = 0; l < L; ++l)
+      x[l] = *reinterpret_cast<const v4i32 *>(src[l] + cc);
+  };
+  auto put_x = [&](const v4i32 (&x)[L], unsigned char *buf) {
+#pragma unroll
+    for (int l = 0; l < L; ++l)
+      *reinterpret_cast<v4i32 *>(buf + l * 32 * kRowBytes + lds_at) = x[l];
+  };
+  // quarter t of a chunk: 8 of the 16 k of run t / 2
+  auto convert = [&](const v4i32 (&w)[GP * 2], int t, int g) {
+    const v4i32 &q = w[g * 2 + t / 2];
+    return t % 2 == 0 ? frag_from(q[0], q[1]) : frag_from(q[2], q[3]);
+  };
+  fetch_x(0, xr[0]);
+  fetch_x(1, xr[1]);
+#pragma unroll
+  for (int u = 0; u < kRing - 1; ++u) {
+    fetch_w(u, wr[u]);
+    if (u + 2 < kRing)
+      fetch_x(u + 2, xr[u + 2]);
+  }
+  if (a.slices == 1)
+    for (int i = tid; i < kWaves * kSpan; i += kThreads) {
+      const int n = ctile * kWaves * kSpan + i;
+      scale_s[i] = n < a.N ? a.scale[n] : 0.f;
+      bias_s[i] = a.bias && n < a.N ? a.bias[n] : 0.f;
+    }
+
+  f32x16 acc[GP][RB];
+#pragma unroll
+  for (int g = 0; g < GP; ++g)
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
-      acc[g][rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+      acc[g][rb] = f32x16{};
 
-  const int4 *wp[kGroupsPerWave];
-#pragma unroll
-  for (int g = 0; g < kGroupsPerWave; ++g) // groups past the end repeat the last one
-    wp[g] = a.W + ((size_t)min(g0 + g, a.groups - 1) * a.chunks) * 64 + lane;
-  const size_t term_stride = (size_t)a.Mp * a.Kp;
-  // this wavefront fetches row block `wave` of the activation tile (with three
-  // row blocks the fourth wavefront repeats the third's loads and stages nothing)
-  const int my_rb = min(wave, RB - 1);
-  const u16 *ap = a.Abf + (size_t)(m0 + my_rb * 16 + (lane & 15)) * a.Kp + (lane >> 4) * 16;
-
-  FetchRegs<TERMS> ring[kRing];
-  // chunks past the end are fetched again from the last chunk (never used):
-  // every fetch is exactly L loads, which is what keeps the counts below exact
-  auto fetch = [&](int c, FetchRegs<TERMS> &f) {
-    const int cc = min(c, a.chunks - 1);
-#pragma unroll
-    for (int g = 0; g < kGroupsPerWave; ++g)
-      issue_load(f.w[g], wp[g] + (size_t)cc * 64);
-#pragma unroll
-    for (int t = 0; t < TERMS; ++t) {
-      const u16 *src = ap + t * term_stride + (size_t)cc * kTileK;
-      issue_load(f.a[t][0], src);
-      issue_load(f.a[t][1], src + 8);
-    }
-  };
-  auto stage = [&](const FetchRegs<TERMS> &f, int buf) { // own row block -> LDS
-    if (wave >= RB)
-      return;
-#pragma unroll
-    for (int t = 0; t < TERMS; ++t) {
-      v4i32 *dst = frag_s + (((size_t)buf * TERMS + t) * 2 * RB + wave * 2) * kWave + lane;
-      dst[0] = f.a[t][0];
-      dst[kWave] = f.a[t][1];
-    }
-  };
-#pragma unroll
-  for (int u = 0; u < kRing; ++u)
-    fetch(u, ring[u]);
-  wait_loads<(kRing - 1) * L, TERMS>(ring[0]); // chunk 0 has arrived
-  stage(ring[0], 0);
+  unsigned char *cur = lds, *next = lds + kBuf, *fill = lds + 2 * kBuf;
+  put_x(xr[0], cur);
+  put_x(xr[1], next);
+  fetch_x(kRing, xr[0]);
   __syncthreads();
-  for (int c0 = 0; c0 < a.chunks; c0 += kRing) {
+  v4i32 frag[4];
+  bf16x8 wf[2][GP];
+  // sub-step u of a chunk: layer u % L, quarter u / L
+  auto load_frag = [&](const unsigned char *buf, int u, v4i32 &f) {
+    f = *reinterpret_cast<const v4i32 *>(buf + col * kRowBytes + up * 32 +
+                                         u % L * 32 * kRowBytes + u / L / 2 * 64 + u / L % 2 * 16);
+  };
+  load_frag(cur, 0, frag[0]);
+  load_frag(cur, 1, frag[1]);
 #pragma unroll
-    for (int u = 0; u < kRing; ++u) {
-      const int c = c0 + u;
-      if (c < a.chunks) {
-        const int buf = c & 1;
-        FetchRegs<TERMS> &cur = ring[u];
-        FetchRegs<TERMS> &nxt = ring[(u + 1) % kRing];
-        // in flight: chunks c+1 .. c+kRing-1 (chunk c was waited for when it was
-        // staged).  Release chunk c+1 and put its row block into the other
-        // buffer, whose readers passed the barrier that closed chunk c-1.
-        wait_loads<(kRing - 2) * L, TERMS>(nxt);
-        stage(nxt, buf ^ 1);
-        bf16x8 wf[kGroupsPerWave][2];
+  for (int g = 0; g < GP; ++g)
+    wf[0][g] = convert(wr[0], 0, g);
+  auto step = [&](int c, const v4i32 (&w)[GP * 2], const v4i32 (&w_next)[GP * 2],
+                  v4i32 (&w_new)[GP * 2], v4i32 (&x)[L], v4i32 (&x_new)[L]) {
 #pragma unroll
-        for (int g = 0; g < kGroupsPerWave; ++g) {
-          wf[g][0] = frag_from(cur.w[g].x, cur.w[g].y);
-          wf[g][1] = frag_from(cur.w[g].z, cur.w[g].w);
-        }
+    for (int u = 0; u < 4 * L; ++u) {
+      const int t = u / L, l = u % L;
+      // fragments are asked for two sub-steps ahead of their products (one takes less than
+      // the way through LDS), and stay there: left to itself the scheduler moves them to
+      // their use
+      load_frag(u + 2 < 4 * L ? cur : next, (u + 2) % (4 * L), frag[(u + 2) & 3]);
+      if (u == 0)
+        fetch_w(c + kRing - 1, w_new);
+      if (u == 1)
+        put_x(x, fill);
+      if (u == 2)
+        fetch_x(c + kRing + 1, x_new);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int t = 0; t < TERMS; ++t)
-#pragma unroll
-          for (int rb = 0; rb < RB; ++rb) {
-            const v4i32 *src = frag_s + (((size_t)buf * TERMS + t) * 2 * RB + rb * 2) * kWave + lane;
-            union {
-              v4i32 i;
-              bf16x8 v;
-            } a0, a1;
-            a0.i = src[0];
-            a1.i = src[kWave];
-#pragma unroll
-            for (int g = 0; g < kGroupsPerWave; ++g) {
-              acc[g][rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[g][0], a0.v, acc[g][rb], 0, 0, 0);
-              acc[g][rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[g][1], a1.v, acc[g][rb], 0, 0, 0);
-            }
-          }
-        // the registers of chunk c are free: fetch the chunk kRing further on
-        // (its weights were converted above; wf holds them now)
-        fetch(c + kRing, cur);
-        __syncthreads();
+      for (int g = 0; g < GP; ++g) {
+        union {
+          v4i32 i;
+          bf16x8 v;
+        } f;
+        f.i = frag[u & 3];
+        acc[g][l / TERMS] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[t & 1][g], f.v,
+                                                                    acc[g][l / TERMS], 0, 0, 0);
+        // behind a product that takes 32 cycles: a piece of the next quarter's weights
+        if (g % L == l)
+          wf[(t + 1) & 1][g] = t < 3 ? convert(w, t + 1, g) : convert(w_next, 0, g);
       }
+      __builtin_amdgcn_sched_barrier(0);
     }
+    __syncthreads();
+    unsigned char *b = cur;
+    cur = next;
+    next = fill;
+    fill = b;
+  };
+  // step c: weights from slot c, new ones into slot c - 1; rows c + 2 go to LDS, new ones
+  // into slot c + 1 (all modulo kRing)
+  for (int c0 = 0; c0 < nch; c0 += kRing) {
+#pragma unroll
+    for (int u = 0; u < kRing; ++u)
+      if (c0 + u < nch)
+        step(c0 + u, wr[u], wr[(u + 1) % kRing], wr[(u + kRing - 1) % kRing], xr[(u + 2) % kRing],
+             xr[(u + 1) % kRing]);
   }
-  // loads of the repeated last chunk may still be in flight: the ring registers
-  // stay allocated until they have landed (without these ties the compiler may
-  // put a temporary of the epilogue into one of them before the wait, and the
-  // late load would overwrite it)
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-#pragma unroll
-  for (int u = 0; u < kRing; ++u)
-    wait_loads<0, TERMS>(ring[u]);
 
-  // ---- epilogue: lane holds channels n..n+3 of row m for each row block ------
+  // ---- epilogue: a lane holds channels 8 q + 4 up + 0..3, q = 0..3, of row `col` of every
+  // tile; the wavefront turns 32 rows around in its own part of LDS (free now: every
+  // wavefront is past the last barrier of the loop) and writes whole row segments
+  float *tile = reinterpret_cast<float *>(lds) + wave * (32 * kTurn);
+  const int n0 = g0 * kTileN;
+  constexpr int kQuads = kSpan / 4; // float4 of a row
+  const size_t at = ((size_t)(rbk * a.ncols + ctile) * a.slices + slice) * kWaves + wave;
+  float *part = a.partial + at * kRows * kSpan;
+  const bool vec = (a.ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(a.C) & 15) == 0;
 #pragma unroll
-  for (int g = 0; g < kGroupsPerWave; ++g) {
-    if (g0 + g >= a.groups)
-      continue;
-    const int n = (g0 + g) * kTileN + (lane >> 4) * 4;
-    float s[4], b[4];
+  for (int rb = 0; rb < RB; ++rb) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      s[r] = n + r < a.N ? a.scale[n + r] : 0.f;
-      b[r] = (a.bias && n + r < a.N) ? a.bias[n + r] : 0.f;
-    }
-    const bool vec = n + 3 < a.N && (a.ldc & 3) == 0 &&
-                     (reinterpret_cast<uintptr_t>(a.C) & 15) == 0;
+    for (int g = 0; g < GP; ++g)
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-      const int m = m0 + rb * 16 + (lane & 15);
-      if (m >= a.M)
-        continue;
-      float v[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        v[r] = acc[g][rb][r] * s[r];
-      float *c = a.C + (int64_t)m * a.ldc + n;
-      if (vec) {
-        float4 o = make_float4(v[0], v[1], v[2], v[3]);
-        if (a.accumulate) {
-          const float4 p = *reinterpret_cast<const float4 *>(c);
-          o = make_float4(p.x + o.x, p.y + o.y, p.z + o.z, p.w + o.w);
-        } else {
-          o = make_float4(b[0] + o.x, b[1] + o.y, b[2] + o.z, b[3] + o.w);
+      for (int q = 0; q < 4; ++q) {
+        const int ch = g * 32 + 8 * q + 4 * up;
+        float4 o = make_float4(acc[g][rb][4 * q], acc[g][rb][4 * q + 1], acc[g][rb][4 * q + 2],
+                               acc[g][rb][4 * q + 3]);
+        if (a.slices == 1) {
+          const float4 s = *reinterpret_cast<const float4 *>(scale_s + wave * kSpan + ch);
+          const float4 b = *reinterpret_cast<const float4 *>(bias_s + wave * kSpan + ch);
+          o = make_float4(b.x + o.x * s.x, b.y + o.y * s.y, b.z + o.z * s.z, b.w + o.w * s.w);
         }
-        *reinterpret_cast<float4 *>(c) = o;
+        *reinterpret_cast<float4 *>(tile + col * kTurn + ch) = o;
+      }
+#pragma unroll
+    for (int i = 0; i < kQuads / 2; ++i) {
+      const int idx = lane + 64 * i, row = idx / kQuads, c4 = idx % kQuads;
+      const float4 o = *reinterpret_cast<const float4 *>(tile + row * kTurn + c4 * 4);
+      if (a.slices > 1) {
+        *reinterpret_cast<float4 *>(part + (size_t)(rb * 32 + row) * kSpan + c4 * 4) = o;
+        continue;
+      }
+      const int m = m0 + rb * 32 + row, n = n0 + c4 * 4;
+      if (m >= a.M || n >= a.N)
+        continue;
+      float *cp = a.C + (int64_t)m * a.ldc + n;
+      if (vec && n + 3 < a.N) {
+        float4 q = o;
+        if (a.accumulate) {
+          const float4 p = *reinterpret_cast<const float4 *>(cp);
+          q = make_float4(p.x + q.x, p.y + q.y, p.z + q.z, p.w + q.w);
+        }
+        *reinterpret_cast<float4 *>(cp) = q;
       } else {
+        const float v[4] = {o.x, o.y, o.z, o.w};
 #pragma unroll
         for (int r = 0; r < 4; ++r)
           if (n + r < a.N)
-            c[r] = a.accumulate ? c[r] + v[r] : b[r] + v[r];
+            cp[r] = a.accumulate ? cp[r] + v[r] : v[r];
       }
     }
   }
+}
+
+// What a wavefront needs before its first fetch arrives in SGPRs (this file is built
+// with -amdgpu-kernarg-preload-count); the rest is loaded behind the fetch.
+#define BH_BF16_LEADING                                                                            \
+  const u16 *Abf, const int4 *W, int Mp, int Kp, int groups, int chunks, int ncols, int slices,    \
+      int chunks_per_slice, int ids_padded, GemmArgs a
+#define BH_BF16_TAKE                                                                               \
+  a.Abf = Abf;                                                                                     \
+  a.W = W;                                                                                         \
+  a.Mp = Mp;                                                                                       \
+  a.Kp = Kp;                                                                                       \
+  a.groups = groups;                                                                               \
+  a.chunks = chunks;                                                                               \
+  a.ncols = ncols;                                                                                 \
+  a.slices = slices;                                                                               \
+  a.chunks_per_slice = chunks_per_slice;                                                           \
+  a.ids_padded = ids_padded;
+
+// Blocks of 32 rows per workgroup.
+constexpr int row_blocks(int terms, int gp) { return terms == 1 && gp == 2 ? 2 : 1; }
+
+// 128 channels per workgroup, and 256
+template <int TERMS>
+__global__ void __launch_bounds__(kWaves *kWave) gemm_w8_bf16_kernel(BH_BF16_LEADING) {
+  BH_BF16_TAKE
+  multiply_tile<TERMS, 1, 1>(a);
+}
+template <int TERMS>
+__global__ void __launch_bounds__(kWaves *kWave) gemm_w8_bf16_wide_kernel(BH_BF16_LEADING) {
+  BH_BF16_TAKE
+  multiply_tile<TERMS, row_blocks(TERMS, 2), 2>(a);
+}
+
+// C (+)= scale[n] * sum over the K slices, in slice order (+ bias); four loads are in flight
+// at a time (slices past the end repeat the last one and are not added).
+__global__ void __launch_bounds__(256) add_slices_kernel(GemmArgs a) {
+  const int n4 = (a.N + 3) / 4;
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (int64_t)a.M * n4)
+    return;
+  const int m = (int)(i / n4), n = (int)(i % n4) * 4;
+  const int tile = m / a.tile_rows * a.ncols + n / (kWaves * a.span), wave = n / a.span % kWaves;
+  const size_t row = ((size_t)tile * a.slices * kWaves + wave) * a.tile_rows + m % a.tile_rows;
+  const size_t stride = (size_t)kWaves * a.tile_rows * a.span;
+  const float *p = a.partial + row * a.span + n % a.span;
+  float *c = a.C + (int64_t)m * a.ldc + n;
+  float s[4], b[4], v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const bool in = n + r < a.N;
+    s[r] = in ? a.scale[n + r] : 0.f;
+    b[r] = !in ? 0.f : a.accumulate ? c[r] : a.bias ? a.bias[n + r] : 0.f;
+  }
+  for (int sl = 0; sl < a.slices; sl += 4) {
+    float4 q[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      q[u] = *reinterpret_cast<const float4 *>(p + (size_t)min(sl + u, a.slices - 1) * stride);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (sl + u < a.slices) {
+        v[0] += q[u].x;
+        v[1] += q[u].y;
+        v[2] += q[u].z;
+        v[3] += q[u].w;
+      }
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (n + r < a.N)
+      c[r] = b[r] + v[r] * s[r];
 }
 
 // bf16 staging of the activations: one grow-only device buffer per stream, so
@@ -558,27 +515,102 @@ int staging_for(hipStream_t stream, size_t bytes, const GemmW8Args &in, u16 **ou
 }
 
 BH_VARIANT_FAMILY(WideFamily, "gemm_w8_bf16_wide_kernel");
-BH_VARIANT_FAMILY(SplitFamily, "gemm_w8_bf16_kernel");
+BH_VARIANT_FAMILY(NarrowFamily, "gemm_w8_bf16_kernel");
 
-template <int TERMS, int RB>
-int launch_wide(const GemmArgs &a, unsigned blocks, hipStream_t stream) {
-  constexpr size_t lds = sizeof(v4i32) * 2 * TERMS * 2 * RB * kWave;
-  BH_NOTE_VARIANT(WideFamily, TERMS, RB);
-  hipLaunchKernelGGL((gemm_w8_bf16_wide_kernel<TERMS, RB>), dim3(blocks),
-                     dim3(kSlices * kWave), lds, stream, a);
+template <class Kernel>
+int launch_tiles(Kernel kernel, const GemmArgs &a, unsigned blocks, hipStream_t stream) {
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kWaves * kWave), 0, stream, a.Abf, a.W, a.Mp, a.Kp,
+                     a.groups, a.chunks, a.ncols, a.slices, a.chunks_per_slice, a.ids_padded, a);
   BH_CHECK_HIP(hipGetLastError());
   return BUDDY_HIP_OK;
 }
 
-template <int TERMS>
-int launch_terms(const GemmArgs &a, unsigned blocks, hipStream_t stream) {
-  constexpr size_t lds = sizeof(float) * kSlices * 64 * kWave;
-  auto kernel = gemm_w8_bf16_kernel<TERMS>;
-  static DynLdsOnce dyn_lds;
-  BH_CHECK_HIP(ensure_dyn_lds(dyn_lds, reinterpret_cast<const void *>(kernel),
-                              (int)lds));
-  BH_NOTE_VARIANT(SplitFamily, TERMS);
-  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kSlices * kWave), lds, stream, a);
+// Channel tiles per wavefront and K slices for a launch, by an estimate of its time in
+// microseconds.  An XCD (32 compute units) works on 64 workgroups at a time, two to a compute
+// unit.  A chunk of 64 k on L layers of 32 rows (terms, blocks of rows) takes a compute unit
+// with two workgroups 0.14 + 0.38 L us, one that has its compute unit to itself 0.34 + 0.16 L
+// us (with one channel tile 0.24 + 0.21 L and 0.2 + 0.075 L); a last round that fills less
+// than half runs at the latter.  Fitted to these, microseconds (one term; three; in brackets
+// 16 x 16 x 32 products, on tiles of 64 x 64 whose wavefronts split K or of 48 or 64 rows x
+// 256 channels):
+//   8960 -> 1536, with the adding of its slices: 17 rows 11 [38]; 16 [97], 150: 17 [41]; 31
+//     [98], 1024: 46 [78]; 94 [200], 1931: 84 [119]; 168 [307]
+//   1536 -> 17920: 17 rows 12 [18]; 16 [42], 150: 23 [29]; 34 [51], 512: 45 [62]; 85 [147],
+//     1931: 127 [175]; 300 [433]
+//   1536 -> 2048: 150 rows 11.2 [11.5]; 14.8 [21.6], 1024: 15.6 [19.3]; 26 [44]
+struct TilePlan {
+  int gp = 0, slices = 1;
+  double us = 0;
+};
+TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, int terms) {
+  TilePlan best;
+  for (int gp = 1; gp <= 2; ++gp) {
+    const int layers = terms * row_blocks(terms, gp);
+    const int64_t rows = ceil_div(M, 32 * row_blocks(terms, gp));
+    const int64_t ncols = ceil_div(channels, kWaves * 32 * gp);
+    const double alone = gp == 2 ? 0.34 + 0.16 * layers : 0.20 + 0.075 * layers;
+    const double full = gp == 2 ? 0.14 + 0.38 * layers : 0.24 + 0.21 * layers;
+    for (int s = 1; s <= 16; ++s) {
+      const int64_t per_xcd = ceil_div(ncols * s, 8) * rows;
+      if (s > 1 && per_xcd > 256)
+        break;
+      const int64_t cps = ceil_div(chunks, s);
+      if (ceil_div(chunks, cps) != s)
+        continue; // the last slice would be empty
+      const double store = s > 1 ? 2.0 : 0.0; // of the partial sums
+      const double full_us = full * (double)cps + 4.0 + store;
+      const double alone_us = alone * (double)cps + 5.0 + store;
+      const int64_t left = per_xcd % 64;
+      double us = (double)(per_xcd / 64) * full_us +
+                  (left == 0 ? 0.0 : 2 * left <= 64 ? alone_us : full_us);
+      if (s > 1) // the kernel that adds the slices: 4 us and its bytes
+        us += 4.0 + 4.0 * (double)(M * s) * (double)(ncols * 128 * gp) / 5e6;
+      if (!best.gp || us < best.us - 1e-9)
+        best = {gp, s, us};
+    }
+  }
+  return best;
+}
+
+int launch_plan(const TilePlan &plan, GemmArgs &a, int terms, hipStream_t stream) {
+  a.tile_rows = 32 * row_blocks(terms, plan.gp);
+  a.span = 32 * plan.gp;
+  a.ncols = (int)ceil_div(a.N, kWaves * a.span);
+  a.row_tiles = (int)ceil_div(a.M, a.tile_rows);
+  a.slices = plan.slices;
+  a.chunks_per_slice = (int)ceil_div(a.chunks, plan.slices);
+  a.ids_padded = (int)round_up((int64_t)a.ncols * a.slices, 8);
+  a.partial = nullptr;
+  if (a.slices > 1) {
+    const size_t tile_floats = (size_t)a.tile_rows * kWaves * a.span;
+    char *ws = nullptr;
+    if (int rc = gemm_slices_workspace(
+            stream, sizeof(float) * tile_floats * a.slices * (size_t)a.ncols * a.row_tiles, &ws))
+      return rc;
+    a.partial = reinterpret_cast<float *>(ws);
+  }
+  const unsigned blocks = (unsigned)a.ids_padded * a.row_tiles;
+  int rc;
+  if (plan.gp == 1) {
+    if (terms == 1) {
+      BH_NOTE_VARIANT(NarrowFamily, 1);
+      rc = launch_tiles(gemm_w8_bf16_kernel<1>, a, blocks, stream);
+    } else {
+      BH_NOTE_VARIANT(NarrowFamily, 3);
+      rc = launch_tiles(gemm_w8_bf16_kernel<3>, a, blocks, stream);
+    }
+  } else if (terms == 1) {
+    BH_NOTE_VARIANT(WideFamily, 1);
+    rc = launch_tiles(gemm_w8_bf16_wide_kernel<1>, a, blocks, stream);
+  } else {
+    BH_NOTE_VARIANT(WideFamily, 3);
+    rc = launch_tiles(gemm_w8_bf16_wide_kernel<3>, a, blocks, stream);
+  }
+  if (rc || a.slices == 1)
+    return rc;
+  const int64_t threads = (int64_t)a.M * ceil_div(a.N, 4);
+  hipLaunchKernelGGL(add_slices_kernel, dim3((unsigned)ceil_div(threads, 256)), dim3(256), 0,
+                     stream, a);
   BH_CHECK_HIP(hipGetLastError());
   return BUDDY_HIP_OK;
 }
@@ -653,8 +685,6 @@ int launch_gemm_w8(const GemmW8Args &in, hipStream_t stream) {
   const GemmStagingLayout layout = gemm_staging_layout(in.M, in.K);
   a.Mp = layout.rows_padded;
   a.Kp = layout.cols_padded;
-  a.ncols = (int)ceil_div(a.groups, kGroupsPerWave);
-  a.cols_padded = (int)round_up(a.ncols, 8);
   a.accumulate = in.accumulate ? 1 : 0;
   u16 *abf = static_cast<u16 *>(const_cast<void *>(in.staged));
   bool staged = in.staged != nullptr;
@@ -677,24 +707,7 @@ int launch_gemm_w8(const GemmW8Args &in, hipStream_t stream) {
                        in.terms, abf);
     BH_CHECK_HIP(hipGetLastError());
   }
-  // wide matrices: a workgroup per 64 rows x 256 channels, no split of K
-  const int wide_cols = (int)ceil_div(a.groups, kGroupsPerWave * kSlices);
-  if ((int64_t)wide_cols * (a.Mp / kRowsPerWave) >= 200) {
-    // 64 or 48 rows per workgroup: the chip runs 256 workgroups at a time (one
-    // wavefront per SIMD), so the time is rounds x rows; ties go to 64 rows,
-    // which convert each weight tile fewer times
-    const int64_t wg4 = wide_cols * ceil_div(in.M, 64), wg3 = wide_cols * ceil_div(in.M, 48);
-    const bool three = ceil_div(wg3, 256) * 3 < ceil_div(wg4, 256) * 4;
-    const int rows = three ? 48 : 64;
-    a.ncols = wide_cols;
-    a.cols_padded = (int)round_up(wide_cols, 8);
-    const unsigned wb = (unsigned)(a.cols_padded * ceil_div(in.M, rows));
-    if (three)
-      return in.terms == 1 ? launch_wide<1, 3>(a, wb, stream) : launch_wide<3, 3>(a, wb, stream);
-    return in.terms == 1 ? launch_wide<1, 4>(a, wb, stream) : launch_wide<3, 4>(a, wb, stream);
-  }
-  const unsigned blocks = (unsigned)(a.cols_padded * (a.Mp / kRowsPerWave));
-  return in.terms == 1 ? launch_terms<1>(a, blocks, stream) : launch_terms<3>(a, blocks, stream);
+  return launch_plan(plan_tiles(in.M, in.N, a.chunks, in.terms), a, in.terms, stream);
 }
 
 void release_gemm_staging(hipStream_t stream) {

@@ -275,6 +275,31 @@ def test_int8_matmul_tile_edges(bh, oracle, M, K, N):
             assert (np.abs(have.cpu().numpy() - expect) <= 24 * 2.0**-24 * size).all()
 
 
+@pytest.mark.parametrize("M,K,N", [
+    (17, 64, 1), (31, 65, 127), (32, 128, 128), (33, 192, 129), (64, 257, 255), (65, 320, 257),
+    (100, 1000, 31), (17, 5000, 48), (97, 8960, 513), (300, 4100, 1100)])
+def test_bf16_matmul_tile_edges(M, K, N):
+    """One bf16 term and three: against the sums in 64 bits."""
+    q, s = synthetic.quantized_linear(K, N, M + K + N)
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn((M, K), generator=g, device="cuda")
+    c0 = torch.randn((M, N), generator=g, device="cuda")
+    qh, sh = q.cpu().numpy().astype(np.float64), s.cpu().numpy().astype(np.float64)
+    packed = ops.pack_w8(q)
+    for exact in (False, True):
+        xh = x.cpu().numpy() if exact else bf16_round(x.cpu().numpy())
+        # f32 sums of exact products, each addition within 2^-24 of the sum of the
+        # magnitudes so far: their walk stays within 4 sqrt(K) of these
+        size = np.abs(xh).astype(np.float64) @ np.abs(qh) * sh + np.abs(c0.cpu().numpy())
+        want = xh.astype(np.float64) @ qh * sh
+        got = ops.gemm_w8a32(x, packed, s, K, N, exact=exact)
+        more = c0.clone()
+        ops.gemm_w8a32(x, packed, s, K, N, out=more, accumulate=True, exact=exact)
+        for have, expect in ((got, want), (more, want + c0.cpu().numpy())):
+            err = np.abs(have.cpu().numpy() - expect)
+            assert (err <= 4 * np.sqrt(K + 16) * 2.0**-24 * size).all()
+
+
 def test_every_bf16_prefill_matmul_variant(bh, oracle):
     bh.buddy_hip_variant_reset()
     for M, K, N in GEMM_BF16_SHAPES:
