@@ -54,7 +54,8 @@ struct Session {
   int *state = nullptr;         // device: token, pos, step
   int *token_log = nullptr;     // device: greedy tokens by step
   int token_log_cap = 0;
-  int *host_state = nullptr;    // pinned staging for token/pos/step
+  // pinned: token, position, step, and behind them the logits, as hand_out leaves them
+  int *host_state = nullptr;
   // Host-side mirror of the device's (position, step): what the next enqueued
   // step will use.  -1 until set_state; every step advances both on the device,
   // so the host can refuse steps that would leave the cache or the token log.
@@ -81,7 +82,10 @@ struct Session {
   int invalidate_graph();
   int check_steps(int steps, const char *who) const;
   int run_step();
+  // Enqueues token, position and step, and what a step finds prepared.
   int set_state(int token, int pos, int step);
+  // Ends a call: waits for the stream, then next_token and (both optional) the logits.
+  int hand_out(float *logits_out, int *next_token);
 };
 
 inline Session *as_session(buddy_hip_session *s) { return reinterpret_cast<Session *>(s); }

@@ -607,3 +607,26 @@ def test_greedy_pick_taken_from_the_lm_head_launch_keeps_the_first_maximum(bh, o
         tok = (tok * 7919 + 13) % shape.vocab  # other rows of the embedding
     sess.close()
     assert len(seen) >= 1
+
+
+@pytest.mark.parametrize("vocab", [1024, 1029])
+def test_logits_reach_every_kind_of_memory(vocab):
+    """Pageable host memory (through the session's pinned buffer), pinned host memory and
+    device memory (copied to directly) hold the session's logits, bit for bit."""
+    shape = Shape(layers=1, hidden=256, heads=4, kv_heads=2, head_dim=128, inter=512, vocab=vocab,
+                  max_len=64, rms_eps=1e-6)
+    sess, _ = synthetic.build_session(shape, context=5)
+    lib = bma.lib()
+    pageable = np.full(vocab, np.nan, np.float32)
+    pinned = torch.full((vocab,), float("nan"), pin_memory=True)
+    device = torch.full((vocab,), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    chosen = set()
+    for at in (pageable.ctypes.data, pinned.data_ptr(), device.data_ptr()):
+        nxt = ctypes.c_int(-1)
+        assert lib.buddy_hip_session_decode(sess._h, 7, 5, at, ctypes.byref(nxt)) == 0
+        chosen.add(nxt.value)
+    assert chosen == {int(pageable.argmax())}
+    np.testing.assert_array_equal(pageable, pinned.numpy())
+    np.testing.assert_array_equal(pageable, device.cpu().numpy())
+    sess.close()
