@@ -639,10 +639,10 @@ __device__ __forceinline__ void multiply_tile(const GemmI8Args &a) {
   a.row_tiles = row_tiles;
 
 // 128 channels per workgroup, and 256
-template <int D>
+template <int D, bool PAIR>
 __global__ void __launch_bounds__(kSlices *kWave) gemm_w8_i8_kernel(BH_I8_LEADING) {
   BH_I8_TAKE
-  multiply_tile<D, 1, 1, false>(a);
+  multiply_tile<D, 1, 1, PAIR>(a);
 }
 template <int D, bool PAIR>
 __global__ void __launch_bounds__(kSlices *kWave) gemm_w8_i8_wide_kernel(BH_I8_LEADING) {
@@ -839,9 +839,10 @@ int launch_wide(const GemmI8Args &a, unsigned blocks, hipStream_t stream) {
   return launch_tiles(gemm_w8_i8_wide_kernel<D, PAIR>, a, blocks, stream);
 }
 
-template <int D> int launch_narrow(const GemmI8Args &a, unsigned blocks, hipStream_t stream) {
-  BH_NOTE_VARIANT(NarrowFamily, D);
-  return launch_tiles(gemm_w8_i8_kernel<D>, a, blocks, stream);
+template <int D, bool PAIR>
+int launch_narrow(const GemmI8Args &a, unsigned blocks, hipStream_t stream) {
+  BH_NOTE_VARIANT(NarrowFamily, D, (int)PAIR);
+  return launch_tiles(gemm_w8_i8_kernel<D, PAIR>, a, blocks, stream);
 }
 
 } // namespace
@@ -942,13 +943,15 @@ namespace {
 // 0.21: the way through LDS); a last round that fills less than half runs at the latter.
 // Fitted to these, microseconds (three planes; two; in brackets 16 x 16 x 64 instructions
 // on tiles of 32 or 64 rows x 128 or 256 channels):
-//   gate | up, 1536 -> 2 x 8960: 27 rows 13.7 [18.4]; 12.1 [15.0], 256: 32.6 [30.6]; 27.3
+//   gate | up, 1536 -> 2 x 8960: 27 rows 11.2 [18.4]; 10.0 [15.0], 256: 32.6 [30.6]; 27.3
 //     [23.3], 512: 52.3 [58.8]; 42.7 [44.3], 1931: 180 [201]; 141 [150]
 //   down, 8960 -> 1536, with the adding of its slices: 27 rows 12.7 [16.9]; 11.1 [15.1],
 //     512: 34 [36]; 29 [28], 1931: 96 [112]; 77 [95]
 //   q|k|v, 1536 -> 2048: 100 rows 10.0 [13.3]; 8.2 [12.6], 512: 12.5 [15.8]; 9.9 [11.8],
 //     1024: 17.2 [30.4]; 14.4 [22.7]
 //   one plane: 1536 -> 8960: 512 rows 18.6 [21.2], 2048: 52 [69]
+// (gate | up at 27 rows with two channel tiles: 13.7, and 18.7 in a prompt, whose weights come
+// from memory, against 14.9 with one: twice the compute units ask for them.)
 // (A tile of 64 rows x 256 channels, one workgroup to a compute unit, takes as long per
 // row; its rounds are coarser: gate | up at 512 rows 61.8, at 256 rows 40.6.)
 // The (column tile, slice) pairs of an XCD keep their row tiles together; where their number
@@ -963,7 +966,7 @@ TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, bool may_split, dou
                     int64_t sum_wgs) {
   TilePlan best;
   constexpr int64_t kRoom = 64;
-  for (int gp = PAIR ? 2 : 1; gp <= 2; ++gp) {
+  for (int gp = 1; gp <= 2; ++gp) {
     const int64_t ncols = ceil_div(channels, kSlices * gp * (PAIR ? 16 : 32));
     const int layers = D * row_blocks(D, gp);
     const int64_t rows = ceil_div(M, 32 * row_blocks(D, gp));
@@ -1021,9 +1024,8 @@ int launch_plan(const TilePlan &plan, GemmI8Args &a, hipStream_t stream) {
     a.partial = reinterpret_cast<float *>(ws);
   }
   const unsigned blocks = (unsigned)(a.ids_padded * a.band_rows);
-  if constexpr (!PAIR)
-    if (plan.gp == 1)
-      return launch_narrow<D>(a, blocks, stream);
+  if (plan.gp == 1)
+    return launch_narrow<D, PAIR>(a, blocks, stream);
   return launch_wide<D, PAIR>(a, blocks, stream);
 }
 
