@@ -599,7 +599,11 @@ int launch_wide(const RowsGemm &a, hipStream_t stream) {
 // still fill the 256 compute units.  Above that the tile with the lowest estimate: tiles
 // per compute unit x steps of 64 k x what a step of such a tile takes (us, measured with
 // K of 1536 to 8960 on full and on partly filled chips), plus what a tile takes to
-// begin and to store.
+// begin and to store.  Tiles of 16 rows x 64 channels stay the best of few rows, whose
+// launches are bound by how many compute units ask for the weights (bfloat16, us against
+// 32 or 64 x 128): 8960 -> 1536 at 24 rows 21.2 vs 28.4, at 150 22.7 vs 31.3, at 220 36.0
+// vs 31.5; 1536 -> 1536 at 64 rows 5.6 vs 6.9; 1536 -> 17920 at 64 rows 18.4 vs 12.4.  In
+// f32, whose three terms make the products the longer part, they gain nothing.
 template <typename T, int OUT, bool GROUPED>
 int launch_shape(const RowsGemm &a, hipStream_t stream) {
   const int64_t rows = GROUPED ? ceil_div(a.list_total, a.experts) : a.rows;
@@ -622,15 +626,23 @@ int launch_shape(const RowsGemm &a, hipStream_t stream) {
         return launch_wide<T, 1, 1, OUT, GROUPED>(a, stream);
     return launch_wide<T, 1, 2, OUT, GROUPED>(a, stream);
   } else {
-    const double tall = cost(128, 256, 1.02, 7.0);
+    // few rows: 16-row tiles of 64 channels, while they are few rounds of the chip
+    const double tall = cost(128, 256, 1.02, 7.0), flat = cost(16, 64 * P, 0.13 * P, 2.5);
     if constexpr (kPair) {
-      const double half = cost(64, 256, 0.60, 5.0), low = cost(32, 256, 0.40, 4.0);
+      // fewer workgroups than half the chip draw the weights from memory too slowly
+      auto thin = [&](int rt) { return workgroups(rt, 128) < 128 ? 6.0 : 0.0; };
+      const double half = cost(64, 256, 0.60, 5.0) + thin(64);
+      const double low = cost(32, 256, 0.40, 4.0) + thin(32);
+      if (flat <= std::min({tall, half, low}))
+        return launch_variant<T, 1, P, OUT, GROUPED>(a, stream);
       if (tall <= std::min(half, low))
         return launch_wide<T, 4, 2, OUT, GROUPED>(a, stream);
       return half <= low ? launch_wide<T, 2, 2, OUT, GROUPED>(a, stream)
                          : launch_wide<T, 1, 2, OUT, GROUPED>(a, stream);
     } else {
       const double half = cost(64, 128, 0.29, 4.5), low = cost(32, 128, 0.21, 4.0);
+      if (flat <= std::min({tall, half, low}))
+        return launch_variant<T, 1, P, OUT, GROUPED>(a, stream);
       if (tall <= std::min(half, low))
         return launch_wide<T, 4, 2, OUT, GROUPED>(a, stream);
       return half <= low ? launch_wide<T, 2, 1, OUT, GROUPED>(a, stream)
