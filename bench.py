@@ -535,8 +535,7 @@ def bench_prefill(bh, args):
         "detail": res, "gemm_flop": gemm_flop, "attention_flop": attn_flop,
         # algorithmic flops 2 M K N (each digit plane is not counted again)
         # over the time of the whole pass, against the dense int8 peak
-        "roofline": {"kernel": "gemm_w8_i8_wide_kernel<3, 4, 5> (gate, up), <3, 4, 4> (down), "
-                               "gemm_w8_i8_kernel<3> (q|k|v, o)",
+        "roofline": {"kernel": "gemm_w8_i8_wide_kernel<3, true> (gate, up), <3, false> (down, o), gemm_w8_i8_kernel<3, false> (q|k|v)",
                      "bound": "mfma", "achieved": res["i8_3digit"]["gemm_tflops"],
                      "peak": MFMA_I8_PEAK_TOPS, "unit": "TFLOP/s",
                      "frac": res["i8_3digit"]["mfma_frac"], "traffic": None},
