@@ -86,6 +86,7 @@ def _declare(lib):
         "buddy_hip_last_error": (c_char_p, []),
         "buddy_hip_device_count": (c_int, []),
         "buddy_hip_variant_report": (i64, [vp, i64]),
+        "buddy_hip_tile_report": (i64, [vp, i64]),
         "buddy_hip_variant_reset": (None, []),
         "buddy_hip_w8_packed_bytes": (sz, [i64, i64]),
         "buddy_hip_pack_w8": (c_int, [vp, i64, i64, vp, vp]),

@@ -38,6 +38,7 @@ int caught(const char *where) noexcept {
 
 namespace {
 struct VariantEntry {
+  VariantList list;
   std::string name;
   std::atomic<long long> launches{0};
 };
@@ -53,7 +54,7 @@ VariantTable &variants() {
 }
 } // namespace
 
-int register_variant(const char *family, std::initializer_list<int> params) {
+int register_variant(VariantList list, const char *family, std::initializer_list<int> params) {
   std::string name = family;
   name += '<';
   bool first = true;
@@ -67,6 +68,7 @@ int register_variant(const char *family, std::initializer_list<int> params) {
   VariantTable &t = variants();
   std::lock_guard<std::mutex> lock(t.mu);
   t.entries.emplace_back();
+  t.entries.back().list = list;
   t.entries.back().name = std::move(name);
   return (int)t.entries.size() - 1;
 }
@@ -80,17 +82,16 @@ void note_variant_launch(int id) {
   }
   e->launches.fetch_add(1, std::memory_order_relaxed);
 }
-} // namespace bh
 
-extern "C" {
-
-int64_t buddy_hip_variant_report(char *text, int64_t capacity) try {
-  bh::VariantTable &t = bh::variants();
+namespace {
+int64_t report_variants(VariantList list, char *text, int64_t capacity) {
+  VariantTable &t = variants();
   std::string out;
   {
     std::lock_guard<std::mutex> lock(t.mu);
-    for (const bh::VariantEntry &e : t.entries)
-      out += e.name + '\t' + std::to_string(e.launches.load(std::memory_order_relaxed)) + '\n';
+    for (const VariantEntry &e : t.entries)
+      if (e.list == list)
+        out += e.name + '\t' + std::to_string(e.launches.load(std::memory_order_relaxed)) + '\n';
   }
   if (text && capacity > 0) {
     const size_t n = std::min(out.size(), (size_t)capacity - 1);
@@ -98,6 +99,20 @@ int64_t buddy_hip_variant_report(char *text, int64_t capacity) try {
     text[n] = 0;
   }
   return (int64_t)out.size() + 1;
+}
+} // namespace
+} // namespace bh
+
+extern "C" {
+
+int64_t buddy_hip_variant_report(char *text, int64_t capacity) try {
+  return bh::report_variants(bh::VariantList::kHandScheduled, text, capacity);
+} catch (...) {
+  return 0;
+}
+
+int64_t buddy_hip_tile_report(char *text, int64_t capacity) try {
+  return bh::report_variants(bh::VariantList::kTiles, text, capacity);
 } catch (...) {
   return 0;
 }

@@ -86,15 +86,23 @@ constexpr int kTileBytes = 1024;   // one wavefront-wide 128-bit load
 // is loaded (a static member of Variant<Family, params...>, instantiated where
 // the launch site names it) and counts its launches, so that a test can ask
 // whether every compiled variant of such a kernel has met the oracle
-// (buddy_hip_variant_report).
-int register_variant(const char *family, std::initializer_list<int> params);
+// (buddy_hip_variant_report).  Kernels whose loads the compiler schedules, but
+// whose tile an estimate picks, are listed apart (buddy_hip_tile_report).
+enum class VariantList { kHandScheduled, kTiles };
+int register_variant(VariantList list, const char *family, std::initializer_list<int> params);
 void note_variant_launch(int id);
 template <typename Family, int... P> struct Variant {
-  static inline const int id = register_variant(Family::name, {P...});
+  static inline const int id = register_variant(Family::list, Family::name, {P...});
 };
 #define BH_VARIANT_FAMILY(tag, text)                                           \
   struct tag {                                                                 \
     static constexpr const char *name = text;                                  \
+    static constexpr ::bh::VariantList list = ::bh::VariantList::kHandScheduled; \
+  }
+#define BH_TILE_FAMILY(tag, text)                                              \
+  struct tag {                                                                 \
+    static constexpr const char *name = text;                                  \
+    static constexpr ::bh::VariantList list = ::bh::VariantList::kTiles;       \
   }
 #define BH_NOTE_VARIANT(...) ::bh::note_variant_launch(::bh::Variant<__VA_ARGS__>::id)
 

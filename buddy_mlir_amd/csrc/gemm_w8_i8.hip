@@ -823,6 +823,7 @@ reduce_slices_norm_kernel(const float *p_partial, const float *p_steps, int p_N,
 
 BH_VARIANT_FAMILY(WideFamily, "gemm_w8_i8_wide_kernel");
 BH_VARIANT_FAMILY(NarrowFamily, "gemm_w8_i8_kernel");
+BH_TILE_FAMILY(NarrowPairFamily, "gemm_w8_i8_kernel pair");
 
 template <class Kernel>
 int launch_tiles(Kernel kernel, const GemmI8Args &a, unsigned blocks, hipStream_t stream) {
@@ -841,7 +842,10 @@ int launch_wide(const GemmI8Args &a, unsigned blocks, hipStream_t stream) {
 
 template <int D, bool PAIR>
 int launch_narrow(const GemmI8Args &a, unsigned blocks, hipStream_t stream) {
-  BH_NOTE_VARIANT(NarrowFamily, D, (int)PAIR);
+  if constexpr (PAIR)
+    BH_NOTE_VARIANT(NarrowPairFamily, D);
+  else
+    BH_NOTE_VARIANT(NarrowFamily, D);
   return launch_tiles(gemm_w8_i8_kernel<D, PAIR>, a, blocks, stream);
 }
 

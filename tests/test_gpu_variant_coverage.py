@@ -25,10 +25,11 @@ from test_gpu_prefill import (SCALE, SILU_PAIR_SHAPES, bf16_round, fixed_point_r
 pytestmark = pytest.mark.gpu
 
 
-def report(bh):
-    n = bh.buddy_hip_variant_report(None, 0)
+def report(bh, of="variant"):
+    write = getattr(bh, f"buddy_hip_{of}_report")
+    n = write(None, 0)
     buf = ctypes.create_string_buffer(n)
-    bh.buddy_hip_variant_report(buf, n)
+    write(buf, n)
     out = {}
     for line in buf.value.decode().splitlines():
         name, hits = line.split("\t")
@@ -239,7 +240,7 @@ def test_every_int8_prefill_matmul_variant(bh, oracle):
         gemm_case(oracle, M, K, N, "digits2")
     for M, K, N in W8A8_SPLIT_K_SHAPES:
         w8a8_case(bh, oracle, M, K, N)
-    for M, K, N in SILU_PAIR_SHAPES[1:6]:  # the paired variants
+    for M, K, N in SILU_PAIR_SHAPES[1:5]:  # the paired variants
         silu_pair_case(oracle, M, K, N)
         silu_pair_case(oracle, M, K, N, digits=2)
     for fam in ("gemm_w8_i8_wide_kernel", "gemm_w8_i8_kernel"):
@@ -298,6 +299,17 @@ def test_bf16_matmul_tile_edges(M, K, N):
         for have, expect in ((got, want), (more, want + c0.cpu().numpy())):
             err = np.abs(have.cpu().numpy() - expect)
             assert (err <= 4 * np.sqrt(K + 16) * 2.0**-24 * size).all()
+
+
+@pytest.mark.parametrize("M,K,N", [(17, 64, 16), (27, 1536, 8960), (32, 200, 48), (31, 320, 4496)])
+@pytest.mark.parametrize("digits", [2, 3])
+def test_silu_pair_of_few_rows(bh, oracle, M, K, N, digits):
+    """Up to 32 rows the pair runs on tiles of 128 channels of both matrices together: one
+    channel group, a tile less one group, whole tiles; one chunk of K and more than are
+    asked for ahead."""
+    bh.buddy_hip_variant_reset()
+    silu_pair_case(oracle, M, K, N, digits=digits)
+    assert {k for k, v in report(bh, "tile").items() if v} == {f"gemm_w8_i8_kernel pair<{digits}>"}
 
 
 def test_every_bf16_prefill_matmul_variant(bh, oracle):
