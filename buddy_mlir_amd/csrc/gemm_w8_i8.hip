@@ -267,10 +267,7 @@ struct GemmI8Args {
   float *C;
   int64_t ldc;
   int M, N, Mp, Kp, groups, chunks;
-  int ncols;       // column tiles
-  // the row tiles are shared out over bands of band_rows; ids_padded workgroup ids per row
-  // of a band: column tiles x slices x bands, padded to the XCD count
-  int ids_padded, band_rows, row_tiles;
+  int ncols, row_tiles, panel; // column tiles, row tiles, and how they are placed
   int span;      // channels per wavefront, where K is split
   int tile_rows; // rows per workgroup, where K is split
   // K split over `slices` workgroups per tile, chunks_per_slice chunks each
@@ -320,6 +317,44 @@ typedef int v16i32 __attribute__((ext_vector_type(16)));
 constexpr int row_blocks(int D, int gp) { return D == 1 && gp == 2 ? 3 : 1; }
 constexpr int kWideRow = kTileK + 16; // bytes of a row in LDS: fragment reads meet every bank once
 
+// Ids equal modulo 8 run on the same XCD.  An XCD takes a run of an eighth of all tiles, in
+// panels of `panel` (column tile, K slice) pairs by all row tiles: the workgroups that it
+// runs at the same time share rows and weights in its L2, and no XCD has more than one tile
+// above another.  (Pairs shared out to the XCDs, all of an XCD's pairs for a row tile before
+// the next row tile: the weights of many columns leave the L2 between two row tiles.
+// 4096 -> 2 x 14336, two planes: 640 rows 252 us so, 182 in panels; 1536 -> 8960, whose 35
+// columns made it cut the rows into bands besides, 4096 rows 274 and 160.)
+//
+// panel == 0: the pairs are shared out to the XCDs after all (false: a padding id).
+__device__ __forceinline__ bool place_tile(int units, int rows, int panel, int &unit, int &row) {
+  const int id = blockIdx.x;
+  if (panel == 0) {
+    const int ids = (units + 7) & ~7;
+    row = id / ids;
+    unit = id - row * ids;
+    return unit < units;
+  }
+  const int total = units * rows, die = id % 8;
+  const int t = die * (total / 8) + min(die, total % 8) + id / 8;
+  const int p = t / (panel * rows), rest = t - p * panel * rows;
+  const int width = min(panel, units - p * panel);
+  row = rest / width;
+  unit = p * panel + rest - row * width;
+  return true;
+}
+// The 64 workgroups of an XCD are 4 pairs by 16 row tiles at a time, with fewer row tiles
+// all of them by as many pairs as it takes, one pair after the other.  Of few row tiles every
+// pair should be on one XCD only and workgroups that start one behind the other on different
+// weights (100 rows, 1536 -> 2 x 8960, two planes: 17.8 us shared out, 19.5 in panels; 224
+// rows 23.5 and 23.0), unless that gives an XCD a second workgroup on a compute unit that its
+// share alone does not, or notably more of them.
+inline int panel_for(int64_t units, int row_tiles) {
+  const int64_t most = ceil_div(units, 8) * row_tiles, tiles = units * row_tiles;
+  if (row_tiles <= 5 && (most <= 32 || (tiles > 8 * 32 && 100 * 8 * most <= 106 * tiles)))
+    return 0;
+  return row_tiles <= 16 ? 1 : row_tiles <= 32 ? 2 : 4;
+}
+
 // sum_j 256^j acc_j as f32 (each int32 sum is exact; the conversions round to 24
 // bits, like an f32 accumulator would)
 template <int D> __device__ __forceinline__ float combine(const v16i32 (&acc)[D], int r) {
@@ -359,12 +394,9 @@ __device__ __forceinline__ void multiply_tile(const GemmI8Args &a) {
   __shared__ float step_s[kRows];
   const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, up = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // ids equal modulo 8 run on the same XCD: the row tiles of one (column tile, K slice,
-  // band) do, and share its weights in that XCD's L2
-  const int id = blockIdx.x % a.ids_padded, units = a.ncols * a.slices;
-  const int unit = id % units, rbk = id / units * a.band_rows + blockIdx.x / a.ids_padded;
-  if (rbk >= a.row_tiles)
-    return; // padding id, or a last band with fewer rows
+  int unit, rbk;
+  if (!place_tile(a.ncols * a.slices, a.row_tiles, a.panel, unit, rbk))
+    return;
   const int ctile = unit % a.ncols, slice = unit / a.ncols;
   const int m0 = rbk * kRows;
   const int half_groups = a.groups / 2; // PAIR only
@@ -623,7 +655,7 @@ __device__ __forceinline__ void multiply_tile(const GemmI8Args &a) {
 // with -amdgpu-kernarg-preload-count); the rest is loaded behind the fetch.
 #define BH_I8_LEADING                                                                              \
   const int8_t *planes, const int4 *W, int Mp, int Kp, int groups, int chunks, int ncols,          \
-      int slices, int chunks_per_slice, int ids_padded, int band_rows, int row_tiles, GemmI8Args a
+      int slices, int chunks_per_slice, int row_tiles, int panel, GemmI8Args a
 #define BH_I8_TAKE                                                                                 \
   a.planes = planes;                                                                               \
   a.W = W;                                                                                         \
@@ -634,9 +666,8 @@ __device__ __forceinline__ void multiply_tile(const GemmI8Args &a) {
   a.ncols = ncols;                                                                                 \
   a.slices = slices;                                                                               \
   a.chunks_per_slice = chunks_per_slice;                                                           \
-  a.ids_padded = ids_padded;                                                                       \
-  a.band_rows = band_rows;                                                                         \
-  a.row_tiles = row_tiles;
+  a.row_tiles = row_tiles;                                                                         \
+  a.panel = panel;
 
 // 128 channels per workgroup, and 256
 template <int D, bool PAIR>
@@ -829,7 +860,7 @@ template <class Kernel>
 int launch_tiles(Kernel kernel, const GemmI8Args &a, unsigned blocks, hipStream_t stream) {
   hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kSlices * kWave), 0, stream, a.planes, a.W, a.Mp,
                      a.Kp, a.groups, a.chunks, a.ncols, a.slices, a.chunks_per_slice,
-                     a.ids_padded, a.band_rows, a.row_tiles, a);
+                     a.row_tiles, a.panel, a);
   BH_CHECK_HIP(hipGetLastError());
   return BUDDY_HIP_OK;
 }
@@ -939,8 +970,8 @@ int gemm_slices_workspace(hipStream_t stream, size_t bytes, char **out) {
 
 namespace {
 
-// Channel tiles per wavefront, K slices and bands of rows for a launch, by an estimate of
-// its time in microseconds.  An XCD (32 compute units) works on 64 workgroups at a time, two
+// Channel tiles per wavefront and K slices for a launch, by an estimate of its time in
+// microseconds.  An XCD (32 compute units) works on 64 workgroups at a time, two
 // to a compute unit.  A chunk of 64 k on L layers of 32 rows (planes, blocks of rows) takes
 // a compute unit with two workgroups 0.18 + 0.16 L us, one that has its compute unit to
 // itself 0.15 + 0.08 L us (with one channel tile 0.2 + 0.085 L and 0.06 + 0.07 L, at least
@@ -958,11 +989,8 @@ namespace {
 // from memory, against 14.9 with one: twice the compute units ask for them.)
 // (A tile of 64 rows x 256 channels, one workgroup to a compute unit, takes as long per
 // row; its rounds are coarser: gate | up at 512 rows 61.8, at 256 rows 40.6.)
-// The (column tile, slice) pairs of an XCD keep their row tiles together; where their number
-// is a poor multiple of 8 the rows are cut into bands, which share the XCDs more evenly and
-// read the weights once per band (4096 rows, 512 -> 512: 9.0 us, in one band 25.5).
 struct TilePlan {
-  int gp = 0, slices = 1, bands = 1;
+  int gp = 0, slices = 1;
   double us = 0;
 };
 template <int D, bool PAIR>
@@ -977,15 +1005,7 @@ TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, bool may_split, dou
     const double alone = gp == 2 ? 0.15 + 0.08 * layers : std::max(0.21, 0.06 + 0.07 * layers);
     const double full = gp == 2 ? 0.18 + 0.16 * layers : 0.2 + 0.085 * layers;
     for (int s = 1; s <= (may_split ? 16 : 1); ++s) {
-      int bands = 1;
-      int64_t per_xcd = ceil_div(ncols * s, 8) * rows;
-      for (int b = 2; b <= 8; b *= 2) {
-        const int64_t share = ceil_div(ncols * s * b, 8) * ceil_div(rows, b);
-        if (10 * share < 9 * per_xcd) {
-          per_xcd = share;
-          bands = b;
-        }
-      }
+      const int64_t per_xcd = ceil_div(ncols * s * rows, 8);
       if (s > 1 && per_xcd > 4 * kRoom)
         break;
       const int64_t cps = ceil_div(chunks, s);
@@ -1003,7 +1023,7 @@ TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, bool may_split, dou
       else
         us += norm_us;
       if (!best.gp || us < best.us - 1e-9)
-        best = {gp, s, bands, us};
+        best = {gp, s, us};
     }
   }
   return best;
@@ -1015,10 +1035,8 @@ int launch_plan(const TilePlan &plan, GemmI8Args &a, hipStream_t stream) {
   a.tile_rows = 32 * row_blocks(D, plan.gp);
   a.span = 32 * plan.gp;
   a.row_tiles = (int)ceil_div(a.M, a.tile_rows);
-  a.band_rows = (int)ceil_div(a.row_tiles, plan.bands);
   a.slices = plan.slices;
   a.chunks_per_slice = (int)ceil_div(a.chunks, plan.slices);
-  a.ids_padded = (int)round_up((int64_t)a.ncols * a.slices * plan.bands, 8);
   if (plan.slices > 1) {
     const size_t tile_floats = (size_t)a.tile_rows * kSlices * a.span;
     const size_t bytes = sizeof(float) * tile_floats * plan.slices * (size_t)a.ncols * a.row_tiles;
@@ -1027,7 +1045,11 @@ int launch_plan(const TilePlan &plan, GemmI8Args &a, hipStream_t stream) {
       return rc;
     a.partial = reinterpret_cast<float *>(ws);
   }
-  const unsigned blocks = (unsigned)(a.ids_padded * a.band_rows);
+  const int64_t units = (int64_t)a.ncols * a.slices;
+  a.panel = panel_for(units, a.row_tiles);
+  const int64_t tiles = (a.panel ? units : round_up(units, 8)) * a.row_tiles;
+  BH_REQUIRE(tiles < (1u << 31), "gemm_w8: %lld tiles", (long long)tiles);
+  const unsigned blocks = (unsigned)tiles;
   if (plan.gp == 1)
     return launch_narrow<D, PAIR>(a, blocks, stream);
   return launch_wide<D, PAIR>(a, blocks, stream);
