@@ -28,6 +28,11 @@ struct PromptFold {
   const float *ml = nullptr;    // [slots][256 rows][2]: max (of the scores times log2 e), sum of the weights
   const PromptBlock *blocks = nullptr; // [kv_heads][blocks]
   int group = 0, nblk = 0;
+  // the operands, for rows that are to be computed again (f32_row)
+  const float *q = nullptr, *k = nullptr, *v = nullptr;
+  int64_t q_stride = 0, q_hstride = 0, kv_stride = 0;
+  int q_offset = 0;
+  float scale = 0.f; // of the scores, times log2 e
 };
 
 // Short prompts at the start of a sequence are quicker with attn_prefill.hip, which needs
@@ -49,8 +54,52 @@ int launch_attn_fold_to_digits(const PromptFold &fold, int64_t o_stride, int hea
                                void *staged, hipStream_t stream);
 
 #if defined(__HIPCC__)
-// four values d .. d + 3 of query head h at token t
-__device__ __forceinline__ void folded4(const PromptFold &f, int64_t out_stride, int t, int h, int d,
+// The row of query head h at token t once more, in f32 sums, key after key: 32 lanes that
+// hold four values each from d on.  A row comes to this when its sum of weights is NaN:
+// because it is to be, or because the bfloat16 terms of an operand do not exist (an
+// infinity, a value above the largest bfloat16 one) or of a score leave the range that the
+// score itself is in.  An infinite score of -inf has no weight, and an infinite value makes
+// its own channel infinite, as in the other attention kernels.  (1900 keys: some 0.4 ms.)
+__device__ __forceinline__ void f32_row(const PromptFold &f, int t, int h, int d, float (&v)[4]) {
+#pragma clang fp contract(off) // a score is rounded before the maximum is taken from it
+  const int64_t head = (int64_t)(h / f.group) * f.kv_stride * kPromptD;
+  const float *kp = f.k + head + d, *vp = f.v + head + d;
+  const float4 q = *reinterpret_cast<const float4 *>(f.q + (int64_t)t * f.q_stride +
+                                                     (int64_t)h * f.q_hstride + d);
+  float m = -1.0e30f, l = 0.f;
+  // a NaN in the query row itself: what was left is the result
+  const unsigned long long nan = __ballot(q.x != q.x || q.y != q.y || q.z != q.z || q.w != q.w);
+  if ((nan >> (threadIdx.x & 32)) & 0xffffffffu)
+    return;
+  v[0] = v[1] = v[2] = v[3] = 0.f;
+#pragma unroll 1
+  for (int key = 0; key <= f.q_offset + t; ++key) {
+    const float4 k4 = *reinterpret_cast<const float4 *>(kp + (int64_t)key * kPromptD);
+    const float4 v4 = *reinterpret_cast<const float4 *>(vp + (int64_t)key * kPromptD);
+    float s = fmaf(q.w, k4.w, fmaf(q.z, k4.z, fmaf(q.y, k4.y, q.x * k4.x)));
+#pragma unroll
+    for (int o = 1; o < 32; o <<= 1)
+      s += __shfl_xor(s, o, 64);
+    s *= f.scale;
+    const float mx = fmaxf(m, s), old = __builtin_amdgcn_exp2f(m - mx);
+    const float w = __builtin_amdgcn_exp2f(s - mx);
+    m = mx;
+    l = fmaf(l, old, w);
+    v[0] = fmaf(v4.x, w, v[0] * old);
+    v[1] = fmaf(v4.y, w, v[1] * old);
+    v[2] = fmaf(v4.z, w, v[2] * old);
+    v[3] = fmaf(v4.w, w, v[3] * old);
+    if (l != l) // the same in all lanes of the row
+      break;
+  }
+  const float inv = 1.0f / l;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    v[e] *= inv;
+}
+
+// four values d .. d + 3 of query head h at token t, from where the launch left them
+__device__ __forceinline__ void left4(const PromptFold &f, int64_t out_stride, int t, int h, int d,
                                         float (&v)[4]) {
   const int kvh = h / f.group, row = t * f.group + (h - kvh * f.group);
   const PromptBlock b = f.blocks[kvh * f.nblk + row / kPromptRows];
@@ -105,6 +154,16 @@ __device__ __forceinline__ void folded4(const PromptFold &f, int64_t out_stride,
 #pragma unroll
   for (int e = 0; e < 4; ++e)
     v[e] = s[e] * inv;
+}
+
+// ... finished.  Called by all 32 lanes of a row together, half a wavefront.
+__device__ __forceinline__ void folded4(const PromptFold &f, int64_t out_stride, int t, int h, int d,
+                                        float (&v)[4]) {
+  left4(f, out_stride, t, h, d, v);
+  const float largest = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+  const bool again = !(largest < INFINITY) || v[0] != v[0] || v[1] != v[1] || v[2] != v[2] || v[3] != v[3];
+  if ((__ballot(again) >> (threadIdx.x & 32)) & 0xffffffffu)
+    f32_row(f, t, h, d, v);
 }
 #endif
 

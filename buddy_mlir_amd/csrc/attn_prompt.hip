@@ -233,9 +233,9 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
       x[e] = *reinterpret_cast<const float *>(raw + 2048 + e * 256 + lane * 4);
     const float rest = put_values(x, buf);
     if (rest != rest) {
-      // A value that is not finite must not reach rows that do not see its key, whose
+      // A value that has no terms must not reach rows that do not see its key, whose
       // weight there is zero: it goes in as zero, and its key makes NaN of the rows that
-      // do see it (see add_values).
+      // do see it (see add_values), which the fold then computes again.
 #pragma unroll
       for (int e = 0; e < 8; ++e)
         if (!(fabsf(x[e]) < 3.3895e38f)) {
@@ -533,6 +533,14 @@ int launch_attn_prompt(const AttnPrefillArgs &in, void *workspace, PromptFold &f
   fold.blocks = a.blocks;
   fold.group = a.group;
   fold.nblk = a.nblk;
+  fold.q = a.q;
+  fold.k = a.k;
+  fold.v = a.v;
+  fold.q_stride = a.q_stride;
+  fold.q_hstride = a.q_hstride;
+  fold.kv_stride = a.kv_stride;
+  fold.q_offset = a.q_offset;
+  fold.scale = a.scale;
   return BUDDY_HIP_OK;
 }
 

@@ -8,7 +8,7 @@ import torch
 
 import buddy_mlir_amd as bma
 from buddy_mlir_amd import ops, synthetic
-from buddy_mlir_amd.session import Shape
+from buddy_mlir_amd.session import DecoderSession, Shape
 from parity import check_close
 from test_gpu_decode import SMALL, oracle_model
 
@@ -424,9 +424,8 @@ def test_prompt_attention_equals_token_by_token(heads, kv_heads, before, n):
 
 @pytest.mark.parametrize("bad", [float("nan"), float("inf")])
 def test_prompt_attention_keeps_non_finite_tokens_from_earlier_rows(bad):
-    """A token in the middle of a long prompt whose embedding is not finite, and a cache row
-    whose values are not: rows that do not see them are what they are without, bit for bit;
-    rows that do are NaN."""
+    """A token in the middle of a long prompt whose embedding is not finite: rows that do not
+    see it are what they are without, bit for bit; rows that do are NaN."""
     shape = Shape(layers=2, hidden=256, heads=6, kv_heads=1, head_dim=128, inter=256, vocab=320,
                   max_len=720)
     toks = (synthetic.first_tokens(shape, 700, seed=1) % 300).astype(np.int32)
@@ -446,6 +445,89 @@ def test_prompt_attention_keeps_non_finite_tokens_from_earlier_rows(bad):
         np.testing.assert_array_equal(got[:at], want[:at])
         assert np.isnan(got[at:]).any(axis=1).all()
     sess.close()
+
+
+@pytest.mark.parametrize("precision", ["digits", "exact"])
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), 3.4e38])
+def test_prompt_attention_of_a_key_beyond_bfloat16(bad, precision):
+    """A cached key with one channel infinite, or larger than any bfloat16 value: a row of
+    whose query that channel is negative gives it a score of -inf and no weight.  Finite and
+    non-finite rows are those of the decode step, whose attention is another kernel."""
+    before, n = 200, 150
+    shape = Shape(layers=2, hidden=256, heads=1, kv_heads=1, head_dim=128, inter=256, vocab=320,
+                  max_len=before + n + 8)
+    toks = synthetic.first_tokens(shape, n, seed=3).astype(np.int32)
+    rows = []
+    for by_token in (False, True):
+        sess, _ = synthetic.build_session(shape, context=before, ln_jitter=0.1)
+        k = sess.get_kv(0)
+        k[0, 77, 9] = bad
+        sess.set_kv(0, k)
+        if by_token:
+            for i, t in enumerate(toks):
+                sess.decode(int(t), before + i, want_logits=False)
+        else:
+            sess.prefill(toks, before, precision=precision)
+        rows.append([sess.get_kv(j)[0, before:before + n] for j in (2, 3)])
+        sess.close()
+    for got, want in zip(*rows):
+        finite = np.isfinite(want).all(axis=1)
+        assert finite.sum() > n // 4
+        if np.isinf(bad):
+            assert (~finite).sum() > n // 4
+        assert not np.isfinite(got[~finite]).all(axis=1).any()
+        check_close(got[finite], want[finite])
+
+
+@pytest.mark.parametrize("at", [0, 3, 4, 15, 16, 31, 63, 70])
+@pytest.mark.parametrize("size", [3.4e38, 8e38])  # above the largest bfloat16 value; infinite
+def test_prompt_attention_of_a_value_beyond_bfloat16(at, size):
+    """One channel of one token's value is huge or infinite, its key is not: rows ahead of
+    the token are what they are without, bit for bit, also in its tile of 32 keys.  Behind it
+    a huge value changes its own channel alone (o_proj takes nothing from that channel, and
+    the other channels give what they give without it); an infinite one makes NaN of 0 * inf."""
+    before, n, c, big = 128, 96, 5, 310
+    shape = Shape(layers=2, hidden=256, heads=2, kv_heads=1, head_dim=128, inter=256, vocab=320,
+                  max_len=before + n + 8)
+
+    def session(factor):
+        sess = DecoderSession(shape)
+        g = synthetic.make_globals(shape)
+        g["embed"][:, 0] = 0.0
+        g["embed"][big, 0] = 0.05
+        sess.set_globals(g["embed"], g["inv_freq"], g["ln_f"], g["w_lm"], g["s_lm"])
+        for i in range(shape.layers):
+            w = synthetic.make_layer(shape, i, 0.1)
+            if i == 0:  # channel c of the values is that of the big token's embedding, or 0
+                w["wv"][:, c] = 0
+                w["wv"][0, c] = 100
+                w["sv"][c] = factor
+                w["wo"][c::128] = 0
+            sess.set_layer(i, w)
+        for j in range(2 * shape.layers):
+            sess.set_kv(j, synthetic.make_kv(shape, j, before))
+        torch.cuda.synchronize()
+        return sess
+
+    toks = (synthetic.first_tokens(shape, n, seed=5) % 300).astype(np.int32)
+    toks[at] = big
+    rows, factor = [], 1.0
+    for want_size in (None, size):
+        sess = session(factor)
+        sess.prefill(toks, before, precision="exact")
+        rows.append([sess.get_kv(j)[0, before:before + n] for j in (2, 3)])
+        value = abs(float(sess.get_kv(1)[0, before + at, c]))
+        if want_size is None:
+            factor = size / value
+        else:
+            assert np.isinf(value) if size > 3.5e38 else 3.3962e38 < value < np.inf
+        sess.close()
+    for want, got in zip(*rows):
+        np.testing.assert_array_equal(got[:at], want[:at])
+        if size > 3.5e38:
+            assert not np.isfinite(got[at:]).all(axis=1).any()
+        else:
+            check_close(got[at:], want[at:])
 
 
 def test_wide_hidden_size_through_the_slice_adding_norm_kernel(oracle):
