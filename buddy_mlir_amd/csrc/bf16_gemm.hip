@@ -326,6 +326,22 @@ __device__ __forceinline__ void split3(uint4 v, uint2 (&out)[3]) {
                    __builtin_amdgcn_perm(t[p][3], t[p][2], 0x07060302u)};
 }
 
+// one row times one channel in f32, until the sum is NaN; w: the channel's runs of 8 k, 16
+// runs apart
+__device__ __forceinline__ float f32_sum(const float *x, const uint4 *w, int K) {
+  float sum = 0.f;
+#pragma unroll 1
+  for (int k = 0; k < K && sum == sum; k += 8) {
+    const uint4 q = w[k / 8 * 16];
+    const unsigned d[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (k + e < K)
+        sum = fmaf(x[k + e], e & 1 ? bf_hi(d[e / 2]) : bf_lo(d[e / 2]), sum);
+  }
+  return sum;
+}
+
 __device__ __forceinline__ f32x16 mfma_bf16_wide(uint4 a, uint4 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
                                                  __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
@@ -513,6 +529,38 @@ rows_gemm_wide_kernel(const uint4 *__restrict__ W, int ktiles, int steps, GemmDe
     const int lr = row0 + r * 32 + (lane & 31);
     if (lr >= rows)
       continue;
+    if constexpr (kTerms > 1) {
+      // An infinite weight times a term that is zero is NaN where the f32 product is
+      // infinite: what came out as NaN is added up again without terms.
+      bool nan = false;
+#pragma unroll
+      for (int n = 0; n < GT * 16; ++n)
+        nan |= acc[n / 16][r][n % 16] != acc[n / 16][r][n % 16];
+      if (nan) {
+        int pr;
+        if constexpr (GROUPED)
+          pr = list[lr] / a.list_div;
+        else
+          pr = (a.ring_base + lr) & a.ring_mask;
+        const float *x = static_cast<const float *>(a.A) + (int64_t)pr * a.lda;
+#pragma unroll 1
+        for (int n = 0; n < GT * 16; ++n) {
+          float v = 0.f;
+#pragma unroll
+          for (int i = 0; i < GT * 16; ++i)
+            v = i == n ? acc[i / 16][r][i % 16] : v;
+          const int tile = n / 16, of = 8 * (n % 16 / 4) + (lane >> 5) * 4 + n % 4; // of 32 channels
+          const int group = ch0 + 2 * (kPair ? tile % kTilesOut : tile) + of / 16;
+          if (v == v || group >= a.groups)
+            continue;
+          const uint4 *w = W + ((int64_t)((kPair ? tile / kTilesOut : 0) * a.groups + group) * ktiles) * 64 + of % 16;
+          v = f32_sum(x, w, a.K);
+#pragma unroll
+          for (int i = 0; i < GT * 16; ++i)
+            acc[i / 16][r][i % 16] = i == n ? v : acc[i / 16][r][i % 16];
+        }
+      }
+    }
     int orow = lr;
     if constexpr (GROUPED)
       orow = list[lr];

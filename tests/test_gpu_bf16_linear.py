@@ -146,6 +146,39 @@ def test_f32_rows_keep_every_bit_and_their_infinities(bh):
             np.testing.assert_array_equal(got[7], bad * np.sign(b[:, 30]))
 
 
+@pytest.mark.parametrize("M,K,Nout", [(17, 96, 33), (40, 100, 130), (33, 1000, 8200)])
+def test_f32_rows_times_infinite_weights(bh, M, K, Nout):
+    """An infinite weight makes its channel infinite with the sign of the product, whatever
+    terms the row's value has; NaN beside another infinity or a row's zero.  Every other
+    channel is what it is without."""
+    rng = np.random.default_rng(K)
+    w = N.bf16(rng.standard_normal((Nout, K)))
+    a = rng.standard_normal((M, K)).astype(np.float32)
+    a[::2] = N.bf16(a[::2])   # one term
+    a[1, 50] = 0.0
+    w[7, 50], w[20, 90], w[Nout - 1, K - 1] = np.inf, -np.inf, np.inf
+    w[21, 3], w[21, 4] = np.inf, np.inf  # +-inf or NaN, by the signs of two values
+    dev = torch.from_numpy(N.to_bf16_bits(w).view(np.int16)).cuda()
+    tiles = torch.empty(bh.buddy_hip_bf16_tiles_bytes(K, Nout), dtype=torch.uint8, device="cuda")
+    lda, ldc = (K + 7) // 8 * 8, (Nout + 15) // 16 * 16
+    buf = np.full((M, lda), np.nan, np.float32)
+    buf[:, :K] = a
+    A, C = torch.from_numpy(buf).cuda(), torch.empty((M, ldc), device="cuda")
+    torch.cuda.synchronize()
+    assert bh.buddy_hip_pack_bf16_tiles(dev.data_ptr(), K, Nout, tiles.data_ptr(), None) == 0
+    assert bh.buddy_hip_gemm_bf16(A.data_ptr(), lda, 1, tiles.data_ptr(), C.data_ptr(), ldc,
+                                  M, K, Nout, None) == 0
+    torch.cuda.synchronize()
+    got = C.cpu().numpy()[:, :Nout]
+    with np.errstate(invalid="ignore"):
+        want = a.astype(np.float64) @ w.astype(np.float64).T
+    assert np.isnan(want).any() and np.isinf(want).any()
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    fin = np.isfinite(want)
+    assert np.abs(got[fin] - want[fin]).max() < 3e-6 * np.abs(want[fin]).max()
+
+
 @pytest.mark.parametrize("K,Nout", [(64, 16), (1, 3), (37, 50), (2048, 96), (2052, 70), (4100, 33),
                                     (8200, 17), (9001, 20), (1536, 40000), (300, 4100)])
 def test_one_row(bh, K, Nout):
