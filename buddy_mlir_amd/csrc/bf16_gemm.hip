@@ -68,8 +68,8 @@ template <> __device__ __forceinline__ void store4<bf16_bits>(bf16_bits *p, f32x
 // runs at the same time share rows and channels.  Of experts' tiles the die takes a run of
 // row blocks too, so that an expert's weights come to one or two L2s and not to all eight.
 constexpr int kDies = 8, kPanel = 4;
-__device__ __forceinline__ void place_tile(int gy, int &bx, int &by) {
-  const int gx = gridDim.x, total = gx * gy, id = blockIdx.y * gx + blockIdx.x;
+__device__ __forceinline__ void place_tile(int gx, int gy, int &bx, int &by) {
+  const int total = gx * gy, id = blockIdx.y * gx + blockIdx.x;
   const int die = id % kDies, q = total / kDies, r = total % kDies;
   const int t = die * q + min(die, r) + id / kDies;
   const int panel = t / (kPanel * gy), rest = t - panel * kPanel * gy;
@@ -115,7 +115,7 @@ __device__ __forceinline__ int find_expert(const int *counts, int experts, int r
 
 template <typename T, int RT, int GT, int OUT, bool GROUPED>
 __global__ void __launch_bounds__(kGemmThreads)
-rows_gemm_kernel(const uint4 *__restrict__ W, int ktiles, int steps, GemmDev a) {
+rows_gemm_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int columns, int row_blocks, GemmDev a) {
   using Tr = ActTraits<T>;
   constexpr bool kPair = OUT == kOutExpertAct;
   constexpr int kGroups = kPair ? GT / 2 : GT; // channel groups of the result per wavefront
@@ -126,18 +126,21 @@ rows_gemm_kernel(const uint4 *__restrict__ W, int ktiles, int steps, GemmDev a) 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-  int bx = blockIdx.x, by = blockIdx.y;
-  if constexpr (!GROUPED)
-    place_tile(gridDim.y, bx, by);
+  int bx, by;
+  if constexpr (GROUPED) {
+    const int id = blockIdx.y * columns + blockIdx.x;
+    by = id / columns; // counts the row blocks of all experts
+    bx = id - by * columns;
+  } else {
+    place_tile(columns, row_blocks, bx, by);
+  }
   int row0 = by * kRows, rows = a.rows;
   const int *list = nullptr;
   if constexpr (GROUPED) {
-    // blockIdx.y counts the row blocks of all experts
-    int block = blockIdx.y;
-    const int e = find_expert(a.counts, a.experts, kRows, lane, block);
+    const int e = find_expert(a.counts, a.experts, kRows, lane, by);
     if (e < 0)
       return; // more workgroups than row blocks
-    row0 = block * kRows;
+    row0 = by * kRows;
     rows = a.counts[e];
     list = a.lists + (int64_t)e * a.list_cap;
     W += (int64_t)e * a.expert_tiles * 64;
@@ -351,7 +354,8 @@ constexpr int kWideK = 64; // k per step
 
 template <typename T, int RT, int GT, int OUT, bool GROUPED>
 __global__ void __launch_bounds__(kGemmThreads)
-rows_gemm_wide_kernel(const uint4 *__restrict__ W, int ktiles, int steps, GemmDev a) {
+rows_gemm_wide_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int columns, int row_blocks,
+                      GemmDev a) {
   constexpr bool kPair = OUT == kOutExpertAct;
   constexpr int kTilesOut = kPair ? GT / 2 : GT; // 32-channel tiles of the result per wavefront
   constexpr int kTerms = sizeof(T) == 4 ? 3 : 1;
@@ -365,24 +369,24 @@ rows_gemm_wide_kernel(const uint4 *__restrict__ W, int ktiles, int steps, GemmDe
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-  int bx = blockIdx.x, by = blockIdx.y;
+  int bx, by;
   if constexpr (!GROUPED)
-    place_tile(gridDim.y, bx, by);
-  int row0 = by * kRows, rows = a.rows;
+    place_tile(columns, row_blocks, bx, by);
+  int row0, rows = a.rows;
   const int *list = nullptr;
   if constexpr (GROUPED) {
     const int blocks = count_blocks(a.counts, a.experts, kRows, lane);
-    if ((int)(blockIdx.y * gridDim.x + blockIdx.x) >= blocks * (int)gridDim.x)
+    if ((int)(blockIdx.y * columns + blockIdx.x) >= blocks * columns)
       return; // more workgroups than tiles
-    place_tile(blocks, bx, by);
+    place_tile(columns, blocks, bx, by);
     const int e = find_expert(a.counts, a.experts, kRows, lane, by);
     if (e < 0)
       return;
-    row0 = by * kRows;
     rows = a.counts[e];
     list = a.lists + (int64_t)e * a.list_cap;
     W += (int64_t)e * a.expert_tiles * 64;
   }
+  row0 = by * kRows;
 
   // the runs this thread moves: fixed rows, k advancing by the step
   const T *src[kLoads];
@@ -532,11 +536,11 @@ rows_gemm_wide_kernel(const uint4 *__restrict__ W, int ktiles, int steps, GemmDe
     if constexpr (kTerms > 1) {
       // An infinite weight times a term that is zero is NaN where the f32 product is
       // infinite: what came out as NaN is added up again without terms.
-      bool nan = false;
+      float most = acc[0][r][0]; // NaN if one of them is
 #pragma unroll
-      for (int n = 0; n < GT * 16; ++n)
-        nan |= acc[n / 16][r][n % 16] != acc[n / 16][r][n % 16];
-      if (nan) {
+      for (int n = 1; n < GT * 16; ++n)
+        most = __builtin_elementwise_maximum(most, acc[n / 16][r][n % 16]);
+      if (most != most) {
         int pr;
         if constexpr (GROUPED)
           pr = list[lr] / a.list_div;
@@ -622,10 +626,14 @@ int launch_tiles(F kernel, int elems, const RowsGemm &a, hipStream_t stream) {
   const int64_t blocks = GROUPED ? std::min<int64_t>(ceil_div(a.list_total, ROWS) + a.experts,
                                                      a.list_total)
                                  : ceil_div(a.rows, ROWS);
-  BH_REQUIRE(blocks <= 65535, "rows_gemm: %lld row blocks", (long long)blocks);
-  hipLaunchKernelGGL(kernel,
-                     dim3((unsigned)ceil_div(d.groups * 16, CHANNELS), (unsigned)blocks), dim3(kGemmThreads),
-                     0, stream, a.W.tiles, a.W.ktiles, (int)ceil_div(a.W.K, elems), d);
+  const int64_t columns = ceil_div(d.groups * 16, CHANNELS);
+  BH_REQUIRE(blocks * columns < (int64_t)1 << 31, "rows_gemm: %lld row blocks", (long long)blocks);
+  // The second dimension of a grid ends at 65535 (2.1 million rows in tiles of 32): then all
+  // in the first.  (Always so, launches of 4 us took 0.2 longer.)
+  const dim3 grid = blocks <= 65535 ? dim3((unsigned)columns, (unsigned)blocks)
+                                    : dim3((unsigned)(blocks * columns));
+  hipLaunchKernelGGL(kernel, grid, dim3(kGemmThreads), 0, stream, a.W.tiles,
+                     a.W.ktiles, (int)ceil_div(a.W.K, elems), (int)columns, (int)blocks, d);
   BH_CHECK_HIP(hipGetLastError());
   return BUDDY_HIP_OK;
 }

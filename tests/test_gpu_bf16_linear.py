@@ -146,6 +146,21 @@ def test_f32_rows_keep_every_bit_and_their_infinities(bh):
             np.testing.assert_array_equal(got[7], bad * np.sign(b[:, 30]))
 
 
+@pytest.mark.parametrize("dtype,M", [(1, 2_100_000), (0, 4_200_000)])
+def test_more_row_blocks_than_a_grid_dimension_has(bh, dtype, M):
+    K, Nout = 8, 16
+    w, tiles = make(bh, K, Nout, 9)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    A = torch.randn((M, K), generator=g, device="cuda").to(torch.float32 if dtype else torch.bfloat16)
+    C = torch.zeros((M, Nout), device="cuda")
+    torch.cuda.synchronize()
+    assert bh.buddy_hip_gemm_bf16(A.data_ptr(), K, dtype, tiles.data_ptr(), C.data_ptr(), Nout,
+                                  M, K, Nout, None) == 0
+    torch.cuda.synchronize()
+    want = A.double() @ torch.from_numpy(w).cuda().T
+    assert float((C - want).abs().max()) < 3e-6 * float(want.abs().max())
+
+
 @pytest.mark.parametrize("M,K,Nout", [(17, 96, 33), (40, 100, 130), (33, 1000, 8200)])
 def test_f32_rows_times_infinite_weights(bh, M, K, Nout):
     """An infinite weight makes its channel infinite with the sign of the product, whatever
