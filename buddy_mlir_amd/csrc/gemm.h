@@ -81,7 +81,9 @@ int launch_gemm_w8a8_plane(const void *plane, const int8_t *W, const float *wsca
                            hipStream_t stream);
 
 // split-K workspace of the int8 and bf16 matmuls, one grow-only buffer per stream (dropped
-// together with the staging)
+// together with the staging).  While the stream is being captured it does not grow: then
+// *out is null where it is too small, and the caller leaves K whole.  A buffer that a capture
+// was given stays until the release.
 int gemm_slices_workspace(hipStream_t stream, size_t bytes, char **out);
 void release_gemm_i8_workspace(hipStream_t stream);
 

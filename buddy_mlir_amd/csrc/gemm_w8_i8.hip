@@ -36,6 +36,7 @@
 #include <cstdlib>
 #include <map>
 #include <mutex>
+#include <vector>
 
 namespace bh {
 namespace {
@@ -945,25 +946,47 @@ namespace {
 struct Workspace {
   char *ptr = nullptr;
   size_t bytes = 0;
+  bool recorded = false;    // a capture was given ptr
+  std::vector<char *> held; // outgrown ones that captures were given
 };
 std::mutex g_workspace_mutex;
 std::map<hipStream_t, Workspace> g_workspace;
+
+bool captures(hipStream_t stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return status != hipStreamCaptureStatusNone;
+}
 
 } // namespace
 
 int gemm_slices_workspace(hipStream_t stream, size_t bytes, char **out) {
   std::lock_guard<std::mutex> lock(g_workspace_mutex);
   Workspace &w = g_workspace[stream];
+  const bool capturing = captures(stream);
+  *out = nullptr;
   if (w.bytes < bytes) {
-    if (w.ptr) {
+    if (capturing)
+      return BUDDY_HIP_OK;
+    if (w.ptr && w.recorded) {
+      // a graph may hold it; at least twice as much next, so that all that are held
+      // together stay below the one in use
+      bytes = std::max(bytes, 2 * w.bytes);
+      w.held.push_back(w.ptr);
+    } else if (w.ptr) {
       BH_CHECK_HIP(hipStreamSynchronize(stream)); // an earlier matmul may still use it
       BH_CHECK_HIP(hipFree(w.ptr));
-      w.ptr = nullptr;
-      w.bytes = 0;
     }
+    w.ptr = nullptr;
+    w.bytes = 0;
+    w.recorded = false;
     BH_CHECK_HIP(hipMalloc(reinterpret_cast<void **>(&w.ptr), bytes));
     w.bytes = bytes;
   }
+  w.recorded |= capturing;
   *out = w.ptr;
   return BUDDY_HIP_OK;
 }
@@ -1029,6 +1052,8 @@ TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, bool may_split, dou
   return best;
 }
 
+// a.partial stays null where K was to be split and no workspace could be had: the caller
+// comes back with a plan that leaves K whole.
 template <int D, bool PAIR>
 int launch_plan(const TilePlan &plan, GemmI8Args &a, hipStream_t stream) {
   a.ncols = (int)ceil_div(a.N, kSlices * (PAIR ? 16 : 32) * plan.gp);
@@ -1043,6 +1068,8 @@ int launch_plan(const TilePlan &plan, GemmI8Args &a, hipStream_t stream) {
     char *ws = nullptr;
     if (int rc = gemm_slices_workspace(stream, bytes, &ws))
       return rc;
+    if (!ws)
+      return BUDDY_HIP_OK;
     a.partial = reinterpret_cast<float *>(ws);
   }
   const int64_t units = (int64_t)a.ncols * a.slices;
@@ -1062,10 +1089,13 @@ void release_gemm_i8_workspace(hipStream_t stream) {
   auto it = g_workspace.find(stream);
   if (it == g_workspace.end())
     return;
-  if (it->second.ptr) {
+  Workspace &w = it->second;
+  if (w.ptr || !w.held.empty())
     (void)hipStreamSynchronize(stream);
-    (void)hipFree(it->second.ptr);
-  }
+  if (w.ptr)
+    (void)hipFree(w.ptr);
+  for (char *p : w.held)
+    (void)hipFree(p);
   g_workspace.erase(it);
 }
 
@@ -1116,9 +1146,14 @@ int launch_gemm_w8_digits_d(const GemmW8Args &in, const void *planes, hipStream_
     return launch_rmsnorm_to_digits(in.C, in.ldc, in.then_norm_w, (int)in.M, (int)in.N,
                                     in.then_norm_eps, in.digits, in.then_norm_staged, stream);
   };
-  const TilePlan plan = plan_tiles<D, false>(in.M, in.N, a.chunks, true, pending_norm, 0);
+  TilePlan plan = plan_tiles<D, false>(in.M, in.N, a.chunks, true, pending_norm, 0);
   if (int rc = launch_plan<D, false>(plan, a, stream))
     return rc;
+  if (plan.slices > 1 && !a.partial) {
+    plan = plan_tiles<D, false>(in.M, in.N, a.chunks, false, pending_norm, 0);
+    if (int rc = launch_plan<D, false>(plan, a, stream))
+      return rc;
+  }
   if (plan.slices == 1)
     return then_norm();
   const GemmStagingLayout next = gemm_staging_layout(in.M, in.N);
@@ -1184,10 +1219,16 @@ int launch_gemm_w8a8_plane(const void *plane, const int8_t *W, const float *wsca
   // sums in the workspace (f32 ones would round above 2^24) and a second kernel
   // adds them exactly
   const int64_t reduce_wgs = ceil_div(M * ceil_div(N, 4), 256);
-  const TilePlan plan = plan_tiles<1, false>(M, N, a.chunks, true, 0.0, reduce_wgs);
+  TilePlan plan = plan_tiles<1, false>(M, N, a.chunks, true, 0.0, reduce_wgs);
   a.int_partials = plan.slices > 1;
   if (int rc = launch_plan<1, false>(plan, a, stream))
     return rc;
+  if (plan.slices > 1 && !a.partial) {
+    plan = plan_tiles<1, false>(M, N, a.chunks, false, 0.0, reduce_wgs);
+    a.int_partials = 0;
+    if (int rc = launch_plan<1, false>(plan, a, stream))
+      return rc;
+  }
   if (plan.slices > 1) {
     hipLaunchKernelGGL(reduce_slices_i32_kernel, dim3((unsigned)reduce_wgs), dim3(256), 0, stream,
                        a);

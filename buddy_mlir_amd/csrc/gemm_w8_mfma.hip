@@ -542,7 +542,7 @@ struct TilePlan {
   int gp = 0, slices = 1;
   double us = 0;
 };
-TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, int terms) {
+TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, int terms, bool may_split) {
   TilePlan best;
   for (int gp = 1; gp <= 2; ++gp) {
     const int layers = terms * row_blocks(terms, gp);
@@ -550,7 +550,7 @@ TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, int terms) {
     const int64_t ncols = ceil_div(channels, kWaves * 32 * gp);
     const double alone = gp == 2 ? 0.34 + 0.16 * layers : 0.20 + 0.075 * layers;
     const double full = gp == 2 ? 0.14 + 0.38 * layers : 0.24 + 0.21 * layers;
-    for (int s = 1; s <= 16; ++s) {
+    for (int s = 1; s <= (may_split ? 16 : 1); ++s) {
       const int64_t per_xcd = ceil_div(ncols * s, 8) * rows;
       if (s > 1 && per_xcd > 256)
         break;
@@ -587,6 +587,8 @@ int launch_plan(const TilePlan &plan, GemmArgs &a, int terms, hipStream_t stream
     if (int rc = gemm_slices_workspace(
             stream, sizeof(float) * tile_floats * a.slices * (size_t)a.ncols * a.row_tiles, &ws))
       return rc;
+    if (!ws) // under capture: K whole
+      return launch_plan(plan_tiles(a.M, a.N, a.chunks, terms, false), a, terms, stream);
     a.partial = reinterpret_cast<float *>(ws);
   }
   const unsigned blocks = (unsigned)a.ids_padded * a.row_tiles;
@@ -707,7 +709,7 @@ int launch_gemm_w8(const GemmW8Args &in, hipStream_t stream) {
                        in.terms, abf);
     BH_CHECK_HIP(hipGetLastError());
   }
-  return launch_plan(plan_tiles(in.M, in.N, a.chunks, in.terms), a, in.terms, stream);
+  return launch_plan(plan_tiles(in.M, in.N, a.chunks, in.terms, true), a, in.terms, stream);
 }
 
 void release_gemm_staging(hipStream_t stream) {

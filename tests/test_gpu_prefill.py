@@ -225,6 +225,56 @@ def test_prefill_gemm_silu_pair_refusals(bh):
     torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("mode", ["bf16", "exact", "digits", "digits2"])
+def test_captured_matmul_keeps_its_workspace(mode):
+    """A stream that ran its largest product can record a smaller one, whose K slices may
+    want more workspace (then K stays whole); eager products that want more afterwards leave
+    the recorded one its buffer."""
+    K, N = 8960, 1536
+    kw = dict(exact=mode == "exact", digits={"digits": 3, "digits2": 2}.get(mode, False))
+    q, s = synthetic.quantized_linear(K, N, 5)
+    packed = ops.pack_w8(q)
+    x = torch.randn((1931, K), generator=torch.Generator(device="cuda").manual_seed(2), device="cuda")
+    w64 = q.double() * s.double()
+    more = [(n, ops.pack_w8(torch.cat([q] * (n // N), 1).contiguous()), torch.cat([s] * (n // N)))
+            for n in (3072, 4608, 6144)]
+    stream = torch.cuda.Stream()
+    outs = {M: torch.empty((M, N), device="cuda") for M in (400, 300, 100)}
+    with torch.cuda.stream(stream):
+        ops.gemm_w8a32(x, packed, s, K, N, **kw)
+    torch.cuda.synchronize()
+    graphs = []
+    for M, out in outs.items():
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=stream):
+            ops.gemm_w8a32(x[:M], packed, s, K, N, out=out, **kw)
+        graphs.append(g)
+        with torch.cuda.stream(stream):  # eager: the next capture finds its workspace
+            ops.gemm_w8a32(x[:M], packed, s, K, N, **kw)
+        torch.cuda.synchronize()
+    xh = x[:400].double()
+    if mode == "bf16":
+        xh = x[:400].bfloat16().double()
+    elif mode == "digits2":
+        xh = torch.from_numpy(fixed_point_round(x[:400].cpu().numpy(), 2)[0]).cuda().double()
+    want = xh @ w64
+    first = {}
+    for turn in range(4):
+        for (M, out), g in zip(outs.items(), graphs):
+            out.fill_(7.0)
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            first.setdefault(M, out.clone())
+            assert torch.equal(out, first[M])
+            err = float((out - want[:M]).abs().max())
+            assert err < 2e-5 * float(want.abs().max()), (M, err)
+        n, p, sc = more[turn % 3]
+        with torch.cuda.stream(stream):
+            ops.gemm_w8a32(x[:300 + 100 * turn], p, sc, K, n, **kw)
+        torch.cuda.synchronize()
+
+
 @pytest.mark.parametrize("exact", [True, False])
 @pytest.mark.parametrize("M,K,N", [(100, 256, 96), (490, 136, 6600)])
 def test_prefill_gemm_accumulates(oracle, M, K, N, exact):
