@@ -313,9 +313,10 @@ template <int D> __device__ __forceinline__ float scaled(float v, float step, fl
 // other; a tile is a group of the first and the same group of the second, so that a lane
 // holds matching channels of both, and the result is SiLU(first) * second ([M, N / 2]).
 typedef int v16i32 __attribute__((ext_vector_type(16)));
-// Blocks of 32 rows per workgroup: the weights of 256 channels are used for three layers of
-// 32 rows or more (one plane of one block: 512 rows, 1536 -> 8960, 31.2 us; of three 18.6).
-constexpr int row_blocks(int D, int gp) { return D == 1 && gp == 2 ? 3 : 1; }
+// Blocks of 32 rows of the tile of 256 channels that every launch of some size can use (of
+// one plane, whose weights are otherwise used for too little: 512 rows, 1536 -> 8960, 31.2 us
+// on blocks of one; of two 26, of three 25).
+constexpr int wide_blocks(int D) { return D == 1 ? 2 : 1; }
 constexpr int kWideRow = kTileK + 16; // bytes of a row in LDS: fragment reads meet every bank once
 
 // Ids equal modulo 8 run on the same XCD.  An XCD takes a run of an eighth of all tiles, in
@@ -670,7 +671,7 @@ __device__ __forceinline__ void multiply_tile(const GemmI8Args &a) {
   a.row_tiles = row_tiles;                                                                         \
   a.panel = panel;
 
-// 128 channels per workgroup, and 256
+// 32 rows x 128 channels per workgroup; 256 channels; the others of kTiles
 template <int D, bool PAIR>
 __global__ void __launch_bounds__(kSlices *kWave) gemm_w8_i8_kernel(BH_I8_LEADING) {
   BH_I8_TAKE
@@ -679,7 +680,12 @@ __global__ void __launch_bounds__(kSlices *kWave) gemm_w8_i8_kernel(BH_I8_LEADIN
 template <int D, bool PAIR>
 __global__ void __launch_bounds__(kSlices *kWave) gemm_w8_i8_wide_kernel(BH_I8_LEADING) {
   BH_I8_TAKE
-  multiply_tile<D, row_blocks(D, 2), 2, PAIR>(a);
+  multiply_tile<D, wide_blocks(D), 2, PAIR>(a);
+}
+template <int D, int RB, int GP, bool PAIR>
+__global__ void __launch_bounds__(kSlices *kWave) gemm_w8_i8_tall_kernel(BH_I8_LEADING) {
+  BH_I8_TAKE
+  multiply_tile<D, RB, GP, PAIR>(a);
 }
 
 // Where the sums of row m, channels n.. of the first K slice lie.
@@ -856,6 +862,7 @@ reduce_slices_norm_kernel(const float *p_partial, const float *p_steps, int p_N,
 BH_VARIANT_FAMILY(WideFamily, "gemm_w8_i8_wide_kernel");
 BH_VARIANT_FAMILY(NarrowFamily, "gemm_w8_i8_kernel");
 BH_TILE_FAMILY(NarrowPairFamily, "gemm_w8_i8_kernel pair");
+BH_TILE_FAMILY(TallFamily, "gemm_w8_i8_tall_kernel");
 
 template <class Kernel>
 int launch_tiles(Kernel kernel, const GemmI8Args &a, unsigned blocks, hipStream_t stream) {
@@ -879,6 +886,12 @@ int launch_narrow(const GemmI8Args &a, unsigned blocks, hipStream_t stream) {
   else
     BH_NOTE_VARIANT(NarrowFamily, D);
   return launch_tiles(gemm_w8_i8_kernel<D, PAIR>, a, blocks, stream);
+}
+
+template <int D, int RB, int GP, bool PAIR>
+int launch_tall(const GemmI8Args &a, unsigned blocks, hipStream_t stream) {
+  BH_NOTE_VARIANT(TallFamily, D, RB, GP, (int)PAIR);
+  return launch_tiles(gemm_w8_i8_tall_kernel<D, RB, GP, PAIR>, a, blocks, stream);
 }
 
 } // namespace
@@ -993,62 +1006,93 @@ int gemm_slices_workspace(hipStream_t stream, size_t bytes, char **out) {
 
 namespace {
 
-// Channel tiles per wavefront and K slices for a launch, by an estimate of its time in
-// microseconds.  An XCD (32 compute units) works on 64 workgroups at a time, two
-// to a compute unit.  A chunk of 64 k on L layers of 32 rows (planes, blocks of rows) takes
-// a compute unit with two workgroups 0.18 + 0.16 L us, one that has its compute unit to
-// itself 0.15 + 0.08 L us (with one channel tile 0.2 + 0.085 L and 0.06 + 0.07 L, at least
-// 0.21: the way through LDS); a last round that fills less than half runs at the latter.
-// Fitted to these, microseconds (three planes; two; in brackets 16 x 16 x 64 instructions
-// on tiles of 32 or 64 rows x 128 or 256 channels):
-//   gate | up, 1536 -> 2 x 8960: 27 rows 11.2 [18.4]; 10.0 [15.0], 256: 32.6 [30.6]; 27.3
-//     [23.3], 512: 52.3 [58.8]; 42.7 [44.3], 1931: 180 [201]; 141 [150]
+// Tile and K slices for a launch, by an estimate of its time in microseconds.  An XCD (32
+// compute units) works on 64 workgroups at a time, two to a compute unit, or on 32 where a
+// tile's registers leave room for one.  A chunk of 64 k takes a workgroup that has its
+// compute unit to itself `alone`, two that share one `both`, each beside a fixed part; a last
+// round that fills less than half runs at the former.  Fitted to launches of 32 to 4096 rows
+// of 1536, 4096, 8960 and 14336 k.  Microseconds, with the tiles of 256 channels beside them
+// (in brackets 16 x 16 x 64 instructions on tiles of 48 or 64 rows x 256 or 320 channels):
+//   gate | up, 1536 -> 2 x 8960, three planes; two: 27 rows 11.2 [18.4]; 10.0 [15.0], 256:
+//     28 (32.6) [30.6]; 22 (27.3) [23.3], 512: 52 [58.8]; 38 (42.7) [44.3], 1931: 173 [201]; 130
+//     (136) [150]
 //   down, 8960 -> 1536, with the adding of its slices: 27 rows 12.7 [16.9]; 11.1 [15.1],
-//     512: 34 [36]; 29 [28], 1931: 96 [112]; 77 [95]
+//     512: 34 [36]; 28 [28], 1931: 90 (96) [112]; 72 (77) [95]
 //   q|k|v, 1536 -> 2048: 100 rows 10.0 [13.3]; 8.2 [12.6], 512: 12.5 [15.8]; 9.9 [11.8],
 //     1024: 17.2 [30.4]; 14.4 [22.7]
-//   one plane: 1536 -> 8960: 512 rows 18.6 [21.2], 2048: 52 [69]
+//   4096 -> 2 x 14336 with the conversion: 1024 rows 361 (359) [343]; 252 (288) [265],
+//     4096: 1320 (1391) [1372]; 980 (1075) [1042]
+//   one plane: 1536 -> 8960: 256 rows 14 (18) [18], 512: 18.6 [21.2], 2048: 52 [69]
 // (gate | up at 27 rows with two channel tiles: 13.7, and 18.7 in a prompt, whose weights come
 // from memory, against 14.9 with one: twice the compute units ask for them.)
-// (A tile of 64 rows x 256 channels, one workgroup to a compute unit, takes as long per
-// row; its rounds are coarser: gate | up at 512 rows 61.8, at 256 rows 40.6.)
+// Tiles that fill a compute unit alone have coarser rounds and use an operand more often
+// (64 rows x 256 channels: long sums and many rows; 32 x 640 and 96 x 256: row counts for
+// which they come to a whole round and the others to a little more than one).
+struct TileShape {
+  int rb, gp;           // blocks of 32 rows; tiles of 32 channels per wavefront
+  bool shares;          // two workgroups to a compute unit
+  double alone, alone0; // us per chunk and beside that
+  double both, both0;
+};
+constexpr TileShape kTiles1[] = {{1, 1, true, 0.21, 4.5, 0.285, 4.5},
+                                 {wide_blocks(1), 2, true, 0.33, 5.0, 0.54, 4.0},
+                                 {3, 2, true, 0.39, 5.0, 0.66, 4.0}};
+constexpr TileShape kTiles2[] = {{1, 1, true, 0.21, 4.5, 0.37, 4.5},
+                                 {wide_blocks(2), 2, true, 0.295, 4.7, 0.50, 4.0},
+                                 {2, 2, false, 0.44, 5.2, 0, 0},
+                                 {1, 3, true, 0.39, 5.0, 0.73, 4.2},
+                                 {3, 2, false, 0.59, 6.0, 0, 0}};
+constexpr TileShape kTiles3[] = {{1, 1, true, 0.27, 4.5, 0.455, 4.5},
+                                 {wide_blocks(3), 2, true, 0.35, 4.7, 0.66, 4.0},
+                                 {2, 2, false, 0.60, 5.8, 0, 0},
+                                 {1, 5, false, 0.88, 7.0, 0, 0}};
+
 struct TilePlan {
-  int gp = 0, slices = 1;
+  int rb = 0, gp = 0, slices = 1;
   double us = 0;
 };
 template <int D, bool PAIR>
 TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, bool may_split, double norm_us,
                     int64_t sum_wgs) {
   TilePlan best;
-  constexpr int64_t kRoom = 64;
-  for (int gp = 1; gp <= 2; ++gp) {
-    const int64_t ncols = ceil_div(channels, kSlices * gp * (PAIR ? 16 : 32));
-    const int layers = D * row_blocks(D, gp);
-    const int64_t rows = ceil_div(M, 32 * row_blocks(D, gp));
-    const double alone = gp == 2 ? 0.15 + 0.08 * layers : std::max(0.21, 0.06 + 0.07 * layers);
-    const double full = gp == 2 ? 0.18 + 0.16 * layers : 0.2 + 0.085 * layers;
+  auto consider = [&](const TileShape &t) {
+    const int64_t ncols = ceil_div(channels, kSlices * t.gp * (PAIR ? 16 : 32));
+    const int64_t rows = ceil_div(M, 32 * t.rb);
     for (int s = 1; s <= (may_split ? 16 : 1); ++s) {
       const int64_t per_xcd = ceil_div(ncols * s * rows, 8);
-      if (s > 1 && per_xcd > 4 * kRoom)
+      if (s > 1 && per_xcd > 256)
         break;
       const int64_t cps = ceil_div(chunks, s);
       if (ceil_div(chunks, cps) != s)
         continue; // the last slice would be empty
       const double store = s > 1 ? 2.0 : 0.0; // of the partial sums
-      const double full_us = full * (double)cps + (gp == 2 ? 4.0 : 4.5) + store;
-      const double alone_us = alone * (double)cps + (gp == 2 ? 5.0 : 4.5) + store;
-      const int64_t left = per_xcd % kRoom;
-      const double last_us = left == 0 ? 0.0 : 2 * left <= kRoom ? alone_us : full_us;
-      double us = (double)(per_xcd / kRoom) * full_us + last_us;
+      const double alone_us = t.alone * (double)cps + t.alone0 + store;
+      double us;
+      if (t.shares) {
+        const double both_us = t.both * (double)cps + t.both0 + store;
+        const int64_t left = per_xcd % 64;
+        us = (double)(per_xcd / 64) * both_us + (left == 0 ? 0.0 : left <= 32 ? alone_us : both_us);
+      } else {
+        us = (double)ceil_div(per_xcd, 32) * alone_us;
+      }
       if (s > 1) // the kernel that adds the slices: 3 us and its bytes
-        us += 3.0 + 4.0 * (double)(M * s) * (double)(ncols * 128 * gp) / 5e6 +
+        us += 3.0 + 4.0 * (double)(M * s) * (double)(ncols * 128 * t.gp) / 4e6 +
               0.002 * (double)sum_wgs;
       else
         us += norm_us;
       if (!best.gp || us < best.us - 1e-9)
-        best = {gp, s, us};
+        best = {t.rb, t.gp, s, us};
     }
-  }
+  };
+  if constexpr (D == 1)
+    for (const TileShape &t : kTiles1)
+      consider(t);
+  else if constexpr (D == 2)
+    for (const TileShape &t : kTiles2)
+      consider(t);
+  else
+    for (const TileShape &t : kTiles3)
+      consider(t);
   return best;
 }
 
@@ -1057,7 +1101,7 @@ TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, bool may_split, dou
 template <int D, bool PAIR>
 int launch_plan(const TilePlan &plan, GemmI8Args &a, hipStream_t stream) {
   a.ncols = (int)ceil_div(a.N, kSlices * (PAIR ? 16 : 32) * plan.gp);
-  a.tile_rows = 32 * row_blocks(D, plan.gp);
+  a.tile_rows = 32 * plan.rb;
   a.span = 32 * plan.gp;
   a.row_tiles = (int)ceil_div(a.M, a.tile_rows);
   a.slices = plan.slices;
@@ -1079,7 +1123,21 @@ int launch_plan(const TilePlan &plan, GemmI8Args &a, hipStream_t stream) {
   const unsigned blocks = (unsigned)tiles;
   if (plan.gp == 1)
     return launch_narrow<D, PAIR>(a, blocks, stream);
-  return launch_wide<D, PAIR>(a, blocks, stream);
+  if (plan.gp == 2 && plan.rb == wide_blocks(D))
+    return launch_wide<D, PAIR>(a, blocks, stream);
+  if constexpr (D == 3) {
+    if (plan.gp == 2)
+      return launch_tall<D, 2, 2, PAIR>(a, blocks, stream);
+    return launch_tall<D, 1, 5, PAIR>(a, blocks, stream);
+  } else if constexpr (D == 2) {
+    if (plan.gp == 3)
+      return launch_tall<D, 1, 3, PAIR>(a, blocks, stream);
+    if (plan.rb == 2)
+      return launch_tall<D, 2, 2, PAIR>(a, blocks, stream);
+    return launch_tall<D, 3, 2, PAIR>(a, blocks, stream);
+  } else {
+    return launch_tall<D, 3, 2, PAIR>(a, blocks, stream);
+  }
 }
 
 } // namespace

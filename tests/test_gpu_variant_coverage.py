@@ -312,6 +312,57 @@ def test_silu_pair_of_few_rows(bh, oracle, M, K, N, digits):
     assert {k for k, v in report(bh, "tile").items() if v} == {f"gemm_w8_i8_kernel pair<{digits}>"}
 
 
+# The tiles that a compute unit takes alone, or that some row counts come out even on:
+# <planes, blocks of 32 rows, tiles of 32 channels per wavefront, pair>, rows and channels
+# that end inside a tile, two chunks of K, and K in slices (the cases of K > 4000)
+TALL = {(3, 2, 2, 0): [(385, 2000, 5001), (770, 8950, 1531)], (3, 2, 2, 1): [(97, 2000, 8976)],
+        (3, 1, 5, 0): [(513, 200, 8890)], (3, 1, 5, 1): [(225, 65, 8976)],
+        (2, 2, 2, 0): [(225, 1530, 12801), (97, 4100, 8890)], (2, 2, 2, 1): [(97, 1530, 12800)],
+        (2, 1, 3, 0): [(513, 65, 8890), (513, 4100, 1111)], (2, 1, 3, 1): [(257, 65, 8976)],
+        (2, 3, 2, 0): [(385, 1000, 12801)], (2, 3, 2, 1): [(225, 1000, 8976)],
+        (1, 3, 2, 0): [(777, 65, 12801), (65, 4100, 12801)]}
+
+
+def test_every_tall_int8_tile_has_a_case(bh):
+    assert {k for k in report(bh, "tile") if k.startswith("gemm_w8_i8_tall_kernel<")} == {
+        "gemm_w8_i8_tall_kernel<%d, %d, %d, %d>" % v for v in TALL}
+
+
+@pytest.mark.parametrize("variant,M,K,N", [(v, *c) for v, cs in TALL.items() for c in cs])
+def test_tall_int8_tiles(bh, oracle, variant, M, K, N):
+    bh.buddy_hip_variant_reset()
+    digits, pair = variant[0], variant[3]
+    if digits == 1:
+        w8a8_case(bh, oracle, M, K, N)  # bit for bit
+    else:
+        packs, want, size = [], [], []
+        x = torch.randn((M, K), generator=torch.Generator(device="cuda").manual_seed(M),
+                        device="cuda")
+        rounded, step = fixed_point_round(x.cpu().numpy(), digits=digits)
+        rounded = torch.from_numpy(rounded.astype(np.float64)).cuda()
+        most = rounded.abs() + torch.from_numpy(step).cuda() * 2.0**16
+        for i in range(1 + pair):
+            q, s = synthetic.quantized_linear(K, N, M + K + N + i)
+            packs.append((ops.pack_w8(q), s))
+            want.append(rounded @ q.double() * s.double())
+            # the roundings of test_int8_matmul_tile_edges
+            size.append(24 * 2.0**-24 * (most @ q.double().abs() * s.double()))
+        got = ops.gemm_w8a32(x, torch.cat([p for p, _ in packs]), torch.cat([s for _, s in packs]),
+                             K, N, digits=digits, silu_pair=bool(pair)).double()
+        if pair:
+            # SiLU has a slope of at most 1.1; its exponential is off by a few roundings of
+            # its argument
+            silu = want[0] / (1 + torch.exp(-want[0]))
+            exact = silu * want[1]
+            bound = 1.1 * size[0] * (want[1].abs() + size[1]) + silu.abs() * size[1] + \
+                exact.abs() * (1 + want[0].abs()) * 2.0**-21
+        else:
+            exact, bound = want[0], size[0]
+        assert bool(((got - exact).abs() <= bound).all())
+    ran = {k for k, v in report(bh, "tile").items() if v and "tall" in k}
+    assert ran == {"gemm_w8_i8_tall_kernel<%d, %d, %d, %d>" % variant}
+
+
 def test_every_bf16_prefill_matmul_variant(bh, oracle):
     bh.buddy_hip_variant_reset()
     for M, K, N in GEMM_BF16_SHAPES:
