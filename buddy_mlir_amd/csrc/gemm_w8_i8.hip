@@ -1053,7 +1053,7 @@ struct TilePlan {
 };
 template <int D, bool PAIR>
 TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, bool may_split, double norm_us,
-                    int64_t sum_wgs) {
+                    double split_norm_us, int64_t sum_wgs) {
   TilePlan best;
   auto consider = [&](const TileShape &t) {
     const int64_t ncols = ceil_div(channels, kSlices * t.gp * (PAIR ? 16 : 32));
@@ -1077,7 +1077,7 @@ TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, bool may_split, dou
       }
       if (s > 1) // the kernel that adds the slices: 3 us and its bytes
         us += 3.0 + 4.0 * (double)(M * s) * (double)(ncols * 128 * t.gp) / 4e6 +
-              0.002 * (double)sum_wgs;
+              0.002 * (double)sum_wgs + split_norm_us;
       else
         us += norm_us;
       if (!best.gp || us < best.us - 1e-9)
@@ -1189,13 +1189,14 @@ int launch_gemm_w8_digits_d(const GemmW8Args &in, const void *planes, hipStream_
                "gemm_w8: the SiLU pair needs two matrices of a multiple of 16 channels, no "
                "bias, no accumulation");
     a.N = (int)(in.N / 2);
-    return launch_plan<D, true>(plan_tiles<D, true>(in.M, a.N, a.chunks, false, 0.0, 0), a, stream);
+    return launch_plan<D, true>(plan_tiles<D, true>(in.M, a.N, a.chunks, false, 0.0, 0.0, 0), a, stream);
   }
   // A norm that is to follow (then_norm_w) costs a launch of its own, about
   // 5 us, unless the kernel that adds K slices writes its planes (it holds whole
   // rows, up to kRowCache columns).
-  const double pending_norm = in.then_norm_w ? 5.0 : 0.0;
   const bool slices_fuse_norm = gemm_staging_layout(in.M, in.N).cols_padded <= kRowCache;
+  const double norm_us = in.then_norm_w ? 5.0 : 0.0;
+  const double split_norm_us = slices_fuse_norm ? 0.0 : norm_us;
   // the RMSNorm of the finished rows into digit planes, where the caller asked
   // for it and no kernel of the matmul holds whole rows
   auto then_norm = [&]() -> int {
@@ -1204,11 +1205,11 @@ int launch_gemm_w8_digits_d(const GemmW8Args &in, const void *planes, hipStream_
     return launch_rmsnorm_to_digits(in.C, in.ldc, in.then_norm_w, (int)in.M, (int)in.N,
                                     in.then_norm_eps, in.digits, in.then_norm_staged, stream);
   };
-  TilePlan plan = plan_tiles<D, false>(in.M, in.N, a.chunks, true, pending_norm, 0);
+  TilePlan plan = plan_tiles<D, false>(in.M, in.N, a.chunks, true, norm_us, split_norm_us, 0);
   if (int rc = launch_plan<D, false>(plan, a, stream))
     return rc;
   if (plan.slices > 1 && !a.partial) {
-    plan = plan_tiles<D, false>(in.M, in.N, a.chunks, false, pending_norm, 0);
+    plan = plan_tiles<D, false>(in.M, in.N, a.chunks, false, norm_us, 0.0, 0);
     if (int rc = launch_plan<D, false>(plan, a, stream))
       return rc;
   }
@@ -1277,12 +1278,12 @@ int launch_gemm_w8a8_plane(const void *plane, const int8_t *W, const float *wsca
   // sums in the workspace (f32 ones would round above 2^24) and a second kernel
   // adds them exactly
   const int64_t reduce_wgs = ceil_div(M * ceil_div(N, 4), 256);
-  TilePlan plan = plan_tiles<1, false>(M, N, a.chunks, true, 0.0, reduce_wgs);
+  TilePlan plan = plan_tiles<1, false>(M, N, a.chunks, true, 0.0, 0.0, reduce_wgs);
   a.int_partials = plan.slices > 1;
   if (int rc = launch_plan<1, false>(plan, a, stream))
     return rc;
   if (plan.slices > 1 && !a.partial) {
-    plan = plan_tiles<1, false>(M, N, a.chunks, false, 0.0, reduce_wgs);
+    plan = plan_tiles<1, false>(M, N, a.chunks, false, 0.0, 0.0, reduce_wgs);
     a.int_partials = 0;
     if (int rc = launch_plan<1, false>(plan, a, stream))
       return rc;

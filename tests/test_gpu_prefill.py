@@ -602,6 +602,24 @@ def test_wide_hidden_size_through_the_slice_adding_norm_kernel(oracle):
     sess.close()
 
 
+@pytest.mark.parametrize("n", [20, 70])
+def test_hidden_size_beyond_the_slice_adding_norm_kernel(n):
+    """hidden = 12352: a row is longer than that kernel holds; the norm is a launch of its own
+    behind products with whole sums and with K in slices."""
+    shape = Shape(layers=2, hidden=12352, heads=8, kv_heads=2, head_dim=128, inter=2048,
+                  vocab=320, max_len=128)
+    toks = synthetic.first_tokens(shape, n, seed=n).astype(np.int32)
+    sess, _ = synthetic.build_session(shape, context=0, ln_jitter=0.1)
+    _, got = sess.prefill(toks, 0)
+    rows = [sess.get_kv(j)[:, :n].copy() for j in range(4)]
+    for i, t in enumerate(toks):
+        _, want = sess.decode(int(t), i, want_logits=i + 1 == n)
+    check_close(got, want)
+    for j in range(4):
+        check_close(rows[j], sess.get_kv(j)[:, :n])
+    sess.close()
+
+
 @pytest.mark.timeout(900)
 def test_qwen2_1p5b_shape_512_token_prefill(oracle):
     """The full 28-layer shape, a prompt of 512 tokens as one block (digit-plane
