@@ -49,7 +49,7 @@ struct PromptArgs {
   PromptBlock *blocks;
 };
 
-// tiles of keys that block b of 128 rows sees
+// tiles of keys that block b of 256 rows sees
 __device__ __forceinline__ int tiles_of(const PromptArgs &a, int b) {
   const int row = min((b + 1) * kPromptRows, a.q_len * a.group) - 1;
   return (min(a.k_len, a.q_offset + row / a.group + 1) + kKeys - 1) / kKeys;
@@ -117,8 +117,8 @@ constexpr int kProdB[6] = {2, 0, 1, 1, 0, 0};
 
 // Workgroup i takes an equal share of all (KV head, row block, key tile) triples in that
 // order, wherever it begins and ends: blocks it holds whole leave as finished rows, the
-// others as partial results.  Its four wavefronts have 32 rows each and share the tiles,
-// which one wavefront quarter each turns into terms a tile ahead.
+// others as partial results.  Its eight wavefronts have 32 rows each and share the tiles,
+// of which each turns an eighth into terms a tile ahead.
 //   S^T[key, row] = K . Q^T;  O^T[d, row] += V^T . P^T
 // and the registers of S^T are the operand P^T as they lie: a lane has keys
 // 8 j + 4 (lane / 32) + 0..3 of row lane % 32, and V^T is stored with its keys in that

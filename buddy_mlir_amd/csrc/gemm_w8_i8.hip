@@ -27,8 +27,8 @@
 // padded, followed by the row steps (f32 [rows_padded]).  A lane's operand is 16
 // contiguous bytes of a plane row.
 //
-// Workgroups take 32 rows x 128 or 256 channels, with the activation fragments shared
-// through LDS.
+// Workgroups take 32 rows x 128 or 256 channels, or one of the other tiles of kTiles1 to
+// kTiles3, with the activation fragments shared through LDS.
 #include "attn_fold.h"
 #include "gemm.h"
 

@@ -621,8 +621,7 @@ int launch_plan(const TilePlan &plan, GemmArgs &a, int terms, hipStream_t stream
 
 GemmStagingLayout gemm_staging_layout(int64_t M, int64_t K) {
   GemmStagingLayout l;
-  // padded rows cover the last 64-row block and the last 48-row block
-  l.rows_padded = (int)std::max(round_up(M, 64), round_up(M, 48));
+  l.rows_padded = (int)round_up(M, 32); // rows of a tile beyond these repeat the last
   l.cols_padded = (int)round_up(K, kTileK);
   return l;
 }

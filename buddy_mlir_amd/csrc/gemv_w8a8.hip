@@ -17,8 +17,8 @@
 // midend/lib/Conversion/MatMulOptimization/MatMulBlisVectorization.cpp:668-724):
 // the quantised activations are written as one plane in the layout the prefill
 // matmul reads, by two launches (partial maxima over the tensor, then one
-// workgroup per row), and the prefill kernel multiplies it with whole K per
-// workgroup, so that the int32 sums stay whole.
+// workgroup per row), and the prefill kernel multiplies it; where K goes to several
+// workgroups, their int32 sums are added as integers.
 #include "common.h"
 #include <algorithm>
 #include "gemm.h"
