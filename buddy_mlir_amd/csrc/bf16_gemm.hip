@@ -3,9 +3,10 @@
 //
 // Weights go from memory to registers as they lie, each of the four wavefronts of a
 // workgroup its own channels; the activation rows are the B operand and are shared
-// through LDS.  Both are requested three steps ahead.  Up to 16 rows a tile of 16
-// channels x 32 k is the A operand as it lies, and f32 activations are multiplied by
-// v_mfma_f32_16x16x4_f32; above that see rows_gemm_wide_kernel.
+// through LDS.  Both are requested three steps ahead.  Up to 16 rows, and for some more
+// bfloat16 ones (launch_shape), a tile of 16 channels x 32 k is the A operand as it lies, and
+// f32 activations are multiplied by v_mfma_f32_16x16x4_f32; above that see
+// rows_gemm_wide_kernel.
 #include "bf16_linear.h"
 #include "bf16_dev.h"
 
@@ -113,13 +114,13 @@ __device__ __forceinline__ int find_expert(const int *counts, int experts, int r
   return -1;
 }
 
-template <typename T, int RT, int GT, int OUT, bool GROUPED>
+template <typename T, int GT, int OUT, bool GROUPED>
 __global__ void __launch_bounds__(kGemmThreads)
 rows_gemm_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int columns, int row_blocks, GemmDev a) {
   using Tr = ActTraits<T>;
   constexpr bool kPair = OUT == kOutExpertAct;
   constexpr int kGroups = kPair ? GT / 2 : GT; // channel groups of the result per wavefront
-  constexpr int kRows = 16 * RT;
+  constexpr int kRows = 16;
   constexpr int kRuns = kRows * 8;                               // 16-byte runs per step
   constexpr int kLoads = (kRuns + kGemmThreads - 1) / kGemmThreads;
   __shared__ __attribute__((aligned(16))) unsigned char lds[2][kRows * kLdsRow];
@@ -193,12 +194,10 @@ rows_gemm_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int columns
   for (int s = 0; s < kStages - 1; ++s)
     fetch(s, wr[s], ar[s]);
 
-  f32x4 acc[GT][RT];
+  f32x4 acc[GT];
 #pragma unroll
   for (int g = 0; g < GT; ++g)
-#pragma unroll
-    for (int r = 0; r < RT; ++r)
-      acc[g][r] = f32x4{0.f, 0.f, 0.f, 0.f};
+    acc[g] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   const int frag_at = (lane & 15) * kLdsRow + (lane >> 4) * 8 * (int)sizeof(T);
   auto step = [&](int s, uint4 (&w)[GT * Tr::kTiles], uint4 (&x)[kLoads], uint4 (&w_next)[GT * Tr::kTiles],
@@ -216,11 +215,8 @@ rows_gemm_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int columns
     __syncthreads(); // the other buffer was last read before the previous barrier
 #pragma unroll
     for (int t = 0; t < Tr::kTiles; ++t) {
-      Frag<T> b[RT];
-#pragma unroll
-      for (int r = 0; r < RT; ++r)
-        b[r].load(reinterpret_cast<const T *>(buf + frag_at + r * 16 * kLdsRow +
-                                              t * kBfTileK * (int)sizeof(T)));
+      Frag<T> b;
+      b.load(reinterpret_cast<const T *>(buf + frag_at + t * kBfTileK * (int)sizeof(T)));
 #pragma unroll
       for (int g = 0; g < GT; ++g) {
         Frag<T> wf;
@@ -228,9 +224,7 @@ rows_gemm_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int columns
           wf.v = w[g * Tr::kTiles + t];
         else
           wf = widen(w[g * Tr::kTiles + t]);
-#pragma unroll
-        for (int r = 0; r < RT; ++r)
-          acc[g][r] = mfma32(wf, b[r], acc[g][r]);
+        acc[g] = mfma32(wf, b, acc[g]);
       }
     }
   };
@@ -250,39 +244,36 @@ rows_gemm_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int columns
     step(s + 2, wr[2], ar[2], wr[1], ar[1], lds[0]);
 
   // a lane holds channels (lane / 16) * 4 + 0..3 of row lane % 16 of every tile
+  const int lr = row0 + (lane & 15);
+  if (lr >= rows)
+    return;
+  int orow = lr;
+  if constexpr (GROUPED)
+    orow = list[lr];
 #pragma unroll
-  for (int r = 0; r < RT; ++r) {
-    const int lr = row0 + r * 16 + (lane & 15);
-    if (lr >= rows)
+  for (int g = 0; g < kGroups; ++g) {
+    if (ch0 + g >= a.groups)
       continue;
-    int orow = lr;
-    if constexpr (GROUPED)
-      orow = list[lr];
+    const int ch = (ch0 + g) * 16 + (lane >> 4) * 4;
+    f32x4 v = acc[g];
+    if constexpr (OUT == kOutExpertAct) {
+      const f32x4 up = acc[g + kGroups];
 #pragma unroll
-    for (int g = 0; g < kGroups; ++g) {
-      if (ch0 + g >= a.groups)
-        continue;
-      const int ch = (ch0 + g) * 16 + (lane >> 4) * 4;
-      f32x4 v = acc[g][r];
-      if constexpr (OUT == kOutExpertAct) {
-        const f32x4 up = acc[g + kGroups][r];
+      for (int j = 0; j < 4; ++j)
+        v[j] = gated_act(a.act, v[j], up[j], a.limit);
+      store4<T>(static_cast<T *>(a.C) + (int64_t)orow * a.ldc + ch, v);
+    } else if constexpr (OUT == kOutF32) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          v[j] = gated_act(a.act, v[j], up[j], a.limit);
-        store4<T>(static_cast<T *>(a.C) + (int64_t)orow * a.ldc + ch, v);
-      } else if constexpr (OUT == kOutF32) {
+      for (int j = 0; j < 4; ++j)
+        if (ch + j < a.silu_channels)
+          v[j] = silu_f(v[j]);
+      store4<float>(static_cast<float *>(a.C) + (int64_t)orow * a.ldc + ch, v);
+    } else if constexpr (OUT == kOutAct) {
+      store4<T>(static_cast<T *>(a.C) + (int64_t)orow * a.ldc + ch, v);
+    } else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (ch + j < a.silu_channels)
-            v[j] = silu_f(v[j]);
-        store4<float>(static_cast<float *>(a.C) + (int64_t)orow * a.ldc + ch, v);
-      } else if constexpr (OUT == kOutAct) {
-        store4<T>(static_cast<T *>(a.C) + (int64_t)orow * a.ldc + ch, v);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          store_act<T>(static_cast<T *>(a.C) + (int64_t)(ch + j) * a.ldc + orow, v[j]);
-      }
+      for (int j = 0; j < 4; ++j)
+        store_act<T>(static_cast<T *>(a.C) + (int64_t)(ch + j) * a.ldc + orow, v[j]);
     }
   }
 }
@@ -638,15 +629,20 @@ int launch_tiles(F kernel, int elems, const RowsGemm &a, hipStream_t stream) {
   return BUDDY_HIP_OK;
 }
 
-// RT tiles of 16 rows, GT channel groups per wavefront (pairs count twice)
-template <typename T, int RT, int GT, int OUT, bool GROUPED>
-int launch_variant(const RowsGemm &a, hipStream_t stream) {
-  return launch_tiles<T, 16 * RT, 64 * (OUT == kOutExpertAct ? GT / 2 : GT), OUT, GROUPED>(
-      rows_gemm_kernel<T, RT, GT, OUT, GROUPED>, ActTraits<T>::kElems, a, stream);
+BH_TILE_FAMILY(RowsFamily, "rows_gemm_kernel");
+BH_TILE_FAMILY(WideFamily, "rows_gemm_wide_kernel");
+
+// 16 rows, GT channel groups per wavefront (pairs count twice)
+template <typename T, int GT, int OUT, bool GROUPED>
+int launch_flat(const RowsGemm &a, hipStream_t stream) {
+  BH_NOTE_VARIANT(RowsFamily, sizeof(T) == 4, GT, OUT, GROUPED);
+  return launch_tiles<T, 16, 64 * (OUT == kOutExpertAct ? GT / 2 : GT), OUT, GROUPED>(
+      rows_gemm_kernel<T, GT, OUT, GROUPED>, ActTraits<T>::kElems, a, stream);
 }
 // RT tiles of 32 rows, GT tiles of 32 channels per wavefront
 template <typename T, int RT, int GT, int OUT, bool GROUPED>
 int launch_wide(const RowsGemm &a, hipStream_t stream) {
+  BH_NOTE_VARIANT(WideFamily, sizeof(T) == 4, RT, GT, OUT, GROUPED);
   return launch_tiles<T, 32 * RT, 128 * (OUT == kOutExpertAct ? GT / 2 : GT), OUT, GROUPED>(
       rows_gemm_wide_kernel<T, RT, GT, OUT, GROUPED>, kWideK, a, stream);
 }
@@ -670,8 +666,8 @@ int launch_shape(const RowsGemm &a, hipStream_t stream) {
     return ceil_div(a.W.N, ch) * ceil_div(rows, rt) * all_blocks;
   };
   if (rows <= 16)
-    return workgroups(16, 128) >= 256 ? launch_variant<T, 1, 2 * P, OUT, GROUPED>(a, stream)
-                                      : launch_variant<T, 1, P, OUT, GROUPED>(a, stream);
+    return workgroups(16, 128) >= 256 ? launch_flat<T, 2 * P, OUT, GROUPED>(a, stream)
+                                      : launch_flat<T, P, OUT, GROUPED>(a, stream);
   const double steps = (double)ceil_div(a.W.K, kWideK);
   auto cost = [&](int rt, int ch, double step_us, double fixed_us) {
     return (double)ceil_div(workgroups(rt, ch / P), 256) * steps * step_us + fixed_us;
@@ -690,7 +686,7 @@ int launch_shape(const RowsGemm &a, hipStream_t stream) {
       const double half = cost(64, 256, 0.60, 5.0) + thin(64);
       const double low = cost(32, 256, 0.40, 4.0) + thin(32);
       if (flat <= std::min({tall, half, low}))
-        return launch_variant<T, 1, P, OUT, GROUPED>(a, stream);
+        return launch_flat<T, P, OUT, GROUPED>(a, stream);
       if (tall <= std::min(half, low))
         return launch_wide<T, 4, 2, OUT, GROUPED>(a, stream);
       return half <= low ? launch_wide<T, 2, 2, OUT, GROUPED>(a, stream)
@@ -698,7 +694,7 @@ int launch_shape(const RowsGemm &a, hipStream_t stream) {
     } else {
       const double half = cost(64, 128, 0.29, 4.5), low = cost(32, 128, 0.21, 4.0);
       if (flat <= std::min({tall, half, low}))
-        return launch_variant<T, 1, P, OUT, GROUPED>(a, stream);
+        return launch_flat<T, P, OUT, GROUPED>(a, stream);
       if (tall <= std::min(half, low))
         return launch_wide<T, 4, 2, OUT, GROUPED>(a, stream);
       return half <= low ? launch_wide<T, 2, 1, OUT, GROUPED>(a, stream)

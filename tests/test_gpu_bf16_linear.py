@@ -5,6 +5,7 @@ import pytest
 import torch
 
 import nukopel_oracle as N
+from test_gpu_variant_coverage import report
 
 pytestmark = pytest.mark.gpu
 
@@ -77,9 +78,9 @@ def sums64(a, w):
     return d.cpu().numpy()
 
 
-# tiles of 32 x 128, 32 x 256 (f32), 64 x 128 and 128 x 256 with a remainder in rows, in
-# pairs of channel groups and in K: below, at and beyond a step, and fewer steps than the
-# kernel asks for ahead
+# f32: tiles of 32 x 128 and 32 x 256 with a remainder in rows, in pairs of channel groups
+# and in K: below, at and beyond a step, and fewer steps than the kernel asks for ahead.
+# bfloat16: 16 x 64 tiles for the first five, 64 x 128 and 128 x 256 (see also below)
 @pytest.mark.parametrize("dtype", [0, 1])
 @pytest.mark.parametrize("M,K,Nout", [
     (17, 63, 33), (31, 64, 16), (33, 65, 48), (32, 129, 130), (65, 193, 144), (97, 1000, 8200),
@@ -107,6 +108,37 @@ def test_wide_tiles(bh, M, K, Nout, dtype):
     err = np.abs(got[:, :Nout] - want).max()
     assert err < 3e-6 * max(1.0, np.abs(want).max()), err
     assert (got[:, (Nout + 15) // 16 * 16:] == 7.0).all()
+
+
+# the same edges of K in bfloat16, at row and channel counts for which the estimate takes
+# each of the wide tiles: <RT tiles of 32 rows, GT tiles of 32 channels per wavefront>
+WIDE = {(1, 1): [(129, 1, 40016), (129, 63, 40016), (161, 64, 33001), (97, 65, 24001),
+                 (449, 129, 4100), (65, 193, 20020), (513, 260, 1500), (33, 8960, 6001)],
+        (2, 1): [(161, 1, 40016), (225, 63, 30000), (289, 64, 24001), (97, 65, 30000),
+                 (129, 129, 20020), (97, 193, 15001), (257, 260, 5000)],
+        (4, 2): [(1931, 193, 20020), (257, 8960, 20020)]}
+
+
+@pytest.mark.parametrize("tile,M,K,Nout", [(t, *c) for t, cs in WIDE.items() for c in cs])
+def test_wide_tiles_of_bfloat16_rows(bh, tile, M, K, Nout):
+    w, tiles = make(bh, K, Nout, M + K)
+    a = N.bf16(np.random.default_rng(M).standard_normal((M, K)).astype(np.float32))
+    lda, ldc = (K + 7) // 8 * 8, (Nout + 15) // 16 * 16 + 4
+    buf = np.full((M, lda), 0x7FC0, np.uint16)
+    buf[:, :K] = N.to_bf16_bits(a)
+    A = torch.from_numpy(buf.view(np.int16)).cuda()
+    C = torch.full((M, ldc), 7.0, device="cuda")
+    torch.cuda.synchronize()
+    bh.buddy_hip_variant_reset()
+    assert bh.buddy_hip_gemm_bf16(A.data_ptr(), lda, 0, tiles.data_ptr(), C.data_ptr(), ldc,
+                                  M, K, Nout, None) == 0
+    torch.cuda.synchronize()
+    assert {k for k, v in report(bh, "tile").items() if v} == {
+        "rows_gemm_wide_kernel<0, %d, %d, 0, 0>" % tile}
+    want = torch.from_numpy(np.asarray(a, np.float64)).cuda() @ torch.from_numpy(w).cuda().T
+    err = float((C[:, :Nout] - want).abs().max())
+    assert err < 3e-6 * max(1.0, float(want.abs().max())), err
+    assert bool((C[:, (Nout + 15) // 16 * 16:] == 7.0).all())
 
 
 def test_f32_rows_keep_every_bit_and_their_infinities(bh):

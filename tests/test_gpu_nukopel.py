@@ -14,6 +14,7 @@ import nukopel_models as M
 import nukopel_oracle as N
 from buddy_mlir_amd import BuddyHipError
 from buddy_mlir_amd.session import FolderSession, Sampler
+from test_gpu_variant_coverage import report
 
 pytestmark = pytest.mark.gpu
 
@@ -106,6 +107,38 @@ def test_mechanism_alone(tmp_path, what, dtype):
     s = FolderSession(folder, dtype, max_len=80)
     check(all_rows(s, tokens), want, dtype, "prompt")
     check(feed(s, tokens, [3] + [1] * 67), want, dtype, "decoding")
+
+
+# rows_gemm_wide_kernel<f32, RT, GT, 3, experts>: gate and up on tiles of 32 RT rows x 64 GT
+# channels of each, of experts (whose counts are uneven) and of the shared one, whose widths
+# end inside a tile; and <f32, RT, GT, 0, 1>, the experts' way back
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width,ff,experts,top,shared,n,tiles", [
+    (136, 2100, 6, 2, 0, 150, ["0, 1, 2, 3, 1"]),
+    (136, 4100, 6, 2, 0, 300, ["0, 2, 2, 3, 1"]),
+    (72, 4100, 9, 4, 0, 1300, ["0, 4, 2, 3, 1", "0, 1, 1, 0, 1"]),
+    (136, 1010, 9, 4, 0, 1300, ["0, 2, 2, 3, 1", "0, 2, 1, 0, 1"]),
+    (72, 40, 2, 1, 2100, 700, ["0, 1, 2, 3, 0"]),
+    (72, 40, 2, 1, 8200, 700, ["0, 2, 2, 3, 0"]),
+    (250, 40, 2, 1, 8200, 1290, ["0, 4, 2, 3, 0", "0, 1, 1, 0, 0"])])
+def test_feed_forward_on_wide_tiles(tmp_path, bh, width, ff, experts, top, shared, n, tiles, dtype):
+    cfg = M.config([M.latent(window=1, mlp=M.moe(experts=experts, top=top, ff=ff, shared_ff=shared))],
+                   width=width, vocab=width)
+
+    def edit(t):
+        t["head"] = np.eye(width)
+        t["l0.mix.o"] *= 0.0  # the feed-forward alone
+    folder, t = M.build(tmp_path, cfg, n, edit)
+    tokens = tokens_for(cfg, n)
+    want = N.forward(cfg, t, tokens)
+    s = FolderSession(folder, dtype, max_len=n + 8)
+    bh.buddy_hip_variant_reset()
+    check(all_rows(s, tokens), want, dtype, "prompt")
+    ran = {k for k, v in report(bh, "tile").items() if v}
+    if dtype == "bfloat16":
+        assert {f"rows_gemm_wide_kernel<{v}>" for v in tiles} <= ran, ran
+    else:
+        assert "rows_gemm_wide_kernel<1, 1, 2, 3, %d>" % (shared == 0) in ran, ran
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
