@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import nukopel_oracle as N
-from test_gpu_variant_coverage import report
+from test_gpu_variant_coverage import tiles_run
 
 pytestmark = pytest.mark.gpu
 
@@ -133,7 +133,7 @@ def test_wide_tiles_of_bfloat16_rows(bh, tile, M, K, Nout):
     assert bh.buddy_hip_gemm_bf16(A.data_ptr(), lda, 0, tiles.data_ptr(), C.data_ptr(), ldc,
                                   M, K, Nout, None) == 0
     torch.cuda.synchronize()
-    assert {k for k, v in report(bh, "tile").items() if v} == {
+    assert {k for k, v in tiles_run(bh).items() if v} == {
         "rows_gemm_wide_kernel<0, %d, %d, 0, 0>" % tile}
     want = torch.from_numpy(np.asarray(a, np.float64)).cuda() @ torch.from_numpy(w).cuda().T
     err = float((C[:, :Nout] - want).abs().max())

@@ -14,7 +14,7 @@ import nukopel_models as M
 import nukopel_oracle as N
 from buddy_mlir_amd import BuddyHipError
 from buddy_mlir_amd.session import FolderSession, Sampler
-from test_gpu_variant_coverage import report
+from test_gpu_variant_coverage import tiles_run
 
 pytestmark = pytest.mark.gpu
 
@@ -134,7 +134,7 @@ def test_feed_forward_on_wide_tiles(tmp_path, bh, width, ff, experts, top, share
     s = FolderSession(folder, dtype, max_len=n + 8)
     bh.buddy_hip_variant_reset()
     check(all_rows(s, tokens), want, dtype, "prompt")
-    ran = {k for k, v in report(bh, "tile").items() if v}
+    ran = {k for k, v in tiles_run(bh).items() if v}
     if dtype == "bfloat16":
         assert {f"rows_gemm_wide_kernel<{v}>" for v in tiles} <= ran, ran
     else:

@@ -8,7 +8,8 @@ import torch
 
 import buddy_mlir_amd as bma
 from buddy_mlir_amd import ops, synthetic
-from buddy_mlir_amd.session import DecoderSession, Shape
+from buddy_mlir_amd.session import Shape
+from buddy_mlir_amd.session import DecoderSession
 from parity import check_close
 from test_gpu_decode import SMALL, oracle_model
 

@@ -25,16 +25,24 @@ from test_gpu_prefill import (SCALE, SILU_PAIR_SHAPES, bf16_round, fixed_point_r
 pytestmark = pytest.mark.gpu
 
 
-def report(bh, of="variant"):
-    write = getattr(bh, f"buddy_hip_{of}_report")
-    n = write(None, 0)
+def report(bh):
+    n = bh.buddy_hip_variant_report(None, 0)
     buf = ctypes.create_string_buffer(n)
-    write(buf, n)
+    bh.buddy_hip_variant_report(buf, n)
     out = {}
     for line in buf.value.decode().splitlines():
         name, hits = line.split("\t")
         out[name] = int(hits)
     return out
+
+
+def tiles_run(bh):
+    """Launches of the matrix products whose tile an estimate picks, by tile."""
+    n = bh.buddy_hip_tile_report(None, 0)
+    buf = ctypes.create_string_buffer(n)
+    bh.buddy_hip_tile_report(buf, n)
+    return {name: int(hits) for name, hits in
+            (line.split("\t") for line in buf.value.decode().splitlines())}
 
 
 def launched(bh, family):
@@ -309,7 +317,7 @@ def test_silu_pair_of_few_rows(bh, oracle, M, K, N, digits):
     asked for ahead."""
     bh.buddy_hip_variant_reset()
     silu_pair_case(oracle, M, K, N, digits=digits)
-    assert {k for k, v in report(bh, "tile").items() if v} == {f"gemm_w8_i8_kernel pair<{digits}>"}
+    assert {k for k, v in tiles_run(bh).items() if v} == {f"gemm_w8_i8_kernel pair<{digits}>"}
 
 
 # The tiles that a compute unit takes alone, or that some row counts come out even on:
@@ -324,7 +332,7 @@ TALL = {(3, 2, 2, 0): [(385, 2000, 5001), (770, 8950, 1531)], (3, 2, 2, 1): [(97
 
 
 def test_every_tall_int8_tile_has_a_case(bh):
-    assert {k for k in report(bh, "tile") if k.startswith("gemm_w8_i8_tall_kernel<")} == {
+    assert {k for k in tiles_run(bh) if k.startswith("gemm_w8_i8_tall_kernel<")} == {
         "gemm_w8_i8_tall_kernel<%d, %d, %d, %d>" % v for v in TALL}
 
 
@@ -359,7 +367,7 @@ def test_tall_int8_tiles(bh, oracle, variant, M, K, N):
         else:
             exact, bound = want[0], size[0]
         assert bool(((got - exact).abs() <= bound).all())
-    ran = {k for k, v in report(bh, "tile").items() if v and "tall" in k}
+    ran = {k for k, v in tiles_run(bh).items() if v and "tall" in k}
     assert ran == {"gemm_w8_i8_tall_kernel<%d, %d, %d, %d>" % variant}
 
 
