@@ -100,7 +100,7 @@ __device__ __forceinline__ void f32_row(const PromptFold &f, int t, int h, int d
 
 // four values d .. d + 3 of query head h at token t, from where the launch left them
 __device__ __forceinline__ void left4(const PromptFold &f, int64_t out_stride, int t, int h, int d,
-                                        float (&v)[4]) {
+                                      float (&v)[4]) {
   const int kvh = h / f.group, row = t * f.group + (h - kvh * f.group);
   const PromptBlock b = f.blocks[kvh * f.nblk + row / kPromptRows];
   if (b.parts == 0) {
@@ -156,13 +156,19 @@ __device__ __forceinline__ void left4(const PromptFold &f, int64_t out_stride, i
     v[e] = s[e] * inv;
 }
 
-// ... finished.  Called by all 32 lanes of a row together, half a wavefront.
-__device__ __forceinline__ void folded4(const PromptFold &f, int64_t out_stride, int t, int h, int d,
-                                        float (&v)[4]) {
-  left4(f, out_stride, t, h, d, v);
-  const float largest = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
-  const bool again = !(largest < INFINITY) || v[0] != v[0] || v[1] != v[1] || v[2] != v[2] || v[3] != v[3];
-  if ((__ballot(again) >> (threadIdx.x & 32)) & 0xffffffffu)
+// left4 leaves something that is not finite where a row is to be computed again.
+__device__ __forceinline__ bool to_repair(const float (&v)[4]) {
+  unsigned most = 0;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    most = max(most, __float_as_uint(v[e]) & 0x7fffffffu);
+  return most >= 0x7f800000u;
+}
+// ... which is done here, behind everything else (inside the loop over the heads: 600 tokens
+// of 12 heads, all finite, 13.9 us; behind it 12.2; not at all 11.3).  Called by all 32 lanes
+// of a row together, half a wavefront, with what left4 gave.
+__device__ __forceinline__ void repair4(const PromptFold &f, int t, int h, int d, float (&v)[4]) {
+  if ((__ballot(to_repair(v)) >> (threadIdx.x & 32)) & 0xffffffffu)
     f32_row(f, t, h, d, v);
 }
 #endif

@@ -462,10 +462,22 @@ constexpr int kFoldThreads = 512;
 __global__ void __launch_bounds__(kFoldThreads)
 attn_fold_rows_kernel(PromptFold f, float *out, int64_t o_stride, int heads) {
   const int t = blockIdx.x;
+  float *row = out + (int64_t)t * o_stride;
+  bool bad = false;
   for (int i = threadIdx.x * 4; i < heads * kPromptD; i += 4 * kFoldThreads) {
     float v[4];
-    folded4(f, o_stride, t, i / kPromptD, i % kPromptD, v);
-    *reinterpret_cast<float4 *>(out + (int64_t)t * o_stride + i) = float4{v[0], v[1], v[2], v[3]};
+    left4(f, o_stride, t, i / kPromptD, i % kPromptD, v);
+    bad |= to_repair(v);
+    *reinterpret_cast<float4 *>(row + i) = float4{v[0], v[1], v[2], v[3]};
+  }
+  if (__any(bad)) {
+#pragma unroll 1
+    for (int i = threadIdx.x * 4; i < heads * kPromptD; i += 4 * kFoldThreads) {
+      const float4 q = *reinterpret_cast<const float4 *>(row + i);
+      float v[4] = {q.x, q.y, q.z, q.w};
+      repair4(f, t, i / kPromptD, i % kPromptD, v);
+      *reinterpret_cast<float4 *>(row + i) = float4{v[0], v[1], v[2], v[3]};
+    }
   }
 }
 

@@ -66,6 +66,7 @@ __device__ __forceinline__ void load4(const float *p, int k0, int n, float (&v)[
   }
 }
 struct PlainRow {
+  static constexpr bool kRepairs = false;
   const float *a;
   int n;
   __device__ __forceinline__ void operator()(int k0, float (&v)[4]) const {
@@ -73,6 +74,7 @@ struct PlainRow {
   }
 };
 struct NormRow { // w * (x * rs)
+  static constexpr bool kRepairs = false;
   const float *x, *w;
   float rs;
   int n;
@@ -91,6 +93,7 @@ __device__ __forceinline__ float silu_times(float g, float u) {
   return (g * sig) * u;
 }
 struct SiluMulRow { // silu(g) * u
+  static constexpr bool kRepairs = false;
   const float *g, *u;
   int n;
   __device__ __forceinline__ void operator()(int k0, float (&v)[4]) const {
@@ -104,13 +107,18 @@ struct SiluMulRow { // silu(g) * u
 };
 
 struct FoldedRow { // the attention's output at one token, added up from its parts
+  static constexpr bool kRepairs = true;
   const PromptFold &f;
   int64_t o_stride;
   int t, n;
   __device__ __forceinline__ void operator()(int k0, float (&v)[4]) const {
     v[0] = v[1] = v[2] = v[3] = 0.f;
     if (k0 < n)
-      folded4(f, o_stride, t, k0 / kPromptD, k0 % kPromptD, v);
+      left4(f, o_stride, t, k0 / kPromptD, k0 % kPromptD, v);
+  }
+  __device__ __forceinline__ void repair(int k0, float (&v)[4]) const {
+    if (k0 < n)
+      repair4(f, t, k0 / kPromptD, k0 % kPromptD, v);
   }
 };
 
@@ -132,27 +140,48 @@ __device__ __forceinline__ void row_to_digits(const F &f, int n, int row, int D,
   // NaN step, so that every result of the row is NaN -- what the reference's f32
   // multiply-add chain makes of such a row (MatMulBlisVectorization.cpp:644-740)
   unsigned mb = 0;
-  constexpr unsigned kAbs = 0x7fffffffu;
-#pragma unroll 3
-  for (int k0 = threadIdx.x * 4; k0 < Kp; k0 += kRowThreads * 4) {
-    float v[4];
-    f(k0, v);
+  auto note = [&](const float (&v)[4]) {
+    constexpr unsigned kAbs = 0x7fffffffu;
     mb = max(max(mb, max(__float_as_uint(v[0]) & kAbs, __float_as_uint(v[1]) & kAbs)),
              max(__float_as_uint(v[2]) & kAbs, __float_as_uint(v[3]) & kAbs));
-    if (cached)
-      *reinterpret_cast<float4 *>(cache + k0) = make_float4(v[0], v[1], v[2], v[3]);
-  }
-  mb = wave_max_u32(mb);
-  __syncthreads(); // red may still be read by the caller's own reduction
-  if ((threadIdx.x & 63) == 0)
-    red[threadIdx.x >> 6] = __uint_as_float(mb);
-  __syncthreads();
-  {
+  };
+  auto row_max = [&]() {
+    mb = wave_max_u32(mb);
+    __syncthreads(); // red may still be read by the caller's own reduction
+    if ((threadIdx.x & 63) == 0)
+      red[threadIdx.x >> 6] = __uint_as_float(mb);
+    __syncthreads();
     unsigned m2 = __float_as_uint(red[0]);
 #pragma unroll
     for (int w = 1; w < kRowThreads / 64; ++w)
       m2 = max(m2, __float_as_uint(red[w]));
     mb = m2;
+  };
+#pragma unroll 3
+  for (int k0 = threadIdx.x * 4; k0 < Kp; k0 += kRowThreads * 4) {
+    float v[4];
+    f(k0, v);
+    note(v);
+    if (cached)
+      *reinterpret_cast<float4 *>(cache + k0) = make_float4(v[0], v[1], v[2], v[3]);
+  }
+  row_max();
+  bool repaired = false; // once more where the source can do better than this
+  if constexpr (F::kRepairs) {
+    repaired = mb >= 0x7f800000u; // the same in all threads
+    if (repaired) {
+      mb = 0;
+#pragma unroll 1
+      for (int k0 = threadIdx.x * 4; k0 < Kp; k0 += kRowThreads * 4) {
+        float v[4];
+        f(k0, v);
+        f.repair(k0, v);
+        note(v);
+        if (cached)
+          *reinterpret_cast<float4 *>(cache + k0) = make_float4(v[0], v[1], v[2], v[3]);
+      }
+      row_max();
+    }
   }
   const bool finite = mb < 0x7f800000u;
   const float step = finite ? digit_step(__uint_as_float(mb), D) : __uint_as_float(0x7fc00000u);
@@ -169,6 +198,10 @@ __device__ __forceinline__ void row_to_digits(const F &f, int n, int row, int D,
       v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
     } else {
       f(k0, v);
+      if constexpr (F::kRepairs) {
+        if (repaired)
+          f.repair(k0, v);
+      }
     }
     int X[4];
 #pragma unroll

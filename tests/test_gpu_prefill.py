@@ -530,6 +530,32 @@ def test_prompt_attention_of_a_key_beyond_bfloat16(bad, precision):
         check_close(got[finite], want[finite])
 
 
+@pytest.mark.parametrize("heads,kv_heads", [(20, 4), (100, 20)])
+def test_prompt_attention_of_a_key_beyond_bfloat16_in_long_rows(heads, kv_heads):
+    """More heads than a workgroup of the fold has half wavefronts; a row of 12800 values,
+    which the kernel that writes its digits computes twice."""
+    before, n = 600, 9
+    shape = Shape(layers=2, hidden=256, heads=heads, kv_heads=kv_heads, head_dim=128, inter=256,
+                  vocab=320, max_len=before + n + 8)
+    toks = synthetic.first_tokens(shape, n, seed=4).astype(np.int32)
+    rows = []
+    for by_token in (False, True):
+        sess, _ = synthetic.build_session(shape, context=before, ln_jitter=0.1)
+        k = sess.get_kv(0)
+        k[kv_heads - 1, 77, 9] = 3.4e38
+        sess.set_kv(0, k)
+        if by_token:
+            for i, t in enumerate(toks):
+                sess.decode(int(t), before + i, want_logits=False)
+        else:
+            sess.prefill(toks, before)
+        rows.append([sess.get_kv(j)[:, before:before + n] for j in (2, 3)])
+        sess.close()
+    for got, want in zip(*rows):
+        assert np.isfinite(want).all()
+        check_close(got, want)
+
+
 @pytest.mark.parametrize("at", [0, 3, 4, 15, 16, 31, 63, 70])
 @pytest.mark.parametrize("size", [3.4e38, 8e38])  # above the largest bfloat16 value; infinite
 def test_prompt_attention_of_a_value_beyond_bfloat16(at, size):
