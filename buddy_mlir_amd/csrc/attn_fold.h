@@ -35,11 +35,9 @@ struct PromptFold {
   float scale = 0.f; // of the scores, times log2 e
 };
 
-// Short prompts at the start of a sequence are quicker with attn_prefill.hip, which needs
-// no partial results: 256 tokens take 18.3 us there and 18.8 here, 512 tokens 27.5 and 27.1
-// (a whole prompt of 512 4.83 ms there and 4.89 here), 1024 tokens 63 and 52; with 200
-// positions before 8 tokens 15.9 and 13.4, with 120 before 3 tokens 11.8 and 12.3.
-inline bool attn_prompt_pays(int q_len, int q_offset) { return q_len > 640 || q_offset >= 128; }
+// Whether launch_attn_prompt and the fold behind it are to be taken for a session's prompt, or
+// attn_prefill.hip and the conversion behind that; `digits`: the fold writes digit planes.
+bool attn_prompt_pays(int q_len, int q_offset, int heads, int kv_heads, bool digits);
 
 // Attention of a session's prompt tokens (no mask), on a workspace of
 // attn_prompt_workspace_bytes; what it leaves is described by `fold`.

@@ -16,14 +16,15 @@
 // phases, with the values a tile behind the scores: the same 6 us.)  What a launch costs
 // beside its tiles is some 9 us: the share, queries and their terms, the first tile's way.
 // 12 query heads, 2 KV heads, us per layer, this kernel and the fold behind it against
-// attn_prefill.hip and the conversion behind that:
-//   1931 tokens 112 vs 167, 4096 tokens 332 vs 655, 150 behind 1900 36 vs 106,
-//   27 behind 1900 24 vs 100, 512 tokens 27 vs 28, 256 tokens 18.8 vs 18.3, 27 tokens 17 vs 13
+// attn_prefill.hip and the conversion behind that (attn_prompt_pays says which is taken):
+//   2000 tokens 104 vs 156, 4096 tokens 332 vs 655, 150 behind 1900 36 vs 102,
+//   27 behind 1900 27 vs 98, 512 tokens 28 vs 25, 256 tokens 21 vs 17
 #include "attn.h"
 #include "attn_fold.h"
 #include "bf16_dev.h"
 
 #include <algorithm>
+#include <cmath>
 
 namespace bh {
 namespace {
@@ -483,6 +484,68 @@ attn_fold_rows_kernel(PromptFold f, float *out, int64_t o_stride, int heads) {
 
 } // namespace
 
+// The (KV head, row block, key tile) triples of a launch and who takes them.
+namespace {
+BH_TILE_FAMILY(PromptFamily, "attn_prompt_kernel");
+struct PromptShare {
+  int64_t rows, tiles; // rows of a KV head; tiles of all
+  int nblk, workgroups;
+};
+PromptShare share_out(int q_len, int q_offset, int heads, int kv_heads) {
+  PromptShare s;
+  const int group = heads / kv_heads;
+  s.rows = (int64_t)q_len * group;
+  s.nblk = (int)ceil_div(s.rows, kPromptRows);
+  s.tiles = 0;
+  for (int b = 0; b < s.nblk; ++b) {
+    const int64_t last = std::min((int64_t)(b + 1) * kPromptRows, s.rows) - 1;
+    s.tiles += ceil_div(q_offset + last / group + 1, kKeys);
+  }
+  s.tiles *= kv_heads;
+  s.workgroups = (int)std::min<int64_t>(kPromptWorkgroups, s.tiles); // each at least a tile
+  return s;
+}
+} // namespace
+
+// An estimate of both ways in microseconds, fitted to 528 launches of 1 to 64 heads, 1 to 16 KV
+// heads, 2 to 2000 tokens behind 0 to 1900.  Of those the choice is up to 15 % slower than the
+// better way and 0.5 % on average.  us, this way and the other, where the line lies:
+//   12 heads, 2 KV heads: 27 behind 128 15.8, 17.5, 300 behind 128 28.0, 24.5, behind 400 36.2,
+//     37.1, 512 alone 27.7, 25.3, 700 38.8, 35.0, 1024 49.3, 53.2
+//   64 and 8: 27 behind 128 24.7, 20.0, 300 behind 128 51.9, 56.1, 640 alone 84.8, 106
+//   one head: 300 behind 64 19.0, 20.9, 8 behind 128 12.4, 10.7
+// The estimate is off by a tenth here and there.  More than 640 tokens go this way in doubt,
+// which keeps what is not finite to the rows that see it (700 tokens of 6 heads, one KV head:
+// 28.5 and 29.3); short prompts with little ahead of them the other.
+bool attn_prompt_pays(int q_len, int q_offset, int heads, int kv_heads, bool digits) {
+  const double kilo_rows = 1e-4 * q_len * heads; // tens of thousands of (token, head)
+  // attn_prefill.hip: blocks of 16 queries, two together while a workgroup of eight wavefronts
+  // per pair fits the chip; steps of 16 keys per wavefront
+  const int64_t nqb = ceil_div(q_len, 16);
+  double steps;
+  if (nqb == 1)
+    steps = (double)ceil_div(q_offset + q_len, 16) / 8;
+  else if (heads * ceil_div(nqb, 2) <= 256)
+    steps = (2.0 * q_offset + q_len + 16) / 128;
+  else
+    steps = (1.0 * heads * q_len * q_len / (16 * 32 * 256) +
+             (double)ceil_div(heads * nqb, 256) * q_offset / 16) / 8;
+  const double other = 7.9 + (nqb > 1 ? 2.1 : 0.0) + 3.0 * steps + 5.8 * kilo_rows;
+  // here: tiles of the longest share, wavefronts that have rows, blocks that begin and end, and
+  // the fold's trips to memory and its bytes
+  const PromptShare s = share_out(q_len, q_offset, heads, kv_heads);
+  const double share = (double)s.tiles / s.workgroups;
+  const double parts = (double)ceil_div(q_offset + q_len, kKeys) / share;
+  const int64_t waves = std::min<int64_t>(8, ceil_div(s.rows, 32));
+  const double trips = parts <= 4 ? 1 : parts <= 8 ? 2 : 2 * std::ceil(parts / 16);
+  const double here = 10.6 + 5.7 * (double)(ceil_div(s.tiles, s.workgroups) - 1) +
+                      1.4 * (double)std::max<int64_t>(0, waves - 4) + 5.0 * s.workgroups / 256 +
+                      2.0 * s.nblk * kv_heads / s.workgroups + (double)ceil_div(heads, 16) * trips +
+                      0.82 * kilo_rows * std::min(parts, 20.0) +
+                      (digits ? 0.0 : 3.0); // bfloat16 modes convert the fold's rows in a launch of its own
+  return here < (q_len > 640 ? 1.08 : q_offset >= 128 ? 1.0 : 0.9) * other;
+}
+
 size_t attn_prompt_workspace_bytes(int q_len, int heads, int kv_heads) {
   const size_t blocks = (size_t)kv_heads * ceil_div((int64_t)q_len * (heads / kv_heads), kPromptRows);
   return kPromptSlots * kPromptRows * (kPromptD + 2) * sizeof(float) + blocks * sizeof(PromptBlock);
@@ -516,27 +579,20 @@ int launch_attn_prompt(const AttnPrefillArgs &in, void *workspace, PromptFold &f
   a.k_len = in.k_len;
   a.q_offset = in.k_len - in.q_len;
   a.scale = (float)(in.scale * 1.4426950408889634);
-  const int64_t rows = (int64_t)in.q_len * a.group;
-  BH_REQUIRE(rows < (1 << 30), "attn_prompt: q_len %d too long", in.q_len);
-  a.nblk = (int)ceil_div(rows, kPromptRows);
+  BH_REQUIRE((int64_t)in.q_len * a.group < (1 << 30), "attn_prompt: q_len %d too long", in.q_len);
+  const PromptShare share = share_out(in.q_len, a.q_offset, in.heads, in.kv_heads);
+  BH_REQUIRE(share.tiles < (1u << 30), "attn_prompt: %lld tiles of keys", (long long)share.tiles);
+  a.nblk = share.nblk;
   a.acc = static_cast<float *>(workspace);
   a.ml = a.acc + kPromptSlots * kPromptRows * kPromptD;
   a.blocks = reinterpret_cast<PromptBlock *>(a.ml + kPromptSlots * kPromptRows * 2);
-  int64_t tiles = 0;
-  for (int b = 0; b < a.nblk; ++b) {
-    const int64_t last = std::min((int64_t)(b + 1) * kPromptRows, rows) - 1;
-    tiles += ceil_div(std::min<int64_t>(in.k_len, a.q_offset + last / a.group + 1), kKeys);
-  }
-  tiles *= in.kv_heads;
-  // every workgroup at least a tile
-  BH_REQUIRE(tiles < (1u << 30), "attn_prompt: %lld tiles of keys", (long long)tiles);
-  const int G = (int)std::min<int64_t>(kPromptWorkgroups, tiles);
-  a.per_head = (int)(tiles / in.kv_heads);
-  a.share = (int)(tiles / G);
-  a.extra = (int)(tiles % G);
+  a.per_head = (int)(share.tiles / in.kv_heads);
+  a.share = (int)(share.tiles / share.workgroups);
+  a.extra = (int)(share.tiles % share.workgroups);
+  BH_NOTE_VARIANT(PromptFamily, kPromptRows);
   static DynLdsOnce dyn_lds;
   BH_CHECK_HIP(ensure_dyn_lds(dyn_lds, reinterpret_cast<const void *>(attn_prompt_kernel), kLds));
-  hipLaunchKernelGGL(attn_prompt_kernel, dim3((unsigned)G), dim3(kThreads), kLds, stream, a.k, a.v,
+  hipLaunchKernelGGL(attn_prompt_kernel, dim3((unsigned)share.workgroups), dim3(kThreads), kLds, stream, a.k, a.v,
                      a.kv_stride, a.share, a.extra, a.per_head, a.nblk, a.group, a.q_len, a.k_len, a.q_offset, a);
   BH_CHECK_HIP(hipGetLastError());
   fold.out = in.out;

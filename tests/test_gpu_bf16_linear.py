@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import nukopel_oracle as N
-from test_gpu_variant_coverage import tiles_run
+from tile_report import tiles_run
 
 pytestmark = pytest.mark.gpu
 

@@ -14,7 +14,7 @@ import nukopel_models as M
 import nukopel_oracle as N
 from buddy_mlir_amd import BuddyHipError
 from buddy_mlir_amd.session import FolderSession, Sampler
-from test_gpu_variant_coverage import tiles_run
+from tile_report import tiles_run
 
 pytestmark = pytest.mark.gpu
 

@@ -12,6 +12,7 @@ from buddy_mlir_amd.session import Shape
 from buddy_mlir_amd.session import DecoderSession
 from parity import check_close
 from test_gpu_decode import SMALL, oracle_model
+from tile_report import tiles_run
 
 pytestmark = pytest.mark.gpu
 
@@ -473,6 +474,33 @@ def test_prompt_attention_equals_token_by_token(heads, kv_heads, before, n):
         sess.close()
 
 
+# on both sides of the line between the two attentions: one token, behind whole key tiles and
+# behind a last one of a single key; tokens that fill blocks of 256 rows and some that do not;
+# few heads and many
+@pytest.mark.parametrize("heads,kv_heads,before,n,precision,split", [
+    (6, 1, 128, 1, "digits", 0), (6, 1, 600, 1, "digits", 1), (6, 1, 607, 1, "exact", 1),
+    (8, 1, 129, 32, "exact", 0), (8, 1, 600, 32, "exact", 1), (12, 2, 128, 300, "digits", 0),
+    (12, 2, 400, 300, "digits", 1), (12, 2, 0, 801, "digits", 0), (12, 2, 0, 901, "digits", 1),
+    (64, 8, 128, 27, "digits", 0), (64, 8, 1200, 33, "digits", 1), (1, 1, 128, 96, "exact", 1)])
+def test_which_prompt_attention(bh, heads, kv_heads, before, n, precision, split):
+    shape = Shape(layers=2, hidden=256, heads=heads, kv_heads=kv_heads, head_dim=128, inter=256,
+                  vocab=320, max_len=before + n + 8)
+    toks = synthetic.first_tokens(shape, n, seed=before + n).astype(np.int32)
+    sess, _ = synthetic.build_session(shape, context=before, ln_jitter=0.1)
+    bh.buddy_hip_variant_reset()
+    _, got = sess.prefill(toks, before, precision=precision)
+    assert tiles_run(bh)["attn_prompt_kernel<256>"] == split * shape.layers
+    rows = [sess.get_kv(j)[:, before:before + n] for j in (2, 3)]
+    sess.close()
+    sess, _ = synthetic.build_session(shape, context=before, ln_jitter=0.1)
+    for i, t in enumerate(toks):
+        _, want = sess.decode(int(t), before + i, want_logits=i + 1 == n)
+    check_close(got, want)
+    for j in (2, 3):
+        check_close(rows[j - 2], sess.get_kv(j)[:, before:before + n])
+    sess.close()
+
+
 @pytest.mark.parametrize("bad", [float("nan"), float("inf")])
 def test_prompt_attention_keeps_non_finite_tokens_from_earlier_rows(bad):
     """A token in the middle of a long prompt whose embedding is not finite: rows that do not
@@ -534,7 +562,7 @@ def test_prompt_attention_of_a_key_beyond_bfloat16(bad, precision):
 def test_prompt_attention_of_a_key_beyond_bfloat16_in_long_rows(heads, kv_heads):
     """More heads than a workgroup of the fold has half wavefronts; a row of 12800 values,
     which the kernel that writes its digits computes twice."""
-    before, n = 600, 9
+    before, n = 600, 17
     shape = Shape(layers=2, hidden=256, heads=heads, kv_heads=kv_heads, head_dim=128, inter=256,
                   vocab=320, max_len=before + n + 8)
     toks = synthetic.first_tokens(shape, n, seed=4).astype(np.int32)
@@ -563,7 +591,7 @@ def test_prompt_attention_of_a_value_beyond_bfloat16(at, size):
     the token are what they are without, bit for bit, also in its tile of 32 keys.  Behind it
     a huge value changes its own channel alone (o_proj takes nothing from that channel, and
     the other channels give what they give without it); an infinite one makes NaN of 0 * inf."""
-    before, n, c, big = 128, 96, 5, 310
+    before, n, c, big = 192, 96, 5, 310
     shape = Shape(layers=2, hidden=256, heads=2, kv_heads=1, head_dim=128, inter=256, vocab=320,
                   max_len=before + n + 8)
 

@@ -19,6 +19,7 @@ import oracle_lib
 from buddy_mlir_amd import ops, synthetic
 from buddy_mlir_amd.session import Shape
 from parity import check_close
+from tile_report import tiles_run
 from test_gpu_prefill import (SCALE, SILU_PAIR_SHAPES, bf16_round, fixed_point_round, run_attn,
                               silu_pair_case)
 
@@ -34,15 +35,6 @@ def report(bh):
         name, hits = line.split("\t")
         out[name] = int(hits)
     return out
-
-
-def tiles_run(bh):
-    """Launches of the matrix products whose tile an estimate picks, by tile."""
-    n = bh.buddy_hip_tile_report(None, 0)
-    buf = ctypes.create_string_buffer(n)
-    bh.buddy_hip_tile_report(buf, n)
-    return {name: int(hits) for name, hits in
-            (line.split("\t") for line in buf.value.decode().splitlines())}
 
 
 def launched(bh, family):
