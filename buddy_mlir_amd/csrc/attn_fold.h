@@ -15,7 +15,6 @@ namespace bh {
 constexpr int kPromptRows = 256;       // rows of a block
 constexpr int kPromptD = 128;          // head size
 constexpr int kPromptWorkgroups = 256; // at most, each with up to two partial results
-constexpr size_t kPromptSlots = 2 * kPromptWorkgroups;
 
 // Where the parts of a block lie: part 0 in slot `first`, part j > 0 in slot
 // 2 * (owner + j).  parts == 0: the finished rows are in the output already.
@@ -40,9 +39,10 @@ struct PromptFold {
 bool attn_prompt_pays(int q_len, int q_offset, int heads, int kv_heads, bool digits);
 
 // Attention of a session's prompt tokens (no mask), on a workspace of
-// attn_prompt_workspace_bytes; what it leaves is described by `fold`.
+// attn_prompt_workspace_bytes for at least as many tokens and positions; what it leaves is
+// described by `fold`.
 struct AttnPrefillArgs;
-size_t attn_prompt_workspace_bytes(int q_len, int heads, int kv_heads);
+size_t attn_prompt_workspace_bytes(int q_len, int k_len, int heads, int kv_heads);
 int launch_attn_prompt(const AttnPrefillArgs &a, void *workspace, PromptFold &fold, hipStream_t stream);
 // the finished rows [tokens, heads, 128] in place ...
 int launch_attn_fold_rows(const PromptFold &fold, float *out, int64_t o_stride, int heads, int tokens,

@@ -546,9 +546,11 @@ bool attn_prompt_pays(int q_len, int q_offset, int heads, int kv_heads, bool dig
   return here < (q_len > 640 ? 1.08 : q_offset >= 128 ? 1.0 : 0.9) * other;
 }
 
-size_t attn_prompt_workspace_bytes(int q_len, int heads, int kv_heads) {
-  const size_t blocks = (size_t)kv_heads * ceil_div((int64_t)q_len * (heads / kv_heads), kPromptRows);
-  return kPromptSlots * kPromptRows * (kPromptD + 2) * sizeof(float) + blocks * sizeof(PromptBlock);
+// Two slots for every workgroup there can be: 67 MB where all compute units have tiles.
+size_t attn_prompt_workspace_bytes(int q_len, int k_len, int heads, int kv_heads) {
+  const int64_t blocks = (int64_t)kv_heads * ceil_div((int64_t)q_len * (heads / kv_heads), kPromptRows);
+  const size_t slots = 2 * (size_t)std::min<int64_t>(kPromptWorkgroups, blocks * ceil_div(k_len, kKeys));
+  return slots * kPromptRows * (kPromptD + 2) * sizeof(float) + (size_t)blocks * sizeof(PromptBlock);
 }
 
 int launch_attn_prompt(const AttnPrefillArgs &in, void *workspace, PromptFold &fold, hipStream_t stream) {
@@ -584,8 +586,9 @@ int launch_attn_prompt(const AttnPrefillArgs &in, void *workspace, PromptFold &f
   BH_REQUIRE(share.tiles < (1u << 30), "attn_prompt: %lld tiles of keys", (long long)share.tiles);
   a.nblk = share.nblk;
   a.acc = static_cast<float *>(workspace);
-  a.ml = a.acc + kPromptSlots * kPromptRows * kPromptD;
-  a.blocks = reinterpret_cast<PromptBlock *>(a.ml + kPromptSlots * kPromptRows * 2);
+  const size_t slots = 2 * (size_t)share.workgroups;
+  a.ml = a.acc + slots * kPromptRows * kPromptD;
+  a.blocks = reinterpret_cast<PromptBlock *>(a.ml + slots * kPromptRows * 2);
   a.per_head = (int)(share.tiles / in.kv_heads);
   a.share = (int)(share.tiles / share.workgroups);
   a.extra = (int)(share.tiles % share.workgroups);

@@ -416,8 +416,8 @@ struct Qwen2Session : Session {
     BH_CHECK_HIP(hipGetLastError());
     int rc;
     const bool folded = attn_prompt_pays(n, start_pos, S.heads, S.kv_heads, gemm_digits != 0);
-    if (folded && !pf_attn_ws) // for as many rows as the other buffers have
-      BH_CHECK_HIP(hipMalloc(&pf_attn_ws, attn_prompt_workspace_bytes(pf_rows, S.heads, S.kv_heads)));
+    if (folded && !pf_attn_ws) // for as many rows as the other buffers have, behind any context
+      BH_CHECK_HIP(hipMalloc(&pf_attn_ws, attn_prompt_workspace_bytes(pf_rows, S.max_len, S.heads, S.kv_heads)));
     bool normed_ahead = false; // pf_xn_bf already holds this layer's normed input
     for (int i = 0; i < S.layers; ++i) {
       Layer &L = layers[(size_t)i];

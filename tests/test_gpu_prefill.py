@@ -501,6 +501,22 @@ def test_which_prompt_attention(bh, heads, kv_heads, before, n, precision, split
     sess.close()
 
 
+def test_workspace_of_the_prompt_attention_follows_the_session(bh):
+    """One KV head behind 640 positions has 20 tiles of keys for 20 workgroups: 5 MB of partial
+    results, not the 67 MB of a full chip."""
+    shape = Shape(layers=1, hidden=256, heads=6, kv_heads=1, head_dim=128, inter=256, vocab=320,
+                  max_len=640)
+    sess, _ = synthetic.build_session(shape, context=600, ln_jitter=0.1)
+    sess.prefill(np.arange(30, dtype=np.int32), 0)  # the other buffers
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    bh.buddy_hip_variant_reset()
+    sess.prefill(np.arange(30, dtype=np.int32), 600)
+    assert tiles_run(bh)["attn_prompt_kernel<256>"] == 1
+    assert free - torch.cuda.mem_get_info()[0] < 16 << 20
+    sess.close()
+
+
 @pytest.mark.parametrize("bad", [float("nan"), float("inf")])
 def test_prompt_attention_keeps_non_finite_tokens_from_earlier_rows(bad):
     """A token in the middle of a long prompt whose embedding is not finite: rows that do not
