@@ -18,10 +18,11 @@
 //  * workgroups take 32 or 64 rows x 128 or 256 channels, and K is split over
 //    several of them where a matrix is too narrow to fill the chip;
 //  * workgroup ids are laid out so that the row tiles of one column tile run
-//    on the same XCD (ids equal modulo 8) and share the weight tiles in its L2;
+//    on the same XCD and share the weight tiles in its L2 (tile_place.h);
 //  * the per-channel scale is applied once to the f32 accumulators, where the
 //    reference multiplies every element before the FMA.
 #include "gemm.h"
+#include "tile_place.h"
 
 #include <algorithm>
 #include <map>
@@ -177,7 +178,7 @@ struct GemmArgs {
   // K split over `slices` workgroups per tile, chunks_per_slice chunks of 64 each (the last
   // may hold fewer, never none)
   int slices, chunks_per_slice;
-  int ids_padded, row_tiles; // ids per row tile: ncols x slices, padded to the XCD count
+  int row_tiles, panel;      // and how the tiles are placed
   float *partial;            // [tile][slice][wavefront][row][channel], where K is split
   int span, tile_rows;       // channels per wavefront, rows per workgroup
   int accumulate;
@@ -208,11 +209,9 @@ __device__ __forceinline__ void multiply_tile(const GemmArgs &a) {
   __shared__ __attribute__((aligned(16))) float scale_s[kWaves * kSpan], bias_s[kWaves * kSpan];
   const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, up = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // ids equal modulo 8 run on the same XCD: the row tiles of one (column tile, K slice) do,
-  // and share its weights in that XCD's L2
-  const int unit = blockIdx.x % a.ids_padded, rbk = blockIdx.x / a.ids_padded;
-  if (unit >= a.ncols * a.slices)
-    return; // padding id
+  int unit, rbk;
+  if (!place_tile(a.ncols * a.slices, a.row_tiles, a.panel, unit, rbk))
+    return;
   const int ctile = unit % a.ncols, slice = unit / a.ncols;
   const int m0 = rbk * kRows;
   const int g0 = (ctile * kWaves + wave) * (kSpan / 16); // first channel group of this wavefront
@@ -403,7 +402,7 @@ __device__ __forceinline__ void multiply_tile(const GemmArgs &a) {
 // with -amdgpu-kernarg-preload-count); the rest is loaded behind the fetch.
 #define BH_BF16_LEADING                                                                            \
   const u16 *Abf, const int4 *W, int Mp, int Kp, int groups, int chunks, int ncols, int slices,    \
-      int chunks_per_slice, int ids_padded, GemmArgs a
+      int chunks_per_slice, int row_tiles, int panel, GemmArgs a
 #define BH_BF16_TAKE                                                                               \
   a.Abf = Abf;                                                                                     \
   a.W = W;                                                                                         \
@@ -414,7 +413,8 @@ __device__ __forceinline__ void multiply_tile(const GemmArgs &a) {
   a.ncols = ncols;                                                                                 \
   a.slices = slices;                                                                               \
   a.chunks_per_slice = chunks_per_slice;                                                           \
-  a.ids_padded = ids_padded;
+  a.row_tiles = row_tiles;                                                                         \
+  a.panel = panel;
 
 // Blocks of 32 rows per workgroup.
 constexpr int row_blocks(int terms, int gp) { return terms == 1 && gp == 2 ? 2 : 1; }
@@ -520,7 +520,7 @@ BH_VARIANT_FAMILY(NarrowFamily, "gemm_w8_bf16_kernel");
 template <class Kernel>
 int launch_tiles(Kernel kernel, const GemmArgs &a, unsigned blocks, hipStream_t stream) {
   hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kWaves * kWave), 0, stream, a.Abf, a.W, a.Mp, a.Kp,
-                     a.groups, a.chunks, a.ncols, a.slices, a.chunks_per_slice, a.ids_padded, a);
+                     a.groups, a.chunks, a.ncols, a.slices, a.chunks_per_slice, a.row_tiles, a.panel, a);
   BH_CHECK_HIP(hipGetLastError());
   return BUDDY_HIP_OK;
 }
@@ -551,7 +551,7 @@ TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, int terms, bool may
     const double alone = gp == 2 ? 0.34 + 0.16 * layers : 0.20 + 0.075 * layers;
     const double full = gp == 2 ? 0.14 + 0.38 * layers : 0.24 + 0.21 * layers;
     for (int s = 1; s <= (may_split ? 16 : 1); ++s) {
-      const int64_t per_xcd = ceil_div(ncols * s, 8) * rows;
+      const int64_t per_xcd = ceil_div(ncols * s * rows, 8);
       if (s > 1 && per_xcd > 256)
         break;
       const int64_t cps = ceil_div(chunks, s);
@@ -579,7 +579,6 @@ int launch_plan(const TilePlan &plan, GemmArgs &a, int terms, hipStream_t stream
   a.row_tiles = (int)ceil_div(a.M, a.tile_rows);
   a.slices = plan.slices;
   a.chunks_per_slice = (int)ceil_div(a.chunks, plan.slices);
-  a.ids_padded = (int)round_up((int64_t)a.ncols * a.slices, 8);
   a.partial = nullptr;
   if (a.slices > 1) {
     const size_t tile_floats = (size_t)a.tile_rows * kWaves * a.span;
@@ -591,7 +590,11 @@ int launch_plan(const TilePlan &plan, GemmArgs &a, int terms, hipStream_t stream
       return launch_plan(plan_tiles(a.M, a.N, a.chunks, terms, false), a, terms, stream);
     a.partial = reinterpret_cast<float *>(ws);
   }
-  const unsigned blocks = (unsigned)a.ids_padded * a.row_tiles;
+  const int64_t units = (int64_t)a.ncols * a.slices;
+  a.panel = panel_for(units, a.row_tiles);
+  const int64_t tiles = (a.panel ? units : round_up(units, 8)) * a.row_tiles;
+  BH_REQUIRE(tiles < (1u << 31), "gemm_w8: %lld tiles", (long long)tiles);
+  const unsigned blocks = (unsigned)tiles;
   int rc;
   if (plan.gp == 1) {
     if (terms == 1) {

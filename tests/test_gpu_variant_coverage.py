@@ -301,6 +301,14 @@ def test_bf16_matmul_tile_edges(M, K, N):
             assert (err <= 4 * np.sqrt(K + 16) * 2.0**-24 * size).all()
 
 
+# tiles shared out to the dies in panels of 1, 2 and 4 columns and without; a last panel that
+# is narrower, and totals that eight does not divide
+@pytest.mark.parametrize("M,K,N", [(150, 64, 700), (321, 130, 1100), (700, 72, 1300),
+                                   (1100, 200, 1300), (2500, 72, 514), (4100, 64, 2700)])
+def test_bf16_matmul_panels(M, K, N):
+    test_bf16_matmul_tile_edges(M, K, N)
+
+
 @pytest.mark.parametrize("M,K,N", [(17, 64, 16), (27, 1536, 8960), (32, 200, 48), (31, 320, 4496)])
 @pytest.mark.parametrize("digits", [2, 3])
 def test_silu_pair_of_few_rows(bh, oracle, M, K, N, digits):
