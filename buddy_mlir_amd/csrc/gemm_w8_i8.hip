@@ -1018,6 +1018,7 @@ namespace {
 //     1024: 17.2 [30.4]; 14.4 [22.7]
 //   4096 -> 2 x 14336 with the conversion: 1024 rows 361 (359) [343]; 252 (288) [265],
 //     4096: 1320 (1391) [1372]; 980 (1075) [1042]
+//   14336 -> 4096 with both: 33 rows 34.3 [32.6]; 26.7 [29.6], 768: 156 [148]; 108 [143]
 //   one plane: 1536 -> 8960: 256 rows 14 (18) [18], 512: 18.6 [21.2], 2048: 52 [69]
 // (gate | up at 27 rows with two channel tiles: 13.7, and 18.7 in a prompt, whose weights come
 // from memory, against 14.9 with one: twice the compute units ask for them.)
@@ -1033,11 +1034,11 @@ struct TileShape {
 constexpr TileShape kTiles1[] = {{1, 1, true, 0.21, 4.5, 0.285, 4.5},
                                  {wide_blocks(1), 2, true, 0.33, 5.0, 0.54, 4.0},
                                  {3, 2, true, 0.39, 5.0, 0.66, 4.0}};
-constexpr TileShape kTiles2[] = {{1, 1, true, 0.21, 4.5, 0.37, 4.5},
-                                 {wide_blocks(2), 2, true, 0.295, 4.7, 0.50, 4.0},
-                                 {2, 2, false, 0.44, 5.2, 0, 0},
-                                 {1, 3, true, 0.39, 5.0, 0.73, 4.2},
-                                 {3, 2, false, 0.59, 6.0, 0, 0}};
+constexpr TileShape kTiles2[] = {{1, 1, true, 0.232, 4.6, 0.33, 3.8},
+                                 {wide_blocks(2), 2, true, 0.34, 5.2, 0.50, 6.1},
+                                 {2, 2, false, 0.446, 6.8, 0, 0},
+                                 {1, 3, true, 0.428, 6.0, 0.71, 8.3},
+                                 {3, 2, false, 0.606, 8.1, 0, 0}};
 constexpr TileShape kTiles3[] = {{1, 1, true, 0.27, 4.5, 0.455, 4.5},
                                  {wide_blocks(3), 2, true, 0.35, 4.7, 0.66, 4.0},
                                  {2, 2, false, 0.60, 5.8, 0, 0},

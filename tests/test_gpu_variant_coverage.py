@@ -326,7 +326,7 @@ def test_silu_pair_of_few_rows(bh, oracle, M, K, N, digits):
 TALL = {(3, 2, 2, 0): [(385, 2000, 5001), (770, 8950, 1531)], (3, 2, 2, 1): [(97, 2000, 8976)],
         (3, 1, 5, 0): [(513, 200, 8890)], (3, 1, 5, 1): [(225, 65, 8976)],
         (2, 2, 2, 0): [(225, 1530, 12801), (97, 4100, 8890)], (2, 2, 2, 1): [(97, 1530, 12800)],
-        (2, 1, 3, 0): [(513, 65, 8890), (513, 4100, 1111)], (2, 1, 3, 1): [(257, 65, 8976)],
+        (2, 1, 3, 0): [(257, 65, 8890), (641, 8950, 1111)], (2, 1, 3, 1): [(225, 65, 4496)],
         (2, 3, 2, 0): [(385, 1000, 12801)], (2, 3, 2, 1): [(225, 1000, 8976)],
         (1, 3, 2, 0): [(777, 65, 12801), (65, 4100, 12801)]}
 
