@@ -15,7 +15,10 @@ namespace bh {
 namespace {
 
 constexpr int kRowThreads = 512, kRowWaves = kRowThreads / 64;
-constexpr int kAhead = 8; // weight tiles a wavefront keeps in flight
+// Weight tiles a wavefront keeps in flight, of each matrix: with the slices below, the whole
+// run at an input width of 1536.  gate | up 1536 -> 2 x 8960 (55 MB) takes 12.3 us with 6 and
+// 12.5 with 4, 14.4 with gate and up on wavefronts of their own and eight tiles each.
+constexpr int kAhead = 6;
 
 __global__ void __launch_bounds__(256)
 pack_bf16_kernel(const uint16_t *__restrict__ src, int64_t sn, int64_t sk, int N, int K, int ktiles,
@@ -52,6 +55,41 @@ __device__ __forceinline__ float dot_tile(const uint4 w, const float *a, float a
   acc = fmaf(bf_hi(w.w), hi[3], acc);
   return acc;
 }
+
+// A wavefront's run of tiles [t0, t1) of MATS matrices along the same k, U tiles of each in
+// flight.  A tile's registers take the next one as soon as they are read, and the
+// activations of a k come out of LDS once for all matrices.
+template <int MATS, int U> struct TileRun {
+  uint4 w[MATS][U];
+  const uint4 *wp[MATS];
+  __device__ __forceinline__ void request(int t0, int t1) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int m = 0; m < MATS; ++m)
+        w[m][u] = wp[m][(int64_t)min(t0 + u, t1 - 1) * 64];
+  }
+  __device__ __forceinline__ void run(const float *ap, int t0, int t1, float (&acc)[MATS]) {
+    int t = t0;
+    for (; t + U < t1; t += U) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+#pragma unroll
+        for (int m = 0; m < MATS; ++m) {
+          acc[m] = dot_tile(w[m][u], ap + (t + u) * kBfTileK, acc[m]);
+          w[m][u] = wp[m][(int64_t)min(t + U + u, t1 - 1) * 64];
+        }
+        __builtin_amdgcn_sched_barrier(0); // else all refills move up and take registers of their own
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (t + u < t1)
+#pragma unroll
+        for (int m = 0; m < MATS; ++m)
+          acc[m] = dot_tile(w[m][u], ap + (t + u) * kBfTileK, acc[m]);
+  }
+};
 
 // sum over the workgroup; `red` is used once per call site
 __device__ __forceinline__ float block_sum(float v, float *red) {
@@ -100,6 +138,43 @@ __device__ __forceinline__ void keep_row(const RowTail &a, int K, int p, int i, 
   a.conv_next[(int64_t)((p + 1) & 1) * K + i] = c;
 }
 
+// The same for four values at a time and up to four taps.  The launch lasts as long as the
+// workgroup that does this, so the earlier rows and the weights are asked for ahead of the
+// norms and not at their use.
+template <int R> struct RowKeeper {
+  static constexpr int kTaps = 4;
+  f32x4 e[kTaps - 2][R], w[kTaps - 1][R]; // row p + 1 - b in e[b - 2], its weight in w[b - 1]
+  static __device__ __forceinline__ bool fits(const RowTail &a) { return a.conv_w && a.taps <= kTaps; }
+  static __device__ __forceinline__ int slot(const RowTail &a, int p, int b) {
+    const int s = p % a.taps + 1 - b;
+    return s < 0 ? s + a.taps : s;
+  }
+  __device__ __forceinline__ void request(const RowTail &a, int K, int p, const int (&at)[R],
+                                          const bool (&in)[R]) {
+#pragma unroll
+    for (int b = 1; b < kTaps; ++b)
+      if (b < a.taps)
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const int i = in[r] ? at[r] : 0;
+          w[b - 1][r] = load4(a.conv_w + (int64_t)(a.taps - 1 - b) * K + i);
+          if (b > 1 && b <= p + 1)
+            e[b - 2][r] = load4(a.conv_ring + (int64_t)slot(a, p, b) * K + i);
+        }
+  }
+  __device__ __forceinline__ void store(const RowTail &a, int K, int p, int r, int i, f32x4 h) const {
+    save4(a.conv_ring + (int64_t)slot(a, p, 1) * K + i, h);
+    f32x4 c{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int b = kTaps - 1; b >= 1; --b)
+      if (b < a.taps && b <= p + 1)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          c[j] = fmaf(w[b - 1][r][j], b == 1 ? h[j] : e[b > 1 ? b - 2 : 0][r][j], c[j]);
+    save4(a.conv_next + (int64_t)((p + 1) & 1) * K + i, c);
+  }
+};
+
 // The finished input row into act[0 .. Kp).  R > 0: K is a multiple of 4 and at most
 // 2048 * R, and every thread keeps its 4 * R values in registers from one trip to
 // memory.  R = 0: any K.  `keeper`: this workgroup stores what the row leaves behind.
@@ -107,11 +182,12 @@ template <int INPUT, int R>
 struct RowPrologue {
   f32x4 x[R], y[R], c[2][R], w[R];
   const float *yp;
-  int at[R];
+  int at[R], p;
   bool in[R];
   __device__ __forceinline__ void request(const float *src, const float *ysrc, const float *conv_next,
                                           int K, const RowTail &a) {
     yp = ysrc;
+    p = INPUT == kRowNorm && a.conv_w ? *a.pos : 0;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       at[r] = (r * kRowThreads + (int)threadIdx.x) * 4;
@@ -203,6 +279,12 @@ struct RowPrologue {
           save4(a.row_out + at[r], x[r]);
       }
     } else if constexpr (INPUT == kRowNorm) {
+      constexpr bool kAhead = R <= 2; // beyond that its registers are too many
+      RowKeeper<kAhead ? R : 1> kept;
+      const bool quick = kAhead && keeper && kept.fits(a);
+      if constexpr (kAhead)
+        if (quick)
+          kept.request(a, K, p, at, in);
       if (yp) {
         const float ry = a.out_gain / sqrtf(block_sum(squares(y), red[0]) / (float)K + a.eps);
 #pragma unroll
@@ -215,7 +297,6 @@ struct RowPrologue {
         }
       }
       const float g = a.gain / sqrtf(block_sum(squares(x), red[1]) / (float)K + a.eps);
-      const int p = a.conv_w ? *a.pos : 0;
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         f32x4 h;
@@ -227,10 +308,14 @@ struct RowPrologue {
 #pragma unroll
           for (int j = 0; j < 4; ++j)
             x[r][j] += fmaf(w[r][j], h[j], p == 0 ? 0.f : p & 1 ? c[1][r][j] : c[0][r][j]);
-          if (keeper && in[r])
+          if (quick && in[r]) {
+            if constexpr (kAhead)
+              kept.store(a, K, p, r, at[r], h);
+          } else if (keeper && in[r]) {
 #pragma unroll
             for (int j = 0; j < 4; ++j)
               keep_row(a, K, p, at[r] + j, h[j]);
+          }
         }
         if (keeper && a.row_out && in[r])
           save4(a.row_out + at[r], x[r]);
@@ -332,7 +417,7 @@ struct RowPrologue<INPUT, 0> {
 // Grid: workgroups of 8 wavefronts = (8 >> ks_shift) channel groups x (1 <<
 // ks_shift) slices of k that meet in LDS in slice order.  kRowNorm, kRowResidual: one
 // workgroup more, which multiplies nothing and stores what the row leaves behind.
-// GATED: neighbouring channel groups are group i of one matrix and of the other.
+// GATED: a wavefront has group g of both matrices.  `groups`: of one matrix.
 template <int INPUT, int R, bool GATED>
 __global__ void __launch_bounds__(kRowThreads)
 row_gemv_kernel(const uint4 *__restrict__ W, const float *__restrict__ src,
@@ -340,7 +425,8 @@ row_gemv_kernel(const uint4 *__restrict__ W, const float *__restrict__ src,
                 int ks_shift, int slice_tiles, RowTail a) {
   extern __shared__ __attribute__((aligned(16))) float act[]; // [Kp]
   __shared__ float red[2][kRowWaves];
-  __shared__ float part[kRowWaves][16];
+  constexpr int kMats = GATED ? 2 : 1;
+  __shared__ float part[kMats][kRowWaves][16];
   const int Kp = ktiles * kBfTileK;
   const int tid = threadIdx.x, lane = tid & 63;
   // the row's values first: loads return in order, and these come from the L2
@@ -355,48 +441,33 @@ row_gemv_kernel(const uint4 *__restrict__ W, const float *__restrict__ src,
   const int g = blockIdx.x * (kRowWaves >> ks_shift) + (wave >> ks_shift);
   const int gl = min(g, groups - 1); // a wavefront past the last group repeats it and stores nothing
   const int t0 = slice * slice_tiles, t1 = min(t0 + slice_tiles, ktiles);
-  const uint4 *wp = W + (int64_t)(GATED ? (gl & 1) * (groups >> 1) + (gl >> 1) : gl) * ktiles * 64 + lane;
-  uint4 w[kAhead];
+  TileRun<kMats, kAhead> tiles;
 #pragma unroll
-  for (int u = 0; u < kAhead; ++u)
-    w[u] = wp[(int64_t)min(t0 + u, ktiles - 1) * 64];
+  for (int m = 0; m < kMats; ++m)
+    tiles.wp[m] = W + (int64_t)(m * groups + gl) * ktiles * 64 + lane;
+  tiles.request(t0, t1);
   row.finish(act, K, Kp, a, false, red);
   __syncthreads();
 
-  const float *ap = act + (lane >> 4) * 8;
-  float acc = 0.f;
-  for (int t = t0; t < t1; t += kAhead) {
-    uint4 n[kAhead];
-    const bool more = t + kAhead < t1;
-    if (more) {
+  float acc[kMats] = {};
+  tiles.run(act + (lane >> 4) * 8, t0, t1, acc);
 #pragma unroll
-      for (int u = 0; u < kAhead; ++u)
-        n[u] = wp[(int64_t)min(t + kAhead + u, ktiles - 1) * 64];
-    }
-#pragma unroll
-    for (int u = 0; u < kAhead; ++u)
-      if (t + u < t1)
-        acc = dot_tile(w[u], ap + (t + u) * kBfTileK, acc);
-    if (more) {
-#pragma unroll
-      for (int u = 0; u < kAhead; ++u)
-        w[u] = n[u];
-    }
+  for (int m = 0; m < kMats; ++m) {
+    acc[m] = sum_rows(acc[m]);
+    if (lane < 16)
+      part[m][wave][lane] = acc[m];
   }
-  acc = sum_rows(acc);
-  if (lane < 16)
-    part[wave][lane] = acc;
   __syncthreads();
   const int gi = tid >> 4;
   if constexpr (GATED) {
-    if (gi < (kRowWaves >> ks_shift) / 2) {
-      const int go = blockIdx.x * ((kRowWaves >> ks_shift) / 2) + gi;
+    if (gi < (kRowWaves >> ks_shift)) {
+      const int go = blockIdx.x * (kRowWaves >> ks_shift) + gi;
       float vg = 0.f, vu = 0.f;
       for (int s = 0; s < (1 << ks_shift); ++s) {
-        vg += part[((2 * gi) << ks_shift) + s][tid & 15];
-        vu += part[((2 * gi + 1) << ks_shift) + s][tid & 15];
+        vg += part[0][(gi << ks_shift) + s][tid & 15];
+        vu += part[kMats - 1][(gi << ks_shift) + s][tid & 15];
       }
-      if (go < groups / 2)
+      if (go < groups)
         a.out[go * 16 + (tid & 15)] = gated_act(a.act, vg, vu, 0.f);
     }
     return;
@@ -405,7 +476,7 @@ row_gemv_kernel(const uint4 *__restrict__ W, const float *__restrict__ src,
     const int go = blockIdx.x * (kRowWaves >> ks_shift) + gi;
     float v = 0.f;
     for (int s = 0; s < (1 << ks_shift); ++s)
-      v += part[(gi << ks_shift) + s][tid & 15];
+      v += part[0][(gi << ks_shift) + s][tid & 15];
     const int n = go * 16 + (tid & 15);
     if (n < a.silu_channels)
       v = silu_f(v);
@@ -479,25 +550,33 @@ struct MoeGateUp {
   float *chosen_logit;
 };
 
-// Grid (channel groups, top + shared): 8 wavefronts = gate and up of
-// (4 >> ks_shift) channel groups x (1 << ks_shift) slices of k.
-template <int R>
+// Grid (channel groups, top + shared): 8 wavefronts = (8 >> ks_shift) channel groups,
+// gate and up in one wavefront, x (1 << ks_shift) slices of k.  H4: the row's values go
+// in fours, at most one per thread, asked for together with the router's logits, so that
+// the weights' addresses wait for one trip to memory.
+template <int R, bool H4>
 __global__ void __launch_bounds__(kRowThreads)
 moe_gate_up_kernel(const float *__restrict__ h, const float *__restrict__ logits, int ks_shift,
                    int slice_tiles, MoeGateUp a) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
-  __shared__ float part[kRowWaves][16];
+  __shared__ float part[2][kRowWaves][16];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int per = (kRowWaves / 2) >> ks_shift;
+  const int per = kRowWaves >> ks_shift;
   const int slot = blockIdx.y;
   const bool is_shared = slot >= a.top;
   const int groups = is_shared ? a.shared_groups : a.groups;
   if ((int)blockIdx.x * per >= groups)
     return;
   const int Kp = a.ktiles * kBfTileK;
-  for (int i = tid; i < Kp; i += kRowThreads)
-    lds[i] = i < a.width ? h[i] : 0.f;
+  f32x4 h4{0.f, 0.f, 0.f, 0.f};
+  if constexpr (H4) {
+    if (4 * tid < a.width)
+      h4 = load4(h + 4 * tid);
+  } else {
+    for (int i = tid; i < Kp; i += kRowThreads)
+      lds[i] = i < a.width ? h[i] : 0.f;
+  }
   const uint4 *W = a.shared_gate_up;
   if (!is_shared) {
     float z = 0.f;
@@ -508,47 +587,34 @@ moe_gate_up_kernel(const float *__restrict__ h, const float *__restrict__ logits
       a.chosen_logit[slot] = z;
     }
   }
-  const int mat = wave & 1, slice = (wave >> 1) & ((1 << ks_shift) - 1);
-  const int g = blockIdx.x * per + (wave >> (1 + ks_shift)), gl = min(g, groups - 1);
+  const int slice = wave & ((1 << ks_shift) - 1);
+  const int g = blockIdx.x * per + (wave >> ks_shift), gl = min(g, groups - 1);
   const int t0 = slice * slice_tiles, t1 = min(t0 + slice_tiles, a.ktiles);
-  const uint4 *wp = W + (int64_t)(mat * groups + gl) * a.ktiles * 64 + lane;
-  uint4 w[kAhead];
+  TileRun<2, kAhead> tiles;
 #pragma unroll
-  for (int u = 0; u < kAhead; ++u)
-    w[u] = wp[(int64_t)min(t0 + u, a.ktiles - 1) * 64];
+  for (int m = 0; m < 2; ++m)
+    tiles.wp[m] = W + (int64_t)(m * groups + gl) * a.ktiles * 64 + lane;
+  tiles.request(t0, t1);
+  if constexpr (H4)
+    if (4 * tid < Kp)
+      save4(lds + 4 * tid, h4);
   __syncthreads();
-  const float *ap = lds + (lane >> 4) * 8;
-  float acc = 0.f;
-  for (int t = t0; t < t1; t += kAhead) {
-    uint4 n[kAhead];
-    const bool more = t + kAhead < t1;
-    if (more) {
+  float acc[2] = {};
+  tiles.run(lds + (lane >> 4) * 8, t0, t1, acc);
 #pragma unroll
-      for (int u = 0; u < kAhead; ++u)
-        n[u] = wp[(int64_t)min(t + kAhead + u, a.ktiles - 1) * 64];
-    }
-#pragma unroll
-    for (int u = 0; u < kAhead; ++u)
-      if (t + u < t1)
-        acc = dot_tile(w[u], ap + (t + u) * kBfTileK, acc);
-    if (more) {
-#pragma unroll
-      for (int u = 0; u < kAhead; ++u)
-        w[u] = n[u];
-    }
+  for (int m = 0; m < 2; ++m) {
+    acc[m] = sum_rows(acc[m]);
+    if (lane < 16)
+      part[m][wave][lane] = acc[m];
   }
-  acc = sum_rows(acc);
-  if (lane < 16)
-    part[wave][lane] = acc;
   __syncthreads();
   const int gi = tid >> 4;
   if (gi < per) {
     const int go = blockIdx.x * per + gi;
     float vg = 0.f, vu = 0.f;
     for (int s = 0; s < (1 << ks_shift); ++s) {
-      const int wv = (gi << (1 + ks_shift)) + 2 * s;
-      vg += part[wv][tid & 15];
-      vu += part[wv + 1][tid & 15];
+      vg += part[0][(gi << ks_shift) + s][tid & 15];
+      vu += part[1][(gi << ks_shift) + s][tid & 15];
     }
     if (go < groups)
       a.act[(int64_t)slot * a.act_stride + go * 16 + (tid & 15)] =
@@ -569,56 +635,98 @@ struct MoeDown {
 // cut the concatenation of the chosen experts' k (and the shared expert's) into
 // slices.  With HALF a load covers the 8 channels of two consecutive tiles, so it
 // still moves whole 128-byte lines; every expert has an even number of tiles.
-template <int WAVES, bool HALF>
+// A wavefront asks for U loads of its run at once and for their activations ahead of
+// them, each value once, and hands those round through an LDS range of its own: fetched
+// by every lane for itself they are twice the bytes of the weights on the way from the L2
+// to the compute unit (8960 -> 1536, 27.5 MB: 10.3 us with that and two trips to memory for
+// the weights, 7.2 us now; four experts of 1792 and the shared one, whose weights wait for
+// the choice: 10.5 and 7.6).
+template <int WAVES, bool HALF, int U>
 __global__ void __launch_bounds__(WAVES * 64)
 moe_down_kernel(const uint4 *__restrict__ down, const float *__restrict__ act,
                 const int *__restrict__ chosen, int slice_tiles, MoeDown a) {
+  constexpr int kStep = HALF ? 2 : 1;                 // tiles per load
+  constexpr int kQuads = U * kStep * kBfTileK / 4;    // activations of U loads, in fours
+  constexpr int kReq = (kQuads + 63) / 64;
   __shared__ float part[WAVES][16];
-  constexpr int kStep = HALF ? 2 : 1; // tiles per load
+  __shared__ __attribute__((aligned(16))) float staged[WAVES][kReq * 256];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = HALF ? blockIdx.x >> 1 : blockIdx.x, half = HALF ? blockIdx.x & 1 : 0;
   // this lane's 16 bytes of a load and the k they hold
   const int run = HALF ? (lane >> 5) * 64 + ((lane >> 3) & 3) * 16 + half * 8 + (lane & 7) : lane;
   const int k_at = HALF ? (lane >> 5) * kBfTileK + ((lane >> 3) & 3) * 8 : (lane >> 4) * 8;
-  // lane j: the j-th chosen expert and its softmax weight
+  // lane j: the j-th chosen expert and its logit
   const int cj = a.top > 0 ? chosen[min(lane, a.top - 1)] : 0;
   const float zj = lane < a.top ? a.chosen_logit[lane] : -INFINITY;
-  const float most = wave_max(zj); // with all lanes, not under the condition below
-  const float ej = lane < a.top ? expf(zj - most) : 0.f;
-  const float wj = ej / wave_sum(ej);
 
   const int routed = a.top * a.ktiles, total = routed + a.shared_ktiles;
   const int t0 = min(wave * slice_tiles, total), t1 = min(t0 + slice_tiles, total);
   // walks the tiles of the concatenation: segment, tile inside it
   int seg = t0 < routed ? t0 / a.ktiles : a.top;
   int off = t0 < routed ? t0 - seg * a.ktiles : t0 - routed;
-  int left = t1 - t0;
-  float acc = 0.f;
-  while (left > 0) {
-    const bool sh = seg >= a.top;
-    const int kt = sh ? a.shared_ktiles : a.ktiles;
-    const int n = min(left, kt - off);
-    const int e = sh ? 0 : __builtin_amdgcn_readlane(cj, min(seg, 63));
-    const float wt = sh ? 1.0f : lane_f(wj, min(seg, 63));
-    const uint4 *wp = (sh ? a.shared_down : down + (int64_t)e * a.groups * kt * 64) +
-                      ((int64_t)g * kt + off) * 64 + run;
-    const float *ap = act + (int64_t)seg * a.act_stride + off * kBfTileK + k_at;
-    float s = 0.f;
-    for (int t = 0; t < n; t += kAhead * kStep) {
-      uint4 w[kAhead];
+  uint4 w[U];
+  f32x4 av[kReq];
+  int segs[U];
+  auto request = [&](int t) {
 #pragma unroll
-      for (int u = 0; u < kAhead; ++u)
-        w[u] = wp[(int64_t)min(t + u * kStep, n - kStep) * 64];
-#pragma unroll
-      for (int u = 0; u < kAhead; ++u)
-        if (t + u * kStep < n)
-          s = dot_tile(w[u], ap + (t + u * kStep) * kBfTileK, s);
+    for (int r = 0; r < kReq; ++r) {
+      const int i = r * 64 + lane, tile = min(t + (i >> 3), t1 - 1);
+      const int sg = tile < routed ? tile / a.ktiles : a.top;
+      const int in = tile < routed ? tile - sg * a.ktiles : tile - routed;
+      av[r] = load4(act + (int64_t)sg * a.act_stride + in * kBfTileK + (i & 7) * 4);
     }
-    acc = fmaf(wt, s, acc);
-    left -= n;
-    off = 0;
-    ++seg;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool sh = seg >= a.top;
+      const int kt = sh ? a.shared_ktiles : a.ktiles;
+      const int e = __builtin_amdgcn_readlane(cj, min(seg, 63));
+      segs[u] = seg;
+      w[u] = ((sh ? a.shared_down : down + (int64_t)e * a.groups * kt * 64) +
+              ((int64_t)g * kt + off) * 64)[run];
+      if (t + (u + 1) * kStep < t1) { // loads past the run's end repeat its last one
+        off += kStep;
+        if (off >= kt) {
+          off = 0;
+          ++seg;
+        }
+      }
+    }
+  };
+  float acc = 0.f;
+  if (t0 < t1) {
+    request(t0);
+    const float most = wave_max(zj); // with all lanes, not under the condition below
+    const float ej = lane < a.top ? expf(zj - most) : 0.f;
+    const float wj = ej / wave_sum(ej);
+    auto weight = [&](int sg) { return sg >= a.top ? 1.0f : lane_f(wj, min(sg, 63)); };
+    float *mine = staged[wave];
+    float s = 0.f;
+    int cur = segs[0];
+    for (int t = t0;;) {
+#pragma unroll
+      for (int r = 0; r < kReq; ++r)
+        save4(mine + (r * 64 + lane) * 4, av[r]);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (t + u * kStep < t1) {
+          if (segs[u] != cur) {
+            acc = fmaf(weight(cur), s, acc);
+            s = 0.f;
+            cur = segs[u];
+          }
+          s = dot_tile(w[u], mine + u * kStep * kBfTileK + k_at, s);
+        }
+      t += U * kStep;
+      if (t >= t1)
+        break;
+      request(t);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+    acc = fmaf(weight(cur), s, acc);
   }
   acc = sum_rows(acc);
   if constexpr (HALF)
@@ -637,6 +745,30 @@ moe_down_kernel(const uint4 *__restrict__ down, const float *__restrict__ act,
 
 // slices start at even tiles
 int down_slice(int total, int waves) { return (int)round_up(ceil_div(total, waves), 2); }
+
+template <int WAVES, bool HALF>
+void launch_down_slices(const uint4 *down, const float *act, const int *chosen, int total, const MoeDown &d,
+                        hipStream_t stream) {
+  const int slice = down_slice(total, WAVES), loads = slice / (HALF ? 2 : 1);
+  const dim3 grid((HALF ? 2 : 1) * d.groups), block(WAVES * 64);
+  // nine loads hold a slice of 8960 inputs and halves (8960 -> 1536: 10.3 us with eight, 7.2 with
+  // nine); fourteen where they save a trip to memory
+  if (ceil_div(loads, 14) < ceil_div(loads, 9))
+    hipLaunchKernelGGL((moe_down_kernel<WAVES, HALF, 14>), grid, block, 0, stream, down, act, chosen, slice, d);
+  else
+    hipLaunchKernelGGL((moe_down_kernel<WAVES, HALF, 9>), grid, block, 0, stream, down, act, chosen, slice, d);
+}
+int launch_down(const uint4 *down, const float *act, const int *chosen, int total, const MoeDown &d,
+                hipStream_t stream) {
+  if (total >= 64 && d.groups < 192) // fewer workgroups than compute units: halves
+    launch_down_slices<16, true>(down, act, chosen, total, d, stream);
+  else if (total >= 64)
+    launch_down_slices<16, false>(down, act, chosen, total, d, stream);
+  else
+    launch_down_slices<4, false>(down, act, chosen, total, d, stream);
+  BH_CHECK_HIP(hipGetLastError());
+  return BUDDY_HIP_OK;
+}
 
 int shift_for(int v) {
   int s = 0;
@@ -677,20 +809,14 @@ int launch_row_gemv(const RowGemv &a, hipStream_t stream) {
       W.ktiles >= 64 && (W.groups() < 192 || W.ktiles > 256)) {
     // a long row and few channels: as many slices of k as the experts' down product takes
     MoeDown d{W.tiles, W.groups(), 0, 1, W.ktiles, 0, nullptr, a.out};
-    if (W.groups() < 192)
-      hipLaunchKernelGGL((moe_down_kernel<16, true>), dim3(2 * W.groups()), dim3(1024), 0, stream,
-                         (const uint4 *)nullptr, a.src, (const int *)nullptr, down_slice(W.ktiles, 16), d);
-    else
-      hipLaunchKernelGGL((moe_down_kernel<16, false>), dim3(W.groups()), dim3(1024), 0, stream,
-                         (const uint4 *)nullptr, a.src, (const int *)nullptr, down_slice(W.ktiles, 16), d);
-    BH_CHECK_HIP(hipGetLastError());
-    return BUDDY_HIP_OK;
+    return launch_down(nullptr, a.src, nullptr, W.ktiles, d, stream);
   }
-  // slices of k: doubled while the launch has fewer than 2048 wavefronts and each
-  // keeps four tiles
-  const int groups = W.groups();
+  // slices of k: doubled while the launch has fewer than 4096 wavefronts and each
+  // keeps four tiles (2048: 13.8 us against 12.5 for gate | up of 1536 -> 2 x 8960, 19.7
+  // against 18.7 for a head of 1536 -> 32768)
+  const int groups = a.gated ? W.groups() / 2 : W.groups();
   int ks = 1;
-  while (ks < (a.gated ? kRowWaves / 2 : kRowWaves) && (int64_t)groups * ks < 2048 && W.ktiles / (2 * ks) >= 4)
+  while (ks < kRowWaves && (int64_t)groups * ks < 4096 && W.ktiles / (2 * ks) >= 4)
     ks *= 2;
   const int shift = shift_for(ks), per = kRowWaves >> shift;
   const int slice_tiles = (int)ceil_div(W.ktiles, ks);
@@ -773,25 +899,29 @@ int launch_row_moe(const RowMoe &a, hipStream_t stream) {
   BH_REQUIRE(a.act_stride >= 64 * ceil_div(std::max(a.experts.ff, shared ? a.shared.ff : 0), 64),
              "row_moe: activation rows too short");
   int ks = 1;
-  while (ks < kRowWaves / 2 && u.ktiles / (2 * ks) >= 4)
+  while (ks < kRowWaves && u.ktiles / (2 * ks) >= 4)
     ks *= 2;
-  const int shift = shift_for(ks), per = (kRowWaves / 2) >> shift;
+  const int shift = shift_for(ks), per = kRowWaves >> shift;
   const size_t lds = sizeof(float) * (size_t)u.ktiles * kBfTileK;
   BH_REQUIRE(lds <= 150 * 1024, "row_moe: a row of %d values does not fit LDS", a.width);
   const dim3 grid((unsigned)ceil_div(std::max(u.groups, u.shared_groups), per),
                   (unsigned)(a.top + (shared ? 1 : 0)));
   const int slice_tiles = (int)ceil_div(u.ktiles, ks);
-#define BH_GU(R)                                                                                \
+#define BH_GU(R, H4)                                                                            \
   do {                                                                                          \
     static DynLdsOnce once;                                                                     \
-    BH_CHECK_HIP(ensure_dyn_lds(once, (const void *)moe_gate_up_kernel<R>, 150 * 1024));        \
-    hipLaunchKernelGGL(moe_gate_up_kernel<R>, grid, dim3(kRowThreads), lds, stream, a.h,        \
+    BH_CHECK_HIP(ensure_dyn_lds(once, (const void *)moe_gate_up_kernel<R, H4>, 150 * 1024));    \
+    hipLaunchKernelGGL((moe_gate_up_kernel<R, H4>), grid, dim3(kRowThreads), lds, stream, a.h,  \
                        a.logits, shift, slice_tiles, u);                                        \
   } while (0)
-  if (a.experts.count <= 64)
-    BH_GU(1);
+  const bool quads = a.width % 4 == 0 && ((uintptr_t)a.h & 15) == 0 &&
+                     u.ktiles * kBfTileK <= 4 * kRowThreads;
+  if (a.experts.count <= 64 && quads)
+    BH_GU(1, true);
+  else if (a.experts.count <= 64)
+    BH_GU(1, false);
   else
-    BH_GU(kMaxExperts / 64);
+    BH_GU(kMaxExperts / 64, false);
 #undef BH_GU
   BH_CHECK_HIP(hipGetLastError());
   MoeDown d{};
@@ -803,19 +933,7 @@ int launch_row_moe(const RowMoe &a, hipStream_t stream) {
   d.act_stride = a.act_stride;
   d.chosen_logit = a.weights;
   d.out = a.out;
-  const int total = a.top * d.ktiles + d.shared_ktiles;
-  auto slice = [&](int waves) { return down_slice(total, waves); };
-  if (total >= 64 && d.groups < 192) // fewer workgroups than compute units: halves
-    hipLaunchKernelGGL((moe_down_kernel<16, true>), dim3(2 * d.groups), dim3(1024), 0, stream,
-                       a.experts.down, a.act, a.chosen, slice(16), d);
-  else if (total >= 64)
-    hipLaunchKernelGGL((moe_down_kernel<16, false>), dim3(d.groups), dim3(1024), 0, stream,
-                       a.experts.down, a.act, a.chosen, slice(16), d);
-  else
-    hipLaunchKernelGGL((moe_down_kernel<4, false>), dim3(d.groups), dim3(256), 0, stream,
-                       a.experts.down, a.act, a.chosen, slice(4), d);
-  BH_CHECK_HIP(hipGetLastError());
-  return BUDDY_HIP_OK;
+  return launch_down(a.experts.down, a.act, a.chosen, a.top * d.ktiles + d.shared_ktiles, d, stream);
 }
 
 } // namespace bh

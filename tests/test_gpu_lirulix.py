@@ -104,6 +104,18 @@ def test_mechanism_alone(tmp_path, what, dtype):
     check(feed(s, tokens, [3] + [1] * 67), want, dtype, "decoding")
 
 
+# a decode step's gate | up (runs of tiles on both sides of what a wavefront has in flight) and its
+# down product: halves and whole channel groups, one trip to memory and several
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width,ff", [(72, 2100), (72, 8960), (72, 13000), (72, 20000), (3100, 9000), (1536, 33)])
+def test_one_row_through_the_feed_forward(tmp_path, width, ff, dtype):
+    cfg = M.config([M.full(heads=1, ff=ff)], width=width, vocab=64)
+    folder, t = M.build(tmp_path, cfg, ff)
+    tokens = tokens_for(cfg, 5)
+    s = FolderSession(folder, dtype, max_len=16)
+    check(feed(s, tokens, [1] * 5), L.forward(cfg, t, tokens), dtype)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("block", [0, 16, 80])
 def test_portions_do_not_matter(tmp_path, dtype, block):

@@ -109,6 +109,23 @@ def test_mechanism_alone(tmp_path, what, dtype):
     check(feed(s, tokens, [3] + [1] * 67), want, dtype, "decoding")
 
 
+# moe_down_kernel: a wavefront's slice of the experts' k on both sides of its 9 and 14 loads, in
+# one trip and in several, with many experts in one trip, halves of a channel group (fewer than
+# 192 of them) and whole ones; moe_gate_up_kernel: runs of fewer tiles than in flight and of more
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width,ff,experts,top,shared", [
+    (72, 64, 36, 36, 200), (72, 130, 3, 3, 0), (72, 1792, 4, 4, 1792), (72, 2100, 5, 5, 2000),
+    (70, 3200, 4, 4, 3500), (72, 4100, 4, 4, 4100), (3100, 700, 3, 2, 900), (3076, 2100, 3, 3, 2100),
+    (1536, 40, 3, 2, 72), (1602, 72, 3, 2, 40)])
+def test_one_row_through_the_experts(tmp_path, width, ff, experts, top, shared, dtype):
+    cfg = M.config([M.latent(window=3, mlp=M.moe(experts=experts, top=top, ff=ff, shared_ff=shared))],
+                   width=width, vocab=64, taps=4)
+    folder, t = M.build(tmp_path, cfg, ff)
+    tokens = tokens_for(cfg, 7)
+    s = FolderSession(folder, dtype, max_len=16)
+    check(feed(s, tokens, [1] * 7), N.forward(cfg, t, tokens), dtype)
+
+
 # rows_gemm_wide_kernel<f32, RT, GT, 3, experts>: gate and up on tiles of 32 RT rows x 64 GT
 # channels of each, of experts (whose counts are uneven) and of the shared one, whose widths
 # end inside a tile; and <f32, RT, GT, 0, 1>, the experts' way back
