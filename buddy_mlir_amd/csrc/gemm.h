@@ -46,13 +46,20 @@ struct GemmStagingLayout {
   size_t bytes(int terms) const {
     return sizeof(unsigned short) * (size_t)terms * rows_padded * cols_padded;
   }
-  // digit planes: [digits][rows_padded][cols_padded] int8, then the row steps
-  // (f32 [rows_padded])
+  // digit planes: rows_padded x cols_padded int8 in each, as plane_at places them, then the
+  // row steps (f32 [rows_padded])
   size_t bytes_digits(int digits) const {
     return (size_t)digits * rows_padded * cols_padded + sizeof(float) * (size_t)rows_padded;
   }
 };
 GemmStagingLayout gemm_staging_layout(int64_t M, int64_t K);
+// Where a digit plane's value lies: blocks of 32 rows x 64 k, 2 KiB each, all planes of a
+// block one behind the other, then the next 64 k, then the next 32 rows.  Kp: cols_padded.
+constexpr int kPlaneBlock = 32 * kTileK;
+__host__ __device__ inline size_t plane_at(int row, int k, int plane, int planes, int Kp) {
+  return (((size_t)(row / 32) * (Kp / kTileK) + k / kTileK) * planes + plane) * kPlaneBlock +
+         row % 32 * kTileK + k % kTileK;
+}
 // Producers that write their result straight into a staging buffer:
 //   RMSNorm rows: y = w * (x * rsqrt(mean(x^2) + eps))
 //   SiLU(g) * u   (g and u rows `ld` floats apart)

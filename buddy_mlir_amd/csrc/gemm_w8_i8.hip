@@ -23,9 +23,10 @@
 // row (an infinity gives the reference +-inf or NaN per column; here NaN).
 // |d q| <= 2^14, so K may not exceed 2^17.
 //
-// Digit planes lie like the bf16 terms do: [digit][row][k] int8, rows and k zero
-// padded, followed by the row steps (f32 [rows_padded]).  A lane's operand is 16
-// contiguous bytes of a plane row.
+// Digit planes lie in blocks of 32 rows x 64 k (plane_at), rows and k zero padded, followed
+// by the row steps (f32 [rows_padded]): what a workgroup fetches at once is one run of
+// memory.  (Rows of K bytes: a load instruction asks for half a cache line of each of 16
+// rows.)  A lane's operand is 16 contiguous bytes of a row of a block.
 //
 // Workgroups take 32 rows x 128 or 256 channels, or one of the other tiles of kTiles1 to
 // kTiles3, with the activation fragments shared through LDS.
@@ -37,6 +38,7 @@
 #include <cstdlib>
 #include <map>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 namespace bh {
@@ -45,6 +47,7 @@ namespace {
 constexpr int kSlices = 4;    // wavefronts per workgroup
 
 typedef int v4i32 __attribute__((ext_vector_type(4)));
+typedef int v2i32 __attribute__((ext_vector_type(2)));
 
 // ---- f32 rows -> digit planes ------------------------------------------------
 
@@ -191,7 +194,6 @@ __device__ __forceinline__ void row_to_digits(const F &f, int n, int row, int D,
   float *steps = reinterpret_cast<float *>(planes + (size_t)D * Mp * Kp);
   if (threadIdx.x == 0)
     steps[row] = step;
-  const size_t plane = (size_t)Mp * Kp;
   for (int k0 = threadIdx.x * 4; k0 < Kp; k0 += kRowThreads * 4) {
     float v[4];
     if (cached) {
@@ -208,7 +210,7 @@ __device__ __forceinline__ void row_to_digits(const F &f, int n, int row, int D,
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       X[e] = finite ? (int)rintf(v[e] * inv) : 0;
-    int8_t *dst = planes + (size_t)row * Kp + k0;
+    int8_t *dst = planes + plane_at(row, k0, 0, D, Kp);
     for (int j = 0; j < D; ++j) {
       unsigned word = 0;
 #pragma unroll
@@ -218,7 +220,7 @@ __device__ __forceinline__ void row_to_digits(const F &f, int n, int row, int D,
         X[e] = (X[e] - d) >> 8; // exact: X - d is a multiple of 256
         word |= (unsigned)(d & 0xff) << (8 * e);
       }
-      *reinterpret_cast<unsigned *>(dst + j * plane) = word;
+      *reinterpret_cast<unsigned *>(dst + j * kPlaneBlock) = word;
     }
   }
 }
@@ -226,7 +228,7 @@ __device__ __forceinline__ void row_to_digits(const F &f, int n, int row, int D,
 __device__ __forceinline__ void padding_to_digits(int row, int D, int Mp, int Kp, int8_t *planes) {
   for (int j = 0; j < D; ++j)
     for (int k0 = threadIdx.x * 4; k0 < Kp; k0 += kRowThreads * 4)
-      *reinterpret_cast<unsigned *>(planes + ((size_t)j * Mp + row) * Kp + k0) = 0u;
+      *reinterpret_cast<unsigned *>(planes + plane_at(row, k0, j, D, Kp)) = 0u;
   if (threadIdx.x == 0)
     reinterpret_cast<float *>(planes + (size_t)D * Mp * Kp)[row] = 1.0f;
 }
@@ -294,7 +296,7 @@ silu_mul_to_digits_kernel(const float *__restrict__ g, const float *__restrict__
 // ---- the matmul ----------------------------------------------------------------
 
 struct GemmI8Args {
-  const int8_t *planes; // [D][Mp][Kp]
+  const int8_t *planes; // blocks of plane_at
   const float *steps;   // [Mp]
   const int4 *W;
   const float *scale;
@@ -325,7 +327,7 @@ template <int D> __device__ __forceinline__ float scaled(float v, float step, fl
 // that has its SIMD to itself issues that instruction at its full rate, the 16 x 16 x 64
 // one at two thirds of it, and it reads half as many operands per product.  Its A operand
 // is 32 channels x 32 k: the lanes take it from the tiles of two channel groups.  What
-// bounds it: 1931 rows of gate | up run at 1.73 P operations/s (16 x 16 x 64: 1.57), half
+// bounds it: 1931 rows of gate | up run at 1.87 P operations/s (16 x 16 x 64: 1.57), half
 // of what the instruction alone reaches; twice the rows per weight give no more (below).
 //
 // The digit planes' rows go through LDS, shared by the wavefronts; weights go from memory
@@ -375,9 +377,9 @@ __device__ __forceinline__ void multiply_tile(const GemmI8Args &a) {
   constexpr int kSpan = kWidth * GP;        // ... and per wavefront
   constexpr int kRows = 32 * RB;            // rows of the tile
   constexpr int L = D * RB;                 // layers of 32 rows: plane l % D of row block l / D
-  constexpr int kRuns = L * 32 * 4;         // 16-byte runs of a chunk's rows
   constexpr int kThreads = kSlices * kWave;
-  constexpr int kLoads = (kRuns + kThreads - 1) / kThreads;
+  // a thread's loads of a chunk's rows: 16 bytes of two layers at a time, 8 of an odd last one
+  constexpr int kQuad = L / 2, kLoads = (L + 1) / 2;
   constexpr int kBuf = L * 32 * kWideRow;
   constexpr int kTurn = kSpan + 4;          // floats of a row of the epilogue's tile
   constexpr int kTurned = kSlices * 32 * kTurn * 4;
@@ -385,6 +387,13 @@ __device__ __forceinline__ void multiply_tile(const GemmI8Args &a) {
   constexpr int kScales = kSlices * 32 * GP;
   // chunks of weights and of rows in registers
   constexpr int kRing = 4;
+  constexpr int kFetches = 2 * GP + kLoads; // loads of a chunk
+  // the first load issued with sub-step u
+  auto first_fetch = [](int u) constexpr {
+    if (D > 1 || L == 1)
+      return u * kFetches / (2 * L);
+    return u == 0 ? 0 : u <= 2 ? 2 * GP : kFetches;
+  };
   __shared__ __attribute__((aligned(16))) unsigned char lds[kLds];
   // the epilogue's operands, asked for as the launch starts: scales (PAIR: of both
   // matrices), bias, row steps
@@ -414,18 +423,20 @@ __device__ __forceinline__ void multiply_tile(const GemmI8Args &a) {
   }
   const int8_t *src[kLoads];
   int lds_at[kLoads];
-  bool mine[kLoads];
 #pragma unroll
   for (int i = 0; i < kLoads; ++i) {
-    const int idx = i * kThreads + tid, l = min(idx / 128, L - 1);
-    const int r = idx / 4 % 32, q = idx & 3;
-    mine[i] = idx < kRuns;
-    src[i] = a.planes +
-             ((size_t)(l % D) * a.Mp + min(m0 + l / D * 32 + r, a.Mp - 1)) * a.Kp +
-             (size_t)cb * kTileK + q * 16;
-    lds_at[i] = (l * 32 + r) * kWideRow + q * 16;
+    const int run = i < kQuad ? 16 : 8, at = tid * run; // of layers 2 i and 2 i + 1
+    const int l = 2 * i + at / kPlaneBlock, r = at % kPlaneBlock / kTileK, k = at % kTileK;
+    const int block = min(m0 / 32 + l / D, a.Mp / 32 - 1);
+    src[i] = a.planes + (((size_t)block * a.chunks + cb) * D + l % D) * kPlaneBlock + r * kTileK + k;
+    lds_at[i] = (l * 32 + r) * kWideRow + k;
   }
-  v4i32 wr[kRing][GP * 2], xr[kRing][kLoads];
+  struct Rows {
+    v4i32 q[kQuad ? kQuad : 1];
+    v2i32 h;
+  };
+  v4i32 wr[kRing][GP * 2];
+  Rows xr[kRing];
   auto fetch_w = [&](int c, v4i32 (&w)[GP * 2]) {
     const size_t cc = (size_t)min(c, nch - 1) * 64;
 #pragma unroll
@@ -434,17 +445,28 @@ __device__ __forceinline__ void multiply_tile(const GemmI8Args &a) {
       for (int g = 0; g < GP; ++g)
         w[g * 2 + h] = wp[g][cc + h * 32];
   };
-  auto fetch_x = [&](int c, v4i32 (&x)[kLoads]) {
-    const size_t cc = (size_t)min(c, nch - 1) * kTileK;
-#pragma unroll
-    for (int i = 0; i < kLoads; ++i)
-      x[i] = *reinterpret_cast<const v4i32 *>(src[i] + cc);
+  auto fetch_run = [&](int i, size_t cc, Rows &x) {
+    if (i < kQuad)
+      x.q[i] = *reinterpret_cast<const v4i32 *>(src[i] + cc);
+    else
+      x.h = *reinterpret_cast<const v2i32 *>(src[i] + cc);
   };
-  auto put_x = [&](const v4i32 (&x)[kLoads], unsigned char *buf) {
+  auto put_run = [&](int i, const Rows &x, unsigned char *buf) {
+    if (i < kQuad)
+      *reinterpret_cast<v4i32 *>(buf + lds_at[i]) = x.q[i];
+    else
+      *reinterpret_cast<v2i32 *>(buf + lds_at[i]) = x.h;
+  };
+  auto fetch_x = [&](int c, Rows &x) {
+    const size_t cc = (size_t)min(c, nch - 1) * (D * kPlaneBlock);
 #pragma unroll
     for (int i = 0; i < kLoads; ++i)
-      if (kRuns % kThreads == 0 || mine[i])
-        *reinterpret_cast<v4i32 *>(buf + lds_at[i]) = x[i];
+      fetch_run(i, cc, x);
+  };
+  auto put_x = [&](const Rows &x, unsigned char *buf) {
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i)
+      put_run(i, x, buf);
   };
   fetch_x(0, xr[0]);
   fetch_x(1, xr[1]);
@@ -487,20 +509,30 @@ __device__ __forceinline__ void multiply_tile(const GemmI8Args &a) {
   load_frag(cur, 0, frag[0]);
   load_frag(cur, 1, frag[1]);
   // f: the slot of sub-step 0's fragments
-  auto step = [&](int c, int f, v4i32 (&w)[GP * 2], v4i32 (&w_new)[GP * 2], v4i32 (&x)[kLoads],
-                  v4i32 (&x_new)[kLoads]) {
+  auto step = [&](int c, int f, v4i32 (&w)[GP * 2], v4i32 (&w_new)[GP * 2], const Rows &x,
+                  Rows &x_new) {
+    const size_t wc = (size_t)min(c + kRing - 1, nch - 1) * 64;
+    const size_t xc = (size_t)min(c + kRing + 1, nch - 1) * (D * kPlaneBlock);
 #pragma unroll
     for (int u = 0; u < 2 * L; ++u) {
       // fragments are asked for two sub-steps ahead of their products (one takes less than
       // the way through LDS), and stay there: left to itself the scheduler moves them to
       // their use
       load_frag(u + 2 < 2 * L ? cur : next, (u + 2) % (2 * L), frag[(f + u + 2) & 3]);
-      if (u == 0)
-        fetch_w(c + kRing - 1, w_new);
-      if (u == 1)
-        put_x(x, fill);
-      if (u == (L > 1 ? 2 : 1))
-        fetch_x(c + kRing + 1, x_new);
+      // a chunk's loads, weights first: evenly between its products (all at its start: 171
+      // against 167 us for gate | up of 1931 rows, 193 against 180 on 64 x 256 tiles), for one
+      // plane, which has a third of the products, at the start (19.2 against 21)
+#pragma unroll
+      for (int i = first_fetch(u); i < first_fetch(u + 1); ++i) {
+        if (i < 2 * GP)
+          w_new[i % GP * 2 + i / GP] = wp[i % GP][wc + i / GP * 32];
+        else
+          fetch_run(i - 2 * GP, xc, x_new);
+      }
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i)
+        if (u == (i + 1 < 2 * L - 2 ? i + 1 : 1))
+          put_run(i, x, fill);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int g = 0; g < GP; ++g)
@@ -516,12 +548,29 @@ __device__ __forceinline__ void multiply_tile(const GemmI8Args &a) {
   };
   // step c: weights from slot c, new ones into slot c - 1; rows c + 2 go to LDS, new ones
   // into slot c + 1 (all modulo kRing)
-  for (int c0 = 0; c0 < nch; c0 += kRing) {
-#pragma unroll
-    for (int u = 0; u < kRing; ++u)
-      if (c0 + u < nch)
-        step(c0 + u, (u * 2 * L) & 3, wr[u], wr[(u + kRing - 1) % kRing], xr[(u + 2) % kRing],
-             xr[(u + 1) % kRing]);
+  auto turn = [&](int c0, auto slot) {
+    constexpr int u = slot;
+    step(c0 + u, (u * 2 * L) & 3, wr[u], wr[(u + kRing - 1) % kRing], xr[(u + 2) % kRing],
+         xr[(u + 1) % kRing]);
+  };
+  // No branch within a round of the ring: where paths of fewer steps join, the compiler waits
+  // for all loads but those of the shortest path ahead of any register it uses again.
+  using std::integral_constant;
+  int c0 = 0;
+  for (; c0 + kRing <= nch; c0 += kRing) {
+    turn(c0, integral_constant<int, 0>{});
+    turn(c0, integral_constant<int, 1>{});
+    turn(c0, integral_constant<int, 2>{});
+    turn(c0, integral_constant<int, 3>{});
+  }
+  static_assert(kRing == 4, "a round is written out");
+  if (c0 < nch) {
+    turn(c0, integral_constant<int, 0>{});
+    if (c0 + 1 < nch) {
+      turn(c0, integral_constant<int, 1>{});
+      if (c0 + 2 < nch)
+        turn(c0, integral_constant<int, 2>{});
+    }
   }
 
   // ---- epilogue ---------------------------------------------------------
@@ -1006,20 +1055,18 @@ namespace {
 // compute units) works on 64 workgroups at a time, two to a compute unit, or on 32 where a
 // tile's registers leave room for one.  A chunk of 64 k takes a workgroup that has its
 // compute unit to itself `alone`, two that share one `both`, each beside a fixed part; a last
-// round that fills less than half runs at the former.  Fitted to launches of 32 to 4096 rows
-// of 1536, 4096, 8960 and 14336 k.  Microseconds, with the tiles of 256 channels beside them
-// (in brackets 16 x 16 x 64 instructions on tiles of 48 or 64 rows x 256 or 320 channels):
-//   gate | up, 1536 -> 2 x 8960, three planes; two: 27 rows 11.2 [18.4]; 10.0 [15.0], 256:
-//     28 (32.6) [30.6]; 22 (27.3) [23.3], 512: 52 [58.8]; 38 (42.7) [44.3], 1931: 173 [201]; 130
-//     (136) [150]
-//   down, 8960 -> 1536, with the adding of its slices: 27 rows 12.7 [16.9]; 11.1 [15.1],
-//     512: 34 [36]; 28 [28], 1931: 90 (96) [112]; 72 (77) [95]
-//   q|k|v, 1536 -> 2048: 100 rows 10.0 [13.3]; 8.2 [12.6], 512: 12.5 [15.8]; 9.9 [11.8],
-//     1024: 17.2 [30.4]; 14.4 [22.7]
-//   4096 -> 2 x 14336 with the conversion: 1024 rows 361 (359) [343]; 252 (288) [265],
-//     4096: 1320 (1391) [1372]; 980 (1075) [1042]
-//   14336 -> 4096 with both: 33 rows 34.3 [32.6]; 26.7 [29.6], 768: 156 [148]; 108 [143]
-//   one plane: 1536 -> 8960: 256 rows 14 (18) [18], 512: 18.6 [21.2], 2048: 52 [69]
+// round that fills less than half runs at the former.  Fitted to
+// launches of 20 to 1931 rows of 1536, 4096, 8960 and 14336 k, every tile with every K split: what
+// it picks is 1.0 (three planes) and 1.4 % (two) off the best on average, 9 and 15 at most.
+// Microseconds of a product with three planes in a prompt (in brackets with rows of K bytes per
+// plane, a branch at every chunk and its loads all at the chunk's start):
+//   gate | up, 1536 -> 2 x 8960: 27 rows 12.4 [14.4], 512: 54 [59], 1931: 171.5 [182]
+//   down, 8960 -> 1536: 27 rows 5.7 [6.5], 512: 25 [30], 1931: 81.5 [89]
+//   q|k|v, 1536 -> 2048: 512 rows 11.6 [14.5]
+//   one plane, 1536 -> 8960: 512 rows 19.1 [20.3]
+// The card holds its clock at 1.9 GHz under the large ones, whose matrix pipes are half busy:
+// without any loads in the loop gate | up of 1931 rows takes 119 us, with loads that all hit the
+// L1 157.
 // (gate | up at 27 rows with two channel tiles: 13.7, and 18.7 in a prompt, whose weights come
 // from memory, against 14.9 with one: twice the compute units ask for them.)
 // Tiles that fill a compute unit alone have coarser rounds and use an operand more often
@@ -1034,15 +1081,15 @@ struct TileShape {
 constexpr TileShape kTiles1[] = {{1, 1, true, 0.21, 4.5, 0.285, 4.5},
                                  {wide_blocks(1), 2, true, 0.33, 5.0, 0.54, 4.0},
                                  {3, 2, true, 0.39, 5.0, 0.66, 4.0}};
-constexpr TileShape kTiles2[] = {{1, 1, true, 0.232, 4.6, 0.33, 3.8},
-                                 {wide_blocks(2), 2, true, 0.34, 5.2, 0.50, 6.1},
-                                 {2, 2, false, 0.446, 6.8, 0, 0},
-                                 {1, 3, true, 0.428, 6.0, 0.71, 8.3},
-                                 {3, 2, false, 0.606, 8.1, 0, 0}};
-constexpr TileShape kTiles3[] = {{1, 1, true, 0.27, 4.5, 0.455, 4.5},
-                                 {wide_blocks(3), 2, true, 0.35, 4.7, 0.66, 4.0},
-                                 {2, 2, false, 0.60, 5.8, 0, 0},
-                                 {1, 5, false, 0.88, 7.0, 0, 0}};
+constexpr TileShape kTiles2[] = {{1, 1, true, 0.194, 4.15, 0.379, 3.85},
+                                 {wide_blocks(2), 2, true, 0.303, 5.0, 0.51, 6.05},
+                                 {2, 2, false, 0.446, 7.1, 0, 0},
+                                 {1, 3, true, 0.428, 6.0, 0.913, 10.0},
+                                 {3, 2, false, 0.621, 9.9, 0, 0}};
+constexpr TileShape kTiles3[] = {{1, 1, true, 0.216, 3.2, 0.455, 4.5},
+                                 {wide_blocks(3), 2, true, 0.35, 4.7, 0.676, 4.0},
+                                 {2, 2, false, 0.591, 6.3, 0, 0},
+                                 {1, 5, false, 0.855, 7.0, 0, 0}};
 
 struct TilePlan {
   int rb = 0, gp = 0, slices = 1;

@@ -92,7 +92,7 @@ w8a8_absmax_parts_kernel(const float *__restrict__ x, int64_t n, float *__restri
     part[blockIdx.x] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
 }
 
-// stage 2: workgroup `row` writes row `row` of the plane ([Mp][Kp], zeros past M
+// stage 2: workgroup `row` writes row `row` of the plane (zeros past M
 // and K) and its step, the activation scale (1 for padding rows)
 __global__ void __launch_bounds__(256)
 w8a8_rows_to_plane_kernel(const float *__restrict__ x, int M, int K, int Kp,
@@ -131,7 +131,7 @@ w8a8_rows_to_plane_kernel(const float *__restrict__ x, int M, int K, int Kp,
         word |= ((unsigned)(int)r & 0xffu) << (8 * e);
       }
     }
-    *reinterpret_cast<unsigned *>(plane + (size_t)row * Kp + k0) = word;
+    *reinterpret_cast<unsigned *>(plane + plane_at(row, k0, 0, 1, Kp)) = word;
   }
 }
 
