@@ -16,6 +16,7 @@ namespace bh {
 namespace {
 
 constexpr int kGemmThreads = 256;
+constexpr int kWideK = 64; // k per step of the tiles of 32 rows and more
 constexpr int kStages = 4;
 constexpr int kRowBytes = 128;           // of one row per step
 constexpr int kLdsRow = kRowBytes + 16;  // padded: rows start 4 banks apart
@@ -32,6 +33,8 @@ struct GemmDev {
   const int *counts, *lists;
   int experts, list_cap, list_div;
   int64_t expert_tiles;
+  int slice_steps;      // kOutF32, not grouped: steps of a slice of k
+  int64_t slice_stride; // ... and from one slice's sums to the next in C
 };
 
 template <typename T> struct ActTraits;
@@ -147,6 +150,14 @@ rows_gemm_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int columns
     W += (int64_t)e * a.expert_tiles * 64;
   }
 
+  // this workgroup's slice of k
+  int K = a.K, first = 0;
+  if constexpr (OUT == kOutF32 && !GROUPED) {
+    first = blockIdx.z * a.slice_steps;
+    steps = min(a.slice_steps, steps - first);
+    K -= first * Tr::kElems;
+  }
+
   // the runs this thread moves: fixed rows, k advancing by the step
   const T *src[kLoads];
   int run_k[kLoads];
@@ -164,7 +175,7 @@ rows_gemm_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int columns
       pr = list[lr] / a.list_div;
     else
       pr = (a.ring_base + lr) & a.ring_mask;
-    src[i] = static_cast<const T *>(a.A) + (int64_t)pr * a.lda;
+    src[i] = static_cast<const T *>(a.A) + (int64_t)pr * a.lda + first * Tr::kElems;
   }
 
   const int ch0 = (bx * 4 + wave) * kGroups; // first channel group of this wavefront
@@ -172,13 +183,13 @@ rows_gemm_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int columns
 #pragma unroll
   for (int g = 0; g < GT; ++g) {
     const int mat = kPair ? g / kGroups : 0, gg = min(ch0 + (kPair ? g % kGroups : g), a.groups - 1);
-    wp[g] = W + ((int64_t)(mat * a.groups + gg) * ktiles) * 64 + lane;
+    wp[g] = W + ((int64_t)(mat * a.groups + gg) * ktiles + first * Tr::kTiles) * 64 + lane;
   }
 
   uint4 wr[kStages][GT * Tr::kTiles], ar[kStages][kLoads];
   constexpr int kRunElems = 16 / (int)sizeof(T);
-  const int last_run = (a.K - 1) / kRunElems * kRunElems;
-  const bool ragged = a.K % Tr::kElems != 0; // the last step reaches past K
+  const int last_run = (K - 1) / kRunElems * kRunElems;
+  const bool ragged = K % Tr::kElems != 0; // the last step reaches past K
   auto fetch = [&](int s, uint4 (&w)[GT * Tr::kTiles], uint4 (&x)[kLoads]) {
     const int t = min(s, steps - 1) * Tr::kTiles;
 #pragma unroll
@@ -205,7 +216,7 @@ rows_gemm_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int columns
     if (ragged && s == steps - 1) {
 #pragma unroll
       for (int i = 0; i < kLoads; ++i)
-        x[i] = keep_run<T>(x[i], a.K - s * Tr::kElems - run_k[i]);
+        x[i] = keep_run<T>(x[i], K - s * Tr::kElems - run_k[i]);
     }
 #pragma unroll
     for (int i = 0; i < kLoads; ++i)
@@ -267,7 +278,7 @@ rows_gemm_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int columns
       for (int j = 0; j < 4; ++j)
         if (ch + j < a.silu_channels)
           v[j] = silu_f(v[j]);
-      store4<float>(static_cast<float *>(a.C) + (int64_t)orow * a.ldc + ch, v);
+      store4<float>(static_cast<float *>(a.C) + blockIdx.z * a.slice_stride + (int64_t)orow * a.ldc + ch, v);
     } else if constexpr (OUT == kOutAct) {
       store4<T>(static_cast<T *>(a.C) + (int64_t)orow * a.ldc + ch, v);
     } else {
@@ -341,8 +352,6 @@ __device__ __forceinline__ f32x16 mfma_bf16_wide(uint4 a, uint4 b, f32x16 c) {
                                                  __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-constexpr int kWideK = 64; // k per step
-
 template <typename T, int RT, int GT, int OUT, bool GROUPED>
 __global__ void __launch_bounds__(kGemmThreads)
 rows_gemm_wide_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int columns, int row_blocks,
@@ -378,6 +387,13 @@ rows_gemm_wide_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int co
     W += (int64_t)e * a.expert_tiles * 64;
   }
   row0 = by * kRows;
+  // this workgroup's slice of k
+  int K = a.K, first = 0;
+  if constexpr (OUT == kOutF32 && !GROUPED) {
+    first = blockIdx.z * a.slice_steps;
+    steps = min(a.slice_steps, steps - first);
+    K -= first * kWideK;
+  }
 
   // the runs this thread moves: fixed rows, k advancing by the step
   const T *src[kLoads];
@@ -394,7 +410,7 @@ rows_gemm_wide_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int co
       pr = list[lr] / a.list_div;
     else
       pr = (a.ring_base + lr) & a.ring_mask;
-    src[i] = static_cast<const T *>(a.A) + (int64_t)pr * a.lda;
+    src[i] = static_cast<const T *>(a.A) + (int64_t)pr * a.lda + first * kWideK;
   }
 
   const int ch0 = (bx * 4 + wave) * kTilesOut * 2; // first channel group of this wavefront
@@ -403,12 +419,12 @@ rows_gemm_wide_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int co
   for (int g = 0; g < GT; ++g) {
     const int mat = kPair ? g / kTilesOut : 0;
     const int gg = min(ch0 + 2 * (kPair ? g % kTilesOut : g) + ((lane >> 4) & 1), a.groups - 1);
-    wp[g] = W + ((int64_t)(mat * a.groups + gg) * ktiles) * 64 + (lane >> 5) * 16 + (lane & 15);
+    wp[g] = W + ((int64_t)(mat * a.groups + gg) * ktiles + first * 2) * 64 + (lane >> 5) * 16 + (lane & 15);
   }
 
   uint4 wr[4][GT * 4], xr[4][kLoads];
-  const int last_run = (a.K - 1) / kRunElems * kRunElems;
-  const bool ragged = a.K % kWideK != 0; // the last step reaches past K
+  const int last_run = (K - 1) / kRunElems * kRunElems;
+  const bool ragged = K % kWideK != 0; // the last step reaches past K
   auto fetch_w = [&](int s, uint4 (&w)[GT * 4]) {
     const int t = min(s, steps - 1) * 2;
 #pragma unroll
@@ -427,7 +443,7 @@ rows_gemm_wide_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int co
     if (ragged && s == steps - 1) {
 #pragma unroll
       for (int i = 0; i < kLoads; ++i)
-        x[i] = keep_run<T>(x[i], a.K - s * kWideK - run_k);
+        x[i] = keep_run<T>(x[i], K - s * kWideK - run_k);
     }
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
@@ -537,7 +553,7 @@ rows_gemm_wide_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int co
           pr = list[lr] / a.list_div;
         else
           pr = (a.ring_base + lr) & a.ring_mask;
-        const float *x = static_cast<const float *>(a.A) + (int64_t)pr * a.lda;
+        const float *x = static_cast<const float *>(a.A) + (int64_t)pr * a.lda + first * kWideK;
 #pragma unroll 1
         for (int n = 0; n < GT * 16; ++n) {
           float v = 0.f;
@@ -548,8 +564,8 @@ rows_gemm_wide_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int co
           const int group = ch0 + 2 * (kPair ? tile % kTilesOut : tile) + of / 16;
           if (v == v || group >= a.groups)
             continue;
-          const uint4 *w = W + ((int64_t)((kPair ? tile / kTilesOut : 0) * a.groups + group) * ktiles) * 64 + of % 16;
-          v = f32_sum(x, w, a.K);
+          const uint4 *w = W + ((int64_t)((kPair ? tile / kTilesOut : 0) * a.groups + group) * ktiles + first * 2) * 64 + of % 16;
+          v = f32_sum(x, w, min(K, steps * kWideK));
 #pragma unroll
           for (int i = 0; i < GT * 16; ++i)
             acc[i / 16][r][i % 16] = i == n ? v : acc[i / 16][r][i % 16];
@@ -580,7 +596,7 @@ rows_gemm_wide_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int co
           for (int i = 0; i < 4; ++i)
             if (ch + i < a.silu_channels)
               v[i] = silu_f(v[i]);
-          store4<float>(static_cast<float *>(a.C) + (int64_t)orow * a.ldc + ch, v);
+          store4<float>(static_cast<float *>(a.C) + blockIdx.z * a.slice_stride + (int64_t)orow * a.ldc + ch, v);
         } else if constexpr (OUT == kOutAct) {
           store4<T>(static_cast<T *>(a.C) + (int64_t)orow * a.ldc + ch, v);
         } else {
@@ -614,6 +630,11 @@ int launch_tiles(F kernel, int elems, const RowsGemm &a, hipStream_t stream) {
   d.list_cap = a.list_cap;
   d.list_div = a.list_div;
   d.expert_tiles = a.expert_tiles;
+  const int steps = (int)ceil_div(a.W.K, elems);
+  // slices of equal steps but the last, none of them empty
+  d.slice_steps = (int)ceil_div(ceil_div(a.W.K, kWideK), a.slices) * (kWideK / elems);
+  d.slice_stride = a.slice_stride;
+  const unsigned slices = a.slices > 1 ? (unsigned)ceil_div(steps, d.slice_steps) : 1;
   const int64_t blocks = GROUPED ? std::min<int64_t>(ceil_div(a.list_total, ROWS) + a.experts,
                                                      a.list_total)
                                  : ceil_div(a.rows, ROWS);
@@ -621,10 +642,10 @@ int launch_tiles(F kernel, int elems, const RowsGemm &a, hipStream_t stream) {
   BH_REQUIRE(blocks * columns < (int64_t)1 << 31, "rows_gemm: %lld row blocks", (long long)blocks);
   // The second dimension of a grid ends at 65535 (2.1 million rows in tiles of 32): then all
   // in the first.  (Always so, launches of 4 us took 0.2 longer.)
-  const dim3 grid = blocks <= 65535 ? dim3((unsigned)columns, (unsigned)blocks)
-                                    : dim3((unsigned)(blocks * columns));
+  const dim3 grid = blocks <= 65535 ? dim3((unsigned)columns, (unsigned)blocks, slices)
+                                    : dim3((unsigned)(blocks * columns), 1, slices);
   hipLaunchKernelGGL(kernel, grid, dim3(kGemmThreads), 0, stream, a.W.tiles,
-                     a.W.ktiles, (int)ceil_div(a.W.K, elems), (int)columns, (int)blocks, d);
+                     a.W.ktiles, steps, (int)columns, (int)blocks, d);
   BH_CHECK_HIP(hipGetLastError());
   return BUDDY_HIP_OK;
 }
@@ -656,8 +677,9 @@ int launch_wide(const RowsGemm &a, hipStream_t stream) {
 // 32 or 64 x 128): 8960 -> 1536 at 24 rows 21.2 vs 28.4, at 150 22.7 vs 31.3, at 220 36.0
 // vs 31.5; 1536 -> 1536 at 64 rows 5.6 vs 6.9; 1536 -> 17920 at 64 rows 18.4 vs 12.4.  In
 // f32, whose three terms make the products the longer part, they gain nothing.
+constexpr double kSliceUs = 0.5; // of slices besides
 template <typename T, int OUT, bool GROUPED>
-int launch_shape(const RowsGemm &a, hipStream_t stream) {
+int launch_shape(const RowsGemm &a, hipStream_t stream, int *slices) {
   const int64_t rows = GROUPED ? ceil_div(a.list_total, a.experts) : a.rows;
   const int64_t all_blocks = GROUPED ? std::min<int64_t>(a.experts, a.list_total) : 1;
   constexpr bool kPair = OUT == kOutExpertAct;
@@ -665,66 +687,103 @@ int launch_shape(const RowsGemm &a, hipStream_t stream) {
   auto workgroups = [&](int rt, int ch) {
     return ceil_div(a.W.N, ch) * ceil_div(rows, rt) * all_blocks;
   };
-  if (rows <= 16)
-    return workgroups(16, 128) >= 256 ? launch_flat<T, 2 * P, OUT, GROUPED>(a, stream)
-                                      : launch_flat<T, P, OUT, GROUPED>(a, stream);
-  const double steps = (double)ceil_div(a.W.K, kWideK);
+  if (rows <= 16) {
+    RowsGemm b = a;
+    b.slices = 1;
+    return workgroups(16, 128) >= 256 ? launch_flat<T, 2 * P, OUT, GROUPED>(b, stream)
+                                      : launch_flat<T, P, OUT, GROUPED>(b, stream);
+  }
+  // With slices of k that the caller adds: the tile and the number of slices together, which
+  // cost the bytes of their sums.  8960 -> 1536: 777
+  // bfloat16 rows 50 us whole and 38 in three slices, 300 f32 rows 72 and 36 in four; whole prompts
+  // of 20 to 500 tokens 1.08 to 1.48 times as fast.
+  const int64_t steps = ceil_div(a.W.K, kWideK);
+  int cut = 1; // slices of the estimate that was the lowest of a tile
+  struct Cost {
+    double us;
+    int slices;
+    bool operator<=(const Cost &o) const { return us <= o.us; }
+    bool operator<(const Cost &o) const { return us < o.us; }
+  };
   auto cost = [&](int rt, int ch, double step_us, double fixed_us) {
-    return (double)ceil_div(workgroups(rt, ch / P), 256) * steps * step_us + fixed_us;
+    Cost best{1e30, 1};
+    for (int s = 1; s <= a.slices; ++s) {
+      const int64_t per = ceil_div(steps, s);
+      if (ceil_div(steps, per) != s)
+        continue; // the last slice would be empty
+      const double us = (double)(ceil_div(workgroups(rt, ch / P) * s, 256) * per) * step_us + fixed_us +
+                        (s - 1) * 8e-6 / 4.8 * (double)rows * a.W.N + (s > 1 ? kSliceUs : 0.0);
+      if (us < best.us)
+        best = {us, s};
+    }
+    return best;
+  };
+  auto with = [&](const Cost &c) {
+    cut = c.slices;
+    RowsGemm b = a;
+    b.slices = cut;
+    return b;
+  };
+  auto done = [&](int rc) {
+    if (slices)
+      *slices = cut;
+    return rc;
   };
   if constexpr (sizeof(T) == 4) {
-    if constexpr (!kPair)
-      if (cost(32, 128, 0.46, 4.0) <= cost(32, 256, 0.80, 4.5))
-        return launch_wide<T, 1, 1, OUT, GROUPED>(a, stream);
-    return launch_wide<T, 1, 2, OUT, GROUPED>(a, stream);
+    const Cost wide = cost(32, 256, 0.80, 4.5);
+    if constexpr (!kPair) {
+      const Cost low = cost(32, 128, 0.46, 4.0);
+      if (low <= wide)
+        return done(launch_wide<T, 1, 1, OUT, GROUPED>(with(low), stream));
+    }
+    return done(launch_wide<T, 1, 2, OUT, GROUPED>(with(wide), stream));
   } else {
     // few rows: 16-row tiles of 64 channels, while they are few rounds of the chip
-    const double tall = cost(128, 256, 1.02, 7.0), flat = cost(16, 64 * P, 0.13 * P, 2.5);
+    const Cost tall = cost(128, 256, 1.02, 7.0), flat = cost(16, 64 * P, 0.13 * P, 2.5);
+    Cost half, low;
     if constexpr (kPair) {
       // fewer workgroups than half the chip draw the weights from memory too slowly
       auto thin = [&](int rt) { return workgroups(rt, 128) < 128 ? 6.0 : 0.0; };
-      const double half = cost(64, 256, 0.60, 5.0) + thin(64);
-      const double low = cost(32, 256, 0.40, 4.0) + thin(32);
-      if (flat <= std::min({tall, half, low}))
-        return launch_flat<T, P, OUT, GROUPED>(a, stream);
-      if (tall <= std::min(half, low))
-        return launch_wide<T, 4, 2, OUT, GROUPED>(a, stream);
-      return half <= low ? launch_wide<T, 2, 2, OUT, GROUPED>(a, stream)
-                         : launch_wide<T, 1, 2, OUT, GROUPED>(a, stream);
+      half = cost(64, 256, 0.60, 5.0);
+      half.us += thin(64);
+      low = cost(32, 256, 0.40, 4.0);
+      low.us += thin(32);
     } else {
-      const double half = cost(64, 128, 0.29, 4.5), low = cost(32, 128, 0.21, 4.0);
-      if (flat <= std::min({tall, half, low}))
-        return launch_flat<T, P, OUT, GROUPED>(a, stream);
-      if (tall <= std::min(half, low))
-        return launch_wide<T, 4, 2, OUT, GROUPED>(a, stream);
-      return half <= low ? launch_wide<T, 2, 1, OUT, GROUPED>(a, stream)
-                         : launch_wide<T, 1, 1, OUT, GROUPED>(a, stream);
+      half = cost(64, 128, 0.29, 4.5);
+      low = cost(32, 128, 0.21, 4.0);
     }
+    if (flat <= std::min({tall, half, low}))
+      return done(launch_flat<T, P, OUT, GROUPED>(with(flat), stream));
+    if (tall <= std::min(half, low))
+      return done(launch_wide<T, 4, 2, OUT, GROUPED>(with(tall), stream));
+    constexpr int GT = kPair ? 2 : 1;
+    return done(half <= low ? launch_wide<T, 2, GT, OUT, GROUPED>(with(half), stream)
+                            : launch_wide<T, 1, GT, OUT, GROUPED>(with(low), stream));
   }
 }
 
-template <typename T> int launch_typed(const RowsGemm &a, hipStream_t stream) {
+template <typename T> int launch_typed(const RowsGemm &a, hipStream_t stream, int *slices) {
   const bool grouped = a.counts != nullptr;
   switch (a.out) {
   case kOutF32:
-    return grouped ? launch_shape<T, kOutF32, true>(a, stream)
-                   : launch_shape<T, kOutF32, false>(a, stream);
+    return grouped ? launch_shape<T, kOutF32, true>(a, stream, slices)
+                   : launch_shape<T, kOutF32, false>(a, stream, slices);
   case kOutAct:
     BH_REQUIRE(!grouped, "rows_gemm: form not compiled for expert lists");
-    return launch_shape<T, kOutAct, false>(a, stream);
+    return launch_shape<T, kOutAct, false>(a, stream, slices);
   case kOutActTrans:
     BH_REQUIRE(!grouped, "rows_gemm: form not compiled for expert lists");
-    return launch_shape<T, kOutActTrans, false>(a, stream);
+    return launch_shape<T, kOutActTrans, false>(a, stream, slices);
   case kOutExpertAct:
-    return grouped ? launch_shape<T, kOutExpertAct, true>(a, stream)
-                   : launch_shape<T, kOutExpertAct, false>(a, stream);
+    return grouped ? launch_shape<T, kOutExpertAct, true>(a, stream, slices)
+                   : launch_shape<T, kOutExpertAct, false>(a, stream, slices);
   }
   return fail(BUDDY_HIP_ERR_ARG, "rows_gemm: output form %d", (int)a.out);
 }
 
 } // namespace
 
-int launch_rows_gemm(const RowsGemm &a, hipStream_t stream) {
+int launch_rows_gemm(const RowsGemm &a, hipStream_t stream, int *slices) {
   const Bf16Matrix &W = a.W;
   BH_REQUIRE(W.tiles && W.K > 0 && W.N > 0 && W.N % 16 == 0 && W.ktiles == bf16_ktiles(W.K) &&
                  a.A && a.C && a.rows >= 0,
@@ -737,9 +796,14 @@ int launch_rows_gemm(const RowsGemm &a, hipStream_t stream) {
              "rows_gemm: result rows (ldc %d, N %d)", a.ldc, W.N);
   BH_REQUIRE(!a.counts || (a.lists && a.experts > 0 && a.list_cap > 0 && a.list_div > 0),
              "rows_gemm: expert lists");
+  BH_REQUIRE(a.slices >= 1 && (a.slices == 1 || (slices && a.out == kOutF32 && !a.silu_channels && !a.counts &&
+                                                 a.slice_stride >= (int64_t)a.rows * a.ldc && a.slice_stride % 4 == 0)),
+             "rows_gemm: slices of k");
+  if (slices)
+    *slices = 1;
   if (a.counts ? a.list_total == 0 : a.rows == 0)
     return BUDDY_HIP_OK;
-  return a.f32 ? launch_typed<float>(a, stream) : launch_typed<bf16_bits>(a, stream);
+  return a.f32 ? launch_typed<float>(a, stream, slices) : launch_typed<bf16_bits>(a, stream, slices);
 }
 
 } // namespace bh

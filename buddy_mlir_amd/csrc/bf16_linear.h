@@ -132,7 +132,12 @@ struct RowsGemm {
   const int *lists = nullptr;  // [experts][list_cap]
   int list_cap = 0, list_div = 1, list_total = 0; // total: assignments over all experts
   int64_t expert_tiles = 0;    // 1 KiB tiles from one expert's matrix to the next
+  // kOutF32 without silu_channels, not grouped: K may be cut into up to `slices` slices, whose
+  // sums lie `slice_stride` floats apart in C and are the caller's to add, in slice order
+  int slices = 1;
+  int64_t slice_stride = 0;
 };
-int launch_rows_gemm(const RowsGemm &a, hipStream_t stream);
+// `slices`: how many there are
+int launch_rows_gemm(const RowsGemm &a, hipStream_t stream, int *slices = nullptr);
 
 } // namespace bh

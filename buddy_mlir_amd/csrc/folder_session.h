@@ -198,6 +198,26 @@ struct FolderSession : Session {
     g.ldc = ldc;
     return g;
   }
+  // What a product whose K is cut into slices may leave, so many floats for a block of `rows`
+  // rows and `width` channels; and such a product, for the norm behind it to add.
+  static constexpr int kMaxSlices = 8;
+  static constexpr int64_t kSliceFloats = 4 << 20; // 16 MB, unless a single slice is more
+  // rows from which the tiles of one slice fill the chip (prompts of 1200 tokens take as long
+  // either way, of 777 1.04 to 1.1 times as long without slices)
+  static constexpr int kSliceRows = 1024;
+  static size_t sliced_floats(int rows, int width) {
+    const int64_t one = (int64_t)rows * width, few = (int64_t)std::min(rows, kSliceRows) * width;
+    return (size_t)std::max(one, std::min(kMaxSlices * few, kSliceFloats));
+  }
+  int sliced_product(const Bf16Matrix &W, const void *A, int lda, int rows, float *y, NormRows &pend) {
+    RowsGemm g = gemm(W, A, lda, rows, kOutF32, y, W.N);
+    g.slice_stride = (int64_t)rows * W.N;
+    if (rows <= kSliceRows)
+      g.slices = (int)std::clamp<int64_t>((int64_t)sliced_floats(rows, W.N) / g.slice_stride, 1, kMaxSlices);
+    pend.y = y;
+    pend.y_stride = g.slice_stride;
+    return launch_rows_gemm(g, stream, &pend.y_slices);
+  }
   // The head on the listed rows of a block.  `pend`: the last residual sum and norm;
   // `row`: [width], `act`: [kLogitRows][ld_act], `out`: [kLogitRows][head.N].
   int logit_rows(NormRows pend, const Bf16Matrix &head, const int *rows, int n_rows, float *row,

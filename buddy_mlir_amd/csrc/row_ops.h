@@ -20,6 +20,8 @@ struct NormRows {
   bool write_x = false;          // x' goes back into x
   const float *y = nullptr;      // [rows][ldy], or null
   int ldy = 0;
+  int y_slices = 1;              // y is the sum of so many, in order,
+  int64_t y_stride = 0;          // this many floats apart
   const float *expert_out = nullptr; // [rows * top][lde]
   const float *expert_w = nullptr;   // [rows][top]
   int lde = 0, top = 0;

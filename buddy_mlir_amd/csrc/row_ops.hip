@@ -86,6 +86,12 @@ __global__ void __launch_bounds__(256) norm_rows_kernel(NormRows a) {
       Run<V> y{};
       if (a.y)
         y = load_run<V>(a.y + r * a.ldy + i);
+      for (int s = 1; s < a.y_slices; ++s) {
+        const Run<V> e = load_run<V>(a.y + s * a.y_stride + r * a.ldy + i);
+#pragma unroll
+        for (int k = 0; k < V; ++k)
+          y.v[k] += e.v[k];
+      }
       for (int j = 0; j < a.top; ++j) {
         const float w = a.expert_w[r * a.top + j];
         const Run<V> e = load_run<V>(a.expert_out + (r * a.top + j) * a.lde + i);
@@ -304,12 +310,12 @@ int launch_embed_rows(const uint16_t *table, const int *tokens, int rows, int wi
 int launch_norm_rows(const NormRows &a, hipStream_t stream) {
   BH_REQUIRE(a.x && a.rows > 0 && a.width > 0 && (!a.pick || !a.write_x) &&
                  (!a.expert_out || (a.expert_w && a.top > 0)) && (a.expert_out || a.top == 0) &&
-                 (!a.add || a.plain_y),
+                 (!a.add || a.plain_y) && (a.y_slices == 1 || a.y),
              "norm_rows: bad argument");
   const size_t lds = 2 * sizeof(float) * (size_t)a.width;
   constexpr size_t kLimit = 150 * 1024;
   BH_REQUIRE(lds <= kLimit, "norm_rows: a row of %d values does not fit LDS", a.width);
-  bool quads = a.width % 4 == 0 && a.ldy % 4 == 0 && a.lde % 4 == 0 && a.ld_act % 4 == 0;
+  bool quads = a.width % 4 == 0 && a.ldy % 4 == 0 && a.y_stride % 4 == 0 && a.lde % 4 == 0 && a.ld_act % 4 == 0;
   for (const void *p : {(const void *)a.x, (const void *)a.y, (const void *)a.expert_out,
                         (const void *)a.add, (const void *)a.norm_w, (const void *)a.out_f32, (const void *)a.out_act})
     quads = quads && ((uintptr_t)p & 15) == 0;

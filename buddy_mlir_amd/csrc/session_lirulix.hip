@@ -464,7 +464,7 @@ struct LirulixSession : FolderSession {
       ff = std::max(ff, (size_t)round_up(cfg.layers[i].ff, 16));
     }
     int rc = block_alloc(&pf_x, 4 * n * cfg.width);
-    rc |= block_alloc(&pf_y, 4 * n * width16());
+    rc |= block_alloc(&pf_y, 4 * sliced_floats(rows, width16()));
     rc |= block_alloc(&pf_act, T * n * ld_act);
     rc |= block_alloc(&pf_proj, 4 * n * max_proj);
     rc |= block_alloc(&pf_mix, T * n * ld_mix);
@@ -539,11 +539,11 @@ struct LirulixSession : FolderSession {
       a.norm_w = norm;
       a.out_act = pf_act;
       pend.y = nullptr;
+      pend.y_slices = 1;
       return launch_norm_rows(a, stream);
     };
     auto product = [&](const Bf16Matrix &M, const void *A, int lda) {
-      pend.y = pf_y;
-      return launch_rows_gemm(gemm(M, A, lda, n, kOutF32, pf_y, M.N), stream);
+      return sliced_product(M, A, lda, n, pf_y, pend);
     };
     for (const LirulixRun &r : runs) {
       const LirulixLayer &L = layers[(size_t)r.layer];

@@ -489,7 +489,7 @@ struct NukopelSession : FolderSession {
     }
     int rc = block_alloc(&pf_x, 4 * n * cfg.width);
     rc |= block_alloc(&pf_h, 4 * n * cfg.width);
-    rc |= block_alloc(&pf_y, 4 * n * width16());
+    rc |= block_alloc(&pf_y, 4 * sliced_floats(rows, width16()));
     rc |= block_alloc(&pf_act, T * n * ld_act);
     rc |= block_alloc(&pf_proj, 4 * n * max_proj);
     rc |= block_alloc(&pf_mix, T * n * ld_mix);
@@ -579,7 +579,7 @@ struct NukopelSession : FolderSession {
     return launch_gated_norm_rows(g, stream);
   }
 
-  int moe_rows(NukopelLayer &L, const LayerConfig &c, int n) {
+  int moe_rows(NukopelLayer &L, const LayerConfig &c, int n, NormRows &pend) {
     int rc;
     if ((rc = launch_rows_gemm(gemm(L.router, pf_act, ld_act, n, kOutF32, pf_router, L.router.N), stream)))
       return rc;
@@ -622,10 +622,10 @@ struct NukopelSession : FolderSession {
       su.limit = c.shared_expert.limit;
       if ((rc = launch_rows_gemm(su, stream)))
         return rc;
-      if ((rc = launch_rows_gemm(gemm(L.shared_down, pf_shared, L.shared_gate_up.N, n, kOutF32, pf_y,
-                                      L.shared_down.N), stream)))
-        return rc;
+      return sliced_product(L.shared_down, pf_shared, L.shared_gate_up.N, n, pf_y, pend);
     }
+    pend.y = nullptr;
+    pend.y_slices = 1;
     return BUDDY_HIP_OK;
   }
 
@@ -671,9 +671,8 @@ struct NukopelSession : FolderSession {
         return rc;
       if ((rc = c.latent ? latent_rows(L, n, start) : linear_rows(L, n)))
         return rc;
-      if ((rc = launch_rows_gemm(gemm(L.o, pf_mix, ld_mix, n, kOutF32, pf_y, L.o.N), stream)))
+      if ((rc = sliced_product(L.o, pf_mix, ld_mix, n, pf_y, pend)))
         return rc;
-      pend.y = pf_y;
       pend.expert_out = nullptr;
       pend.top = 0;
       pend.out_gain = L.norm1b;
@@ -686,9 +685,8 @@ struct NukopelSession : FolderSession {
       b.out_act = pf_act;
       if ((rc = launch_norm_rows(b, stream)))
         return rc;
-      if ((rc = moe_rows(L, c, n)))
+      if ((rc = moe_rows(L, c, n, pend)))
         return rc;
-      pend.y = c.shared ? pf_y : nullptr;
       pend.expert_out = pf_experts;
       pend.expert_w = pf_weights;
       pend.top = c.top;

@@ -116,6 +116,20 @@ def test_one_row_through_the_feed_forward(tmp_path, width, ff, dtype):
     check(feed(s, tokens, [1] * 5), L.forward(cfg, t, tokens), dtype)
 
 
+# products of a prompt whose K is cut into slices that the norm behind them adds: K that ends inside
+# a step, slices of unequal length, rows on both sides of a tile, several portions of other sizes
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width,ff,n", [(72, 8970, 17), (72, 8970, 33), (200, 4100, 97), (72, 2310, 130),
+                                        (46, 5001, 65), (1536, 1700, 300)])
+def test_prompt_products_in_slices_of_k(tmp_path, width, ff, n, dtype):
+    cfg = M.config([M.full(heads=1, ff=ff), M.delta(ff=ff)], loop=(0, 2, 2), width=width, vocab=64)
+    folder, t = M.build(tmp_path, cfg, ff)
+    tokens = tokens_for(cfg, n + 21)
+    want = L.forward(cfg, t, tokens)
+    s = FolderSession(folder, dtype, max_len=n + 32)
+    check(feed(s, tokens, [n, 20, 1]), want, dtype)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("block", [0, 16, 80])
 def test_portions_do_not_matter(tmp_path, dtype, block):
