@@ -35,8 +35,8 @@ struct PromptFold {
 };
 
 // Whether launch_attn_prompt and the fold behind it are to be taken for a session's prompt, or
-// attn_prefill.hip and the conversion behind that; `digits`: the fold writes digit planes.
-bool attn_prompt_pays(int q_len, int q_offset, int heads, int kv_heads, bool digits);
+// attn_prefill.hip and the conversion behind that.
+bool attn_prompt_pays(int q_len, int q_offset, int heads, int kv_heads);
 
 // Attention of a session's prompt tokens (no mask), on a workspace of
 // attn_prompt_workspace_bytes for at least as many tokens and positions; what it leaves is
@@ -44,10 +44,10 @@ bool attn_prompt_pays(int q_len, int q_offset, int heads, int kv_heads, bool dig
 struct AttnPrefillArgs;
 size_t attn_prompt_workspace_bytes(int q_len, int k_len, int heads, int kv_heads);
 int launch_attn_prompt(const AttnPrefillArgs &a, void *workspace, PromptFold &fold, hipStream_t stream);
-// the finished rows [tokens, heads, 128] in place ...
-int launch_attn_fold_rows(const PromptFold &fold, float *out, int64_t o_stride, int heads, int tokens,
-                          hipStream_t stream);
-// ... or as the digit planes of the matmul behind the attention (gemm_w8_i8.hip)
+// the finished rows as the bf16 terms of the matmul behind the attention (gemm_w8_mfma.hip) ...
+int launch_attn_fold_to_terms(const PromptFold &fold, int64_t o_stride, int heads, int tokens, int terms,
+                              unsigned short *staged, hipStream_t stream);
+// ... or as its digit planes (gemm_w8_i8.hip)
 int launch_attn_fold_to_digits(const PromptFold &fold, int64_t o_stride, int heads, int tokens, int digits,
                                void *staged, hipStream_t stream);
 

@@ -458,30 +458,6 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
   }
 }
 
-// the finished rows where other consumers want them: one workgroup per token
-constexpr int kFoldThreads = 512;
-__global__ void __launch_bounds__(kFoldThreads)
-attn_fold_rows_kernel(PromptFold f, float *out, int64_t o_stride, int heads) {
-  const int t = blockIdx.x;
-  float *row = out + (int64_t)t * o_stride;
-  bool bad = false;
-  for (int i = threadIdx.x * 4; i < heads * kPromptD; i += 4 * kFoldThreads) {
-    float v[4];
-    left4(f, o_stride, t, i / kPromptD, i % kPromptD, v);
-    bad |= to_repair(v);
-    *reinterpret_cast<float4 *>(row + i) = float4{v[0], v[1], v[2], v[3]};
-  }
-  if (__any(bad)) {
-#pragma unroll 1
-    for (int i = threadIdx.x * 4; i < heads * kPromptD; i += 4 * kFoldThreads) {
-      const float4 q = *reinterpret_cast<const float4 *>(row + i);
-      float v[4] = {q.x, q.y, q.z, q.w};
-      repair4(f, t, i / kPromptD, i % kPromptD, v);
-      *reinterpret_cast<float4 *>(row + i) = float4{v[0], v[1], v[2], v[3]};
-    }
-  }
-}
-
 } // namespace
 
 // The (KV head, row block, key tile) triples of a launch and who takes them.
@@ -517,7 +493,7 @@ PromptShare share_out(int q_len, int q_offset, int heads, int kv_heads) {
 // The estimate is off by a tenth here and there.  More than 640 tokens go this way in doubt,
 // which keeps what is not finite to the rows that see it (700 tokens of 6 heads, one KV head:
 // 28.5 and 29.3); short prompts with little ahead of them the other.
-bool attn_prompt_pays(int q_len, int q_offset, int heads, int kv_heads, bool digits) {
+bool attn_prompt_pays(int q_len, int q_offset, int heads, int kv_heads) {
   const double kilo_rows = 1e-4 * q_len * heads; // tens of thousands of (token, head)
   // attn_prefill.hip: blocks of 16 queries, two together while a workgroup of eight wavefronts
   // per pair fits the chip; steps of 16 keys per wavefront
@@ -541,8 +517,7 @@ bool attn_prompt_pays(int q_len, int q_offset, int heads, int kv_heads, bool dig
   const double here = 10.6 + 5.7 * (double)(ceil_div(s.tiles, s.workgroups) - 1) +
                       1.4 * (double)std::max<int64_t>(0, waves - 4) + 5.0 * s.workgroups / 256 +
                       2.0 * s.nblk * kv_heads / s.workgroups + (double)ceil_div(heads, 16) * trips +
-                      0.82 * kilo_rows * std::min(parts, 20.0) +
-                      (digits ? 0.0 : 3.0); // bfloat16 modes convert the fold's rows in a launch of its own
+                      0.82 * kilo_rows * std::min(parts, 20.0);
   return here < (q_len > 640 ? 1.08 : q_offset >= 128 ? 1.0 : 0.9) * other;
 }
 
@@ -612,13 +587,6 @@ int launch_attn_prompt(const AttnPrefillArgs &in, void *workspace, PromptFold &f
   fold.kv_stride = a.kv_stride;
   fold.q_offset = a.q_offset;
   fold.scale = a.scale;
-  return BUDDY_HIP_OK;
-}
-
-int launch_attn_fold_rows(const PromptFold &fold, float *out, int64_t o_stride, int heads, int tokens,
-                          hipStream_t stream) {
-  hipLaunchKernelGGL(attn_fold_rows_kernel, dim3(tokens), dim3(kFoldThreads), 0, stream, fold, out, o_stride, heads);
-  BH_CHECK_HIP(hipGetLastError());
   return BUDDY_HIP_OK;
 }
 

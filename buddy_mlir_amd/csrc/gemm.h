@@ -20,19 +20,18 @@ struct GemmW8Args {
   // relative to each row's maximum) and multiply on the int8 matrix cores;
   // 0: bf16 terms as above
   int digits = 0;
-  // digits only: W holds two matrices of N / 2 channels one behind the other
-  // (scales likewise), and C [M, N / 2] = SiLU(A . first) * (A . second)
+  // W holds two matrices of N / 2 channels one behind the other
+  // (scales likewise), and C [M, N / 2] = SiLU(A . first) * (A . second); without digits the
+  // result leaves as bf16 terms in silu_staged (layout of gemm_staging_layout(M, N / 2))
   bool silu_pair = false;
-  // digits only: the finished rows of C also leave as RMSNorm(row) * then_norm_w
-  // in digit planes (then_norm_staged: layout of gemm_staging_layout(M, N)), the
+  void *silu_staged = nullptr;
+  // the finished rows of C also leave as RMSNorm(row) * then_norm_w in digit planes or
+  // terms (then_norm_staged: layout of gemm_staging_layout(M, N)), the
   // input of the matmul that follows -- written by the kernel that adds the K
   // slices where there is one, by a launch of its own otherwise
   const float *then_norm_w = nullptr;
   float then_norm_eps = 0.f;
   void *then_norm_staged = nullptr;
-  // A (same pointer, shape, terms, contents) was the input of the previous
-  // matmul on this stream: its bf16 copy is still staged, skip the conversion
-  bool reuse_staged_a = false;
   // Caller-provided staging of A (written by one of the producers below for
   // exactly this M, K and terms / digits): no conversion, A itself is not read.
   const void *staged = nullptr;

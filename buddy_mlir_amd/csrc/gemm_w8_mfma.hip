@@ -21,12 +21,14 @@
 //    on the same XCD and share the weight tiles in its L2 (tile_place.h);
 //  * the per-channel scale is applied once to the f32 accumulators, where the
 //    reference multiplies every element before the FMA.
+#include "attn_fold.h"
 #include "gemm.h"
 #include "tile_place.h"
 
 #include <algorithm>
 #include <map>
 #include <mutex>
+#include <type_traits>
 
 namespace bh {
 namespace {
@@ -107,6 +109,50 @@ __device__ __forceinline__ void store_terms(float (&r)[8], int terms, u16 *out,
   }
 }
 
+// the same for four
+__device__ __forceinline__ void store_terms4(const float (&v)[4], int terms, u16 *out, size_t term_stride) {
+  float r[4] = {v[0], v[1], v[2], v[3]};
+  for (int t = 0; t < terms; ++t) {
+    u16 h[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      h[e] = bf16_rne(r[e]);
+      r[e] -= bf16_to_f32(h[e]);
+    }
+    *reinterpret_cast<uint2 *>(out + t * term_stride) = make_uint2(pack2(h[0], h[1]), pack2(h[2], h[3]));
+  }
+}
+
+__device__ __forceinline__ float silu_times(float g, float u) {
+  const float sig = 1.0f / (1.0f + expf(-g));
+  return (g * sig) * u;
+}
+
+// One workgroup per token: the attention's output, added up from its parts, as the terms of
+// the matmul behind it (in f32 rows and a conversion: 8.7 + 4.4 us for 150 tokens).
+__global__ void __launch_bounds__(512)
+attn_fold_to_terms_kernel(PromptFold f, int64_t o_stride, int n, int terms, int Mp, u16 *__restrict__ out) {
+  const int t = blockIdx.x;
+  u16 *row = out + (size_t)t * n;
+  const size_t term_stride = (size_t)Mp * n;
+  bool bad = false;
+  for (int i = threadIdx.x * 4; i < n; i += 4 * 512) {
+    float v[4];
+    left4(f, o_stride, t, i / kPromptD, i % kPromptD, v);
+    bad |= to_repair(v);
+    store_terms4(v, terms, row + i, term_stride);
+  }
+  if (__any(bad)) {
+#pragma unroll 1
+    for (int i = threadIdx.x * 4; i < n; i += 4 * 512) {
+      float v[4];
+      left4(f, o_stride, t, i / kPromptD, i % kPromptD, v);
+      repair4(f, t, i / kPromptD, i % kPromptD, v);
+      store_terms4(v, terms, row + i, term_stride);
+    }
+  }
+}
+
 // One workgroup per row: y = w * (x * rsqrt(sum(x^2) / n + eps)) -> staging
 __global__ void __launch_bounds__(256)
 rmsnorm_to_staging_kernel(const float *__restrict__ x, const float *__restrict__ w, int n,
@@ -159,10 +205,8 @@ silu_mul_to_staging_kernel(const float *__restrict__ g, const float *__restrict_
     }
   }
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const float sig = 1.0f / (1.0f + expf(-gv[e]));
-    r[e] = k0 + e < n ? (gv[e] * sig) * uv[e] : 0.f;
-  }
+  for (int e = 0; e < 8; ++e)
+    r[e] = k0 + e < n ? silu_times(gv[e], uv[e]) : 0.f;
   store_terms(r, terms, out + (size_t)row * Kp + k0, (size_t)Mp * Kp);
 }
 
@@ -182,6 +226,8 @@ struct GemmArgs {
   float *partial;            // [tile][slice][wavefront][row][channel], where K is split
   int span, tile_rows;       // channels per wavefront, rows per workgroup
   int accumulate;
+  u16 *pair_out; // PAIR: the result's terms [terms][Mp][pair_Kp]
+  int pair_Kp;
 };
 
 // A tile of 32 RB rows x 128 GP channels, on v_mfma_f32_32x32x16_bf16 (GP tiles of 32 channels per wavefront); every
@@ -194,19 +240,29 @@ struct GemmArgs {
 // first fragments were read during step c - 1, and fills buffer (c + 2) % 3, last read before
 // the previous barrier).  The weights of a quarter of a chunk are converted while the
 // quarter before it is multiplied.
+//
+// A round of the ring has no branch: where paths of fewer chunks join, the compiler waits for
+// all loads but those of the shortest path ahead of any register it uses again.
+//
+// PAIR: W holds two matrices of a.groups / 2 channel groups each, one behind the other; a tile
+// of 32 channels is a group of the first and the same group of the second, and what is stored
+// is SiLU(first) * second as the terms of the next matmul's input (as f32 and a launch that
+// reads it back: 22.9 + 5.3 us for 150 rows of 1536 -> 2 x 8960, 19.9 now).
 constexpr int kRing = 4;               // chunks in registers
 constexpr int kRowBytes = 2 * kTileK + 16; // of a row in LDS: reads meet every bank once
 
-template <int TERMS, int RB, int GP>
+template <int TERMS, int RB, int GP, bool PAIR>
 __device__ __forceinline__ void multiply_tile(const GemmArgs &a) {
   constexpr int L = TERMS * RB; // layers of 32 rows: term l % TERMS of row block l / TERMS
-  constexpr int kRows = 32 * RB, kSpan = 32 * GP, kThreads = kWaves * kWave;
+  constexpr int kWidth = PAIR ? 16 : 32; // channels of the result per tile
+  constexpr int kRows = 32 * RB, kSpan = kWidth * GP, kThreads = kWaves * kWave;
+  constexpr int kScales = kWaves * 32 * GP;
   constexpr int kBuf = L * 32 * kRowBytes;
   constexpr int kTurn = kSpan + 4; // floats of a row of the epilogue's tile
   constexpr int kTurned = kWaves * 32 * kTurn * 4;
   constexpr int kLds = 3 * kBuf > kTurned ? 3 * kBuf : kTurned;
   __shared__ __attribute__((aligned(16))) unsigned char lds[kLds];
-  __shared__ __attribute__((aligned(16))) float scale_s[kWaves * kSpan], bias_s[kWaves * kSpan];
+  __shared__ __attribute__((aligned(16))) float scale_s[kScales], bias_s[PAIR ? 4 : kScales];
   const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, up = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int unit, rbk;
@@ -217,11 +273,14 @@ __device__ __forceinline__ void multiply_tile(const GemmArgs &a) {
   const int g0 = (ctile * kWaves + wave) * (kSpan / 16); // first channel group of this wavefront
   const int cb = slice * a.chunks_per_slice;
   const int nch = min(a.chunks_per_slice, a.chunks - cb); // chunks of this slice, >= 1
+  const int half_groups = a.groups / 2; // PAIR only
 
   const v4i32 *wp[GP];
 #pragma unroll
   for (int g = 0; g < GP; ++g) { // groups past the end repeat the last one
-    const int gg = min(g0 + 2 * g + ((lane >> 4) & 1), a.groups - 1);
+    const int second = (lane >> 4) & 1; // group of the tile
+    const int gg = PAIR ? min(g0 + g, half_groups - 1) + second * half_groups
+                        : min(g0 + 2 * g + second, a.groups - 1);
     wp[g] = reinterpret_cast<const v4i32 *>(a.W) + ((size_t)gg * a.chunks + cb) * 64 + up * 16 +
             (lane & 15);
   }
@@ -233,6 +292,7 @@ __device__ __forceinline__ void multiply_tile(const GemmArgs &a) {
              (size_t)cb * kTileK + (tid & 7) * 8;
   const int lds_at = tid / 8 * kRowBytes + (tid & 7) * 16;
   v4i32 wr[kRing][GP * 2], xr[kRing][L];
+  constexpr int kFetches = 2 * GP + L; // loads of a chunk
   auto fetch_w = [&](int c, v4i32 (&w)[GP * 2]) {
     const size_t cc = (size_t)min(c, nch - 1) * 64;
 #pragma unroll
@@ -266,10 +326,11 @@ __device__ __forceinline__ void multiply_tile(const GemmArgs &a) {
       fetch_x(u + 2, xr[u + 2]);
   }
   if (a.slices == 1)
-    for (int i = tid; i < kWaves * kSpan; i += kThreads) {
-      const int n = ctile * kWaves * kSpan + i;
-      scale_s[i] = n < a.N ? a.scale[n] : 0.f;
-      bias_s[i] = a.bias && n < a.N ? a.bias[n] : 0.f;
+    for (int i = tid; i < kScales; i += kThreads) {
+      const int mtx = PAIR ? i / (kScales / 2) : 0, n = ctile * kWaves * kSpan + (PAIR ? i % (kScales / 2) : i);
+      scale_s[i] = n < a.N ? a.scale[(size_t)mtx * a.N + n] : 0.f;
+      if constexpr (!PAIR)
+        bias_s[i] = a.bias && n < a.N ? a.bias[n] : 0.f;
     }
 
   f32x16 acc[GP][RB];
@@ -298,6 +359,8 @@ __device__ __forceinline__ void multiply_tile(const GemmArgs &a) {
     wf[0][g] = convert(wr[0], 0, g);
   auto step = [&](int c, const v4i32 (&w)[GP * 2], const v4i32 (&w_next)[GP * 2],
                   v4i32 (&w_new)[GP * 2], v4i32 (&x)[L], v4i32 (&x_new)[L]) {
+    const size_t wc = (size_t)min(c + kRing - 1, nch - 1) * 64;
+    const size_t xc = (size_t)min(c + kRing + 1, nch - 1) * kTileK;
 #pragma unroll
     for (int u = 0; u < 4 * L; ++u) {
       const int t = u / L, l = u % L;
@@ -305,12 +368,16 @@ __device__ __forceinline__ void multiply_tile(const GemmArgs &a) {
       // the way through LDS), and stay there: left to itself the scheduler moves them to
       // their use
       load_frag(u + 2 < 4 * L ? cur : next, (u + 2) % (4 * L), frag[(u + 2) & 3]);
-      if (u == 0)
-        fetch_w(c + kRing - 1, w_new);
-      if (u == 1)
-        put_x(x, fill);
-      if (u == 2)
-        fetch_x(c + kRing + 1, x_new);
+      // the chunk's loads evenly between its products, weights first
+#pragma unroll
+      for (int i = u * kFetches / (4 * L); i < (u + 1) * kFetches / (4 * L); ++i) {
+        if (i < 2 * GP)
+          w_new[i % GP * 2 + i / GP] = wp[i % GP][wc + i / GP * 32];
+        else
+          x_new[i - 2 * GP] = *reinterpret_cast<const v4i32 *>(src[i - 2 * GP] + xc);
+      }
+      if (u >= 1 && u <= L)
+        *reinterpret_cast<v4i32 *>(fill + (u - 1) * 32 * kRowBytes + lds_at) = x[u - 1];
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int g = 0; g < GP; ++g) {
@@ -335,20 +402,65 @@ __device__ __forceinline__ void multiply_tile(const GemmArgs &a) {
   };
   // step c: weights from slot c, new ones into slot c - 1; rows c + 2 go to LDS, new ones
   // into slot c + 1 (all modulo kRing)
-  for (int c0 = 0; c0 < nch; c0 += kRing) {
-#pragma unroll
-    for (int u = 0; u < kRing; ++u)
-      if (c0 + u < nch)
-        step(c0 + u, wr[u], wr[(u + 1) % kRing], wr[(u + kRing - 1) % kRing], xr[(u + 2) % kRing],
-             xr[(u + 1) % kRing]);
+  auto turn = [&](int c0, auto slot) {
+    constexpr int u = slot;
+    step(c0 + u, wr[u], wr[(u + 1) % kRing], wr[(u + kRing - 1) % kRing], xr[(u + 2) % kRing],
+         xr[(u + 1) % kRing]);
+  };
+  using std::integral_constant;
+  int c0 = 0;
+  for (; c0 + kRing <= nch; c0 += kRing) {
+    turn(c0, integral_constant<int, 0>{});
+    turn(c0, integral_constant<int, 1>{});
+    turn(c0, integral_constant<int, 2>{});
+    turn(c0, integral_constant<int, 3>{});
+  }
+  static_assert(kRing == 4, "a round is written out");
+  if (c0 < nch) {
+    turn(c0, integral_constant<int, 0>{});
+    if (c0 + 1 < nch) {
+      turn(c0, integral_constant<int, 1>{});
+      if (c0 + 2 < nch)
+        turn(c0, integral_constant<int, 2>{});
+    }
   }
 
   // ---- epilogue: a lane holds channels 8 q + 4 up + 0..3, q = 0..3, of row `col` of every
   // tile; the wavefront turns 32 rows around in its own part of LDS (free now: every
   // wavefront is past the last barrier of the loop) and writes whole row segments
   float *tile = reinterpret_cast<float *>(lds) + wave * (32 * kTurn);
-  const int n0 = g0 * kTileN;
+  const int n0 = g0 * kTileN; // (PAIR: groups of 16 channels of the result as well)
   constexpr int kQuads = kSpan / 4; // float4 of a row
+  if constexpr (PAIR) {
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+#pragma unroll
+      for (int g = 0; g < GP; ++g)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const int ch = g * 16 + 8 * q + 4 * up;
+          const float *sg = scale_s + wave * kSpan + ch, *su = sg + kScales / 2;
+          float o[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            o[i] = silu_times(acc[g][rb][4 * q + i] * sg[i], acc[g][rb][4 * q + 8 + i] * su[i]);
+          *reinterpret_cast<float4 *>(tile + col * kTurn + ch) = make_float4(o[0], o[1], o[2], o[3]);
+        }
+#pragma unroll
+      for (int i = 0; i < kQuads / 2; ++i) {
+        const int idx = lane + 64 * i, row = idx / kQuads, c4 = idx % kQuads;
+        const float4 o = *reinterpret_cast<const float4 *>(tile + row * kTurn + c4 * 4);
+        const int m = m0 + rb * 32 + row, n = n0 + c4 * 4;
+        if (m >= a.M || n >= a.pair_Kp)
+          continue;
+        // a.N is a multiple of 16: four channels are in the result or in its padding
+        const float v[4] = {o.x, o.y, o.z, o.w}, none[4] = {0.f, 0.f, 0.f, 0.f};
+        store_terms4(n < a.N ? v : none, TERMS, a.pair_out + (size_t)m * a.pair_Kp + n,
+                     (size_t)a.Mp * a.pair_Kp);
+      }
+    }
+    return;
+  }
   const size_t at = ((size_t)(rbk * a.ncols + ctile) * a.slices + slice) * kWaves + wave;
   float *part = a.partial + at * kRows * kSpan;
   const bool vec = (a.ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(a.C) & 15) == 0;
@@ -420,15 +532,15 @@ __device__ __forceinline__ void multiply_tile(const GemmArgs &a) {
 constexpr int row_blocks(int terms, int gp) { return terms == 1 && gp == 2 ? 2 : 1; }
 
 // 128 channels per workgroup, and 256
-template <int TERMS>
+template <int TERMS, bool PAIR>
 __global__ void __launch_bounds__(kWaves *kWave) gemm_w8_bf16_kernel(BH_BF16_LEADING) {
   BH_BF16_TAKE
-  multiply_tile<TERMS, 1, 1>(a);
+  multiply_tile<TERMS, 1, 1, PAIR>(a);
 }
-template <int TERMS>
+template <int TERMS, bool PAIR>
 __global__ void __launch_bounds__(kWaves *kWave) gemm_w8_bf16_wide_kernel(BH_BF16_LEADING) {
   BH_BF16_TAKE
-  multiply_tile<TERMS, row_blocks(TERMS, 2), 2>(a);
+  multiply_tile<TERMS, row_blocks(TERMS, 2), 2, PAIR>(a);
 }
 
 // C (+)= scale[n] * sum over the K slices, in slice order (+ bias); four loads are in flight
@@ -471,6 +583,76 @@ __global__ void __launch_bounds__(256) add_slices_kernel(GemmArgs a) {
       c[r] = b[r] + v[r] * s[r];
 }
 
+// The same, one workgroup per row, which then writes RMSNorm(row) * w as the terms of the next
+// matmul's input.  lds: [Kp2] the row, [Kp2] norm weights.  Everything in memory is asked for
+// ahead of the row's one sum (150 rows of 1536 in five slices: 4.2 + 4.9 us in two launches,
+// 5.1 in this one).
+constexpr int kNormThreads = 512;
+constexpr int kNormColumns = 12288; // 96 KB of LDS
+__global__ void __launch_bounds__(kNormThreads)
+add_slices_norm_kernel(GemmArgs a, const float *__restrict__ norm_w, float inv_n, float eps, int terms,
+                       int Kp2, u16 *__restrict__ out) {
+  __shared__ float red[kNormThreads / 64];
+  extern __shared__ __attribute__((aligned(16))) float xrow[];
+  float *wrow = xrow + Kp2;
+  const int m = blockIdx.x;
+  const size_t stride = (size_t)kWaves * a.tile_rows * a.span;
+  float *c = a.C + (int64_t)m * a.ldc;
+  float ss = 0.f;
+  for (int n = threadIdx.x * 4; n < Kp2; n += kNormThreads * 4) {
+    float s[4], b[4], w[4], v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const bool in = n + r < a.N;
+      s[r] = in ? a.scale[n + r] : 0.f;
+      b[r] = !in ? 0.f : a.accumulate ? c[n + r] : a.bias ? a.bias[n + r] : 0.f;
+      w[r] = in ? norm_w[n + r] : 0.f;
+    }
+    if (n < a.N) {
+      const int tile = m / a.tile_rows * a.ncols + n / (kWaves * a.span), wave = n / a.span % kWaves;
+      const size_t row = ((size_t)tile * a.slices * kWaves + wave) * a.tile_rows + m % a.tile_rows;
+      const float *p = a.partial + row * a.span + n % a.span;
+      for (int sl = 0; sl < a.slices; sl += 4) {
+        float4 q[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          q[u] = *reinterpret_cast<const float4 *>(p + (size_t)min(sl + u, a.slices - 1) * stride);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (sl + u < a.slices) {
+            v[0] += q[u].x;
+            v[1] += q[u].y;
+            v[2] += q[u].z;
+            v[3] += q[u].w;
+          }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      v[r] = n + r < a.N ? b[r] + v[r] * s[r] : 0.f;
+      if (n + r < a.N)
+        c[n + r] = v[r];
+      ss = fmaf(v[r], v[r], ss);
+    }
+    *reinterpret_cast<float4 *>(xrow + n) = make_float4(v[0], v[1], v[2], v[3]);
+    *reinterpret_cast<float4 *>(wrow + n) = make_float4(w[0], w[1], w[2], w[3]);
+  }
+  ss = wave_sum(ss);
+  if ((threadIdx.x & 63) == 0)
+    red[threadIdx.x >> 6] = ss;
+  __syncthreads();
+  float tot = 0.f;
+#pragma unroll
+  for (int i = 0; i < kNormThreads / 64; i += 2)
+    tot += red[i] + red[i + 1];
+  const float rs = 1.0f / sqrtf(tot * inv_n + eps);
+  for (int n = threadIdx.x * 4; n < Kp2; n += kNormThreads * 4) { // the thread's own values
+    const float4 x = *reinterpret_cast<const float4 *>(xrow + n), w = *reinterpret_cast<const float4 *>(wrow + n);
+    const float v[4] = {w.x * (x.x * rs), w.y * (x.y * rs), w.z * (x.z * rs), w.w * (x.w * rs)};
+    store_terms4(v, terms, out + (size_t)m * Kp2 + n, (size_t)a.Mp * Kp2);
+  }
+}
+
 // bf16 staging of the activations: one grow-only device buffer per stream, so
 // that calls on different streams do not share it.  Calls on one stream are
 // ordered, and the buffer is only read by the matmul that follows the
@@ -478,28 +660,13 @@ __global__ void __launch_bounds__(256) add_slices_kernel(GemmArgs a) {
 struct Staging {
   u16 *ptr = nullptr;
   size_t bytes = 0;
-  // what the buffer holds
-  const float *src = nullptr;
-  int64_t lda = 0;
-  int M = 0, K = 0, terms = 0;
 };
 std::mutex g_staging_mutex;
 std::map<hipStream_t, Staging> g_staging;
 
-// what the staged copy holds: bf16 terms (1..3) or digit planes (16 + digits)
-int precision_key(const GemmW8Args &in) { return in.digits ? 16 + in.digits : in.terms; }
-
-int staging_for(hipStream_t stream, size_t bytes, const GemmW8Args &in, u16 **out,
-                bool *holds_input) {
+int staging_for(hipStream_t stream, size_t bytes, u16 **out) {
   std::lock_guard<std::mutex> lock(g_staging_mutex);
   Staging &s = g_staging[stream];
-  *holds_input = in.reuse_staged_a && s.ptr && s.src == in.A && s.lda == in.lda &&
-                 s.M == (int)in.M && s.K == (int)in.K && s.terms == precision_key(in);
-  s.src = in.A;
-  s.lda = in.lda;
-  s.M = (int)in.M;
-  s.K = (int)in.K;
-  s.terms = precision_key(in);
   if (s.bytes < bytes) {
     if (s.ptr) {
       BH_CHECK_HIP(hipStreamSynchronize(stream)); // an earlier matmul may still read it
@@ -516,6 +683,7 @@ int staging_for(hipStream_t stream, size_t bytes, const GemmW8Args &in, u16 **ou
 
 BH_VARIANT_FAMILY(WideFamily, "gemm_w8_bf16_wide_kernel");
 BH_VARIANT_FAMILY(NarrowFamily, "gemm_w8_bf16_kernel");
+BH_TILE_FAMILY(PairFamily, "gemm_w8_bf16_kernel pair"); // terms, channel tiles per wavefront
 
 template <class Kernel>
 int launch_tiles(Kernel kernel, const GemmArgs &a, unsigned blocks, hipStream_t stream) {
@@ -542,12 +710,15 @@ struct TilePlan {
   int gp = 0, slices = 1;
   double us = 0;
 };
-TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, int terms, bool may_split) {
+// A norm of the finished rows is a launch of its own, 5 us, unless the kernel that adds the
+// slices does it.
+TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, int terms, bool may_split, bool pair,
+                    double norm_us, double split_norm_us) {
   TilePlan best;
   for (int gp = 1; gp <= 2; ++gp) {
     const int layers = terms * row_blocks(terms, gp);
     const int64_t rows = ceil_div(M, 32 * row_blocks(terms, gp));
-    const int64_t ncols = ceil_div(channels, kWaves * 32 * gp);
+    const int64_t ncols = ceil_div(channels, kWaves * (pair ? 16 : 32) * gp);
     const double alone = gp == 2 ? 0.34 + 0.16 * layers : 0.20 + 0.075 * layers;
     const double full = gp == 2 ? 0.14 + 0.38 * layers : 0.24 + 0.21 * layers;
     for (int s = 1; s <= (may_split ? 16 : 1); ++s) {
@@ -564,7 +735,9 @@ TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, int terms, bool may
       double us = (double)(per_xcd / 64) * full_us +
                   (left == 0 ? 0.0 : 2 * left <= 64 ? alone_us : full_us);
       if (s > 1) // the kernel that adds the slices: 4 us and its bytes
-        us += 4.0 + 4.0 * (double)(M * s) * (double)(ncols * 128 * gp) / 5e6;
+        us += 4.0 + 4.0 * (double)(M * s) * (double)(ncols * 128 * gp) / 5e6 + split_norm_us;
+      else
+        us += norm_us;
       if (!best.gp || us < best.us - 1e-9)
         best = {gp, s, us};
     }
@@ -572,10 +745,31 @@ TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, int terms, bool may
   return best;
 }
 
-int launch_plan(const TilePlan &plan, GemmArgs &a, int terms, hipStream_t stream) {
+template <int GP, bool PAIR>
+int launch_width(const GemmArgs &a, int terms, unsigned blocks, hipStream_t stream) {
+  auto run = [&](auto t) {
+    constexpr int T = t;
+    if constexpr (PAIR)
+      BH_NOTE_VARIANT(PairFamily, T, GP);
+    else if constexpr (GP == 1)
+      BH_NOTE_VARIANT(NarrowFamily, T);
+    else
+      BH_NOTE_VARIANT(WideFamily, T);
+    if constexpr (GP == 1)
+      return launch_tiles(gemm_w8_bf16_kernel<T, PAIR>, a, blocks, stream);
+    else
+      return launch_tiles(gemm_w8_bf16_wide_kernel<T, PAIR>, a, blocks, stream);
+  };
+  return terms == 1 ? run(std::integral_constant<int, 1>{}) : run(std::integral_constant<int, 3>{});
+}
+
+int launch_plan(const TilePlan &plan, GemmArgs &a, const GemmW8Args &in, hipStream_t stream) {
+  const int terms = in.terms;
+  const GemmStagingLayout next = gemm_staging_layout(in.M, in.N);
+  const bool fuses = next.cols_padded <= kNormColumns;
   a.tile_rows = 32 * row_blocks(terms, plan.gp);
   a.span = 32 * plan.gp;
-  a.ncols = (int)ceil_div(a.N, kWaves * a.span);
+  a.ncols = (int)ceil_div(a.N, kWaves * (a.pair_out ? a.span / 2 : a.span));
   a.row_tiles = (int)ceil_div(a.M, a.tile_rows);
   a.slices = plan.slices;
   a.chunks_per_slice = (int)ceil_div(a.chunks, plan.slices);
@@ -587,7 +781,7 @@ int launch_plan(const TilePlan &plan, GemmArgs &a, int terms, hipStream_t stream
             stream, sizeof(float) * tile_floats * a.slices * (size_t)a.ncols * a.row_tiles, &ws))
       return rc;
     if (!ws) // under capture: K whole
-      return launch_plan(plan_tiles(a.M, a.N, a.chunks, terms, false), a, terms, stream);
+      return launch_plan(plan_tiles(a.M, a.N, a.chunks, terms, false, false, 0.0, 0.0), a, in, stream);
     a.partial = reinterpret_cast<float *>(ws);
   }
   const int64_t units = (int64_t)a.ncols * a.slices;
@@ -596,28 +790,35 @@ int launch_plan(const TilePlan &plan, GemmArgs &a, int terms, hipStream_t stream
   BH_REQUIRE(tiles < (1u << 31), "gemm_w8: %lld tiles", (long long)tiles);
   const unsigned blocks = (unsigned)tiles;
   int rc;
-  if (plan.gp == 1) {
-    if (terms == 1) {
-      BH_NOTE_VARIANT(NarrowFamily, 1);
-      rc = launch_tiles(gemm_w8_bf16_kernel<1>, a, blocks, stream);
-    } else {
-      BH_NOTE_VARIANT(NarrowFamily, 3);
-      rc = launch_tiles(gemm_w8_bf16_kernel<3>, a, blocks, stream);
-    }
-  } else if (terms == 1) {
-    BH_NOTE_VARIANT(WideFamily, 1);
-    rc = launch_tiles(gemm_w8_bf16_wide_kernel<1>, a, blocks, stream);
-  } else {
-    BH_NOTE_VARIANT(WideFamily, 3);
-    rc = launch_tiles(gemm_w8_bf16_wide_kernel<3>, a, blocks, stream);
-  }
-  if (rc || a.slices == 1)
+  if (a.pair_out)
+    return plan.gp == 1 ? launch_width<1, true>(a, terms, blocks, stream)
+                        : launch_width<2, true>(a, terms, blocks, stream);
+  rc = plan.gp == 1 ? launch_width<1, false>(a, terms, blocks, stream)
+                    : launch_width<2, false>(a, terms, blocks, stream);
+  if (rc)
     return rc;
-  const int64_t threads = (int64_t)a.M * ceil_div(a.N, 4);
-  hipLaunchKernelGGL(add_slices_kernel, dim3((unsigned)ceil_div(threads, 256)), dim3(256), 0,
-                     stream, a);
-  BH_CHECK_HIP(hipGetLastError());
-  return BUDDY_HIP_OK;
+  u16 *normed = static_cast<u16 *>(in.then_norm_staged);
+  if (a.slices > 1 && in.then_norm_w && fuses) {
+    const size_t lds = 2 * sizeof(float) * (size_t)next.cols_padded;
+    if (lds > 48 * 1024) {
+      static DynLdsOnce once;
+      BH_CHECK_HIP(ensure_dyn_lds(once, reinterpret_cast<const void *>(add_slices_norm_kernel),
+                                  (int)(2 * sizeof(float) * kNormColumns)));
+    }
+    hipLaunchKernelGGL(add_slices_norm_kernel, dim3((unsigned)a.M), dim3(kNormThreads), lds, stream, a,
+                       in.then_norm_w, 1.0f / (float)a.N, in.then_norm_eps, terms, next.cols_padded, normed);
+    BH_CHECK_HIP(hipGetLastError());
+    return BUDDY_HIP_OK;
+  }
+  if (a.slices > 1) {
+    const int64_t threads = (int64_t)a.M * ceil_div(a.N, 4);
+    hipLaunchKernelGGL(add_slices_kernel, dim3((unsigned)ceil_div(threads, 256)), dim3(256), 0,
+                       stream, a);
+    BH_CHECK_HIP(hipGetLastError());
+  }
+  return in.then_norm_w ? launch_rmsnorm_to_staging(a.C, in.then_norm_w, a.M, a.N, in.then_norm_eps, terms,
+                                                    normed, stream)
+                        : BUDDY_HIP_OK;
 }
 
 } // namespace
@@ -640,6 +841,17 @@ int launch_rmsnorm_to_staging(const float *x, const float *w, int rows, int n, f
   return BUDDY_HIP_OK;
 }
 
+int launch_attn_fold_to_terms(const PromptFold &fold, int64_t o_stride, int heads, int tokens, int terms,
+                              unsigned short *staged, hipStream_t stream) {
+  const int64_t K = (int64_t)heads * kPromptD;
+  BH_REQUIRE(fold.blocks && staged && tokens > 0 && terms >= 1 && terms <= 3, "attn_fold_to_terms: bad argument");
+  const GemmStagingLayout l = gemm_staging_layout(tokens, K); // K is a multiple of 64: no padding
+  hipLaunchKernelGGL(attn_fold_to_terms_kernel, dim3(tokens), dim3(512), 0, stream, fold, o_stride, (int)K,
+                     terms, l.rows_padded, staged);
+  BH_CHECK_HIP(hipGetLastError());
+  return BUDDY_HIP_OK;
+}
+
 int launch_silu_mul_to_staging(const float *g, const float *u, int64_t ld, int rows, int n, int terms,
                                unsigned short *staged, hipStream_t stream) {
   BH_REQUIRE(g && u && staged && rows > 0 && n > 0 && terms >= 1 && terms <= 3,
@@ -654,16 +866,20 @@ int launch_silu_mul_to_staging(const float *g, const float *u, int64_t ld, int r
 }
 
 int launch_gemm_w8(const GemmW8Args &in, hipStream_t stream) {
-  BH_REQUIRE((in.A || in.staged) && in.W && in.scale && in.C, "gemm_w8: null pointer");
+  BH_REQUIRE((in.A || in.staged) && in.W && in.scale && (in.C || (in.silu_staged && !in.digits)),
+             "gemm_w8: null pointer");
   BH_REQUIRE(in.M > 0 && in.K > 0 && in.N > 0 && in.M < (1 << 24) &&
                  in.K < (1 << 24) && in.N < (1 << 24),
              "gemm_w8: bad shape M=%lld K=%lld N=%lld", (long long)in.M,
              (long long)in.K, (long long)in.N);
-  BH_REQUIRE((in.staged || in.lda >= in.K) && in.ldc >= (in.silu_pair ? in.N / 2 : in.N),
+  BH_REQUIRE((in.staged || in.lda >= in.K) && (!in.C || in.ldc >= (in.silu_pair ? in.N / 2 : in.N)),
              "gemm_w8: row stride below row length");
-  BH_REQUIRE(!in.silu_pair || in.digits, "gemm_w8: the SiLU pair runs on digit planes only");
-  BH_REQUIRE(!in.then_norm_w || (in.digits && in.then_norm_staged),
-             "gemm_w8: a following norm needs digit planes and a buffer for them");
+  BH_REQUIRE(!in.silu_pair || in.digits || (in.silu_staged && in.staged && in.N % (2 * kTileN) == 0 && !in.bias &&
+                                            !in.accumulate && !in.then_norm_w),
+             "gemm_w8: the SiLU pair of bfloat16 terms needs staged rows, two matrices of a multiple of 16 "
+             "channels and a buffer for its terms");
+  BH_REQUIRE(!in.then_norm_w || (in.then_norm_staged && (in.digits || in.ldc == in.N)),
+             "gemm_w8: a following norm needs a buffer for its rows");
   // one bf16 term (activations cast to bf16) or three (every f32 bit); three
   // digit planes (23 bits below the row's maximum) or two (15 bits: the fixed
   // point counterpart of the bf16 cast, for the same third less matrix work)
@@ -691,10 +907,10 @@ int launch_gemm_w8(const GemmW8Args &in, hipStream_t stream) {
   a.Kp = layout.cols_padded;
   a.accumulate = in.accumulate ? 1 : 0;
   u16 *abf = static_cast<u16 *>(const_cast<void *>(in.staged));
-  bool staged = in.staged != nullptr;
+  const bool staged = in.staged != nullptr;
   const size_t staging_bytes =
       in.digits ? layout.bytes_digits(in.digits) : layout.bytes(in.terms);
-  int rc = staged ? BUDDY_HIP_OK : staging_for(stream, staging_bytes, in, &abf, &staged);
+  int rc = staged ? BUDDY_HIP_OK : staging_for(stream, staging_bytes, &abf);
   if (rc)
     return rc;
   if (in.digits) {
@@ -711,7 +927,17 @@ int launch_gemm_w8(const GemmW8Args &in, hipStream_t stream) {
                        in.terms, abf);
     BH_CHECK_HIP(hipGetLastError());
   }
-  return launch_plan(plan_tiles(in.M, in.N, a.chunks, in.terms, true), a, in.terms, stream);
+  a.pair_out = nullptr;
+  if (in.silu_pair) {
+    a.N = (int)(in.N / 2);
+    a.pair_out = static_cast<u16 *>(in.silu_staged);
+    a.pair_Kp = gemm_staging_layout(in.M, a.N).cols_padded;
+    return launch_plan(plan_tiles(in.M, a.N, a.chunks, in.terms, false, true, 0.0, 0.0), a, in, stream);
+  }
+  const double norm_us = in.then_norm_w ? 5.0 : 0.0;
+  const bool fuses = gemm_staging_layout(in.M, in.N).cols_padded <= kNormColumns;
+  return launch_plan(plan_tiles(in.M, in.N, a.chunks, in.terms, true, false, norm_us, fuses ? 0.0 : norm_us),
+                     a, in, stream);
 }
 
 void release_gemm_staging(hipStream_t stream) {

@@ -108,7 +108,7 @@ struct Qwen2Session : Session {
   size_t kv_rows_cap = 0;
   unsigned short *pf_xn_bf = nullptr, *pf_g_bf = nullptr; // bf16 matmul inputs
   void *pf_attn_ws = nullptr;          // partial results of the attention
-  unsigned short *pf_att_dg = nullptr; // digit planes of the attention output (o_proj's input)
+  unsigned short *pf_att_dg = nullptr; // digit planes or terms of the attention output (o_proj's input)
   int gemm_terms = 3; // bf16 terms per activation in the prefill matmuls (3 = exact)
   int gemm_digits = 3; // int8 digit planes instead of bf16 terms when not 0
 
@@ -340,14 +340,18 @@ struct Qwen2Session : Session {
                             lg = gemm_staging_layout(rows, S.inter);
     BH_CHECK_HIP(hipMalloc((void **)&pf_xn_bf, std::max(lx.bytes(3), lx.bytes_digits(3))));
     BH_CHECK_HIP(hipMalloc((void **)&pf_g_bf, std::max(lg.bytes(3), lg.bytes_digits(3))));
-    BH_CHECK_HIP(hipMalloc((void **)&pf_att_dg, gemm_staging_layout(rows, QN).bytes_digits(3)));
+    const GemmStagingLayout la = gemm_staging_layout(rows, QN);
+    BH_CHECK_HIP(hipMalloc((void **)&pf_att_dg, std::max(la.bytes(3), la.bytes_digits(3))));
     pf_rows = rows;
     return BUDDY_HIP_OK;
   }
 
   int gemm(const float *A, const PackedLinear &W, float *C, int64_t M, bool accumulate,
-           bool same_input_as_before = false) {
+           const float *then_norm_w = nullptr, void *then_norm_staged = nullptr) {
     GemmW8Args g;
+    g.then_norm_w = then_norm_w;
+    g.then_norm_eps = shape.rms_eps;
+    g.then_norm_staged = then_norm_staged;
     g.A = A;
     g.lda = W.K;
     g.W = W.w;
@@ -361,7 +365,6 @@ struct Qwen2Session : Session {
     g.accumulate = accumulate;
     g.terms = gemm_terms;
     g.digits = gemm_digits;
-    g.reuse_staged_a = same_input_as_before;
     return launch_gemm_w8(g, stream);
   }
   // the same with the input already staged as bf16 terms
@@ -415,7 +418,7 @@ struct Qwen2Session : Session {
                        pf_tokens, (int64_t)S.hidden, (int64_t)S.vocab, pf_x);
     BH_CHECK_HIP(hipGetLastError());
     int rc;
-    const bool folded = attn_prompt_pays(n, start_pos, S.heads, S.kv_heads, gemm_digits != 0);
+    const bool folded = attn_prompt_pays(n, start_pos, S.heads, S.kv_heads);
     if (folded && !pf_attn_ws) // for as many rows as the other buffers have, behind any context
       BH_CHECK_HIP(hipMalloc(&pf_attn_ws, attn_prompt_workspace_bytes(pf_rows, S.max_len, S.heads, S.kv_heads)));
     bool normed_ahead = false; // pf_xn_bf already holds this layer's normed input
@@ -474,18 +477,21 @@ struct Qwen2Session : Session {
                               true, 0, L.ln2, pf_xn_bf)))
           return rc;
       } else {
-        if (folded && (rc = launch_attn_fold_rows(fold, pf_att, a.o_stride, S.heads, n, stream)))
+        // likewise with bf16 terms
+        if (folded && (rc = launch_attn_fold_to_terms(fold, a.o_stride, S.heads, n, gemm_terms, pf_att_dg,
+                                                      stream)))
           return rc;
-        if ((rc = gemm(pf_att, L.o, pf_x, n, true)))
-          return rc;
-        if ((rc = norm_to_staging(pf_x, L.ln2, n, pf_xn_bf)))
+        if ((rc = folded ? gemm_staged(pf_att_dg, L.o, pf_x, n, true, 0, L.ln2, pf_xn_bf)
+                         : gemm(pf_att, L.o, pf_x, n, true, L.ln2, pf_xn_bf)))
           return rc;
       }
       const int64_t ld_gu = 2 * (int64_t)S.inter;
-      if (L.gate_up_joint && gemm_digits) {
+      const Layer *nx = i + 1 < S.layers ? &layers[(size_t)i + 1] : nullptr;
+      const bool ahead = nx && !nx->qkv_f32;
+      if (L.gate_up_joint) {
         // gate and up in one launch whose workgroups hold matching tiles of
-        // both: SiLU(gate) * up leaves the matmul, and one pass turns it into
-        // the digit planes of down's input
+        // both: SiLU(gate) * up leaves the matmul as the terms of down's input, or, since
+        // digit planes need whole rows, in f32, and one pass turns it into those
         GemmW8Args g;
         g.staged = pf_xn_bf;
         g.W = L.gate.w;
@@ -495,35 +501,26 @@ struct Qwen2Session : Session {
         g.M = n;
         g.K = L.gate.K;
         g.N = 2 * L.gate.N;
+        g.terms = gemm_terms;
         g.digits = gemm_digits;
         g.silu_pair = true;
+        g.silu_staged = pf_g_bf;
         if ((rc = launch_gemm_w8(g, stream)))
           return rc;
-        if ((rc = launch_activations_to_digits(pf_g, S.inter, n, S.inter, gemm_digits, pf_g_bf,
+        if (gemm_digits && (rc = launch_activations_to_digits(pf_g, S.inter, n, S.inter, gemm_digits, pf_g_bf,
                                                stream)))
           return rc;
         // down's finished rows go on as the next layer's normed q|k|v input
-        const Layer *nx = i + 1 < S.layers ? &layers[(size_t)i + 1] : nullptr;
-        const bool ahead = nx && !nx->qkv_f32;
         if ((rc = gemm_staged(pf_g_bf, L.down, pf_x, n, true, 0, ahead ? nx->ln1 : nullptr,
                               ahead ? pf_xn_bf : nullptr)))
           return rc;
         normed_ahead = ahead;
         continue;
       }
-      if (L.gate_up_joint) {
-        // gate | up as one matrix of 2 * inter channels: one launch, whose second
-        // round of tiles starts while the first one drains
-        PackedLinear both = L.gate;
-        both.N = 2 * L.gate.N;
-        if ((rc = gemm_staged(pf_xn_bf, both, pf_g, n, false, ld_gu)))
-          return rc;
-      } else {
-        if ((rc = gemm_staged(pf_xn_bf, L.gate, pf_g, n, false, ld_gu)))
-          return rc;
-        if ((rc = gemm_staged(pf_xn_bf, L.up, pf_u, n, false, ld_gu)))
-          return rc;
-      }
+      if ((rc = gemm_staged(pf_xn_bf, L.gate, pf_g, n, false, ld_gu)))
+        return rc;
+      if ((rc = gemm_staged(pf_xn_bf, L.up, pf_u, n, false, ld_gu)))
+        return rc;
       if ((rc = silu_mul_to_staging(pf_g, pf_u, n, pf_g_bf)))
         return rc;
       if ((rc = gemm_staged(pf_g_bf, L.down, pf_x, n, true)))

@@ -501,6 +501,38 @@ def test_which_prompt_attention(bh, heads, kv_heads, before, n, precision, split
     sess.close()
 
 
+# bfloat16 modes: gate and up as one product whose result leaves as terms, on tiles of one and of
+# two channel tiles per wavefront, a result that ends inside 64 channels; the norm behind o and down
+# in the kernel that adds slices of K and as a launch of its own; the attention's fold as terms
+@pytest.mark.parametrize("precision", ["bf16", "exact"])
+@pytest.mark.parametrize("hidden,inter,before,n,gp", [
+    (256, 272, 0, 5, 1), (256, 1040, 0, 33, 1), (256, 8976, 0, 65, 0), (256, 8976, 0, 150, 2),
+    (1536, 8960, 0, 300, 2), (1536, 48, 600, 40, 1), (320, 4112, 600, 70, 0)])
+def test_prompt_layers_in_bf16_terms(bh, hidden, inter, before, n, gp, precision):
+    shape = Shape(layers=2, hidden=hidden, heads=6, kv_heads=1, head_dim=128, inter=inter, vocab=320,
+                  max_len=before + n + 8)
+    toks = synthetic.first_tokens(shape, n, seed=n + inter).astype(np.int32)
+    sess, _ = synthetic.build_session(shape, context=before, ln_jitter=0.1)
+    bh.buddy_hip_variant_reset()
+    _, got = sess.prefill(toks, before, precision=precision)
+    ran = {k for k, v in tiles_run(bh).items() if v and k.startswith("gemm_w8_bf16_kernel pair")}
+    terms = 1 if precision == "bf16" else 3
+    assert len(ran) == 1 and (gp == 0 or ran == {f"gemm_w8_bf16_kernel pair<{terms}, {gp}>"}), ran
+    rows = [sess.get_kv(j)[:, before:before + n] for j in (2, 3)]
+    sess.close()
+    sess, _ = synthetic.build_session(shape, context=before, ln_jitter=0.1)
+    for i, t in enumerate(toks):
+        _, want = sess.decode(int(t), before + i, want_logits=i + 1 == n)
+    pairs = [(got, want)] + [(rows[j - 2], sess.get_kv(j)[:, before:before + n]) for j in (2, 3)]
+    sess.close()
+    for g, w in pairs:
+        if precision == "exact":
+            check_close(g, w)
+        else:  # 2^-9 per activation, some ten roundings on the way
+            g, w = np.asarray(g, np.float64), np.asarray(w, np.float64)
+            assert np.linalg.norm(g - w) < 10 * 2.0**-9 * np.linalg.norm(w)
+
+
 def test_workspace_of_the_prompt_attention_follows_the_session(bh):
     """One KV head behind 640 positions has 20 tiles of keys for 20 workgroups: 5 MB of partial
     results, not the 67 MB of a full chip."""
