@@ -696,16 +696,13 @@ int launch_tiles(Kernel kernel, const GemmArgs &a, unsigned blocks, hipStream_t 
 // Channel tiles per wavefront and K slices for a launch, by an estimate of its time in
 // microseconds.  An XCD (32 compute units) works on 64 workgroups at a time, two to a compute
 // unit.  A chunk of 64 k on L layers of 32 rows (terms, blocks of rows) takes a compute unit
-// with two workgroups 0.14 + 0.38 L us, one that has its compute unit to itself 0.34 + 0.16 L
-// us (with one channel tile 0.24 + 0.21 L and 0.2 + 0.075 L); a last round that fills less
-// than half runs at the latter.  Fitted to these, microseconds (one term; three; in brackets
-// 16 x 16 x 32 products, on tiles of 64 x 64 whose wavefronts split K or of 48 or 64 rows x
-// 256 channels):
-//   8960 -> 1536, with the adding of its slices: 17 rows 11 [38]; 16 [97], 150: 17 [41]; 31
-//     [98], 1024: 46 [78]; 94 [200], 1931: 84 [119]; 168 [307]
-//   1536 -> 17920: 17 rows 12 [18]; 16 [42], 150: 23 [29]; 34 [51], 512: 45 [62]; 85 [147],
-//     1931: 127 [175]; 300 [433]
-//   1536 -> 2048: 150 rows 11.2 [11.5]; 14.8 [21.6], 1024: 15.6 [19.3]; 26 [44]
+// with two workgroups 0.20 + 0.38 L us, one that has its compute unit to itself 0.29 + 0.14 L
+// us (with one channel tile 0.20 + 0.185 L and 0.17 + 0.073 L); a last round that fills less
+// than half runs at the latter.  Fitted to launches of 20 to 1931 rows of 1536, 4096, 8960 and
+// 14336 k, both tiles with every K split: what it picks is 2.2 % off the best on average.
+// Microseconds of a product in a prompt of 150 rows, one term (in brackets with a branch at every
+// chunk and its loads at the chunk's start): 1536 -> 2048 10.9 [14.1], 1536 -> 2 x 8960 19.9
+// [22.9], 8960 -> 1536 11.6 [13.0] without the adding of its slices.
 struct TilePlan {
   int gp = 0, slices = 1;
   double us = 0;
@@ -719,8 +716,8 @@ TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, int terms, bool may
     const int layers = terms * row_blocks(terms, gp);
     const int64_t rows = ceil_div(M, 32 * row_blocks(terms, gp));
     const int64_t ncols = ceil_div(channels, kWaves * (pair ? 16 : 32) * gp);
-    const double alone = gp == 2 ? 0.34 + 0.16 * layers : 0.20 + 0.075 * layers;
-    const double full = gp == 2 ? 0.14 + 0.38 * layers : 0.24 + 0.21 * layers;
+    const double alone = gp == 2 ? 0.291 + 0.141 * layers : 0.172 + 0.073 * layers;
+    const double full = gp == 2 ? 0.203 + 0.38 * layers : 0.20 + 0.185 * layers;
     for (int s = 1; s <= (may_split ? 16 : 1); ++s) {
       const int64_t per_xcd = ceil_div(ncols * s * rows, 8);
       if (s > 1 && per_xcd > 256)
@@ -729,8 +726,8 @@ TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, int terms, bool may
       if (ceil_div(chunks, cps) != s)
         continue; // the last slice would be empty
       const double store = s > 1 ? 2.0 : 0.0; // of the partial sums
-      const double full_us = full * (double)cps + 4.0 + store;
-      const double alone_us = alone * (double)cps + 5.0 + store;
+      const double full_us = full * (double)cps + 5.95 + store;
+      const double alone_us = alone * (double)cps + 4.15 + store;
       const int64_t left = per_xcd % 64;
       double us = (double)(per_xcd / 64) * full_us +
                   (left == 0 ? 0.0 : 2 * left <= 64 ? alone_us : full_us);
