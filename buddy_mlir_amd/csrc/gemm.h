@@ -5,6 +5,14 @@
 
 namespace bh {
 
+// What follows a product that is q | k | v of heads of 128: q rotated in place, k rotated into
+// the cache, v copied there (launch_rope_kv_write).
+struct RopeKv {
+  const float *inv_freq = nullptr; // [64]
+  float *kcache = nullptr, *vcache = nullptr;
+  int heads = 0, kv_heads = 0, max_len = 0, start_pos = 0;
+};
+
 struct GemmW8Args {
   const float *A = nullptr; // [M, K], row stride lda
   int64_t lda = 0;
@@ -32,6 +40,9 @@ struct GemmW8Args {
   const float *then_norm_w = nullptr;
   float then_norm_eps = 0.f;
   void *then_norm_staged = nullptr;
+  // digits only: C is q | k | v, and what follows it is done too, by the kernel that adds the
+  // K slices where there is one, else by a launch of its own (ldc == N, no accumulation)
+  const RopeKv *then_rope = nullptr;
   // Caller-provided staging of A (written by one of the producers below for
   // exactly this M, K and terms / digits): no conversion, A itself is not read.
   const void *staged = nullptr;

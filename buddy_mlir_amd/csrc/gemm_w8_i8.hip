@@ -30,6 +30,7 @@
 //
 // Workgroups take 32 rows x 128 or 256 channels, or one of the other tiles of kTiles1 to
 // kTiles3, with the activation fragments shared through LDS.
+#include "attn.h"
 #include "attn_fold.h"
 #include "gemm.h"
 #include "tile_place.h"
@@ -801,6 +802,88 @@ reduce_slices_kernel(GemmI8Args a) {
     }
 }
 
+// The same where C is q | k | v and what follows it is the rotation and the cache rows: a
+// thread has four channels of a q or k head and their partners 64 further on, or four of v.
+// Its angles are worked out while its loads are on their way (27 rows of 2048 channels: 4.7 us
+// and 3.4 in a launch behind it, 5.4 in this one; prompts of 3 to 100 tokens 2 to 5 % shorter).
+// Small workgroups: a short prompt's few loads then come in through many compute units.
+constexpr int kRopeThreads = 64;
+__global__ void __launch_bounds__(kRopeThreads)
+reduce_slices_rope_kernel(GemmI8Args a, RopeKv r) {
+  constexpr int kHalf = kAttnHeadDim / 2;
+  const int turned = (r.heads + r.kv_heads) * (kHalf / 4), per_row = turned + r.kv_heads * (kAttnHeadDim / 4);
+  const int64_t i = (int64_t)blockIdx.x * kRopeThreads + threadIdx.x;
+  if (i >= (int64_t)a.M * per_row)
+    return;
+  const int m = (int)(i / per_row), t = (int)(i % per_row), pos = r.start_pos + m;
+  const size_t slice_stride = (size_t)kSlices * a.tile_rows * a.span;
+  const float step = a.steps[m];
+  float *row = a.C + (int64_t)m * a.ldc;
+  // a quad's first eight slices and its operands
+  struct Quad {
+    float4 q[8];
+    FinishOperands f;
+    const float *p;
+  };
+  auto request = [&](int n, Quad &x) {
+    x.p = first_slice(a, m, n);
+    x.f = load_finish_operands(a, row + n, n);
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      x.q[u] = *reinterpret_cast<const float4 *>(x.p + (size_t)min(u, a.slices - 1) * slice_stride);
+  };
+  auto finish = [&](Quad &x, float (&v)[4]) {
+    v[0] = v[1] = v[2] = v[3] = 0.f;
+    for (int sl = 0;;) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (sl + u < a.slices) {
+          v[0] += x.q[u].x; v[1] += x.q[u].y; v[2] += x.q[u].z; v[3] += x.q[u].w;
+        }
+      sl += 8;
+      if (sl >= a.slices)
+        break;
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        x.q[u] = *reinterpret_cast<const float4 *>(x.p + (size_t)min(sl + u, a.slices - 1) * slice_stride);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      v[e] = x.f.bias[e] + (v[e] * step) * x.f.scale[e];
+  };
+  if (t >= turned) { // v
+    const int at = (t - turned) * 4, head = at / kAttnHeadDim, d = at % kAttnHeadDim;
+    Quad x;
+    request((r.heads + r.kv_heads) * kAttnHeadDim + at, x);
+    float v[4];
+    finish(x, v);
+    *reinterpret_cast<float4 *>(r.vcache + ((int64_t)head * r.max_len + pos) * kAttnHeadDim + d) =
+        make_float4(v[0], v[1], v[2], v[3]);
+    return;
+  }
+  const int head = t / (kHalf / 4), j = t % (kHalf / 4) * 4, n = head * kAttnHeadDim + j;
+  Quad x, y;
+  request(n, x);
+  request(n + kHalf, y);
+  float s[4], c[4], lo[4], hi[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    sincosf(r.inv_freq[j + e] * (float)pos, &s[e], &c[e]);
+  finish(x, lo);
+  finish(y, hi);
+  float4 nlo, nhi;
+  float *l4 = &nlo.x, *h4 = &nhi.x;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    l4[e] = lo[e] * c[e] + (-hi[e]) * s[e];
+    h4[e] = hi[e] * c[e] + lo[e] * s[e];
+  }
+  float *dst = head < r.heads ? row + n
+                              : r.kcache + ((int64_t)(head - r.heads) * r.max_len + pos) * kAttnHeadDim + j;
+  *reinterpret_cast<float4 *>(dst) = nlo;
+  *reinterpret_cast<float4 *>(dst + kHalf) = nhi;
+}
+
 // One plane (the w8a8 matmul): the slices hold int32 sums, added exactly; then
 // C = f32(sum) * (step * scale[n]) in that order (linalg.py:12833-12845), and the
 // sums themselves where the caller asked for them.
@@ -1239,11 +1322,17 @@ int launch_gemm_w8_digits_d(const GemmW8Args &in, const void *planes, hipStream_
   // 5 us, unless the kernel that adds K slices writes its planes (it holds whole
   // rows, up to kRowCache columns).
   const bool slices_fuse_norm = gemm_staging_layout(in.M, in.N).cols_padded <= kRowCache;
-  const double norm_us = in.then_norm_w ? 5.0 : 0.0;
-  const double split_norm_us = slices_fuse_norm ? 0.0 : norm_us;
+  // The rotation behind q | k | v likewise: 4 us.
+  const double norm_us = in.then_norm_w ? 5.0 : in.then_rope ? 4.0 : 0.0;
+  const double split_norm_us = in.then_rope ? 0.5 : slices_fuse_norm ? 0.0 : norm_us;
   // the RMSNorm of the finished rows into digit planes, where the caller asked
   // for it and no kernel of the matmul holds whole rows
   auto then_norm = [&]() -> int {
+    if (in.then_rope) {
+      const RopeKv &r = *in.then_rope;
+      return launch_rope_kv_write(in.C, in.ldc, r.inv_freq, r.kcache, r.vcache, r.heads, r.kv_heads,
+                                  kAttnHeadDim, r.max_len, r.start_pos, (int)in.M, stream);
+    }
     if (!in.then_norm_w)
       return BUDDY_HIP_OK;
     return launch_rmsnorm_to_digits(in.C, in.ldc, in.then_norm_w, (int)in.M, (int)in.N,
@@ -1274,6 +1363,14 @@ int launch_gemm_w8_digits_d(const GemmW8Args &in, const void *planes, hipStream_
                        a.tile_rows, a, in.then_norm_w, 1.0f / (float)in.N, in.then_norm_eps,
                        in.digits, next.rows_padded, next.cols_padded,
                        static_cast<int8_t *>(in.then_norm_staged));
+    BH_CHECK_HIP(hipGetLastError());
+    return BUDDY_HIP_OK;
+  }
+  if (in.then_rope) {
+    const RopeKv &r = *in.then_rope;
+    const int64_t quads = (int64_t)a.M * (r.heads + 3 * r.kv_heads) * (kAttnHeadDim / 8);
+    hipLaunchKernelGGL(reduce_slices_rope_kernel, dim3((unsigned)ceil_div(quads, kRopeThreads)),
+                       dim3(kRopeThreads), 0, stream, a, r);
     BH_CHECK_HIP(hipGetLastError());
     return BUDDY_HIP_OK;
   }

@@ -21,6 +21,7 @@
 //    on the same XCD and share the weight tiles in its L2 (tile_place.h);
 //  * the per-channel scale is applied once to the f32 accumulators, where the
 //    reference multiplies every element before the FMA.
+#include "attn.h"
 #include "attn_fold.h"
 #include "gemm.h"
 #include "tile_place.h"
@@ -877,6 +878,16 @@ int launch_gemm_w8(const GemmW8Args &in, hipStream_t stream) {
              "channels and a buffer for its terms");
   BH_REQUIRE(!in.then_norm_w || (in.then_norm_staged && (in.digits || in.ldc == in.N)),
              "gemm_w8: a following norm needs a buffer for its rows");
+  if (in.then_rope) {
+    const RopeKv &r = *in.then_rope;
+    BH_REQUIRE(in.digits && !in.silu_pair && !in.accumulate && !in.then_norm_w && in.ldc == in.N && r.inv_freq &&
+                   r.kcache && r.vcache && r.heads > 0 && r.kv_heads > 0 &&
+                   in.N == (int64_t)(r.heads + 2 * r.kv_heads) * kAttnHeadDim && r.start_pos >= 0 &&
+                   r.start_pos + in.M <= r.max_len &&
+                   ((reinterpret_cast<uintptr_t>(in.C) | reinterpret_cast<uintptr_t>(r.kcache) |
+                     reinterpret_cast<uintptr_t>(r.vcache)) & 15) == 0,
+               "gemm_w8: q | k | v with what follows it");
+  }
   // one bf16 term (activations cast to bf16) or three (every f32 bit); three
   // digit planes (23 bits below the row's maximum) or two (15 bits: the fixed
   // point counterpart of the bf16 cast, for the same third less matrix work)

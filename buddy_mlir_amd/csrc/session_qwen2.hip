@@ -370,11 +370,12 @@ struct Qwen2Session : Session {
   // the same with the input already staged as bf16 terms
   int gemm_staged(const unsigned short *staged, const PackedLinear &W, float *C, int64_t M,
                   bool accumulate, int64_t ldc = 0, const float *then_norm_w = nullptr,
-                  void *then_norm_staged = nullptr) {
+                  void *then_norm_staged = nullptr, const RopeKv *then_rope = nullptr) {
     GemmW8Args g;
     g.then_norm_w = then_norm_w;
     g.then_norm_eps = shape.rms_eps;
     g.then_norm_staged = then_norm_staged;
+    g.then_rope = then_rope;
     g.staged = staged;
     g.W = W.w;
     g.scale = W.s;
@@ -424,6 +425,7 @@ struct Qwen2Session : Session {
     bool normed_ahead = false; // pf_xn_bf already holds this layer's normed input
     for (int i = 0; i < S.layers; ++i) {
       Layer &L = layers[(size_t)i];
+      bool rotated = false; // the q|k|v matmul has also done what follows it
       if (L.qkv_f32) {
         if ((rc = launch_rmsnorm(pf_x, L.ln1, pf_xn, n, S.hidden, S.rms_eps, stream)))
           return rc;
@@ -438,12 +440,22 @@ struct Qwen2Session : Session {
         if (!normed_ahead && (rc = norm_to_staging(pf_x, L.ln1, n, pf_xn_bf)))
           return rc;
         normed_ahead = false;
-        if ((rc = gemm_staged(pf_xn_bf, L.qkv, pf_qkv, n, false)))
+        RopeKv rope;
+        rope.inv_freq = inv_freq;
+        rope.kcache = L.kc;
+        rope.vcache = L.vc;
+        rope.heads = S.heads;
+        rope.kv_heads = S.kv_heads;
+        rope.max_len = S.max_len;
+        rope.start_pos = start_pos;
+        rotated = gemm_digits != 0;
+        if ((rc = gemm_staged(pf_xn_bf, L.qkv, pf_qkv, n, false, 0, nullptr, nullptr,
+                              rotated ? &rope : nullptr)))
           return rc;
       }
-      if ((rc = launch_rope_kv_write(pf_qkv, QKV, inv_freq, L.kc, L.vc, S.heads,
-                                     S.kv_heads, S.head_dim, S.max_len, start_pos,
-                                     n, stream)))
+      if (!rotated && (rc = launch_rope_kv_write(pf_qkv, QKV, inv_freq, L.kc, L.vc, S.heads,
+                                                 S.kv_heads, S.head_dim, S.max_len, start_pos,
+                                                 n, stream)))
         return rc;
       AttnPrefillArgs a;
       a.q = pf_qkv;

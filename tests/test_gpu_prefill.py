@@ -501,6 +501,31 @@ def test_which_prompt_attention(bh, heads, kv_heads, before, n, precision, split
     sess.close()
 
 
+# q | k | v with the rotation and the cache rows behind it: K in more slices than are asked for at
+# once, in few and in one; one head and many; tokens behind a context
+@pytest.mark.parametrize("precision", ["digits", "digits2"])
+@pytest.mark.parametrize("hidden,heads,kv_heads,before,n", [
+    (2048, 1, 1, 0, 3), (1536, 2, 1, 7, 40), (320, 6, 3, 130, 17), (64, 12, 2, 0, 33), (256, 12, 2, 3, 900)])
+def test_rotation_behind_qkv(hidden, heads, kv_heads, before, n, precision):
+    shape = Shape(layers=2, hidden=hidden, heads=heads, kv_heads=kv_heads, head_dim=128, inter=64, vocab=320,
+                  max_len=before + n + 8)
+    toks = synthetic.first_tokens(shape, n, seed=n).astype(np.int32)
+    sess, _ = synthetic.build_session(shape, context=before, ln_jitter=0.1)
+    sess.prefill(toks, before, precision=precision)
+    rows = [sess.get_kv(j)[:, :before + n] for j in range(4)]
+    sess.close()
+    sess, _ = synthetic.build_session(shape, context=before, ln_jitter=0.1)
+    for i, t in enumerate(toks):
+        sess.decode(int(t), before + i, want_logits=False)
+    for j in range(4):
+        want = sess.get_kv(j)[:, :before + n]
+        if precision == "digits":
+            check_close(rows[j], want)
+        else:  # 2^-15 of a row's largest value, in K and V of the first layer and all ahead of the second
+            assert np.linalg.norm(rows[j] - want) < 2.0**-10 * np.linalg.norm(want)
+    sess.close()
+
+
 # bfloat16 modes: gate and up as one product whose result leaves as terms, on tiles of one and of
 # two channel tiles per wavefront, a result that ends inside 64 channels; the norm behind o and down
 # in the kernel that adds slices of K and as a launch of its own; the attention's fold as terms
