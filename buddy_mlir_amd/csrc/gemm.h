@@ -13,6 +13,14 @@ struct RopeKv {
   int heads = 0, kv_heads = 0, max_len = 0, start_pos = 0;
 };
 
+// The unscaled sums of a product's K slices, [tile][slice][wavefront][row][channel] with tiles
+// of tile_rows rows x 4 wavefronts of `span` channels, `ncols` of them side by side, and what
+// makes results of them: bias[n] + (sum * steps[m]) * scale[n] (no steps: 1).
+struct SliceSums {
+  const float *partial = nullptr, *steps = nullptr, *scale = nullptr, *bias = nullptr;
+  int slices = 0, span = 0, tile_rows = 0, ncols = 0, N = 0;
+};
+
 struct GemmW8Args {
   const float *A = nullptr; // [M, K], row stride lda
   int64_t lda = 0;
@@ -40,7 +48,7 @@ struct GemmW8Args {
   const float *then_norm_w = nullptr;
   float then_norm_eps = 0.f;
   void *then_norm_staged = nullptr;
-  // digits only: C is q | k | v, and what follows it is done too, by the kernel that adds the
+  // C is q | k | v, and what follows it is done too, by the kernel that adds the
   // K slices where there is one, else by a launch of its own (ldc == N, no accumulation)
   const RopeKv *then_rope = nullptr;
   // Caller-provided staging of A (written by one of the producers below for
@@ -84,6 +92,9 @@ int launch_silu_mul_to_digits(const float *g, const float *u, int64_t ld, int ro
                               void *staged, hipStream_t stream);
 int launch_activations_to_digits(const float *A, int64_t lda, int64_t M, int64_t K,
                                  int digits, void *staged, hipStream_t stream);
+// q | k | v [M, ldc] out of its slices, and what follows it (gemm_w8_i8.hip)
+int launch_slices_rope(const SliceSums &sums, const RopeKv &rope, float *C, int64_t ldc, int M,
+                       hipStream_t stream);
 // the matmul over digit planes (called by launch_gemm_w8 when digits != 0)
 int launch_gemm_w8_digits(const GemmW8Args &a, const void *planes, hipStream_t stream);
 

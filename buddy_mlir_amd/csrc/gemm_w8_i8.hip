@@ -735,7 +735,8 @@ __global__ void __launch_bounds__(kSlices *kWave) gemm_w8_i8_tall_kernel(BH_I8_L
 }
 
 // Where the sums of row m, channels n.. of the first K slice lie.
-__device__ __forceinline__ const float *first_slice(const GemmI8Args &a, int m, int n) {
+template <class Args> // GemmI8Args, SliceSums
+__device__ __forceinline__ const float *first_slice(const Args &a, int m, int n) {
   const int tile = m / a.tile_rows * a.ncols + n / (kSlices * a.span), wave = n / a.span % kSlices;
   const size_t row =
       ((size_t)tile * a.slices * kSlices + wave) * a.tile_rows + m % a.tile_rows;
@@ -809,25 +810,28 @@ reduce_slices_kernel(GemmI8Args a) {
 // Small workgroups: a short prompt's few loads then come in through many compute units.
 constexpr int kRopeThreads = 64;
 __global__ void __launch_bounds__(kRopeThreads)
-reduce_slices_rope_kernel(GemmI8Args a, RopeKv r) {
+reduce_slices_rope_kernel(SliceSums a, RopeKv r, float *C, int64_t ldc, int M) {
   constexpr int kHalf = kAttnHeadDim / 2;
   const int turned = (r.heads + r.kv_heads) * (kHalf / 4), per_row = turned + r.kv_heads * (kAttnHeadDim / 4);
   const int64_t i = (int64_t)blockIdx.x * kRopeThreads + threadIdx.x;
-  if (i >= (int64_t)a.M * per_row)
+  if (i >= (int64_t)M * per_row)
     return;
   const int m = (int)(i / per_row), t = (int)(i % per_row), pos = r.start_pos + m;
   const size_t slice_stride = (size_t)kSlices * a.tile_rows * a.span;
-  const float step = a.steps[m];
-  float *row = a.C + (int64_t)m * a.ldc;
+  const float step = a.steps ? a.steps[m] : 1.0f;
+  float *row = C + (int64_t)m * ldc;
   // a quad's first eight slices and its operands
   struct Quad {
     float4 q[8];
-    FinishOperands f;
+    float scale[4], bias[4];
     const float *p;
   };
   auto request = [&](int n, Quad &x) {
     x.p = first_slice(a, m, n);
-    x.f = load_finish_operands(a, row + n, n);
+    load4(a.scale, n, a.N, x.scale);
+    x.bias[0] = x.bias[1] = x.bias[2] = x.bias[3] = 0.f;
+    if (a.bias)
+      load4(a.bias, n, a.N, x.bias);
 #pragma unroll
     for (int u = 0; u < 8; ++u)
       x.q[u] = *reinterpret_cast<const float4 *>(x.p + (size_t)min(u, a.slices - 1) * slice_stride);
@@ -849,7 +853,7 @@ reduce_slices_rope_kernel(GemmI8Args a, RopeKv r) {
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      v[e] = x.f.bias[e] + (v[e] * step) * x.f.scale[e];
+      v[e] = x.bias[e] + (v[e] * step) * x.scale[e];
   };
   if (t >= turned) { // v
     const int at = (t - turned) * 4, head = at / kAttnHeadDim, d = at % kAttnHeadDim;
@@ -1284,6 +1288,15 @@ void release_gemm_i8_workspace(hipStream_t stream) {
   g_workspace.erase(it);
 }
 
+int launch_slices_rope(const SliceSums &sums, const RopeKv &r, float *C, int64_t ldc, int M,
+                       hipStream_t stream) {
+  const int64_t quads = (int64_t)M * (r.heads + 3 * r.kv_heads) * (kAttnHeadDim / 8);
+  hipLaunchKernelGGL(reduce_slices_rope_kernel, dim3((unsigned)ceil_div(quads, kRopeThreads)),
+                     dim3(kRopeThreads), 0, stream, sums, r, C, ldc, M);
+  BH_CHECK_HIP(hipGetLastError());
+  return BUDDY_HIP_OK;
+}
+
 // `planes` holds the digit planes and row steps of the activations (written by
 // one of the producers above for exactly this M, K and digit count).
 namespace {
@@ -1322,9 +1335,10 @@ int launch_gemm_w8_digits_d(const GemmW8Args &in, const void *planes, hipStream_
   // 5 us, unless the kernel that adds K slices writes its planes (it holds whole
   // rows, up to kRowCache columns).
   const bool slices_fuse_norm = gemm_staging_layout(in.M, in.N).cols_padded <= kRowCache;
-  // The rotation behind q | k | v likewise: 4 us.
+  // The rotation behind q | k | v likewise: 4 us, in the kernel that adds slices 0.5 and what the
+  // angles take, which every head works out for itself there.
   const double norm_us = in.then_norm_w ? 5.0 : in.then_rope ? 4.0 : 0.0;
-  const double split_norm_us = in.then_rope ? 0.5 : slices_fuse_norm ? 0.0 : norm_us;
+  const double split_norm_us = in.then_rope ? 0.5 + 0.004 * (double)in.M : slices_fuse_norm ? 0.0 : norm_us;
   // the RMSNorm of the finished rows into digit planes, where the caller asked
   // for it and no kernel of the matmul holds whole rows
   auto then_norm = [&]() -> int {
@@ -1366,14 +1380,9 @@ int launch_gemm_w8_digits_d(const GemmW8Args &in, const void *planes, hipStream_
     BH_CHECK_HIP(hipGetLastError());
     return BUDDY_HIP_OK;
   }
-  if (in.then_rope) {
-    const RopeKv &r = *in.then_rope;
-    const int64_t quads = (int64_t)a.M * (r.heads + 3 * r.kv_heads) * (kAttnHeadDim / 8);
-    hipLaunchKernelGGL(reduce_slices_rope_kernel, dim3((unsigned)ceil_div(quads, kRopeThreads)),
-                       dim3(kRopeThreads), 0, stream, a, r);
-    BH_CHECK_HIP(hipGetLastError());
-    return BUDDY_HIP_OK;
-  }
+  if (in.then_rope)
+    return launch_slices_rope({a.partial, a.steps, a.scale, a.bias, a.slices, a.span, a.tile_rows, a.ncols, a.N},
+                              *in.then_rope, a.C, a.ldc, a.M, stream);
   const int64_t threads = (int64_t)a.M * ((a.N + 3) / 4);
   hipLaunchKernelGGL(reduce_slices_kernel, dim3((unsigned)ceil_div(threads, 256)), dim3(256), 0,
                      stream, a);

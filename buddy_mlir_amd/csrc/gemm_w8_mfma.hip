@@ -709,7 +709,8 @@ struct TilePlan {
   double us = 0;
 };
 // A norm of the finished rows is a launch of its own, 5 us, unless the kernel that adds the
-// slices does it.
+// slices does it; the rotation of q and k 4 us, there 0.5 and what its angles
+// take, which every head works out for itself.
 TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, int terms, bool may_split, bool pair,
                     double norm_us, double split_norm_us) {
   TilePlan best;
@@ -808,6 +809,14 @@ int launch_plan(const TilePlan &plan, GemmArgs &a, const GemmW8Args &in, hipStre
     BH_CHECK_HIP(hipGetLastError());
     return BUDDY_HIP_OK;
   }
+  if (in.then_rope) {
+    const RopeKv &r = *in.then_rope;
+    if (a.slices > 1)
+      return launch_slices_rope({a.partial, nullptr, a.scale, a.bias, a.slices, a.span, a.tile_rows, a.ncols, a.N},
+                                r, a.C, a.ldc, a.M, stream);
+    return launch_rope_kv_write(a.C, a.ldc, r.inv_freq, r.kcache, r.vcache, r.heads, r.kv_heads, kAttnHeadDim,
+                                r.max_len, r.start_pos, a.M, stream);
+  }
   if (a.slices > 1) {
     const int64_t threads = (int64_t)a.M * ceil_div(a.N, 4);
     hipLaunchKernelGGL(add_slices_kernel, dim3((unsigned)ceil_div(threads, 256)), dim3(256), 0,
@@ -880,7 +889,7 @@ int launch_gemm_w8(const GemmW8Args &in, hipStream_t stream) {
              "gemm_w8: a following norm needs a buffer for its rows");
   if (in.then_rope) {
     const RopeKv &r = *in.then_rope;
-    BH_REQUIRE(in.digits && !in.silu_pair && !in.accumulate && !in.then_norm_w && in.ldc == in.N && r.inv_freq &&
+    BH_REQUIRE(!in.silu_pair && !in.accumulate && !in.then_norm_w && in.ldc == in.N && r.inv_freq &&
                    r.kcache && r.vcache && r.heads > 0 && r.kv_heads > 0 &&
                    in.N == (int64_t)(r.heads + 2 * r.kv_heads) * kAttnHeadDim && r.start_pos >= 0 &&
                    r.start_pos + in.M <= r.max_len &&
@@ -942,10 +951,11 @@ int launch_gemm_w8(const GemmW8Args &in, hipStream_t stream) {
     a.pair_Kp = gemm_staging_layout(in.M, a.N).cols_padded;
     return launch_plan(plan_tiles(in.M, a.N, a.chunks, in.terms, false, true, 0.0, 0.0), a, in, stream);
   }
-  const double norm_us = in.then_norm_w ? 5.0 : 0.0;
+  const double norm_us = in.then_norm_w ? 5.0 : in.then_rope ? 4.0 : 0.0;
   const bool fuses = gemm_staging_layout(in.M, in.N).cols_padded <= kNormColumns;
-  return launch_plan(plan_tiles(in.M, in.N, a.chunks, in.terms, true, false, norm_us, fuses ? 0.0 : norm_us),
-                     a, in, stream);
+  const double split_norm_us = in.then_rope ? 0.5 + 0.004 * (double)in.M : fuses ? 0.0 : norm_us;
+  return launch_plan(plan_tiles(in.M, in.N, a.chunks, in.terms, true, false, norm_us, split_norm_us), a, in,
+                     stream);
 }
 
 void release_gemm_staging(hipStream_t stream) {

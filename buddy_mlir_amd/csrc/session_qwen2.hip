@@ -425,7 +425,6 @@ struct Qwen2Session : Session {
     bool normed_ahead = false; // pf_xn_bf already holds this layer's normed input
     for (int i = 0; i < S.layers; ++i) {
       Layer &L = layers[(size_t)i];
-      bool rotated = false; // the q|k|v matmul has also done what follows it
       if (L.qkv_f32) {
         if ((rc = launch_rmsnorm(pf_x, L.ln1, pf_xn, n, S.hidden, S.rms_eps, stream)))
           return rc;
@@ -435,8 +434,8 @@ struct Qwen2Session : Session {
                                     L.qkv.K, L.qkv.N, L.qkv.N, true, stream)))
           return rc;
       } else {
-        // the norm writes the matmul's input format directly (digit planes: the
-        // previous layer's down matmul already has)
+        // the norm writes the matmul's input format directly (the previous layer's down
+        // matmul already has), and the matmul does what follows it
         if (!normed_ahead && (rc = norm_to_staging(pf_x, L.ln1, n, pf_xn_bf)))
           return rc;
         normed_ahead = false;
@@ -448,12 +447,10 @@ struct Qwen2Session : Session {
         rope.kv_heads = S.kv_heads;
         rope.max_len = S.max_len;
         rope.start_pos = start_pos;
-        rotated = gemm_digits != 0;
-        if ((rc = gemm_staged(pf_xn_bf, L.qkv, pf_qkv, n, false, 0, nullptr, nullptr,
-                              rotated ? &rope : nullptr)))
+        if ((rc = gemm_staged(pf_xn_bf, L.qkv, pf_qkv, n, false, 0, nullptr, nullptr, &rope)))
           return rc;
       }
-      if (!rotated && (rc = launch_rope_kv_write(pf_qkv, QKV, inv_freq, L.kc, L.vc, S.heads,
+      if (L.qkv_f32 && (rc = launch_rope_kv_write(pf_qkv, QKV, inv_freq, L.kc, L.vc, S.heads,
                                                  S.kv_heads, S.head_dim, S.max_len, start_pos,
                                                  n, stream)))
         return rc;
