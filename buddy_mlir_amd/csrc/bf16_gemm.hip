@@ -301,7 +301,7 @@ rows_gemm_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int columns
 // ones.
 //
 // What bounds it: a step of 128 rows x 256 channels is 1024 cycles of matrix instructions
-// and takes 1725 at 2.0 GHz, with the loads of the rows and their way into LDS in the
+// and takes some 1620 at 2.0 GHz, with the loads of the rows and their way into LDS in the
 // wavefront's one stream of instructions, and the clock falls with the power the matrix
 // cores draw (2.4 to 1.9 GHz).  Against 16 x 16 tiles (us, rows x K x channels):
 //   bfloat16  2048 x 4096 x 4096   82.0 -> 75.2    f32   523 -> 216
@@ -423,6 +423,7 @@ rows_gemm_wide_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int co
   }
 
   uint4 wr[4][GT * 4], xr[4][kLoads];
+  constexpr int kFetches = GT * 4 + kLoads; // loads of a step
   const int last_run = (K - 1) / kRunElems * kRunElems;
   const bool ragged = K % kWideK != 0; // the last step reaches past K
   auto fetch_w = [&](int s, uint4 (&w)[GT * 4]) {
@@ -493,17 +494,34 @@ rows_gemm_wide_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int co
   load_frag(cur, 0, frag[0]);
   auto step = [&](int s, uint4 (&w)[GT * 4], uint4 (&w_new)[GT * 4], uint4 (&x)[kLoads],
                   uint4 (&x_new)[kLoads]) {
+    const int wt = min(s + 3, steps - 1) * 2, xk = min(min(s + 5, steps - 1) * kWideK + run_k, last_run);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       // the next fragments are asked for ahead of the products that cover their way, and
       // stay there: left to itself the scheduler moves them to their use
       load_frag(u < 3 ? cur : next, (u + 1) & 3, frag[(u + 1) & 1]);
-      if (u == 0)
-        fetch_w(s + 3, w_new);
+      // Of a tile that has its compute unit to itself the step's loads go evenly between its
+      // products, weights first (gate | up of 16 experts, 2048 x 4 rows of 1536 -> 2 x 1792: 158
+      // us with all at once, 148.5 so); of the others, which hide each other's, in two parts (90.4
+      // and 91.4 for the experts' way back).
+      if constexpr (RT == 4) {
+#pragma unroll
+        for (int i = u * kFetches / 4; i < (u + 1) * kFetches / 4; ++i) {
+          if (i < GT * 4) {
+            const int g = i % GT, q = i / GT;
+            w_new[g * 4 + q] = wp[g][(int64_t)(wt + q / 2) * 64 + (q & 1) * 32];
+          } else {
+            x_new[i - GT * 4] = *reinterpret_cast<const uint4 *>(src[i - GT * 4] + xk);
+          }
+        }
+      } else {
+        if (u == 0)
+          fetch_w(s + 3, w_new);
+        if (u == 2)
+          fetch_x(s + 5, x_new);
+      }
       if (u == 1)
         put_x(s + 2, x, fill);
-      if (u == 2)
-        fetch_x(s + 5, x_new);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int p = kTerms - 1; p >= 0; --p)
