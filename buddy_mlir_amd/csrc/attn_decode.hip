@@ -402,28 +402,41 @@ __global__ void __launch_bounds__(kWaves * 64)
     constexpr bool kWhole = decltype(whole_chunk)::value;
     for (int hh = h_lo; hh < h_hi; ++hh) {
       const float4 q4 = *reinterpret_cast<const float4 *>(q_s[hh] + c4 * 4);
-      float sc[kR];
+      float d[kR];
 #pragma unroll
       for (int i = 0; i < kR; ++i) {
-        const int p = pw0 + par + 2 * i;
         const float4 k4 = kreg[i];
-        float d = fmaf(q4.x, k4.x, fmaf(q4.y, k4.y, fmaf(q4.z, k4.z, q4.w * k4.w)));
-        d = row16_sum(d);
-        d += __shfl_xor(d, 16, 64);
-        sc[i] = kWhole || p <= pos ? d * a.scale : -INFINITY;
+        d[i] = fmaf(q4.x, k4.x, fmaf(q4.y, k4.y, fmaf(q4.z, k4.z, q4.w * k4.w)));
       }
-      float m_w = kSeedM;
+      // The sums of eight keys over the 32 lanes of a half, halving the keys a lane still
+      // carries with each of three exchanges: lane l ends up with key key_of(l), so there is
+      // one exponential a lane and not eight (12000 positions: 11.4 -> 10.7 us).
+      static_assert(kR == 8, "three halvings");
+      const bool b3 = lane & 8, b2 = lane & 4, b1 = lane & 2;
 #pragma unroll
-      for (int i = 0; i < kR; ++i)
-        m_w = fmaxf(m_w, sc[i]);
-      m_w = fmaxf(m_w, __shfl_xor(m_w, 32, 64));
-      float l_w = 0.f;
+      for (int i = 0; i < 4; ++i)
+        d[i] = (b3 ? d[2 * i + 1] : d[2 * i]) + dpp_f<0x140>(b3 ? d[2 * i] : d[2 * i + 1]); // lane ^ 15
 #pragma unroll
-      for (int i = 0; i < kR; ++i) {
-        sc[i] = fast_exp(sc[i] - m_w);
-        l_w += sc[i];
-      }
+      for (int i = 0; i < 2; ++i)
+        d[i] = (b2 ? d[2 * i + 1] : d[2 * i]) + dpp_f<0x141>(b2 ? d[2 * i] : d[2 * i + 1]); // lane ^ 7
+      float s = (b1 ? d[1] : d[0]) + dpp_f<0x4E>(b1 ? d[0] : d[1]);                         // lane ^ 2
+      s += dpp_f<0xB1>(s);                                                                  // lane ^ 1
+      s += __shfl_xor(s, 16, 64);
+      const int mine = pw0 + par + 2 * ((lane >> 3 & 1) + (lane >> 1 & 2) + (lane << 1 & 4));
+      s = kWhole || mine <= pos ? s * a.scale : -INFINITY;
+      // over the eight keys of the half, each once, and both halves
+      float m_w = fmaxf(s, dpp_f<0x140>(s));
+      m_w = fmaxf(m_w, dpp_f<0x141>(m_w));
+      m_w = fmaxf(m_w, dpp_f<0x4E>(m_w));
+      m_w = fmaxf(fmaxf(kSeedM, m_w), __shfl_xor(m_w, 32, 64));
+      s = fast_exp(s - m_w);
+      float l_w = s + dpp_f<0x140>(s);
+      l_w += dpp_f<0x141>(l_w);
+      l_w += dpp_f<0x4E>(l_w);
       l_w += __shfl_xor(l_w, 32, 64);
+      // every lane of a row of 16 gets the weight of key i from lane 8 i0 + 4 i1 + 2 i2
+      float sc[kR] = {dpp_f<0x150>(s), dpp_f<0x158>(s), dpp_f<0x154>(s), dpp_f<0x15C>(s),
+                      dpp_f<0x152>(s), dpp_f<0x15A>(s), dpp_f<0x156>(s), dpp_f<0x15E>(s)};
       float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
       for (int i = 0; i < kR; ++i) {
