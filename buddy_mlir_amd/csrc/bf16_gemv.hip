@@ -829,7 +829,7 @@ int launch_row_gemv(const RowGemv &a, hipStream_t stream) {
   const dim3 grid((unsigned)(ceil_div(groups, per) + keeper)), block(kRowThreads);
   bool quads = W.K % 4 == 0 && a.head_dim % 4 == 0;
   for (const void *p : {(const void *)a.src, (const void *)a.y, (const void *)a.x_out,
-                        (const void *)a.row_out, (const void *)a.conv_w, (const void *)a.conv_next,
+                        (const void *)a.row_out, (const void *)a.conv_w, (const void *)a.conv_ring, (const void *)a.conv_next,
                         (const void *)a.weight, (const void *)a.gate, (const void *)a.add,
                         (const void *)a.norm_w})
     quads = quads && ((uintptr_t)p & 15) == 0;
