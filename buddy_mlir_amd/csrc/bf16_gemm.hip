@@ -670,11 +670,17 @@ int launch_tiles(F kernel, int elems, const RowsGemm &a, hipStream_t stream) {
 
 BH_TILE_FAMILY(RowsFamily, "rows_gemm_kernel");
 BH_TILE_FAMILY(WideFamily, "rows_gemm_wide_kernel");
+// ... and those of them whose K was cut
+BH_TILE_FAMILY(RowsSlicesFamily, "rows_gemm_kernel slices");
+BH_TILE_FAMILY(WideSlicesFamily, "rows_gemm_wide_kernel slices");
 
 // 16 rows, GT channel groups per wavefront (pairs count twice)
 template <typename T, int GT, int OUT, bool GROUPED>
 int launch_flat(const RowsGemm &a, hipStream_t stream) {
   BH_NOTE_VARIANT(RowsFamily, sizeof(T) == 4, GT, OUT, GROUPED);
+  if constexpr (OUT == kOutF32 && !GROUPED)
+    if (a.slices > 1)
+      BH_NOTE_VARIANT(RowsSlicesFamily, sizeof(T) == 4, GT);
   return launch_tiles<T, 16, 64 * (OUT == kOutExpertAct ? GT / 2 : GT), OUT, GROUPED>(
       rows_gemm_kernel<T, GT, OUT, GROUPED>, ActTraits<T>::kElems, a, stream);
 }
@@ -682,6 +688,9 @@ int launch_flat(const RowsGemm &a, hipStream_t stream) {
 template <typename T, int RT, int GT, int OUT, bool GROUPED>
 int launch_wide(const RowsGemm &a, hipStream_t stream) {
   BH_NOTE_VARIANT(WideFamily, sizeof(T) == 4, RT, GT, OUT, GROUPED);
+  if constexpr (OUT == kOutF32 && !GROUPED)
+    if (a.slices > 1)
+      BH_NOTE_VARIANT(WideSlicesFamily, sizeof(T) == 4, RT, GT);
   return launch_tiles<T, 32 * RT, 128 * (OUT == kOutExpertAct ? GT / 2 : GT), OUT, GROUPED>(
       rows_gemm_wide_kernel<T, RT, GT, OUT, GROUPED>, kWideK, a, stream);
 }

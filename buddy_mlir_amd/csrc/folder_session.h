@@ -209,10 +209,12 @@ struct FolderSession : Session {
     const int64_t one = (int64_t)rows * width, few = (int64_t)std::min(rows, kSliceRows) * width;
     return (size_t)std::max(one, std::min(kMaxSlices * few, kSliceFloats));
   }
-  int sliced_product(const Bf16Matrix &W, const void *A, int lda, int rows, float *y, NormRows &pend) {
+  // `whole`: never cut.
+  int sliced_product(const Bf16Matrix &W, const void *A, int lda, int rows, float *y, NormRows &pend,
+                     bool whole = false) {
     RowsGemm g = gemm(W, A, lda, rows, kOutF32, y, W.N);
     g.slice_stride = (int64_t)rows * W.N;
-    if (rows <= kSliceRows)
+    if (!whole && rows <= kSliceRows)
       g.slices = (int)std::clamp<int64_t>((int64_t)sliced_floats(rows, W.N) / g.slice_stride, 1, kMaxSlices);
     pend.y = y;
     pend.y_stride = g.slice_stride;

@@ -130,3 +130,29 @@ def row_errors(got, want):
     d -= d.mean(-1, keepdims=True)
     w = want - want.mean(-1, keepdims=True)
     return np.sqrt((d * d).mean(-1) / np.maximum((w * w).mean(-1), 1e-12))
+
+
+def clear_tokens(cfg, t, n, gap, seed=0):
+    """n tokens at which no router is in doubt: in every layer the weakest chosen logit of every
+    row is at least `gap` times the row's largest above the strongest that is not chosen."""
+    rng = np.random.default_rng(seed)
+    tokens = rng.integers(0, cfg["vocab"], n).astype(np.int32)
+    route, doubt = N.route, np.zeros(n, bool)
+
+    def watched(h, router, top):
+        z = np.sort(h @ router.T, -1)[:, ::-1]
+        if top < z.shape[1]:
+            doubt[:] |= z[:, top - 1] - z[:, top] < gap * np.abs(z).max(-1)
+        return route(h, router, top)
+    N.route = watched
+    try:
+        for _ in range(20 * n):
+            doubt[:] = False
+            N.forward(cfg, t, tokens)
+            if not doubt.any():
+                return tokens
+            at = int(doubt.argmax())  # rows ahead of it do not see it
+            tokens[at] = rng.integers(0, cfg["vocab"])
+    finally:
+        N.route = route
+    raise AssertionError("no such tokens")

@@ -109,6 +109,25 @@ def test_mechanism_alone(tmp_path, what, dtype):
     check(feed(s, tokens, [3] + [1] * 67), want, dtype, "decoding")
 
 
+# A bfloat16 prompt's routers read rounded rows, where the last bit of a sum can choose another
+# expert: neither the output product nor the shared expert's way back is cut into slices of K.  At
+# tokens whose routers are not in doubt, every row is within the bound.  (A margin of 0.15 of the
+# largest logit is some ten times what the rounding of two layers moves one.)
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n", [17, 45, 130])
+def test_no_slices_of_k_ahead_of_rounded_routers(tmp_path, bh, n, dtype):
+    moe = M.moe(experts=4, top=1, shared_ff=4100)
+    cfg = M.config([M.latent(heads=16, vdim=128, mlp=moe), M.linear(decay=[0.9] * 16, vdim=128, mlp=moe)],
+                   width=72, vocab=300)
+    folder, t = M.build(tmp_path, cfg, n)
+    tokens = M.clear_tokens(cfg, t, n, 0.15)
+    s = FolderSession(folder, dtype, max_len=n + 8)
+    bh.buddy_hip_variant_reset()
+    check(all_rows(s, tokens), N.forward(cfg, t, tokens), dtype, strict=True)
+    cut = {k for k, v in tiles_run(bh).items() if v and "slices" in k}
+    assert bool(cut) == (dtype == "float32"), cut
+
+
 # moe_down_kernel: a wavefront's slice of the experts' k on both sides of its 9 and 14 loads, in
 # one trip and in several, with many experts in one trip, halves of a channel group (fewer than
 # 192 of them) and whole ones; moe_gate_up_kernel: runs of fewer tiles than in flight and of more
