@@ -686,8 +686,8 @@ BH_TILE_FAMILY(WideFamily, "rows_gemm_wide_kernel");
 BH_TILE_FAMILY(RowsSlicesFamily, "rows_gemm_kernel slices");
 BH_TILE_FAMILY(WideSlicesFamily, "rows_gemm_wide_kernel slices");
 
-// 16 rows, GT channel groups per wavefront (pairs count twice)
-template <typename T, int GT, int OUT, bool GROUPED>
+// 16 rows, GT channel groups per wavefront (pairs count twice).  CUT: K may be in slices.
+template <typename T, int GT, int OUT, bool GROUPED, bool CUT>
 int launch_flat(const RowsGemm &a, hipStream_t stream) {
   BH_NOTE_VARIANT(RowsFamily, sizeof(T) == 4, GT, OUT, GROUPED);
   auto run = [&](auto sliced) {
@@ -695,7 +695,7 @@ int launch_flat(const RowsGemm &a, hipStream_t stream) {
     return launch_tiles<16, 64 * (OUT == kOutExpertAct ? GT / 2 : GT), GROUPED, S>(
         rows_gemm_kernel<T, GT, OUT, GROUPED, S>, ActTraits<T>::kElems, a, stream);
   };
-  if constexpr (OUT == kOutF32 && !GROUPED)
+  if constexpr (CUT)
     if (a.slices > 1) {
       BH_NOTE_VARIANT(RowsSlicesFamily, sizeof(T) == 4, GT);
       return run(std::true_type{});
@@ -703,7 +703,7 @@ int launch_flat(const RowsGemm &a, hipStream_t stream) {
   return run(std::false_type{});
 }
 // RT tiles of 32 rows, GT tiles of 32 channels per wavefront
-template <typename T, int RT, int GT, int OUT, bool GROUPED>
+template <typename T, int RT, int GT, int OUT, bool GROUPED, bool CUT>
 int launch_wide(const RowsGemm &a, hipStream_t stream) {
   BH_NOTE_VARIANT(WideFamily, sizeof(T) == 4, RT, GT, OUT, GROUPED);
   auto run = [&](auto sliced) {
@@ -711,7 +711,7 @@ int launch_wide(const RowsGemm &a, hipStream_t stream) {
     return launch_tiles<32 * RT, 128 * (OUT == kOutExpertAct ? GT / 2 : GT), GROUPED, S>(
         rows_gemm_wide_kernel<T, RT, GT, OUT, GROUPED, S>, kWideK, a, stream);
   };
-  if constexpr (OUT == kOutF32 && !GROUPED)
+  if constexpr (CUT)
     if (a.slices > 1) {
       BH_NOTE_VARIANT(WideSlicesFamily, sizeof(T) == 4, RT, GT);
       return run(std::true_type{});
@@ -735,14 +735,15 @@ int launch_shape(const RowsGemm &a, hipStream_t stream, int *slices) {
   const int64_t all_blocks = GROUPED ? std::min<int64_t>(a.experts, a.list_total) : 1;
   constexpr bool kPair = OUT == kOutExpertAct;
   constexpr int P = kPair ? 2 : 1; // groups come in pairs
+  constexpr bool CUT = OUT == kOutF32 && !GROUPED;
   auto workgroups = [&](int rt, int ch) {
     return ceil_div(a.W.N, ch) * ceil_div(rows, rt) * all_blocks;
   };
   if (rows <= 16) {
     RowsGemm b = a;
     b.slices = 1;
-    return workgroups(16, 128) >= 256 ? launch_flat<T, 2 * P, OUT, GROUPED>(b, stream)
-                                      : launch_flat<T, P, OUT, GROUPED>(b, stream);
+    return workgroups(16, 128) >= 256 ? launch_flat<T, 2 * P, OUT, GROUPED, false>(b, stream)
+                                      : launch_flat<T, P, OUT, GROUPED, false>(b, stream);
   }
   // With slices of k that the caller adds: the tile and the number of slices together, which
   // cost the bytes of their sums.  8960 -> 1536: 777
@@ -785,9 +786,9 @@ int launch_shape(const RowsGemm &a, hipStream_t stream, int *slices) {
     if constexpr (!kPair) {
       const Cost low = cost(32, 128, 0.46, 4.0);
       if (low <= wide)
-        return done(launch_wide<T, 1, 1, OUT, GROUPED>(with(low), stream));
+        return done(launch_wide<T, 1, 1, OUT, GROUPED, CUT>(with(low), stream));
     }
-    return done(launch_wide<T, 1, 2, OUT, GROUPED>(with(wide), stream));
+    return done(launch_wide<T, 1, 2, OUT, GROUPED, CUT>(with(wide), stream));
   } else {
     // few rows: 16-row tiles of 64 channels, while they are few rounds of the chip
     const Cost tall = cost(128, 256, 1.02, 7.0), flat = cost(16, 64 * P, 0.13 * P, 2.5);
@@ -804,12 +805,12 @@ int launch_shape(const RowsGemm &a, hipStream_t stream, int *slices) {
       low = cost(32, 128, 0.21, 4.0);
     }
     if (flat <= std::min({tall, half, low}))
-      return done(launch_flat<T, P, OUT, GROUPED>(with(flat), stream));
+      return done(launch_flat<T, P, OUT, GROUPED, CUT>(with(flat), stream));
     if (tall <= std::min(half, low))
-      return done(launch_wide<T, 4, 2, OUT, GROUPED>(with(tall), stream));
+      return done(launch_wide<T, 4, 2, OUT, GROUPED, CUT>(with(tall), stream));
     constexpr int GT = kPair ? 2 : 1;
-    return done(half <= low ? launch_wide<T, 2, GT, OUT, GROUPED>(with(half), stream)
-                            : launch_wide<T, 1, GT, OUT, GROUPED>(with(low), stream));
+    return done(half <= low ? launch_wide<T, 2, GT, OUT, GROUPED, CUT>(with(half), stream)
+                            : launch_wide<T, 1, GT, OUT, GROUPED, CUT>(with(low), stream));
   }
 }
 
