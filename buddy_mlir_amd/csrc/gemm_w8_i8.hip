@@ -1288,8 +1288,14 @@ void release_gemm_i8_workspace(hipStream_t stream) {
   g_workspace.erase(it);
 }
 
+BH_TILE_FAMILY(SlicesRopeFamily, "reduce_slices_rope_kernel"); // trips for eight slices: one, more
+
 int launch_slices_rope(const SliceSums &sums, const RopeKv &r, float *C, int64_t ldc, int M,
                        hipStream_t stream) {
+  if (sums.slices <= 8)
+    BH_NOTE_VARIANT(SlicesRopeFamily, 1);
+  else
+    BH_NOTE_VARIANT(SlicesRopeFamily, 2);
   const int64_t quads = (int64_t)M * (r.heads + 3 * r.kv_heads) * (kAttnHeadDim / 8);
   hipLaunchKernelGGL(reduce_slices_rope_kernel, dim3((unsigned)ceil_div(quads, kRopeThreads)),
                      dim3(kRopeThreads), 0, stream, sums, r, C, ldc, M);

@@ -685,6 +685,8 @@ int staging_for(hipStream_t stream, size_t bytes, u16 **out) {
 BH_VARIANT_FAMILY(WideFamily, "gemm_w8_bf16_wide_kernel");
 BH_VARIANT_FAMILY(NarrowFamily, "gemm_w8_bf16_kernel");
 BH_TILE_FAMILY(PairFamily, "gemm_w8_bf16_kernel pair"); // terms, channel tiles per wavefront
+BH_TILE_FAMILY(SlicesNormFamily, "add_slices_norm_kernel"); // more LDS than a launch gets unasked
+BH_TILE_FAMILY(NormBehindFamily, "add_slices_kernel and a norm behind it"); // 1
 
 template <class Kernel>
 int launch_tiles(Kernel kernel, const GemmArgs &a, unsigned blocks, hipStream_t stream) {
@@ -799,7 +801,10 @@ int launch_plan(const TilePlan &plan, GemmArgs &a, const GemmW8Args &in, hipStre
   u16 *normed = static_cast<u16 *>(in.then_norm_staged);
   if (a.slices > 1 && in.then_norm_w && fuses) {
     const size_t lds = 2 * sizeof(float) * (size_t)next.cols_padded;
-    if (lds > 48 * 1024) {
+    if (lds <= 48 * 1024) {
+      BH_NOTE_VARIANT(SlicesNormFamily, 0);
+    } else {
+      BH_NOTE_VARIANT(SlicesNormFamily, 1);
       static DynLdsOnce once;
       BH_CHECK_HIP(ensure_dyn_lds(once, reinterpret_cast<const void *>(add_slices_norm_kernel),
                                   (int)(2 * sizeof(float) * kNormColumns)));
@@ -818,6 +823,8 @@ int launch_plan(const TilePlan &plan, GemmArgs &a, const GemmW8Args &in, hipStre
                                 r.max_len, r.start_pos, a.M, stream);
   }
   if (a.slices > 1) {
+    if (in.then_norm_w)
+      BH_NOTE_VARIANT(NormBehindFamily, 1);
     const int64_t threads = (int64_t)a.M * ceil_div(a.N, 4);
     hipLaunchKernelGGL(add_slices_kernel, dim3((unsigned)ceil_div(threads, 256)), dim3(256), 0,
                        stream, a);

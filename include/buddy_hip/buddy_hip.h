@@ -54,7 +54,8 @@ int buddy_hip_device_count(void);
  * report needs.  A variant is listed from the moment the library is loaded,
  * launched or not, so a test can tell which ones its cases did not reach.
  * buddy_hip_tile_report does the same for matrix products whose tile an
- * estimate of their time picks.  buddy_hip_variant_reset sets every count back
+ * estimate of their time picks, and for the kernels behind the ones whose K it
+ * cut into slices.  buddy_hip_variant_reset sets every count back
  * to 0.  Host only; no counterpart in the reference. */
 int64_t buddy_hip_variant_report(char *text, int64_t capacity);
 int64_t buddy_hip_tile_report(char *text, int64_t capacity);

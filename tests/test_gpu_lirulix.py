@@ -15,6 +15,7 @@ import lirulix_models as M
 import lirulix_oracle as L
 from buddy_mlir_amd import BuddyHipError
 from buddy_mlir_amd.session import FolderSession, Sampler
+from tile_report import tiles_run
 
 pytestmark = pytest.mark.gpu
 
@@ -116,18 +117,46 @@ def test_one_row_through_the_feed_forward(tmp_path, width, ff, dtype):
     check(feed(s, tokens, [1] * 5), L.forward(cfg, t, tokens), dtype)
 
 
-# products of a prompt whose K is cut into slices that the norm behind them adds: K that ends inside
-# a step, slices of unequal length, rows on both sides of a tile, several portions of other sizes
+# products of a prompt whose K is cut into slices that the norm behind them adds, on every tile that
+# takes slices: K that ends inside a step, slices of unequal length, rows on both sides of a tile,
+# several portions of other sizes.  `tiles`: of the longest portion in bfloat16 and in f32, as
+# "rows_gemm_kernel slices<f32, channel groups per wavefront>" (16 rows) and
+# "rows_gemm_wide_kernel slices<f32, tiles of 32 rows, of 32 channels per wavefront>"
+FLAT, LOW, HALF, TALL = "kernel slices<0, 1>", "wide_kernel slices<0, 1, 1>", "wide_kernel slices<0, 2, 1>", \
+    "wide_kernel slices<0, 4, 2>"
+LOW32, WIDE32 = "wide_kernel slices<1, 1, 1>", "wide_kernel slices<1, 1, 2>"
+
+
+def slices_run(bh):
+    return {k for k, v in tiles_run(bh).items() if v and "slices" in k}
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("width,ff,n", [(72, 8970, 17), (72, 8970, 33), (200, 4100, 97), (72, 2310, 130),
-                                        (46, 5001, 65), (1536, 1700, 300)])
-def test_prompt_products_in_slices_of_k(tmp_path, width, ff, n, dtype):
+@pytest.mark.parametrize("width,ff,n,tiles", [
+    (72, 8970, 17, (FLAT, LOW32)), (72, 8970, 33, (FLAT, LOW32)), (200, 4100, 97, (FLAT, LOW32)),
+    (72, 2310, 130, (FLAT, LOW32)), (46, 5001, 65, (FLAT, LOW32)), (72, 5001, 777, (LOW, LOW32)),
+    (1536, 1700, 300, (LOW, LOW32)), (1536, 2310, 400, (HALF, WIDE32))])
+def test_prompt_products_in_slices_of_k(tmp_path, bh, width, ff, n, tiles, dtype):
     cfg = M.config([M.full(heads=1, ff=ff), M.delta(ff=ff)], loop=(0, 2, 2), width=width, vocab=64)
     folder, t = M.build(tmp_path, cfg, ff)
     tokens = tokens_for(cfg, n + 21)
     want = L.forward(cfg, t, tokens)
     s = FolderSession(folder, dtype, max_len=n + 32)
+    bh.buddy_hip_variant_reset()
     check(feed(s, tokens, [n, 20, 1]), want, dtype)
+    assert "rows_gemm_" + tiles[dtype == "float32"] in slices_run(bh), slices_run(bh)
+
+
+# an output product that is wide and has few rows: tiles of 128 rows in slices
+def test_wide_output_product_in_slices_of_k(tmp_path, bh):
+    cfg = M.config([M.full(heads=16, vdim=400, ff=None)], width=12336, vocab=32)
+    folder, t = M.build(tmp_path, cfg, 1)
+    tokens = tokens_for(cfg, 66)
+    want = L.forward(cfg, t, tokens)
+    s = FolderSession(folder, "bfloat16", max_len=80)
+    bh.buddy_hip_variant_reset()
+    check(all_rows(s, tokens), want, "bfloat16")
+    assert slices_run(bh) == {"rows_gemm_" + TALL}
 
 
 @pytest.mark.parametrize("dtype", DTYPES)

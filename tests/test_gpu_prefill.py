@@ -502,16 +502,23 @@ def test_which_prompt_attention(bh, heads, kv_heads, before, n, precision, split
 
 
 # q | k | v with the rotation and the cache rows behind it: K in more slices than are asked for at
-# once, in few and in one; one head and many; tokens behind a context
+# once (2 trips), in two to eight (1) and whole (0), of digit planes and of terms; one head and many;
+# tokens behind a context
 @pytest.mark.parametrize("precision", ["digits", "digits2", "exact", "bf16"])
-@pytest.mark.parametrize("hidden,heads,kv_heads,before,n", [
-    (2048, 1, 1, 0, 3), (1536, 2, 1, 7, 40), (320, 6, 3, 130, 17), (64, 12, 2, 0, 33), (256, 12, 2, 3, 900)])
-def test_rotation_behind_qkv(hidden, heads, kv_heads, before, n, precision):
+@pytest.mark.parametrize("hidden,heads,kv_heads,before,n,trips", [
+    (2048, 1, 1, 0, 3, (2, 2)), (1536, 2, 1, 7, 40, (2, 2)), (1536, 12, 2, 0, 27, (1, 2)),
+    (1536, 12, 2, 5, 100, (1, 1)), (320, 6, 3, 130, 17, (0, 0)), (64, 12, 2, 0, 33, (0, 0)),
+    (256, 12, 2, 3, 900, (0, 0))])
+def test_rotation_behind_qkv(bh, hidden, heads, kv_heads, before, n, trips, precision):
     shape = Shape(layers=2, hidden=hidden, heads=heads, kv_heads=kv_heads, head_dim=128, inter=64, vocab=320,
                   max_len=before + n + 8)
     toks = synthetic.first_tokens(shape, n, seed=n).astype(np.int32)
     sess, _ = synthetic.build_session(shape, context=before, ln_jitter=0.1)
+    bh.buddy_hip_variant_reset()
     sess.prefill(toks, before, precision=precision)
+    ran, trips = tiles_run(bh), trips[not precision.startswith("digits")]
+    assert [ran[f"reduce_slices_rope_kernel<{k}>"] for k in (1, 2)] == \
+        [shape.layers * (trips == k) for k in (1, 2)]
     rows = [sess.get_kv(j)[:, :before + n] for j in range(4)]
     sess.close()
     sess, _ = synthetic.build_session(shape, context=before, ln_jitter=0.1)
@@ -519,6 +526,8 @@ def test_rotation_behind_qkv(hidden, heads, kv_heads, before, n, precision):
         sess.decode(int(t), before + i, want_logits=False)
     for j in range(4):
         want = sess.get_kv(j)[:, :before + n]
+        np.testing.assert_array_equal(rows[j][:, :before], want[:, :before])
+        rows[j], want = rows[j][:, before:], want[:, before:]
         if precision in ("digits", "exact"):
             check_close(rows[j], want)
         else:  # some ten roundings on the way: of 2^-15 of a row's largest value, of 2^-9 of each
@@ -709,9 +718,10 @@ def test_prompt_attention_of_a_value_beyond_bfloat16(at, size):
             check_close(got[at:], want[at:])
 
 
-def test_wide_hidden_size_through_the_slice_adding_norm_kernel(oracle):
+@pytest.mark.parametrize("precision", ["digits", "exact"])
+def test_wide_hidden_size_through_the_slice_adding_norm_kernel(bh, oracle, precision):
     """hidden = 9216: the kernel that adds the K slices of o_proj / down and
-    writes the next RMSNorm's digit planes keeps two copies of a row in LDS,
+    writes the next RMSNorm's digit planes or terms keeps two copies of a row in LDS,
     72 KiB here -- more than the 64 KiB a kernel gets without asking.  A
     prompt of 64 tokens (one row tile: the matmuls then split K over
     workgroups) against 64 oracle decode steps."""
@@ -723,7 +733,10 @@ def test_wide_hidden_size_through_the_slice_adding_norm_kernel(oracle):
     toks = synthetic.first_tokens(shape, 64, seed=23).tolist()
     for pos, t in enumerate(toks):
         otok, ologits = om.decode_step(t, pos, kv)
-    nxt, logits = sess.prefill(toks, 0)
+    bh.buddy_hip_variant_reset()
+    nxt, logits = sess.prefill(toks, 0, precision=precision)
+    if precision == "exact":
+        assert tiles_run(bh)["add_slices_norm_kernel<1>"]
     check_close(logits, ologits)
     assert nxt == otok
     for j in range(2 * shape.layers):
@@ -731,15 +744,19 @@ def test_wide_hidden_size_through_the_slice_adding_norm_kernel(oracle):
     sess.close()
 
 
+@pytest.mark.parametrize("precision", ["digits", "exact"])
 @pytest.mark.parametrize("n", [20, 70])
-def test_hidden_size_beyond_the_slice_adding_norm_kernel(n):
+def test_hidden_size_beyond_the_slice_adding_norm_kernel(bh, n, precision):
     """hidden = 12352: a row is longer than that kernel holds; the norm is a launch of its own
     behind products with whole sums and with K in slices."""
     shape = Shape(layers=2, hidden=12352, heads=8, kv_heads=2, head_dim=128, inter=2048,
                   vocab=320, max_len=128)
     toks = synthetic.first_tokens(shape, n, seed=n).astype(np.int32)
     sess, _ = synthetic.build_session(shape, context=0, ln_jitter=0.1)
-    _, got = sess.prefill(toks, 0)
+    bh.buddy_hip_variant_reset()
+    _, got = sess.prefill(toks, 0, precision=precision)
+    if precision == "exact":
+        assert bool(tiles_run(bh)["add_slices_kernel and a norm behind it<1>"]) == (n == 20)
     rows = [sess.get_kv(j)[:, :n].copy() for j in range(4)]
     for i, t in enumerate(toks):
         _, want = sess.decode(int(t), i, want_logits=i + 1 == n)
