@@ -728,7 +728,10 @@ int launch_wide(const RowsGemm &a, hipStream_t stream) {
 // 32 or 64 x 128): 8960 -> 1536 at 24 rows 21.2 vs 28.4, at 150 22.7 vs 31.3, at 220 36.0
 // vs 31.5; 1536 -> 1536 at 64 rows 5.6 vs 6.9; 1536 -> 17920 at 64 rows 18.4 vs 12.4.  In
 // f32, whose three terms make the products the longer part, they gain nothing.
-constexpr double kSliceUs = 0.5; // of slices besides
+// What slices cost besides their bytes, in the norm that adds them: with half of that, products of
+// 256 to 1024 inputs were cut whose prompts then took 1 to 2 % longer (Lirulix of width 256, 64 bfloat16
+// tokens: 221.6 us whole, 226.5 cut).
+constexpr double kSliceUs = 1.0;
 template <typename T, int OUT, bool GROUPED>
 int launch_shape(const RowsGemm &a, hipStream_t stream, int *slices) {
   const int64_t rows = GROUPED ? ceil_div(a.list_total, a.experts) : a.rows;

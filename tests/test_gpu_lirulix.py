@@ -147,9 +147,21 @@ def test_prompt_products_in_slices_of_k(tmp_path, bh, width, ff, n, tiles, dtype
     assert "rows_gemm_" + tiles[dtype == "float32"] in slices_run(bh), slices_run(bh)
 
 
+# ... and stays whole where the steps that a slice saves are fewer than what adding slices takes
+@pytest.mark.parametrize("width,ff,n", [(256, 512, 33), (512, 512, 45)])
+def test_short_products_stay_whole(tmp_path, bh, width, ff, n):
+    cfg = M.config([M.full(heads=1, ff=ff)], width=width, vocab=64)
+    folder, t = M.build(tmp_path, cfg, ff)
+    tokens = tokens_for(cfg, n)
+    s = FolderSession(folder, "bfloat16", max_len=n + 8)
+    bh.buddy_hip_variant_reset()
+    check(all_rows(s, tokens), L.forward(cfg, t, tokens), "bfloat16")
+    assert not slices_run(bh)
+
+
 # an output product that is wide and has few rows: tiles of 128 rows in slices
 def test_wide_output_product_in_slices_of_k(tmp_path, bh):
-    cfg = M.config([M.full(heads=16, vdim=400, ff=None)], width=12336, vocab=32)
+    cfg = M.config([M.full(heads=16, vdim=450, ff=None)], width=12336, vocab=32)
     folder, t = M.build(tmp_path, cfg, 1)
     tokens = tokens_for(cfg, 66)
     want = L.forward(cfg, t, tokens)
