@@ -1143,8 +1143,9 @@ namespace {
 // tile's registers leave room for one.  A chunk of 64 k takes a workgroup that has its
 // compute unit to itself `alone`, two that share one `both`, each beside a fixed part; a last
 // round that fills less than half runs at the former.  Fitted to
-// launches of 20 to 1931 rows of 1536, 4096, 8960 and 14336 k, every tile with every K split: what
-// it picks is 1.0 (three planes) and 1.4 % (two) off the best on average, 9 and 15 at most.
+// launches of 20 to 1931 rows of 1536, 4096, 8960 and 14336 k, every tile with every K split.  Of 264
+// launches of 17 to 2048 rows under the profiler its pick is 1.7 (three planes) and 2.8 % (two) off the
+// best on average.
 // Microseconds of a product with three planes in a prompt (in brackets with rows of K bytes per
 // plane, a branch at every chunk and its loads all at the chunk's start):
 //   gate | up, 1536 -> 2 x 8960: 27 rows 12.4 [14.4], 512: 54 [59], 1931: 171.5 [182]
@@ -1154,8 +1155,8 @@ namespace {
 // The card holds its clock at 1.9 GHz under the large ones, whose matrix pipes are half busy:
 // without any loads in the loop gate | up of 1931 rows takes 119 us, with loads that all hit the
 // L1 157.
-// (gate | up at 27 rows with two channel tiles: 13.7, and 18.7 in a prompt, whose weights come
-// from memory, against 14.9 with one: twice the compute units ask for them.)
+// (gate | up of 28 rows with weights from memory: two channel tiles 15.4, one 11.4, for which twice
+// the compute units ask.)
 // Tiles that fill a compute unit alone have coarser rounds and use an operand more often
 // (64 rows x 256 channels: long sums and many rows; 32 x 640 and 96 x 256: row counts for
 // which they come to a whole round and the others to a little more than one).

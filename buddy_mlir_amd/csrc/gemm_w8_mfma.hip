@@ -232,9 +232,10 @@ struct GemmArgs {
 };
 
 // A tile of 32 RB rows x 128 GP channels, on v_mfma_f32_32x32x16_bf16 (GP tiles of 32 channels per wavefront); every
-// wavefront runs the workgroup's whole share of K.  What bounds it: 1931 rows of 1536 -> 17920
-// run at 0.84 PFLOP/s, half of what the instruction alone reaches, with the conversion of the
-// weights and the way of the rows through LDS in the wavefronts' stream of instructions.
+// wavefront runs the workgroup's whole share of K.  What bounds it: gate | up of 1931 rows, one
+// term, takes 126 us in a prompt, 0.84 PFLOP/s and half of what the instruction alone reaches, with
+// the conversion of the weights and the way of the rows through LDS in the wavefronts' stream of
+// instructions.
 //
 // Rows go through LDS, weights from memory to registers.  Weights are asked for three
 // chunks of 64 k ahead, rows five (two of them in LDS: step c multiplies buffer c % 3, whose
@@ -702,7 +703,8 @@ int launch_tiles(Kernel kernel, const GemmArgs &a, unsigned blocks, hipStream_t 
 // with two workgroups 0.20 + 0.38 L us, one that has its compute unit to itself 0.29 + 0.14 L
 // us (with one channel tile 0.20 + 0.185 L and 0.17 + 0.073 L); a last round that fills less
 // than half runs at the latter.  Fitted to launches of 20 to 1931 rows of 1536, 4096, 8960 and
-// 14336 k, both tiles with every K split: what it picks is 2.2 % off the best on average.
+// 14336 k, both tiles with every K split.  Of 528 launches of 17 to 2048 rows under the profiler its
+// pick is 2.1 (one term) and 1.1 % (three) off the best on average.
 // Microseconds of a product in a prompt of 150 rows, one term (in brackets with a branch at every
 // chunk and its loads at the chunk's start): 1536 -> 2048 10.9 [14.1], 1536 -> 2 x 8960 19.9
 // [22.9], 8960 -> 1536 11.6 [13.0] without the adding of its slices.
