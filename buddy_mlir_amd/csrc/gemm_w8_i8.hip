@@ -372,6 +372,141 @@ __device__ __forceinline__ float4 int_bits(const v16i32 &acc, int q) {
                      __int_as_float(acc[4 * q + 2]), __int_as_float(acc[4 * q + 3]));
 }
 
+constexpr int turn_floats(int span) { return span + 4; } // of a row of the epilogue's tile
+constexpr int turned_bytes(int span) { return kSlices * 32 * turn_floats(span) * 4; }
+
+// The way of a tile's sums out, behind the last barrier of the loop over K (`lds` is free).
+template <int D, int RB, int GP, bool PAIR>
+__device__ __forceinline__ void finish_tile(const GemmI8Args &a, const v16i32 (&acc)[GP][RB][D], unsigned char *lds,
+                                            const float *scale_s, const float *bias_s, const float *step_s,
+                                            int ctile, int rbk, int slice, int g0, int m0, int wave, int lane) {
+  constexpr int kWidth = PAIR ? 16 : 32, kSpan = kWidth * GP, kRows = 32 * RB;
+  constexpr int kTurn = turn_floats(kSpan), kScales = kSlices * 32 * GP;
+  const int col = lane & 31, up = lane >> 5;
+  // A lane holds channels 8 q + 4 up + 0..3, q = 0..3, of row `col` of every tile: stored
+  // as they are, a store instruction would write 32-byte pieces of 32 rows.  Each
+  // wavefront turns its 32 rows around in its own part of LDS (free now: every wavefront
+  // is past the last barrier of the loop) and writes whole row segments.
+  float *tile = reinterpret_cast<float *>(lds) + wave * (32 * kTurn);
+  const int n0 = g0 * kTileN;
+  auto turn_in = [&](int g, int q, float4 v) {
+    *reinterpret_cast<float4 *>(tile + col * kTurn + g * kWidth + 8 * q + 4 * up) = v;
+  };
+  constexpr int kQuads = kSpan / 4; // float4 of a row
+  if (a.slices > 1) {
+    // unscaled sums of this slice, [wavefront][row][channel]; the kernel that adds the
+    // slices finishes the tile
+    const size_t at = ((size_t)(rbk * a.ncols + ctile) * a.slices + slice) * kSlices + wave;
+    float *part = a.partial + at * kRows * kSpan;
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+#pragma unroll
+      for (int g = 0; g < GP; ++g)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const v16i32(&t)[D] = acc[g][rb];
+          float4 o = make_float4(combine<D>(t, 4 * q), combine<D>(t, 4 * q + 1),
+                                 combine<D>(t, 4 * q + 2), combine<D>(t, 4 * q + 3));
+          if constexpr (D == 1) {
+            if (a.int_partials) // exact beyond 2^24: the bits travel as they are
+              o = int_bits(t[0], q);
+          }
+          turn_in(g, q, o);
+        }
+#pragma unroll
+      for (int i = 0; i < kQuads / 2; ++i) {
+        const int idx = lane + 64 * i, row = idx / kQuads, c4 = idx % kQuads;
+        *reinterpret_cast<float4 *>(part + (size_t)(rb * 32 + row) * kSpan + c4 * 4) =
+            *reinterpret_cast<const float4 *>(tile + row * kTurn + c4 * 4);
+      }
+    }
+    return;
+  }
+  const bool vec = (a.ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(a.C) & 15) == 0;
+  const float *scales = scale_s + wave * kSpan;
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    const float row_step = step_s[rb * 32 + col];
+#pragma unroll
+    for (int g = 0; g < GP; ++g)
+#pragma unroll
+      for (int q = 0; q < kWidth / 8; ++q) {
+        const int ch = g * kWidth + 8 * q + 4 * up;
+        const v16i32(&t)[D] = acc[g][rb];
+        const float4 sc = *reinterpret_cast<const float4 *>(scales + ch);
+        const float s[4] = {sc.x, sc.y, sc.z, sc.w};
+        float o[4];
+        if constexpr (PAIR) {
+          const float4 su = *reinterpret_cast<const float4 *>(scales + kScales / 2 + ch);
+          const float s2[4] = {su.x, su.y, su.z, su.w};
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            o[i] = silu_times(scaled<D>(combine<D>(t, 4 * q + i), row_step, s[i]),
+                              scaled<D>(combine<D>(t, 4 * q + 8 + i), row_step, s2[i]));
+        } else {
+          const float4 bb = *reinterpret_cast<const float4 *>(bias_s + wave * kSpan + ch);
+          const float b[4] = {bb.x, bb.y, bb.z, bb.w};
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            o[i] = b[i] + scaled<D>(combine<D>(t, 4 * q + i), row_step, s[i]);
+        }
+        turn_in(g, q, make_float4(o[0], o[1], o[2], o[3]));
+      }
+#pragma unroll
+    for (int i = 0; i < kQuads / 2; ++i) {
+      const int idx = lane + 64 * i, row = idx / kQuads, c4 = idx % kQuads;
+      const float4 o = *reinterpret_cast<const float4 *>(tile + row * kTurn + c4 * 4);
+      const int m = m0 + rb * 32 + row, n = n0 + c4 * 4;
+      if (m >= a.M || n >= a.N)
+        continue;
+      float *cp = a.C + (int64_t)m * a.ldc + n;
+      if (vec && n + 3 < a.N) {
+        float4 q = o;
+        if (a.accumulate) {
+          const float4 p = *reinterpret_cast<const float4 *>(cp);
+          q = make_float4(p.x + q.x, p.y + q.y, p.z + q.z, p.w + q.w);
+        }
+        *reinterpret_cast<float4 *>(cp) = q;
+      } else {
+        const float v[4] = {o.x, o.y, o.z, o.w};
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (n + r < a.N)
+            cp[r] = a.accumulate ? cp[r] + v[r] : v[r];
+      }
+    }
+    if constexpr (D == 1) {
+      if (a.sums) { // the same turn for the integer sums, carried as float bit patterns
+#pragma unroll
+        for (int g = 0; g < GP; ++g)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            turn_in(g, q, int_bits(acc[g][rb][0], q));
+        const bool ivec = (a.N & 3) == 0 && (reinterpret_cast<uintptr_t>(a.sums) & 15) == 0;
+#pragma unroll
+        for (int i = 0; i < kQuads / 2; ++i) {
+          const int idx = lane + 64 * i, row = idx / kQuads, c4 = idx % kQuads;
+          const float4 q = *reinterpret_cast<const float4 *>(tile + row * kTurn + c4 * 4);
+          const v4i32 o = {__float_as_int(q.x), __float_as_int(q.y), __float_as_int(q.z),
+                           __float_as_int(q.w)};
+          const int m = m0 + rb * 32 + row, n = n0 + c4 * 4;
+          if (m >= a.M || n >= a.N)
+            continue;
+          int32_t *cp = a.sums + (int64_t)m * a.N + n;
+          if (ivec) {
+            *reinterpret_cast<v4i32 *>(cp) = o;
+          } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (n + r < a.N)
+                cp[r] = o[r];
+          }
+        }
+      }
+    }
+  }
+}
+
 template <int D, int RB, int GP, bool PAIR>
 __device__ __forceinline__ void multiply_tile(const GemmI8Args &a) {
   constexpr int kWidth = PAIR ? 16 : 32;    // channels of the result per tile
@@ -382,8 +517,7 @@ __device__ __forceinline__ void multiply_tile(const GemmI8Args &a) {
   // a thread's loads of a chunk's rows: 16 bytes of two layers at a time, 8 of an odd last one
   constexpr int kQuad = L / 2, kLoads = (L + 1) / 2;
   constexpr int kBuf = L * 32 * kWideRow;
-  constexpr int kTurn = kSpan + 4;          // floats of a row of the epilogue's tile
-  constexpr int kTurned = kSlices * 32 * kTurn * 4;
+  constexpr int kTurned = turned_bytes(kSpan);
   constexpr int kLds = 3 * kBuf > kTurned ? 3 * kBuf : kTurned;
   constexpr int kScales = kSlices * 32 * GP;
   // chunks of weights and of rows in registers
@@ -574,129 +708,183 @@ __device__ __forceinline__ void multiply_tile(const GemmI8Args &a) {
     }
   }
 
-  // ---- epilogue ---------------------------------------------------------
-  // A lane holds channels 8 q + 4 up + 0..3, q = 0..3, of row `col` of every tile: stored
-  // as they are, a store instruction would write 32-byte pieces of 32 rows.  Each
-  // wavefront turns its 32 rows around in its own part of LDS (free now: every wavefront
-  // is past the last barrier of the loop) and writes whole row segments.
-  float *tile = reinterpret_cast<float *>(lds) + wave * (32 * kTurn);
-  const int n0 = g0 * kTileN;
-  auto turn_in = [&](int g, int q, float4 v) {
-    *reinterpret_cast<float4 *>(tile + col * kTurn + g * kWidth + 8 * q + 4 * up) = v;
-  };
-  constexpr int kQuads = kSpan / 4; // float4 of a row
-  if (a.slices > 1) {
-    // unscaled sums of this slice, [wavefront][row][channel]; the kernel that adds the
-    // slices finishes the tile
-    const size_t at = ((size_t)(rbk * a.ncols + ctile) * a.slices + slice) * kSlices + wave;
-    float *part = a.partial + at * kRows * kSpan;
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-#pragma unroll
-      for (int g = 0; g < GP; ++g)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const v16i32(&t)[D] = acc[g][rb];
-          float4 o = make_float4(combine<D>(t, 4 * q), combine<D>(t, 4 * q + 1),
-                                 combine<D>(t, 4 * q + 2), combine<D>(t, 4 * q + 3));
-          if constexpr (D == 1) {
-            if (a.int_partials) // exact beyond 2^24: the bits travel as they are
-              o = int_bits(t[0], q);
-          }
-          turn_in(g, q, o);
-        }
-#pragma unroll
-      for (int i = 0; i < kQuads / 2; ++i) {
-        const int idx = lane + 64 * i, row = idx / kQuads, c4 = idx % kQuads;
-        *reinterpret_cast<float4 *>(part + (size_t)(rb * 32 + row) * kSpan + c4 * 4) =
-            *reinterpret_cast<const float4 *>(tile + row * kTurn + c4 * 4);
-      }
-    }
+  finish_tile<D, RB, GP, PAIR>(a, acc, lds, scale_s, bias_s, step_s, ctile, rbk, slice, g0, m0, wave, lane);
+}
+
+// The same product for tiles of many sums, two workgroups to a compute unit: two wavefronts on a
+// SIMD have 256 registers each, of which the sums of 64 rows x 64 channels in three planes are
+// 192, so the rows come from memory to LDS past the registers, three chunks ahead, and the weights
+// half a chunk at a time, three of them ahead.  One workgroup loads and stores beside the
+// products of the other.
+//
+// What bounds it: power.  gate | up of 1931 rows with three planes takes 146 us (the same tile
+// alone on its compute unit, rows through registers, 180; 32 rows x 256 channels two to a compute
+// unit 170), and 108 where rows and weights are zero: the clock falls from 2.3 to below 1.8 GHz
+// with what the matrix cores draw.  Conflicts in LDS (a third of its cycles with pieces permuted by
+// r / 2) or none, and either order of the products of a fragment, made no difference.
+//
+// A plane's block lies in LDS as it lies in memory but for the four 16-byte pieces of a row, which
+// are permuted by the row's number: piece p of row r is where p ^ (r / 4 % 4) would be, and the
+// fragment reads of sixteen rows in a line meet every bank once.
+//
+// The loads into LDS are not the compiler's: landed<N> waits until at most N loads are under way
+// that were issued behind the ones asked about.  Every step issues kDma loads into LDS and 2 GP of
+// weights in that order; the asm statements may write any memory as far as the compiler knows, so
+// no load of weights moves across one of them.
+__device__ __forceinline__ void load_1k_to_lds(const void *base, unsigned lane_offset, unsigned to) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_offset), "s"(base),
+               "s"(to)
+               : "memory", "m0");
+}
+template <int N> __device__ __forceinline__ void landed() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// the tiles of gemm_w8_i8_tall_kernel that go this way
+constexpr bool tall_shares(int D, int GP) { return D >= 2 && GP == 2; }
+
+template <int D, int RB, int GP, bool PAIR>
+__device__ __forceinline__ void multiply_block(const GemmI8Args &a) {
+  constexpr int kWidth = PAIR ? 16 : 32, kSpan = kWidth * GP, kRows = 32 * RB, L = D * RB;
+  constexpr int kThreads = kSlices * kWave;
+  constexpr int kRing = 4;                    // chunks of rows in LDS, half chunks of weights in registers
+  constexpr int kBuf = L * kPlaneBlock;
+  constexpr int kDma = 2 * L / kSlices;       // a wavefront's loads of 1 KiB of a chunk's rows
+  static_assert(2 * L % kSlices == 0 && (2 * L) % 4 == 0, "every wavefront brings as much; fragment slots repeat");
+  constexpr int kLds = kRing * kBuf > turned_bytes(kSpan) ? kRing * kBuf : turned_bytes(kSpan);
+  constexpr int kScales = kSlices * 32 * GP;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[kLds];
+  __shared__ __attribute__((aligned(16))) float scale_s[kScales], bias_s[PAIR ? 4 : kScales];
+  __shared__ float step_s[kRows];
+  const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, up = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int unit, rbk;
+  if (!place_tile(a.ncols * a.slices, a.row_tiles, a.panel, unit, rbk))
     return;
-  }
-  const bool vec = (a.ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(a.C) & 15) == 0;
-  const float *scales = scale_s + wave * kSpan;
+  const int ctile = unit % a.ncols, slice = unit / a.ncols;
+  const int m0 = rbk * kRows;
+  const int half_groups = a.groups / 2; // PAIR only
+  const int glast = PAIR ? half_groups - 1 : a.groups - 1;
+  const int g0 = (ctile * kSlices + wave) * (kSpan / 16);
+  const int cb = slice * a.chunks_per_slice;
+  const int nch = min(a.chunks_per_slice, a.chunks - cb);
+
+  // weights: a base per channel tile, and how far from it this lane's group lies
+  const char *wb[GP];
+  unsigned woff[GP];
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {
-    const float row_step = step_s[rb * 32 + col];
+  for (int g = 0; g < GP; ++g) {
+    const int second = (lane >> 4) & 1, first = min(PAIR ? g0 + g : g0 + 2 * g, glast);
+    const int gg = PAIR ? first + second * half_groups : min(g0 + 2 * g + second, glast);
+    wb[g] = reinterpret_cast<const char *>(a.W) + ((size_t)first * a.chunks + cb) * 1024;
+    woff[g] = (unsigned)(gg - first) * (unsigned)a.chunks * 1024u + (unsigned)(up * 16 + (lane & 15)) * 16u;
+  }
+  v4i32 wr[kRing][GP];
+  auto fetch_w = [&](int c, int half, int g, v4i32 &w) {
+    // a scalar base: 64-bit addresses of every lane would take registers there are not
+    const uintptr_t at = reinterpret_cast<uintptr_t>(wb[g]) + (size_t)min(c, nch - 1) * 1024 + half * 512;
+    const uintptr_t base = (uintptr_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)at) |
+                           (uintptr_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(at >> 32)) << 32;
+    w = *(const __attribute__((address_space(1))) v4i32 *)((const __attribute__((address_space(1))) char *)base + woff[g]);
+  };
+  // rows: 1 KiB `i` of this wavefront is rows 16 (j % 2) .. + 15 of layer j / 2, j = 4 i + wave
+  const unsigned lds0 = (unsigned)__builtin_amdgcn_readfirstlane(
+      (int)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds);
+  const unsigned row_off = (unsigned)(lane >> 2) * kTileK + (unsigned)((lane & 3) ^ (lane >> 4)) * 16u;
+  const int8_t *rows_at[kDma];
+#pragma unroll
+  for (int i = 0; i < kDma; ++i) {
+    const int j = i * kSlices + wave, l = j / 2;
+    const int block = min(m0 / 32 + l / D, a.Mp / 32 - 1);
+    rows_at[i] = a.planes + (((size_t)block * a.chunks + cb) * D + l % D) * kPlaneBlock + j % 2 * 1024;
+  }
+  auto bring = [&](int c, int buf, int i) {
+    load_1k_to_lds(rows_at[i] + (size_t)min(c, nch - 1) * (D * kPlaneBlock), row_off,
+                   lds0 + buf * kBuf + (i * kSlices + wave) * 1024);
+  };
+#pragma unroll
+  for (int c = 0; c < kRing - 1; ++c)
+#pragma unroll
+    for (int i = 0; i < kDma; ++i)
+      bring(c, c, i);
+#pragma unroll
+  for (int h = 0; h < kRing - 1; ++h)
 #pragma unroll
     for (int g = 0; g < GP; ++g)
-#pragma unroll
-      for (int q = 0; q < kWidth / 8; ++q) {
-        const int ch = g * kWidth + 8 * q + 4 * up;
-        const v16i32(&t)[D] = acc[g][rb];
-        const float4 sc = *reinterpret_cast<const float4 *>(scales + ch);
-        const float s[4] = {sc.x, sc.y, sc.z, sc.w};
-        float o[4];
-        if constexpr (PAIR) {
-          const float4 su = *reinterpret_cast<const float4 *>(scales + kScales / 2 + ch);
-          const float s2[4] = {su.x, su.y, su.z, su.w};
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            o[i] = silu_times(scaled<D>(combine<D>(t, 4 * q + i), row_step, s[i]),
-                              scaled<D>(combine<D>(t, 4 * q + 8 + i), row_step, s2[i]));
-        } else {
-          const float4 bb = *reinterpret_cast<const float4 *>(bias_s + wave * kSpan + ch);
-          const float b[4] = {bb.x, bb.y, bb.z, bb.w};
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            o[i] = b[i] + scaled<D>(combine<D>(t, 4 * q + i), row_step, s[i]);
-        }
-        turn_in(g, q, make_float4(o[0], o[1], o[2], o[3]));
-      }
-#pragma unroll
-    for (int i = 0; i < kQuads / 2; ++i) {
-      const int idx = lane + 64 * i, row = idx / kQuads, c4 = idx % kQuads;
-      const float4 o = *reinterpret_cast<const float4 *>(tile + row * kTurn + c4 * 4);
-      const int m = m0 + rb * 32 + row, n = n0 + c4 * 4;
-      if (m >= a.M || n >= a.N)
-        continue;
-      float *cp = a.C + (int64_t)m * a.ldc + n;
-      if (vec && n + 3 < a.N) {
-        float4 q = o;
-        if (a.accumulate) {
-          const float4 p = *reinterpret_cast<const float4 *>(cp);
-          q = make_float4(p.x + q.x, p.y + q.y, p.z + q.z, p.w + q.w);
-        }
-        *reinterpret_cast<float4 *>(cp) = q;
-      } else {
-        const float v[4] = {o.x, o.y, o.z, o.w};
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (n + r < a.N)
-            cp[r] = a.accumulate ? cp[r] + v[r] : v[r];
-      }
+      fetch_w(h / 2, h % 2, g, wr[h][g]);
+  if (a.slices == 1) {
+    const int n0 = ctile * kSlices * kSpan;
+    for (int i = tid; i < kScales; i += kThreads) {
+      const int mtx = PAIR ? i / (kScales / 2) : 0, n = n0 + (PAIR ? i % (kScales / 2) : i);
+      scale_s[i] = n < a.N ? a.scale[(size_t)mtx * a.N + n] : 0.f;
+      if constexpr (!PAIR)
+        bias_s[i] = a.bias && n < a.N ? a.bias[n] : 0.f;
     }
-    if constexpr (D == 1) {
-      if (a.sums) { // the same turn for the integer sums, carried as float bit patterns
+    for (int i = tid; i < kRows; i += kThreads)
+      step_s[i] = m0 + i < a.M ? a.steps[m0 + i] : 0.f;
+  }
+
+  v16i32 acc[GP][RB][D];
 #pragma unroll
-        for (int g = 0; g < GP; ++g)
+  for (int g = 0; g < GP; ++g)
 #pragma unroll
-          for (int q = 0; q < 4; ++q)
-            turn_in(g, q, int_bits(acc[g][rb][0], q));
-        const bool ivec = (a.N & 3) == 0 && (reinterpret_cast<uintptr_t>(a.sums) & 15) == 0;
+    for (int l = 0; l < L; ++l)
+      acc[g][l / D][l % D] = v16i32{};
+
+  landed<(kRing - 1) * GP + kDma>(); // chunks 0 and 1
+  __syncthreads();
+  const int frag_at[2] = {col * kTileK + (up ^ ((col >> 2) & 3)) * 16,
+                          col * kTileK + ((2 + up) ^ ((col >> 2) & 3)) * 16};
+  v4i32 frag[4];
+  // sub-step u of a chunk: layer u % L, k half u / L
+  auto load_frag = [&](int buf, int u, v4i32 &f) {
+    f = *reinterpret_cast<const v4i32 *>(lds + buf * kBuf + u % L * kPlaneBlock + frag_at[u / L]);
+  };
+  load_frag(0, 0, frag[0]);
+  load_frag(0, 1, frag[1]);
+  // step c = c0 + slot: chunk c in buffer `slot`, chunk c + 3 into the one before it
+  auto step = [&](int c0, auto slot) {
+    constexpr int sl = slot;
+    const int c = c0 + sl;
 #pragma unroll
-        for (int i = 0; i < kQuads / 2; ++i) {
-          const int idx = lane + 64 * i, row = idx / kQuads, c4 = idx % kQuads;
-          const float4 q = *reinterpret_cast<const float4 *>(tile + row * kTurn + c4 * 4);
-          const v4i32 o = {__float_as_int(q.x), __float_as_int(q.y), __float_as_int(q.z),
-                           __float_as_int(q.w)};
-          const int m = m0 + rb * 32 + row, n = n0 + c4 * 4;
-          if (m >= a.M || n >= a.N)
-            continue;
-          int32_t *cp = a.sums + (int64_t)m * a.N + n;
-          if (ivec) {
-            *reinterpret_cast<v4i32 *>(cp) = o;
-          } else {
+    for (int u = 0; u < 2 * L; ++u) {
+      load_frag(u + 2 < 2 * L ? sl : (sl + 1) % kRing, (u + 2) % (2 * L), frag[(u + 2) & 3]);
+      const int h = u / L, ahead = h + kRing - 1;
+      if (u < kDma)
+        bring(c + kRing - 1, (sl + kRing - 1) % kRing, u);
+      const int g = u - kDma - h * (L - kDma); // behind those
+      if (g >= 0 && g < GP)
+        fetch_w(c + ahead / 2, ahead % 2, g, wr[(2 * sl + ahead) % kRing][g]);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-              if (n + r < a.N)
-                cp[r] = o[r];
-          }
-        }
-      }
+      for (int g = 0; g < GP; ++g)
+        acc[g][u % L / D][u % D] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wr[(2 * sl + h) % kRing][g], frag[u & 3],
+                                                                         acc[g][u % L / D][u % D], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    landed<4 * GP + kDma>(); // chunk c + 2, issued at the start of step c - 1
+    __syncthreads();
+  };
+  using std::integral_constant;
+  int c0 = 0;
+  for (; c0 + kRing <= nch; c0 += kRing) {
+    step(c0, integral_constant<int, 0>{});
+    step(c0, integral_constant<int, 1>{});
+    step(c0, integral_constant<int, 2>{});
+    step(c0, integral_constant<int, 3>{});
+  }
+  static_assert(kRing == 4, "a round is written out");
+  if (c0 < nch) {
+    step(c0, integral_constant<int, 0>{});
+    if (c0 + 1 < nch) {
+      step(c0, integral_constant<int, 1>{});
+      if (c0 + 2 < nch)
+        step(c0, integral_constant<int, 2>{});
     }
   }
+  landed<0>(); // of the chunks asked for beyond the last: the tile's way out goes through their LDS
+  __syncthreads();
+  finish_tile<D, RB, GP, PAIR>(a, acc, lds, scale_s, bias_s, step_s, ctile, rbk, slice, g0, m0, wave, lane);
 }
 
 // What a wavefront needs before its first fetch arrives in SGPRs (this file is built
@@ -729,9 +917,13 @@ __global__ void __launch_bounds__(kSlices *kWave) gemm_w8_i8_wide_kernel(BH_I8_L
   multiply_tile<D, wide_blocks(D), 2, PAIR>(a);
 }
 template <int D, int RB, int GP, bool PAIR>
-__global__ void __launch_bounds__(kSlices *kWave) gemm_w8_i8_tall_kernel(BH_I8_LEADING) {
+__global__ void __launch_bounds__(kSlices *kWave, tall_shares(D, GP) ? 2 : 1)
+gemm_w8_i8_tall_kernel(BH_I8_LEADING) {
   BH_I8_TAKE
-  multiply_tile<D, RB, GP, PAIR>(a);
+  if constexpr (tall_shares(D, GP))
+    multiply_block<D, RB, GP, PAIR>(a);
+  else
+    multiply_tile<D, RB, GP, PAIR>(a);
 }
 
 // Where the sums of row m, channels n.. of the first K slice lie.
@@ -1143,23 +1335,19 @@ namespace {
 // tile's registers leave room for one.  A chunk of 64 k takes a workgroup that has its
 // compute unit to itself `alone`, two that share one `both`, each beside a fixed part; a last
 // round that fills less than half runs at the former.  Fitted to
-// launches of 20 to 1931 rows of 1536, 4096, 8960 and 14336 k, every tile with every K split.  Of 264
-// launches of 17 to 2048 rows under the profiler its pick is 1.7 (three planes) and 2.8 % (two) off the
-// best on average.
-// Microseconds of a product with three planes in a prompt (in brackets with rows of K bytes per
-// plane, a branch at every chunk and its loads all at the chunk's start):
-//   gate | up, 1536 -> 2 x 8960: 27 rows 12.4 [14.4], 512: 54 [59], 1931: 171.5 [182]
-//   down, 8960 -> 1536: 27 rows 5.7 [6.5], 512: 25 [30], 1931: 81.5 [89]
-//   q|k|v, 1536 -> 2048: 512 rows 11.6 [14.5]
-//   one plane, 1536 -> 8960: 512 rows 19.1 [20.3]
-// The card holds its clock at 1.9 GHz under the large ones, whose matrix pipes are half busy:
-// without any loads in the loop gate | up of 1931 rows takes 119 us, with loads that all hit the
-// L1 157.
+// launches of 27 to 1931 rows of 1536, 4096, 8960 and 14336 k, every tile with every K split: over
+// 120 such products, conversion and slices included, the picks are 0.4 (three planes) and 0.9 % (two)
+// off the best on average.
+// Microseconds of a product with three planes in a prompt (in brackets with tiles of 64 x 256 that
+// fill a compute unit alone, which then were the pick for down at 512 rows only):
+//   gate | up, 1536 -> 2 x 8960: 27 rows 12.4, 512: 48.8 [52.4], 1931: 146 [164]
+//   down, 8960 -> 1536: 27 rows 5.7, 512: 24.7 [24.9], 1931: 71.5 [78.5]
+//   q|k|v, 1536 -> 2048: 512 rows 11.6
+//   one plane, 1536 -> 8960: 512 rows 19.1
 // (gate | up of 28 rows with weights from memory: two channel tiles 15.4, one 11.4, for which twice
 // the compute units ask.)
-// Tiles that fill a compute unit alone have coarser rounds and use an operand more often
-// (64 rows x 256 channels: long sums and many rows; 32 x 640 and 96 x 256: row counts for
-// which they come to a whole round and the others to a little more than one).
+// 64 x 256 and 96 x 256 use an operand more often: long sums and many rows; 32 x 640: row counts for
+// which it comes to a whole round and the others to a little more than one.
 struct TileShape {
   int rb, gp;           // blocks of 32 rows; tiles of 32 channels per wavefront
   bool shares;          // two workgroups to a compute unit
@@ -1171,12 +1359,12 @@ constexpr TileShape kTiles1[] = {{1, 1, true, 0.21, 4.5, 0.285, 4.5},
                                  {3, 2, true, 0.39, 5.0, 0.66, 4.0}};
 constexpr TileShape kTiles2[] = {{1, 1, true, 0.194, 4.15, 0.379, 3.85},
                                  {wide_blocks(2), 2, true, 0.303, 5.0, 0.51, 6.05},
-                                 {2, 2, false, 0.446, 7.1, 0, 0},
+                                 {2, 2, true, 0.493, 6.2, 0.969, 2.28},
                                  {1, 3, true, 0.428, 6.0, 0.913, 10.0},
-                                 {3, 2, false, 0.621, 9.9, 0, 0}};
+                                 {3, 2, true, 0.656, 5.56, 1.259, 3.1}};
 constexpr TileShape kTiles3[] = {{1, 1, true, 0.216, 3.2, 0.455, 4.5},
                                  {wide_blocks(3), 2, true, 0.35, 4.7, 0.676, 4.0},
-                                 {2, 2, false, 0.591, 6.3, 0, 0},
+                                 {2, 2, true, 0.546, 5.29, 1.002, 6.81},
                                  {1, 5, false, 0.855, 7.0, 0, 0}};
 
 struct TilePlan {

@@ -411,3 +411,14 @@ def test_prefill_attention_and_no_unlisted_family(bh, oracle):
              "gemm_w8_i8_kernel", "gemm_w8_bf16_wide_kernel", "gemm_w8_bf16_kernel",
              "attn_prefill_kernel", "gemv_w8a32_digits_kernel")
     assert {name.split("<")[0] for name in report(bh)} == set(known)
+
+
+# The tiles of two and three row blocks whose rows come past the registers: one to eight chunks of
+# 64 k (a ring of four, its rounds and every rest of one), the last one whole or not
+@pytest.mark.parametrize("variant,M,K,N", [
+    ((3, 2, 2, 0), 257, 40, 15001), *(((3, 2, 2, 0), 385, k, 12281) for k in (65, 192, 250, 300, 384, 440, 500)),
+    ((3, 2, 2, 1), 257, 130, 8976), ((3, 2, 2, 1), 257, 310, 8976),
+    ((2, 2, 2, 0), 257, 64, 15001), ((2, 2, 2, 0), 257, 190, 15001), ((2, 2, 2, 0), 257, 330, 15001),
+    ((2, 3, 2, 0), 321, 128, 8873), ((2, 3, 2, 0), 641, 256, 12281), ((2, 3, 2, 0), 641, 400, 12281)])
+def test_tall_int8_tiles_of_few_chunks(bh, oracle, variant, M, K, N):
+    test_tall_int8_tiles(bh, oracle, variant, M, K, N)
