@@ -309,10 +309,14 @@ rows_gemm_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int columns
 // exact, the sums f32: three matrix instructions at sixteen times the rate of the f32
 // ones.
 //
-// What bounds it: a step of 128 rows x 256 channels is 1024 cycles of matrix instructions
-// and takes some 1620 at 2.0 GHz, with the loads of the rows and their way into LDS in the
-// wavefront's one stream of instructions, and the clock falls with the power the matrix
-// cores draw (2.4 to 1.9 GHz).  Against 16 x 16 tiles (us, rows x K x channels):
+// What bounds it: on tiles of 128 bfloat16 rows, two to a compute unit, a chip full of them
+// multiplies at 1.0 PFLOP/s however long K is (large plain products reach 1.15), which is what
+// the power allows: the clock falls with what the matrix cores draw.  A round of 24 steps is
+// 43 us of that and 15 of its beginning and its activation and stores.  With the rows through
+// registers, one such tile to a compute unit and its loads between its products: gate | up of 16
+// experts, 2048 x 4 rows of 1536 -> 2 x 1792, 148 us, now 120; 777 x 1536 -> 2 x 8960 68, now 58.
+// (Rows past the registers for the tiles of 32 and 64 rows too: 8960 -> 1536 at 777 rows 47 us
+// whole, 56 so; 1536 -> 1536 of 400 rows 8.1 and 8.5.)  Against 16 x 16 tiles (us, rows x K x channels):
 //   bfloat16  2048 x 4096 x 4096   82.0 -> 75.2    f32   523 -> 216
 //             2048 x 1536 x 7168   72.4 -> 66.7          341 -> 154
 //              777 x 8960 x 1536   60.4 -> 41.3          307 -> 115
@@ -361,9 +365,23 @@ __device__ __forceinline__ f32x16 mfma_bf16_wide(uint4 a, uint4 b, f32x16 c) {
                                                  __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
+// 1 KiB from memory past the registers into LDS: a lane's 16 bytes at `from` to `to` + 16 lane.  Not
+// the compiler's load: landed<N> waits until at most N loads are under way that were issued behind
+// the ones asked about.  No load moves across one of these statements, which may write any memory
+// as far as the compiler knows.
+__device__ __forceinline__ void load_1k_to_lds(const void *from, unsigned to) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(to) : "memory", "m0");
+}
+template <int N> __device__ __forceinline__ void landed() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// Tiles of 128 bfloat16 rows run two to a compute unit.
+template <typename T, int RT> constexpr bool kBrings = sizeof(T) == 2 && RT == 4;
+
 template <typename T, int RT, int GT, int OUT, bool GROUPED, bool SLICED>
-__global__ void __launch_bounds__(kGemmThreads)
-rows_gemm_wide_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int columns, int row_blocks,
+__global__ void __launch_bounds__(kGemmThreads, (kBrings<T, RT> ? 2 : 1))
+rows_gemm_wide_kernel(const uint4 *W, int ktiles, int steps, int columns, int row_blocks,
                       DevOf<SLICED> a) {
   constexpr bool kPair = OUT == kOutExpertAct;
   constexpr int kTilesOut = kPair ? GT / 2 : GT; // 32-channel tiles of the result per wavefront
@@ -374,7 +392,8 @@ rows_gemm_wide_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int co
   constexpr int kLoads = kRows * kRowRuns / kGemmThreads;
   constexpr int kPlane = kRows * kLdsRow, kBuf = kTerms * kPlane;
   static_assert(kRows * kRowRuns % kGemmThreads == 0, "every thread moves the same number of runs");
-  __shared__ __attribute__((aligned(16))) unsigned char lds[3 * kBuf];
+  constexpr int kBrought = kRows * kRowBytes; // of a step's rows, where they come past the registers
+  __shared__ __attribute__((aligned(16))) unsigned char lds[kBrings<T, RT> ? 4 * kBrought : 3 * kBuf];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
@@ -405,24 +424,6 @@ rows_gemm_wide_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int co
     a.C = static_cast<float *>(a.C) + blockIdx.z * a.slice_stride;
   }
 
-  // the runs this thread moves: fixed rows, k advancing by the step
-  const T *src[kLoads];
-  int lds_at[kLoads];
-  const int run_k = tid % kRowRuns * kRunElems;
-#pragma unroll
-  for (int i = 0; i < kLoads; ++i) {
-    const int r = (i * kGemmThreads + tid) / kRowRuns;
-    lds_at[i] = r * kLdsRow + run_k * 2;
-    // a row past the end repeats the last one: its column of the result is not stored
-    const int lr = min(row0 + r, rows - 1);
-    int pr;
-    if constexpr (GROUPED)
-      pr = list[lr] / a.list_div;
-    else
-      pr = (a.ring_base + lr) & a.ring_mask;
-    src[i] = static_cast<const T *>(a.A) + (int64_t)pr * a.lda + first * kWideK;
-  }
-
   const int ch0 = (bx * 4 + wave) * kTilesOut * 2; // first channel group of this wavefront
   const uint4 *wp[GT];
 #pragma unroll
@@ -432,44 +433,6 @@ rows_gemm_wide_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int co
     wp[g] = W + ((int64_t)(mat * a.groups + gg) * ktiles + first * 2) * 64 + (lane >> 5) * 16 + (lane & 15);
   }
 
-  uint4 wr[4][GT * 4], xr[4][kLoads];
-  constexpr int kFetches = GT * 4 + kLoads; // loads of a step
-  const int last_run = (K - 1) / kRunElems * kRunElems;
-  const bool ragged = K % kWideK != 0; // the last step reaches past K
-  auto fetch_w = [&](int s, uint4 (&w)[GT * 4]) {
-    const int t = min(s, steps - 1) * 2;
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int g = 0; g < GT; ++g)
-        w[g * 4 + u] = wp[g][(int64_t)(t + u / 2) * 64 + (u & 1) * 32];
-  };
-  auto fetch_x = [&](int s, uint4 (&x)[kLoads]) {
-    const int k = min(min(s, steps - 1) * kWideK + run_k, last_run);
-#pragma unroll
-    for (int i = 0; i < kLoads; ++i)
-      x[i] = *reinterpret_cast<const uint4 *>(src[i] + k);
-  };
-  auto put_x = [&](int s, uint4 (&x)[kLoads], unsigned char *buf) {
-    if (ragged && s == steps - 1) {
-#pragma unroll
-      for (int i = 0; i < kLoads; ++i)
-        x[i] = keep_run<T>(x[i], K - s * kWideK - run_k);
-    }
-#pragma unroll
-    for (int i = 0; i < kLoads; ++i) {
-      if constexpr (kTerms == 1) {
-        *reinterpret_cast<uint4 *>(buf + lds_at[i]) = x[i];
-      } else {
-        uint2 t[3];
-        split3(x[i], t);
-#pragma unroll
-        for (int p = 0; p < 3; ++p)
-          *reinterpret_cast<uint2 *>(buf + p * kPlane + lds_at[i]) = t[p];
-      }
-    }
-  };
-
   f32x16 acc[GT][RT];
 #pragma unroll
   for (int g = 0; g < GT; ++g)
@@ -477,90 +440,254 @@ rows_gemm_wide_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int co
     for (int r = 0; r < RT; ++r)
       acc[g][r] = f32x16{};
 
-  const int frag_at = (lane & 31) * kLdsRow + (lane >> 5) * 16;
-  uint4 frag[2][kTerms][RT];
-  auto load_frag = [&](const unsigned char *buf, int u, uint4 (&f)[kTerms][RT]) {
+  if constexpr (kBrings<T, RT>) {
+    // Rows come to LDS past the registers, three steps ahead, weights a quarter of a step (16 k) at
+    // a time, seven of them ahead: 256 registers a wavefront.  LDS holds rows of 128 bytes whose
+    // eight 16-byte pieces are permuted by the row's number (piece p of row r where p ^ (r / 2 % 8)
+    // would be), so that the fragments of sixteen rows in a line meet every bank once.
+    // landed<N>: see gemm_w8_i8.hip's tiles of this kind; a step issues GT loads
+    // of weights in each quarter and RT into LDS, one ahead of those of each of its first quarters.  What K has beyond whole steps follows at the end, on its own.
+    constexpr int kAhead = 7, kSlots = 8;
+    const int whole = min(steps, K / kWideK);
+    const int f = ((wave & 1) * 4 + (lane >> 4)) & 7;
+    const char *src[RT];
 #pragma unroll
-    for (int p = 0; p < kTerms; ++p)
+    for (int i = 0; i < RT; ++i) {
+      const int lr = min(row0 + (i * 4 + wave) * 8 + (lane >> 3), rows - 1);
+      int pr;
+      if constexpr (GROUPED)
+        pr = list[lr] / a.list_div;
+      else
+        pr = (a.ring_base + lr) & a.ring_mask;
+      src[i] = static_cast<const char *>(a.A) + ((int64_t)pr * a.lda + first * kWideK) * 2 + ((lane & 7) ^ f) * 16;
+    }
+    const unsigned lds0 = (unsigned)__builtin_amdgcn_readfirstlane(
+        (int)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds);
+    auto bring = [&](int s, int buf, int i) {
+      load_1k_to_lds(src[i] + (int64_t)min(s, whole - 1) * kRowBytes, lds0 + buf * kBrought + (i * 4 + wave) * 1024);
+    };
+    uint4 wr[kSlots][GT];
+    auto fetch = [&](int q, uint4 (&w)[GT]) { // quarter q of all
+#pragma unroll
+      for (int g = 0; g < GT; ++g)
+        w[g] = wp[g][(int64_t)min(q, 4 * whole - 1) * 32];
+    };
+    int frag_at[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      frag_at[u] = (lane & 31) * kRowBytes + ((2 * u + (lane >> 5)) ^ ((lane >> 1) & 7)) * 16;
+    uint4 frag[2][RT];
+    auto load_frag = [&](int buf, int u, uint4 (&x)[RT]) {
 #pragma unroll
       for (int r = 0; r < RT; ++r)
-        f[p][r] = *reinterpret_cast<const uint4 *>(buf + p * kPlane + frag_at + r * 32 * kLdsRow + u * 32);
-  };
-
-  // Step s multiplies buffer s % 3, whose first fragments were read during step s - 1, and
-  // fills buffer (s + 2) % 3, last read before the previous barrier.
-  unsigned char *cur = lds, *next = lds + kBuf, *fill = lds + 2 * kBuf;
-  fetch_x(0, xr[0]);
-  fetch_x(1, xr[1]);
-  fetch_w(0, wr[0]);
-  fetch_x(2, xr[2]);
-  fetch_w(1, wr[1]);
-  fetch_x(3, xr[3]);
-  fetch_w(2, wr[2]);
-  put_x(0, xr[0], cur);
-  put_x(1, xr[1], next);
-  fetch_x(4, xr[0]);
-  __syncthreads();
-  load_frag(cur, 0, frag[0]);
-  auto step = [&](int s, uint4 (&w)[GT * 4], uint4 (&w_new)[GT * 4], uint4 (&x)[kLoads],
-                  uint4 (&x_new)[kLoads]) {
-    const int wt = min(s + 3, steps - 1) * 2, xk = min(min(s + 5, steps - 1) * kWideK + run_k, last_run);
+        x[r] = *reinterpret_cast<const uint4 *>(lds + buf * kBrought + r * 32 * kRowBytes + frag_at[u]);
+    };
+    auto multiply = [&](const uint4 (&w)[GT], const uint4 (&x)[RT]) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      // the next fragments are asked for ahead of the products that cover their way, and
-      // stay there: left to itself the scheduler moves them to their use
-      load_frag(u < 3 ? cur : next, (u + 1) & 3, frag[(u + 1) & 1]);
-      // Of a tile that has its compute unit to itself the step's loads go evenly between its
-      // products, weights first (gate | up of 16 experts, 2048 x 4 rows of 1536 -> 2 x 1792: 158
-      // us with all at once, 148.5 so); of the others, which hide each other's, in two parts (90.4
-      // and 91.4 for the experts' way back).
-      if constexpr (RT == 4) {
+      for (int g = 0; g < GT; ++g)
 #pragma unroll
-        for (int i = u * kFetches / 4; i < (u + 1) * kFetches / 4; ++i) {
-          if (i < GT * 4) {
-            const int g = i % GT, q = i / GT;
-            w_new[g * 4 + q] = wp[g][(int64_t)(wt + q / 2) * 64 + (q & 1) * 32];
-          } else {
-            x_new[i - GT * 4] = *reinterpret_cast<const uint4 *>(src[i - GT * 4] + xk);
-          }
+        for (int r = 0; r < RT; ++r)
+          acc[g][r] = mfma_bf16_wide(w[g], x[r], acc[g][r]);
+    };
+    if (whole > 0) {
+#pragma unroll
+      for (int s = 0; s < 3; ++s)
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+          bring(s, s, i);
+#pragma unroll
+      for (int q = 0; q < kAhead; ++q)
+        fetch(q, wr[q]);
+      landed<RT + kAhead * GT>(); // steps 0 and 1
+      __syncthreads();
+      load_frag(0, 0, frag[0]);
+      // step s0 + slot: from buffer `slot`; step s + 3 goes into the one before it
+      auto step = [&](int s0, auto slot) {
+        constexpr int sl = slot;
+        const int s = s0 + sl;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          load_frag(u < 3 ? sl : (sl + 1) & 3, (u + 1) & 3, frag[(u + 1) & 1]);
+          bring(s + 3, (sl + 3) & 3, u);
+          fetch(4 * s + u + kAhead, wr[(4 * sl + u + kAhead) % kSlots]);
+          __builtin_amdgcn_sched_barrier(0);
+          multiply(wr[(4 * sl + u) % kSlots], frag[u & 1]);
+          __builtin_amdgcn_sched_barrier(0);
         }
-      } else {
+        landed<GT + 4 * (1 + GT)>(); // step s + 2, whose last load is in quarter 3 of step s - 1
+        __syncthreads();
+      };
+      using std::integral_constant;
+      int s = 0;
+      for (; s + 4 <= whole; s += 4) {
+        step(s, integral_constant<int, 0>{});
+        step(s, integral_constant<int, 1>{});
+        step(s, integral_constant<int, 2>{});
+        step(s, integral_constant<int, 3>{});
+      }
+      if (s < whole) {
+        step(s, integral_constant<int, 0>{});
+        if (s + 1 < whole) {
+          step(s, integral_constant<int, 1>{});
+          if (s + 2 < whole)
+            step(s, integral_constant<int, 2>{});
+        }
+      }
+      landed<0>(); // steps asked for beyond the last
+      __syncthreads();
+    }
+    if (whole < steps) { // the rest of K
+      const int r0 = tid / kRowRuns, q = tid % kRowRuns, k = whole * kWideK + q * kRunElems;
+      const int last_run = (K - 1) / kRunElems * kRunElems;
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i) {
+        const int r = r0 + i * (kGemmThreads / kRowRuns), lr = min(row0 + r, rows - 1);
+        int pr;
+        if constexpr (GROUPED)
+          pr = list[lr] / a.list_div;
+        else
+          pr = (a.ring_base + lr) & a.ring_mask;
+        const T *p = static_cast<const T *>(a.A) + (int64_t)pr * a.lda + first * kWideK;
+        const uint4 x = keep_run<T>(*reinterpret_cast<const uint4 *>(p + min(k, last_run)), K - k);
+        *reinterpret_cast<uint4 *>(lds + r * kRowBytes + (q ^ (r >> 1 & 7)) * 16) = x;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        uint4 w[GT];
+#pragma unroll
+        for (int g = 0; g < GT; ++g)
+          w[g] = wp[g][(int64_t)(4 * whole + u) * 32];
+        load_frag(0, u, frag[0]);
+        multiply(w, frag[0]);
+      }
+    }
+  } else {
+    // the runs this thread moves: fixed rows, k advancing by the step
+    const T *src[kLoads];
+    int lds_at[kLoads];
+    const int run_k = tid % kRowRuns * kRunElems;
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const int r = (i * kGemmThreads + tid) / kRowRuns;
+      lds_at[i] = r * kLdsRow + run_k * 2;
+      // a row past the end repeats the last one: its column of the result is not stored
+      const int lr = min(row0 + r, rows - 1);
+      int pr;
+      if constexpr (GROUPED)
+        pr = list[lr] / a.list_div;
+      else
+        pr = (a.ring_base + lr) & a.ring_mask;
+      src[i] = static_cast<const T *>(a.A) + (int64_t)pr * a.lda + first * kWideK;
+    }
+
+    uint4 wr[4][GT * 4], xr[4][kLoads];
+      const int last_run = (K - 1) / kRunElems * kRunElems;
+    const bool ragged = K % kWideK != 0; // the last step reaches past K
+    auto fetch_w = [&](int s, uint4 (&w)[GT * 4]) {
+      const int t = min(s, steps - 1) * 2;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int g = 0; g < GT; ++g)
+          w[g * 4 + u] = wp[g][(int64_t)(t + u / 2) * 64 + (u & 1) * 32];
+    };
+    auto fetch_x = [&](int s, uint4 (&x)[kLoads]) {
+      const int k = min(min(s, steps - 1) * kWideK + run_k, last_run);
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i)
+        x[i] = *reinterpret_cast<const uint4 *>(src[i] + k);
+    };
+    auto put_x = [&](int s, uint4 (&x)[kLoads], unsigned char *buf) {
+      if (ragged && s == steps - 1) {
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i)
+          x[i] = keep_run<T>(x[i], K - s * kWideK - run_k);
+      }
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i) {
+        if constexpr (kTerms == 1) {
+          *reinterpret_cast<uint4 *>(buf + lds_at[i]) = x[i];
+        } else {
+          uint2 t[3];
+          split3(x[i], t);
+#pragma unroll
+          for (int p = 0; p < 3; ++p)
+            *reinterpret_cast<uint2 *>(buf + p * kPlane + lds_at[i]) = t[p];
+        }
+      }
+    };
+
+    const int frag_at = (lane & 31) * kLdsRow + (lane >> 5) * 16;
+    uint4 frag[2][kTerms][RT];
+    auto load_frag = [&](const unsigned char *buf, int u, uint4 (&f)[kTerms][RT]) {
+#pragma unroll
+      for (int p = 0; p < kTerms; ++p)
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+          f[p][r] = *reinterpret_cast<const uint4 *>(buf + p * kPlane + frag_at + r * 32 * kLdsRow + u * 32);
+    };
+
+    // Step s multiplies buffer s % 3, whose first fragments were read during step s - 1, and
+    // fills buffer (s + 2) % 3, last read before the previous barrier.
+    unsigned char *cur = lds, *next = lds + kBuf, *fill = lds + 2 * kBuf;
+    fetch_x(0, xr[0]);
+    fetch_x(1, xr[1]);
+    fetch_w(0, wr[0]);
+    fetch_x(2, xr[2]);
+    fetch_w(1, wr[1]);
+    fetch_x(3, xr[3]);
+    fetch_w(2, wr[2]);
+    put_x(0, xr[0], cur);
+    put_x(1, xr[1], next);
+    fetch_x(4, xr[0]);
+    __syncthreads();
+    load_frag(cur, 0, frag[0]);
+    auto step = [&](int s, uint4 (&w)[GT * 4], uint4 (&w_new)[GT * 4], uint4 (&x)[kLoads],
+                    uint4 (&x_new)[kLoads]) {
+  #pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        // the next fragments are asked for ahead of the products that cover their way, and
+        // stay there: left to itself the scheduler moves them to their use
+        load_frag(u < 3 ? cur : next, (u + 1) & 3, frag[(u + 1) & 1]);
+        // the step's loads in two parts (evenly between its products 91.4 us against 90.4 for an
+        // experts' way back: several workgroups of a compute unit hide each other's)
         if (u == 0)
           fetch_w(s + 3, w_new);
         if (u == 2)
           fetch_x(s + 5, x_new);
+        if (u == 1)
+          put_x(s + 2, x, fill);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int p = kTerms - 1; p >= 0; --p)
+#pragma unroll
+          for (int g = 0; g < GT; ++g)
+#pragma unroll
+            for (int r = 0; r < RT; ++r)
+              acc[g][r] = mfma_bf16_wide(w[g * 4 + u], frag[u & 1][p][r], acc[g][r]);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      if (u == 1)
-        put_x(s + 2, x, fill);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int p = kTerms - 1; p >= 0; --p)
-#pragma unroll
-        for (int g = 0; g < GT; ++g)
-#pragma unroll
-          for (int r = 0; r < RT; ++r)
-            acc[g][r] = mfma_bf16_wide(w[g * 4 + u], frag[u & 1][p][r], acc[g][r]);
-      __builtin_amdgcn_sched_barrier(0);
+      __syncthreads();
+      unsigned char *t = cur;
+      cur = next;
+      next = fill;
+      fill = t;
+    };
+    int s = 0;
+    for (; s + 4 <= steps; s += 4) {
+      step(s, wr[0], wr[3], xr[2], xr[1]);
+      step(s + 1, wr[1], wr[0], xr[3], xr[2]);
+      step(s + 2, wr[2], wr[1], xr[0], xr[3]);
+      step(s + 3, wr[3], wr[2], xr[1], xr[0]);
     }
-    __syncthreads();
-    unsigned char *t = cur;
-    cur = next;
-    next = fill;
-    fill = t;
-  };
-  int s = 0;
-  for (; s + 4 <= steps; s += 4) {
-    step(s, wr[0], wr[3], xr[2], xr[1]);
-    step(s + 1, wr[1], wr[0], xr[3], xr[2]);
-    step(s + 2, wr[2], wr[1], xr[0], xr[3]);
-    step(s + 3, wr[3], wr[2], xr[1], xr[0]);
+    if (s < steps)
+      step(s, wr[0], wr[3], xr[2], xr[1]);
+    if (s + 1 < steps)
+      step(s + 1, wr[1], wr[0], xr[3], xr[2]);
+    if (s + 2 < steps)
+      step(s + 2, wr[2], wr[1], xr[0], xr[3]);
   }
-  if (s < steps)
-    step(s, wr[0], wr[3], xr[2], xr[1]);
-  if (s + 1 < steps)
-    step(s + 1, wr[1], wr[0], xr[3], xr[2]);
-  if (s + 2 < steps)
-    step(s + 2, wr[2], wr[1], xr[0], xr[3]);
 
   // a lane holds channels 8 j + (lane / 32) * 4 + 0..3, j = 0..3, of row lane % 32 of every tile
 #pragma unroll
@@ -722,8 +849,9 @@ int launch_wide(const RowsGemm &a, hipStream_t stream) {
 // Up to 16 rows the product is bound by the weights: 16-row tiles, wide ones where they
 // still fill the 256 compute units.  Above that the tile with the lowest estimate: tiles
 // per compute unit x steps of 64 k x what a step of such a tile takes (us, measured with
-// K of 1536 to 8960 on full and on partly filled chips), plus what a tile takes to
-// begin and to store.  Tiles of 16 rows x 64 channels stay the best of few rows, whose
+// K of 1536 to 8960 on full and on partly filled chips; those of 128 rows fitted again to
+// nine matrices at 24 to 2048 rows, of which the picks are 0.6 % off the best tile on average),
+// plus what a tile takes to begin and to store.  Tiles of 16 rows x 64 channels stay the best of few rows, whose
 // launches are bound by how many compute units ask for the weights (bfloat16, us against
 // 32 or 64 x 128): 8960 -> 1536 at 24 rows 21.2 vs 28.4, at 150 22.7 vs 31.3, at 220 36.0
 // vs 31.5; 1536 -> 1536 at 64 rows 5.6 vs 6.9; 1536 -> 17920 at 64 rows 18.4 vs 12.4.  In
@@ -794,7 +922,7 @@ int launch_shape(const RowsGemm &a, hipStream_t stream, int *slices) {
     return done(launch_wide<T, 1, 2, OUT, GROUPED, CUT>(with(wide), stream));
   } else {
     // few rows: 16-row tiles of 64 channels, while they are few rounds of the chip
-    const Cost tall = cost(128, 256, 1.02, 7.0), flat = cost(16, 64 * P, 0.13 * P, 2.5);
+    const Cost tall = cost(128, 256, 0.68, 7.0), flat = cost(16, 64 * P, 0.13 * P, 2.5);
     Cost half, low;
     if constexpr (kPair) {
       // fewer workgroups than half the chip draw the weights from memory too slowly

@@ -251,3 +251,12 @@ def test_refusals(bh):
         assert bh.buddy_hip_gemm_bf16(*args) != 0
     assert bh.buddy_hip_gemv_bf16(None, p, p, 64, 16, None) != 0
     assert bh.buddy_hip_bf16_tiles_bytes(0, 4) == 0
+
+
+# The tile of 128 rows, which come past the registers: no whole step of 64 k, one to seven of them
+# (a ring of four, its rounds and every rest of one), and what is left of K behind them
+@pytest.mark.parametrize("M,K,Nout", [(1931, 40, 30000), (1931, 64, 30000), (1931, 100, 12001), (1931, 128, 12000),
+                                      (1025, 230, 12001), (1025, 256, 12000), (1025, 320, 12000), (257, 390, 20016),
+                                      (257, 448, 20016)])
+def test_steps_of_the_tile_of_128_rows(bh, M, K, Nout):
+    test_wide_tiles_of_bfloat16_rows(bh, (4, 2), M, K, Nout)
