@@ -941,6 +941,115 @@ gemm_w8_i8_tall_kernel(BH_I8_LEADING) {
     multiply_tile<D, RB, GP, PAIR>(a);
 }
 
+// ---- few f32 rows as they come -------------------------------------------------------
+// The output and down products of a short prompt: up to 128 rows that no kernel before has as
+// digits.  A launch that turns them into planes takes 2 to 5 us, most of which is the launch; here
+// every workgroup turns its own slice of 32 rows into digits, each row with the step of its largest
+// magnitude in the slice, which is never coarser than that of the whole row, and its sums leave
+// scaled.  (A NaN or an infinity gives its slice a NaN step and the row's sums with it.)
+//
+// What bounds it: one trip to memory.  A workgroup takes 32 rows x 128 channels x C chunks of 64 k
+// and asks for all of its rows and then all of its weights at once; the digits are made while the
+// weights are on their way, and there is one barrier.  27 rows of 8960 -> 1536: 9.8 us, and
+// 5.2 + 7.1 as two launches; of 1536 -> 1536 4.3, and 2.8 + 4.3.
+template <int D, int C>
+__global__ void __launch_bounds__(kSlices *kWave)
+gemm_w8_i8_rows_kernel(const float *A, const int4 *W, int lda, int M, int K, int groups, int chunks, int ncols,
+                       int slices, float *partial) {
+  constexpr int kTurn = turn_floats(32);
+  __shared__ __attribute__((aligned(16))) unsigned char planes[C * D * kPlaneBlock];
+  __shared__ __attribute__((aligned(16))) float turned[kSlices * 32 * kTurn];
+  __shared__ float step_s[32];
+  const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, up = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ctile = blockIdx.x, slice = blockIdx.y, m0 = blockIdx.z * 32;
+  const int cb = slice * C, nch = min(C, chunks - cb); // chunks of this slice, >= 1
+
+  // eight threads to a row, each with every eighth run of four values
+  const int r = tid >> 3, j = tid & 7;
+  float v[2 * C][4];
+  const float *row = A + (int64_t)min(m0 + r, M - 1) * lda;
+  const int k0 = cb * kTileK + j * 4;
+#pragma unroll
+  for (int i = 0; i < 2 * C; ++i) {
+    const float4 q = *reinterpret_cast<const float4 *>(row + min(k0 + i * 32, K - 4));
+    v[i][0] = q.x; v[i][1] = q.y; v[i][2] = q.z; v[i][3] = q.w;
+  }
+  const v4i32 *wp = reinterpret_cast<const v4i32 *>(W) +
+                    ((size_t)min((ctile * kSlices + wave) * 2 + ((lane >> 4) & 1), groups - 1) * chunks + cb) * 64 +
+                    up * 16 + (lane & 15);
+  v4i32 w[C][2];
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      w[c][h] = wp[(size_t)min(c, nch - 1) * 64 + h * 32];
+  __builtin_amdgcn_sched_barrier(0); // all of them before the first value is looked at
+
+  // (Values beyond K repeat the row's last ones, and weights are zero there; rows beyond M repeat the
+  // last row, and nobody reads their sums.)
+  unsigned mb = 0;
+#pragma unroll
+  for (int i = 0; i < 2 * C; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      mb = max(mb, __float_as_uint(v[i][e]) & 0x7fffffffu);
+#pragma unroll
+  for (int o = 1; o < 8; o <<= 1)
+    mb = max(mb, (unsigned)__shfl_xor((int)mb, o, 64));
+  const bool finite = mb < 0x7f800000u;
+  const float step = finite ? digit_step(__uint_as_float(mb), D) : __uint_as_float(0x7fc00000u);
+  const float inv = finite ? 1.0f / step : 0.f;
+  if (j == 0)
+    step_s[r] = step;
+  // pieces of 16 bytes permuted by the row's number, as in multiply_block
+#pragma unroll
+  for (int i = 0; i < 2 * C; ++i) {
+    unsigned word[3];
+    digits_of(v[i], inv, D, word);
+    const int k4 = (i & 1) * 8 + j;
+    unsigned char *dst = planes + (i / 2) * (D * kPlaneBlock) + r * kTileK + ((k4 >> 2) ^ (r >> 2 & 3)) * 16 + (k4 & 3) * 4;
+#pragma unroll
+    for (int p = 0; p < D; ++p)
+      *reinterpret_cast<unsigned *>(dst + p * kPlaneBlock) = word[p];
+  }
+  __syncthreads();
+
+  v16i32 acc[D];
+#pragma unroll
+  for (int p = 0; p < D; ++p)
+    acc[p] = v16i32{};
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+    if (c < nch) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int p = 0; p < D; ++p) {
+          const v4i32 f = *reinterpret_cast<const v4i32 *>(planes + (c * D + p) * kPlaneBlock + col * kTileK +
+                                                           ((2 * h + up) ^ (col >> 2 & 3)) * 16);
+          acc[p] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[c][h], f, acc[p], 0, 0, 0);
+        }
+    }
+
+  // out as finish_tile leaves the sums of a slice, but scaled
+  float *tile = turned + wave * (32 * kTurn);
+  const float s = step_s[col];
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    *reinterpret_cast<float4 *>(tile + col * kTurn + 8 * q + 4 * up) =
+        make_float4(combine<D>(acc, 4 * q) * s, combine<D>(acc, 4 * q + 1) * s, combine<D>(acc, 4 * q + 2) * s,
+                    combine<D>(acc, 4 * q + 3) * s);
+  const size_t at = ((size_t)(blockIdx.z * ncols + ctile) * slices + slice) * kSlices + wave;
+  float *part = partial + at * 32 * 32;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int idx = lane + 64 * i, rr = idx / 8, c4 = idx % 8;
+    *reinterpret_cast<float4 *>(part + rr * 32 + c4 * 4) =
+        *reinterpret_cast<const float4 *>(tile + rr * kTurn + c4 * 4);
+  }
+}
+
 // Where the sums of row m, channels n.. of the first K slice lie.
 template <class Args> // GemmI8Args, SliceSums
 __device__ __forceinline__ const float *first_slice(const Args &a, int m, int n) {
@@ -987,7 +1096,7 @@ __device__ __forceinline__ FinishOperands load_finish_operands(const GemmI8Args 
   return f;
 }
 
-// C (+)= step[m] * scale[n] * sum over slices of the unscaled sums, slice order.
+// C (+)= step[m] * scale[n] * sum over slices of the unscaled sums, slice order (no steps: 1).
 __global__ void __launch_bounds__(256)
 reduce_slices_kernel(GemmI8Args a) {
   const int n4 = (a.N + 3) / 4;
@@ -997,7 +1106,7 @@ reduce_slices_kernel(GemmI8Args a) {
   const int m = (int)(i / n4), n = (int)(i % n4) * 4;
   const size_t slice_stride = (size_t)kSlices * a.tile_rows * a.span;
   const float *p = first_slice(a, m, n);
-  const float step = a.steps[m];
+  const float step = a.steps ? a.steps[m] : 1.0f;
   float *c = a.C + (int64_t)m * a.ldc + n;
   const FinishOperands f = load_finish_operands(a, c, n);
   float v[4];
@@ -1156,7 +1265,7 @@ reduce_slices_norm_kernel(const float *p_partial, const float *p_steps, int p_N,
   const int m = blockIdx.x;
   const int n4 = (a.N + 3) / 4;
   const size_t slice_stride = (size_t)kSlices * a.tile_rows * a.span;
-  const float step = a.steps[m];
+  const float step = a.steps ? a.steps[m] : 1.0f;
   float s = 0.f;
   for (int q4 = threadIdx.x; q4 < n4; q4 += kRowThreads) {
     const int n = q4 * 4;
@@ -1510,6 +1619,50 @@ int launch_slices_rope(const SliceSums &sums, const RopeKv &r, float *C, int64_t
 // `planes` holds the digit planes and row steps of the activations (written by
 // one of the producers above for exactly this M, K and digit count).
 namespace {
+// The RMSNorm of the finished rows into digit planes, or the rotation of q | k | v, where the caller
+// asked for it and no kernel of the matmul holds whole rows.
+int norm_behind(const GemmW8Args &in, hipStream_t stream) {
+  if (in.then_rope) {
+    const RopeKv &r = *in.then_rope;
+    return launch_rope_kv_write(in.C, in.ldc, r.inv_freq, r.kcache, r.vcache, r.heads, r.kv_heads,
+                                kAttnHeadDim, r.max_len, r.start_pos, (int)in.M, stream);
+  }
+  if (!in.then_norm_w)
+    return BUDDY_HIP_OK;
+  return launch_rmsnorm_to_digits(in.C, in.ldc, in.then_norm_w, (int)in.M, (int)in.N,
+                                  in.then_norm_eps, in.digits, in.then_norm_staged, stream);
+}
+
+// What follows a product whose K is in slices: their sum, and what the caller wants behind it.
+int add_slices(const GemmW8Args &in, const GemmI8Args &a, hipStream_t stream) {
+  const GemmStagingLayout next = gemm_staging_layout(in.M, in.N);
+  if (in.then_norm_w && next.cols_padded <= kRowCache) {
+    // the kernel that adds the slices holds whole rows: it writes the planes too
+    const size_t row_lds = 2 * sizeof(float) * (size_t)next.cols_padded;
+    if (row_lds > 48 * 1024) { // up to 96 KiB at kRowCache columns
+      static DynLdsOnce dyn_lds;
+      BH_CHECK_HIP(ensure_dyn_lds(dyn_lds,
+                                  reinterpret_cast<const void *>(reduce_slices_norm_kernel),
+                                  (int)(2 * sizeof(float) * kRowCache)));
+    }
+    hipLaunchKernelGGL(reduce_slices_norm_kernel, dim3((unsigned)a.M), dim3(kRowThreads),
+                       row_lds, stream, a.partial, a.steps, a.N, a.ncols, a.slices, a.span,
+                       a.tile_rows, a, in.then_norm_w, 1.0f / (float)in.N, in.then_norm_eps,
+                       in.digits, next.rows_padded, next.cols_padded,
+                       static_cast<int8_t *>(in.then_norm_staged));
+    BH_CHECK_HIP(hipGetLastError());
+    return BUDDY_HIP_OK;
+  }
+  if (in.then_rope)
+    return launch_slices_rope({a.partial, a.steps, a.scale, a.bias, a.slices, a.span, a.tile_rows, a.ncols, a.N},
+                              *in.then_rope, a.C, a.ldc, a.M, stream);
+  const int64_t threads = (int64_t)a.M * ((a.N + 3) / 4);
+  hipLaunchKernelGGL(reduce_slices_kernel, dim3((unsigned)ceil_div(threads, 256)), dim3(256), 0,
+                     stream, a);
+  BH_CHECK_HIP(hipGetLastError());
+  return norm_behind(in, stream);
+}
+
 template <int D>
 int launch_gemm_w8_digits_d(const GemmW8Args &in, const void *planes, hipStream_t stream) {
   GemmI8Args a;
@@ -1549,19 +1702,6 @@ int launch_gemm_w8_digits_d(const GemmW8Args &in, const void *planes, hipStream_
   // angles take, which every head works out for itself there.
   const double norm_us = in.then_norm_w ? 5.0 : in.then_rope ? 4.0 : 0.0;
   const double split_norm_us = in.then_rope ? 0.5 + 0.004 * (double)in.M : slices_fuse_norm ? 0.0 : norm_us;
-  // the RMSNorm of the finished rows into digit planes, where the caller asked
-  // for it and no kernel of the matmul holds whole rows
-  auto then_norm = [&]() -> int {
-    if (in.then_rope) {
-      const RopeKv &r = *in.then_rope;
-      return launch_rope_kv_write(in.C, in.ldc, r.inv_freq, r.kcache, r.vcache, r.heads, r.kv_heads,
-                                  kAttnHeadDim, r.max_len, r.start_pos, (int)in.M, stream);
-    }
-    if (!in.then_norm_w)
-      return BUDDY_HIP_OK;
-    return launch_rmsnorm_to_digits(in.C, in.ldc, in.then_norm_w, (int)in.M, (int)in.N,
-                                    in.then_norm_eps, in.digits, in.then_norm_staged, stream);
-  };
   TilePlan plan = plan_tiles<D, false>(in.M, in.N, a.chunks, true, norm_us, split_norm_us, 0);
   if (int rc = launch_plan<D, false>(plan, a, stream))
     return rc;
@@ -1571,39 +1711,90 @@ int launch_gemm_w8_digits_d(const GemmW8Args &in, const void *planes, hipStream_
       return rc;
   }
   if (plan.slices == 1)
-    return then_norm();
-  const GemmStagingLayout next = gemm_staging_layout(in.M, in.N);
-  if (in.then_norm_w && slices_fuse_norm) {
-    // the kernel that adds the slices holds whole rows: it writes the planes too
-    const size_t row_lds = 2 * sizeof(float) * (size_t)next.cols_padded;
-    if (row_lds > 48 * 1024) { // up to 96 KiB at kRowCache columns
-      static DynLdsOnce dyn_lds;
-      BH_CHECK_HIP(ensure_dyn_lds(dyn_lds,
-                                  reinterpret_cast<const void *>(reduce_slices_norm_kernel),
-                                  (int)(2 * sizeof(float) * kRowCache)));
-    }
-    hipLaunchKernelGGL(reduce_slices_norm_kernel, dim3((unsigned)a.M), dim3(kRowThreads),
-                       row_lds, stream, a.partial, a.steps, a.N, a.ncols, a.slices, a.span,
-                       a.tile_rows, a, in.then_norm_w, 1.0f / (float)in.N, in.then_norm_eps,
-                       in.digits, next.rows_padded, next.cols_padded,
-                       static_cast<int8_t *>(in.then_norm_staged));
-    BH_CHECK_HIP(hipGetLastError());
-    return BUDDY_HIP_OK;
-  }
-  if (in.then_rope)
-    return launch_slices_rope({a.partial, a.steps, a.scale, a.bias, a.slices, a.span, a.tile_rows, a.ncols, a.N},
-                              *in.then_rope, a.C, a.ldc, a.M, stream);
-  const int64_t threads = (int64_t)a.M * ((a.N + 3) / 4);
-  hipLaunchKernelGGL(reduce_slices_kernel, dim3((unsigned)ceil_div(threads, 256)), dim3(256), 0,
-                     stream, a);
-  BH_CHECK_HIP(hipGetLastError());
-  return then_norm();
+    return norm_behind(in, stream);
+  return add_slices(in, a, stream);
 }
 } // namespace
 
 int launch_gemm_w8_digits(const GemmW8Args &in, const void *planes, hipStream_t stream) {
   return in.digits == 2 ? launch_gemm_w8_digits_d<2>(in, planes, stream)
                         : launch_gemm_w8_digits_d<3>(in, planes, stream);
+}
+
+namespace {
+BH_TILE_FAMILY(RowsFamily, "gemm_w8_i8_rows_kernel"); // planes, chunks of a slice
+
+// Chunks of 64 k to a slice: the fewest that leave at most sixteen slices, whose sums have to be
+// added, and at most a workgroup per compute unit, whose loads are one trip; 0: no such cut.
+int rows_chunks(int64_t M, int64_t K, int64_t N) {
+  const int64_t chunks = ceil_div(K, kTileK), tiles = ceil_div(N, kSlices * 32) * ceil_div(M, 32);
+  for (int c : {2, 3, 5, 9, 14})
+    if (ceil_div(chunks, c) <= 16 && ceil_div(chunks, c) * tiles <= 256)
+      return c;
+  return 0;
+}
+
+template <int D, int C> int launch_rows(const GemmW8Args &in, const GemmI8Args &a, hipStream_t stream) {
+  BH_NOTE_VARIANT(RowsFamily, D, C);
+  hipLaunchKernelGGL((gemm_w8_i8_rows_kernel<D, C>), dim3(a.ncols, a.slices, a.row_tiles), dim3(kSlices * kWave), 0,
+                     stream, in.A, a.W, (int)in.lda, a.M, (int)in.K, a.groups, a.chunks, a.ncols, a.slices, a.partial);
+  BH_CHECK_HIP(hipGetLastError());
+  return BUDDY_HIP_OK;
+}
+template <int D> int launch_rows_of(int c, const GemmW8Args &in, const GemmI8Args &a, hipStream_t stream) {
+  switch (c) {
+  case 2:
+    return launch_rows<D, 2>(in, a, stream);
+  case 3:
+    return launch_rows<D, 3>(in, a, stream);
+  case 5:
+    return launch_rows<D, 5>(in, a, stream);
+  case 9:
+    return launch_rows<D, 9>(in, a, stream);
+  default:
+    return launch_rows<D, 14>(in, a, stream);
+  }
+}
+} // namespace
+
+int launch_gemm_w8_digits_rows(const GemmW8Args &in, bool *done, hipStream_t stream) {
+  *done = false;
+  BH_REQUIRE(in.A && in.W && in.scale && in.C && in.M > 0 && in.K > 0 && in.N > 0 && in.lda >= in.K && in.ldc >= in.N &&
+                 (in.digits == 2 || in.digits == 3) && !in.staged && !in.silu_pair && !in.then_rope,
+             "gemm_w8: rows as they come");
+  // rows are read 16 bytes at a time; beyond 128 of them (three planes: 129 rows 2426 -> 2335 us a
+  // prompt, 256 the same; two: 180 rows 1 % longer) a launch for the digits is a small part
+  const bool aligned = ((in.K | in.lda) & 3) == 0 && (reinterpret_cast<uintptr_t>(in.A) & 15) == 0;
+  const int c = in.M <= 128 && aligned && in.lda < (1 << 30) ? rows_chunks(in.M, in.K, in.N) : 0;
+  if (!c)
+    return BUDDY_HIP_OK;
+  GemmI8Args a{};
+  a.W = reinterpret_cast<const int4 *>(in.W);
+  a.scale = in.scale;
+  a.bias = in.bias;
+  a.C = in.C;
+  a.ldc = in.ldc;
+  a.M = (int)in.M;
+  a.N = (int)in.N;
+  a.groups = (int)ceil_div(in.N, kTileN);
+  a.chunks = (int)ceil_div(in.K, kTileK);
+  a.accumulate = in.accumulate ? 1 : 0;
+  a.ncols = (int)ceil_div(in.N, kSlices * 32);
+  a.row_tiles = (int)ceil_div(in.M, 32);
+  a.tile_rows = a.span = 32;
+  a.chunks_per_slice = c;
+  a.slices = (int)ceil_div(a.chunks, c);
+  const size_t bytes = sizeof(float) * 32 * kSlices * 32 * (size_t)a.slices * a.ncols * a.row_tiles;
+  char *ws = nullptr;
+  if (int rc = gemm_slices_workspace(stream, bytes, &ws))
+    return rc;
+  if (!ws) // under capture, and none of this size
+    return BUDDY_HIP_OK;
+  a.partial = reinterpret_cast<float *>(ws);
+  if (int rc = in.digits == 2 ? launch_rows_of<2>(c, in, a, stream) : launch_rows_of<3>(c, in, a, stream))
+    return rc;
+  *done = true;
+  return add_slices(in, a, stream);
 }
 
 // The w8a8 matmul for more than 16 rows: `plane` holds the int8 activations as

@@ -390,6 +390,33 @@ struct Qwen2Session : Session {
     g.digits = gemm_digits;
     return launch_gemm_w8(g, stream);
   }
+  // W's product with f32 rows [M, W.K] in digit modes, added to C; `planes` holds them as digits
+  // where the product does not turn them into those itself
+  int gemm_digit_rows(const float *A, const PackedLinear &W, float *C, int64_t M, const float *then_norm_w,
+                      void *then_norm_staged, unsigned short *planes) {
+    GemmW8Args g;
+    g.then_norm_w = then_norm_w;
+    g.then_norm_eps = shape.rms_eps;
+    g.then_norm_staged = then_norm_staged;
+    g.A = A;
+    g.lda = W.K;
+    g.W = W.w;
+    g.scale = W.s;
+    g.C = C;
+    g.ldc = W.N;
+    g.M = M;
+    g.K = W.K;
+    g.N = W.N;
+    g.accumulate = true;
+    g.digits = gemm_digits;
+    bool done = false;
+    int rc = launch_gemm_w8_digits_rows(g, &done, stream);
+    if (rc || done)
+      return rc;
+    if ((rc = launch_activations_to_digits(A, W.K, M, W.K, gemm_digits, planes, stream)))
+      return rc;
+    return gemm_staged(planes, W, C, M, true, 0, then_norm_w, then_norm_staged);
+  }
   // RMSNorm rows / SiLU(g) * u written straight into the matmul's input format
   int norm_to_staging(const float *x, const float *w, int rows, unsigned short *staged) {
     const auto &S = shape;
@@ -477,13 +504,11 @@ struct Qwen2Session : Session {
         // o_proj's finished rows go on as the normed input of gate and up: where
         // the matmul splits K over workgroups, the kernel that adds the slices
         // holds whole rows and writes those digit planes itself
-        if ((rc = folded ? launch_attn_fold_to_digits(fold, a.o_stride, S.heads, n, gemm_digits,
-                                                      pf_att_dg, stream)
-                         : launch_activations_to_digits(pf_att, a.o_stride, n, a.o_stride, gemm_digits,
-                                                        pf_att_dg, stream)))
+        if (folded && (rc = launch_attn_fold_to_digits(fold, a.o_stride, S.heads, n, gemm_digits, pf_att_dg,
+                                                       stream)))
           return rc;
-        if ((rc = gemm_staged(reinterpret_cast<const unsigned short *>(pf_att_dg), L.o, pf_x, n,
-                              true, 0, L.ln2, pf_xn_bf)))
+        if ((rc = folded ? gemm_staged(pf_att_dg, L.o, pf_x, n, true, 0, L.ln2, pf_xn_bf)
+                         : gemm_digit_rows(pf_att, L.o, pf_x, n, L.ln2, pf_xn_bf, pf_att_dg)))
           return rc;
       } else {
         // likewise with bf16 terms
@@ -500,7 +525,7 @@ struct Qwen2Session : Session {
       if (L.gate_up_joint) {
         // gate and up in one launch whose workgroups hold matching tiles of
         // both: SiLU(gate) * up leaves the matmul as the terms of down's input, or, since
-        // digit planes need whole rows, in f32, and one pass turns it into those
+        // digit planes need whole rows, in f32
         GemmW8Args g;
         g.staged = pf_xn_bf;
         g.W = L.gate.w;
@@ -516,12 +541,11 @@ struct Qwen2Session : Session {
         g.silu_staged = pf_g_bf;
         if ((rc = launch_gemm_w8(g, stream)))
           return rc;
-        if (gemm_digits && (rc = launch_activations_to_digits(pf_g, S.inter, n, S.inter, gemm_digits, pf_g_bf,
-                                               stream)))
-          return rc;
         // down's finished rows go on as the next layer's normed q|k|v input
-        if ((rc = gemm_staged(pf_g_bf, L.down, pf_x, n, true, 0, ahead ? nx->ln1 : nullptr,
-                              ahead ? pf_xn_bf : nullptr)))
+        const float *next_norm = ahead ? nx->ln1 : nullptr;
+        void *next_in = ahead ? pf_xn_bf : nullptr;
+        if ((rc = gemm_digits ? gemm_digit_rows(pf_g, L.down, pf_x, n, next_norm, next_in, pf_g_bf)
+                              : gemm_staged(pf_g_bf, L.down, pf_x, n, true, 0, next_norm, next_in)))
           return rc;
         normed_ahead = ahead;
         continue;

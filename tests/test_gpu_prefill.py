@@ -813,3 +813,36 @@ def test_session_prefill_refuses_overflow(bh):
     with pytest.raises(bma.BuddyHipError):
         sess.prefill(list(range(10)), SMALL.max_len - 5)
     sess.close()
+
+
+# Output and down products of few rows that are turned into digits within the product: every number
+# of chunks to a slice, a last slice of fewer, K that ends inside a chunk, one and two tiles of rows;
+# and one row too many
+@pytest.mark.parametrize("precision", ["digits", "digits2"])
+@pytest.mark.parametrize("hidden,heads,inter,n,chunks", [
+    (384, 3, 336, 2, {2}), (1536, 12, 8960, 27, {2, 9}), (1536, 12, 8960, 64, {3, 14}), (256, 4, 4112, 33, {2, 5}),
+    (100, 1, 16, 17, {2}), (1536, 12, 336, 128, {2, 5}), (384, 3, 336, 129, set())])
+def test_few_rows_become_digits_within_the_product(bh, hidden, heads, inter, n, chunks, precision):
+    shape = Shape(layers=2, hidden=hidden, heads=heads, kv_heads=1, head_dim=128, inter=inter, vocab=320, max_len=n + 8) \
+        if heads <= 8 else Shape(layers=2, hidden=hidden, heads=heads, kv_heads=2, head_dim=128, inter=inter, vocab=320,
+                                 max_len=n + 8)
+    toks = synthetic.first_tokens(shape, n, seed=n + inter).astype(np.int32)
+    sess, _ = synthetic.build_session(shape, context=0, ln_jitter=0.1)
+    bh.buddy_hip_variant_reset()
+    _, got = sess.prefill(toks, 0, precision=precision)
+    planes = 3 if precision == "digits" else 2
+    ran = {k for k, v in tiles_run(bh).items() if v and k.startswith("gemm_w8_i8_rows_kernel")}
+    assert ran == {f"gemm_w8_i8_rows_kernel<{planes}, {c}>" for c in chunks}
+    rows = [sess.get_kv(j)[:, :n] for j in (2, 3)]
+    sess.close()
+    sess, _ = synthetic.build_session(shape, context=0, ln_jitter=0.1)
+    for i, t in enumerate(toks):
+        _, want = sess.decode(int(t), i, want_logits=i + 1 == n)
+    pairs = [(got, want)] + [(rows[j - 2], sess.get_kv(j)[:, :n]) for j in (2, 3)]
+    sess.close()
+    for g, w in pairs:
+        if planes == 3:
+            check_close(g, w)
+        else:  # some ten roundings on the way, of 2^-15 of a row's largest value
+            g, w = np.asarray(g, np.float64), np.asarray(w, np.float64)
+            assert np.linalg.norm(g - w) < 2.0**-10 * np.linalg.norm(w)
