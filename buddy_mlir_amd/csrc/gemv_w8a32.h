@@ -44,6 +44,9 @@ struct GemvArgs {
   float *argmax_v = nullptr;
   int *argmax_i = nullptr;
   int *argmax_groups = nullptr;
+  // optional room for the sums of slices of K (gemv_batch_sums_bytes), 16-byte aligned
+  float *sums = nullptr;
+  size_t sums_bytes = 0;
   int M = 1;
   int64_t K = 0, N = 0;
   int epilogue = kEpiStore;
@@ -55,5 +58,9 @@ int launch_gemv(const GemvArgs &a, hipStream_t stream);
 // three bf16 terms of every activation (every f32 bit; BUDDY_HIP_GEMV_BATCH=bf16).
 int launch_gemv_i8(const GemvArgs &a, hipStream_t stream);
 int launch_gemv_mfma(const GemvArgs &a, hipStream_t stream);
+// ... and those shapes of them whose loads can all be on their way at once; done stays false, and
+// nothing has been launched, where this is none of them
+int launch_gemv_batch(const GemvArgs &a, bool *done, hipStream_t stream);
+size_t gemv_batch_sums_bytes(int64_t M, int64_t K);
 
 } // namespace bh

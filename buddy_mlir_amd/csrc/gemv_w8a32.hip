@@ -1602,7 +1602,11 @@ int launch_gemv(const GemvArgs &a, hipStream_t stream) {
   {
     if (a.argmax_groups)
       *a.argmax_groups = 0;
-    return batch_bf16() ? launch_gemv_mfma(a, stream) : launch_gemv_i8(a, stream);
+    if (batch_bf16())
+      return launch_gemv_mfma(a, stream);
+    bool done = false;
+    const int rc = launch_gemv_batch(a, &done, stream);
+    return rc || done ? rc : launch_gemv_i8(a, stream);
   }
   // the kernel is compiled for 1, 2, 4, 8 and 16 rows; extra rows are zero-
   // filled in LDS and never stored
@@ -1735,10 +1739,16 @@ int buddy_hip_linear_w8a32(const buddy_hip_linear_desc *d,
   return bh::launch_gemv(a, bh::as_stream(stream));
 } BH_CATCH_INT("buddy_hip_linear_w8a32")
 
+namespace {
+size_t mlp_rows_bytes(int64_t M, int64_t inter) {
+  return (sizeof(float) * (size_t)M * (size_t)inter + 255) & ~(size_t)255;
+}
+} // namespace
+
 size_t buddy_hip_mlp_block_workspace_bytes(int64_t M, int64_t inter) {
   if (M < 1 || M > 16 || inter < 1)
     return 0;
-  return (sizeof(float) * (size_t)M * (size_t)inter + 255) & ~(size_t)255;
+  return mlp_rows_bytes(M, inter) + bh::gemv_batch_sums_bytes(M, inter);
 }
 
 int buddy_hip_mlp_block_w8a32(const buddy_hip_mlp_block_desc *d, buddy_hip_stream stream) try {
@@ -1749,10 +1759,11 @@ int buddy_hip_mlp_block_w8a32(const buddy_hip_mlp_block_desc *d, buddy_hip_strea
   BH_REQUIRE(d->M >= 1 && d->M <= 16, "mlp_block_w8a32: M=%lld outside 1..16", (long long)d->M);
   BH_REQUIRE(d->hidden > 0 && d->inter > 0 && d->ldx >= d->hidden && d->ldy >= d->hidden,
              "mlp_block_w8a32: bad shape or row stride");
-  BH_REQUIRE(d->workspace_bytes >= buddy_hip_mlp_block_workspace_bytes(d->M, d->inter) &&
-                 (reinterpret_cast<uintptr_t>(d->workspace) & 15) == 0,
-             "mlp_block_w8a32: workspace of %zu bytes (16-byte aligned) needed, %zu given",
-             buddy_hip_mlp_block_workspace_bytes(d->M, d->inter), d->workspace_bytes);
+  // (room for the rows alone is enough: down's K then stays within workgroups)
+  const size_t rows_bytes = mlp_rows_bytes(d->M, d->inter);
+  BH_REQUIRE(d->workspace_bytes >= rows_bytes && (reinterpret_cast<uintptr_t>(d->workspace) & 15) == 0,
+             "mlp_block_w8a32: workspace of %zu bytes (16-byte aligned) needed, %zu given", rows_bytes,
+             d->workspace_bytes);
   hipStream_t s = bh::as_stream(stream);
   float *h = static_cast<float *>(d->workspace); // [M, inter] between the two launches
   bh::GemvArgs g;
@@ -1785,6 +1796,8 @@ int buddy_hip_mlp_block_w8a32(const buddy_hip_mlp_block_desc *d, buddy_hip_strea
   w.K = d->inter;
   w.N = d->hidden;
   w.epilogue = (d->flags & BUDDY_HIP_GEMV_ACCUMULATE) ? bh::kEpiAccum : bh::kEpiStore;
+  w.sums = reinterpret_cast<float *>(static_cast<char *>(d->workspace) + rows_bytes);
+  w.sums_bytes = d->workspace_bytes - rows_bytes;
   return bh::launch_gemv(w, s);
 } BH_CATCH_INT("buddy_hip_mlp_block_w8a32")
 

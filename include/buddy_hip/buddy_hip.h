@@ -205,11 +205,11 @@ int buddy_hip_gemv_w8a32(const float *A, const int8_t *packed,
  *   y (+)= (SiLU(x' . gate) * (x' . up)) . down,   x' = RMSNorm(x) * norm_w or x
  * (subgraph0_decode_simplify.mlir:210-260 over M rows): the two launches of
  * buddy_hip_linear_w8a32 that make it (gate and up fused with SiLU * mul, then
- * down) behind one call, with the same kernels and roundings.  All three
+ * down) behind one call, with the same roundings of the activations.  All three
  * matrices are wave-tile packed ([hidden, inter] twice, [inter, hidden]).  The
- * intermediate rows [M, inter] f32 live in `workspace`
- * (buddy_hip_mlp_block_workspace_bytes(M, inter) bytes, 16-byte aligned).  No
- * counterpart in the reference, whose decode kernels are m == 1 only. */
+ * intermediate rows [M, inter] f32 and, from five rows on, sums of slices of a long
+ * `inter` live in `workspace` (buddy_hip_mlp_block_workspace_bytes(M, inter) bytes, 16-byte
+ * aligned; 4 M inter rounded up to 256 is enough, without the latter).  No counterpart in the reference, whose decode kernels are m == 1 only. */
 typedef struct buddy_hip_mlp_block_desc {
   const float *x;          /* [M, hidden], row stride ldx */
   int64_t ldx;

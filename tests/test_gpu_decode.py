@@ -630,3 +630,48 @@ def test_logits_reach_every_kind_of_memory(vocab):
     np.testing.assert_array_equal(pageable, pinned.numpy())
     np.testing.assert_array_equal(pageable, device.cpu().numpy())
     sess.close()
+
+
+# Blocks whose products ask for all they need at once: <channel groups of a workgroup, groups of four
+# rows> of the pair, chunks of a slice of down's K; slices without a chunk and with fewer than the
+# others, K that ends inside a chunk, channels inside a group; rows that are not finite; and a workspace
+# without room for the slices' sums
+@pytest.mark.parametrize("M,H,I,pair,chunks", [
+    (5, 1020, 4096, (1, 2), 4), (8, 1084, 4100, (2, 2), 4), (9, 1536, 8960, (3, 4), 8), (16, 1348, 12292, (4, 4), 16),
+    (12, 1152, 4034 + 2, (1, 4), 4)])
+def test_mlp_block_in_one_trip(bh, oracle, M, H, I, pair, chunks):
+    from tile_report import tiles_run
+    qg, sg = synthetic.quantized_linear(H, I, 41)
+    qu, su = synthetic.quantized_linear(H, I, 42)
+    qd, sd = synthetic.quantized_linear(I, H, 43)
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn((M, H), generator=g, device="cuda")
+    x[1] *= 1e-6
+    x[2] *= 1e5
+    w = 1 + 0.1 * torch.randn(H, generator=g, device="cuda")
+    y0 = torch.randn((M, H), generator=g, device="cuda")
+    packs = [t for q, s in ((qg, sg), (qu, su), (qd, sd)) for t in (ops.pack_w8(q), s)]
+    bh.buddy_hip_variant_reset()
+    plain = ops.mlp_block_w8a32(x, *packs, H, I)
+    full = ops.mlp_block_w8a32(x, *packs, H, I, y=y0.clone(), norm_w=w, norm_eps=1e-6, accumulate=True)
+    torch.cuda.synchronize()
+    assert {k: v for k, v in tiles_run(bh).items() if v and k.startswith("batch_")} == {
+        "batch_pair_kernel<%d, %d>" % pair: 2, f"batch_slice_kernel<{chunks}>": 2}
+    tight = torch.empty((4 * M * I + 255) // 256 * 256, dtype=torch.uint8, device="cuda")
+    small = ops.mlp_block_w8a32(x, *packs, H, I, workspace=tight)
+    torch.cuda.synchronize()
+    assert tiles_run(bh)[f"batch_slice_kernel<{chunks}>"] == 2
+    hq = [t.cpu().numpy() for t in (qg, sg, qu, su, qd, sd)]
+    want = mlp_block_oracle(oracle, x.cpu().numpy(), *hq)
+    want_full = mlp_block_oracle(oracle, x.cpu().numpy(), *hq, norm_w=w.cpu().numpy(), eps=np.float32(1e-6),
+                                 y0=y0.cpu().numpy())
+    for m in range(M):
+        check_close(plain.cpu().numpy()[m], want[m])
+        check_close(small.cpu().numpy()[m], want[m])
+        check_close(full.cpu().numpy()[m], want_full[m])
+    x[0, H - 1] = float("nan")
+    x[3, 0] = float("-inf")
+    got = ops.mlp_block_w8a32(x, *packs, H, I).cpu().numpy()
+    assert np.isnan(got[[0, 3]]).all()
+    rest = [m for m in range(M) if m not in (0, 3)]
+    np.testing.assert_array_equal(got[rest], plain.cpu().numpy()[rest])
