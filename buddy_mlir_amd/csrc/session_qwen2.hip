@@ -140,8 +140,11 @@ struct Qwen2Session : Session {
   }
 
   int gemv(const float *A, const PackedLinear &W0, const PackedLinear *W1,
-           const float *norm_w, float *C, int epi) {
+           const float *norm_w, float *C, int epi, int rows = 1, float *sums = nullptr,
+           size_t sums_bytes = 0) {
     GemvArgs g;
+    g.sums = sums;
+    g.sums_bytes = sums_bytes;
     g.A = A;
     g.lda = W0.K;
     g.W0 = W0.w;
@@ -156,7 +159,7 @@ struct Qwen2Session : Session {
     g.norm_inv_k = 1.0f / (float)W0.K;
     g.C = C;
     g.ldc = W0.N;
-    g.M = 1;
+    g.M = rows;
     g.K = W0.K;
     g.N = W0.N;
     g.epilogue = epi;
@@ -435,6 +438,10 @@ struct Qwen2Session : Session {
                                       staged, stream);
   }
 
+  static constexpr int kFewTokens = 16;
+  // channels from which on q | k | v of few tokens go that way: fewer leave most of the chip without
+  // a workgroup, where the prompt's product cuts K over several
+  static constexpr int kFewChannels = 128 * 16;
   // Prompt processing for tokens already in pf_tokens: fills cache rows
   // start_pos .. start_pos+n-1 and leaves the final hidden states in pf_x
   // (op order of a layer: subgraph0_decode_simplify.mlir:60-232 over n rows).
@@ -449,6 +456,13 @@ struct Qwen2Session : Session {
     const bool folded = attn_prompt_pays(n, start_pos, S.heads, S.kv_heads);
     if (folded && !pf_attn_ws) // for as many rows as the other buffers have, behind any context
       BH_CHECK_HIP(hipMalloc(&pf_attn_ws, attn_prompt_workspace_bytes(pf_rows, S.max_len, S.heads, S.kv_heads)));
+    // Up to 16 tokens go through the products of a decode step, which read f32 rows, norm them, turn
+    // them into digits of 2^-23 of their largest and add to the residual themselves: five to seven
+    // launches a layer for the prompt's eight, whose tiles of 32 rows are mostly padding here.  (Not where
+    // every bit of the rows was asked for.)  Qwen2-1.5B's shape, us a prompt, those against the prompt's own:
+    // 1 token 878 and 1504, 2 973 and 1491, 5 1165 and 1527, 9 1236 and 1545, 16 1272 and 1546; cast to
+    // bfloat16 913 and 1516, 971 and 1504, 1166 and 1503, 1228 and 1524, 1278 and 1539.
+    const bool few = n <= kFewTokens && (gemm_digits || (gemm_terms == 1 && QKV >= kFewChannels));
     bool normed_ahead = false; // pf_xn_bf already holds this layer's normed input
     for (int i = 0; i < S.layers; ++i) {
       Layer &L = layers[(size_t)i];
@@ -459,6 +473,9 @@ struct Qwen2Session : Session {
           return rc;
         if ((rc = launch_matmul_f32(pf_xn, L.qkv_f32, pf_qkv, n, L.qkv.N, L.qkv.K,
                                     L.qkv.K, L.qkv.N, L.qkv.N, true, stream)))
+          return rc;
+      } else if (few && L.qkv.N >= kFewChannels) {
+        if ((rc = gemv(pf_x, L.qkv, nullptr, L.ln1, pf_qkv, kEpiStore, n)))
           return rc;
       } else {
         // the norm writes the matmul's input format directly (the previous layer's down
@@ -477,7 +494,8 @@ struct Qwen2Session : Session {
         if ((rc = gemm_staged(pf_xn_bf, L.qkv, pf_qkv, n, false, 0, nullptr, nullptr, &rope)))
           return rc;
       }
-      if (L.qkv_f32 && (rc = launch_rope_kv_write(pf_qkv, QKV, inv_freq, L.kc, L.vc, S.heads,
+      const bool rotated = !L.qkv_f32 && !(few && L.qkv.N >= kFewChannels);
+      if (!rotated && (rc = launch_rope_kv_write(pf_qkv, QKV, inv_freq, L.kc, L.vc, S.heads,
                                                  S.kv_heads, S.head_dim, S.max_len, start_pos,
                                                  n, stream)))
         return rc;
@@ -500,6 +518,28 @@ struct Qwen2Session : Session {
       PromptFold fold;
       if ((rc = folded ? launch_attn_prompt(a, pf_attn_ws, fold, stream) : launch_attn_prefill(a, stream)))
         return rc;
+      const int64_t ld_gu = 2 * (int64_t)S.inter;
+      const Layer *nx = i + 1 < S.layers ? &layers[(size_t)i + 1] : nullptr;
+      const bool ahead = nx && !nx->qkv_f32;
+      if (few && L.gate_up_joint) {
+        if (folded) {
+          if ((rc = gemm_digits ? launch_attn_fold_to_digits(fold, a.o_stride, S.heads, n, gemm_digits, pf_att_dg, stream)
+                                : launch_attn_fold_to_terms(fold, a.o_stride, S.heads, n, gemm_terms, pf_att_dg, stream)) ||
+              (rc = gemm_staged(pf_att_dg, L.o, pf_x, n, true)))
+            return rc;
+        } else if ((rc = gemv(pf_att, L.o, nullptr, nullptr, pf_x, kEpiAccum, n))) {
+          return rc;
+        }
+        const size_t sums_bytes = gemv_batch_sums_bytes(n, S.inter);
+        char *sums = nullptr;
+        if (sums_bytes && (rc = gemm_slices_workspace(stream, sums_bytes, &sums)))
+          return rc;
+        if ((rc = gemv(pf_x, L.gate, &L.up, L.ln2, pf_g, kEpiSiluMul, n)) ||
+            (rc = gemv(pf_g, L.down, nullptr, nullptr, pf_x, kEpiAccum, n, reinterpret_cast<float *>(sums),
+                       sums ? sums_bytes : 0)))
+          return rc;
+        continue;
+      }
       if (gemm_digits) {
         // o_proj's finished rows go on as the normed input of gate and up: where
         // the matmul splits K over workgroups, the kernel that adds the slices
@@ -519,9 +559,6 @@ struct Qwen2Session : Session {
                          : gemm(pf_att, L.o, pf_x, n, true, L.ln2, pf_xn_bf)))
           return rc;
       }
-      const int64_t ld_gu = 2 * (int64_t)S.inter;
-      const Layer *nx = i + 1 < S.layers ? &layers[(size_t)i + 1] : nullptr;
-      const bool ahead = nx && !nx->qkv_f32;
       if (L.gate_up_joint) {
         // gate and up in one launch whose workgroups hold matching tiles of
         // both: SiLU(gate) * up leaves the matmul as the terms of down's input, or, since

@@ -820,7 +820,7 @@ def test_session_prefill_refuses_overflow(bh):
 # and one row too many
 @pytest.mark.parametrize("precision", ["digits", "digits2"])
 @pytest.mark.parametrize("hidden,heads,inter,n,chunks", [
-    (384, 3, 336, 2, {2}), (1536, 12, 8960, 27, {2, 9}), (1536, 12, 8960, 64, {3, 14}), (256, 4, 4112, 33, {2, 5}),
+    (384, 3, 336, 18, {2}), (1536, 12, 8960, 27, {2, 9}), (1536, 12, 8960, 64, {3, 14}), (256, 4, 4112, 33, {2, 5}),
     (100, 1, 16, 17, {2}), (1536, 12, 336, 128, {2, 5}), (384, 3, 336, 129, set())])
 def test_few_rows_become_digits_within_the_product(bh, hidden, heads, inter, n, chunks, precision):
     shape = Shape(layers=2, hidden=hidden, heads=heads, kv_heads=1, head_dim=128, inter=inter, vocab=320, max_len=n + 8) \
@@ -846,3 +846,39 @@ def test_few_rows_become_digits_within_the_product(bh, hidden, heads, inter, n, 
         else:  # some ten roundings on the way, of 2^-15 of a row's largest value
             g, w = np.asarray(g, np.float64), np.asarray(w, np.float64)
             assert np.linalg.norm(g - w) < 2.0**-10 * np.linalg.norm(w)
+
+
+# Up to 16 tokens through the products of a decode step: every row count at which their kernels change,
+# q | k | v of enough channels and of fewer, behind a context whose attention leaves parts to fold, gate and up
+# apart (a width that sixteen does not divide), and one token too many
+@pytest.mark.parametrize("precision", ["digits", "digits2", "bf16"])
+@pytest.mark.parametrize("hidden,heads,kv_heads,inter,before,n", [
+    (384, 12, 2, 336, 0, 1), (384, 12, 2, 336, 0, 2), (1088, 12, 2, 4112, 7, 5), (384, 12, 2, 336, 3, 9),
+    (1536, 12, 2, 8960, 0, 16), (384, 12, 2, 336, 400, 8), (384, 3, 1, 336, 0, 6), (384, 12, 2, 330, 0, 4),
+    (384, 12, 2, 336, 0, 17)])
+def test_prompts_of_few_tokens(bh, hidden, heads, kv_heads, inter, before, n, precision):
+    shape = Shape(layers=2, hidden=hidden, heads=heads, kv_heads=kv_heads, head_dim=128, inter=inter, vocab=320,
+                  max_len=before + n + 8)
+    toks = synthetic.first_tokens(shape, n, seed=n + inter).astype(np.int32)
+    sess, _ = synthetic.build_session(shape, context=before, ln_jitter=0.1)
+    bh.buddy_hip_variant_reset()
+    _, got = sess.prefill(toks, before, precision=precision)
+    wide = (heads + 2 * kv_heads) * 128 >= 2048
+    few = n <= 16 and inter % 16 == 0 and (wide or precision != "bf16")
+    ran = {k for k, v in tiles_run(bh).items() if v and ("pair" in k and "batch" not in k or "rope" in k or "rows_kernel" in k)}
+    if few and wide or n > 16:
+        assert bool(ran) == (n > 16), ran
+    rows = [sess.get_kv(j)[:, before:before + n] for j in (2, 3)]
+    sess.close()
+    sess, _ = synthetic.build_session(shape, context=before, ln_jitter=0.1)
+    for i, t in enumerate(toks):
+        _, want = sess.decode(int(t), before + i, want_logits=i + 1 == n)
+    pairs = [(got, want)] + [(rows[j - 2], sess.get_kv(j)[:, before:before + n]) for j in (2, 3)]
+    sess.close()
+    for g, w in pairs:
+        if precision == "digits" or few and wide and before < 200:
+            check_close(g, w)
+        else:
+            bound = 2.0**-10 if precision == "digits2" else 10 * 2.0**-9
+            g, w = np.asarray(g, np.float64), np.asarray(w, np.float64)
+            assert np.linalg.norm(g - w) < bound * np.linalg.norm(w)
