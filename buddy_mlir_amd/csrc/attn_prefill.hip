@@ -56,7 +56,8 @@ constexpr int lds_floats(int waves) { return kQFloats + waves * kSlotFloats + 2 
 // proportion to their key blocks; those of a query block split its key blocks
 // into equal contiguous shares, each with its own running (max, sum, output), and
 // the partial results meet in LDS at the end.  W = 8 and pairs while the launch
-// is at most one workgroup per compute unit.  A longer launch balances itself
+// is at most one workgroup per compute unit, and one query block (part 0 empty) while that is so
+// without pairs.  A longer launch balances itself
 // better with many workgroups of unequal length, the longest first: then a
 // workgroup takes one query block (part 0 empty), W = 4, two workgroups per
 // compute unit, so that one's staging and merge overlap the other's key loop.
@@ -434,18 +435,22 @@ int launch_attn_prefill(const AttnPrefillArgs &in, hipStream_t stream) {
   const int pairs = (a.nqb + 1) / 2;
   BH_REQUIRE(pairs <= 65535, "attn_prefill: q_len %d too long", in.q_len);
   constexpr int kComputeUnits = 256; // MI355X
-  a.paired = (int64_t)in.heads * pairs <= kComputeUnits;
+  // one query block to a workgroup of eight wavefronts while there are compute units for them (12 heads:
+  // 27 tokens 7.9 us, in pairs 8.7; 64 7.8 and 10.2; 128 8.9 and 12.7; 256 11.5 and 15.6; 330 15.5 and
+  // 16.9), then two
+  const bool eight = (int64_t)in.heads * pairs <= kComputeUnits;
+  a.paired = eight && (int64_t)in.heads * a.nqb > kComputeUnits;
   // group | paired << 12 | (65536 / group + 1) << 13: (h * multiplier) >> 16 == h / group
   // while heads * group < 65536
   BH_REQUIRE(a.group >= 1 && a.group < 4096 && (int64_t)in.heads * a.group < 65536,
              "attn_prefill: heads=%d group=%d", in.heads, a.group);
   const int gp = a.group | a.paired << 12 | (65536 / a.group + 1) << 13;
-  if (a.paired) {
+  if (eight) {
     static DynLdsOnce dyn_lds;
     BH_CHECK_HIP(ensure_dyn_lds(dyn_lds, reinterpret_cast<const void *>(attn_prefill_kernel<8>),
                                 (int)(lds_floats(8) * sizeof(float))));
     BH_NOTE_VARIANT(AttnPrefillFamily, 8);
-    hipLaunchKernelGGL(attn_prefill_kernel<8>, dim3(in.heads, (unsigned)pairs), dim3(8 * kWave),
+    hipLaunchKernelGGL(attn_prefill_kernel<8>, dim3(in.heads, (unsigned)(a.paired ? pairs : a.nqb)), dim3(8 * kWave),
                        lds_floats(8) * sizeof(float), stream, a.k, a.v, a.mask, a.kv_stride, gp, a.nqb,
                        a.q_len, a.k_len, a.q_offset, a);
   } else {

@@ -882,3 +882,9 @@ def test_prompts_of_few_tokens(bh, hidden, heads, kv_heads, inter, before, n, pr
             bound = 2.0**-10 if precision == "digits2" else 10 * 2.0**-9
             g, w = np.asarray(g, np.float64), np.asarray(w, np.float64)
             assert np.linalg.norm(g - w) < bound * np.linalg.norm(w)
+
+
+# The last launch of one query block to a workgroup of eight wavefronts, and the first of two
+@pytest.mark.parametrize("H,HKV,Lq,Lk", [(16, 4, 256, 256), (16, 4, 257, 300), (128, 16, 32, 40), (128, 16, 33, 33)])
+def test_prefill_attention_pairs_where_the_chip_is_full(bh, oracle, H, HKV, Lq, Lk):
+    test_prefill_attention_launches_of_several_rounds(bh, oracle, H, HKV, Lq, Lk)
