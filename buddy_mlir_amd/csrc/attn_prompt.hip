@@ -17,8 +17,8 @@
 // beside its tiles is some 9 us: the share, queries and their terms, the first tile's way.
 // 12 query heads, 2 KV heads, us per layer, this kernel and the fold behind it against
 // attn_prefill.hip and the conversion behind that (attn_prompt_pays says which is taken):
-//   2000 tokens 104 vs 156, 4096 tokens 332 vs 655, 150 behind 1900 36 vs 102,
-//   27 behind 1900 27 vs 98, 512 tokens 28 vs 25, 256 tokens 21 vs 17
+//   2000 tokens 104 vs 156, 4096 tokens 332 vs 655, 150 behind 1900 36 vs 64,
+//   27 behind 1900 27 vs 58, 512 tokens 28 vs 25, 256 tokens 21 vs 17
 #include "attn.h"
 #include "attn_fold.h"
 #include "bf16_dev.h"
@@ -483,30 +483,34 @@ PromptShare share_out(int q_len, int q_offset, int heads, int kv_heads) {
 }
 } // namespace
 
-// An estimate of both ways in microseconds, fitted to 528 launches of 1 to 64 heads, 1 to 16 KV
-// heads, 2 to 2000 tokens behind 0 to 1900.  Of those the choice is up to 15 % slower than the
-// better way and 0.5 % on average.  us, this way and the other, where the line lies:
-//   12 heads, 2 KV heads: 27 behind 128 15.8, 17.5, 300 behind 128 28.0, 24.5, behind 400 36.2,
-//     37.1, 512 alone 27.7, 25.3, 700 38.8, 35.0, 1024 49.3, 53.2
-//   64 and 8: 27 behind 128 24.7, 20.0, 300 behind 128 51.9, 56.1, 640 alone 84.8, 106
-//   one head: 300 behind 64 19.0, 20.9, 8 behind 128 12.4, 10.7
-// The estimate is off by a tenth here and there.  More than 640 tokens go this way in doubt,
-// which keeps what is not finite to the rows that see it (700 tokens of 6 heads, one KV head:
-// 28.5 and 29.3); short prompts with little ahead of them the other.
-bool attn_prompt_pays(int q_len, int q_offset, int heads, int kv_heads) {
+// An estimate of both ways in microseconds, fitted to 1568 prompts of 12 layers: eight shapes of 1 to
+// 64 heads, 4 to 640 tokens behind 0 to 1200, in three modes.  `converts`: behind the other way the
+// rows take a launch of their own to become the output product's input, which the fold is here
+// (not up to 16 tokens as f32, nor up to 128 as digits, which that product makes itself).
+// The choice is up to 13 % of a layer slower than the better way and 0.25 % on average.  us a
+// layer with its products, the other way and this one, where the line lies:
+//   12 heads, 2 KV heads, digits: 4 behind 400 40.9, 42.3, behind 700 47.0, 43.9, 32 behind 256
+//     53.3, 54.9, behind 700 60.7, 58.0, 256 behind 400 70.1, 70.1, 500 alone 74.9, 75.6, behind
+//     128 79.5, 86.7, behind 400 93.0, 90.3
+//   64 and 8, digits: 32 behind 256 63.6, 77.2, 128 behind 700 107.7, 107.0, 256 behind 128 111,
+//     115, behind 256 123, 118, 500 alone 165, 160
+//   one head, every bit: 64 behind 64 54.7, 56.5, behind 128 57.4, 56.8, 256 behind 64 65.6, 64.6
+// More than 32 tokens behind 400 and more go this way in doubt, up to 6 us: it asks for each key
+// once for all heads of a KV head, and what is not finite stays with the rows that see it.
+bool attn_prompt_pays(int q_len, int q_offset, int heads, int kv_heads, bool converts) {
   const double kilo_rows = 1e-4 * q_len * heads; // tens of thousands of (token, head)
-  // attn_prefill.hip: blocks of 16 queries, two together while a workgroup of eight wavefronts
-  // per pair fits the chip; steps of 16 keys per wavefront
+  // attn_prefill.hip: blocks of 16 queries, one to a workgroup of eight wavefronts, then two, while
+  // those fit the chip; steps of 16 keys per wavefront
   const int64_t nqb = ceil_div(q_len, 16);
   double steps;
-  if (nqb == 1)
-    steps = (double)ceil_div(q_offset + q_len, 16) / 8;
+  if (nqb == 1 || heads * nqb <= 256)
+    steps = 2.7 * (double)ceil_div(q_offset + q_len, 16) / 8;
   else if (heads * ceil_div(nqb, 2) <= 256)
-    steps = (2.0 * q_offset + q_len + 16) / 128;
+    steps = 1.5 + 2.4 * (2.0 * q_offset + q_len + 16) / 128;
   else
-    steps = (1.0 * heads * q_len * q_len / (16 * 32 * 256) +
-             (double)ceil_div(heads * nqb, 256) * q_offset / 16) / 8;
-  const double other = 7.9 + (nqb > 1 ? 2.1 : 0.0) + 3.0 * steps + 5.8 * kilo_rows;
+    steps = 3.3 + 2.7 * (1.0 * heads * q_len * q_len / (16 * 32 * 256) +
+                         (double)ceil_div(heads * nqb, 256) * q_offset / 16) / 8;
+  const double other = 4.7 + (converts ? 3.9 : 0.0) + steps + 3.3 * kilo_rows;
   // here: tiles of the longest share, wavefronts that have rows, blocks that begin and end, and
   // the fold's trips to memory and its bytes
   const PromptShare s = share_out(q_len, q_offset, heads, kv_heads);
@@ -514,11 +518,12 @@ bool attn_prompt_pays(int q_len, int q_offset, int heads, int kv_heads) {
   const double parts = (double)ceil_div(q_offset + q_len, kKeys) / share;
   const int64_t waves = std::min<int64_t>(8, ceil_div(s.rows, 32));
   const double trips = parts <= 4 ? 1 : parts <= 8 ? 2 : 2 * std::ceil(parts / 16);
-  const double here = 10.6 + 5.7 * (double)(ceil_div(s.tiles, s.workgroups) - 1) +
-                      1.4 * (double)std::max<int64_t>(0, waves - 4) + 5.0 * s.workgroups / 256 +
-                      2.0 * s.nblk * kv_heads / s.workgroups + (double)ceil_div(heads, 16) * trips +
-                      0.82 * kilo_rows * std::min(parts, 20.0);
-  return here < (q_len > 640 ? 1.08 : q_offset >= 128 ? 1.0 : 0.9) * other;
+  const double here = 10.6 + 5.1 * (double)(ceil_div(s.tiles, s.workgroups) - 1) +
+                      0.8 * (double)std::max<int64_t>(0, waves - 4) + 4.3 * s.workgroups / 256 +
+                      0.85 * s.nblk * kv_heads / s.workgroups +
+                      0.9 * (double)ceil_div(heads, 16) * trips +
+                      0.46 * kilo_rows * std::min(parts, 20.0);
+  return here < other + (q_len > 32 && q_offset >= 400 ? 6.0 : 0.0);
 }
 
 // Two slots for every workgroup there can be: 67 MB where all compute units have tiles.

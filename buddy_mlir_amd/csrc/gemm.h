@@ -100,6 +100,7 @@ int launch_gemm_w8_digits(const GemmW8Args &a, const void *planes, hipStream_t s
 // the matmul over few f32 rows A (not staged), turned into digits slice by slice of K, whose steps
 // are never coarser than a row's own; done stays false where there are too many rows or no cut of K
 // suits: nothing has been launched then
+constexpr int kDigitRowsMax = 128;
 int launch_gemm_w8_digits_rows(const GemmW8Args &a, bool *done, hipStream_t stream);
 
 int launch_gemm_w8(const GemmW8Args &a, hipStream_t stream);

@@ -1762,10 +1762,10 @@ int launch_gemm_w8_digits_rows(const GemmW8Args &in, bool *done, hipStream_t str
   BH_REQUIRE(in.A && in.W && in.scale && in.C && in.M > 0 && in.K > 0 && in.N > 0 && in.lda >= in.K && in.ldc >= in.N &&
                  (in.digits == 2 || in.digits == 3) && !in.staged && !in.silu_pair && !in.then_rope,
              "gemm_w8: rows as they come");
-  // rows are read 16 bytes at a time; beyond 128 of them (three planes: 129 rows 2426 -> 2335 us a
+  // rows are read 16 bytes at a time; beyond kDigitRowsMax (three planes: 129 rows 2426 -> 2335 us a
   // prompt, 256 the same; two: 180 rows 1 % longer) a launch for the digits is a small part
   const bool aligned = ((in.K | in.lda) & 3) == 0 && (reinterpret_cast<uintptr_t>(in.A) & 15) == 0;
-  const int c = in.M <= 128 && aligned && in.lda < (1 << 30) ? rows_chunks(in.M, in.K, in.N) : 0;
+  const int c = in.M <= kDigitRowsMax && aligned && in.lda < (1 << 30) ? rows_chunks(in.M, in.K, in.N) : 0;
   if (!c)
     return BUDDY_HIP_OK;
   GemmI8Args a{};

@@ -453,9 +453,6 @@ struct Qwen2Session : Session {
                        pf_tokens, (int64_t)S.hidden, (int64_t)S.vocab, pf_x);
     BH_CHECK_HIP(hipGetLastError());
     int rc;
-    const bool folded = attn_prompt_pays(n, start_pos, S.heads, S.kv_heads);
-    if (folded && !pf_attn_ws) // for as many rows as the other buffers have, behind any context
-      BH_CHECK_HIP(hipMalloc(&pf_attn_ws, attn_prompt_workspace_bytes(pf_rows, S.max_len, S.heads, S.kv_heads)));
     // Up to 16 tokens go through the products of a decode step, which read f32 rows, norm them, turn
     // them into digits of 2^-23 of their largest and add to the residual themselves: five to seven
     // launches a layer for the prompt's eight, whose tiles of 32 rows are mostly padding here.  (Not where
@@ -463,6 +460,11 @@ struct Qwen2Session : Session {
     // 1 token 878 and 1504, 2 973 and 1491, 5 1165 and 1527, 9 1236 and 1545, 16 1272 and 1546; cast to
     // bfloat16 913 and 1516, 971 and 1504, 1166 and 1503, 1228 and 1524, 1278 and 1539.
     const bool few = n <= kFewTokens && (gemm_digits || (gemm_terms == 1 && QKV >= kFewChannels));
+    // attention's rows go to their product as they are (few) or it makes their digits (gemm_digit_rows)
+    const bool converts = !few && !(gemm_digits && n <= kDigitRowsMax);
+    const bool folded = attn_prompt_pays(n, start_pos, S.heads, S.kv_heads, converts);
+    if (folded && !pf_attn_ws) // for as many rows as the other buffers have, behind any context
+      BH_CHECK_HIP(hipMalloc(&pf_attn_ws, attn_prompt_workspace_bytes(pf_rows, S.max_len, S.heads, S.kv_heads)));
     bool normed_ahead = false; // pf_xn_bf already holds this layer's normed input
     for (int i = 0; i < S.layers; ++i) {
       Layer &L = layers[(size_t)i];
