@@ -17,13 +17,26 @@ namespace {
 
 constexpr int kTile = kHeadKeyTile;
 
-// coordinate i of the rotated head that lies at v; cs: [cos | sin] of the pairs
+// coordinate i of a rotated head out of the head at v: itself and the one it is turned with; cs:
+// [cos | sin] of the pairs
+struct Turned {
+  float own, other;
+  __device__ __forceinline__ void load(const float *v, int i, int half) {
+    own = v[i];
+    other = v[i < half ? i + half : i < 2 * half ? i - half : i];
+  }
+  __device__ __forceinline__ float by(int i, int half, const float *cs) const {
+    if (i >= 2 * half)
+      return own;
+    const int f = i < half ? i : i - half;
+    const float c = cs[f], s = cs[half + f];
+    return i < half ? own * c - other * s : own * c + other * s;
+  }
+};
 __device__ __forceinline__ float turned(const float *v, int i, int half, const float *cs) {
-  if (i >= 2 * half)
-    return v[i];
-  const int f = i < half ? i : i - half;
-  const float u = v[f], w = v[f + half], c = cs[f], s = cs[half + f];
-  return i < half ? u * c - w * s : w * c + u * s;
+  Turned t;
+  t.load(v, i, half);
+  return t.by(i, half, cs);
 }
 template <typename T> __device__ __forceinline__ float as_stored(float v) {
   return sizeof(T) == 2 ? bf_f(f_bf(v)) : v;
@@ -76,6 +89,22 @@ head_part_kernel(const float *__restrict__ proj, T *__restrict__ keys, T *__rest
   const int q0 = blockIdx.z * 16, nq = min(16, a.group - q0);
   T *kc = keys + (int64_t)gm * a.rows * dim32;
   T *vc = values_t + (int64_t)g * vdim16 * a.rows;
+  // the new position's projections and the rotation's frequencies, asked for ahead of all that waits
+  // for the position: a trip to memory less in the chain
+  constexpr int kAheadQ = 4;
+  Turned qt[kAheadQ], kt;
+  auto query_at = [&](int h) {
+    return proj + a.q_at + (int64_t)((g * a.group + q0 + min(h, nq - 1)) * a.maps + map) * a.dim;
+  };
+#pragma unroll
+  for (int j = 0; j < kAheadQ; ++j) {
+    const int i = tid + j * 256, h = i / dim32, d = i - h * dim32;
+    qt[j].load(query_at(h), min(d, a.dim - 1), a.half);
+  }
+  const float *new_key = proj + a.k_at + (int64_t)gm * a.dim;
+  kt.load(new_key, min(tid, a.dim - 1), a.half);
+  const float vt = proj[a.v_at + (int64_t)g * a.vdim + min(tid, a.vdim - 1)];
+  const double turn = tid < a.half ? turns[tid] : 0.0;
   const int p = *pos;
   const int lo = max(0, p - a.window + 1);
   const int first = (lo & ~(kTile - 1)) + blockIdx.x * a.tiles * kTile;
@@ -116,28 +145,39 @@ head_part_kernel(const float *__restrict__ proj, T *__restrict__ keys, T *__rest
 
   for (int f = tid; f < a.half; f += 256) {
     float c, s;
-    rotation(turns[f], p, c, s);
+    rotation(f == tid ? turn : turns[f], p, c, s);
     cs[f] = c * a.rot_gain;
     cs[a.half + f] = s * a.rot_gain;
   }
   __syncthreads();
-  for (int i = tid; i < 16 * dim32; i += 256) {
+  auto keep_query = [&](int h, int d, const Turned &t) {
+    qs[h * qrow + d] = h < nq && d < a.dim ? t.by(d, a.half, cs) * a.scale : 0.f;
+  };
+#pragma unroll
+  for (int j = 0; j < kAheadQ; ++j) {
+    const int i = tid + j * 256, h = i / dim32, d = i - h * dim32;
+    if (h < 16)
+      keep_query(h, d, qt[j]);
+  }
+  for (int i = tid + kAheadQ * 256; i < 16 * dim32; i += 256) {
     const int h = i / dim32, d = i - h * dim32;
-    float v = 0.f;
+    Turned t{};
     if (h < nq && d < a.dim)
-      v = turned(proj + a.q_at + (int64_t)((g * a.group + q0 + h) * a.maps + map) * a.dim, d, a.half, cs) * a.scale;
-    qs[h * qrow + d] = v;
+      t.load(query_at(h), d, a.half);
+    keep_query(h, d, t);
   }
   if (has_new) {
     const bool keeper = blockIdx.z == 0;
     for (int d = tid; d < dim32; d += 256) {
-      const float v = d < a.dim ? turned(proj + a.k_at + (int64_t)gm * a.dim, d, a.half, cs) : 0.f;
+      if (d != tid)
+        kt.load(new_key, min(d, a.dim - 1), a.half);
+      const float v = d < a.dim ? kt.by(d, a.half, cs) : 0.f;
       nk[d] = as_stored<T>(v);
       if (keeper)
         store_act<T>(kc + (int64_t)(p & a.ring_mask) * dim32 + d, v);
     }
     for (int c = tid; c < vdim16; c += 256) {
-      const float v = c < a.vdim ? proj[a.v_at + (int64_t)g * a.vdim + c] : 0.f;
+      const float v = c < a.vdim ? (c == tid ? vt : proj[a.v_at + (int64_t)g * a.vdim + c]) : 0.f;
       nv[c] = as_stored<T>(v);
       if (keeper && map == 0)
         store_act<T>(vc + (int64_t)c * a.rows + (p & a.ring_mask), v);
