@@ -146,7 +146,7 @@ finish_step_kernel(const float *__restrict__ pv, const int *__restrict__ pi,
                    const Table *__restrict__ table, float table_scale, int64_t hidden,
                    int64_t vocab, float *__restrict__ x, const float *__restrict__ inv_freq,
                    int half, float *__restrict__ rope, int advance, int log_cap,
-                   const float *__restrict__ norm_w, float eps) {
+                   const float *__restrict__ norm_w, float eps, StepGiven given) {
   __shared__ float sv[16];
   __shared__ int si[16];
   __shared__ int s_tok, s_pos;
@@ -155,9 +155,15 @@ finish_step_kernel(const float *__restrict__ pv, const int *__restrict__ pi,
   // the pick (only thread 0 uses them)
   int st_tok = 0, st_pos = 0, st_step = 0;
   if (threadIdx.x == 0) {
-    st_tok = state[0];
-    st_pos = state[1];
-    st_step = state[2];
+    if (given.token >= 0 || given.at) {
+      state[0] = st_tok = given.at ? given.at[0] : given.token;
+      state[1] = st_pos = given.at ? given.at[1] : given.pos;
+      state[2] = st_step = given.at ? given.at[2] : given.step;
+    } else {
+      st_tok = state[0];
+      st_pos = state[1];
+      st_step = state[2];
+    }
   }
   if (nparts > 0) {
     float v = -INFINITY;
@@ -254,14 +260,14 @@ finish_step_kernel(const float *__restrict__ pv, const int *__restrict__ pi,
 int launch_finish_step(const float *cand_v, const int *cand_i, int nparts, int *state,
                        int *token_log, const float *table, int64_t hidden, int64_t vocab,
                        float *x, const float *inv_freq, int head_dim, float *rope,
-                       bool advance, int token_log_cap, hipStream_t stream) {
+                       bool advance, int token_log_cap, hipStream_t stream, StepGiven given) {
   BH_REQUIRE(state && table && x && inv_freq && rope && head_dim > 0 &&
-                 head_dim / 2 <= 256 && (nparts == 0 || (cand_v && cand_i && token_log)),
+                 head_dim / 2 <= 256 && (nparts == 0 || (cand_v && cand_i && token_log && !given.any())),
              "finish_step: bad argument");
   hipLaunchKernelGGL(finish_step_kernel<float>, dim3(1), dim3(nparts > 1024 ? 1024 : 256), 0,
                      stream, cand_v, cand_i, nparts, state, token_log, table, 1.0f, hidden, vocab,
                      x, inv_freq, head_dim / 2, rope, advance ? 1 : 0, token_log_cap,
-                     (const float *)nullptr, 0.f);
+                     (const float *)nullptr, 0.f, given);
   BH_CHECK_HIP(hipGetLastError());
   return BUDDY_HIP_OK;
 }
@@ -269,13 +275,13 @@ int launch_finish_step(const float *cand_v, const int *cand_i, int nparts, int *
 int launch_finish_step_bf16(const float *cand_v, const int *cand_i, int nparts, int *state,
                             int *token_log, const uint16_t *table, float table_scale,
                             const float *norm_w, float eps, int64_t hidden, int64_t vocab, float *x,
-                            bool advance, int token_log_cap, hipStream_t stream) {
-  BH_REQUIRE(state && table && x && (nparts == 0 || (cand_v && cand_i && token_log)),
+                            bool advance, int token_log_cap, hipStream_t stream, StepGiven given) {
+  BH_REQUIRE(state && table && x && (nparts == 0 || (cand_v && cand_i && token_log && !given.any())),
              "finish_step: bad argument");
   hipLaunchKernelGGL(finish_step_kernel<uint16_t>, dim3(1), dim3(nparts > 1024 ? 1024 : 256), 0,
                      stream, cand_v, cand_i, nparts, state, token_log, table, table_scale, hidden,
                      vocab, x, (const float *)nullptr, 0, (float *)nullptr, advance ? 1 : 0,
-                     token_log_cap, norm_w, eps);
+                     token_log_cap, norm_w, eps, given);
   BH_CHECK_HIP(hipGetLastError());
   return BUDDY_HIP_OK;
 }

@@ -8,24 +8,17 @@
 // captured once into a hipGraph and replayed; greedy decoding feeds the argmax
 // straight into the next step's embedding gather without a host round trip.
 #include "session_base.h"
-#include "elementwise.h"
 
 #include <algorithm>
+#include <chrono>
 #include <cstring>
+#include <thread>
 #include <vector>
 
 namespace bh {
 namespace {
 
-constexpr size_t kHostWords = 4; // ahead of the logits in the pinned buffer
-
-__global__ void write_state_kernel(int *state, int token, int pos, int step) {
-  if (threadIdx.x == 0) {
-    state[0] = token;
-    state[1] = pos;
-    state[2] = step;
-  }
-}
+constexpr size_t kGivenWord = 4, kHostWords = 8; // what is given, the logits in the pinned buffer
 
 // State and n logits into the pinned buffer: one launch in place of a copy of the state and
 // one of the logits through the runtime's staging, which blocks.  With the state of the
@@ -33,7 +26,7 @@ __global__ void write_state_kernel(int *state, int token, int pos, int step) {
 // layers behind a prompt of 45, each with its logits, took 7277 us instead of 7975.
 __global__ void __launch_bounds__(256)
 hand_out_kernel(const int *__restrict__ state, const float *__restrict__ logits, int n,
-                int *__restrict__ out) {
+                int *__restrict__ out, int *__restrict__ done) {
   const int i = (blockIdx.x * 256 + threadIdx.x) * 4;
   if (i == 0)
     for (int w = 0; w < 3; ++w)
@@ -44,7 +37,13 @@ hand_out_kernel(const int *__restrict__ state, const float *__restrict__ logits,
   else
     for (int e = i; e < n; ++e)
       dst[e] = logits[e];
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0)
+    __hip_atomic_store(done + blockIdx.x, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
+size_t done_word(int vocab) { return kHostWords + (size_t)round_up(vocab, 4); }
+int hand_blocks(int n) { return (int)std::max<int64_t>(1, ceil_div(n, 1024)); }
 
 // Memory that the runtime does not know: a copy to it goes through a buffer of its own,
 // piece by piece, and blocks.
@@ -89,7 +88,8 @@ int Session::init(int vocab_size, int capacity, hipStream_t on_stream) {
   rc |= alloc(&group_max_i, groups);
   if (rc)
     return rc;
-  BH_CHECK_HIP(hipHostMalloc((void **)&host_state, 4 * (kHostWords + (size_t)vocab)));
+  BH_CHECK_HIP(hipHostMalloc((void **)&host_state, 4 * (done_word(vocab) + (size_t)hand_blocks(vocab)),
+                             hipHostMallocCoherent));
   BH_CHECK_HIP(hipMemsetAsync(state, 0, 4 * sizeof(int), stream));
   BH_CHECK_HIP(hipStreamSynchronize(stream));
   return BUDDY_HIP_OK;
@@ -118,14 +118,23 @@ int Session::check_steps(int steps, const char *who) const {
   return BUDDY_HIP_OK;
 }
 
-int Session::run_step() {
+int Session::enqueue_whole_step(bool hands) {
+  int rc = BUDDY_HIP_OK;
+  if (hands)
+    rc = prepare_step({-1, 0, 0, host_state + kGivenWord});
+  if (!rc)
+    rc = enqueue_step(next_pos);
+  return rc || !hands ? rc : enqueue_hand_out(vocab);
+}
+
+int Session::run_step(bool hands) {
   int rc = check_steps(1, "decode step");
   if (rc)
     return rc;
   if (!use_graph) {
-    rc = enqueue_step(next_pos);
+    rc = enqueue_whole_step(hands);
   } else {
-    const std::pair<int, int> key = step_key(next_pos);
+    const std::pair<std::pair<int, int>, bool> key{step_key(next_pos), hands};
     auto it = graphs.find(key);
     if (it == graphs.end()) {
       if (graphs.size() >= kMaxStepGraphs) {
@@ -137,7 +146,7 @@ int Session::run_step() {
     StepGraph &g = it->second;
     if (!g.exec) {
       BH_CHECK_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-      rc = enqueue_step(next_pos);
+      rc = enqueue_whole_step(hands);
       hipError_t e = hipStreamEndCapture(stream, &g.graph);
       if (!rc && e != hipSuccess)
         rc = fail(BUDDY_HIP_ERR_HIP, "hipStreamEndCapture: %s", hipGetErrorString(e));
@@ -175,9 +184,40 @@ int Session::set_state(int token, int pos, int step) {
     return rc;
   next_pos = pos;
   next_step = step;
-  hipLaunchKernelGGL(write_state_kernel, dim3(1), dim3(64), 0, stream, state, token, pos, step);
+  return prepare_step({token, pos, step});
+}
+
+int *Session::hand_done() const { return host_state + done_word(vocab); }
+
+int Session::enqueue_hand_out(int n) {
+  hipLaunchKernelGGL(hand_out_kernel, dim3((unsigned)hand_blocks(n)), dim3(256), 0, stream, state,
+                     logits, n, host_state, hand_done());
   BH_CHECK_HIP(hipGetLastError());
-  return prepare_step();
+  return BUDDY_HIP_OK;
+}
+
+// Its last kernel says in the pinned buffer that it is there.
+// The words are looked at for up to kLookUs, which a step is shorter than; whoever takes longer, or
+// has failed, is waited for (and reported) by the runtime, whose wait sleeps and takes up to 20 us
+// to come back.
+int Session::wait_hand_out(int n) {
+  constexpr int kLookUs = 2000, kYieldUs = 100;
+  const int blocks = hand_blocks(n);
+  const auto t0 = std::chrono::steady_clock::now();
+  for (int b = 0; b < blocks;) {
+    if (__atomic_load_n(hand_done() + b, __ATOMIC_ACQUIRE)) {
+      ++b;
+      continue;
+    }
+    const auto us = std::chrono::duration_cast<std::chrono::microseconds>(std::chrono::steady_clock::now() - t0);
+    if (us.count() > kLookUs) {
+      BH_CHECK_HIP(hipStreamSynchronize(stream));
+      return BUDDY_HIP_OK;
+    }
+    if (us.count() > kYieldUs)
+      std::this_thread::yield();
+  }
+  return BUDDY_HIP_OK;
 }
 
 int Session::hand_out(float *logits_out, int *next_token) {
@@ -186,12 +226,47 @@ int Session::hand_out(float *logits_out, int *next_token) {
     BH_CHECK_HIP(hipMemcpyAsync(logits_out, logits, sizeof(float) * vocab, hipMemcpyDefault,
                                 stream));
   const int n = staged ? vocab : 0;
-  hipLaunchKernelGGL(hand_out_kernel, dim3((unsigned)std::max<int64_t>(1, ceil_div(n, 1024))),
-                     dim3(256), 0, stream, state, logits, n, host_state);
-  BH_CHECK_HIP(hipGetLastError());
-  BH_CHECK_HIP(hipStreamSynchronize(stream));
+  std::fill_n(hand_done(), hand_blocks(n), 0);
+  int rc = enqueue_hand_out(n);
+  if (rc)
+    return rc;
+  if (logits_out && !staged)
+    BH_CHECK_HIP(hipStreamSynchronize(stream));
+  else if ((rc = wait_hand_out(n)))
+    return rc;
   if (staged)
     std::memcpy(logits_out, host_state + kHostWords, sizeof(float) * vocab);
+  if (next_token)
+    *next_token = host_state[0];
+  return BUDDY_HIP_OK;
+}
+
+int Session::step_and_hand_out(int token, int pos, float *logits_out, int *next_token) {
+  // a step that other calls have captured serves the first of these too: capturing costs some 400 us
+  bool apart = !logits_out || !pageable(logits_out);
+  if (!apart && use_graph) {
+    const auto it = graphs.find({step_key(pos), false});
+    if (it != graphs.end() && !it->second.handed)
+      apart = it->second.handed = true;
+  }
+  int rc;
+  if (apart) {
+    if ((rc = set_state(token, pos, 0)) || (rc = run_step()))
+      return rc;
+    return hand_out(logits_out, next_token);
+  }
+  if ((rc = seek(pos)))
+    return rc;
+  next_pos = pos;
+  next_step = 0;
+  int *given = host_state + kGivenWord;
+  given[0] = token;
+  given[1] = pos;
+  given[2] = 0;
+  std::fill_n(hand_done(), hand_blocks(vocab), 0);
+  if ((rc = run_step(true)) || (rc = wait_hand_out(vocab)))
+    return rc;
+  std::memcpy(logits_out, host_state + kHostWords, sizeof(float) * vocab);
   if (next_token)
     *next_token = host_state[0];
   return BUDDY_HIP_OK;
@@ -226,14 +301,11 @@ int buddy_hip_session_decode_mirror(buddy_hip_session *hs, int token, int pos,
   BH_REQUIRE(pos >= 0 && pos < s->max_len,
              "session_decode: position %d outside the cache (max_len %d)", pos,
              s->max_len);
-  if ((rc = s->set_state(token, pos, 0)))
+  if (!kv_rows_out)
+    return s->step_and_hand_out(token, pos, logits_out, next_token);
+  // and the cache rows this step wrote, all layers
+  if ((rc = s->set_state(token, pos, 0)) || (rc = s->run_step()) || (rc = s->copy_kv_rows(pos, 1, kv_rows_out)))
     return rc;
-  if ((rc = s->run_step()))
-    return rc;
-  if (kv_rows_out) { // the cache rows this step wrote, all layers
-    if ((rc = s->copy_kv_rows(pos, 1, kv_rows_out)))
-      return rc;
-  }
   return s->hand_out(logits_out, next_token);
 } BH_CATCH_INT("buddy_hip_session_decode_mirror")
 

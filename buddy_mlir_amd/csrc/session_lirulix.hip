@@ -439,14 +439,14 @@ struct LirulixSession : FolderSession {
     g.valid = cfg.vocab;
     if ((rc = launch_row_gemv(g, stream)))
       return rc;
-    return finish(group_max_v, group_max_i, head.groups(), true);
+    return finish(group_max_v, group_max_i, head.groups(), true, {});
   }
 
-  int finish(const float *cand_v, const int *cand_i, int parts, bool advance) {
+  int finish(const float *cand_v, const int *cand_i, int parts, bool advance, const StepGiven &given) {
     return launch_finish_step_bf16(cand_v, cand_i, parts, state, token_log, embed, 1.0f, embed_norm,
-                                   cfg.eps, cfg.width, cfg.vocab, x[0], advance, token_log_cap, stream);
+                                   cfg.eps, cfg.width, cfg.vocab, x[0], advance, token_log_cap, stream, given);
   }
-  int prepare_step() override { return finish(nullptr, nullptr, 0, false); }
+  int prepare_step(const StepGiven &given) override { return finish(nullptr, nullptr, 0, false, given); }
 
   // ---- many tokens -----------------------------------------------------------------
   int alloc_block(int rows) override {

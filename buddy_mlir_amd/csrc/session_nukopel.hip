@@ -457,9 +457,9 @@ struct NukopelSession : FolderSession {
                                    cfg.embed_scale, nullptr, 0.f, W, cfg.vocab, x[0], true, token_log_cap, stream);
   }
 
-  int prepare_step() override {
+  int prepare_step(const StepGiven &given) override {
     return launch_finish_step_bf16(nullptr, nullptr, 0, state, token_log, embed, cfg.embed_scale,
-                                   nullptr, 0.f, cfg.width, cfg.vocab, x[0], false, token_log_cap, stream);
+                                   nullptr, 0.f, cfg.width, cfg.vocab, x[0], false, token_log_cap, stream, given);
   }
 
   // ---- many tokens -----------------------------------------------------------------

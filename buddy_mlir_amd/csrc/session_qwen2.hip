@@ -298,11 +298,11 @@ struct Qwen2Session : Session {
   }
 
   // After the host wrote token/position: embedding row and RoPE table of the step.
-  int prepare_step() override {
+  int prepare_step(const StepGiven &given) override {
     const auto &S = shape;
     return launch_finish_step(nullptr, nullptr, 0, state, token_log, embed, S.hidden, S.vocab,
                               x, inv_freq, S.head_dim, rope, false, token_log_cap,
-                              stream);
+                              stream, given);
   }
 
   int ensure_prefill_buffers(int rows) {

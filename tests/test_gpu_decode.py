@@ -517,6 +517,34 @@ def test_small_model_greedy_feedback_matches_stepwise(oracle):
     sess.close()
 
 
+@pytest.mark.parametrize("vocab", [1, 1021, 1024, 1025, 4100])
+def test_a_step_with_its_logits_in_one_graph(vocab):
+    """The graph that begins with the token the host gives and ends with the logits in pinned
+    memory, the one that greedy steps captured, and launches without a graph: the same bits."""
+    shape = Shape(layers=1, hidden=256, heads=2, kv_heads=1, head_dim=128, inter=256, vocab=vocab,
+                  max_len=64, rms_eps=1e-6)
+    rng = np.random.default_rng(vocab)
+    fed = rng.integers(0, vocab, 12)
+    runs = []
+    for graph, greedy_first in ((False, False), (True, False), (True, True)):
+        sess, _ = synthetic.build_session(shape, context=16, ln_jitter=0.1)
+        sess.use_graph(graph)
+        if greedy_first:
+            sess.decode_greedy(int(fed[0]), 16, 1)
+        out = []
+        for i, tok in enumerate(fed):
+            nxt, logits = sess.decode(int(tok), 16 + i)
+            out.append(logits)
+            assert nxt == int(logits.argmax())
+            if i % 3 == 1:  # other calls in between: no logits, and steps of the device's own
+                assert sess.decode(int(tok), 16 + i, want_logits=False)[0] == nxt
+                sess.decode_greedy(nxt, 17 + i, 2)
+        runs.append(np.stack(out))
+        sess.close()
+    np.testing.assert_array_equal(runs[0], runs[1])
+    np.testing.assert_array_equal(runs[0], runs[2])
+
+
 def test_session_refuses_bad_arguments(bh):
     sess, _ = synthetic.build_session(SMALL, context=0)
     with pytest.raises(bma.BuddyHipError):
