@@ -37,7 +37,7 @@ hand_out_kernel(const int *__restrict__ state, const float *__restrict__ logits,
   else
     for (int e = i; e < n; ++e)
       dst[e] = logits[e];
-  __threadfence_system();
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // a fence of all: 22 us for 608 KB, not 16
   __syncthreads();
   if (threadIdx.x == 0)
     __hip_atomic_store(done + blockIdx.x, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
