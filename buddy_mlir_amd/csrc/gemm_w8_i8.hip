@@ -523,7 +523,7 @@ __device__ __forceinline__ void finish_tile(const GemmI8Args &a, const v16i32 (&
 }
 
 template <int D, int RB, int GP, bool PAIR>
-__device__ __forceinline__ void multiply_tile(const GemmI8Args &a) {
+__device__ __forceinline__ void multiply_tile(const GemmI8Args &a, int unit, int rbk, int row0 = 0) {
   constexpr int kWidth = PAIR ? 16 : 32;    // channels of the result per tile
   constexpr int kSpan = kWidth * GP;        // ... and per wavefront
   constexpr int kRows = 32 * RB;            // rows of the tile
@@ -551,11 +551,8 @@ __device__ __forceinline__ void multiply_tile(const GemmI8Args &a) {
   __shared__ float step_s[kRows];
   const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, up = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  int unit, rbk;
-  if (!place_tile(a.ncols * a.slices, a.row_tiles, a.panel, unit, rbk))
-    return;
   const int ctile = unit % a.ncols, slice = unit / a.ncols;
-  const int m0 = rbk * kRows;
+  const int m0 = row0 + rbk * kRows;
   const int half_groups = a.groups / 2; // PAIR only
   const int glast = PAIR ? half_groups - 1 : a.groups - 1;
   const int g0 = (ctile * kSlices + wave) * (kSpan / 16); // first channel group of this wavefront
@@ -759,7 +756,7 @@ template <int N> __device__ __forceinline__ void landed() {
 constexpr bool tall_shares(int D, int GP) { return D >= 2 && GP == 2; }
 
 template <int D, int RB, int GP, bool PAIR>
-__device__ __forceinline__ void multiply_block(const GemmI8Args &a) {
+__device__ __forceinline__ void multiply_block(const GemmI8Args &a, int unit, int rbk) {
   constexpr int kWidth = PAIR ? 16 : 32, kSpan = kWidth * GP, kRows = 32 * RB, L = D * RB;
   constexpr int kThreads = kSlices * kWave;
   constexpr int kRing = 4;                    // chunks of rows in LDS, half chunks of weights in registers
@@ -773,9 +770,6 @@ __device__ __forceinline__ void multiply_block(const GemmI8Args &a) {
   __shared__ float step_s[kRows];
   const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, up = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  int unit, rbk;
-  if (!place_tile(a.ncols * a.slices, a.row_tiles, a.panel, unit, rbk))
-    return;
   const int ctile = unit % a.ncols, slice = unit / a.ncols;
   const int m0 = rbk * kRows;
   const int half_groups = a.groups / 2; // PAIR only
@@ -924,21 +918,55 @@ __device__ __forceinline__ void multiply_block(const GemmI8Args &a) {
 template <int D, bool PAIR>
 __global__ void __launch_bounds__(kSlices *kWave) gemm_w8_i8_kernel(BH_I8_LEADING) {
   BH_I8_TAKE
-  multiply_tile<D, 1, 1, PAIR>(a);
+  int unit, rbk;
+  if (!place_tile(a.ncols * a.slices, a.row_tiles, a.panel, unit, rbk))
+    return;
+  multiply_tile<D, 1, 1, PAIR>(a, unit, rbk);
 }
 template <int D, bool PAIR>
 __global__ void __launch_bounds__(kSlices *kWave) gemm_w8_i8_wide_kernel(BH_I8_LEADING) {
   BH_I8_TAKE
-  multiply_tile<D, wide_blocks(D), 2, PAIR>(a);
+  int unit, rbk;
+  if (!place_tile(a.ncols * a.slices, a.row_tiles, a.panel, unit, rbk))
+    return;
+  multiply_tile<D, wide_blocks(D), 2, PAIR>(a, unit, rbk);
 }
 template <int D, int RB, int GP, bool PAIR>
 __global__ void __launch_bounds__(kSlices *kWave, tall_shares(D, GP) ? 2 : 1)
 gemm_w8_i8_tall_kernel(BH_I8_LEADING) {
   BH_I8_TAKE
+  int unit, rbk;
+  if (!place_tile(a.ncols * a.slices, a.row_tiles, a.panel, unit, rbk))
+    return;
   if constexpr (tall_shares(D, GP))
-    multiply_block<D, RB, GP, PAIR>(a);
+    multiply_block<D, RB, GP, PAIR>(a, unit, rbk);
   else
-    multiply_tile<D, RB, GP, PAIR>(a);
+    multiply_tile<D, RB, GP, PAIR>(a, unit, rbk);
+}
+
+// Row tiles of 64 x 256 as far as they make whole rounds of two to a compute unit, the rows behind
+// them in tiles of 32 x 128, which start as the last round ends: what a few large tiles of one more
+// round would keep a part of the chip on for two thirds of a round, small ones spread over all of it.
+// gate | up of three planes, 1536 -> 2 x 8960: 512 rows (560 large tiles for 512 places) 47.3 us, so 44.0;
+// prompts of 449, 512, 960 and 1408 tokens 3.6, 1.5, 2.3 and 1.2 % shorter.  (Of two planes, whose tiles
+// have more shapes, no prompt was shorter.)
+__global__ void __launch_bounds__(kSlices *kWave, 2)
+gemm_w8_i8_tailed_kernel(BH_I8_LEADING, int tail_from, int tail_cols) {
+  BH_I8_TAKE
+  int unit, rbk;
+  if ((int)blockIdx.x < tail_from) {
+    if (place_tile(a.ncols, a.row_tiles, a.panel, unit, rbk))
+      multiply_block<3, 2, 2, true>(a, unit, rbk);
+    return;
+  }
+  const int id = blockIdx.x - tail_from, ids = (tail_cols + 7) & ~7; // a column's tiles on one XCD
+  rbk = id / ids;
+  unit = id - rbk * ids;
+  if (unit >= tail_cols)
+    return;
+  const int row0 = a.row_tiles * 64;
+  a.ncols = tail_cols;
+  multiply_tile<3, 1, 1, true>(a, unit, rbk, row0);
 }
 
 // ---- few f32 rows as they come -------------------------------------------------------
@@ -1311,6 +1339,7 @@ BH_VARIANT_FAMILY(WideFamily, "gemm_w8_i8_wide_kernel");
 BH_VARIANT_FAMILY(NarrowFamily, "gemm_w8_i8_kernel");
 BH_TILE_FAMILY(NarrowPairFamily, "gemm_w8_i8_kernel pair");
 BH_TILE_FAMILY(TallFamily, "gemm_w8_i8_tall_kernel");
+BH_TILE_FAMILY(TailedFamily, "gemm_w8_i8_tailed_kernel");
 
 template <class Kernel>
 int launch_tiles(Kernel kernel, const GemmI8Args &a, unsigned blocks, hipStream_t stream) {
@@ -1334,6 +1363,18 @@ int launch_narrow(const GemmI8Args &a, unsigned blocks, hipStream_t stream) {
   else
     BH_NOTE_VARIANT(NarrowFamily, D);
   return launch_tiles(gemm_w8_i8_kernel<D, PAIR>, a, blocks, stream);
+}
+
+// `blocks` large tiles, as place_tile has them, and the tail
+int launch_tailed(const GemmI8Args &a, unsigned blocks, hipStream_t stream) {
+  BH_NOTE_VARIANT(TailedFamily, 3);
+  const int cols = (int)ceil_div(a.N, kSlices * 16);
+  const unsigned tail = (unsigned)round_up(cols, 8) * (unsigned)ceil_div(a.M - 64 * a.row_tiles, 32);
+  hipLaunchKernelGGL(gemm_w8_i8_tailed_kernel, dim3(blocks + tail), dim3(kSlices * kWave), 0, stream, a.planes,
+                     a.W, a.Mp, a.Kp, a.groups, a.chunks, a.ncols, a.slices, a.chunks_per_slice, a.row_tiles,
+                     a.panel, a, (int)blocks, cols);
+  BH_CHECK_HIP(hipGetLastError());
+  return BUDDY_HIP_OK;
 }
 
 template <int D, int RB, int GP, bool PAIR>
@@ -1464,7 +1505,7 @@ namespace {
 // off the best on average.
 // Microseconds of a product with three planes in a prompt (in brackets with tiles of 64 x 256 that
 // fill a compute unit alone, which then were the pick for down at 512 rows only):
-//   gate | up, 1536 -> 2 x 8960: 27 rows 12.4, 512: 48.8 [52.4], 1931: 146 [164]
+//   gate | up, 1536 -> 2 x 8960: 27 rows 12.4, 512: 47.3 [52.4] (44.0 with a tail), 1931: 146 [164]
 //   down, 8960 -> 1536: 27 rows 5.7, 512: 24.7 [24.9], 1931: 71.5 [78.5]
 //   q|k|v, 1536 -> 2048: 512 rows 11.6
 //   one plane, 1536 -> 8960: 512 rows 19.1
@@ -1493,6 +1534,7 @@ constexpr TileShape kTiles3[] = {{1, 1, true, 0.216, 3.2, 0.455, 4.5},
 
 struct TilePlan {
   int rb = 0, gp = 0, slices = 1;
+  int tail = 0; // row tiles in front of a tail of small ones (gemm_w8_i8_tailed_kernel)
   double us = 0;
 };
 template <int D, bool PAIR>
@@ -1525,7 +1567,7 @@ TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, bool may_split, dou
       else
         us += norm_us;
       if (!best.gp || us < best.us - 1e-9)
-        best = {t.rb, t.gp, s, us};
+        best = {t.rb, t.gp, s, 0, us};
     }
   };
   if constexpr (D == 1)
@@ -1537,6 +1579,22 @@ TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, bool may_split, dou
   else
     for (const TileShape &t : kTiles3)
       consider(t);
+  if constexpr (D == 3 && PAIR) {
+    // Whole rounds of 64 x 256, then small tiles: alone on their compute units and 4.5 us beside (each
+    // begins with two trips to memory), more from 30 on an XCD on.  512 rows of gate | up have 32 and
+    // 44.0 us (47.3), 1931 rows 50 and 2 us more than with large tiles only.
+    const TileShape &t = kTiles3[2], &small = kTiles3[0];
+    const int64_t ncols = ceil_div(channels, kSlices * 16 * t.gp), rows = ceil_div(M, 32 * t.rb);
+    const int64_t rounds = ncols * rows / 512, large = rounds ? std::min(512 * rounds / ncols, rows - 1) : 0;
+    if (large > 0) {
+      const int64_t tail = ceil_div(channels, kSlices * 16) * ceil_div(M - 32 * t.rb * large, 32);
+      const double beside = (double)(tail - (512 * rounds - ncols * large)) / 8;
+      const double us = (double)rounds * (t.both * chunks + t.both0) + small.alone * chunks + small.alone0 + 4.5 +
+                        0.35 * std::max(0.0, beside - 30) + norm_us;
+      if (beside <= 64 && us < best.us)
+        best = {t.rb, t.gp, 1, (int)large, us};
+    }
+  }
   return best;
 }
 
@@ -1560,11 +1618,15 @@ int launch_plan(const TilePlan &plan, GemmI8Args &a, hipStream_t stream) {
       return BUDDY_HIP_OK;
     a.partial = reinterpret_cast<float *>(ws);
   }
+  if (plan.tail)
+    a.row_tiles = plan.tail;
   const int64_t units = (int64_t)a.ncols * a.slices;
   a.panel = panel_for(units, a.row_tiles);
   const int64_t tiles = (a.panel ? units : round_up(units, 8)) * a.row_tiles;
   BH_REQUIRE(tiles < (1u << 31), "gemm_w8: %lld tiles", (long long)tiles);
   const unsigned blocks = (unsigned)tiles;
+  if (plan.tail)
+    return launch_tailed(a, blocks, stream);
   if (plan.gp == 1)
     return launch_narrow<D, PAIR>(a, blocks, stream);
   if (plan.gp == 2 && plan.rb == wide_blocks(D))

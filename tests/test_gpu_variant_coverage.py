@@ -422,3 +422,30 @@ def test_prefill_attention_and_no_unlisted_family(bh, oracle):
     ((2, 3, 2, 0), 321, 128, 8873), ((2, 3, 2, 0), 641, 256, 12281), ((2, 3, 2, 0), 641, 400, 12281)])
 def test_tall_int8_tiles_of_few_chunks(bh, oracle, variant, M, K, N):
     test_tall_int8_tiles(bh, oracle, variant, M, K, N)
+
+
+# Rounds of large tiles and a tail of small ones: a tail of one row, of a block and a row, of two
+# blocks, behind one and two rounds; the last columns' tiles, of both sizes, not full; K not whole
+@pytest.mark.parametrize("M,K,N", [(449, 1536, 8960), (481, 1500, 8944), (512, 1536, 8976), (960, 1536, 8960),
+                                   (200, 1530, 33008)])
+def test_int8_tiles_with_a_tail(bh, M, K, N):
+    bh.buddy_hip_variant_reset()
+    x = torch.randn((M, K), generator=torch.Generator(device="cuda").manual_seed(M), device="cuda")
+    rounded, step = fixed_point_round(x.cpu().numpy(), digits=3)
+    rounded = torch.from_numpy(rounded.astype(np.float64)).cuda()
+    most = rounded.abs() + torch.from_numpy(step).cuda() * 2.0**16
+    packs, want, size = [], [], []
+    for i in range(2):
+        q, s = synthetic.quantized_linear(K, N, M + K + N + i)
+        packs.append((ops.pack_w8(q), s))
+        want.append(rounded @ q.double() * s.double())
+        size.append(24 * 2.0**-24 * (most @ q.double().abs() * s.double()))
+    got = ops.gemm_w8a32(x, torch.cat([p for p, _ in packs]), torch.cat([s for _, s in packs]),
+                         K, N, digits=3, silu_pair=True).double()
+    silu = want[0] / (1 + torch.exp(-want[0]))
+    exact = silu * want[1]
+    # as in test_tall_int8_tiles
+    bound = 1.1 * size[0] * (want[1].abs() + size[1]) + silu.abs() * size[1] + \
+        exact.abs() * (1 + want[0].abs()) * 2.0**-21
+    assert bool(((got - exact).abs() <= bound).all())
+    assert tiles_run(bh)["gemm_w8_i8_tailed_kernel<3>"] == 1
