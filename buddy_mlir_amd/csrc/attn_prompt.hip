@@ -483,20 +483,21 @@ PromptShare share_out(int q_len, int q_offset, int heads, int kv_heads) {
 }
 } // namespace
 
-// An estimate of both ways in microseconds, fitted to 1568 prompts of 12 layers: eight shapes of 1 to
-// 64 heads, 4 to 640 tokens behind 0 to 1200, in three modes.  `converts`: behind the other way the
+// An estimate of both ways in microseconds, fitted to 1748 prompts of 12 layers: eight shapes of 1 to
+// 64 heads, 4 to 1000 tokens behind 0 to 1200, in three modes.  `converts`: behind the other way the
 // rows take a launch of their own to become the output product's input, which the fold is here
 // (not up to 16 tokens as f32, nor up to 128 as digits, which that product makes itself).
 // The choice is up to 13 % of a layer slower than the better way and 0.25 % on average.  us a
 // layer with its products, the other way and this one, where the line lies:
 //   12 heads, 2 KV heads, digits: 4 behind 400 40.9, 42.3, behind 700 47.0, 43.9, 32 behind 256
 //     53.3, 54.9, behind 700 60.7, 58.0, 256 behind 400 70.1, 70.1, 500 alone 74.9, 75.6, behind
-//     128 79.5, 86.7, behind 400 93.0, 90.3
+//     128 79.5, 86.7, behind 400 93.0, 90.3, 730 alone 99.8, 102.0, 920 115.9, 113.7
 //   64 and 8, digits: 32 behind 256 63.6, 77.2, 128 behind 700 107.7, 107.0, 256 behind 128 111,
 //     115, behind 256 123, 118, 500 alone 165, 160
 //   one head, every bit: 64 behind 64 54.7, 56.5, behind 128 57.4, 56.8, 256 behind 64 65.6, 64.6
-// More than 32 tokens behind 400 and more go this way in doubt, up to 6 us: it asks for each key
-// once for all heads of a KV head, and what is not finite stays with the rows that see it.
+// More than 32 tokens behind 400 and more go this way in doubt, up to 6 us, and more than 640 up to
+// 2.5: it asks for each key once for all heads of a KV head, and what is not finite stays with the
+// rows that see it.
 bool attn_prompt_pays(int q_len, int q_offset, int heads, int kv_heads, bool converts) {
   const double kilo_rows = 1e-4 * q_len * heads; // tens of thousands of (token, head)
   // attn_prefill.hip: blocks of 16 queries, one to a workgroup of eight wavefronts, then two, while
@@ -508,9 +509,9 @@ bool attn_prompt_pays(int q_len, int q_offset, int heads, int kv_heads, bool con
   else if (heads * ceil_div(nqb, 2) <= 256)
     steps = 1.5 + 2.4 * (2.0 * q_offset + q_len + 16) / 128;
   else
-    steps = 3.3 + 2.7 * (1.0 * heads * q_len * q_len / (16 * 32 * 256) +
+    steps = 0.3 + 2.7 * (1.0 * heads * q_len * q_len / (16 * 32 * 256) +
                          (double)ceil_div(heads * nqb, 256) * q_offset / 16) / 8;
-  const double other = 4.7 + (converts ? 3.9 : 0.0) + steps + 3.3 * kilo_rows;
+  const double other = 4.7 + (converts ? 3.9 : 0.0) + steps + 2.5 * kilo_rows;
   // here: tiles of the longest share, wavefronts that have rows, blocks that begin and end, and
   // the fold's trips to memory and its bytes
   const PromptShare s = share_out(q_len, q_offset, heads, kv_heads);
@@ -523,7 +524,7 @@ bool attn_prompt_pays(int q_len, int q_offset, int heads, int kv_heads, bool con
                       0.85 * s.nblk * kv_heads / s.workgroups +
                       0.9 * (double)ceil_div(heads, 16) * trips +
                       0.46 * kilo_rows * std::min(parts, 20.0);
-  return here < other + (q_len > 32 && q_offset >= 400 ? 6.0 : 0.0);
+  return here < other + (q_len > 32 && q_offset >= 400 ? 6.0 : q_len > 640 ? 2.5 : 0.0);
 }
 
 // Two slots for every workgroup there can be: 67 MB where all compute units have tiles.

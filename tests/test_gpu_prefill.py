@@ -504,7 +504,7 @@ def test_which_prompt_attention(bh, heads, kv_heads, before, n, precision, split
 # the same prompt: digits that the output product makes itself, rows that take a launch of their own
 @pytest.mark.parametrize("heads,kv_heads,before,n,precision,split", [
     (12, 2, 310, 27, "digits", 0), (12, 2, 310, 27, "exact", 1), (12, 2, 256, 16, "digits", 0),
-    (12, 2, 700, 16, "digits", 1), (64, 8, 390, 128, "digits", 0), (64, 8, 300, 129, "digits", 1)])
+    (12, 2, 700, 16, "digits", 1), (64, 8, 390, 128, "digits", 0), (64, 8, 390, 256, "digits", 1)])
 def test_which_prompt_attention_by_conversion(bh, heads, kv_heads, before, n, precision, split):
     test_which_prompt_attention(bh, heads, kv_heads, before, n, precision, split)
 
