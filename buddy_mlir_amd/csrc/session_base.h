@@ -96,7 +96,7 @@ struct Session {
   int step_and_hand_out(int token, int pos, float *logits_out, int *next_token);
   int *hand_done() const;
   int enqueue_whole_step(bool hands);
-  int enqueue_hand_out(int n);
+  int enqueue_hand_out(int n, bool says); // says: in the words behind the logits
   int wait_hand_out(int n);
 };
 
