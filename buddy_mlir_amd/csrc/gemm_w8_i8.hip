@@ -754,6 +754,9 @@ template <int N> __device__ __forceinline__ void landed() {
 
 // the tiles of gemm_w8_i8_tall_kernel that go this way
 constexpr bool tall_shares(int D, int GP) { return D >= 2 && GP == 2; }
+// A lane reaches its group of a pair's second matrix by 32 bits from a group of the first: matrices of
+// fewer than 2^22 tiles (1 KiB each).  Larger ones go by multiply_tile, whose lanes have 64-bit addresses.
+inline bool pair_in_reach(int64_t channels, int64_t chunks) { return ceil_div(channels, kTileN) * chunks < (1 << 22); }
 
 template <int D, int RB, int GP, bool PAIR>
 __device__ __forceinline__ void multiply_block(const GemmI8Args &a, int unit, int rbk) {
@@ -1541,7 +1544,10 @@ template <int D, bool PAIR>
 TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, bool may_split, double norm_us,
                     double split_norm_us, int64_t sum_wgs) {
   TilePlan best;
+  const bool in_reach = !PAIR || pair_in_reach(channels, chunks);
   auto consider = [&](const TileShape &t) {
+    if (!in_reach && tall_shares(D, t.gp) && t.rb != wide_blocks(D))
+      return;
     const int64_t ncols = ceil_div(channels, kSlices * t.gp * (PAIR ? 16 : 32));
     const int64_t rows = ceil_div(M, 32 * t.rb);
     for (int s = 1; s <= (may_split ? 16 : 1); ++s) {
@@ -1586,7 +1592,7 @@ TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, bool may_split, dou
     const TileShape &t = kTiles3[2], &small = kTiles3[0];
     const int64_t ncols = ceil_div(channels, kSlices * 16 * t.gp), rows = ceil_div(M, 32 * t.rb);
     const int64_t rounds = ncols * rows / 512, large = rounds ? std::min(512 * rounds / ncols, rows - 1) : 0;
-    if (large > 0) {
+    if (large > 0 && in_reach) {
       const int64_t tail = ceil_div(channels, kSlices * 16) * ceil_div(M - 32 * t.rb * large, 32);
       const double beside = (double)(tail - (512 * rounds - ncols * large)) / 8;
       const double us = (double)rounds * (t.both * chunks + t.both0) + small.alone * chunks + small.alone0 + 4.5 +
@@ -1910,3 +1916,18 @@ int launch_gemm_w8a8_plane(const void *plane, const int8_t *W, const float *wsca
 }
 
 } // namespace bh
+
+extern "C" int buddy_hip_gemm_w8_digits_plan(int64_t M, int64_t K, int64_t N, unsigned flags,
+                                             buddy_hip_digits_plan *out) try {
+  BH_REQUIRE(out, "gemm_w8_digits_plan: null result");
+  BH_REQUIRE(M > 0 && N > 0 && K > 0 && M < (1 << 24) && N < (1 << 24) && K <= (1 << 17),
+             "gemm_w8_digits_plan: bad shape M=%lld K=%lld N=%lld", (long long)M, (long long)K, (long long)N);
+  const bool pair = flags & BUDDY_HIP_GEMM_SILU_PAIR, two = flags & BUDDY_HIP_GEMM_TWO_DIGITS;
+  const int chunks = (int)bh::ceil_div(K, bh::kTileK);
+  const bh::TilePlan p = pair ? two ? bh::plan_tiles<2, true>(M, N, chunks, false, 0, 0, 0)
+                                    : bh::plan_tiles<3, true>(M, N, chunks, false, 0, 0, 0)
+                              : two ? bh::plan_tiles<2, false>(M, N, chunks, true, 0, 0, 0)
+                                    : bh::plan_tiles<3, false>(M, N, chunks, true, 0, 0, 0);
+  *out = {p.rb, p.gp, p.slices, p.tail};
+  return BUDDY_HIP_OK;
+} BH_CATCH_INT("buddy_hip_gemm_w8_digits_plan")

@@ -292,6 +292,16 @@ enum {
 int buddy_hip_gemm_w8a32(const float *A, const int8_t *packed, const float *scale,
                          float *C, int64_t M, int64_t K, int64_t N,
                          unsigned flags, buddy_hip_stream stream);
+/* How that call cuts a product over digit planes (host arithmetic, no device needed);
+ * flags: BUDDY_HIP_GEMM_SILU_PAIR, BUDDY_HIP_GEMM_TWO_DIGITS. */
+typedef struct {
+  int32_t row_blocks;    /* blocks of 32 rows of a workgroup's tile */
+  int32_t channel_tiles; /* tiles of 32 channels (16 of either matrix of a pair) of a wavefront, four of those a workgroup */
+  int32_t slices;        /* of K */
+  int32_t tail_from;     /* row tiles ahead of a tail of 32 x 128 tiles; 0: no tail */
+} buddy_hip_digits_plan;
+int buddy_hip_gemm_w8_digits_plan(int64_t M, int64_t K, int64_t N, unsigned flags,
+                                  buddy_hip_digits_plan *out);
 
 /* ---- element-wise pieces of a decoder layer ------------------------------
  * Stand-alone forms of what the decode step runs fused; constants and op order

@@ -210,6 +210,30 @@ def test_prefill_gemm_silu_pair(oracle, M, K, N):
     silu_pair_case(oracle, M, K, N)
 
 
+@pytest.mark.parametrize("digits", [3, 2])
+def test_prefill_gemm_silu_pair_of_4_gib_matrices(digits):
+    """The second matrix lies 2^32 bytes behind the first: gate's weights are all 1, up's all 2."""
+    M, K, N = 64, 65536, 65536
+    packed = torch.empty(2 * K * N, dtype=torch.int8, device="cuda")
+    packed[:K * N].fill_(1)
+    packed[K * N:].fill_(2)
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn((M, K), generator=g, device="cuda")
+    scale = (0.5 + torch.rand(2 * N, generator=g, device="cuda")) / 256
+    got = ops.gemm_w8a32(x, packed, scale, K, N, digits=digits, silu_pair=True).double()
+    del packed
+    rounded, step = fixed_point_round(x.cpu().numpy(), digits=digits)
+    # both sums: 24 roundings of at most the sum of the digits' magnitudes, as at tile edges
+    size = torch.from_numpy((np.abs(rounded).astype(np.float64) + step * 2.0**16).sum(1)).cuda()[:, None]
+    total = torch.from_numpy(rounded.astype(np.float64).sum(1)).cuda()[:, None]
+    s = scale.double()
+    gate, up, err = total * s[:N], 2 * total * s[N:], 24 * 2.0**-24 * size
+    silu = gate * torch.sigmoid(gate)
+    # SiLU's slope stays below 1.1; ten roundings in it and the product
+    bound = 1.1 * err * s[:N] * up.abs() + silu.abs() * 2 * err * s[N:] + 10 * 2.0**-24 * (gate * up).abs()
+    assert ((got - silu * up).abs() <= bound).all()
+
+
 def test_prefill_gemm_silu_pair_refusals(bh):
     x = torch.zeros((32, 64), device="cuda")
     w = torch.zeros((2 * 64 * 64,), dtype=torch.int8, device="cuda")
