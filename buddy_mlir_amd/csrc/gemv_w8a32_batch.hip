@@ -356,6 +356,8 @@ size_t gemv_batch_sums_bytes(int64_t M, int64_t K) {
 
 int launch_gemv_batch(const GemvArgs &g, bool *done, hipStream_t stream) {
   *done = false;
+  if (g.lda >= 1 << 30) // a row's stride is an int here
+    return BUDDY_HIP_OK;
   const int groups = (int)ceil_div(g.N, kTileN), chunks = (int)ceil_div(g.K, kTileK);
   if (g.epilogue == kEpiSiluMul) {
     // a wavefront's slice fits its registers whole, and the launch is one round of the chip: as many

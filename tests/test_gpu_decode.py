@@ -703,3 +703,26 @@ def test_mlp_block_in_one_trip(bh, oracle, M, H, I, pair, chunks):
     assert np.isnan(got[[0, 3]]).all()
     rest = [m for m in range(M) if m not in (0, 3)]
     np.testing.assert_array_equal(got[rest], plain.cpu().numpy()[rest])
+
+
+@pytest.mark.parametrize("ldx,one_trip", [((1 << 30) - 4, 1), (1 << 30, 0), (1 << 31, 0)])
+def test_mlp_block_rows_far_apart(bh, oracle, ldx, one_trip):
+    """Five rows 4 and 8 GiB apart; the kernel whose rows' stride is an int leaves those of 2^30 on alone."""
+    from tile_report import tiles_run
+    M, H, I = 5, 1024, 256
+    if torch.cuda.mem_get_info()[0] < 4 * ((M - 1) * ldx + H) + (1 << 32):
+        pytest.skip("not enough memory")
+    packs = [t for K, N, seed in ((H, I, 44), (H, I, 45), (I, H, 46))
+             for t in synthetic.quantized_linear(K, N, seed)]
+    rows = torch.randn((M, H), generator=torch.Generator(device="cuda").manual_seed(M), device="cuda")
+    store = torch.empty((M - 1) * ldx + H, device="cuda")
+    x = store.as_strided((M, H), (ldx, 1))
+    x.copy_(rows)
+    bh.buddy_hip_variant_reset()
+    got = ops.mlp_block_w8a32(x, *[ops.pack_w8(t) if t.dtype == torch.int8 else t for t in packs], H, I).cpu().numpy()
+    assert tiles_run(bh)["batch_pair_kernel<1, 2>"] == one_trip
+    del x, store
+    torch.cuda.empty_cache()
+    want = mlp_block_oracle(oracle, rows.cpu().numpy(), *[t.cpu().numpy() for t in packs])
+    for m in range(M):
+        check_close(got[m], want[m])
