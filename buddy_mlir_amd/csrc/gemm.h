@@ -98,9 +98,9 @@ int launch_slices_rope(const SliceSums &sums, const RopeKv &rope, float *C, int6
 // the matmul over digit planes (called by launch_gemm_w8 when digits != 0)
 int launch_gemm_w8_digits(const GemmW8Args &a, const void *planes, hipStream_t stream);
 // the matmul over few f32 rows A (not staged), turned into digits slice by slice of K, whose steps
-// are never coarser than a row's own; done stays false where there are too many rows or no cut of K
-// suits: nothing has been launched then
-constexpr int kDigitRowsMax = 128;
+// are never coarser than a row's own; done stays false where there are too many rows, rows that are not
+// aligned or no cut of K that suits: nothing has been launched then
+bool gemm_w8_takes_rows(int64_t M, int64_t K, int64_t N, int64_t lda); // of rows at an aligned address
 int launch_gemm_w8_digits_rows(const GemmW8Args &a, bool *done, hipStream_t stream);
 
 int launch_gemm_w8(const GemmW8Args &a, hipStream_t stream);

@@ -1794,7 +1794,12 @@ BH_TILE_FAMILY(RowsFamily, "gemm_w8_i8_rows_kernel"); // planes, chunks of a sli
 
 // Chunks of 64 k to a slice: the fewest that leave at most sixteen slices, whose sums have to be
 // added, and at most a workgroup per compute unit, whose loads are one trip; 0: no such cut.
-int rows_chunks(int64_t M, int64_t K, int64_t N) {
+// (8960 -> 1536 has one up to 64 rows, 1536 -> 1536 up to 128.)  Rows are read 16 bytes at a time.
+// Beyond 128 (three planes: 129 rows 2426 -> 2335 us a prompt, 256 the same; two: 180 rows 1 % longer) a
+// launch for the digits is a small part.
+int rows_chunks(int64_t M, int64_t K, int64_t N, int64_t lda) {
+  if (M > 128 || ((K | lda) & 3) != 0 || lda >= (1 << 30))
+    return 0;
   const int64_t chunks = ceil_div(K, kTileK), tiles = ceil_div(N, kSlices * 32) * ceil_div(M, 32);
   for (int c : {2, 3, 5, 9, 14})
     if (ceil_div(chunks, c) <= 16 && ceil_div(chunks, c) * tiles <= 256)
@@ -1825,15 +1830,14 @@ template <int D> int launch_rows_of(int c, const GemmW8Args &in, const GemmI8Arg
 }
 } // namespace
 
+bool gemm_w8_takes_rows(int64_t M, int64_t K, int64_t N, int64_t lda) { return rows_chunks(M, K, N, lda) != 0; }
+
 int launch_gemm_w8_digits_rows(const GemmW8Args &in, bool *done, hipStream_t stream) {
   *done = false;
   BH_REQUIRE(in.A && in.W && in.scale && in.C && in.M > 0 && in.K > 0 && in.N > 0 && in.lda >= in.K && in.ldc >= in.N &&
                  (in.digits == 2 || in.digits == 3) && !in.staged && !in.silu_pair && !in.then_rope,
              "gemm_w8: rows as they come");
-  // rows are read 16 bytes at a time; beyond kDigitRowsMax (three planes: 129 rows 2426 -> 2335 us a
-  // prompt, 256 the same; two: 180 rows 1 % longer) a launch for the digits is a small part
-  const bool aligned = ((in.K | in.lda) & 3) == 0 && (reinterpret_cast<uintptr_t>(in.A) & 15) == 0;
-  const int c = in.M <= kDigitRowsMax && aligned && in.lda < (1 << 30) ? rows_chunks(in.M, in.K, in.N) : 0;
+  const int c = (reinterpret_cast<uintptr_t>(in.A) & 15) == 0 ? rows_chunks(in.M, in.K, in.N, in.lda) : 0;
   if (!c)
     return BUDDY_HIP_OK;
   GemmI8Args a{};

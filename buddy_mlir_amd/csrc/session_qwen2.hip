@@ -461,7 +461,7 @@ struct Qwen2Session : Session {
     // bfloat16 913 and 1516, 971 and 1504, 1166 and 1503, 1228 and 1524, 1278 and 1539.
     const bool few = n <= kFewTokens && (gemm_digits || (gemm_terms == 1 && QKV >= kFewChannels));
     // attention's rows go to their product as they are (few) or it makes their digits (gemm_digit_rows)
-    const bool converts = !few && !(gemm_digits && n <= kDigitRowsMax);
+    const bool converts = !few && !(gemm_digits && gemm_w8_takes_rows(n, layers[0].o.K, S.hidden, layers[0].o.K));
     const bool folded = attn_prompt_pays(n, start_pos, S.heads, S.kv_heads, converts);
     if (folded && !pf_attn_ws) // for as many rows as the other buffers have, behind any context
       BH_CHECK_HIP(hipMalloc(&pf_attn_ws, attn_prompt_workspace_bytes(pf_rows, S.max_len, S.heads, S.kv_heads)));

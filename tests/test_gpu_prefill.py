@@ -506,8 +506,8 @@ def test_prompt_attention_equals_token_by_token(heads, kv_heads, before, n):
     (8, 1, 129, 32, "exact", 0), (8, 1, 600, 32, "exact", 1), (12, 2, 128, 300, "digits", 0),
     (12, 2, 400, 300, "digits", 1), (12, 2, 0, 801, "digits", 0), (12, 2, 0, 901, "digits", 1),
     (64, 8, 128, 27, "digits", 0), (64, 8, 1200, 33, "digits", 1), (1, 1, 128, 96, "exact", 1)])
-def test_which_prompt_attention(bh, heads, kv_heads, before, n, precision, split):
-    shape = Shape(layers=2, hidden=256, heads=heads, kv_heads=kv_heads, head_dim=128, inter=256,
+def test_which_prompt_attention(bh, heads, kv_heads, before, n, precision, split, hidden=256):
+    shape = Shape(layers=2, hidden=hidden, heads=heads, kv_heads=kv_heads, head_dim=128, inter=256,
                   vocab=320, max_len=before + n + 8)
     toks = synthetic.first_tokens(shape, n, seed=before + n).astype(np.int32)
     sess, _ = synthetic.build_session(shape, context=before, ln_jitter=0.1)
@@ -531,6 +531,13 @@ def test_which_prompt_attention(bh, heads, kv_heads, before, n, precision, split
     (12, 2, 700, 16, "digits", 1), (64, 8, 390, 128, "digits", 0), (64, 8, 390, 256, "digits", 1)])
 def test_which_prompt_attention_by_conversion(bh, heads, kv_heads, before, n, precision, split):
     test_which_prompt_attention(bh, heads, kv_heads, before, n, precision, split)
+
+
+# output products of more channels than the chip has compute units for rows of them as they come
+@pytest.mark.parametrize("hidden,made", [(4096, 2), (4224, 0)])
+def test_which_prompt_attention_by_product(bh, hidden, made):
+    test_which_prompt_attention(bh, 8, 1, 390, 100, "digits", 0 if made else 1, hidden=hidden)
+    assert sum(v for k, v in tiles_run(bh).items() if k.startswith("gemm_w8_i8_rows_kernel<3, 9>")) == made
 
 
 # q | k | v with the rotation and the cache rows behind it: K in more slices than are asked for at
