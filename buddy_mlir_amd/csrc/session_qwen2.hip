@@ -438,7 +438,30 @@ struct Qwen2Session : Session {
                                       staged, stream);
   }
 
-  static constexpr int kFewTokens = 16;
+  // Whether n tokens go through the products of a decode step, which read f32 rows, norm them, turn
+  // them into digits of 2^-23 of their largest and add to the residual themselves: five to seven
+  // launches a layer for the prompt's eight, whose tiles of 32 rows are mostly padding here.  (Not where
+  // every bit of the rows was asked for.)  Qwen2-1.5B's shape, us a prompt, those against the prompt's own:
+  // 1 token 878 and 1504, 2 973 and 1491, 5 1165 and 1527, 9 1236 and 1545, 16 1272 and 1546; cast to
+  // bfloat16 913 and 1516, 971 and 1504, 1166 and 1503, 1228 and 1524, 1278 and 1539.
+  // Rows cast to bfloat16 are a third of the digits' products, which larger layers show (us a layer, those
+  // against the prompt's own): 2048 x 11008, 77 M weights, 16 tokens 58 and 64; 2560 x 9728, 90 M, 12
+  // tokens 69 and 69, 16 73 and 68; 3072 x 12288, 138 M, 8 tokens 73 and 79, 12 80 and 78, 16 84 and 79;
+  // 4096 x 14336, 218 M, 8 87 and 93, 16 100 and 94; 5120 x 13824, 275 M, 2 tokens 90 and 112, 4, on the
+  // kernel for up to four rows, 115 and 107, 8 106 and 107, 16 118 and 109; two digit planes: 3072 x 12288
+  // 12 81 and 84, 16 87 and 84, 5120 x 13824 12 114 and 116, 16 119 and 116.  Rows that are not read 16 bytes
+  // at a time have no matrix cores from five on (1534 x 8960, 4 tokens 49 and 56, 8 57 and 57, 16 82 and
+  // 58; digits 8 56 and 65, 16 79 and 66).
+  bool few_tokens(int n) const {
+    const auto &S = shape;
+    const int64_t qn = (int64_t)S.heads * S.head_dim, qkv = qn + 2 * (int64_t)S.kv_heads * S.head_dim;
+    const double weights = 1e-6 * S.hidden * (double)(qkv + qn + 3 * (int64_t)S.inter);
+    if (gemm_digits)
+      return n <= (S.hidden % 4 ? 8 : gemm_digits == 2 && weights > 128 ? 12 : 16);
+    if (gemm_terms != 1 || qkv < kFewChannels || (weights > 250 && (n == 3 || n == 4)))
+      return false;
+    return n <= (S.hidden % 4 ? 4 : weights <= 80 ? 16 : weights <= 128 ? 12 : 8);
+  }
   // channels from which on q | k | v of few tokens go that way: fewer leave most of the chip without
   // a workgroup, where the prompt's product cuts K over several
   static constexpr int kFewChannels = 128 * 16;
@@ -453,13 +476,7 @@ struct Qwen2Session : Session {
                        pf_tokens, (int64_t)S.hidden, (int64_t)S.vocab, pf_x);
     BH_CHECK_HIP(hipGetLastError());
     int rc;
-    // Up to 16 tokens go through the products of a decode step, which read f32 rows, norm them, turn
-    // them into digits of 2^-23 of their largest and add to the residual themselves: five to seven
-    // launches a layer for the prompt's eight, whose tiles of 32 rows are mostly padding here.  (Not where
-    // every bit of the rows was asked for.)  Qwen2-1.5B's shape, us a prompt, those against the prompt's own:
-    // 1 token 878 and 1504, 2 973 and 1491, 5 1165 and 1527, 9 1236 and 1545, 16 1272 and 1546; cast to
-    // bfloat16 913 and 1516, 971 and 1504, 1166 and 1503, 1228 and 1524, 1278 and 1539.
-    const bool few = n <= kFewTokens && (gemm_digits || (gemm_terms == 1 && QKV >= kFewChannels));
+    const bool few = few_tokens(n);
     // attention's rows go to their product as they are (few) or it makes their digits (gemm_digit_rows)
     const bool converts = !few && !(gemm_digits && gemm_w8_takes_rows(n, layers[0].o.K, S.hidden, layers[0].o.K));
     const bool folded = attn_prompt_pays(n, start_pos, S.heads, S.kv_heads, converts);

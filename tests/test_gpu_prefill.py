@@ -923,6 +923,35 @@ def test_prompts_of_few_tokens(bh, hidden, heads, kv_heads, inter, before, n, pr
             assert np.linalg.norm(g - w) < bound * np.linalg.norm(w)
 
 
+# Where that ends: rows cast to bfloat16 in layers of 80, 128 and 250 million weights, and rows that are not
+# read 16 bytes at a time
+@pytest.mark.parametrize("precision,hidden,heads,kv_heads,inter,n,few", [
+    ("bf16", 2048, 16, 2, 11008, 16, True), ("bf16", 2560, 20, 4, 9728, 12, True), ("bf16", 2560, 20, 4, 9728, 13, False),
+    ("bf16", 4096, 32, 8, 11008, 8, True), ("bf16", 4096, 32, 8, 11008, 9, False), ("bf16", 4096, 32, 8, 11008, 4, True),
+    ("bf16", 5120, 40, 8, 13824, 2, True), ("bf16", 5120, 40, 8, 13824, 3, False), ("bf16", 5120, 40, 8, 13824, 4, False),
+    ("bf16", 5120, 40, 8, 13824, 5, True), ("digits", 5120, 40, 8, 13824, 16, True), ("bf16", 1534, 12, 2, 336, 4, True),
+    ("digits2", 4096, 32, 8, 11008, 12, True), ("digits2", 4096, 32, 8, 11008, 13, False),
+    ("bf16", 1534, 12, 2, 336, 5, False), ("digits2", 1534, 12, 2, 336, 8, True), ("digits", 1534, 12, 2, 336, 9, False)])
+def test_which_prompts_have_few_tokens(bh, precision, hidden, heads, kv_heads, inter, n, few):
+    shape = Shape(layers=1, hidden=hidden, heads=heads, kv_heads=kv_heads, head_dim=128, inter=inter, vocab=320,
+                  max_len=n + 8)
+    toks = synthetic.first_tokens(shape, n, seed=n).astype(np.int32)
+    sess, _ = synthetic.build_session(shape, context=0, ln_jitter=0.1)
+    bh.buddy_hip_variant_reset()
+    _, got = sess.prefill(toks, 0, precision=precision)
+    ran = {k for k, v in tiles_run(bh).items() if v and ("pair" in k and "batch" not in k or "rope" in k or "rows_kernel" in k)}
+    assert bool(ran) != few, ran
+    for i, t in enumerate(toks):
+        _, want = sess.decode(int(t), i, want_logits=i + 1 == n)
+    sess.close()
+    if few or precision == "digits":
+        check_close(got, want)
+    else:
+        bound = 2.0**-10 if precision == "digits2" else 10 * 2.0**-9
+        got, want = np.asarray(got, np.float64), np.asarray(want, np.float64)
+        assert np.linalg.norm(got - want) < bound * np.linalg.norm(want)
+
+
 # The last launch of one query block to a workgroup of eight wavefronts, and the first of two
 @pytest.mark.parametrize("H,HKV,Lq,Lk", [(16, 4, 256, 256), (16, 4, 257, 300), (128, 16, 32, 40), (128, 16, 33, 33)])
 def test_prefill_attention_pairs_where_the_chip_is_full(bh, oracle, H, HKV, Lq, Lk):
