@@ -260,3 +260,9 @@ def test_refusals(bh):
                                       (257, 448, 20016)])
 def test_steps_of_the_tile_of_128_rows(bh, M, K, Nout):
     test_wide_tiles_of_bfloat16_rows(bh, (4, 2), M, K, Nout)
+
+
+# The tile of 128 rows goes two to a compute unit: a few more than one to each, and no more than that
+@pytest.mark.parametrize("tile,M,K,Nout", [((2, 1), 777, 2048, 11008), ((4, 2), 640, 2048, 11008)])
+def test_where_the_tile_of_128_rows_fills_the_chip(bh, tile, M, K, Nout):
+    test_wide_tiles_of_bfloat16_rows(bh, tile, M, K, Nout)
