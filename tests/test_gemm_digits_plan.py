@@ -38,6 +38,13 @@ def test_large_tiles_up_to_there(bh):
     assert (p.row_blocks, p.channel_tiles, p.tail_from) == (2, 2, 7)
 
 
+def test_large_tiles_alone_with_k_whole(bh):
+    """o of Qwen2-1.5B, three planes: tiles of 32 x 256 two to a compute unit, not one of 64 x 256 each."""
+    for M in (1100, 1400, 1600, 1800, 1931, 2000):
+        p = plan(bh, M, 1536, 1536)
+        assert (p.row_blocks, p.channel_tiles, p.slices) == (1, 2, 1), M
+
+
 def test_refusals(bh):
     p = Plan()
     for M, K, N in [(0, 64, 16), (17, 0, 16), (17, 64, 0), (17, (1 << 17) + 1, 16), (1 << 24, 64, 16)]:
