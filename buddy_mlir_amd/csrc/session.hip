@@ -63,7 +63,8 @@ bool pageable(const void *p) {
 Session::~Session() {
   if (stream)
     (void)hipStreamSynchronize(stream);
-  drop_graph();
+  for (StepGraphs &kept : graphs)
+    drop_graphs(kept);
   for (void *p : owned)
     (void)hipFree(p);
   if (host_state)
@@ -97,14 +98,14 @@ int Session::init(int vocab_size, int capacity, hipStream_t on_stream) {
   return BUDDY_HIP_OK;
 }
 
-void Session::drop_graph() {
-  for (auto &kv : graphs) {
+void Session::drop_graphs(StepGraphs &kept) {
+  for (auto &kv : kept) {
     if (kv.second.exec)
       (void)hipGraphExecDestroy(kv.second.exec);
     if (kv.second.graph)
       (void)hipGraphDestroy(kv.second.graph);
   }
-  graphs.clear();
+  kept.clear();
 }
 
 // The position and step the device holds must stay inside the cache and the
@@ -136,14 +137,15 @@ int Session::run_step(bool hands) {
   if (!use_graph) {
     rc = enqueue_whole_step(hands);
   } else {
-    const std::pair<std::pair<int, int>, bool> key{step_key(next_pos), hands};
-    auto it = graphs.find(key);
-    if (it == graphs.end()) {
-      if (graphs.size() >= kMaxStepGraphs) {
+    const std::pair<int, int> key = step_key(next_pos);
+    StepGraphs &kept = graphs[hands];
+    auto it = kept.find(key);
+    if (it == kept.end()) {
+      if (kept.size() >= kMaxStepGraphs) {
         BH_CHECK_HIP(hipStreamSynchronize(stream)); // a replay may still be running
-        drop_graph();
+        drop_graphs(kept);
       }
-      it = graphs.emplace(key, StepGraph{}).first;
+      it = kept.emplace(key, StepGraph{}).first;
     }
     StepGraph &g = it->second;
     if (!g.exec) {
@@ -155,7 +157,7 @@ int Session::run_step(bool hands) {
       if (!rc && (e = hipGraphInstantiate(&g.exec, g.graph, nullptr, nullptr, 0)) != hipSuccess)
         rc = fail(BUDDY_HIP_ERR_HIP, "hipGraphInstantiate: %s", hipGetErrorString(e));
       if (rc) {
-        drop_graph(); // a half-built graph is not kept
+        drop_graphs(kept); // a half-built graph is not kept
         return rc;
       }
     }
@@ -173,10 +175,11 @@ int Session::run_step(bool hands) {
 // pointers): whoever may change one of them drops the graph first, and the
 // next step captures a new one.
 int Session::invalidate_graph() {
-  if (!graphs.empty()) {
-    BH_CHECK_HIP(hipStreamSynchronize(stream));
-    drop_graph();
-  }
+  for (StepGraphs &kept : graphs)
+    if (!kept.empty()) {
+      BH_CHECK_HIP(hipStreamSynchronize(stream));
+      drop_graphs(kept);
+    }
   return BUDDY_HIP_OK;
 }
 
@@ -244,8 +247,8 @@ int Session::step_and_hand_out(int token, int pos, float *logits_out, int *next_
   // a step that other calls have captured serves the first of these too: capturing costs some 400 us
   bool apart = !logits_out || !pageable(logits_out);
   if (!apart && use_graph) {
-    const auto it = graphs.find({step_key(pos), false});
-    if (it != graphs.end() && !it->second.handed)
+    const auto it = graphs[0].find(step_key(pos));
+    if (it != graphs[0].end() && !it->second.handed)
       apart = it->second.handed = true;
   }
   int rc;

@@ -67,8 +67,10 @@ struct Session {
     hipGraphExec_t exec = nullptr;
     bool handed = false; // hand_out has followed it
   };
-  // One captured step per key; and one that begins with what the host gives and ends with hand_out.
-  std::map<std::pair<std::pair<int, int>, bool>, StepGraph> graphs;
+  // One captured step per key, and at [1] one that begins with what the host gives and ends with
+  // hand_out; as many of either, so that a caller of both keeps the cuts that a caller of one does.
+  using StepGraphs = std::map<std::pair<int, int>, StepGraph>;
+  StepGraphs graphs[2];
   static constexpr size_t kMaxStepGraphs = 8;
   bool use_graph = true;
   std::vector<void *> owned;
@@ -82,7 +84,7 @@ struct Session {
   }
   // stream (null: one of its own) and the buffers above
   int init(int vocab_size, int capacity, hipStream_t on_stream);
-  void drop_graph();
+  static void drop_graphs(StepGraphs &kept);
   int invalidate_graph();
   int check_steps(int steps, const char *who) const;
   int run_step(bool hands = false);

@@ -726,3 +726,22 @@ def test_mlp_block_rows_far_apart(bh, oracle, ldx, one_trip):
     want = mlp_block_oracle(oracle, rows.cpu().numpy(), *[t.cpu().numpy() for t in packs])
     for m in range(M):
         check_close(got[m], want[m])
+
+
+def test_steps_of_both_kinds_keep_their_graphs(bh):
+    """Greedy steps and steps with their logits at eight cuts of the attention in turn: every step has been
+    captured after the second round (the first logits of a cut may come from the greedy step's graph)."""
+    from test_gpu_variant_coverage import report
+    shape = Shape(layers=1, hidden=256, heads=4, kv_heads=2, head_dim=128, inter=256, vocab=64, max_len=4800)
+    sess, _ = synthetic.build_session(shape, context=4700)
+    cuts = (500, 1152, 1536, 2048, 2304, 3072, 4096, 4608)  # as test_attn_step_plan has them
+    seen = []
+    for turn in range(3):
+        bh.buddy_hip_variant_reset()
+        got = [(sess.decode_greedy(7, p, 2)[0], *sess.decode(7, p)) for p in cuts]
+        seen.append(sum(v for k, v in report(bh).items() if k.startswith("gemv_w8a32_digits_kernel<")))
+        if turn:
+            assert all(a[:2] == b[:2] and (a[2] == b[2]).all() for a, b in zip(got, first))
+        first = got
+    sess.close()
+    assert seen[0] > 0 and seen[1] > 0 and seen[2] == 0, seen
