@@ -125,6 +125,7 @@ def _declare(lib):
         "buddy_hip_session_get_kv_rows": (c_int, [vp, c_int, c_int, vp]),
         "buddy_hip_session_decode_mirror": (c_int, [vp, c_int, c_int, vp, vp, vp]),
         "buddy_hip_session_use_graph": (c_int, [vp, c_int]),
+        "buddy_hip_session_set_look_us": (c_int, [vp, c_int]),
         "buddy_hip_session_decode": (c_int, [vp, c_int, c_int, vp, vp]),
         "buddy_hip_session_decode_greedy": (c_int, [vp, c_int, c_int, c_int, vp]),
         "buddy_hip_session_prefill": (c_int, [vp, vp, c_int, c_int, vp, vp]),

@@ -201,13 +201,18 @@ int Session::enqueue_hand_out(int n, bool says) {
   return BUDDY_HIP_OK;
 }
 
-// Its last kernel says in the pinned buffer that it is there.
-// The words are looked at for up to kLookUs, which a step is shorter than; whoever takes longer, or
-// has failed, is waited for (and reported) by the runtime, whose wait sleeps and takes up to 20 us
-// to come back.
+// Its last kernel says in the pinned buffer that it is there.  The words are looked at for up to
+// look_us; a step that takes longer, or has failed, is waited for (and reported) by the runtime, whose
+// wait sleeps and takes up to 20 us to come back, and so are the steps behind it but every sixteenth,
+// which looks whether steps have become shorter.
 int Session::wait_hand_out(int n) {
-  constexpr int kLookUs = 2000, kYieldUs = 100;
+  constexpr int kYieldUs = 100, kLooksSkipped = 15;
   const int blocks = hand_blocks(n);
+  if (!look_us || looks_skipped > 0) {
+    looks_skipped -= looks_skipped > 0;
+    BH_CHECK_HIP(hipStreamSynchronize(stream));
+    return BUDDY_HIP_OK;
+  }
   const auto t0 = std::chrono::steady_clock::now();
   for (int b = 0; b < blocks;) {
     if (__atomic_load_n(hand_done() + b, __ATOMIC_ACQUIRE)) {
@@ -215,7 +220,8 @@ int Session::wait_hand_out(int n) {
       continue;
     }
     const auto us = std::chrono::duration_cast<std::chrono::microseconds>(std::chrono::steady_clock::now() - t0);
-    if (us.count() > kLookUs) {
+    if (us.count() > look_us) {
+      looks_skipped = kLooksSkipped;
       BH_CHECK_HIP(hipStreamSynchronize(stream));
       return BUDDY_HIP_OK;
     }
@@ -290,6 +296,15 @@ int buddy_hip_session_use_graph(buddy_hip_session *hs, int enable) try {
   s->use_graph = enable != 0;
   return BUDDY_HIP_OK;
 } BH_CATCH_INT("buddy_hip_session_use_graph")
+
+int buddy_hip_session_set_look_us(buddy_hip_session *hs, int us) try {
+  Session *s = bh::as_session(hs);
+  BH_REQUIRE(s, "session_set_look_us: null session");
+  BH_REQUIRE(us >= 0, "session_set_look_us: %d us", us);
+  s->look_us = us;
+  s->looks_skipped = 0;
+  return BUDDY_HIP_OK;
+} BH_CATCH_INT("buddy_hip_session_set_look_us")
 
 int buddy_hip_session_decode_mirror(buddy_hip_session *hs, int token, int pos,
                                     float *logits_out, float *kv_rows_out,

@@ -73,6 +73,7 @@ struct Session {
   StepGraphs graphs[2];
   static constexpr size_t kMaxStepGraphs = 8;
   bool use_graph = true;
+  int look_us = 2000, looks_skipped = 0; // wait_hand_out
   std::vector<void *> owned;
 
   template <typename T> int alloc(T **p, size_t n) {

@@ -84,6 +84,10 @@ class _Session:
     def use_graph(self, enable: bool):
         check(self._lib.buddy_hip_session_use_graph(self._h, int(enable)), "use_graph")
 
+    def set_look_us(self, us: int):
+        """How long `decode` looks for its logits before it sleeps (2000 us; 0: not at all)."""
+        check(self._lib.buddy_hip_session_set_look_us(self._h, us), "set_look_us")
+
     def decode(self, token: int, pos: int, want_logits: bool = True):
         logits = np.empty(self.vocab, np.float32) if want_logits else None
         nxt = c_int(-1)

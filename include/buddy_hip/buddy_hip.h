@@ -456,7 +456,13 @@ int buddy_hip_session_get_kv_rows(buddy_hip_session *s, int row0, int rows, floa
 int buddy_hip_session_use_graph(buddy_hip_session *s, int enable);
 /* One decode step for `token` at cache row `pos` (ModelSession::decode).
  * logits_out (host or device, vocab floats) and next_token may be NULL.
- * next_token is the greedy choice (first maximum).  Synchronous. */
+ * next_token is the greedy choice (first maximum).  Synchronous.
+ * Where the logits go to pageable host memory the calling thread looks for them in pinned
+ * memory, without a pause for 100 us and then yielding, before it sleeps in the runtime: a
+ * core is busy that long.  buddy_hip_session_set_look_us says for how long at most (2000 us
+ * by default, 0: it sleeps at once, which takes some 20 us more of a step); after a step that
+ * took longer only every sixteenth one looks. */
+int buddy_hip_session_set_look_us(buddy_hip_session *s, int us);
 int buddy_hip_session_decode(buddy_hip_session *s, int token, int pos,
                              float *logits_out, int *next_token);
 /* The same, and the cache rows the step wrote are handed back as well:

@@ -745,3 +745,27 @@ def test_steps_of_both_kinds_keep_their_graphs(bh):
         first = got
     sess.close()
     assert seen[0] > 0 and seen[1] > 0 and seen[2] == 0, seen
+
+
+def test_logits_are_waited_for_with_and_without_a_look(bh):
+    """The words of the pinned buffer and the runtime's wait, which a step that takes longer than it may be
+    looked for (1 us) falls back to, hand out the same tokens and logits, step by step."""
+    shape = Shape(layers=1, hidden=256, heads=4, kv_heads=2, head_dim=128, inter=512, vocab=5000, max_len=96)
+    runs = []
+    for us in (2000, 0, 1, None):
+        sess, _ = synthetic.build_session(shape, context=5)
+        if us is None:  # as it was made
+            assert bh.buddy_hip_session_set_look_us(sess._h, -1) != 0
+        else:
+            sess.set_look_us(us)
+        tok, steps = 7, []
+        for pos in range(5, 45):
+            tok, logits = sess.decode(tok, pos)
+            assert tok == int(logits.argmax())
+            steps.append((tok, logits))
+        runs.append(steps)
+        sess.close()
+    for steps in runs[1:]:
+        for (a, x), (b, y) in zip(steps, runs[0]):
+            assert a == b
+            np.testing.assert_array_equal(x, y)
