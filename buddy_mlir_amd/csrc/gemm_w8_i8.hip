@@ -766,6 +766,8 @@ __device__ __forceinline__ void multiply_block(const GemmI8Args &a, int unit, in
   constexpr int kBuf = L * kPlaneBlock;
   constexpr int kDma = 2 * L / kSlices;       // a wavefront's loads of 1 KiB of a chunk's rows
   static_assert(2 * L % kSlices == 0 && (2 * L) % 4 == 0, "every wavefront brings as much; fragment slots repeat");
+  // landed<> counts GP loads of weights in each half of a chunk, behind its loads into LDS
+  static_assert(kDma + GP <= L, "a half of a chunk has room for its loads of weights");
   constexpr int kLds = kRing * kBuf > turned_bytes(kSpan) ? kRing * kBuf : turned_bytes(kSpan);
   constexpr int kScales = kSlices * 32 * GP;
   __shared__ __attribute__((aligned(16))) unsigned char lds[kLds];
