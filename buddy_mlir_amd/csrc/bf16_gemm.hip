@@ -9,6 +9,7 @@
 // rows_gemm_wide_kernel.
 #include "bf16_linear.h"
 #include "bf16_dev.h"
+#include "digits_dev.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -365,17 +366,6 @@ __device__ __forceinline__ f32x16 mfma_bf16_wide(uint4 a, uint4 b, f32x16 c) {
                                                  __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-// 1 KiB from memory past the registers into LDS: a lane's 16 bytes at `from` to `to` + 16 lane.  Not
-// the compiler's load: landed<N> waits until at most N loads are under way that were issued behind
-// the ones asked about.  No load moves across one of these statements, which may write any memory
-// as far as the compiler knows.
-__device__ __forceinline__ void load_1k_to_lds(const void *from, unsigned to) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(to) : "memory", "m0");
-}
-template <int N> __device__ __forceinline__ void landed() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
 // Tiles of 128 bfloat16 rows run two to a compute unit.
 template <typename T, int RT> constexpr bool kBrings = sizeof(T) == 2 && RT == 4;
 
@@ -445,8 +435,8 @@ rows_gemm_wide_kernel(const uint4 *W, int ktiles, int steps, int columns, int ro
     // a time, seven of them ahead: 256 registers a wavefront.  LDS holds rows of 128 bytes whose
     // eight 16-byte pieces are permuted by the row's number (piece p of row r where p ^ (r / 2 % 8)
     // would be), so that the fragments of sixteen rows in a line meet every bank once.
-    // landed<N>: see gemm_w8_i8.hip's tiles of this kind; a step issues GT loads
-    // of weights in each quarter and RT into LDS, one ahead of those of each of its first quarters.  What K has beyond whole steps follows at the end, on its own.
+    // A step issues GT loads of weights in each quarter and RT into LDS, one ahead of those of each of
+    // its four quarters.  What K has beyond whole steps follows at the end, on its own.
     constexpr int kAhead = 7, kSlots = 8;
     const int whole = min(steps, K / kWideK);
     const int f = ((wave & 1) * 4 + (lane >> 4)) & 7;
@@ -582,7 +572,7 @@ rows_gemm_wide_kernel(const uint4 *W, int ktiles, int steps, int columns, int ro
     }
 
     uint4 wr[4][GT * 4], xr[4][kLoads];
-      const int last_run = (K - 1) / kRunElems * kRunElems;
+    const int last_run = (K - 1) / kRunElems * kRunElems;
     const bool ragged = K % kWideK != 0; // the last step reaches past K
     auto fetch_w = [&](int s, uint4 (&w)[GT * 4]) {
       const int t = min(s, steps - 1) * 2;
@@ -645,7 +635,7 @@ rows_gemm_wide_kernel(const uint4 *W, int ktiles, int steps, int columns, int ro
     load_frag(cur, 0, frag[0]);
     auto step = [&](int s, uint4 (&w)[GT * 4], uint4 (&w_new)[GT * 4], uint4 (&x)[kLoads],
                     uint4 (&x_new)[kLoads]) {
-  #pragma unroll
+#pragma unroll
       for (int u = 0; u < 4; ++u) {
         // the next fragments are asked for ahead of the products that cover their way, and
         // stay there: left to itself the scheduler moves them to their use
@@ -903,7 +893,8 @@ int launch_shape(const RowsGemm &a, hipStream_t stream, int *slices) {
       const int64_t per = ceil_div(steps, s);
       if (ceil_div(steps, per) != s)
         continue; // the last slice would be empty
-      const double us = time(workgroups(rt, ch / P) * s, per) + (s - 1) * 8e-6 / 4.8 * (double)rows * a.W.N + (s > 1 ? kSliceUs : 0.0);
+      const double us = time(workgroups(rt, ch / P) * s, per) +
+                        (s - 1) * 8e-6 / 4.8 * (double)rows * a.W.N + (s > 1 ? kSliceUs : 0.0);
       if (us < best.us)
         best = {us, s};
     }

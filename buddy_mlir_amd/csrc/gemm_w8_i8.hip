@@ -32,6 +32,7 @@
 // kTiles3, with the activation fragments shared through LDS.
 #include "attn.h"
 #include "attn_fold.h"
+#include "digits_dev.h"
 #include "gemm.h"
 #include "tile_place.h"
 
@@ -57,30 +58,6 @@ __device__ __forceinline__ float digit_step(float mx, int D) {
   const int ex = (int)((__float_as_uint(mx) >> 23) & 0xffu) - 127; // floor(log2 mx)
   const int e = max(ex + 1 - (8 * D - 2), -126);
   return __uint_as_float((unsigned)(e + 127) << 23);
-}
-
-// Four values as the words of their balanced digits: word j of four bytes, digit j of each.
-// v * inv + 1.5 * 2^23 is rounded to a whole number X, ties to even, in one instruction, and its
-// bits are those of the constant plus X (|X| <= 2^22).  X plus 128 in every digit but the last has the
-// digits' bytes, each with its top bit turned, in place: no carries to take from digit to digit.
-// (Digit by digit with shifts and masks this was 27 instructions a value and is 5.)
-// Of values that are not finite anything may come out, for their step is NaN.
-__device__ __forceinline__ void digits_of(const float (&v)[4], float inv, int D, unsigned (&word)[3]) {
-  const unsigned bias = D == 3 ? 0x8080u : 0x80u;
-  unsigned y[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e)
-    y[e] = __float_as_uint(fmaf(v[e], inv, 12582912.0f)) + (bias - 0x4B400000u);
-  // bytes 0 and 1 of two values each, then of four
-  const unsigned a = __builtin_amdgcn_perm(y[1], y[0], 0x05010400u), b = __builtin_amdgcn_perm(y[3], y[2], 0x05010400u);
-  word[0] = __builtin_amdgcn_perm(b, a, 0x05040100u) ^ 0x80808080u;
-  word[1] = __builtin_amdgcn_perm(b, a, 0x07060302u);
-  word[2] = 0;
-  if (D == 3) {
-    word[1] ^= 0x80808080u;
-    const unsigned c = __builtin_amdgcn_perm(y[1], y[0], 0x0c0c0602u), d = __builtin_amdgcn_perm(y[3], y[2], 0x0c0c0602u);
-    word[2] = __builtin_amdgcn_perm(d, c, 0x05040100u);
-  }
 }
 
 // Row sources: four consecutive values k0..k0+3 of the row (zero past its end).
@@ -667,8 +644,8 @@ __device__ __forceinline__ void multiply_tile(const GemmI8Args &a, int unit, int
       // their use
       load_frag(u + 2 < 2 * L ? cur : next, (u + 2) % (2 * L), frag[(f + u + 2) & 3]);
       // a chunk's loads, weights first: evenly between its products (all at its start: 171
-      // against 167 us for gate | up of 1931 rows, 193 against 180 on 64 x 256 tiles), for one
-      // plane, which has a third of the products, at the start (19.2 against 21)
+      // against 167 us for gate | up of 1931 rows), for one plane, which has a third of the
+      // products, at the start (19.2 against 21)
 #pragma unroll
       for (int i = first_fetch(u); i < first_fetch(u + 1); ++i) {
         if (i < 2 * GP)
@@ -739,18 +716,7 @@ __device__ __forceinline__ void multiply_tile(const GemmI8Args &a, int unit, int
 // are permuted by the row's number: piece p of row r is where p ^ (r / 4 % 4) would be, and the
 // fragment reads of sixteen rows in a line meet every bank once.
 //
-// The loads into LDS are not the compiler's: landed<N> waits until at most N loads are under way
-// that were issued behind the ones asked about.  Every step issues kDma loads into LDS and 2 GP of
-// weights in that order; the asm statements may write any memory as far as the compiler knows, so
-// no load of weights moves across one of them.
-__device__ __forceinline__ void load_1k_to_lds(const void *base, unsigned lane_offset, unsigned to) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_offset), "s"(base),
-               "s"(to)
-               : "memory", "m0");
-}
-template <int N> __device__ __forceinline__ void landed() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
+// Every step issues kDma loads into LDS and 2 GP of weights in that order.
 
 // the tiles of gemm_w8_i8_tall_kernel that go this way
 constexpr bool tall_shares(int D, int GP) { return D >= 2 && GP == 2; }

@@ -14,9 +14,14 @@
 //                       K, whose rows it turns into digits once for all of them; its sums go to a
 //                       workspace and batch_add_kernel adds the slices in order.
 //
+// Which products: the pair where a wavefront's slice fits its registers whole, hidden of 961 to 1536, and
+// up to 16384 channels; the slices from inter = 4033 on for up to 2048 channels.  Others (4096 -> 14336 ->
+// 4096, both products) go one 64 k after the other.
+//
 // What bounds them: the launch, one trip to memory and the weights' way from HBM.  12 rows of
 // 1536 -> 2 x 8960 10.2 us (one 64 k after the other 14.5), 8960 -> 1536 5.0 and 3.7 for the kernel that adds
 // (11.4); both together in a stream 25.8 -> 19.1, at 5 rows 23.5 -> 16.9, at 16 26.7 -> 19.7.
+#include "digits_dev.h"
 #include "gemv_w8a32.h"
 
 namespace bh {
@@ -52,22 +57,17 @@ __device__ __forceinline__ void step_of(unsigned magnitude, float &step, float &
   step = magnitude < 0x7f800000u ? __uint_as_float((unsigned)(e2 + 127) << 23) : __uint_as_float(0x7fc00000u);
   inv = __uint_as_float((unsigned)(127 - e2) << 23);
 }
-// Four values of row `row`, k 4 k4 .. + 3 of a chunk, as digits into the chunk's planes.  (x * inv + 1.5 *
-// 2^23 has the whole number in its mantissa; the constant behind it makes the digits' bytes, the lower
-// two with their top bit turned.)  The 16-byte pieces of a row lie permuted by its number, so that the
-// operand reads of 16 rows meet every bank once.
+// Four values of row `row`, k 4 k4 .. + 3 of a chunk, as digits into the chunk's planes.  The 16-byte
+// pieces of a row lie permuted by its number, so that the operand reads of 16 rows meet every bank once.
 __device__ __forceinline__ int piece_at(int row, int piece) { return row * kTileK + (piece ^ (row >> 2)) * 16; }
 __device__ __forceinline__ void put_digits(const f32x4 &x, float inv, unsigned char *planes, int row, int k4) {
-  unsigned y[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e)
-    y[e] = __float_as_uint(fmaf(x[e], inv, 12582912.0f)) + (0x8080u - 0x4B400000u);
-  const unsigned a = __builtin_amdgcn_perm(y[1], y[0], 0x05010400u), b = __builtin_amdgcn_perm(y[3], y[2], 0x05010400u);
-  const unsigned c = __builtin_amdgcn_perm(y[1], y[0], 0x0c0c0602u), d = __builtin_amdgcn_perm(y[3], y[2], 0x0c0c0602u);
+  const float v[4] = {x[0], x[1], x[2], x[3]};
+  unsigned word[3];
+  digits_of(v, inv, 3, word);
   unsigned *dst = reinterpret_cast<unsigned *>(planes + piece_at(row, k4 >> 2) + (k4 & 3) * 4);
-  dst[0] = __builtin_amdgcn_perm(b, a, 0x05040100u) ^ 0x80808080u;
-  dst[kPlane / 4] = __builtin_amdgcn_perm(b, a, 0x07060302u) ^ 0x80808080u;
-  dst[2 * (kPlane / 4)] = __builtin_amdgcn_perm(d, c, 0x05040100u);
+  dst[0] = word[0];
+  dst[kPlane / 4] = word[1];
+  dst[2 * (kPlane / 4)] = word[2];
 }
 // acc += step * (a tile times the planes): a lane's four channels of row lane % 16
 __device__ __forceinline__ void add_tile(f32x4 &acc, const v4i &w, const v4i (&d)[3], float step) {
@@ -282,7 +282,7 @@ struct AddArgs {
   const float *scale, *bias;
   float *C;
   int64_t ldc;
-  int N, rows, groups, slices, accumulate;
+  int N, accumulate;
 };
 __global__ void __launch_bounds__(64) batch_add_kernel(const float *sums, int slices, int rows, int groups, AddArgs a) {
   const int q = blockIdx.x * 64 + threadIdx.x, m = blockIdx.y, n = q * 4;
@@ -341,8 +341,9 @@ template <int P> int launch_pair_rows(const GemvArgs &g, int groups, int chunks,
 template <int C>
 int launch_slice(const GemvArgs &g, int groups, int chunks, int slices, float *sums, hipStream_t stream) {
   BH_NOTE_VARIANT(SliceFamily, C);
-  hipLaunchKernelGGL((batch_slice_kernel<C>), dim3((unsigned)ceil_div(groups, kWaves), (unsigned)slices), dim3(kThreads), 0,
-                     stream, g.A, reinterpret_cast<const int4 *>(g.W0), (int)g.lda, (int)g.K, g.M, groups, chunks, sums);
+  hipLaunchKernelGGL((batch_slice_kernel<C>), dim3((unsigned)ceil_div(groups, kWaves), (unsigned)slices),
+                     dim3(kThreads), 0, stream, g.A, reinterpret_cast<const int4 *>(g.W0), (int)g.lda, (int)g.K, g.M,
+                     groups, chunks, sums);
   BH_CHECK_HIP(hipGetLastError());
   return BUDDY_HIP_OK;
 }
@@ -351,7 +352,9 @@ int launch_slice(const GemvArgs &g, int groups, int chunks, int slices, float *s
 
 size_t gemv_batch_sums_bytes(int64_t M, int64_t K) {
   // at most a workgroup of 128 channels to a compute unit
-  return M >= 5 && M <= 16 && ceil_div(K, kTileK) >= kSliceChunks ? sizeof(float) * (size_t)M * 256 * kWaves * kTileN : 0;
+  if (M < 5 || M > 16 || ceil_div(K, kTileK) < kSliceChunks)
+    return 0;
+  return sizeof(float) * (size_t)M * 256 * kWaves * kTileN;
 }
 
 int launch_gemv_batch(const GemvArgs &g, bool *done, hipStream_t stream) {

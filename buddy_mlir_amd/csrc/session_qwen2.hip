@@ -542,8 +542,10 @@ struct Qwen2Session : Session {
       const bool ahead = nx && !nx->qkv_f32;
       if (few && L.gate_up_joint) {
         if (folded) {
-          if ((rc = gemm_digits ? launch_attn_fold_to_digits(fold, a.o_stride, S.heads, n, gemm_digits, pf_att_dg, stream)
-                                : launch_attn_fold_to_terms(fold, a.o_stride, S.heads, n, gemm_terms, pf_att_dg, stream)) ||
+          if ((rc = gemm_digits ? launch_attn_fold_to_digits(fold, a.o_stride, S.heads, n, gemm_digits,
+                                                             pf_att_dg, stream)
+                                : launch_attn_fold_to_terms(fold, a.o_stride, S.heads, n, gemm_terms,
+                                                            pf_att_dg, stream)) ||
               (rc = gemm_staged(pf_att_dg, L.o, pf_x, n, true)))
             return rc;
         } else if ((rc = gemv(pf_att, L.o, nullptr, nullptr, pf_x, kEpiAccum, n))) {

@@ -80,7 +80,8 @@ def mlp_block_desc(x, gate, gate_scale, up, up_scale, down, down_scale, y, hidde
 
 def mlp_block_w8a32(x, gate, gate_scale, up, up_scale, down, down_scale, hidden: int,
                     inter: int, y=None, stream=None, **kw):
-    """y (+)= (SiLU(x' . gate) * (x' . up)) . down for 1..16 rows (two launches)."""
+    """y (+)= (SiLU(x' . gate) * (x' . up)) . down for 1..16 rows (two launches, three where down's K
+    is cut into slices)."""
     if y is None:
         y = torch.empty((x.shape[0], hidden), dtype=torch.float32, device=x.device)
     d, ws = mlp_block_desc(x, gate, gate_scale, up, up_scale, down, down_scale, y, hidden,

@@ -209,7 +209,9 @@ int buddy_hip_gemv_w8a32(const float *A, const int8_t *packed,
  * matrices are wave-tile packed ([hidden, inter] twice, [inter, hidden]).  The
  * intermediate rows [M, inter] f32 and, from five rows on, sums of slices of a long
  * `inter` live in `workspace` (buddy_hip_mlp_block_workspace_bytes(M, inter) bytes, 16-byte
- * aligned; 4 M inter rounded up to 256 is enough, without the latter).  No counterpart in the reference, whose decode kernels are m == 1 only. */
+ * aligned).  The slices, a third launch, are for inter >= 4033 and up to 2048 channels of
+ * `hidden`; without them 4 M inter bytes rounded up to 256 are enough.  No counterpart in the
+ * reference, whose decode kernels are m == 1 only. */
 typedef struct buddy_hip_mlp_block_desc {
   const float *x;          /* [M, hidden], row stride ldx */
   int64_t ldx;
@@ -296,7 +298,7 @@ int buddy_hip_gemm_w8a32(const float *A, const int8_t *packed, const float *scal
  * flags: BUDDY_HIP_GEMM_SILU_PAIR, BUDDY_HIP_GEMM_TWO_DIGITS. */
 typedef struct {
   int32_t row_blocks;    /* blocks of 32 rows of a workgroup's tile */
-  int32_t channel_tiles; /* tiles of 32 channels (16 of either matrix of a pair) of a wavefront, four of those a workgroup */
+  int32_t channel_tiles; /* a wavefront's tiles of 32 channels (16 of either matrix of a pair), four wavefronts */
   int32_t slices;        /* of K */
   int32_t tail_from;     /* row tiles ahead of a tail of 32 x 128 tiles; 0: no tail */
 } buddy_hip_digits_plan;
