@@ -154,6 +154,35 @@ def test_w8a8_many_rows_extremes(bh, oracle):
     assert abs(int(wacc[0, 0])) == K * 127 * 128
 
 
+# rows quantised by the workgroups that multiply them against the way of rows that cannot be read
+# 16 bytes at a time: (a tile's edges in rows, channels and k; K in slices; channels one by one)
+@pytest.mark.parametrize("M,K,N", [(2, 1536, 64), (5, 4, 7), (31, 68, 130), (32, 1536, 8960),
+                                   (33, 1536, 33), (64, 1540, 257), (256, 1000, 1111), (3, 3076, 70),
+                                   (16, 8960, 1536), (96, 8960, 1536), (17, 131072, 40)])
+@pytest.mark.parametrize("special", [False, True])
+def test_w8a8_rows_equal_the_general_path(bh, M, K, N, special):
+    q, s = synthetic.quantized_linear(K, N, M + K)
+    packed = ops.pack_w8(q)
+    x = torch.randn((M, K), generator=torch.Generator(device="cuda").manual_seed(N), device="cuda")
+    if special:  # dropped by the maximum, -128 as a value
+        x[M // 2, K // 3] = float("nan")
+        x[0, K - 1] = -float("inf") if M > 16 else float("nan")
+    shifted = torch.empty(M * K + 1, device="cuda")[1:]
+    shifted.copy_(x.reshape(-1))
+    nb = bh.buddy_hip_w8a8_workspace_bytes(M, K)
+    ws = torch.empty(nb, dtype=torch.uint8, device="cuda")
+    got = []
+    for A in (x, shifted):
+        C = torch.full((M, N), 7.0, device="cuda")
+        acc = torch.full((M, N), 7, dtype=torch.int32, device="cuda")
+        torch.cuda.synchronize()
+        sync_check(bh.buddy_hip_w8a8_matmul(A.data_ptr(), packed.data_ptr(), s.data_ptr(), C.data_ptr(),
+                                            acc.data_ptr(), M, K, N, ws.data_ptr(), nb, None))
+        got.append((C.view(torch.int32), acc))
+    assert torch.equal(got[0][1], got[1][1])
+    assert torch.equal(got[0][0], got[1][0])
+
+
 def test_buddy_matmul_f32_entry_point(bh):
     # tests/Conversion/matmul-blis-vectorization.mlir shape: 9x4 . 4x17 of ones
     A = np.ones((9, 4), np.float32)
