@@ -54,8 +54,8 @@ int launch_attn_fold_to_digits(const PromptFold &fold, int64_t o_stride, int hea
 #if defined(__HIPCC__)
 // The row of query head h at token t once more, in f32 sums, key after key: 32 lanes that
 // hold four values each from d on.  A row comes to this when its sum of weights is NaN:
-// because it is to be, or because the bfloat16 terms of an operand do not exist (an
-// infinity, a value above the largest bfloat16 one) or of a score leave the range that the
+// because it is to be, or because the float16 terms of an operand do not exist (an
+// infinity) or leave none to the row's other values (one far above them), or a score's leave the range that the
 // score itself is in.  An infinite score of -inf has no weight, and an infinite value makes
 // its own channel infinite, as in the other attention kernels.  (1900 keys: some 0.4 ms.)
 __device__ __forceinline__ void f32_row(const PromptFold &f, int t, int h, int d, float (&v)[4]) {

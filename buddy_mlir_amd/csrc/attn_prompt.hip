@@ -1,24 +1,25 @@
 // attn_prompt.hip -- causal GQA attention of a session's prompt tokens over its KV cache.
 //
 // The same operation as attn_prefill.hip (flash_attention_for_cpu_prefill_op,
-// frontend/Python/ops/tosa.py:4326-4810) with a workspace and on the bfloat16 matrix
-// cores: an f32 value is the sum of three bfloat16 values of 8 bits each, rounded to
-// nearest, which is every bit of it; of the nine products of two such sums the six of
-// more than 2^-24 of the largest are taken, each exact, all summed in f32.  Six
-// instructions at sixteen times the rate of the f32 matrix instructions.  The error
-// against 64 bits is that of the f32 kernel (a 28-layer prompt of 1931 tokens: 3.6e-6
-// with either).
+// frontend/Python/ops/tosa.py:4326-4810) with a workspace and on the float16 matrix
+// cores: a row of queries, keys or values is brought to a largest magnitude of 2^14 .. 2^15 by a power of
+// two of its own, and an f32 value is then the sum of two float16 values of 11 bits each, rounded to
+// nearest, 2^-24 off at most (a row's small values 2^-40 of its largest one).  Of the four products
+// of two such sums the three of more than 2^-24 are taken, each exact, all summed in f32.  Three
+// instructions at sixteen times the rate of the f32 matrix instructions (with three bfloat16 terms, which need
+// no scales, six: 6 us a tile for 3).  The error against 64 bits is that of those terms and of the f32
+// kernel (28-layer prompts of 150 to 1931 tokens, eleven of them, 5.9e-6 on average with either).
+// The power of two of a value's row goes into its weight, whose running maximum is over both.
 //
-// What bounds it: per tile of 256 rows x 32 keys a SIMD has 6144 cycles of matrix
-// instructions and 3600 of vector instructions (softmax, conversions), which run one
-// after the other as if they were one kind, and the chip draws so much power meanwhile
-// that it clocks at 1.6 GHz: 6 us a tile.  (The two wavefronts of a SIMD in opposite
-// phases, with the values a tile behind the scores: the same 6 us.)  What a launch costs
-// beside its tiles is some 9 us: the share, queries and their terms, the first tile's way.
-// 12 query heads, 2 KV heads, us per layer, this kernel and the fold behind it against
+// What bounds it: per tile of 256 rows x 32 keys a SIMD has 3072 cycles of matrix
+// instructions and some 3600 of vector instructions (softmax, conversions), which overlap in part:
+// 3 us a tile.  What a launch costs beside its tiles: 6 us until the first one is in terms, as much as two
+// tiles to end a block and begin the next (queries and results go through LDS so that a load or store is of whole
+// lines: as operands lie, it was 10 us), and the partial results' way out of the L2s behind it, 33 MB.
+// 1931 tokens of 12 query heads and 2 KV heads 91 -> 53 us, 150 behind 1900 26.6 -> 22.
+// us per layer, this kernel and the fold behind it against
 // attn_prefill.hip and the conversion behind that (attn_prompt_pays says which is taken):
-//   2000 tokens 104 vs 156, 4096 tokens 332 vs 655, 150 behind 1900 36 vs 64,
-//   27 behind 1900 27 vs 58, 512 tokens 28 vs 25, 256 tokens 21 vs 17
+//   1931 tokens 76 vs 150, 150 behind 1900 30 vs 64
 #include "attn.h"
 #include "attn_fold.h"
 #include "bf16_dev.h"
@@ -32,19 +33,20 @@ namespace {
 constexpr int kThreads = 2 * kPromptRows; // a wavefront has 32 rows
 constexpr int kKeys = 32;                 // of a tile
 constexpr int kTerm = kKeys * kPromptD * 2; // bytes of one term of a tile's keys or values
-constexpr int kHalf = 3 * kTerm;          // keys, then values
+constexpr int kHalf = 2 * kTerm;          // keys, then values
 constexpr int kBuf = 2 * kHalf;
-constexpr int kLds = 2 * kBuf + kThreads / 64 * 4096;
+constexpr int kLds = 2 * kBuf + kThreads / 64 * 2 * 4096;
 constexpr float kSeedM = -1.0e30f;        // tosa.py:4383
-constexpr float kSlack = 8.0f;
+constexpr float kBelow = 8.0f, kMost = 15.0f; // log2 of a row's largest weight as it is set, and at most
 
 struct PromptArgs {
   const float *q, *k, *v;
   float *out;
   int64_t q_stride, q_hstride, o_stride, o_hstride, kv_stride;
   int kv_heads, group, q_len, k_len, q_offset, nblk;
-  int per_head;     // tiles of a KV head
-  int share, extra; // tiles of a workgroup; the first `extra` ones take one more
+  int ahead;        // units ahead of a block's first tile
+  int per_head;     // units of a KV head: its tiles and those
+  int share, extra; // units of a workgroup, `ahead` + 1 at least; the first `extra` ones take one more
   float scale;      // of the scores, times log2 e
   float *acc, *ml;
   PromptBlock *blocks;
@@ -64,11 +66,11 @@ __device__ __forceinline__ int wave_scan(int v, int lane) {
   }
   return v;
 }
-// the block that tile t of a KV head belongs to (t becomes the tile within it), or
-// nblk with t the number of tiles beyond the last block
+// the block that unit t of a KV head belongs to (t becomes the unit within it), or
+// nblk with t the number of units beyond the last block
 __device__ __forceinline__ int find_block(const PromptArgs &a, int lane, int &t) {
   for (int base = 0; base < a.nblk; base += 64) {
-    const int n = base + lane < a.nblk ? tiles_of(a, base + lane) : 0;
+    const int n = base + lane < a.nblk ? tiles_of(a, base + lane) + a.ahead : 0;
     const int incl = wave_scan(n, lane);
     const unsigned long long past = __ballot(incl > t);
     if (past) {
@@ -81,43 +83,75 @@ __device__ __forceinline__ int find_block(const PromptArgs &a, int lane, int &t)
   return a.nblk;
 }
 
-__device__ __forceinline__ f32x16 mma(uint4 a, uint4 b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
-                                                 __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ unsigned round2(float x, float y) { // one instruction
-  return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{x, y}), bf16x2));
+__device__ __forceinline__ f32x16 mma(uint4 a, uint4 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
 }
-// two values as three words of two bfloat16 terms; returns NaN where one is not finite
-__device__ __forceinline__ float split2(float x, float y, unsigned &t0, unsigned &t1, unsigned &t2) {
-  t0 = round2(x, y);
-  x -= bf_lo(t0);
-  y -= bf_hi(t0);
-  t1 = round2(x, y);
-  x -= bf_lo(t1);
-  y -= bf_hi(t1);
-  t2 = round2(x, y);
-  return x + y;
+// two values as two words of two float16 terms; what is not finite has a NaN among its terms
+__device__ __forceinline__ void split2(float x, float y, unsigned &t0, unsigned &t1) {
+  const f16x2 h = __builtin_convertvector((f32x2{x, y}), f16x2);
+  t0 = __builtin_bit_cast(unsigned, h);
+  t1 = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{x - (float)h[0], y - (float)h[1]}), f16x2));
 }
-__device__ __forceinline__ float split8(const float (&x)[8], uint4 (&t)[3]) {
-  unsigned w[3][4];
-  float bad = 0.f;
+__device__ __forceinline__ void split8(const float (&x)[8], uint4 (&t)[2]) {
+  unsigned w[2][4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
-    bad += split2(x[2 * i], x[2 * i + 1], w[0][i], w[1][i], w[2][i]);
+    split2(x[2 * i], x[2 * i + 1], w[0][i], w[1][i]);
 #pragma unroll
-  for (int p = 0; p < 3; ++p)
+  for (int p = 0; p < 2; ++p)
     t[p] = uint4{w[p][0], w[p][1], w[p][2], w[p][3]};
-  return bad;
 }
-// the six products of more than 2^-24: (term of a, term of b), small ones first
-constexpr int kProdA[6] = {0, 2, 1, 0, 1, 0};
-constexpr int kProdB[6] = {2, 0, 1, 1, 0, 0};
+// The power of two that brings a magnitude (as bits) to 2^14 .. 2^15, between 2^-114 and 2^126, and its
+// exponent as a float has it.  (An infinity stays one.)
+__device__ __forceinline__ unsigned scale_exponent(unsigned magnitude) { return min(268u - (magnitude >> 23), 253u); }
+__device__ __forceinline__ float pow2(unsigned exponent) { return __uint_as_float(exponent << 23); }
+// maxima and sums over rows of 8 and 16 lanes
+__device__ __forceinline__ unsigned row8_max_u32(unsigned v) {
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, true));
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, true));
+  return max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, true));
+}
+__device__ __forceinline__ unsigned row16_max_u32(unsigned v) {
+  v = row8_max_u32(v);
+  return max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xf, 0xf, true));
+}
+__device__ __forceinline__ int row8_sum_i32(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, true);
+  return v + __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, true);
+}
+__device__ __forceinline__ int row16_sum_i32(int v) {
+  v = row8_sum_i32(v);
+  return v + __builtin_amdgcn_update_dpp(0, v, 0x140, 0xf, 0xf, true);
+}
+__device__ __forceinline__ unsigned magnitude8(const float (&x)[8]) {
+  unsigned m = 0;
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    m = max(m, __float_as_uint(x[e]) & 0x7fffffffu);
+  return m;
+}
+// A row of 128 values in sixteen groups of eight keeps its accuracy, that of every group, while its largest
+// group is not far above the others.  How far a group's magnitude is below the row's in powers of two, 24 at
+// most and none for a group of zeros, comes to more than kStray for all sixteen where one group is 2^12 above
+// the other fifteen, or eight are 2^22 above the other eight.
+constexpr int kStray = 180;
+__device__ __forceinline__ int below(unsigned group, unsigned row) {
+  const int e = (int)(group >> 23);
+  return e ? min((int)(row >> 23) - e, 24) : 0;
+}
+// what a tile's keys are multiplied by at the end, [32] each: of a score; log2 of a value's; its inverse
+struct TileScales {
+  float key[kKeys], value[kKeys], undo[kKeys];
+};
 
 // Workgroup i takes an equal share of all (KV head, row block, key tile) triples in that
-// order, wherever it begins and ends: blocks it holds whole leave as finished rows, the
+// order, wherever it begins and ends; of a long prompt with two units more ahead of each block's first, for to
+// end a block and begin the next takes as long as two tiles (1931 tokens, without them: workgroups end 42 to
+// 64 us after the launch began, with them 40 to 52).  Blocks it holds whole leave as finished rows, the
 // others as partial results.  Its eight wavefronts have 32 rows each and share the tiles,
 // of which each turns an eighth into terms a tile ahead.
 //   S^T[key, row] = K . Q^T;  O^T[d, row] += V^T . P^T
@@ -145,29 +179,33 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
   a.q_offset = p_q_offset;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[]; // [2][kBuf], then 4 KiB per wavefront
   __shared__ unsigned bad_s[3];
+  __shared__ __attribute__((aligned(16))) TileScales scales[2];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 31, up = lane >> 5;
 
-  // this workgroup's tiles [t, t1) of all
+  // this workgroup's units [t0, t1) of all
   const int self = blockIdx.x;
   auto begins = [&](int i) { return i * a.share + min(i, a.extra); };
-  int t = begins(self);
-  const int t0 = t, t1 = begins(self + 1);
+  const int t0 = begins(self), t1 = begins(self + 1);
 
   struct Place {
     int h, b, j, n; // KV head, row block, tile within it, tiles of the block
+    int t;          // unit
   };
   Place at;
   {
-    at.h = t / a.per_head;
-    int r = t - at.h * a.per_head;
+    at.h = t0 / a.per_head;
+    int r = t0 - at.h * a.per_head;
     at.b = find_block(a, lane, r);
-    at.j = r;
+    at.j = max(r - a.ahead, 0);
     at.n = tiles_of(a, at.b);
+    at.t = t0 + max(a.ahead - r, 0);
   }
   auto next_of = [&](Place p) {
+    ++p.t;
     if (++p.j == p.n) {
+      p.t += a.ahead;
       p.j = 0;
       if (++p.b == a.nblk) {
         p.b = 0;
@@ -178,14 +216,14 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
     }
     return p;
   };
+  const int first = at.t; // the workgroup's first tile
 
   // ---- a tile on its way ------------------------------------------------------------
   // Each wavefront brings what it converts itself into 4 KiB of LDS of its own, a tile
   // ahead and past the registers (there are none left), by the four instructions below:
-  // rows 4 wave .. + 3 of the keys, and of the values the eight keys and 64 channels whose
-  // columns its lanes turn.  The compiler does not see these loads; bring_wait() waits for
+  // rows 4 wave .. + 3 of the keys and of the values.  The compiler does not see these loads; bring_wait() waits for
   // them, and nothing else reads that memory.
-  const int g8 = tid & 15, ch = tid & 127, vks = wave >> 2, vhalf = (wave >> 1) & 1;
+  const int g8 = tid & 15;
   unsigned char *raw = lds + 2 * kBuf + wave * 4096;
   auto bring = [&](const Place &p) {
     const float *k = a.k + (int64_t)p.h * a.kv_stride * kPromptD, *v = a.v + (int64_t)p.h * a.kv_stride * kPromptD;
@@ -194,77 +232,193 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
         (int)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)raw);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const float *src;
-      if (i < 2) {
-        const int key = min(k0 + 4 * wave + 2 * i + up, a.k_len - 1);
-        src = k + (int64_t)key * kPromptD + col * 4;
-      } else { // row e of the eight: 16 vks + 8 (e / 4) + 4 vhalf + e % 4
-        const int key = min(k0 + 16 * vks + 8 * (i - 2) + 4 * vhalf + (lane >> 4), a.k_len - 1);
-        src = v + (int64_t)key * kPromptD + (wave & 1) * 64 + (lane & 15) * 4;
-      }
+      const int key = min(k0 + 4 * wave + 2 * (i & 1) + up, a.k_len - 1);
+      const float *src = (i < 2 ? k : v) + (int64_t)key * kPromptD + col * 4;
       asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(to + i * 1024)
                    : "memory", "m0");
     }
   };
   auto bring_wait = []() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
-  auto put_keys = [&](unsigned char *buf) {
-    const float4 x0 = *reinterpret_cast<const float4 *>(raw + (lane >> 4) * 512 + g8 * 32);
-    const float4 x1 = *reinterpret_cast<const float4 *>(raw + (lane >> 4) * 512 + g8 * 32 + 16);
-    const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-    uint4 term[3];
-    split8(x, term);
+  // What this wavefront brought as the tile's terms.  Sixteen lanes have a key's row, eight channels each,
+  // of keys and of values; a lane turns channels lane and lane + 64 of the four values, which are keys
+  // 16 ks + 8 x + 4 half + 0..3.  Everything is read at once.
+  auto row_of = [&](const unsigned char *at, float (&x)[8]) {
+    const float4 x0 = *reinterpret_cast<const float4 *>(at + (lane >> 4) * 512 + g8 * 32);
+    const float4 x1 = *reinterpret_cast<const float4 *>(at + (lane >> 4) * 512 + g8 * 32 + 16);
+    x[0] = x0.x; x[1] = x0.y; x[2] = x0.z; x[3] = x0.w;
+    x[4] = x1.x; x[5] = x1.y; x[6] = x1.z; x[7] = x1.w;
+  };
+  auto columns_of = [&](float (&y)[2][4]) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        y[j][r] = *reinterpret_cast<const float *>(raw + 2048 + r * 512 + (lane + 64 * j) * 4);
+  };
+  auto put_tile = [&](unsigned char *buf, TileScales &sc, unsigned *bad) {
+    float k[8], v[8], y[2][4];
+    row_of(raw, k);
+    row_of(raw + 2048, v);
+    columns_of(y);
     const int key = tid >> 4;
+    {
+      const unsigned group = magnitude8(k), most = row16_max_u32(group), e = scale_exponent(most);
+      const bool stray = row16_sum_i32(below(group, most)) > kStray;
+      if (g8 == 0) // of a stray key NaN: the rows that see it are computed again by the fold
+        sc.key[key] = stray ? __uint_as_float(0x7fc00000u) : pow2(254 - e);
 #pragma unroll
-    for (int p = 0; p < 3; ++p)
-      *reinterpret_cast<uint4 *>(buf + ((p * 8 + (g8 >> 1)) * 64 + (g8 & 1) * 32 + (key ^ g8)) * 16) = term[p];
-  };
-  auto put_values = [&](const float (&x)[8], unsigned char *buf) {
-    uint4 term[3];
-    const float rest = split8(x, term);
+      for (int i = 0; i < 8; ++i)
+        k[i] *= pow2(e);
+      uint4 term[2];
+      split8(k, term);
 #pragma unroll
-    for (int p = 0; p < 3; ++p)
-      *reinterpret_cast<uint4 *>(buf + (((p * 4 + (ch >> 5)) * 2 + vks) * 64 + vhalf * 32 + (ch & 31)) * 16) =
-          term[p];
-    return rest;
-  };
-  auto put_values_checked = [&](unsigned char *buf, unsigned *bad) {
-    float x[8];
+      for (int p = 0; p < 2; ++p)
+        *reinterpret_cast<uint4 *>(buf + ((p * 8 + (g8 >> 1)) * 64 + (g8 & 1) * 32 + (key ^ g8)) * 16) = term[p];
+    }
+    unsigned most;
+    for (;;) {
+      const unsigned group = magnitude8(v);
+      most = row16_max_u32(group);
+      const bool stray = most >= 0x7f800000u || row16_sum_i32(below(group, most)) > kStray;
+      if (__builtin_expect(!__any(stray), 1))
+        break;
+      // A value that has no terms, or leaves none to the others, must not reach rows that do not see its
+      // key, whose weight there is zero, nor other channels: it goes in as zero, and its key
+      // makes NaN of the rows that do see it (see add_values), which the fold then computes again.
+      const unsigned from = most >= 0x7f800000u ? 0x7f800000u : most - min(most, 11u << 23);
 #pragma unroll
-    for (int e = 0; e < 8; ++e)
-      x[e] = *reinterpret_cast<const float *>(raw + 2048 + e * 256 + lane * 4);
-    const float rest = put_values(x, buf);
-    if (rest != rest) {
-      // A value that has no terms must not reach rows that do not see its key, whose
-      // weight there is zero: it goes in as zero, and its key makes NaN of the rows that
-      // do see it (see add_values), which the fold then computes again.
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        if (!(fabsf(x[e]) < 3.3895e38f)) {
-          x[e] = 0.f;
-          atomicOr(bad, 1u << (16 * vks + 8 * (e >> 2) + 4 * vhalf + (e & 3)));
+      for (int i = 0; i < 8; ++i)
+        if (stray && (__float_as_uint(v[i]) & 0x7fffffffu) >= from) {
+          v[i] = 0.f;
+          *reinterpret_cast<float *>(raw + 2048 + (lane >> 4) * 512 + g8 * 32 + i * 4) = 0.f;
         }
-      put_values(x, buf);
+      if (stray && g8 == 0)
+        atomicOr(bad, 1u << key);
+      columns_of(y);
+    }
+    const unsigned e = scale_exponent(most);
+    if (g8 == 0) {
+      sc.value[key] = 127.0f - (float)e;
+      sc.undo[key] = pow2(e);
+    }
+    float by[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      by[r] = __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)(e << 23), 16 * r));
+    const int ks = wave >> 2, x8 = (wave >> 1) & 1, half = wave & 1;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int c = lane + 64 * j;
+      unsigned t[2][2];
+      split2(y[j][0] * by[0], y[j][1] * by[1], t[0][0], t[1][0]);
+      split2(y[j][2] * by[2], y[j][3] * by[3], t[0][1], t[1][1]);
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+        *reinterpret_cast<uint2 *>(buf + kHalf + (((p * 4 + (c >> 5)) * 2 + ks) * 64 + half * 32 + (c & 31)) * 16 +
+                                   x8 * 8) = uint2{t[p][0], t[p][1]};
     }
   };
 
-  uint4 qf[8][3];
+  uint4 qf[8][2];
   f32x16 o[4];
-  float m = kSeedM, l = 0.f; // l: this lane's share
+  float m = kSeedM, l = 0.f; // m: a whole number; l: this lane's share
+  float q_scale = 0.f;       // of a score of this lane's row
   int qpos = 0, pos_first = 0, pos_last = 0; // of this lane's row; of the wavefront's rows
-  auto begin_block = [&](const Place &p) {
-    const int row = min(p.b * kPromptRows + wave * 32 + col, a.q_len * a.group - 1);
-    const int tok = row / a.group, hh = row - tok * a.group;
+  // A block's queries come in as eight lanes to a row, 32 channels at a time (as a lane's own operand they
+  // are pieces of 32 rows to a load, and the address unit sets the pace: 4 us), and are turned in
+  // another 4 KiB of the wavefront's.
+  // this lane, as something to work addresses out from where they are used: kept from block to block they
+  // would take registers there are not
+  auto unkept = [&]() {
+    int l = lane;
+    asm volatile("" : "+v"(l));
+    return l;
+  };
+  const float per_group = 1.0f / (float)a.group;
+  struct Base {
+    int tok, rem, last; // of a block's first row: token, row within it; the last row from that token on
+  };
+  auto base_of = [&](int b) {
+    const int tok = b * kPromptRows / a.group;
+    return Base{tok, b * kPromptRows - tok * a.group, (a.q_len - tok) * a.group - 1};
+  };
+  auto place_of = [&](const Base &base, int r, int &tok) { // row r of the wavefront: its token, and head of the group
+    const int rem = min(base.rem + wave * 32 + r, base.last);
+    const int t = (int)(((float)rem + 0.5f) * per_group);
+    tok = base.tok + t;
+    return rem - t * a.group;
+  };
+  auto ask_queries = [&](const Place &p, float4 (&asked)[16]) {
+    const int lane = unkept();
+    const Base base = base_of(p.b);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      int tok;
+      const int hh = place_of(base, 8 * j + (lane >> 3), tok);
+      const float *src = a.q + (int64_t)tok * a.q_stride + (int64_t)(p.h * a.group + hh) * a.q_hstride + (lane & 7) * 4;
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        asked[4 * c + j] = *reinterpret_cast<const float4 *>(src + c * 32);
+    }
+  };
+  auto begin_block = [&](int b, float4 (&asked)[16]) {
+    const int lane = unkept(), col = lane & 31, up = lane >> 5;
+    int tok;
+    place_of(base_of(b), col, tok);
     qpos = a.q_offset + tok;
     pos_first = __builtin_amdgcn_readfirstlane(qpos);
     pos_last = __builtin_amdgcn_readlane(qpos, 31);
-    const float *src = a.q + (int64_t)tok * a.q_stride + (int64_t)(p.h * a.group + hh) * a.q_hstride + up * 8;
+    unsigned char *turn = raw + kThreads / 64 * 4096;
+    float of_row[4];
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      const float4 x0 = *reinterpret_cast<const float4 *>(src + s * 16);
-      const float4 x1 = *reinterpret_cast<const float4 *>(src + s * 16 + 4);
-      const float y[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-      split8(y, qf[s]);
+    for (int j = 0; j < 4; ++j) { // row 8 j + lane / 8: eight lanes with two groups of eight values each
+      unsigned group[2], most;
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        const float4 u = asked[8 * g + j], v = asked[8 * g + 4 + j];
+        const float y[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+        group[g] = magnitude8(y);
+      }
+      most = row8_max_u32(max(group[0], group[1]));
+      const int sum = row8_sum_i32(below(group[0], most) + below(group[1], most));
+      const unsigned e = scale_exponent(most);
+      of_row[j] = sum > kStray ? __uint_as_float(0x7fc00000u) : pow2(254 - e) * a.scale;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        float4 &u = asked[4 * c + j];
+        u = make_float4(u.x * pow2(e), u.y * pow2(e), u.z * pow2(e), u.w * pow2(e));
+      }
     }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      // 32 channels of all rows as terms, [term][row][64 bytes]; pieces of 16 bytes permuted by the row's number
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float4 u = asked[4 * c + j];
+        const int r = 8 * j + (lane >> 3);
+        uint2 t[2];
+        split2(u.x, u.y, t[0].x, t[1].x);
+        split2(u.z, u.w, t[0].y, t[1].y);
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+          *reinterpret_cast<uint2 *>(turn + p * 2048 + r * 64 + (((lane & 7) >> 1) ^ (r >> 1 & 3)) * 16 +
+                                     (lane & 1) * 8) = t[p];
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+          qf[2 * c + i][p] = *reinterpret_cast<const uint4 *>(turn + p * 2048 + col * 64 +
+                                                              ((2 * i + up) ^ (col >> 1 & 3)) * 16);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if ((lane & 7) == 0) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        *reinterpret_cast<float *>(turn + (8 * j + (lane >> 3)) * 4) = of_row[j];
+    }
+    q_scale = *reinterpret_cast<const float *>(turn + col * 4);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       o[i] = f32x16{};
@@ -273,57 +427,94 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
   };
 
   float w[16];    // scores of this lane's row, then their weights
-  uint4 pf[2][3]; // the weights as terms
+  uint4 pf[2][2]; // the weights as terms
   auto scores = [&](const unsigned char *buf) {
-    f32x16 s0{}, s1{};
+    f32x16 s0{}, s1{}; // the small products by themselves
     // the slot of this lane's key in step s is (col ^ up) ^ 2 s: worked out at each tile,
     // not kept in registers that there are not
     int at_key = up * 512 + (col ^ up) * 16;
     asm volatile("" : "+v"(at_key));
+    // fragments are asked for two steps ahead of their products, and stay there: left to itself the
+    // scheduler moves them to their use, and every one is waited out
+    uint4 kf[3][2];
+    auto ask = [&](int s) {
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+        kf[s % 3][p] = *reinterpret_cast<const uint4 *>(buf + (at_key ^ (32 * s)) + (p * 8 + s) * 1024);
+    };
+    ask(0);
+    ask(1);
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
-      uint4 kf[3];
-#pragma unroll
-      for (int p = 0; p < 3; ++p)
-        kf[p] = *reinterpret_cast<const uint4 *>(buf + (at_key ^ (32 * s)) + (p * 8 + s) * 1024);
-#pragma unroll
-      for (int c = 0; c < 6; c += 2) { // two chains: an instruction waits for the sum it adds to
-        s0 = mma(kf[kProdA[c]], qf[s][kProdB[c]], s0);
-        s1 = mma(kf[kProdA[c + 1]], qf[s][kProdB[c + 1]], s1);
-      }
+      if (s + 2 < 8)
+        ask(s + 2);
+      __builtin_amdgcn_sched_barrier(0);
+      s1 = mma(kf[s % 3][0], qf[s][1], s1);
+      s0 = mma(kf[s % 3][0], qf[s][0], s0);
+      s1 = mma(kf[s % 3][1], qf[s][0], s1);
+      __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int i = 0; i < 16; ++i)
       w[i] = s0[i] + s1[i];
   };
-  auto weights = [&](int k0) {
+  auto weights = [&](int k0, const TileScales &sc) {
+    // this lane's keys are 8 j + 4 up + 0..3
+    auto four = [&](const float (&of)[kKeys], int j) {
+      return *reinterpret_cast<const f32x4 *>(of + 8 * j + 4 * up);
+    };
+    f32x4 by[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const f32x4 k4 = four(sc.key, j);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        w[4 * j + e] *= k4[e];
+    }
     if (k0 + kKeys - 1 > pos_first) { // some of the tile's keys are behind some row
 #pragma unroll
       for (int i = 0; i < 16; ++i)
         w[i] = k0 + 8 * (i >> 2) + 4 * up + (i & 3) <= qpos ? w[i] : -INFINITY;
     }
-    float mt = w[0];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      by[j] = four(sc.value, j);
+    // log2 of the weights times the values' scales, above m, which is whole: one rounding
+    float p[16];
+    auto above = [&]() {
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        p[i] = fmaf(w[i], q_scale, by[i >> 2][i & 3] - m);
+    };
+    above();
+    float mt = p[0];
 #pragma unroll
     for (int i = 1; i < 16; ++i)
-      mt = fmaxf(mt, w[i]);
-    float x, y;
-    lane_pair<32>(mt, x, y);
-    mt = fmaxf(x, y) * a.scale;
-    // the maximum moves, and the sums are rescaled, only when a score exceeds it by more
-    // than kSlack: the weights stay below 2^kSlack
-    if (__any(mt > m + kSlack)) {
-      mt = fmaxf(mt, m);
+      mt = fmaxf(mt, p[i]);
+    // m moves, and the sums are rescaled, only when a weight exceeds 2^kMost
+    if (__any(mt > kMost)) {
+      mt = -INFINITY;
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        mt = fmaxf(mt, fmaf(w[i], q_scale, by[i >> 2][i & 3]));
+      float x, y;
+      lane_pair<32>(mt, x, y);
+      mt = fmaxf(ceilf(fmaxf(x, y)) - kBelow, m);
       const float alpha = __builtin_amdgcn_exp2f(m - mt);
       m = mt;
       l *= alpha;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         o[i] *= alpha;
+      above();
     }
 #pragma unroll
+    for (int j = 0; j < 4; ++j)
+      by[j] = four(sc.undo, j);
+#pragma unroll
     for (int i = 0; i < 16; ++i) {
-      w[i] = __builtin_amdgcn_exp2f(fmaf(w[i], a.scale, -m)); // one rounding before the exponential
-      l += w[i];
+      w[i] = __builtin_amdgcn_exp2f(p[i]);
+      l = fmaf(w[i], by[i >> 2][i & 3], l);
     }
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
@@ -338,20 +529,27 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
       if (last >= 0 && (bad & (last >= 31 ? ~0u : (2u << last) - 1u)))
         l = __uint_as_float(0x7fc00000u);
     }
+    uint4 vf[2][2][2];
+    auto ask = [&](int i) { // 16 keys, two of the four blocks of 32 channels
 #pragma unroll
-    for (int i = 0; i < 4; ++i) { // 16 keys, two of the four blocks of 32 channels
-      uint4 vf[3][2];
-#pragma unroll
-      for (int p = 0; p < 3; ++p)
+      for (int p = 0; p < 2; ++p)
 #pragma unroll
         for (int e = 0; e < 2; ++e)
-          vf[p][e] = *reinterpret_cast<const uint4 *>(
+          vf[i & 1][p][e] = *reinterpret_cast<const uint4 *>(
               buf + (((p * 4 + 2 * (i & 1) + e) * 2 + (i >> 1)) * 64 + lane) * 16);
+    };
+    ask(0);
 #pragma unroll
-      for (int c = 0; c < 6; ++c)
+    for (int i = 0; i < 4; ++i) {
+      if (i < 3)
+        ask(i + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) // small ones first
 #pragma unroll
         for (int e = 0; e < 2; ++e)
-          o[2 * (i & 1) + e] = mma(vf[kProdA[c]][e], pf[i >> 1][kProdB[c]], o[2 * (i & 1) + e]);
+          o[2 * (i & 1) + e] = mma(vf[i & 1][c == 0][e], pf[i >> 1][c == 1], o[2 * (i & 1) + e]);
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
 
@@ -359,29 +557,40 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
     float x, y;
     lane_pair<32>(l, x, y);
     const float sum = x + y;
-    const int r = wave * 32 + col, row = p.b * kPromptRows + r;
-    float *dst;
-    float f = 1.0f;
-    if (whole) {
-      const int tok = row / a.group, hh = row - tok * a.group;
-      dst = a.out + (int64_t)tok * a.o_stride + (int64_t)(p.h * a.group + hh) * a.o_hstride;
-      f = 1.0f / sum;
-    } else {
-      // the first part of this workgroup's share in slot 2 i, one behind it in 2 i + 1
-      const size_t slot = 2 * (size_t)self + (first_tile > t0 ? 1 : 0);
-      dst = a.acc + (slot * kPromptRows + r) * kPromptD;
-      if (up == 0) {
-        a.ml[(slot * kPromptRows + r) * 2] = m;
-        a.ml[(slot * kPromptRows + r) * 2 + 1] = sum;
-      }
+    const int lane = unkept(), col = lane & 31, up = lane >> 5;
+    const int r0 = wave * 32, left = a.q_len * a.group - p.b * kPromptRows - r0; // rows of the wavefront that there are
+    // the first part of this workgroup's share in slot 2 i, one behind it in 2 i + 1
+    const size_t slot = (2 * (size_t)self + (first_tile > first ? 1 : 0)) * kPromptRows + r0;
+    if (!whole && up == 0 && col < left)
+      *reinterpret_cast<float2 *>(a.ml + (slot + col) * 2) = make_float2(m, sum);
+    // turned so that a store writes 128 bytes of each of eight rows (as they lie, 32 of each of 32: twice
+    // as long)
+    unsigned char *turn = raw + kThreads / 64 * 4096;
+    const float f = whole ? 1.0f / sum : 1.0f;
+    const Base base = base_of(p.b);
+    float *dst[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = 8 * i + (lane >> 3);
+      int tok;
+      const int hh = place_of(base, r, tok);
+      dst[i] = (whole ? a.out + (int64_t)tok * a.o_stride + (int64_t)(p.h * a.group + hh) * a.o_hstride
+                      : a.acc + (slot + r) * kPromptD) +
+               (lane & 7) * 4;
     }
-    if (row < a.q_len * a.group) {
 #pragma unroll
-      for (int dt = 0; dt < 4; ++dt)
+    for (int dt = 0; dt < 4; ++dt) { // pieces of 16 bytes permuted by the row's number
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          *reinterpret_cast<float4 *>(dst + dt * 32 + 8 * j + 4 * up) =
-              float4{o[dt][4 * j] * f, o[dt][4 * j + 1] * f, o[dt][4 * j + 2] * f, o[dt][4 * j + 3] * f};
+      for (int j = 0; j < 4; ++j)
+        *reinterpret_cast<float4 *>(turn + col * 128 + ((2 * j + up) ^ (col & 7)) * 16) =
+            float4{o[dt][4 * j] * f, o[dt][4 * j + 1] * f, o[dt][4 * j + 2] * f, o[dt][4 * j + 3] * f};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float4 x = *reinterpret_cast<const float4 *>(turn + (8 * i + (lane >> 3)) * 128 +
+                                                           ((lane & 7) ^ (lane >> 3)) * 16);
+        if (8 * i + (lane >> 3) < left)
+          *reinterpret_cast<float4 *>(dst[i] + dt * 32) = x;
+      }
     }
     if (tid == 0 && from_start) {
       // whoever has the block's first tile says where its parts are
@@ -389,7 +598,7 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
       if (!whole) {
         const int last = first_tile + p.n - 1, longer = a.extra * (a.share + 1);
         const int i = last < longer ? last / (a.share + 1) : a.extra + (last - longer) / a.share;
-        d.first = 2 * self + (first_tile > t0 ? 1 : 0);
+        d.first = 2 * self + (first_tile > first ? 1 : 0);
         d.owner = self;
         d.parts = i - self + 1;
       }
@@ -400,61 +609,73 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
   if (tid < 3)
     bad_s[tid] = 0;
   bring(at);
+  float4 asked[16];
+  ask_queries(at, asked);
   __syncthreads();
   Place nx = next_of(at);
-  begin_block(at);
   bring_wait();
-  put_keys(lds);
-  put_values_checked(lds + kHalf, &bad_s[0]);
-  if (t + 1 < t1)
+  put_tile(lds, scales[0], &bad_s[0]);
+  if (nx.t < t1)
     bring(nx);
-  int seg0 = t; // first tile of the block's part held here
-  bool from_start = at.j == 0;
-  int cur = 0, bad_at = 0; // (t - t0) & 1 and (t - t0) % 3
-  for (;;) {
-    __syncthreads();
-    const int bad_next = bad_at == 2 ? 0 : bad_at + 1, bad_after = bad_next == 2 ? 0 : bad_next + 1;
-    const unsigned bad = __builtin_amdgcn_readfirstlane(bad_s[bad_at]);
-    if (tid == 0)
-      bad_s[bad_after] = 0;
-    const bool more = t + 1 < t1;
-    const Place nn = next_of(nx);
-    unsigned char *buf = lds + cur * kBuf, *other = lds + (cur ^ 1) * kBuf;
-    auto stage = [&]() {
-      if (!more)
-        return;
-      bring_wait();
-      put_keys(other);
-      put_values_checked(other + kHalf, &bad_s[bad_next]);
-      if (t + 2 < t1)
-        bring(nn);
-    };
-    // the two wavefronts of a SIMD in opposite order: one's conversion beside the other's
-    // products
-    if (wave < 4)
-      stage();
-    if (at.j * kKeys <= pos_last) {
-      scores(buf);
-      weights(at.j * kKeys);
-      add_values(buf + kHalf, at.j * kKeys, bad);
+  int cur = 0, bad_at = 0; // which of two, of three
+  bool arrived = false;    // the tile on its way
+  for (;;) { // a block, or the part of it held here, at a time
+    begin_block(at.b, asked);
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      asked[i] = float4{}; // what was in them need not be kept
+    const int seg0 = at.t; // its first tile
+    const bool from_start = at.j == 0;
+    bool more, ends;
+    for (;;) {
+      __syncthreads();
+      const int bad_next = bad_at == 2 ? 0 : bad_at + 1, bad_after = bad_next == 2 ? 0 : bad_next + 1;
+      const unsigned bad = __builtin_amdgcn_readfirstlane(bad_s[bad_at]);
+      if (tid == 0)
+        bad_s[bad_after] = 0;
+      more = nx.t < t1;
+      const Place nn = next_of(nx);
+      unsigned char *buf = lds + cur * kBuf, *other = lds + (cur ^ 1) * kBuf;
+      auto stage = [&]() {
+        if (!more)
+          return;
+        if (!arrived)
+          bring_wait();
+        put_tile(other, scales[cur ^ 1], &bad_s[bad_next]);
+        if (nn.t < t1)
+          bring(nn);
+      };
+      // the two wavefronts of a SIMD in opposite order: one's conversion beside the other's
+      // products
+      if (wave < 4)
+        stage();
+      if (at.j * kKeys <= pos_last) {
+        scores(buf);
+        weights(at.j * kKeys, scales[cur]);
+        add_values(buf + kHalf, at.j * kKeys, bad);
+      }
+      if (wave >= 4)
+        stage();
+      arrived = false;
+      ends = at.j + 1 == at.n;
+      if (ends || !more)
+        break;
+      at = nx;
+      nx = nn;
+      cur ^= 1;
+      bad_at = bad_next;
     }
-    if (wave >= 4)
-      stage();
-    const bool ends = at.j + 1 == at.n;
-    if (ends || !more)
-      end_block(at, seg0, from_start, ends && from_start);
+    if (more)
+      ask_queries(nx, asked); // ahead of the stores, which a load behind them would wait for
+    end_block(at, seg0, from_start, ends && from_start);
     if (!more)
       break;
-    ++t;
-    if (ends) {
-      begin_block(nx);
-      seg0 = t;
-      from_start = true;
-    }
     at = nx;
-    nx = nn;
+    nx = next_of(nx);
     cur ^= 1;
-    bad_at = bad_next;
+    bad_at = bad_at == 2 ? 0 : bad_at + 1;
+    // begin_block waits for the queries, which were asked for behind that tile, and not for the stores
+    arrived = true;
   }
 }
 
@@ -465,7 +686,8 @@ namespace {
 BH_TILE_FAMILY(PromptFamily, "attn_prompt_kernel");
 struct PromptShare {
   int64_t rows, tiles; // rows of a KV head; tiles of all
-  int nblk, workgroups;
+  int64_t units;       // what is shared out
+  int nblk, workgroups, ahead;
 };
 PromptShare share_out(int q_len, int q_offset, int heads, int kv_heads) {
   PromptShare s;
@@ -479,6 +701,8 @@ PromptShare share_out(int q_len, int q_offset, int heads, int kv_heads) {
   }
   s.tiles *= kv_heads;
   s.workgroups = (int)std::min<int64_t>(kPromptWorkgroups, s.tiles); // each at least a tile
+  s.ahead = s.tiles >= 4 * kPromptWorkgroups ? 2 : 0;
+  s.units = s.tiles + s.ahead * (int64_t)s.nblk * kv_heads;
   return s;
 }
 } // namespace
@@ -564,15 +788,16 @@ int launch_attn_prompt(const AttnPrefillArgs &in, void *workspace, PromptFold &f
   a.scale = (float)(in.scale * 1.4426950408889634);
   BH_REQUIRE((int64_t)in.q_len * a.group < (1 << 30), "attn_prompt: q_len %d too long", in.q_len);
   const PromptShare share = share_out(in.q_len, a.q_offset, in.heads, in.kv_heads);
-  BH_REQUIRE(share.tiles < (1u << 30), "attn_prompt: %lld tiles of keys", (long long)share.tiles);
+  BH_REQUIRE(share.units < (1u << 30), "attn_prompt: %lld tiles of keys", (long long)share.units);
   a.nblk = share.nblk;
   a.acc = static_cast<float *>(workspace);
   const size_t slots = 2 * (size_t)share.workgroups;
   a.ml = a.acc + slots * kPromptRows * kPromptD;
   a.blocks = reinterpret_cast<PromptBlock *>(a.ml + slots * kPromptRows * 2);
-  a.per_head = (int)(share.tiles / in.kv_heads);
-  a.share = (int)(share.tiles / share.workgroups);
-  a.extra = (int)(share.tiles % share.workgroups);
+  a.ahead = share.ahead;
+  a.per_head = (int)(share.units / in.kv_heads);
+  a.share = (int)(share.units / share.workgroups);
+  a.extra = (int)(share.units % share.workgroups);
   BH_NOTE_VARIANT(PromptFamily, kPromptRows);
   static DynLdsOnce dyn_lds;
   BH_CHECK_HIP(ensure_dyn_lds(dyn_lds, reinterpret_cast<const void *>(attn_prompt_kernel), kLds));

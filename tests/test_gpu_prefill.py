@@ -706,6 +706,39 @@ def test_prompt_attention_of_a_key_beyond_bfloat16_in_long_rows(heads, kv_heads)
         check_close(got, want)
 
 
+@pytest.mark.parametrize("which,powers", [
+    ("v", [0, -20, 9, 3]), ("v", [30, 31, 28, 30]), ("v", [-100, -90, -95, -100]), ("k", [-30, 0, -3, 2]),
+    ("k", [-120, -120, -119, -118]), ("channel", [10, 10, 10, 10]), ("zero", [0, 0, 0, 0])])
+def test_prompt_attention_over_magnitudes(which, powers):
+    """Rows of cached keys or values that differ by powers of two, are all large or all tiny; one channel of the
+    values 2^10 above the others; rows of zeros: as the decode step has them, whose attention is f32."""
+    before, n = 600, 70
+    shape = Shape(layers=2, hidden=256, heads=6, kv_heads=1, head_dim=128, inter=256, vocab=320,
+                  max_len=before + n + 8)
+    toks = synthetic.first_tokens(shape, n, seed=6).astype(np.int32)
+    rows = []
+    for by_token in (False, True):
+        sess, _ = synthetic.build_session(shape, context=before, ln_jitter=0.1)
+        t = sess.get_kv(0 if which == "k" else 1)
+        if which == "zero":
+            t[0, 5:before:7] = 0
+        elif which == "channel":
+            t[0, :before, 77] *= 2.0**10
+        else:
+            t[0, :before] *= 2.0**np.array(powers, np.float32)[np.arange(before) % 4][:, None]
+        sess.set_kv(0 if which == "k" else 1, t)
+        if by_token:
+            for i, tok in enumerate(toks):
+                sess.decode(int(tok), before + i, want_logits=False)
+        else:
+            sess.prefill(toks, before, precision="exact")
+        rows.append([sess.get_kv(j)[0, before:before + n] for j in (2, 3)])
+        sess.close()
+    for got, want in zip(*rows):
+        assert np.isfinite(want).all()
+        check_close(got, want)
+
+
 @pytest.mark.parametrize("at", [0, 3, 4, 15, 16, 31, 63, 70])
 @pytest.mark.parametrize("size", [3.4e38, 8e38])  # above the largest bfloat16 value; infinite
 def test_prompt_attention_of_a_value_beyond_bfloat16(at, size):
