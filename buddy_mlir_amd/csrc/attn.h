@@ -103,10 +103,8 @@ struct AttnPrefillArgs {
 int launch_attn_prefill(const AttnPrefillArgs &a, hipStream_t stream);
 // Rotates q in place for n_tokens rows of [q | k | v], writes rotated k and v
 // into cache rows start_pos .. start_pos + n_tokens - 1.
-int launch_rope_kv_write(float *qkv, int64_t row_stride, const float *inv_freq,
-                         float *kcache, float *vcache, int heads, int kv_heads,
-                         int head_dim, int max_len, int start_pos, int n_tokens,
-                         hipStream_t stream);
+struct RopeKv;
+int launch_rope_kv_write(float *qkv, int64_t row_stride, const RopeKv &rope, int n_tokens, hipStream_t stream);
 
 size_t attn_decode_workspace_bytes(int heads, int max_len);
 int launch_attn_decode(const AttnDecodeArgs &a, hipStream_t stream);

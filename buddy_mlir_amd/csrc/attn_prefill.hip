@@ -11,8 +11,10 @@
 // head (tosa.py:4578-4579,4700); here the KV head is h / group, so the cache is
 // read in place.  The causal structure is exploited: key blocks that lie wholly
 // in a query block's future are skipped (they are exactly zero after softmax).
-// Arithmetic is f32 throughout, on the f32 matrix cores.
+// Arithmetic is f32 throughout, on the f32 matrix cores.  (A session takes it for prompts behind a context;
+// attn_terms.hip for a prompt alone, attn_prompt.hip for long ones.)
 #include "attn.h"
+#include "attn_terms.h"
 
 #include <type_traits>
 
@@ -360,38 +362,44 @@ attn_prefill_kernel(const float *p_k, const float *p_v, const float *p_mask, int
 
 // One workgroup per token: rotate q in place, rotate k into the cache, copy v.
 __global__ void __launch_bounds__(256)
-rope_kv_write_kernel(float *qkv, int64_t row_stride, const float *inv_freq,
-                     float *kcache, float *vcache, int heads, int kv_heads,
-                     int max_len, int start_pos) {
-  __shared__ float cs[kD / 2], sn[kD / 2];
-  const int t = blockIdx.x, pos = start_pos + t;
+rope_kv_write_kernel(float *qkv, int64_t row_stride, RopeKv r) {
+  __shared__ __attribute__((aligned(16))) float cs[kD / 2], sn[kD / 2];
+  const int t = blockIdx.x, pos = r.start_pos + t;
   if (threadIdx.x < kD / 2) {
     float s, c;
-    sincosf(inv_freq[threadIdx.x] * (float)pos, &s, &c);
+    sincosf(r.inv_freq[threadIdx.x] * (float)pos, &s, &c);
     cs[threadIdx.x] = c;
     sn[threadIdx.x] = s;
   }
   __syncthreads();
+  // sixteen threads to a head, with four channels each and their partners 64 further on
+  constexpr int kHalf = kD / 2;
   float *row = qkv + (int64_t)t * row_stride;
-  const int half = kD / 2;
-  for (int i = threadIdx.x; i < (heads + kv_heads) * half; i += 256) {
-    const int hh = i / half, j = i % half;
-    float *v = row + (int64_t)hh * kD; // q heads first, then k heads
-    const float lo = v[j], hi = v[j + half];
-    const float nlo = lo * cs[j] + (-hi) * sn[j];
-    const float nhi = hi * cs[j] + lo * sn[j];
-    if (hh < heads) {
-      v[j] = nlo;
-      v[j + half] = nhi;
-    } else {
-      float *dst = kcache + ((int64_t)(hh - heads) * max_len + pos) * kD;
-      dst[j] = nlo;
-      dst[j + half] = nhi;
+  const int turned = r.heads + r.kv_heads, j = threadIdx.x % 16 * 4;
+  for (int hh = threadIdx.x / 16; hh < turned + r.kv_heads; hh += 16) { // q heads first, then k, then v
+    float *src = row + (int64_t)hh * kD + j;
+    const float4 l4 = *reinterpret_cast<const float4 *>(src), h4 = *reinterpret_cast<const float4 *>(src + kHalf);
+    const float lo[4] = {l4.x, l4.y, l4.z, l4.w}, hi[4] = {h4.x, h4.y, h4.z, h4.w};
+    if (hh >= turned) {
+      float *dst = r.vcache + ((int64_t)(hh - turned) * r.max_len + pos) * kD + j;
+      *reinterpret_cast<float4 *>(dst) = l4;
+      *reinterpret_cast<float4 *>(dst + kHalf) = h4;
+      if (r.terms.tiles)
+        put_value_terms(r.terms, hh - turned, pos, j / 4, lo, hi);
+      continue;
     }
+    float nlo[4], nhi[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      nlo[e] = lo[e] * cs[j + e] + (-hi[e]) * sn[j + e];
+      nhi[e] = hi[e] * cs[j + e] + lo[e] * sn[j + e];
+    }
+    float *dst = hh < r.heads ? src : r.kcache + ((int64_t)(hh - r.heads) * r.max_len + pos) * kD + j;
+    *reinterpret_cast<float4 *>(dst) = make_float4(nlo[0], nlo[1], nlo[2], nlo[3]);
+    *reinterpret_cast<float4 *>(dst + kHalf) = make_float4(nhi[0], nhi[1], nhi[2], nhi[3]);
+    if (r.terms.tiles && hh >= r.heads)
+      put_key_terms(r.terms, hh - r.heads, pos, j / 4, nlo, nhi);
   }
-  const float *vsrc = row + (int64_t)(heads + kv_heads) * kD;
-  for (int i = threadIdx.x; i < kv_heads * kD; i += 256)
-    vcache[((int64_t)(i / kD) * max_len + pos) * kD + i % kD] = vsrc[i];
 }
 
 } // namespace
@@ -468,18 +476,16 @@ int launch_attn_prefill(const AttnPrefillArgs &in, hipStream_t stream) {
   return BUDDY_HIP_OK;
 }
 
-int launch_rope_kv_write(float *qkv, int64_t row_stride, const float *inv_freq,
-                         float *kcache, float *vcache, int heads, int kv_heads,
-                         int head_dim, int max_len, int start_pos, int n_tokens,
-                         hipStream_t stream) {
-  BH_REQUIRE(qkv && inv_freq && kcache && vcache, "rope_kv_write: null pointer");
-  BH_REQUIRE(head_dim == kD, "rope_kv_write: head_dim %d", head_dim);
-  BH_REQUIRE(n_tokens > 0 && start_pos >= 0 && start_pos + n_tokens <= max_len,
+int launch_rope_kv_write(float *qkv, int64_t row_stride, const RopeKv &r, int n_tokens, hipStream_t stream) {
+  BH_REQUIRE(qkv && r.inv_freq && r.kcache && r.vcache, "rope_kv_write: null pointer");
+  BH_REQUIRE(n_tokens > 0 && r.start_pos >= 0 && r.start_pos + n_tokens <= r.max_len,
              "rope_kv_write: tokens %d..%d outside the cache (max_len %d)",
-             start_pos, start_pos + n_tokens - 1, max_len);
-  hipLaunchKernelGGL(rope_kv_write_kernel, dim3(n_tokens), dim3(256), 0, stream,
-                     qkv, row_stride, inv_freq, kcache, vcache, heads, kv_heads,
-                     max_len, start_pos);
+             r.start_pos, r.start_pos + n_tokens - 1, r.max_len);
+  BH_REQUIRE(row_stride % 4 == 0 &&
+                 ((reinterpret_cast<uintptr_t>(qkv) | reinterpret_cast<uintptr_t>(r.kcache) |
+                   reinterpret_cast<uintptr_t>(r.vcache)) & 15) == 0,
+             "rope_kv_write: rows must be 16-byte aligned");
+  hipLaunchKernelGGL(rope_kv_write_kernel, dim3(n_tokens), dim3(256), 0, stream, qkv, row_stride, r);
   BH_CHECK_HIP(hipGetLastError());
   return BUDDY_HIP_OK;
 }

@@ -2,14 +2,10 @@
 //
 // The same operation as attn_prefill.hip (flash_attention_for_cpu_prefill_op,
 // frontend/Python/ops/tosa.py:4326-4810) with a workspace and on the float16 matrix
-// cores: a row of queries, keys or values is brought to a largest magnitude of 2^14 .. 2^15 by a power of
-// two of its own, and an f32 value is then the sum of two float16 values of 11 bits each, rounded to
-// nearest, 2^-24 off at most (a row's small values 2^-40 of its largest one).  Of the four products
-// of two such sums the three of more than 2^-24 are taken, each exact, all summed in f32.  Three
+// cores, on two float16 terms a value (attn_terms.h): three
 // instructions at sixteen times the rate of the f32 matrix instructions (with three bfloat16 terms, which need
 // no scales, six: 6 us a tile for 3).  The error against 64 bits is that of those terms and of the f32
 // kernel (28-layer prompts of 150 to 1931 tokens, eleven of them, 5.9e-6 on average with either).
-// The power of two of a value's row goes into its weight, whose running maximum is over both.
 //
 // What bounds it: per tile of 256 rows x 32 keys a SIMD has 3072 cycles of matrix
 // instructions and some 3600 of vector instructions (softmax, conversions), which overlap in part:
@@ -21,8 +17,7 @@
 // attn_prefill.hip and the conversion behind that (attn_prompt_pays says which is taken):
 //   1931 tokens 76 vs 150, 150 behind 1900 30 vs 64
 #include "attn.h"
-#include "attn_fold.h"
-#include "bf16_dev.h"
+#include "attn_terms.h"
 
 #include <algorithm>
 #include <cmath>
@@ -31,13 +26,10 @@ namespace bh {
 namespace {
 
 constexpr int kThreads = 2 * kPromptRows; // a wavefront has 32 rows
-constexpr int kKeys = 32;                 // of a tile
-constexpr int kTerm = kKeys * kPromptD * 2; // bytes of one term of a tile's keys or values
-constexpr int kHalf = 2 * kTerm;          // keys, then values
+constexpr int kKeys = kTileKeys;
+constexpr int kHalf = 2 * kTermBytes;     // keys, then values
 constexpr int kBuf = 2 * kHalf;
 constexpr int kLds = 2 * kBuf + kThreads / 64 * 2 * 4096;
-constexpr float kSeedM = -1.0e30f;        // tosa.py:4383
-constexpr float kBelow = 8.0f, kMost = 15.0f; // log2 of a row's largest weight as it is set, and at most
 
 struct PromptArgs {
   const float *q, *k, *v;
@@ -83,81 +75,13 @@ __device__ __forceinline__ int find_block(const PromptArgs &a, int lane, int &t)
   return a.nblk;
 }
 
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ f32x16 mma(uint4 a, uint4 b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-}
-// two values as two words of two float16 terms; what is not finite has a NaN among its terms
-__device__ __forceinline__ void split2(float x, float y, unsigned &t0, unsigned &t1) {
-  const f16x2 h = __builtin_convertvector((f32x2{x, y}), f16x2);
-  t0 = __builtin_bit_cast(unsigned, h);
-  t1 = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{x - (float)h[0], y - (float)h[1]}), f16x2));
-}
-__device__ __forceinline__ void split8(const float (&x)[8], uint4 (&t)[2]) {
-  unsigned w[2][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    split2(x[2 * i], x[2 * i + 1], w[0][i], w[1][i]);
-#pragma unroll
-  for (int p = 0; p < 2; ++p)
-    t[p] = uint4{w[p][0], w[p][1], w[p][2], w[p][3]};
-}
-// The power of two that brings a magnitude (as bits) to 2^14 .. 2^15, between 2^-114 and 2^126, and its
-// exponent as a float has it.  (An infinity stays one.)
-__device__ __forceinline__ unsigned scale_exponent(unsigned magnitude) { return min(268u - (magnitude >> 23), 253u); }
-__device__ __forceinline__ float pow2(unsigned exponent) { return __uint_as_float(exponent << 23); }
-// maxima and sums over rows of 8 and 16 lanes
-__device__ __forceinline__ unsigned row8_max_u32(unsigned v) {
-  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, true));
-  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, true));
-  return max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, true));
-}
-__device__ __forceinline__ unsigned row16_max_u32(unsigned v) {
-  v = row8_max_u32(v);
-  return max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xf, 0xf, true));
-}
-__device__ __forceinline__ int row8_sum_i32(int v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, true);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, true);
-  return v + __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, true);
-}
-__device__ __forceinline__ int row16_sum_i32(int v) {
-  v = row8_sum_i32(v);
-  return v + __builtin_amdgcn_update_dpp(0, v, 0x140, 0xf, 0xf, true);
-}
-__device__ __forceinline__ unsigned magnitude8(const float (&x)[8]) {
-  unsigned m = 0;
-#pragma unroll
-  for (int e = 0; e < 8; ++e)
-    m = max(m, __float_as_uint(x[e]) & 0x7fffffffu);
-  return m;
-}
-// A row of 128 values in sixteen groups of eight keeps its accuracy, that of every group, while its largest
-// group is not far above the others.  How far a group's magnitude is below the row's in powers of two, 24 at
-// most and none for a group of zeros, comes to more than kStray for all sixteen where one group is 2^12 above
-// the other fifteen, or eight are 2^22 above the other eight.
-constexpr int kStray = 180;
-__device__ __forceinline__ int below(unsigned group, unsigned row) {
-  const int e = (int)(group >> 23);
-  return e ? min((int)(row >> 23) - e, 24) : 0;
-}
-// what a tile's keys are multiplied by at the end, [32] each: of a score; log2 of a value's; its inverse
-struct TileScales {
-  float key[kKeys], value[kKeys], undo[kKeys];
-};
-
 // Workgroup i takes an equal share of all (KV head, row block, key tile) triples in that
 // order, wherever it begins and ends; of a long prompt with two units more ahead of each block's first, for to
 // end a block and begin the next takes as long as two tiles (1931 tokens, without them: workgroups end 42 to
 // 64 us after the launch began, with them 40 to 52).  Blocks it holds whole leave as finished rows, the
 // others as partial results.  Its eight wavefronts have 32 rows each and share the tiles,
 // of which each turns an eighth into terms a tile ahead.
-//   S^T[key, row] = K . Q^T;  O^T[d, row] += V^T . P^T
-// and the registers of S^T are the operand P^T as they lie: a lane has keys
-// 8 j + 4 (lane / 32) + 0..3 of row lane % 32, and V^T is stored with its keys in that
-// order.  LDS: [buffer][keys | values][term][step][lane][16 bytes], operands as they are
+// LDS: [buffer][keys | values][term][step][lane][16 bytes], operands as they are
 // read; the keys' slots are permuted within a step so that writing them by rows meets
 // every bank once.
 __global__ void __launch_bounds__(kThreads)
@@ -178,7 +102,6 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
   a.k_len = p_k_len;
   a.q_offset = p_q_offset;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[]; // [2][kBuf], then 4 KiB per wavefront
-  __shared__ unsigned bad_s[3];
   __shared__ __attribute__((aligned(16))) TileScales scales[2];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -255,17 +178,17 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
       for (int r = 0; r < 4; ++r)
         y[j][r] = *reinterpret_cast<const float *>(raw + 2048 + r * 512 + (lane + 64 * j) * 4);
   };
-  auto put_tile = [&](unsigned char *buf, TileScales &sc, unsigned *bad) {
+  auto put_tile = [&](unsigned char *buf, TileScales &sc) {
     float k[8], v[8], y[2][4];
     row_of(raw, k);
     row_of(raw + 2048, v);
     columns_of(y);
     const int key = tid >> 4;
     {
-      const unsigned group = magnitude8(k), most = row16_max_u32(group), e = scale_exponent(most);
-      const bool stray = row16_sum_i32(below(group, most)) > kStray;
-      if (g8 == 0) // of a stray key NaN: the rows that see it are computed again by the fold
-        sc.key[key] = stray ? __uint_as_float(0x7fc00000u) : pow2(254 - e);
+      float undo;
+      const unsigned e = key_scale(k, undo);
+      if (g8 == 0)
+        sc.key[key] = undo;
 #pragma unroll
       for (int i = 0; i < 8; ++i)
         k[i] *= pow2(e);
@@ -275,30 +198,16 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
       for (int p = 0; p < 2; ++p)
         *reinterpret_cast<uint4 *>(buf + ((p * 8 + (g8 >> 1)) * 64 + (g8 & 1) * 32 + (key ^ g8)) * 16) = term[p];
     }
-    unsigned most;
-    for (;;) {
-      const unsigned group = magnitude8(v);
-      most = row16_max_u32(group);
-      const bool stray = most >= 0x7f800000u || row16_sum_i32(below(group, most)) > kStray;
-      if (__builtin_expect(!__any(stray), 1))
-        break;
-      // A value that has no terms, or leaves none to the others, must not reach rows that do not see its
-      // key, whose weight there is zero, nor other channels: it goes in as zero, and its key
-      // makes NaN of the rows that do see it (see add_values), which the fold then computes again.
-      const unsigned from = most >= 0x7f800000u ? 0x7f800000u : most - min(most, 11u << 23);
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        if (stray && (__float_as_uint(v[i]) & 0x7fffffffu) >= from) {
-          v[i] = 0.f;
-          *reinterpret_cast<float *>(raw + 2048 + (lane >> 4) * 512 + g8 * 32 + i * 4) = 0.f;
-        }
-      if (stray && g8 == 0)
-        atomicOr(bad, 1u << key);
+    float log2_of;
+    bool again = false;
+    const unsigned e = value_scale(v, log2_of, [&](int i) {
+      *reinterpret_cast<float *>(raw + 2048 + (lane >> 4) * 512 + g8 * 32 + i * 4) = 0.f;
+      again = true;
+    });
+    if (__any(again))
       columns_of(y);
-    }
-    const unsigned e = scale_exponent(most);
     if (g8 == 0) {
-      sc.value[key] = 127.0f - (float)e;
+      sc.value[key] = log2_of;
       sc.undo[key] = pow2(e);
     }
     float by[4];
@@ -320,9 +229,7 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
   };
 
   uint4 qf[8][2];
-  f32x16 o[4];
-  float m = kSeedM, l = 0.f; // m: a whole number; l: this lane's share
-  float q_scale = 0.f;       // of a score of this lane's row
+  RowState rs;
   int qpos = 0, pos_first = 0, pos_last = 0; // of this lane's row; of the wavefront's rows
   // A block's queries come in as eight lanes to a row, 32 channels at a time (as a lane's own operand they
   // are pieces of 32 rows to a load, and the address unit sets the pace: 4 us), and are turned in
@@ -417,13 +324,13 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
       for (int j = 0; j < 4; ++j)
         *reinterpret_cast<float *>(turn + (8 * j + (lane >> 3)) * 4) = of_row[j];
     }
-    q_scale = *reinterpret_cast<const float *>(turn + col * 4);
+    rs.q_scale = *reinterpret_cast<const float *>(turn + col * 4);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      o[i] = f32x16{};
-    m = kSeedM;
-    l = 0.f;
+      rs.o[i] = f32x16{};
+    rs.m = kSeedM;
+    rs.l = 0.f;
   };
 
   float w[16];    // scores of this lane's row, then their weights
@@ -449,86 +356,16 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
       if (s + 2 < 8)
         ask(s + 2);
       __builtin_amdgcn_sched_barrier(0);
-      s1 = mma(kf[s % 3][0], qf[s][1], s1);
-      s0 = mma(kf[s % 3][0], qf[s][0], s0);
-      s1 = mma(kf[s % 3][1], qf[s][0], s1);
+      s1 = mma_f16(kf[s % 3][0], qf[s][1], s1);
+      s0 = mma_f16(kf[s % 3][0], qf[s][0], s0);
+      s1 = mma_f16(kf[s % 3][1], qf[s][0], s1);
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int i = 0; i < 16; ++i)
       w[i] = s0[i] + s1[i];
   };
-  auto weights = [&](int k0, const TileScales &sc) {
-    // this lane's keys are 8 j + 4 up + 0..3
-    auto four = [&](const float (&of)[kKeys], int j) {
-      return *reinterpret_cast<const f32x4 *>(of + 8 * j + 4 * up);
-    };
-    f32x4 by[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const f32x4 k4 = four(sc.key, j);
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        w[4 * j + e] *= k4[e];
-    }
-    if (k0 + kKeys - 1 > pos_first) { // some of the tile's keys are behind some row
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-        w[i] = k0 + 8 * (i >> 2) + 4 * up + (i & 3) <= qpos ? w[i] : -INFINITY;
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      by[j] = four(sc.value, j);
-    // log2 of the weights times the values' scales, above m, which is whole: one rounding
-    float p[16];
-    auto above = [&]() {
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-        p[i] = fmaf(w[i], q_scale, by[i >> 2][i & 3] - m);
-    };
-    above();
-    float mt = p[0];
-#pragma unroll
-    for (int i = 1; i < 16; ++i)
-      mt = fmaxf(mt, p[i]);
-    // m moves, and the sums are rescaled, only when a weight exceeds 2^kMost
-    if (__any(mt > kMost)) {
-      mt = -INFINITY;
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-        mt = fmaxf(mt, fmaf(w[i], q_scale, by[i >> 2][i & 3]));
-      float x, y;
-      lane_pair<32>(mt, x, y);
-      mt = fmaxf(ceilf(fmaxf(x, y)) - kBelow, m);
-      const float alpha = __builtin_amdgcn_exp2f(m - mt);
-      m = mt;
-      l *= alpha;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        o[i] *= alpha;
-      above();
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      by[j] = four(sc.undo, j);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      w[i] = __builtin_amdgcn_exp2f(p[i]);
-      l = fmaf(w[i], by[i >> 2][i & 3], l);
-    }
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      const float p8[8] = {w[8 * ks], w[8 * ks + 1], w[8 * ks + 2], w[8 * ks + 3],
-                           w[8 * ks + 4], w[8 * ks + 5], w[8 * ks + 6], w[8 * ks + 7]};
-      split8(p8, pf[ks]);
-    }
-  };
-  auto add_values = [&](const unsigned char *buf, int k0, unsigned bad) {
-    if (bad) { // keys up to this row's own position
-      const int last = qpos - k0;
-      if (last >= 0 && (bad & (last >= 31 ? ~0u : (2u << last) - 1u)))
-        l = __uint_as_float(0x7fc00000u);
-    }
+  auto add_values = [&](const unsigned char *buf) {
     uint4 vf[2][2][2];
     auto ask = [&](int i) { // 16 keys, two of the four blocks of 32 channels
 #pragma unroll
@@ -548,21 +385,21 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
       for (int c = 0; c < 3; ++c) // small ones first
 #pragma unroll
         for (int e = 0; e < 2; ++e)
-          o[2 * (i & 1) + e] = mma(vf[i & 1][c == 0][e], pf[i >> 1][c == 1], o[2 * (i & 1) + e]);
+          rs.o[2 * (i & 1) + e] = mma_f16(vf[i & 1][c == 0][e], pf[i >> 1][c == 1], rs.o[2 * (i & 1) + e]);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
 
   auto end_block = [&](const Place &p, int first_tile, bool from_start, bool whole) {
     float x, y;
-    lane_pair<32>(l, x, y);
+    lane_pair<32>(rs.l, x, y);
     const float sum = x + y;
     const int lane = unkept(), col = lane & 31, up = lane >> 5;
     const int r0 = wave * 32, left = a.q_len * a.group - p.b * kPromptRows - r0; // rows of the wavefront that there are
     // the first part of this workgroup's share in slot 2 i, one behind it in 2 i + 1
     const size_t slot = (2 * (size_t)self + (first_tile > first ? 1 : 0)) * kPromptRows + r0;
     if (!whole && up == 0 && col < left)
-      *reinterpret_cast<float2 *>(a.ml + (slot + col) * 2) = make_float2(m, sum);
+      *reinterpret_cast<float2 *>(a.ml + (slot + col) * 2) = make_float2(rs.m, sum);
     // turned so that a store writes 128 bytes of each of eight rows (as they lie, 32 of each of 32: twice
     // as long)
     unsigned char *turn = raw + kThreads / 64 * 4096;
@@ -583,7 +420,7 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         *reinterpret_cast<float4 *>(turn + col * 128 + ((2 * j + up) ^ (col & 7)) * 16) =
-            float4{o[dt][4 * j] * f, o[dt][4 * j + 1] * f, o[dt][4 * j + 2] * f, o[dt][4 * j + 3] * f};
+            float4{rs.o[dt][4 * j] * f, rs.o[dt][4 * j + 1] * f, rs.o[dt][4 * j + 2] * f, rs.o[dt][4 * j + 3] * f};
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float4 x = *reinterpret_cast<const float4 *>(turn + (8 * i + (lane >> 3)) * 128 +
@@ -606,18 +443,16 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
     }
   };
 
-  if (tid < 3)
-    bad_s[tid] = 0;
   bring(at);
   float4 asked[16];
   ask_queries(at, asked);
   __syncthreads();
   Place nx = next_of(at);
   bring_wait();
-  put_tile(lds, scales[0], &bad_s[0]);
+  put_tile(lds, scales[0]);
   if (nx.t < t1)
     bring(nx);
-  int cur = 0, bad_at = 0; // which of two, of three
+  int cur = 0;
   bool arrived = false;    // the tile on its way
   for (;;) { // a block, or the part of it held here, at a time
     begin_block(at.b, asked);
@@ -629,10 +464,6 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
     bool more, ends;
     for (;;) {
       __syncthreads();
-      const int bad_next = bad_at == 2 ? 0 : bad_at + 1, bad_after = bad_next == 2 ? 0 : bad_next + 1;
-      const unsigned bad = __builtin_amdgcn_readfirstlane(bad_s[bad_at]);
-      if (tid == 0)
-        bad_s[bad_after] = 0;
       more = nx.t < t1;
       const Place nn = next_of(nx);
       unsigned char *buf = lds + cur * kBuf, *other = lds + (cur ^ 1) * kBuf;
@@ -641,7 +472,7 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
           return;
         if (!arrived)
           bring_wait();
-        put_tile(other, scales[cur ^ 1], &bad_s[bad_next]);
+        put_tile(other, scales[cur ^ 1]);
         if (nn.t < t1)
           bring(nn);
       };
@@ -651,8 +482,9 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
         stage();
       if (at.j * kKeys <= pos_last) {
         scores(buf);
-        weights(at.j * kKeys, scales[cur]);
-        add_values(buf + kHalf, at.j * kKeys, bad);
+        const int k0 = at.j * kKeys;
+        tile_weights(w, scales[cur], up, k0 + kKeys - 1 > pos_first, qpos - k0, rs, pf);
+        add_values(buf + kHalf);
       }
       if (wave >= 4)
         stage();
@@ -663,7 +495,6 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
       at = nx;
       nx = nn;
       cur ^= 1;
-      bad_at = bad_next;
     }
     if (more)
       ask_queries(nx, asked); // ahead of the stores, which a load behind them would wait for
@@ -673,7 +504,6 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
     at = nx;
     nx = next_of(nx);
     cur ^= 1;
-    bad_at = bad_at == 2 ? 0 : bad_at + 1;
     // begin_block waits for the queries, which were asked for behind that tile, and not for the stores
     arrived = true;
   }

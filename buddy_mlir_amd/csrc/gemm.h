@@ -6,11 +6,17 @@
 namespace bh {
 
 // What follows a product that is q | k | v of heads of 128: q rotated in place, k rotated into
-// the cache, v copied there (launch_rope_kv_write).
+// the cache, v copied there (launch_rope_kv_write), and both as terms.
+// Rows of keys and values as a prompt's attention can take them too (attn_terms.h); no tiles: not wanted.
+struct PromptTerms {
+  unsigned char *tiles = nullptr; // [KV heads][per_head]
+  int per_head = 0;
+};
 struct RopeKv {
   const float *inv_freq = nullptr; // [64]
   float *kcache = nullptr, *vcache = nullptr;
   int heads = 0, kv_heads = 0, max_len = 0, start_pos = 0;
+  PromptTerms terms;
 };
 
 // The unscaled sums of a product's K slices, [tile][slice][wavefront][row][channel] with tiles

@@ -32,6 +32,7 @@
 // kTiles3, with the activation fragments shared through LDS.
 #include "attn.h"
 #include "attn_fold.h"
+#include "attn_terms.h"
 #include "digits_dev.h"
 #include "gemm.h"
 #include "tile_place.h"
@@ -1119,7 +1120,7 @@ reduce_slices_kernel(GemmI8Args a) {
 }
 
 // The same where C is q | k | v and what follows it is the rotation and the cache rows: a
-// thread has four channels of a q or k head and their partners 64 further on, or four of v.
+// thread has four channels of a head and their partners 64 further on.
 // Its angles are worked out while its loads are on their way (27 rows of 2048 channels: 4.7 us
 // and 3.4 in a launch behind it, 5.4 in this one; prompts of 3 to 100 tokens 2 to 5 % shorter).
 // Small workgroups: a short prompt's few loads then come in through many compute units.
@@ -1127,7 +1128,7 @@ constexpr int kRopeThreads = 64;
 __global__ void __launch_bounds__(kRopeThreads)
 reduce_slices_rope_kernel(SliceSums a, RopeKv r, float *C, int64_t ldc, int M) {
   constexpr int kHalf = kAttnHeadDim / 2;
-  const int turned = (r.heads + r.kv_heads) * (kHalf / 4), per_row = turned + r.kv_heads * (kAttnHeadDim / 4);
+  const int turned = r.heads + r.kv_heads, per_row = (turned + r.kv_heads) * (kHalf / 4);
   const int64_t i = (int64_t)blockIdx.x * kRopeThreads + threadIdx.x;
   if (i >= (int64_t)M * per_row)
     return;
@@ -1170,37 +1171,40 @@ reduce_slices_rope_kernel(SliceSums a, RopeKv r, float *C, int64_t ldc, int M) {
     for (int e = 0; e < 4; ++e)
       v[e] = x.bias[e] + (v[e] * step) * x.scale[e];
   };
-  if (t >= turned) { // v
-    const int at = (t - turned) * 4, head = at / kAttnHeadDim, d = at % kAttnHeadDim;
-    Quad x;
-    request((r.heads + r.kv_heads) * kAttnHeadDim + at, x);
-    float v[4];
-    finish(x, v);
-    *reinterpret_cast<float4 *>(r.vcache + ((int64_t)head * r.max_len + pos) * kAttnHeadDim + d) =
-        make_float4(v[0], v[1], v[2], v[3]);
-    return;
-  }
   const int head = t / (kHalf / 4), j = t % (kHalf / 4) * 4, n = head * kAttnHeadDim + j;
   Quad x, y;
   request(n, x);
   request(n + kHalf, y);
+  const bool is_v = head >= turned;
   float s[4], c[4], lo[4], hi[4];
+  if (!is_v) {
 #pragma unroll
-  for (int e = 0; e < 4; ++e)
-    sincosf(r.inv_freq[j + e] * (float)pos, &s[e], &c[e]);
+    for (int e = 0; e < 4; ++e)
+      sincosf(r.inv_freq[j + e] * (float)pos, &s[e], &c[e]);
+  }
   finish(x, lo);
   finish(y, hi);
-  float4 nlo, nhi;
-  float *l4 = &nlo.x, *h4 = &nhi.x;
+  if (is_v) {
+    const int kvh = head - turned;
+    float *dst = r.vcache + ((int64_t)kvh * r.max_len + pos) * kAttnHeadDim + j;
+    *reinterpret_cast<float4 *>(dst) = make_float4(lo[0], lo[1], lo[2], lo[3]);
+    *reinterpret_cast<float4 *>(dst + kHalf) = make_float4(hi[0], hi[1], hi[2], hi[3]);
+    if (r.terms.tiles) // all sixteen lanes of a head's row
+      put_value_terms(r.terms, kvh, pos, j / 4, lo, hi);
+    return;
+  }
+  float nlo[4], nhi[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    l4[e] = lo[e] * c[e] + (-hi[e]) * s[e];
-    h4[e] = hi[e] * c[e] + lo[e] * s[e];
+    nlo[e] = lo[e] * c[e] + (-hi[e]) * s[e];
+    nhi[e] = hi[e] * c[e] + lo[e] * s[e];
   }
   float *dst = head < r.heads ? row + n
                               : r.kcache + ((int64_t)(head - r.heads) * r.max_len + pos) * kAttnHeadDim + j;
-  *reinterpret_cast<float4 *>(dst) = nlo;
-  *reinterpret_cast<float4 *>(dst + kHalf) = nhi;
+  *reinterpret_cast<float4 *>(dst) = make_float4(nlo[0], nlo[1], nlo[2], nlo[3]);
+  *reinterpret_cast<float4 *>(dst + kHalf) = make_float4(nhi[0], nhi[1], nhi[2], nhi[3]);
+  if (r.terms.tiles && head >= r.heads)
+    put_key_terms(r.terms, head - r.heads, pos, j / 4, nlo, nhi);
 }
 
 // One plane (the w8a8 matmul): the slices hold int32 sums, added exactly; then
@@ -1650,7 +1654,7 @@ int launch_slices_rope(const SliceSums &sums, const RopeKv &r, float *C, int64_t
     BH_NOTE_VARIANT(SlicesRopeFamily, 1);
   else
     BH_NOTE_VARIANT(SlicesRopeFamily, 2);
-  const int64_t quads = (int64_t)M * (r.heads + 3 * r.kv_heads) * (kAttnHeadDim / 8);
+  const int64_t quads = (int64_t)M * (r.heads + 2 * r.kv_heads) * (kAttnHeadDim / 8);
   hipLaunchKernelGGL(reduce_slices_rope_kernel, dim3((unsigned)ceil_div(quads, kRopeThreads)),
                      dim3(kRopeThreads), 0, stream, sums, r, C, ldc, M);
   BH_CHECK_HIP(hipGetLastError());
@@ -1665,8 +1669,7 @@ namespace {
 int norm_behind(const GemmW8Args &in, hipStream_t stream) {
   if (in.then_rope) {
     const RopeKv &r = *in.then_rope;
-    return launch_rope_kv_write(in.C, in.ldc, r.inv_freq, r.kcache, r.vcache, r.heads, r.kv_heads,
-                                kAttnHeadDim, r.max_len, r.start_pos, (int)in.M, stream);
+    return launch_rope_kv_write(in.C, in.ldc, r, (int)in.M, stream);
   }
   if (!in.then_norm_w)
     return BUDDY_HIP_OK;

@@ -821,8 +821,7 @@ int launch_plan(const TilePlan &plan, GemmArgs &a, const GemmW8Args &in, hipStre
     if (a.slices > 1)
       return launch_slices_rope({a.partial, nullptr, a.scale, a.bias, a.slices, a.span, a.tile_rows, a.ncols, a.N},
                                 r, a.C, a.ldc, a.M, stream);
-    return launch_rope_kv_write(a.C, a.ldc, r.inv_freq, r.kcache, r.vcache, r.heads, r.kv_heads, kAttnHeadDim,
-                                r.max_len, r.start_pos, a.M, stream);
+    return launch_rope_kv_write(a.C, a.ldc, r, a.M, stream);
   }
   if (a.slices > 1) {
     if (in.then_norm_w)

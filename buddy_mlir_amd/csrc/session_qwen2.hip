@@ -18,7 +18,7 @@
 // feeds the argmax straight into the next step's embedding gather without a
 // host round trip.
 #include "attn.h"
-#include "attn_fold.h"
+#include "attn_terms.h"
 #include "elementwise.h"
 #include "gemm.h"
 #include "gemv_w8a32.h"
@@ -108,6 +108,7 @@ struct Qwen2Session : Session {
   size_t kv_rows_cap = 0;
   unsigned short *pf_xn_bf = nullptr, *pf_g_bf = nullptr; // bf16 matmul inputs
   void *pf_attn_ws = nullptr;          // partial results of the attention
+  unsigned char *pf_terms = nullptr;   // keys and values of a prompt alone as terms
   unsigned short *pf_att_dg = nullptr; // digit planes or terms of the attention output (o_proj's input)
   int gemm_terms = 3; // bf16 terms per activation in the prefill matmuls (3 = exact)
   int gemm_digits = 3; // int8 digit planes instead of bf16 terms when not 0
@@ -323,6 +324,10 @@ struct Qwen2Session : Session {
       (void)hipFree(pf_attn_ws);
       pf_attn_ws = nullptr;
     }
+    if (pf_terms) {
+      (void)hipFree(pf_terms);
+      pf_terms = nullptr;
+    }
     for (unsigned short **p : {&pf_xn_bf, &pf_g_bf, &pf_att_dg})
       if (*p) {
         (void)hipFree(*p);
@@ -345,6 +350,10 @@ struct Qwen2Session : Session {
     BH_CHECK_HIP(hipMalloc((void **)&pf_g_bf, std::max(lg.bytes(3), lg.bytes_digits(3))));
     const GemmStagingLayout la = gemm_staging_layout(rows, QN);
     BH_CHECK_HIP(hipMalloc((void **)&pf_att_dg, std::max(la.bytes(3), la.bytes_digits(3))));
+    // (a tile's keys beyond the prompt are hidden, but must be numbers)
+    const size_t terms = attn_terms_bytes(S.kv_heads, rows);
+    BH_CHECK_HIP(hipMalloc((void **)&pf_terms, terms));
+    BH_CHECK_HIP(hipMemsetAsync(pf_terms, 0, terms, stream));
     pf_rows = rows;
     return BUDDY_HIP_OK;
   }
@@ -482,9 +491,24 @@ struct Qwen2Session : Session {
     const bool folded = attn_prompt_pays(n, start_pos, S.heads, S.kv_heads, converts);
     if (folded && !pf_attn_ws) // for as many rows as the other buffers have, behind any context
       BH_CHECK_HIP(hipMalloc(&pf_attn_ws, attn_prompt_workspace_bytes(pf_rows, S.max_len, S.heads, S.kv_heads)));
+    // a prompt alone that is not shared out: its attention reads terms that the rotation leaves
+    PromptTerms terms;
+    if (!folded && start_pos == 0 && n <= kTermsMostKeys) {
+      terms.tiles = pf_terms;
+      terms.per_head = (int)ceil_div(pf_rows, kTileKeys);
+    }
     bool normed_ahead = false; // pf_xn_bf already holds this layer's normed input
     for (int i = 0; i < S.layers; ++i) {
       Layer &L = layers[(size_t)i];
+      RopeKv rope;
+      rope.inv_freq = inv_freq;
+      rope.kcache = L.kc;
+      rope.vcache = L.vc;
+      rope.heads = S.heads;
+      rope.kv_heads = S.kv_heads;
+      rope.max_len = S.max_len;
+      rope.start_pos = start_pos;
+      rope.terms = terms;
       if (L.qkv_f32) {
         if ((rc = launch_rmsnorm(pf_x, L.ln1, pf_xn, n, S.hidden, S.rms_eps, stream)))
           return rc;
@@ -502,21 +526,11 @@ struct Qwen2Session : Session {
         if (!normed_ahead && (rc = norm_to_staging(pf_x, L.ln1, n, pf_xn_bf)))
           return rc;
         normed_ahead = false;
-        RopeKv rope;
-        rope.inv_freq = inv_freq;
-        rope.kcache = L.kc;
-        rope.vcache = L.vc;
-        rope.heads = S.heads;
-        rope.kv_heads = S.kv_heads;
-        rope.max_len = S.max_len;
-        rope.start_pos = start_pos;
         if ((rc = gemm_staged(pf_xn_bf, L.qkv, pf_qkv, n, false, 0, nullptr, nullptr, &rope)))
           return rc;
       }
       const bool rotated = !L.qkv_f32 && !(few && L.qkv.N >= kFewChannels);
-      if (!rotated && (rc = launch_rope_kv_write(pf_qkv, QKV, inv_freq, L.kc, L.vc, S.heads,
-                                                 S.kv_heads, S.head_dim, S.max_len, start_pos,
-                                                 n, stream)))
+      if (!rotated && (rc = launch_rope_kv_write(pf_qkv, QKV, rope, n, stream)))
         return rc;
       AttnPrefillArgs a;
       a.q = pf_qkv;
@@ -535,7 +549,9 @@ struct Qwen2Session : Session {
       a.k_len = start_pos + n;
       a.scale = scale;
       PromptFold fold;
-      if ((rc = folded ? launch_attn_prompt(a, pf_attn_ws, fold, stream) : launch_attn_prefill(a, stream)))
+      if ((rc = folded          ? launch_attn_prompt(a, pf_attn_ws, fold, stream)
+                : terms.tiles ? launch_attn_terms(a, terms, stream)
+                              : launch_attn_prefill(a, stream)))
         return rc;
       const int64_t ld_gu = 2 * (int64_t)S.inter;
       const Layer *nx = i + 1 < S.layers ? &layers[(size_t)i + 1] : nullptr;
@@ -702,7 +718,7 @@ struct Qwen2Session : Session {
       (void)hipStreamSynchronize(stream);
     for (void *p : {(void *)pf_x, (void *)pf_xn, (void *)pf_qkv, (void *)pf_att, (void *)pf_g,
                     (void *)pf_tokens, (void *)kv_rows, (void *)pf_xn_bf, (void *)pf_g_bf,
-                    (void *)pf_att_dg, pf_attn_ws})
+                    (void *)pf_att_dg, (void *)pf_terms, pf_attn_ws})
       if (p)
         (void)hipFree(p);
     release_gemm_staging(stream);

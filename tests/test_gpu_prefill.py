@@ -706,6 +706,40 @@ def test_prompt_attention_of_a_key_beyond_bfloat16_in_long_rows(heads, kv_heads)
         check_close(got, want)
 
 
+# a prompt alone on the terms that the rotation leaves: part of a block of 32 rows, a tile of 32 keys and one more, a
+# tile to each wavefront and one more, groups that divide a block and that do not; the rotation in the
+# kernel that adds slices and as a launch of its own, q | k | v in f32
+@pytest.mark.parametrize("heads,kv_heads,n", [(6, 1, 1), (12, 2, 2), (12, 2, 27), (4, 4, 32), (6, 2, 33), (5, 1, 100),
+                                              (8, 1, 257), (12, 2, 300), (3, 3, 545)])
+@pytest.mark.parametrize("qkv_f32", [False, True])
+def test_prompt_attention_on_terms_of_the_rotation(bh, heads, kv_heads, n, qkv_f32):
+    """Behind a longer prompt with a token that is not finite, whose terms are left in the buffer."""
+    shape = Shape(layers=2, hidden=256, heads=heads, kv_heads=kv_heads, head_dim=128, inter=256, vocab=320,
+                  max_len=n + 48)
+    toks = (synthetic.first_tokens(shape, n, seed=n) % 300).astype(np.int32)
+    sess, g = DecoderSession(shape), synthetic.make_globals(shape)
+    g["embed"][310, 7] = float("nan")
+    sess.set_globals(g["embed"], g["inv_freq"], g["ln_f"], g["w_lm"], g["s_lm"])
+    for i in range(shape.layers):
+        w = synthetic.make_layer(shape, i, 0.1)
+        for t in "qkv" if qkv_f32 else "":
+            w["f" + t] = w.pop("w" + t).float() * w.pop("s" + t)
+            w["b" + t] = torch.zeros(w["f" + t].shape[1], device="cuda")
+        sess.set_layer(i, w)
+    torch.cuda.synchronize()
+    sess.prefill(np.concatenate([toks[:1], [310], np.tile(toks, 40)[:n + 20]]).astype(np.int32), 0)
+    bh.buddy_hip_variant_reset()
+    _, got = sess.prefill(toks, 0, precision="exact")
+    assert tiles_run(bh)["attn_terms_kernel<32>"] == shape.layers
+    rows = [sess.get_kv(j)[:, :n] for j in (2, 3)]
+    for i, t in enumerate(toks):
+        _, want = sess.decode(int(t), i, want_logits=i + 1 == n)
+    check_close(got, want)
+    for j in (2, 3):
+        check_close(rows[j - 2], sess.get_kv(j)[:, :n])
+    sess.close()
+
+
 @pytest.mark.parametrize("which,powers", [
     ("v", [0, -20, 9, 3]), ("v", [30, 31, 28, 30]), ("v", [-100, -90, -95, -100]), ("k", [-30, 0, -3, 2]),
     ("k", [-120, -120, -119, -118]), ("channel", [10, 10, 10, 10]), ("zero", [0, 0, 0, 0])])
