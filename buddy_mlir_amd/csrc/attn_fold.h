@@ -40,10 +40,12 @@ bool attn_prompt_pays(int q_len, int q_offset, int heads, int kv_heads, bool con
 
 // Attention of a session's prompt tokens (no mask), on a workspace of
 // attn_prompt_workspace_bytes for at least as many tokens and positions; what it leaves is
-// described by `fold`.
+// described by `fold`.  `terms`: of a prompt alone, or none.
 struct AttnPrefillArgs;
+struct PromptTerms;
 size_t attn_prompt_workspace_bytes(int q_len, int k_len, int heads, int kv_heads);
-int launch_attn_prompt(const AttnPrefillArgs &a, void *workspace, PromptFold &fold, hipStream_t stream);
+int launch_attn_prompt(const AttnPrefillArgs &a, const PromptTerms &terms, void *workspace, PromptFold &fold,
+                       hipStream_t stream);
 // the finished rows as the bf16 terms of the matmul behind the attention (gemm_w8_mfma.hip) ...
 int launch_attn_fold_to_terms(const PromptFold &fold, int64_t o_stride, int heads, int tokens, int terms,
                               unsigned short *staged, hipStream_t stream);
@@ -96,7 +98,11 @@ __device__ __forceinline__ void f32_row(const PromptFold &f, int t, int h, int d
     v[e] *= inv;
 }
 
-// four values d .. d + 3 of query head h at token t, from where the launch left them
+// Four values d .. d + 3 of query head h at token t, from where the launch left them; at most kMost parts
+// asked for at once.  Sixteen take registers that leave a compute unit one workgroup of 512 threads: for as
+// many tokens as make two rounds of those.  (1931 tokens 23 us so, four parts at once 14.2.)
+constexpr int kFoldTokens = 512; // up to which sixteen are asked for
+template <int kMost>
 __device__ __forceinline__ void left4(const PromptFold &f, int64_t out_stride, int t, int h, int d,
                                       float (&v)[4]) {
   const int kvh = h / f.group, row = t * f.group + (h - kvh * f.group);
@@ -142,12 +148,12 @@ __device__ __forceinline__ void left4(const PromptFold &f, int64_t out_stride, i
       s[3] = fmaf(q[i].w, w, s[3]);
     }
   };
-  if (b.parts <= 8)
+  if (kMost == 4 || b.parts <= 8)
     for (int j = 0; j < b.parts; j += 4)
       add(j, std::integral_constant<int, 4>{});
   else
-    for (int j = 0; j < b.parts; j += 16)
-      add(j, std::integral_constant<int, 16>{});
+    for (int j = 0; j < b.parts; j += kMost)
+      add(j, std::integral_constant<int, kMost>{});
   const float inv = 1.0f / l;
 #pragma unroll
   for (int e = 0; e < 4; ++e)

@@ -360,45 +360,104 @@ attn_prefill_kernel(const float *p_k, const float *p_v, const float *p_mask, int
   }
 }
 
-// One workgroup per token: rotate q in place, rotate k into the cache, copy v.
+// Rotate q in place, rotate k into the cache, copy v, and both as terms.  The last n_tokens workgroups take a token's
+// query heads each, those ahead of them the keys and values of four tokens.  Sixteen threads to a row have four
+// channels each and their partners 64 further on.  Of the values' terms a channel's four keys lie side by
+// side, so they meet in LDS (two bytes at a time from a workgroup per token 1931 tokens took 13.3 us; so
+// 9.8, without terms 6.5).
+constexpr int kRopeTokens = 4;
 __global__ void __launch_bounds__(256)
-rope_kv_write_kernel(float *qkv, int64_t row_stride, RopeKv r) {
-  __shared__ __attribute__((aligned(16))) float cs[kD / 2], sn[kD / 2];
-  const int t = blockIdx.x, pos = r.start_pos + t;
-  if (threadIdx.x < kD / 2) {
-    float s, c;
-    sincosf(r.inv_freq[threadIdx.x] * (float)pos, &s, &c);
-    cs[threadIdx.x] = c;
-    sn[threadIdx.x] = s;
-  }
-  __syncthreads();
-  // sixteen threads to a head, with four channels each and their partners 64 further on
+rope_kv_write_kernel(float *qkv, int64_t row_stride, int n_tokens, RopeKv r) {
   constexpr int kHalf = kD / 2;
-  float *row = qkv + (int64_t)t * row_stride;
-  const int turned = r.heads + r.kv_heads, j = threadIdx.x % 16 * 4;
-  for (int hh = threadIdx.x / 16; hh < turned + r.kv_heads; hh += 16) { // q heads first, then k, then v
-    float *src = row + (int64_t)hh * kD + j;
-    const float4 l4 = *reinterpret_cast<const float4 *>(src), h4 = *reinterpret_cast<const float4 *>(src + kHalf);
-    const float lo[4] = {l4.x, l4.y, l4.z, l4.w}, hi[4] = {h4.x, h4.y, h4.z, h4.w};
-    if (hh >= turned) {
-      float *dst = r.vcache + ((int64_t)(hh - turned) * r.max_len + pos) * kD + j;
-      *reinterpret_cast<float4 *>(dst) = l4;
-      *reinterpret_cast<float4 *>(dst + kHalf) = h4;
-      if (r.terms.tiles)
-        put_value_terms(r.terms, hh - turned, pos, j / 4, lo, hi);
-      continue;
-    }
-    float nlo[4], nhi[4];
+  __shared__ __attribute__((aligned(16))) unsigned short vt[4][2][kD][kRopeTokens];
+  const int tid = threadIdx.x, j = tid % 16 * 4, groups = (n_tokens + kRopeTokens - 1) / kRopeTokens;
+  auto load = [&](const float *src, float (&lo)[4], float (&hi)[4]) {
+    const float4 l = *reinterpret_cast<const float4 *>(src), h = *reinterpret_cast<const float4 *>(src + kHalf);
+    lo[0] = l.x; lo[1] = l.y; lo[2] = l.z; lo[3] = l.w;
+    hi[0] = h.x; hi[1] = h.y; hi[2] = h.z; hi[3] = h.w;
+  };
+  auto store = [&](float *dst, const float (&lo)[4], const float (&hi)[4]) {
+    *reinterpret_cast<float4 *>(dst) = make_float4(lo[0], lo[1], lo[2], lo[3]);
+    *reinterpret_cast<float4 *>(dst + kHalf) = make_float4(hi[0], hi[1], hi[2], hi[3]);
+  };
+  float s[4], c[4];
+  auto angles = [&](int pos) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      sincosf(r.inv_freq[j + e] * (float)pos, &s[e], &c[e]);
+  };
+  auto turn = [&](float (&lo)[4], float (&hi)[4]) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      nlo[e] = lo[e] * cs[j + e] + (-hi[e]) * sn[j + e];
-      nhi[e] = hi[e] * cs[j + e] + lo[e] * sn[j + e];
+      const float l = lo[e], h = hi[e];
+      lo[e] = l * c[e] + (-h) * s[e];
+      hi[e] = h * c[e] + l * s[e];
     }
-    float *dst = hh < r.heads ? src : r.kcache + ((int64_t)(hh - r.heads) * r.max_len + pos) * kD + j;
-    *reinterpret_cast<float4 *>(dst) = make_float4(nlo[0], nlo[1], nlo[2], nlo[3]);
-    *reinterpret_cast<float4 *>(dst + kHalf) = make_float4(nhi[0], nhi[1], nhi[2], nhi[3]);
-    if (r.terms.tiles && hh >= r.heads)
-      put_key_terms(r.terms, hh - r.heads, pos, j / 4, nlo, nhi);
+  };
+  float lo[4], hi[4];
+  if ((int)blockIdx.x >= groups) {
+    const int t = blockIdx.x - groups;
+    float *row = qkv + (int64_t)t * row_stride + j;
+    if (tid / 16 < r.heads)
+      load(row + tid / 16 * kD, lo, hi);
+    angles(r.start_pos + t);
+    for (int h = tid / 16; h < r.heads; h += 16) {
+      if (h >= 16)
+        load(row + (int64_t)h * kD, lo, hi);
+      turn(lo, hi);
+      store(row + (int64_t)h * kD, lo, hi);
+    }
+    return;
+  }
+  // rows (KV head, key or value, token): four KV heads' values meet at a time
+  const int t0 = blockIdx.x * kRopeTokens, pos0 = r.start_pos + t0;
+  const int u = tid / 16 % kRopeTokens, t = t0 + u, pos = pos0 + u;
+  const bool is = t < n_tokens;
+  angles(pos);
+  for (int h0 = 0; h0 < r.kv_heads; h0 += 4) {
+#pragma unroll
+    for (int pass = 0; pass < 2; ++pass) {
+      const int which = pass * 4 + tid / 64, h = h0 + which / 2; // keys of a head, then its values
+      const bool value = which & 1;
+      if (h >= r.kv_heads)
+        continue;
+      load(qkv + (int64_t)min(t, n_tokens - 1) * row_stride + (int64_t)(r.heads + (value ? r.kv_heads : 0) + h) * kD + j,
+           lo, hi);
+      const int64_t at = ((int64_t)h * r.max_len + pos) * kD + j;
+      if (!value) {
+        turn(lo, hi);
+        if (is) {
+          store(r.kcache + at, lo, hi);
+          if (r.terms.tiles)
+            put_key_terms(r.terms, h, pos, j / 4, lo, hi);
+        }
+        continue;
+      }
+      uint4 term[2] = {};
+      if (is) {
+        store(r.vcache + at, lo, hi);
+        if (r.terms.tiles)
+          value_terms(r.terms, h, pos, j / 4, lo, hi, term);
+      }
+      if (r.terms.tiles) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          const unsigned w[4] = {term[p].x, term[p].y, term[p].z, term[p].w};
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            vt[which / 2][p][kHalf * (e / 4) + j + e % 4][u] = (unsigned short)(e & 1 ? w[e / 2] >> 16 : w[e / 2]);
+        }
+      }
+    }
+    if (r.terms.tiles) { // (positions from 0 on: the four keys are neighbours of one tile)
+      __syncthreads();
+      for (int i = tid; i < min(r.kv_heads - h0, 4) * 2 * kD; i += 256) {
+        const int slot = i / (2 * kD), p = i / kD % 2, ch = i % kD;
+        *reinterpret_cast<uint2 *>(value_term_at(terms_tile(r.terms, h0 + slot, pos0), pos0 % kTileKeys, ch, p)) =
+            *reinterpret_cast<const uint2 *>(vt[slot][p][ch]);
+      }
+      __syncthreads();
+    }
   }
 }
 
@@ -485,7 +544,9 @@ int launch_rope_kv_write(float *qkv, int64_t row_stride, const RopeKv &r, int n_
                  ((reinterpret_cast<uintptr_t>(qkv) | reinterpret_cast<uintptr_t>(r.kcache) |
                    reinterpret_cast<uintptr_t>(r.vcache)) & 15) == 0,
              "rope_kv_write: rows must be 16-byte aligned");
-  hipLaunchKernelGGL(rope_kv_write_kernel, dim3(n_tokens), dim3(256), 0, stream, qkv, row_stride, r);
+  BH_REQUIRE(!r.terms.tiles || r.start_pos % kRopeTokens == 0, "rope_kv_write: terms from position %d on", r.start_pos);
+  hipLaunchKernelGGL(rope_kv_write_kernel, dim3((unsigned)(ceil_div(n_tokens, kRopeTokens) + n_tokens)), dim3(256), 0, stream, qkv,
+                     row_stride, n_tokens, r);
   BH_CHECK_HIP(hipGetLastError());
   return BUDDY_HIP_OK;
 }

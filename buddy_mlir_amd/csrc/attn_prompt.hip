@@ -12,12 +12,14 @@
 // 3 us a tile.  What a launch costs beside its tiles: 6 us until the first one is in terms, as much as two
 // tiles to end a block and begin the next (queries and results go through LDS so that a load or store is of whole
 // lines: as operands lie, it was 10 us), and the partial results' way out of the L2s behind it, 33 MB.
-// 1931 tokens of 12 query heads and 2 KV heads 91 -> 53 us, 150 behind 1900 26.6 -> 22.
+// 150 tokens behind 1900 of 12 query heads and 2 KV heads 26.6 -> 22 us; 1931 tokens 91 -> 53, and 47 where keys and
+// values come as terms (a prompt alone, whose rotation writes them: 6.5 -> 9.8 us).
 // us per layer, this kernel and the fold behind it against
 // attn_prefill.hip and the conversion behind that (attn_prompt_pays says which is taken):
-//   1931 tokens 76 vs 150, 150 behind 1900 30 vs 64
+//   150 behind 1900 30 vs 64
 #include "attn.h"
 #include "attn_terms.h"
+#include "digits_dev.h"
 
 #include <algorithm>
 #include <cmath>
@@ -29,7 +31,12 @@ constexpr int kThreads = 2 * kPromptRows; // a wavefront has 32 rows
 constexpr int kKeys = kTileKeys;
 constexpr int kHalf = 2 * kTermBytes;     // keys, then values
 constexpr int kBuf = 2 * kHalf;
-constexpr int kLds = 2 * kBuf + kThreads / 64 * 2 * 4096;
+// two buffers of terms and 4 KiB of each wavefront for what it converts; three that take tiles of terms as they
+// come, scales behind them; and 4 KiB of each to turn rows in
+constexpr int kTermBuf = kBuf + 1024;
+constexpr int lds_bytes(bool terms) {
+  return (terms ? 3 * kTermBuf : 2 * kBuf + kThreads / 64 * 4096) + kThreads / 64 * 4096;
+}
 
 struct PromptArgs {
   const float *q, *k, *v;
@@ -42,6 +49,8 @@ struct PromptArgs {
   float scale;      // of the scores, times log2 e
   float *acc, *ml;
   PromptBlock *blocks;
+  const unsigned char *terms; // [KV heads][per_head tiles]
+  int terms_per_head;
 };
 
 // tiles of keys that block b of 256 rows sees
@@ -84,6 +93,8 @@ __device__ __forceinline__ int find_block(const PromptArgs &a, int lane, int &t)
 // LDS: [buffer][keys | values][term][step][lane][16 bytes], operands as they are
 // read; the keys' slots are permuted within a step so that writing them by rows meets
 // every bank once.
+// TERMS: keys and values lie as terms already, and come tile by tile two ahead.
+template <bool TERMS>
 __global__ void __launch_bounds__(kThreads)
 attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int p_share, int p_extra,
                    int p_per_head, int p_nblk, int p_group, int p_q_len, int p_k_len, int p_q_offset,
@@ -101,8 +112,8 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
   a.q_len = p_q_len;
   a.k_len = p_k_len;
   a.q_offset = p_q_offset;
-  extern __shared__ __attribute__((aligned(16))) unsigned char lds[]; // [2][kBuf], then 4 KiB per wavefront
-  __shared__ __attribute__((aligned(16))) TileScales scales[2];
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  __shared__ __attribute__((aligned(16))) TileScales scales_s[TERMS ? 1 : 2];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 31, up = lane >> 5;
@@ -148,6 +159,25 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
   // them, and nothing else reads that memory.
   const int g8 = tid & 15;
   unsigned char *raw = lds + 2 * kBuf + wave * 4096;
+  unsigned char *turn = lds + lds_bytes(TERMS) - (kThreads / 64 - wave) * 4096;
+  auto buffer = [&](int i) { return lds + i * (TERMS ? kTermBuf : kBuf); };
+  auto scales_of = [&](int i) -> TileScales & {
+    if constexpr (TERMS)
+      return *reinterpret_cast<TileScales *>(buffer(i) + kBuf);
+    else
+      return scales_s[i];
+  };
+  // a tile of terms: 4 KiB of it to a wavefront, and its scales to the first
+  auto bring_terms = [&](const Place &p, int i) {
+    const unsigned char *tile = a.terms + ((size_t)p.h * a.terms_per_head + p.j) * kTermTile;
+    const unsigned to = (unsigned)__builtin_amdgcn_readfirstlane(
+        (int)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)buffer(i));
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+      load_1k_to_lds(tile + (wave * 4 + n) * 1024, lane * 16, to + (wave * 4 + n) * 1024);
+    if (wave == 0)
+      load_1k_to_lds(tile + kBuf, lane * 16, to + kBuf);
+  };
   auto bring = [&](const Place &p) {
     const float *k = a.k + (int64_t)p.h * a.kv_stride * kPromptD, *v = a.v + (int64_t)p.h * a.kv_stride * kPromptD;
     const int k0 = p.j * kKeys;
@@ -275,7 +305,6 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
     qpos = a.q_offset + tok;
     pos_first = __builtin_amdgcn_readfirstlane(qpos);
     pos_last = __builtin_amdgcn_readlane(qpos, 31);
-    unsigned char *turn = raw + kThreads / 64 * 4096;
     float of_row[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) { // row 8 j + lane / 8: eight lanes with two groups of eight values each
@@ -339,7 +368,7 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
     f32x16 s0{}, s1{}; // the small products by themselves
     // the slot of this lane's key in step s is (col ^ up) ^ 2 s: worked out at each tile,
     // not kept in registers that there are not
-    int at_key = up * 512 + (col ^ up) * 16;
+    int at_key = TERMS ? lane * 16 : up * 512 + (col ^ up) * 16;
     asm volatile("" : "+v"(at_key));
     // fragments are asked for two steps ahead of their products, and stay there: left to itself the
     // scheduler moves them to their use, and every one is waited out
@@ -347,7 +376,8 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
     auto ask = [&](int s) {
 #pragma unroll
       for (int p = 0; p < 2; ++p)
-        kf[s % 3][p] = *reinterpret_cast<const uint4 *>(buf + (at_key ^ (32 * s)) + (p * 8 + s) * 1024);
+        kf[s % 3][p] =
+            *reinterpret_cast<const uint4 *>(buf + (TERMS ? at_key : at_key ^ (32 * s)) + (p * 8 + s) * 1024);
     };
     ask(0);
     ask(1);
@@ -402,7 +432,6 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
       *reinterpret_cast<float2 *>(a.ml + (slot + col) * 2) = make_float2(rs.m, sum);
     // turned so that a store writes 128 bytes of each of eight rows (as they lie, 32 of each of 32: twice
     // as long)
-    unsigned char *turn = raw + kThreads / 64 * 4096;
     const float f = whole ? 1.0f / sum : 1.0f;
     const Base base = base_of(p.b);
     float *dst[4];
@@ -443,17 +472,24 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
     }
   };
 
-  bring(at);
-  float4 asked[16];
-  ask_queries(at, asked);
-  __syncthreads();
   Place nx = next_of(at);
-  bring_wait();
-  put_tile(lds, scales[0]);
-  if (nx.t < t1)
-    bring(nx);
+  float4 asked[16];
+  if constexpr (TERMS) {
+    bring_terms(at, 0);
+    if (nx.t < t1)
+      bring_terms(nx, 1);
+    ask_queries(at, asked); // which begin_block waits for, and with them for those
+  } else {
+    bring(at);
+    ask_queries(at, asked);
+    __syncthreads();
+    bring_wait();
+    put_tile(buffer(0), scales_of(0));
+    if (nx.t < t1)
+      bring(nx);
+  }
   int cur = 0;
-  bool arrived = false;    // the tile on its way
+  bool arrived = false; // the tile on its way
   for (;;) { // a block, or the part of it held here, at a time
     begin_block(at.b, asked);
 #pragma unroll
@@ -466,35 +502,48 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
       __syncthreads();
       more = nx.t < t1;
       const Place nn = next_of(nx);
-      unsigned char *buf = lds + cur * kBuf, *other = lds + (cur ^ 1) * kBuf;
+      const int next = TERMS ? (cur == 2 ? 0 : cur + 1) : cur ^ 1;
+      unsigned char *buf = buffer(cur);
+      if constexpr (TERMS) {
+        if (nn.t < t1) // into the buffer read in the step before
+          bring_terms(nn, next == 2 ? 0 : next + 1);
+      }
       auto stage = [&]() {
         if (!more)
           return;
         if (!arrived)
           bring_wait();
-        put_tile(other, scales[cur ^ 1]);
+        put_tile(buffer(next), scales_of(next));
         if (nn.t < t1)
           bring(nn);
       };
       // the two wavefronts of a SIMD in opposite order: one's conversion beside the other's
       // products
-      if (wave < 4)
+      if (!TERMS && wave < 4)
         stage();
       if (at.j * kKeys <= pos_last) {
         scores(buf);
         const int k0 = at.j * kKeys;
-        tile_weights(w, scales[cur], up, k0 + kKeys - 1 > pos_first, qpos - k0, rs, pf);
+        tile_weights(w, scales_of(cur), up, k0 + kKeys - 1 > pos_first, qpos - k0, rs, pf);
         add_values(buf + kHalf);
       }
-      if (wave >= 4)
+      if constexpr (TERMS) { // the next tile, behind which this step has asked for one more at most
+        if (nn.t >= t1)
+          landed<0>();
+        else if (wave == 0)
+          landed<5>();
+        else
+          landed<4>();
+      } else if (wave >= 4) {
         stage();
+      }
       arrived = false;
       ends = at.j + 1 == at.n;
       if (ends || !more)
         break;
       at = nx;
       nx = nn;
-      cur ^= 1;
+      cur = next;
     }
     if (more)
       ask_queries(nx, asked); // ahead of the stores, which a load behind them would wait for
@@ -503,7 +552,7 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
       break;
     at = nx;
     nx = next_of(nx);
-    cur ^= 1;
+    cur = TERMS ? (cur == 2 ? 0 : cur + 1) : cur ^ 1;
     // begin_block waits for the queries, which were asked for behind that tile, and not for the stores
     arrived = true;
   }
@@ -530,8 +579,9 @@ PromptShare share_out(int q_len, int q_offset, int heads, int kv_heads) {
     s.tiles += ceil_div(q_offset + last / group + 1, kKeys);
   }
   s.tiles *= kv_heads;
-  s.workgroups = (int)std::min<int64_t>(kPromptWorkgroups, s.tiles); // each at least a tile
+  // each at least a tile, and of few no more than the longest share asks for: partial results go with them
   s.ahead = s.tiles >= 4 * kPromptWorkgroups ? 2 : 0;
+  s.workgroups = s.ahead ? kPromptWorkgroups : (int)ceil_div(s.tiles, ceil_div(s.tiles, kPromptWorkgroups));
   s.units = s.tiles + s.ahead * (int64_t)s.nblk * kv_heads;
   return s;
 }
@@ -552,7 +602,13 @@ PromptShare share_out(int q_len, int q_offset, int heads, int kv_heads) {
 // More than 32 tokens behind 400 and more go this way in doubt, up to 6 us, and more than 640 up to
 // 2.5: it asks for each key once for all heads of a KV head, and what is not finite stays with the
 // rows that see it.
+// A prompt alone has attn_terms.hip as the other way, whose workgroups read every key of their 32 rows for
+// themselves: us a layer, that way and this one, 12 heads, 2 KV heads, 400 tokens 126 and 133, 800 195 and 206, 1000
+// 226 and 235, 1500 320 and 323, 1931 405 and 401; 32 and 8, 400 tokens 156 and 165, 600 202 and 210, 800 256 and
+// 252, 1000 301 and 291, 1931 570 and 532.  One line for both: 890 tokens, of more than 22 heads fewer.
 bool attn_prompt_pays(int q_len, int q_offset, int heads, int kv_heads, bool converts) {
+  if (q_offset == 0)
+    return q_len > 890 || (int64_t)q_len * heads > 20000;
   const double kilo_rows = 1e-4 * q_len * heads; // tens of thousands of (token, head)
   // attn_prefill.hip: blocks of 16 queries, one to a workgroup of eight wavefronts, then two, while
   // those fit the chip; steps of 16 keys per wavefront
@@ -588,7 +644,8 @@ size_t attn_prompt_workspace_bytes(int q_len, int k_len, int heads, int kv_heads
   return slots * kPromptRows * (kPromptD + 2) * sizeof(float) + (size_t)blocks * sizeof(PromptBlock);
 }
 
-int launch_attn_prompt(const AttnPrefillArgs &in, void *workspace, PromptFold &fold, hipStream_t stream) {
+int launch_attn_prompt(const AttnPrefillArgs &in, const PromptTerms &terms, void *workspace, PromptFold &fold,
+                       hipStream_t stream) {
   BH_REQUIRE(in.q && in.k && in.v && in.out && workspace && !in.mask, "attn_prompt: null pointer or mask");
   BH_REQUIRE(in.head_dim == kPromptD && in.kv_heads > 0 && in.heads % in.kv_heads == 0 && in.q_len > 0 &&
                  in.k_len >= in.q_len && in.kv_stride >= in.k_len,
@@ -629,10 +686,19 @@ int launch_attn_prompt(const AttnPrefillArgs &in, void *workspace, PromptFold &f
   a.share = (int)(share.units / share.workgroups);
   a.extra = (int)(share.units % share.workgroups);
   BH_NOTE_VARIANT(PromptFamily, kPromptRows);
-  static DynLdsOnce dyn_lds;
-  BH_CHECK_HIP(ensure_dyn_lds(dyn_lds, reinterpret_cast<const void *>(attn_prompt_kernel), kLds));
-  hipLaunchKernelGGL(attn_prompt_kernel, dim3((unsigned)share.workgroups), dim3(kThreads), kLds, stream, a.k, a.v,
-                     a.kv_stride, a.share, a.extra, a.per_head, a.nblk, a.group, a.q_len, a.k_len, a.q_offset, a);
+  a.terms = terms.tiles;
+  a.terms_per_head = terms.per_head;
+  BH_REQUIRE(!terms.tiles || (a.q_offset == 0 && ceil_div(in.k_len, kKeys) <= terms.per_head),
+             "attn_prompt: %d tiles of terms for %d keys", terms.per_head, in.k_len);
+  static DynLdsOnce dyn_lds[2];
+  auto launch = [&](auto kernel, bool on_terms) -> int {
+    BH_CHECK_HIP(ensure_dyn_lds(dyn_lds[on_terms], reinterpret_cast<const void *>(kernel), lds_bytes(on_terms)));
+    hipLaunchKernelGGL(kernel, dim3((unsigned)share.workgroups), dim3(kThreads), lds_bytes(on_terms), stream, a.k, a.v,
+                       a.kv_stride, a.share, a.extra, a.per_head, a.nblk, a.group, a.q_len, a.k_len, a.q_offset, a);
+    return BUDDY_HIP_OK;
+  };
+  if (int rc = terms.tiles ? launch(attn_prompt_kernel<true>, true) : launch(attn_prompt_kernel<false>, false))
+    return rc;
   BH_CHECK_HIP(hipGetLastError());
   fold.out = in.out;
   fold.acc = a.acc;

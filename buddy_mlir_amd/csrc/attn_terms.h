@@ -26,7 +26,7 @@ struct TileScales {
 constexpr int kTermTile = 4 * kTermBytes + 512; // (PromptTerms has them)
 static_assert(sizeof(TileScales) <= 512, "a tile's scales");
 inline size_t attn_terms_bytes(int kv_heads, int max_len) {
-  return (size_t)kv_heads * ceil_div(max_len, kTileKeys) * kTermTile;
+  return (size_t)kv_heads * ceil_div(max_len, kTileKeys) * kTermTile + 512; // scales are read by whole KiB
 }
 // Attention of a session's prompt tokens ahead of which there is nothing, on terms that the rotation of its
 // q | k | v left (finished rows in a.out); up to kTermsMostKeys tokens.
@@ -161,34 +161,39 @@ __device__ __forceinline__ void put_key_terms(const PromptTerms &t, int kvh, int
       *reinterpret_cast<uint2 *>(at + p * kTermBytes) = h ? uint2{term[p].z, term[p].w} : uint2{term[p].x, term[p].y};
   }
 }
-__device__ __forceinline__ void put_value_terms(const PromptTerms &t, int kvh, int pos, int i, const float (&lo)[4],
-                                                const float (&hi)[4]) {
+// Where channel c of key `key` is among term p of a tile's values: key 16 s + 8 x + 4 half + r is value r + 4 x of
+// the eight that lane 32 half + channel has in step s.
+__device__ __forceinline__ unsigned char *value_term_at(unsigned char *tile, int key, int c, int p) {
+  return tile + (2 + p) * kTermBytes + (c / 32 * 2 + key / 16) * 1024 + (key / 4 % 2 * 32 + c % 32) * 16 +
+         (key / 8 % 2 * 4 + key % 4) * 2;
+}
+// the scales of a value's row to its tile, its terms to the caller
+__device__ __forceinline__ void value_terms(const PromptTerms &t, int kvh, int pos, int i, const float (&lo)[4],
+                                            const float (&hi)[4], uint4 (&term)[2]) {
   float x[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}, log2_of;
   const unsigned e = value_scale(x, log2_of, [](int) {});
-  unsigned char *tile = terms_tile(t, kvh, pos);
-  const int key = pos % kTileKeys;
   if (i == 0) {
-    TileScales *sc = reinterpret_cast<TileScales *>(tile + 4 * kTermBytes);
-    sc->value[key] = log2_of;
-    sc->undo[key] = pow2(e);
+    TileScales *sc = reinterpret_cast<TileScales *>(terms_tile(t, kvh, pos) + 4 * kTermBytes);
+    sc->value[pos % kTileKeys] = log2_of;
+    sc->undo[pos % kTileKeys] = pow2(e);
   }
 #pragma unroll
   for (int j = 0; j < 8; ++j)
     x[j] *= pow2(e);
-  uint4 term[2];
   split8(x, term);
-  // key 16 s + 8 x8 + 4 half + r: value r + 4 x8 of the eight that lane 32 half + channel has in step s
-  const int s = key / 16, half = key / 4 % 2, at_key = (key / 8 % 2 * 4 + key % 4) * 2;
+}
+__device__ __forceinline__ void put_value_terms(const PromptTerms &t, int kvh, int pos, int i, const float (&lo)[4],
+                                                const float (&hi)[4]) {
+  uint4 term[2];
+  value_terms(t, kvh, pos, i, lo, hi, term);
+  unsigned char *tile = terms_tile(t, kvh, pos);
 #pragma unroll
   for (int p = 0; p < 2; ++p) {
     const unsigned w[4] = {term[p].x, term[p].y, term[p].z, term[p].w};
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int c = 64 * (j / 4) + 4 * i + j % 4;
-      *reinterpret_cast<unsigned short *>(tile + 2 * kTermBytes + p * kTermBytes + (c / 32 * 2 + s) * 1024 +
-                                          (half * 32 + c % 32) * 16 + at_key) =
+    for (int j = 0; j < 8; ++j)
+      *reinterpret_cast<unsigned short *>(value_term_at(tile, pos % kTileKeys, 64 * (j / 4) + 4 * i + j % 4, p)) =
           (unsigned short)(j & 1 ? w[j / 2] >> 16 : w[j / 2]);
-    }
   }
 }
 

@@ -113,7 +113,7 @@ struct SiluMulRow { // silu(g) * u
   }
 };
 
-struct FoldedRow { // the attention's output at one token, added up from its parts
+template <int kMost> struct FoldedRow { // the attention's output at one token, added up from its parts
   static constexpr bool kRepairs = true;
   const PromptFold &f;
   int64_t o_stride;
@@ -121,7 +121,7 @@ struct FoldedRow { // the attention's output at one token, added up from its par
   __device__ __forceinline__ void operator()(int k0, float (&v)[4]) const {
     v[0] = v[1] = v[2] = v[3] = 0.f;
     if (k0 < n)
-      left4(f, o_stride, t, k0 / kPromptD, k0 % kPromptD, v);
+      left4<kMost>(f, o_stride, t, k0 / kPromptD, k0 % kPromptD, v);
   }
   __device__ __forceinline__ void repair(int k0, float (&v)[4]) const {
     if (k0 < n)
@@ -241,7 +241,8 @@ activations_to_digits_kernel(const float *__restrict__ A, int64_t lda, int M, in
                 row_cache);
 }
 
-__global__ void __launch_bounds__(kRowThreads)
+template <int kMost>
+__global__ void __launch_bounds__(kRowThreads, kMost == 4 ? 8 : 1)
 attn_fold_to_digits_kernel(PromptFold f, int64_t o_stride, int M, int K, int D, int Mp, int Kp,
                            int8_t *__restrict__ planes) {
   __shared__ float red[kRowThreads / 64];
@@ -251,7 +252,7 @@ attn_fold_to_digits_kernel(PromptFold f, int64_t o_stride, int M, int K, int D, 
     padding_to_digits(row, D, Mp, Kp, planes);
     return;
   }
-  row_to_digits(FoldedRow{f, o_stride, row, K}, K, row, D, Mp, Kp, planes, red, row_cache);
+  row_to_digits(FoldedRow<kMost>{f, o_stride, row, K}, K, row, D, Mp, Kp, planes, red, row_cache);
 }
 
 __global__ void __launch_bounds__(kRowThreads)
@@ -1384,7 +1385,8 @@ int launch_attn_fold_to_digits(const PromptFold &fold, int64_t o_stride, int hea
   BH_REQUIRE(fold.blocks && staged && tokens > 0 && (digits == 2 || digits == 3),
              "attn_fold_to_digits: bad argument");
   const GemmStagingLayout l = gemm_staging_layout(tokens, K);
-  hipLaunchKernelGGL(attn_fold_to_digits_kernel, dim3((unsigned)l.rows_padded), dim3(kRowThreads),
+  hipLaunchKernelGGL(tokens > kFoldTokens ? attn_fold_to_digits_kernel<4> : attn_fold_to_digits_kernel<16>,
+                     dim3((unsigned)l.rows_padded), dim3(kRowThreads),
                      row_cache_bytes(l.cols_padded), stream, fold, o_stride, tokens, (int)K, digits,
                      l.rows_padded, l.cols_padded, static_cast<int8_t *>(staged));
   BH_CHECK_HIP(hipGetLastError());

@@ -491,9 +491,9 @@ struct Qwen2Session : Session {
     const bool folded = attn_prompt_pays(n, start_pos, S.heads, S.kv_heads, converts);
     if (folded && !pf_attn_ws) // for as many rows as the other buffers have, behind any context
       BH_CHECK_HIP(hipMalloc(&pf_attn_ws, attn_prompt_workspace_bytes(pf_rows, S.max_len, S.heads, S.kv_heads)));
-    // a prompt alone that is not shared out: its attention reads terms that the rotation leaves
+    // a prompt alone: its attention reads terms that the rotation leaves
     PromptTerms terms;
-    if (!folded && start_pos == 0 && n <= kTermsMostKeys) {
+    if (start_pos == 0 && (folded || n <= kTermsMostKeys)) {
       terms.tiles = pf_terms;
       terms.per_head = (int)ceil_div(pf_rows, kTileKeys);
     }
@@ -549,7 +549,7 @@ struct Qwen2Session : Session {
       a.k_len = start_pos + n;
       a.scale = scale;
       PromptFold fold;
-      if ((rc = folded          ? launch_attn_prompt(a, pf_attn_ws, fold, stream)
+      if ((rc = folded        ? launch_attn_prompt(a, terms, pf_attn_ws, fold, stream)
                 : terms.tiles ? launch_attn_terms(a, terms, stream)
                               : launch_attn_prefill(a, stream)))
         return rc;
