@@ -278,7 +278,7 @@ __device__ __forceinline__ float exp2_f(float x) { return __builtin_amdgcn_exp2f
 struct ChunkParts {
   int dp, v16;                     // dim32, vdim16
   int w, q, kt, b, ut, last, size; // W, G q: [64][dim32]; (G_last / G k)^T: [dim32][64]; b: [64][64];
-                                   // U^T, later u^T: [vdim16][64]; G_last: [dim32]
+                                   // U^T, later u^T: [vdim16][64]; all of these as tile_at has them; G_last: [dim32]
 };
 ChunkParts chunk_parts(const DeltaShape &s) {
   const int d = kC * s.dim32();
@@ -293,6 +293,18 @@ ChunkParts chunk_parts(const DeltaShape &s) {
   p.last = p.ut + kC * s.vdim16();
   p.size = p.last + s.dim32();
   return p;
+}
+// Element k of a row of n in tiles of 16 rows x 32 k, as a wavefront reads them for mfma32: four k side by
+// side, those of the 16 rows beside them, then the next eight k's, and the second four of each eight behind them.  (By
+// rows a load is pieces of 16 of them.)
+__device__ __forceinline__ int tile_at(int row, int k, int n) {
+  return (row / 16 * (n / 32) + k / 32) * 512 + k / 4 % 2 * 256 + (k / 8 % 4 * 16 + row % 16) * 4 + k % 4;
+}
+// this lane's operand out of the tile of rows 16 i .. and k 32 t ..
+__device__ __forceinline__ void load_tile(Frag<float> &f, const float *p, int i, int t, int n) {
+  p += (i * (n / 32) + t) * 512 + (threadIdx.x & 63) * 4;
+  f.lo = *reinterpret_cast<const f32x4 *>(p);
+  f.hi = *reinterpret_cast<const f32x4 *>(p + 256);
 }
 
 struct DeltaPrepArgs {
@@ -561,8 +573,8 @@ __global__ void __launch_bounds__(kChunkThreads) delta_chunk_kernel(DeltaChunkAr
     for (int r = 0; r < 4; ++r) {
       const int t = bi * kBlock + quad * 4 + r, x = bj * kBlock + col;
       as[t * kARow + x] = sa[r] * beta[t];
-      out[a.at.b + t * kC + x] = sb[r];
-      out[a.at.b + x * kC + t] = 0.f;
+      out[a.at.b + tile_at(t, x, kC)] = sb[r];
+      out[a.at.b + tile_at(x, t, kC)] = 0.f;
     }
   }
   // pairs within a block: a lane each, 120 of them on two wavefronts
@@ -588,13 +600,13 @@ __global__ void __launch_bounds__(kChunkThreads) delta_chunk_kernel(DeltaChunkAr
       }
       const int ta = b * kBlock + t, xa = b * kBlock + x;
       as[ta * kARow + xa] = sa * beta[ta];
-      out[a.at.b + ta * kC + xa] = sb;
-      out[a.at.b + xa * kC + ta] = 0.f;
+      out[a.at.b + tile_at(ta, xa, kC)] = sb;
+      out[a.at.b + tile_at(xa, ta, kC)] = 0.f;
     } else {
       // the block's own tokens, four per wavefront at a time
       for (int t = (wave & 1) * 8 + lane - 60; t < (wave & 1) * 8 + 8; t += 4) {
         const int r = b * kBlock + t;
-        out[a.at.b + r * kC + r] = r < rows ? a.dots[(int64_t)(r0 + r) * s.kv_heads + g] : 0.f;
+        out[a.at.b + tile_at(r, r, kC)] = r < rows ? a.dots[(int64_t)(r0 + r) * s.kv_heads + g] : 0.f;
       }
     }
   }
@@ -630,7 +642,7 @@ __global__ void __launch_bounds__(kChunkThreads) delta_chunk_kernel(DeltaChunkAr
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         q[j] *= exp2_f(l[j]);
-      *reinterpret_cast<f32x4 *>(out + a.at.q + t * dp + d) = q;
+      *reinterpret_cast<f32x4 *>(out + a.at.q + tile_at(t, d, dp)) = q;
     }
     for (int i = id; i < kC * cols; i += n) {
       const int t = i % kC, d = i / kC * 4, b = t / kBlock;
@@ -640,7 +652,7 @@ __global__ void __launch_bounds__(kChunkThreads) delta_chunk_kernel(DeltaChunkAr
       const f32x4 k = *reinterpret_cast<const f32x4 *>(ks + t * row_at + d);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        out[a.at.kt + (d + j) * kC + t] = k[j] * exp2_f(l[j]);
+        out[a.at.kt + tile_at(d + j, t, kC)] = k[j] * exp2_f(l[j]);
     }
     for (int d = id; d < dp; d += n)
       out[a.at.last + d] = exp2_f((tot[d] + tot[dp + d]) + (tot[2 * dp + d] + tot[3 * dp + d]));
@@ -699,9 +711,9 @@ __global__ void __launch_bounds__(kChunkThreads) delta_chunk_kernel(DeltaChunkAr
       if (i < dp) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          out[a.at.w + (t + r) * dp + i] = x[b][r];
+          out[a.at.w + tile_at(t + r, i, dp)] = x[b][r];
       } else {
-        *reinterpret_cast<f32x4 *>(out + a.at.ut + v * kC + t) = x[b];
+        *reinterpret_cast<f32x4 *>(out + a.at.ut + tile_at(v, t, kC)) = x[b];
       }
     }
   }
@@ -709,15 +721,19 @@ __global__ void __launch_bounds__(kChunkThreads) delta_chunk_kernel(DeltaChunkAr
 
 struct DeltaCarryArgs {
   int heads, dim, vdim, rows, chunks;
-  const float *parts;
+  float *parts;
   ChunkParts at;
-  float *state, *out; // out: [rows][heads * vdim]
+  float *state, *states, *out; // states: [chunks][heads][vdim16][dim32]; out: [rows][heads * vdim]
 };
 
-// Grid (heads, value slices of 16): the state from chunk to chunk, and the outputs.  A
-// wavefront takes 16 tokens of a chunk (products with the state) and every fourth tile
+// Grid (heads, value slices of 16): the state from chunk to chunk.  A
+// wavefront takes 16 tokens of a chunk (the product with the state) and every fourth tile
 // of 16 key channels (the state itself, in registers).  ND: 32-channel steps, at most.
 // What the chunk after this one needs is on its way meanwhile.
+//
+// What bounds it: the chain of two products and two barriers a chunk, 2.2 us; what only the outputs need is left
+// to delta_out_kernel, which has all chunks at once (777 tokens, 12 heads of 128: 69 us with them and operands
+// read by rows, 31 and 12 behind it).
 template <int ND>
 __global__ void __launch_bounds__(256, 1) delta_carry_kernel(DeltaCarryArgs a) {
   constexpr int dp_max = ND * 32, kTiles = (2 * ND + 3) / 4; // state tiles per wavefront
@@ -737,29 +753,24 @@ __global__ void __launch_bounds__(256, 1) delta_carry_kernel(DeltaCarryArgs a) {
       own[i][r] = d < a.dim && v < a.vdim ? S[(int64_t)d * a.vdim + v] : 0.f;
     }
   struct Chunk {
-    Frag<float> w[ND], q[ND], b[2], k[kTiles][2];
+    Frag<float> w[ND], k[kTiles][2];
     f32x4 u, last[kTiles];
   };
+  const int u_at = a.at.ut + tile_at(v, wave * 16 + quad * 4, kC);
+  auto parts_of = [&](int c) { return a.parts + ((int64_t)c * a.heads + h) * a.at.size; };
   auto fetch = [&](int c, Chunk &x) {
-    const float *p = a.parts + ((int64_t)min(c, a.chunks - 1) * a.heads + h) * a.at.size;
-    const float *row = p + (int64_t)(wave * 16 + col) * dp + quad * 8;
+    const float *p = parts_of(min(c, a.chunks - 1));
 #pragma unroll
-    for (int t = 0; t < ND; ++t) {
-      const int d = min(t, nd - 1) * 32;
-      x.w[t].load(row + a.at.w + d);
-      x.q[t].load(row + a.at.q + d);
-    }
-    x.u = *reinterpret_cast<const f32x4 *>(p + a.at.ut + (int64_t)(v0 + col) * kC + wave * 16 + quad * 4);
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-      x.b[t].load(p + a.at.b + (wave * 16 + col) * kC + t * 32 + quad * 8);
+    for (int t = 0; t < ND; ++t)
+      load_tile(x.w[t], p + a.at.w, wave, min(t, nd - 1), dp);
+    x.u = *reinterpret_cast<const f32x4 *>(p + u_at);
 #pragma unroll
     for (int i = 0; i < kTiles; ++i) {
-      const int d0 = min((wave + i * 4) * 16, dp - 16);
+      const int tile = min(wave + i * 4, dp / 16 - 1);
 #pragma unroll
       for (int t = 0; t < 2; ++t)
-        x.k[i][t].load(p + a.at.kt + (int64_t)(d0 + col) * kC + t * 32 + quad * 8);
-      x.last[i] = *reinterpret_cast<const f32x4 *>(p + a.at.last + d0 + quad * 4);
+        load_tile(x.k[i][t], p + a.at.kt, tile, t, kC);
+      x.last[i] = *reinterpret_cast<const f32x4 *>(p + a.at.last + tile * 16 + quad * 4);
     }
   };
   Chunk cur;
@@ -767,22 +778,27 @@ __global__ void __launch_bounds__(256, 1) delta_carry_kernel(DeltaCarryArgs a) {
   for (int c = 0; c < a.chunks; ++c) {
     Chunk next;
     fetch(c + 1, next);
+    float *kept = a.states + ((int64_t)c * a.heads + h) * a.at.v16 * dp;
 #pragma unroll
-    for (int i = 0; i < kTiles; ++i)
-      if ((wave + i * 4) * 16 < dp)
-        *reinterpret_cast<f32x4 *>(st + col * kSRow + (wave + i * 4) * 16 + quad * 4) = own[i];
+    for (int i = 0; i < kTiles; ++i) {
+      const int d = (wave + i * 4) * 16 + quad * 4;
+      if ((wave + i * 4) * 16 < dp) {
+        *reinterpret_cast<f32x4 *>(st + col * kSRow + d) = own[i];
+        *reinterpret_cast<f32x4 *>(kept + tile_at(v, d, dp)) = own[i];
+      }
+    }
     __syncthreads();
-    f32x4 ws{0.f, 0.f, 0.f, 0.f}, o = ws;
+    f32x4 ws{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < ND; ++t)
       if (t < nd) {
         Frag<float> sf;
         sf.load(st + col * kSRow + t * 32 + quad * 8);
         ws = mfma32(cur.w[t], sf, ws);
-        o = mfma32(cur.q[t], sf, o);
       }
     const f32x4 u = cur.u - ws;
     *reinterpret_cast<f32x4 *>(ut + col * kURow + wave * 16 + quad * 4) = u;
+    *reinterpret_cast<f32x4 *>(parts_of(c) + u_at) = u;
     __syncthreads();
     Frag<float> uf[2];
 #pragma unroll
@@ -796,16 +812,6 @@ __global__ void __launch_bounds__(256, 1) delta_carry_kernel(DeltaCarryArgs a) {
         n = mfma32(cur.k[i][t], uf[t], n);
       own[i] = n;
     }
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-      if (t * 32 <= wave * 16 + 15)
-        o = mfma32(cur.b[t], uf[t], o);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = c * kC + wave * 16 + quad * 4 + r;
-      if (row < a.rows && v < a.vdim)
-        a.out[((int64_t)row * a.heads + h) * a.vdim + v] = o[r];
-    }
     cur = next;
   }
 #pragma unroll
@@ -816,6 +822,44 @@ __global__ void __launch_bounds__(256, 1) delta_carry_kernel(DeltaCarryArgs a) {
       if (d < a.dim && v < a.vdim)
         S[(int64_t)d * a.vdim + v] = own[i][r];
     }
+}
+
+// Grid (chunks, heads, value slices of 16): the outputs of a chunk from the state ahead of it and its writes.  A
+// wavefront takes 16 tokens.
+template <int ND>
+__global__ void __launch_bounds__(256) delta_out_kernel(DeltaCarryArgs a) {
+  const int lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int c = blockIdx.x, h = blockIdx.y, slice = blockIdx.z, v = slice * 16 + col;
+  const int dp = (a.dim + 31) & ~31, nd = dp / 32;
+  const int64_t at = (int64_t)c * a.heads + h;
+  const float *p = a.parts + at * a.at.size, *kept = a.states + at * a.at.v16 * dp;
+  Frag<float> q[ND], s[ND], b[2], u[2];
+#pragma unroll
+  for (int t = 0; t < ND; ++t) {
+    load_tile(q[t], p + a.at.q, wave, min(t, nd - 1), dp);
+    load_tile(s[t], kept, slice, min(t, nd - 1), dp);
+  }
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    load_tile(b[t], p + a.at.b, wave, t, kC);
+    load_tile(u[t], p + a.at.ut, slice, t, kC);
+  }
+  f32x4 o{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int t = 0; t < ND; ++t)
+    if (t < nd)
+      o = mfma32(q[t], s[t], o);
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+    if (t * 32 <= wave * 16 + 15)
+      o = mfma32(b[t], u[t], o);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int row = c * kC + wave * 16 + quad * 4 + r;
+    if (row < a.rows && v < a.vdim)
+      a.out[((int64_t)row * a.heads + h) * a.vdim + v] = o[r];
+  }
 }
 
 struct DeltaGateArgs {
@@ -849,7 +893,7 @@ size_t chunk_lds(const DeltaShape &s) {
   return sizeof(float) * ((size_t)3 * kC * (s.dim32() + 4) + (size_t)kC * (kC + 4) + kBlocks * s.dim32() + kC + kC * (kBlock + 4));
 }
 struct Workspace {
-  size_t conv, dots, decay, gate, out, parts, size; // offsets in floats
+  size_t conv, dots, decay, gate, out, parts, states, size; // offsets in floats
 };
 Workspace workspace(const DeltaShape &s, int rows) {
   Workspace w;
@@ -866,6 +910,7 @@ Workspace workspace(const DeltaShape &s, int rows) {
   w.gate = take(n * s.gate.N);
   w.out = take(n * s.heads * s.vdim);
   w.parts = take((size_t)ceil_div(rows, kC) * s.heads * chunk_parts(s).size);
+  w.states = take((size_t)ceil_div(rows, kC) * s.heads * s.vdim16() * s.dim32());
   w.size = at;
   return w;
 }
@@ -966,17 +1011,22 @@ int launch_delta_chunks(const DeltaRows &a, float *ws, hipStream_t stream) {
   hipLaunchKernelGGL(delta_chunk_kernel, dim3((unsigned)chunks, (unsigned)s.heads), dim3(kChunkThreads),
                      chunk_lds(s), stream, c);
   BH_CHECK_HIP(hipGetLastError());
-  DeltaCarryArgs k{s.heads, s.dim, s.vdim, a.rows, chunks, ws + w.parts, chunk_parts(s), a.state, ws + w.out};
-  const dim3 grid((unsigned)s.heads, (unsigned)(s.vdim16() / 16));
+  DeltaCarryArgs k{s.heads, s.dim, s.vdim, a.rows, chunks, ws + w.parts, chunk_parts(s), a.state, ws + w.states,
+                   ws + w.out};
+  const unsigned slices = (unsigned)(s.vdim16() / 16);
+  auto launch = [&](auto carry, auto outputs) {
+    hipLaunchKernelGGL(carry, dim3((unsigned)s.heads, slices), dim3(256), 0, stream, k);
+    hipLaunchKernelGGL(outputs, dim3((unsigned)chunks, (unsigned)s.heads, slices), dim3(256), 0, stream, k);
+  };
   const int nd = s.dim32() / 32;
   if (nd <= 1)
-    hipLaunchKernelGGL(delta_carry_kernel<1>, grid, dim3(256), 0, stream, k);
+    launch(delta_carry_kernel<1>, delta_out_kernel<1>);
   else if (nd <= 2)
-    hipLaunchKernelGGL(delta_carry_kernel<2>, grid, dim3(256), 0, stream, k);
+    launch(delta_carry_kernel<2>, delta_out_kernel<2>);
   else if (nd <= 4)
-    hipLaunchKernelGGL(delta_carry_kernel<4>, grid, dim3(256), 0, stream, k);
+    launch(delta_carry_kernel<4>, delta_out_kernel<4>);
   else
-    hipLaunchKernelGGL(delta_carry_kernel<8>, grid, dim3(256), 0, stream, k);
+    launch(delta_carry_kernel<8>, delta_out_kernel<8>);
   BH_CHECK_HIP(hipGetLastError());
   return launch_delta_gate(s, ws + w.out, ws + w.gate, s.gate.N, a.rows, a.out, a.out_ld, a.act_f32, stream);
 }
