@@ -734,7 +734,8 @@ rows_gemm_wide_kernel(const uint4 *W, int ktiles, int steps, int columns, int ro
         if constexpr (OUT == kOutExpertAct) {
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            v[i] = gated_act(a.act, v[i], acc[g + kTilesOut][r][4 * j + i], a.limit);
+            v[i] = sizeof(T) == 2 ? gated_act_bf16(a.act, v[i], acc[g + kTilesOut][r][4 * j + i], a.limit)
+                                  : gated_act(a.act, v[i], acc[g + kTilesOut][r][4 * j + i], a.limit);
           store4<T>(static_cast<T *>(a.C) + (int64_t)orow * a.ldc + ch, v);
         } else if constexpr (OUT == kOutF32) {
 #pragma unroll
