@@ -421,7 +421,8 @@ rope_kv_write_kernel(float *qkv, int64_t row_stride, int n_tokens, RopeKv r) {
       const bool value = which & 1;
       if (h >= r.kv_heads)
         continue;
-      load(qkv + (int64_t)min(t, n_tokens - 1) * row_stride + (int64_t)(r.heads + (value ? r.kv_heads : 0) + h) * kD + j,
+      load(qkv + (int64_t)min(t, n_tokens - 1) * row_stride +
+               (int64_t)(r.heads + (value ? r.kv_heads : 0) + h) * kD + j,
            lo, hi);
       const int64_t at = ((int64_t)h * r.max_len + pos) * kD + j;
       if (!value) {
@@ -545,7 +546,8 @@ int launch_rope_kv_write(float *qkv, int64_t row_stride, const RopeKv &r, int n_
                    reinterpret_cast<uintptr_t>(r.vcache)) & 15) == 0,
              "rope_kv_write: rows must be 16-byte aligned");
   BH_REQUIRE(!r.terms.tiles || r.start_pos % kRopeTokens == 0, "rope_kv_write: terms from position %d on", r.start_pos);
-  hipLaunchKernelGGL(rope_kv_write_kernel, dim3((unsigned)(ceil_div(n_tokens, kRopeTokens) + n_tokens)), dim3(256), 0, stream, qkv,
+  hipLaunchKernelGGL(rope_kv_write_kernel, dim3((unsigned)(ceil_div(n_tokens, kRopeTokens) + n_tokens)),
+                     dim3(256), 0, stream, qkv,
                      row_stride, n_tokens, r);
   BH_CHECK_HIP(hipGetLastError());
   return BUDDY_HIP_OK;

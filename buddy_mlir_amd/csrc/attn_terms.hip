@@ -8,8 +8,8 @@
 // finished rows.
 //
 // What bounds it: a launch, a trip to memory for the queries and first keys, one or two tiles to a wavefront (some
-// 1500 cycles of matrix and 900 of vector instructions each, two wavefronts to a SIMD), and the meeting.  12 query heads,
-// 2 KV heads, us against attn_prefill.hip's f32 instructions on rows as they lie: 27 tokens 6.7 and 7.6, 512
+// 1500 cycles of matrix and 900 of vector instructions each, two wavefronts to a SIMD), and the meeting.  12 query
+// heads, 2 KV heads, us against attn_prefill.hip's f32 instructions on rows as they lie: 27 tokens 6.7 and 7.6, 512
 // 12.6 and 23.3; the rotation's launch, which writes the terms, 5.6 and 5.4, 6.1 and 5.3.
 #include "attn.h"
 #include "attn_terms.h"
@@ -56,7 +56,8 @@ attn_terms_kernel(const unsigned char *tiles, const float *q, int64_t q_stride, 
     const uintptr_t u = reinterpret_cast<uintptr_t>(p);
     const uintptr_t base = (uintptr_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)u) |
                            (uintptr_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(u >> 32)) << 32;
-    return *(const __attribute__((address_space(1))) u32x4 *)((const __attribute__((address_space(1))) char *)base + at);
+    const auto *from = (const __attribute__((address_space(1))) char *)base + at;
+    return *(const __attribute__((address_space(1))) u32x4 *)from;
   };
   u32x4 kf[8][2];
   auto ask_keys = [&](int t, int half) {

@@ -315,7 +315,9 @@ rows_gemm_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int columns
 // the power allows: the clock falls with what the matrix cores draw.  A round of 24 steps is
 // 43 us of that and 15 of its beginning and its activation and stores.  With the rows through
 // registers, one such tile to a compute unit and its loads between its products: gate | up of 16
-// experts, 2048 x 4 rows of 1536 -> 2 x 1792, 148 us, now 120; 777 x 1536 -> 2 x 8960 68, now 58.
+// experts, 2048 x 4 rows of 1536 -> 2 x 1792, 148 us, with rows by DMA 120; 777 x 1536 -> 2 x 8960
+// 68 and 58.  With the activation and the stores in cheaper forms (gated_act_bf16, the turn below)
+// 109 and 53.
 // (Rows past the registers for the tiles of 32 and 64 rows too: 8960 -> 1536 at 777 rows 47 us
 // whole, 56 so; 1536 -> 1536 of 400 rows 8.1 and 8.5.)  Against 16 x 16 tiles (us, rows x K x channels):
 //   bfloat16  2048 x 4096 x 4096   82.0 -> 75.2    f32   523 -> 216
@@ -383,7 +385,14 @@ rows_gemm_wide_kernel(const uint4 *W, int ktiles, int steps, int columns, int ro
   constexpr int kPlane = kRows * kLdsRow, kBuf = kTerms * kPlane;
   static_assert(kRows * kRowRuns % kGemmThreads == 0, "every thread moves the same number of runs");
   constexpr int kBrought = kRows * kRowBytes; // of a step's rows, where they come past the registers
-  __shared__ __attribute__((aligned(16))) unsigned char lds[kBrings<T, RT> ? 4 * kBrought : 3 * kBuf];
+  // the way out: 32 rows of a wavefront's channels at a time are turned in LDS, so that a store writes whole row
+  // segments (as the registers lie, pieces of 8 or 16 bytes of 32 rows: 777 x 1536 -> 2 x 8960 55.4 us and so 53.1,
+  // experts' gate | up 114 and 109, their down 77 and 69)
+  constexpr bool kTurns = OUT != kOutActTrans;
+  constexpr int kOutSize = OUT == kOutF32 ? 4 : (int)sizeof(T);
+  constexpr int kSegment = 32 * kTilesOut * kOutSize, kTurnRow = kSegment + 16;
+  constexpr int kTurn = kTurns ? 4 * 32 * kTurnRow : 0, kStage = kBrings<T, RT> ? 4 * kBrought : 3 * kBuf;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[kStage > kTurn ? kStage : kTurn];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
@@ -679,13 +688,12 @@ rows_gemm_wide_kernel(const uint4 *W, int ktiles, int steps, int columns, int ro
       step(s + 2, wr[2], wr[1], xr[0], xr[3]);
   }
 
+  __syncthreads(); // LDS is free
   // a lane holds channels 8 j + (lane / 32) * 4 + 0..3, j = 0..3, of row lane % 32 of every tile
 #pragma unroll
   for (int r = 0; r < RT; ++r) {
     const int lr = row0 + r * 32 + (lane & 31);
-    if (lr >= rows)
-      continue;
-    if constexpr (kTerms > 1) {
+    if (kTerms > 1 && lr < rows) {
       // An infinite weight times a term that is zero is NaN where the f32 product is
       // infinite: what came out as NaN is added up again without terms.
       float most = acc[0][r][0]; // NaN if one of them is
@@ -709,7 +717,8 @@ rows_gemm_wide_kernel(const uint4 *W, int ktiles, int steps, int columns, int ro
           const int group = ch0 + 2 * (kPair ? tile % kTilesOut : tile) + of / 16;
           if (v == v || group >= a.groups)
             continue;
-          const uint4 *w = W + ((int64_t)((kPair ? tile / kTilesOut : 0) * a.groups + group) * ktiles + first * 2) * 64 + of % 16;
+          const int64_t w_at = (int64_t)((kPair ? tile / kTilesOut : 0) * a.groups + group) * ktiles + first * 2;
+          const uint4 *w = W + w_at * 64 + of % 16;
           v = f32_sum(x, w, SLICED ? min(K, steps * kWideK) : K);
 #pragma unroll
           for (int i = 0; i < GT * 16; ++i)
@@ -717,40 +726,57 @@ rows_gemm_wide_kernel(const uint4 *W, int ktiles, int steps, int columns, int ro
         }
       }
     }
-    int orow = lr;
-    if constexpr (GROUPED)
-      orow = list[lr];
+    if constexpr (kTurns) {
+      unsigned char *turn = lds + wave * (32 * kTurnRow);
 #pragma unroll
-    for (int g = 0; g < kTilesOut; ++g) {
+      for (int g = 0; g < kTilesOut; ++g)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int ch = (ch0 + 2 * g) * 16 + 8 * j + (lane >> 5) * 4;
-        if (ch >= a.groups * 16)
-          continue;
-        f32x4 v;
+        for (int j = 0; j < 4; ++j) {
+          const int ch = 32 * g + 8 * j + (lane >> 5) * 4;
+          f32x4 v;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          v[i] = acc[g][r][4 * j + i];
-        if constexpr (OUT == kOutExpertAct) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            v[i] = sizeof(T) == 2 ? gated_act_bf16(a.act, v[i], acc[g + kTilesOut][r][4 * j + i], a.limit)
-                                  : gated_act(a.act, v[i], acc[g + kTilesOut][r][4 * j + i], a.limit);
-          store4<T>(static_cast<T *>(a.C) + (int64_t)orow * a.ldc + ch, v);
-        } else if constexpr (OUT == kOutF32) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (ch + i < a.silu_channels)
-              v[i] = silu_f(v[i]);
-          store4<float>(static_cast<float *>(a.C) + (int64_t)orow * a.ldc + ch, v);
-        } else if constexpr (OUT == kOutAct) {
-          store4<T>(static_cast<T *>(a.C) + (int64_t)orow * a.ldc + ch, v);
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            store_act<T>(static_cast<T *>(a.C) + (int64_t)(ch + i) * a.ldc + orow, v[i]);
+          for (int i = 0; i < 4; ++i) {
+            v[i] = acc[g][r][4 * j + i];
+            if constexpr (OUT == kOutExpertAct) {
+              const float up = acc[g + kTilesOut][r][4 * j + i];
+              v[i] = sizeof(T) == 2 ? gated_act_bf16(a.act, v[i], up, a.limit) : gated_act(a.act, v[i], up, a.limit);
+            } else if constexpr (OUT == kOutF32) {
+              if (ch0 * 16 + ch + i < a.silu_channels)
+                v[i] = silu_f(v[i]);
+            }
+          }
+          unsigned char *to = turn + (lane & 31) * kTurnRow + ch * kOutSize;
+          if constexpr (kOutSize == 4)
+            *reinterpret_cast<f32x4 *>(to) = v;
+          else
+            *reinterpret_cast<uint2 *>(to) = uint2{pack_bf(v[0], v[1]), pack_bf(v[2], v[3])};
         }
+      constexpr int kPieces = kSegment / 16; // of a row
+#pragma unroll
+      for (int i = 0; i < kPieces / 2; ++i) {
+        const int id = i * 64 + lane, row = id / kPieces, ch = id % kPieces * (16 / kOutSize);
+        const int out = row0 + r * 32 + row;
+        const uint4 x = *reinterpret_cast<const uint4 *>(turn + row * kTurnRow + ch * kOutSize);
+        if (out >= rows || ch0 * 16 + ch >= a.groups * 16)
+          continue;
+        int orow = out;
+        if constexpr (GROUPED)
+          orow = list[out];
+        unsigned char *to = static_cast<unsigned char *>(a.C) + ((int64_t)orow * a.ldc + ch0 * 16 + ch) * kOutSize;
+        *reinterpret_cast<uint4 *>(to) = x;
       }
+    } else if (lr < rows) {
+#pragma unroll
+      for (int g = 0; g < kTilesOut; ++g)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int ch = (ch0 + 2 * g) * 16 + 8 * j + (lane >> 5) * 4;
+          if (ch >= a.groups * 16)
+            continue;
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            store_act<T>(static_cast<T *>(a.C) + (int64_t)(ch + i) * a.ldc + lr, acc[g][r][4 * j + i]);
+        }
     }
   }
 }
@@ -981,7 +1007,8 @@ int launch_rows_gemm(const RowsGemm &a, hipStream_t stream, int *slices) {
   BH_REQUIRE(a.lda % 8 == 0 && a.lda >= round_up(W.K, 8) && ((uintptr_t)a.A & 15) == 0,
              "rows_gemm: activation rows must be 16-byte aligned (lda %d, K %d)", a.lda, W.K);
   BH_REQUIRE(((uintptr_t)a.C & 15) == 0 &&
-                 (a.out == kOutActTrans ? a.ldc >= a.rows : (a.ldc % 4 == 0 && a.ldc >= W.N)),
+                 (a.out == kOutActTrans ? a.ldc >= a.rows
+                                         : (a.ldc % (a.out == kOutF32 ? 4 : 8) == 0 && a.ldc >= W.N)),
              "rows_gemm: result rows (ldc %d, N %d)", a.ldc, W.N);
   BH_REQUIRE(!a.counts || (a.lists && a.experts > 0 && a.list_cap > 0 && a.list_div > 0),
              "rows_gemm: expert lists");

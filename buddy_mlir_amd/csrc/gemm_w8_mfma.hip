@@ -130,8 +130,8 @@ __device__ __forceinline__ float silu_times(float g, float u) {
 }
 
 // The attention's output, added up from its parts, as the terms of the matmul behind it (in f32 rows and
-// a conversion: 8.7 + 4.4 us for 150 tokens).  A workgroup per token and four heads: few tokens then come in through all
-// compute units (twelve heads to a workgroup: 150 tokens of 37 parts 8.6 us, so 8.2).
+// a conversion: 8.7 + 4.4 us for 150 tokens).  A workgroup per token and four heads: few tokens then come in through
+// all compute units (twelve heads to a workgroup: 150 tokens of 37 parts 8.6 us, so 8.2).
 constexpr int kFoldThreads = 128;
 template <int kMost>
 __global__ void __launch_bounds__(kFoldThreads, kMost == 4 ? 8 : 1)
@@ -855,8 +855,8 @@ int launch_attn_fold_to_terms(const PromptFold &fold, int64_t o_stride, int head
   BH_REQUIRE(fold.blocks && staged && tokens > 0 && terms >= 1 && terms <= 3, "attn_fold_to_terms: bad argument");
   const GemmStagingLayout l = gemm_staging_layout(tokens, K); // K is a multiple of 64: no padding
   hipLaunchKernelGGL(tokens > kFoldTokens ? attn_fold_to_terms_kernel<4> : attn_fold_to_terms_kernel<16>,
-                     dim3(tokens, (unsigned)ceil_div(K, 4 * kFoldThreads)), dim3(kFoldThreads), 0, stream, fold, o_stride,
-                     (int)K, terms, l.rows_padded, staged);
+                     dim3(tokens, (unsigned)ceil_div(K, 4 * kFoldThreads)), dim3(kFoldThreads), 0, stream, fold,
+                     o_stride, (int)K, terms, l.rows_padded, staged);
   BH_CHECK_HIP(hipGetLastError());
   return BUDDY_HIP_OK;
 }
