@@ -27,7 +27,11 @@ __device__ __forceinline__ bf16_bits f_bf(float f) {
   return __builtin_bit_cast(bf16_bits, b);
 }
 __device__ __forceinline__ unsigned pack_bf(float a, float b) {
-  return (unsigned)f_bf(a) | ((unsigned)f_bf(b) << 16);
+  // (as f_bf of each; as a vector they are one instruction, by themselves three)
+  typedef float two_f32 __attribute__((ext_vector_type(2)));
+  typedef __bf16 two_bf16 __attribute__((ext_vector_type(2)));
+  const two_f32 v = {a, b};
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(v, two_bf16));
 }
 __device__ __forceinline__ float sigmoid_f(float z) { return 1.0f / (1.0f + expf(-z)); }
 __device__ __forceinline__ float silu_f(float z) { return z * sigmoid_f(z); }

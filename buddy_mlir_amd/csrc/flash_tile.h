@@ -76,6 +76,7 @@ template <typename T, int NK, int NV> struct Flash {
       __builtin_amdgcn_sched_barrier(0);
     }
     if (!whole) {
+      asm volatile(""); // a branch: as selects, whole tiles pay as well
 #pragma unroll
       for (int b = 0; b < SUB; ++b)
 #pragma unroll
@@ -171,7 +172,61 @@ template <typename T, int NK, int NV> struct Flash {
         }
     }
   }
+
+  // Where the wavefronts of a block of 64 queries meet, per group of four that shared tiles: sums
+  // [64][kMeetRow], then [64][maximum, sum of weights].
+  static constexpr int kMeetRow = 16 * NV + 4, kMeet = 64 * kMeetRow + 128;
+  __device__ __forceinline__ void leave(float *meet, int query) const {
+    const int quad = threadIdx.x >> 4 & 3;
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+      *reinterpret_cast<f32x4 *>(meet + query * kMeetRow + v * 16 + quad * 4) = o[v];
+    const float sum = sum_rows(l);
+    if (quad == 0) {
+      meet[64 * kMeetRow + 2 * query] = m;
+      meet[64 * kMeetRow + 2 * query + 1] = sum;
+    }
+  }
+  // channels c .. c + 3 of a query over all groups, its maximum and its sum of weights
+  template <int GROUPS>
+  static __device__ __forceinline__ f32x4 met(const float *meet, int query, int c, float &most, float &sum) {
+    const float *ml = meet + 64 * kMeetRow + 2 * query;
+    f32x4 x = *reinterpret_cast<const f32x4 *>(meet + query * kMeetRow + c);
+    most = ml[0];
+    sum = ml[1];
+    if constexpr (GROUPS == 2) {
+      const f32x4 y = *reinterpret_cast<const f32x4 *>(meet + kMeet + query * kMeetRow + c);
+      const float m1 = ml[kMeet], both = fmaxf(most, m1), base = both == -INFINITY ? 0.f : both;
+      const float f0 = fast_exp(most - base), f1 = fast_exp(m1 - base);
+      most = both;
+      sum = sum * f0 + ml[kMeet + 1] * f1;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        x[i] = x[i] * f0 + y[i] * f1;
+    }
+    return x;
+  }
+  // Two groups of wavefronts, of every other tile each, where their sums fit the registers.
+  static constexpr size_t kTileBytes = sizeof(T) * ((size_t)KEYS * kKeyRow + (size_t)16 * NV * kValueRow);
+  static constexpr size_t kGroupLds = kTileBytes > 4 * kMeet ? kTileBytes : 4 * kMeet;
+  static constexpr int kGroups = NV <= 8 ? 2 : 1;
 };
+
+// Four channels of a result row; `whole`: rows and channels are so aligned that one store does.
+template <typename OUT>
+__device__ __forceinline__ void store_channels(OUT *p, f32x4 v, int left, bool whole) {
+  if (whole) {
+    if constexpr (sizeof(OUT) == 4)
+      *reinterpret_cast<f32x4 *>(p) = v;
+    else
+      *reinterpret_cast<uint2 *>(p) = uint2{pack_bf(v[0], v[1]), pack_bf(v[2], v[3])};
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (i < left)
+      store_act<OUT>(p + i, v[i]);
+}
 #endif
 
 } // namespace bh

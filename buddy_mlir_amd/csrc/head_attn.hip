@@ -458,29 +458,34 @@ head_rows_kernel(const float *__restrict__ proj, T *__restrict__ keys, T *__rest
 struct HeadAttnArgs {
   int map_heads, group, maps, vdim, nv, kd, window;
   int rows, start, cache_rows, ring_mask, out_ld;
+  int whole; // four channels of a result at a time
   const float *sink;
 };
 
-// Grid (map heads, query blocks).  A wavefront owns 16 queries, the workgroup's four
-// share tiles of keys through LDS; the next tile is on its way in registers meanwhile.
+// Grid (map heads, query blocks).  A wavefront owns 16 queries, four share tiles of keys
+// through LDS; the next tile is on its way in registers meanwhile.  Two such groups take
+// every other tile each and meet at the end: one of 156 workgroups on 256 compute units is bound by
+// its chain of tiles (777 tokens, 12 heads of 128: one group 24.2 us, two 18.7; two maps of 64 25.8 and
+// 18.0; 300 f32 tokens 31.3 and 28.4).
 // NK: 32-element steps of a key, NV: 16-channel groups of a value, at most; smaller
 // heads are padded with zeros (keys) or with rows whose results are not stored (values).
 // Tiles start at multiples of their size, so none is cut by the end of a ring.  OUT: f32
 // or the activations' type.
 template <typename T, typename OUT, int NK, int NV>
-__global__ void __launch_bounds__(256, NV <= 8 ? 2 : 1)
+__global__ void __launch_bounds__((256 * Flash<T, NK, NV>::kGroups), NV <= 8 ? 2 : 1)
 head_attention_kernel(const T *__restrict__ queries, const T *__restrict__ keys,
                       const T *__restrict__ values_t, OUT *__restrict__ out, HeadAttnArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char raw[];
   using F = Flash<T, NK, NV>;
   constexpr int E = F::E, KEYS = F::KEYS, kBlock = 64;
   constexpr int KL = NK, VL = (NV + 1) / 2; // 16-byte loads per thread and tile
-  const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, quad = lane >> 4;
+  const int tid = threadIdx.x & 255, lane = tid & 63, col = lane & 15, quad = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8);
   const int hm = blockIdx.x, h = hm / a.maps, g = h / a.group, gm = g * a.maps + hm % a.maps;
   const int q0 = (gridDim.y - 1 - blockIdx.y) * kBlock; // long blocks first
-  T *kt = reinterpret_cast<T *>(raw); // [KEYS][kKeyRow]
-  T *vt = kt + KEYS * F::kKeyRow;     // [16 * NV][kValueRow]
+  T *kt = reinterpret_cast<T *>(raw + group * F::kGroupLds); // [KEYS][kKeyRow]
+  T *vt = kt + KEYS * F::kKeyRow;                               // [16 * NV][kValueRow]
 
   const int qi = q0 + wave * 16 + col, my_q = a.start + qi; // this lane's query
   Frag<T> qf[NK];
@@ -516,8 +521,9 @@ head_attention_kernel(const T *__restrict__ queries, const T *__restrict__ keys,
     vdst[i] = F::value_at(r, c);
   }
   u32x4 kr[KL], vr[VL];
+  const int last_tile = key_hi & ~(KEYS - 1);
   auto fetch = [&](int k0) { // positions past the last query's are masked
-    const int slot = k0 & a.ring_mask;
+    const int slot = min(max(k0, key_lo), last_tile) & a.ring_mask;
     const T *kp = kc + (int64_t)slot * a.kd;
 #pragma unroll
     for (int i = 0; i < KL; ++i)
@@ -526,7 +532,11 @@ head_attention_kernel(const T *__restrict__ queries, const T *__restrict__ keys,
     for (int i = 0; i < VL; ++i)
       vr[i] = *reinterpret_cast<const u32x4 *>(vsrc[i] + slot);
   };
-  fetch(key_lo);
+  // one or two tiles are the first group's: the second would save what the meeting costs
+  const bool split = F::kGroups == 2 && key_hi - key_lo >= 2 * KEYS;
+  const int stride = split ? 2 * KEYS : KEYS;
+  const int first = split ? (key_lo & ~(2 * KEYS - 1)) + group * KEYS : key_lo;
+  fetch(first);
   if (a.kd < NK * 32) { // the padding of the keys
     const int pad = NK * 32 - a.kd;
     for (int i = tid; i < KEYS * pad; i += 256)
@@ -534,7 +544,7 @@ head_attention_kernel(const T *__restrict__ queries, const T *__restrict__ keys,
   }
 
   F flash;
-  for (int k0 = key_lo; k0 <= key_hi; k0 += KEYS) {
+  for (int k0 = first; k0 - (split ? group * KEYS : 0) <= key_hi; k0 += stride) { // as often in both groups
     __syncthreads(); // the previous tile has been read
 #pragma unroll
     for (int i = 0; i < KL; ++i)
@@ -543,33 +553,33 @@ head_attention_kernel(const T *__restrict__ queries, const T *__restrict__ keys,
     for (int i = 0; i < VL; ++i)
       F::store_value(vt, vdst[i], vr[i]);
     __syncthreads();
-    fetch(min(k0 + KEYS, key_hi & ~(KEYS - 1)));
-    if (k0 > wave_q1 || k0 + KEYS - 1 <= wave_q0 - a.window)
+    fetch(k0 + stride);
+    if ((!split && group) || k0 < key_lo || k0 > min(wave_q1, key_hi) || k0 + KEYS - 1 <= wave_q0 - a.window)
       continue; // nothing of this tile is visible to this wavefront
     const bool whole = k0 + KEYS - 1 <= wave_q0 && wave_q1 - k0 < a.window;
     flash.tile(kt, vt, qf, whole, my_q - k0, a.window);
   }
-  float sum = sum_rows(flash.l);
-  if (qi >= a.rows)
-    return;
-  float f;
-  if (a.sink) {
-    const float sink = a.sink[h], m = fmaxf(flash.m, sink), e = fast_exp(flash.m - m);
-    f = e / fmaf(sum, e, fast_exp(sink - m));
-  } else {
-    f = 1.0f / sum;
-  }
-  OUT *dst = out + (int64_t)qi * a.out_ld + (int64_t)hm * a.vdim;
+  __syncthreads(); // every tile has been read
+  float *meet = reinterpret_cast<float *>(raw);
+  flash.leave(meet + group * F::kMeet, wave * 16 + col);
+  __syncthreads();
 #pragma unroll
-  for (int v = 0; v < NV; ++v)
-    if (v < a.nv) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int c = v * 16 + quad * 4 + r;
-        if (c < a.vdim)
-          store_act<OUT>(dst + c, flash.o[v][r] * f);
-      }
+  for (int i = 0; i < NV / F::kGroups; ++i) {
+    const int id = i * 256 * F::kGroups + threadIdx.x, query = id / (4 * NV), c = id % (4 * NV) * 4;
+    if (q0 + query >= a.rows || c >= a.vdim)
+      continue;
+    float m, sum;
+    const f32x4 x = F::template met<F::kGroups>(meet, query, c, m, sum);
+    float f;
+    if (a.sink) {
+      const float sink = a.sink[h], most = fmaxf(m, sink), e = fast_exp(m - most);
+      f = e / fmaf(sum, e, fast_exp(sink - most));
+    } else {
+      f = 1.0f / sum;
     }
+    store_channels<OUT>(out + (int64_t)(q0 + query) * a.out_ld + (int64_t)hm * a.vdim + c, x * f, a.vdim - c,
+                        a.whole);
+  }
 }
 
 struct HeadCombineArgs {
@@ -698,20 +708,21 @@ namespace {
 template <typename T, typename OUT, int NK, int NV>
 int launch_attention(const HeadRows &a, OUT *out, const HeadAttnArgs &p, hipStream_t stream) {
   using F = Flash<T, NK, NV>;
-  constexpr size_t lds = sizeof(T) * ((size_t)F::KEYS * F::kKeyRow + (size_t)16 * NV * F::kValueRow);
+  constexpr size_t lds = F::kGroups * F::kGroupLds;
   static_assert(lds <= kLdsLimit, "the tiles must fit LDS");
   static DynLdsOnce once;
   BH_CHECK_HIP(ensure_dyn_lds(once, (const void *)head_attention_kernel<T, OUT, NK, NV>, (int)kLdsLimit));
   hipLaunchKernelGGL((head_attention_kernel<T, OUT, NK, NV>),
-                     dim3((unsigned)p.map_heads, (unsigned)ceil_div(a.rows, 64)), dim3(256), lds, stream,
+                     dim3((unsigned)p.map_heads, (unsigned)ceil_div(a.rows, 64)), dim3(256 * F::kGroups), lds, stream,
                      static_cast<const T *>(a.queries), static_cast<const T *>(a.keys),
                      static_cast<const T *>(a.values_t), out, p);
   BH_CHECK_HIP(hipGetLastError());
   return BUDDY_HIP_OK;
 }
 template <typename T, typename OUT>
-int launch_attention_any(const HeadRows &a, OUT *out, const HeadAttnArgs &p, hipStream_t stream) {
+int launch_attention_any(const HeadRows &a, OUT *out, HeadAttnArgs p, hipStream_t stream) {
   const int nk = p.kd / 32;
+  p.whole = p.vdim % 4 == 0 && p.out_ld % 4 == 0 && ((uintptr_t)out & 15) == 0;
   BH_REQUIRE(nk <= 16 && p.nv <= 32, "head_attention: heads of %d and %d values", a.s.dim, a.s.vdim);
   if (nk <= 2 && p.nv <= 4)
     return launch_attention<T, OUT, 2, 4>(a, out, p, stream);
@@ -733,11 +744,12 @@ template <typename T> int launch_rows(const HeadRows &a, hipStream_t stream) {
   const int value_tiles = (a.start + a.rows - 1) / kTile - a.start / kTile + 1;
   const int value_groups = value_tiles * s.kv_heads * (int)ceil_div(s.vdim16(), kValueSlice);
   const size_t lds = sizeof(float) * std::max((size_t)s.rot_dims, (size_t)kTile * (kValueSlice + 1));
-  hipLaunchKernelGGL(head_rows_kernel<T>, dim3((unsigned)(a.rows + value_groups)), dim3(256), lds, stream, a.proj, static_cast<T *>(a.keys), static_cast<T *>(a.values_t),
-                     static_cast<T *>(a.queries), s.turns, s.dim32(), r);
+  hipLaunchKernelGGL(head_rows_kernel<T>, dim3((unsigned)(a.rows + value_groups)), dim3(256), lds, stream, a.proj,
+                     static_cast<T *>(a.keys), static_cast<T *>(a.values_t), static_cast<T *>(a.queries), s.turns,
+                     s.dim32(), r);
   BH_CHECK_HIP(hipGetLastError());
   HeadAttnArgs p{s.map_heads(), s.heads / s.kv_heads, s.maps, s.vdim, s.vdim16() / 16, s.dim32(), window_of(s),
-                 a.rows, a.start, s.rows, s.ring_mask, a.out_ld, s.sink};
+                 a.rows, a.start, s.rows, s.ring_mask, a.out_ld, 0, s.sink};
   if (s.maps == 1 && !s.gated)
     return launch_attention_any<T, T>(a, static_cast<T *>(a.out), p, stream);
   p.out_ld = s.map_heads() * s.vdim;

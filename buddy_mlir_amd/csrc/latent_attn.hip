@@ -449,31 +449,40 @@ latent_rows_kernel(const float *__restrict__ proj, T *__restrict__ cache, T *__r
 struct LatentAttnArgs {
   int heads, dim16, rot8, vdim, nv, row_elems, window, ring_mask;
   int ld, gate_at, rows, start, first, value_ld, out_ld;
-  int kd; // elements of a query
+  int kd;    // elements of a query
+  int whole; // four channels of a result at a time
 };
 
-// Grid (heads, query blocks).  A wavefront owns 16 queries, the workgroup's four
-// share tiles of kKeys keys through LDS; the next tile is on its way in registers
-// meanwhile.
+// Grid (heads, query blocks).  A wavefront owns 16 queries, four share tiles of kKeys
+// keys through LDS; the next tile is on its way in registers meanwhile.  Two such groups
+// take every other tile each and meet at the end.
+//
+// What bounds it: a pair of tiles takes 2.9 us, 1.7 of them products, softmax and fragments (the
+// eight wavefronts are in the same phase at once: LDS, then vector, then matrix instructions), the
+// rest the next tiles' way in; 2.5 us to begin and as much to meet.  2048 tokens, 12 heads of 128 + 64 in a
+// window of 1024: 384 workgroups, the shortest behind the longest.  One group a workgroup and two
+// workgroups a compute unit 45.7 us, so 44.9.
 // NK: 32-element steps of a key, NV: 16-channel groups of a value, at most; smaller
 // heads are padded with zeros (keys) or with rows whose results are not stored
 // (values), so that the loop has no branches.
 template <typename T, int NK, int NV>
-__global__ void __launch_bounds__(256, NV <= 8 ? 2 : 1)
+__global__ void __launch_bounds__((256 * Flash<T, NK, NV>::kGroups), NV <= 8 ? 2 : 1)
 latent_attention_kernel(const T *__restrict__ queries, const T *__restrict__ keys,
                         const T *__restrict__ values_t, const T *__restrict__ cache,
                         const float *__restrict__ proj, T *__restrict__ out, LatentAttnArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char raw[];
-  constexpr int E = 16 / (int)sizeof(T), KEYS = KeyTile<T>::kKeys;
+  using F = Flash<T, NK, NV>;
+  constexpr int E = F::E, KEYS = F::KEYS;
   constexpr int KL = NK, VL = (NV + 1) / 2; // 16-byte loads per thread and tile
-  const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, quad = lane >> 4;
+  const int tid = threadIdx.x & 255, lane = tid & 63, col = lane & 15, quad = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8);
   const int h = blockIdx.x;
   constexpr int kBlock = 64;
   const int q0 = (gridDim.y - 1 - blockIdx.y) * kBlock; // long blocks first
-  constexpr int kKeyRow = Flash<T, NK, NV>::kKeyRow, kValueRow = Flash<T, NK, NV>::kValueRow;
-  T *kt = reinterpret_cast<T *>(raw); // [KEYS][kKeyRow]
-  T *vt = kt + KEYS * kKeyRow;        // [16 * NV][kValueRow]
+  constexpr int kKeyRow = F::kKeyRow;
+  T *kt = reinterpret_cast<T *>(raw + group * F::kGroupLds); // [KEYS][kKeyRow]
+  T *vt = kt + KEYS * kKeyRow;                                  // [16 * NV][kValueRow]
 
   // this lane's query, also as a key index, and its fragments
   const int qi = q0 + wave * 16 + col, my_q = a.start + qi - a.first;
@@ -516,10 +525,12 @@ latent_attention_kernel(const T *__restrict__ queries, const T *__restrict__ key
     const int id = min(i * 256 + tid, vruns - 1), r = id >> 3, c = id & 7;
     vsrc[i] = values_t + (int64_t)(h * 16 * a.nv + r) * a.value_ld + c * E;
     vcol[i] = c * E;
-    vdst[i] = Flash<T, NK, NV>::value_at(r, c);
+    vdst[i] = F::value_at(r, c);
   }
   u32x4 kr[KL], vr[VL];
-  auto fetch = [&](int k0, u32x4 (&kr)[KL], u32x4 (&vr)[VL]) {
+  const int last_tile = (nkeys - 1) & ~(KEYS - 1);
+  auto fetch = [&](int at) {
+    const int k0 = min(max(at, key_lo), last_tile);
 #pragma unroll
     for (int i = 0; i < KL; ++i) {
       const int k = min(k0 + kkey[i], nkeys - 1); // masked past the end
@@ -530,15 +541,19 @@ latent_attention_kernel(const T *__restrict__ queries, const T *__restrict__ key
     for (int i = 0; i < VL; ++i)
       vr[i] = *reinterpret_cast<const u32x4 *>(vsrc[i] + k0);
   };
-  fetch(key_lo, kr, vr);
+  // one or two tiles are the first group's: the second would save what the meeting costs
+  const bool split = F::kGroups == 2 && key_hi - key_lo >= 2 * KEYS;
+  const int stride = split ? 2 * KEYS : KEYS;
+  const int first = split ? (key_lo & ~(2 * KEYS - 1)) + group * KEYS : key_lo;
+  fetch(first);
   if (runs * E < NK * 32) { // the padding of the keys
     const int pad = NK * 32 - runs * E, at = a.dim16 + a.rot8;
     for (int i = tid; i < KEYS * pad; i += 256)
       kt[(i / pad) * kKeyRow + at + i % pad] = 0;
   }
 
-  Flash<T, NK, NV> flash;
-  for (int k0 = key_lo; k0 <= key_hi; k0 += KEYS) {
+  F flash;
+  for (int k0 = first; k0 - (split ? group * KEYS : 0) <= key_hi; k0 += stride) { // as often in both groups
     __syncthreads(); // the previous tile has been read
 #pragma unroll
     for (int i = 0; i < KL; ++i)
@@ -558,29 +573,36 @@ latent_attention_kernel(const T *__restrict__ queries, const T *__restrict__ key
     }
 #pragma unroll
     for (int i = 0; i < VL; ++i)
-      Flash<T, NK, NV>::store_value(vt, vdst[i], vr[i]);
+      F::store_value(vt, vdst[i], vr[i]);
     __syncthreads();
-    fetch(min(k0 + KEYS, (nkeys - 1) & ~(KEYS - 1)), kr, vr);
-    if (k0 > wave_q1 || k0 + KEYS - 1 <= wave_q0 - a.window)
+    fetch(k0 + stride);
+    if ((!split && group) || k0 < key_lo || k0 > min(wave_q1, key_hi) || k0 + KEYS - 1 <= wave_q0 - a.window)
       continue; // nothing of this tile is visible to this wavefront
     const bool whole = k0 + KEYS - 1 <= wave_q0 && wave_q1 - k0 < a.window;
     flash.tile(kt, vt, qf, whole, my_q - k0, a.window);
   }
-  const float sum = sum_rows(flash.l);
-  if (qi >= a.rows)
-    return;
-  const float f = sigmoid_f(proj[(int64_t)qi * a.ld + a.gate_at + h]) / sum;
-  T *dst = out + (int64_t)qi * a.out_ld + (int64_t)h * a.vdim;
+  constexpr int kTurns = NV / F::kGroups; // of the workgroup's threads over 4 channels each
+  float gate[kTurns];
 #pragma unroll
-  for (int v = 0; v < NV; ++v)
-    if (v < a.nv) {
+  for (int i = 0; i < kTurns; ++i) {
+    const int row = q0 + (i * 256 * F::kGroups + (int)threadIdx.x) / (4 * NV);
+    gate[i] = proj[(int64_t)min(row, a.rows - 1) * a.ld + a.gate_at + h];
+  }
+  __syncthreads(); // every tile has been read
+  float *meet = reinterpret_cast<float *>(raw);
+  flash.leave(meet + group * F::kMeet, wave * 16 + col);
+  __syncthreads();
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int c = v * 16 + quad * 4 + r;
-        if (c < a.vdim)
-          store_act<T>(dst + c, flash.o[v][r] * f);
-      }
-    }
+  for (int i = 0; i < kTurns; ++i) {
+    const int id = i * 256 * F::kGroups + threadIdx.x, query = id / (4 * NV), c = id % (4 * NV) * 4;
+    const int row = q0 + query;
+    if (row >= a.rows || c >= a.vdim)
+      continue;
+    float m, sum;
+    const f32x4 x = F::template met<F::kGroups>(meet, query, c, m, sum);
+    const float f = sigmoid_f(gate[i]) / sum;
+    store_channels<T>(out + (int64_t)row * a.out_ld + (int64_t)h * a.vdim + c, x * f, a.vdim - c, a.whole);
+  }
 }
 
 bool shape_ok(const LatentShape &s) {
@@ -705,13 +727,13 @@ int launch_latent_rows(const LatentRows &a, hipStream_t stream) {
 namespace {
 template <typename T, int NK, int NV>
 int launch_attention(const LatentRows &a, const LatentAttnArgs &p, hipStream_t stream) {
-  constexpr int E = 16 / (int)sizeof(T), KEYS = KeyTile<T>::kKeys;
-  constexpr size_t lds = sizeof(T) * ((size_t)KEYS * (NK * 32 + E) + (size_t)16 * NV * (KEYS + E));
+  using F = Flash<T, NK, NV>;
+  constexpr size_t lds = F::kGroups * F::kGroupLds;
   static_assert(lds <= kLdsLimit, "the tiles must fit LDS");
   static DynLdsOnce once;
   BH_CHECK_HIP(ensure_dyn_lds(once, (const void *)latent_attention_kernel<T, NK, NV>, (int)kLdsLimit));
   hipLaunchKernelGGL((latent_attention_kernel<T, NK, NV>),
-                     dim3((unsigned)a.s.heads, (unsigned)ceil_div(a.rows, 64)), dim3(256), lds,
+                     dim3((unsigned)a.s.heads, (unsigned)ceil_div(a.rows, 64)), dim3(256 * F::kGroups), lds,
                      stream, static_cast<const T *>(a.queries), static_cast<const T *>(a.keys),
                      static_cast<const T *>(a.values_t), static_cast<const T *>(a.cache), a.proj,
                      static_cast<T *>(a.out), p);
@@ -742,7 +764,8 @@ int launch_latent_attention(const LatentRows &a, hipStream_t stream) {
              "latent_attention: bad argument");
   LatentAttnArgs p{s.heads, s.dim16(), s.rot8(), s.vdim, s.vdim16() / 16, s.row_elems(), s.window,
                    s.ring_mask, a.ld, a.gate_at, a.rows, a.start, a.first, a.value_ld, a.out_ld,
-                   s.key_elems()};
+                   s.key_elems(), 0};
+  p.whole = s.vdim % 4 == 0 && a.out_ld % 4 == 0 && ((uintptr_t)a.out & 15) == 0;
   return s.f32 ? launch_attention_any<float>(a, p, stream)
                : launch_attention_any<bf16_bits>(a, p, stream);
 }

@@ -278,6 +278,20 @@ def test_far_keys(tmp_path, dtype, kind, length):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n,start", [(63, 0), (64, 64), (65, 64), (128, 0), (129, 0), (192, 1), (193, 0), (250, 63)])
+def test_blocks_that_see_one_to_five_tiles_of_keys(tmp_path, n, start, dtype):
+    """Tiles of 64 (f32: 32) keys are shared out to two groups of wavefronts from three
+    on; windows that begin inside a tile, heads that fill their padded sizes and do not."""
+    cfg = M.config([M.full(heads=4, kv=2, dim=64, rot=64, vdim=64, ff=None),
+                    M.diff(heads=2, kv=1, dim=20, rot=8, vdim=18, window=100, ff=None),
+                    M.full(heads=3, kv=1, dim=100, rot=30, vdim=127, ff=None)], width=64)
+    folder, t = M.build(tmp_path, cfg, 3)
+    tokens = tokens_for(cfg, start + n, n)
+    s = FolderSession(folder, dtype, max_len=320)
+    check(feed(s, tokens, [start, n] if start else [n]), L.forward(cfg, t, tokens), dtype, (n, start))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_sink_takes_the_weight_that_no_key_earns(tmp_path, dtype):
     """With a sink between the ordinary scores and the needle's, what is found depends
     on the sink alone: nothing without the needle, all of it with."""

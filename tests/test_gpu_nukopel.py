@@ -261,6 +261,19 @@ def test_window_passes_over_decoded_tokens(tmp_path, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n,start", [(63, 0), (64, 64), (65, 64), (128, 0), (129, 0), (192, 1), (193, 0), (250, 63)])
+def test_blocks_that_see_one_to_five_tiles_of_keys(tmp_path, n, start, dtype):
+    """Tiles of 64 (f32: 32) keys are shared out to two groups of wavefronts from three
+    on; windows that begin inside a tile, heads that fill their padded sizes and do not."""
+    cfg = M.config([M.latent(heads=2, dim=128, rot=64, vdim=128, rank=64, window=150, mlp=None),
+                    M.latent(heads=3, dim=30, rot=10, vdim=31, window=300, mlp=None)], width=64)
+    folder, t = M.build(tmp_path, cfg, 3)
+    tokens = tokens_for(cfg, start + n, n)
+    s = FolderSession(folder, dtype, max_len=320)
+    check(feed(s, tokens, [start, n] if start else [n]), N.forward(cfg, t, tokens), dtype, (n, start))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("length", [1030, 4110])
 def test_far_keys_in_long_windows(tmp_path, dtype, length):
     """One key among thousands decides; the spans that change how a step cuts its
