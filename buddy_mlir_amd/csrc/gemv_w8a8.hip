@@ -465,7 +465,10 @@ int launch_rows(const float *A, const int4 *W, const RowsOut &to, int64_t M, int
   int parts = 1;
   if (!own)
     parts = launch_absmax(A, M * K, part, st);
-  const dim3 grid((unsigned)round_up((int64_t)p.ncols * p.slices, 8), (unsigned)p.row_tiles);
+  // a multiple of 8 keeps a column's row tiles on one XCD, which must have compute units for all of them:
+  // 672 rows of 1536 -> 1536 padded to 16 columns were two rounds on four XCDs, 19.6 us
+  const int64_t cols = (int64_t)p.ncols * p.slices, padded = round_up(cols, 8);
+  const dim3 grid((unsigned)(padded * p.row_tiles <= 256 ? padded : cols), (unsigned)p.row_tiles);
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, dim3(kRowsThreads), 0, st, A, W, part, parts, (int)M, (int)K, (int)N,
                        (int)ceil_div(N, kTileN), (int)ceil_div(K, kTileK), p.per_slice, p.ncols, p.slices, out);

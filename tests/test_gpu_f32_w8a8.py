@@ -158,7 +158,8 @@ def test_w8a8_many_rows_extremes(bh, oracle):
 # 16 bytes at a time: (a tile's edges in rows, channels and k; K in slices; channels one by one)
 @pytest.mark.parametrize("M,K,N", [(2, 1536, 64), (5, 4, 7), (31, 68, 130), (32, 1536, 8960),
                                    (33, 1536, 33), (64, 1540, 257), (256, 1000, 1111), (3, 3076, 70),
-                                   (16, 8960, 1536), (96, 8960, 1536), (17, 131072, 40)])
+                                   (16, 8960, 1536), (96, 8960, 1536), (17, 131072, 40),
+                                   (650, 1540, 1530)])
 @pytest.mark.parametrize("special", [False, True])
 def test_w8a8_rows_equal_the_general_path(bh, M, K, N, special):
     q, s = synthetic.quantized_linear(K, N, M + K)
