@@ -12,39 +12,33 @@ constexpr int kAttnChunk = 64; // cache positions per flash-decoding partial (th
 // 256 beyond (8 or 16 wavefronts of 16 positions per workgroup).  From 5120 on
 // (where those launches would outgrow one workgroup per compute unit) the
 // partials are folded by a launch of their own and one workgroup takes all the
-// query heads of a KV head, or half of them (a K/V row then leaves L2 once or
-// twice, not once per head).  Attention and fold cover only the chunks up to the
-// position (rounded up to a multiple of four; 18 with chunks of 64), whatever the
+// query heads of a KV head (a K/V row then leaves L2 once, not once per head).
+// Attention and fold cover only the chunks up to the
+// position (rounded up to a multiple of four; 18, or one of eight, with chunks of 64), whatever the
 // cache's capacity.
 struct AttnStepPlan {
   int chunk;     // cache positions per partial: 64, 128 or 256
   int used;      // partials per head the step produces and folds
   bool own_fold; // a launch of its own folds them; workgroups take whole head groups
-  int head_split; // ... or (2) half a head group each
 };
 inline AttnStepPlan attn_step_plan(int pos, int max_len, int kv_heads) {
   AttnStepPlan p;
-  p.head_split = 1;
   p.own_fold = pos >= 20 * 256;
   if (!p.own_fold) {
     p.chunk = pos < 18 * 64 ? 64 : pos < 18 * 128 ? 128 : 256;
   } else {
-    // Measured on a 12-head, 2-KV-head model from 5 k to 32 k positions (ms per step
-    // for chunk x split): workgroups of 16 wavefronts (chunks of 256) must not
-    // outnumber the 256 compute units, and want at least ~150 of them busy.
-    const int n256 = (pos / 256 + 1) * kv_heads; // workgroups of whole head groups on chunks of 256
-    if (2 * n256 <= 256) {
-      p.chunk = n256 >= 100 ? 256 : 128; // 16 k: 1.005 (256 x 2) vs 1.027; 12 k: 0.986 (128 x 2) vs 0.995
-      p.head_split = 2;
-    } else {
-      p.chunk = 256; // 20 k: 1.138 (256 x 1) vs 1.159 (128 x 1); 17.5 k: 1.147 with 128 x 1
-    }
+    // Measured on a 12-head, 2-KV-head model from 5 k to 32 k positions: the smallest chunks
+    // whose workgroups have a compute unit each, since one takes in some 40 bytes a nanosecond
+    // whatever the others do (us per step on chunks of 64, 128 and 256: 5200 817 / 837 / 955, 8000 838 / 852 / 966,
+    // 10 k 896 / 861 / 976, 16 k 908 / 893 / 978, 20 k 1041 / 1054 / 988, 32 k 1229 / 1117 / 1079).
+    const auto workgroups = [&](int chunk) { return (pos / chunk + 1) * (int64_t)kv_heads; };
+    p.chunk = workgroups(64) <= 256 ? 64 : workgroups(128) <= 256 ? 128 : 256;
   }
   const int all = (max_len + p.chunk - 1) / p.chunk, need = pos / p.chunk + 1;
   // 18 for chunks of 64 (one captured step serves a cache of 1152 positions, and
   // the fold's first trip takes 18 anyway); with larger chunks the next multiple
   // of four: every chunk past the position costs workgroups that find nothing to do
-  int want = (need + 3) / 4 * 4;
+  int want = p.own_fold && p.chunk == 64 ? (need + 7) / 8 * 8 : (need + 3) / 4 * 4;
   if (need <= 18)
     want = p.chunk == 64 || want > 18 ? 18 : want;
   p.used = want < all ? want : all;
@@ -74,7 +68,6 @@ struct AttnDecodeArgs {
   // per (chunk, KV head) for all its query heads, then a fold with all partials
   // in flight instead of chunk by chunk (covers chunks_used partials, no lse)
   bool wide_combine = false;
-  int head_split = 1; // with wide_combine: 2 = two workgroups per (chunk, KV head), half its heads each
   int chunk = kAttnChunk; // cache positions per partial: 64, 128 or 256
   // partials to produce (the first ones; the caller knows the position lies in
   // them); 0: one for every chunk of the cache

@@ -49,7 +49,6 @@ struct AttnArgs {
   float *lse;            // [heads] or null: m + log l of the whole softmax
   int heads, kv_heads, group, max_len, nchunks, chunk;
   int used; // chunks this launch covers (the first ones of nchunks)
-  int head_split; // grouped launches: workgroups per (chunk, KV head), each a share of its heads
   float scale;
   int pairs_padded; // (chunk, kv head) pairs rounded up to the XCD count
 };
@@ -272,12 +271,50 @@ __global__ void __launch_bounds__(kWaves * 64)
 // The same for a step far into a long cache, where the rows of a chunk coming
 // out of L2 once per query head (six times for this model) is what the launch
 // waits for: one workgroup takes all the query heads of a KV head, so that a K/V
-// row is loaded once and multiplied with every head's query.
-template <int kWaves>
+// row is loaded once and multiplied with every head's query on the f32 matrix
+// instructions of 16 blocks of 4 x 4, four heads (one of kSets) at a time: those of 16 x 16
+// would leave ten of sixteen columns idle where a group has six heads.  What bounds it: a compute unit's
+// rows on their way in, some 40 bytes a nanosecond, then about 1300 clocks of products and exchanges.  A step
+// behind 12000 positions 965 us with vector instructions (six heads one after the other, half of them a
+// workgroup), 937 on 16 x 16, 901 so; of these 8.8 us a layer here, before 11.1.
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+// scores of four heads: + q[head][dim e of a quarter's four] * key's dim; the operand with the queries
+// holds dim e of quarter c in block 4 c + e, which goes to the quarter's four blocks
+__device__ __forceinline__ void add_scores(float q, float4 k, v4f (&s)[2]) {
+  s[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(q, k.x, s[0], 2, 0, 0);
+  s[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(q, k.y, s[1], 2, 1, 0);
+  s[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(q, k.z, s[0], 2, 2, 0);
+  s[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(q, k.w, s[1], 2, 3, 0);
+}
+// a[r] summed over the four quarters of a wavefront, r = 0 in the first to 3 in the last
+__device__ __forceinline__ float quarters_sum(v4f a) {
+  const auto sum32 = [](float x, float y) {
+    const auto t = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    return __uint_as_float(t[0]) + __uint_as_float(t[1]);
+  };
+  const float x = sum32(a[0], a[2]), y = sum32(a[1], a[3]);
+  const auto t = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+  return __uint_as_float(t[0]) + __uint_as_float(t[1]);
+}
+// values: + weight of four heads for key kKey, which block kKey holds, * the key's row, two dims a lane
+template <int kKey, int kSets>
+__device__ __forceinline__ void add_values(const float (&w)[kSets], const float2 (&v)[kPW], v4f (&acc)[kSets][2]) {
+  if constexpr (kKey < kPW) {
+#pragma unroll
+    for (int g = 0; g < kSets; ++g) {
+      acc[g][0] = __builtin_amdgcn_mfma_f32_4x4x1f32(w[g], v[kKey].x, acc[g][0], 4, kKey, 0);
+      acc[g][1] = __builtin_amdgcn_mfma_f32_4x4x1f32(w[g], v[kKey].y, acc[g][1], 4, kKey, 0);
+    }
+    add_values<kKey + 1, kSets>(w, v, acc);
+  }
+}
+
+template <int kWaves, int kSets>
 __global__ void __launch_bounds__(kWaves * 64)
     attn_decode_partial_group(const float *p_qkv, float *p_kcache, float *p_vcache,
                               const float *p_rope_table, const int *p_pos, int p_used,
-                              int p_max_len, int p_heads, int p_head_split, AttnArgs rest) {
+                              int p_max_len, int p_heads, AttnArgs rest) {
   AttnArgs a = rest; // the leading parameters arrive in SGPRs (see attn_decode_partial)
   a.qkv = p_qkv;
   a.kcache = p_kcache;
@@ -289,19 +326,16 @@ __global__ void __launch_bounds__(kWaves * 64)
   a.heads = p_heads & 0xfff;
   a.kv_heads = (p_heads >> 12) & 0xfff;
   a.group = p_heads >> 24;
-  a.head_split = p_head_split;
   constexpr int kChunk = kWaves * kPW;
-  constexpr int kR = kPW / 2;
-  __shared__ __attribute__((aligned(16))) float q_s[kMaxGroup][kD], knew_s[kD], vnew_s[kD];
+  static_assert(kPW == 16 && kD == 128 && kMaxGroup <= 8, "what sixteen blocks hold, and two sets of heads");
+  constexpr int kQ = kD + 16; // floats of a query's row: four heads' reads meet every bank once
+  __shared__ __attribute__((aligned(16))) float q_s[kMaxGroup + 1][kQ], knew_s[kD], vnew_s[kD];
   // what the wavefronts leave for the merge, every head of the group at once
   extern __shared__ __attribute__((aligned(16))) float accw_s[]; // [group][kWaves][kD]
   __shared__ float mw_s[kMaxGroup][kWaves], lw_s[kMaxGroup][kWaves];
 
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
-  // grid (pairs_padded, head_split): the workgroups that share a (chunk, KV head)
-  // pair have linear ids equal modulo 8 -- one XCD, one L2 for the pair's rows
-  const int hs = blockIdx.y;
   int chunk = blockIdx.x, kvh = 0;
   if (chunk >= a.used * a.kv_heads)
     return; // padding id
@@ -309,11 +343,8 @@ __global__ void __launch_bounds__(kWaves * 64)
     chunk -= a.used;
     ++kvh;
   }
-  // this workgroup's share of the group's query heads (head_split is 1 or 2)
-  const int per = (a.group + a.head_split - 1) >> (a.head_split - 1);
-  const int h_lo = hs * per, h_hi = min(a.group, h_lo + per);
   const int p0 = chunk * kChunk;
-  const int c4 = lane & 31, par = lane >> 5;
+  const int col = lane & 15, quarter = lane >> 4;
   const int pw0 = p0 + wave * kPW;
   // ---- small operands first: the queries of the group and the token's key, an
   // element and its rotation partner per thread and pass, with their angles ----
@@ -337,29 +368,26 @@ __global__ void __launch_bounds__(kWaves * 64)
       sn[u] = 0.f;
     }
   }
-  float4 kreg[kR], vreg[kR];
+  // A lane's keys and values as the products take them: of key `col` four dims of every sixteen,
+  // and dims 2 lane, 2 lane + 1 of every value
+  float4 kreg[kD / 16];
+  float2 vreg[kPW];
+  const float *krow = a.kcache + ((size_t)kvh * a.max_len + min(pw0 + col, a.max_len - 1)) * kD + quarter * 4;
 #pragma unroll
-  for (int i = 0; i < kR; ++i) {
-    const int row = min(pw0 + par + 2 * i, a.max_len - 1);
-    kreg[i] = *reinterpret_cast<const float4 *>(
-        a.kcache + ((size_t)kvh * a.max_len + row) * kD + c4 * 4);
-  }
+  for (int i = 0; i < kD / 16; ++i)
+    kreg[i] = *reinterpret_cast<const float4 *>(krow + 16 * i);
 #pragma unroll
-  for (int i = 0; i < kR; ++i) {
-    const int row = min(pw0 + par + 2 * i, a.max_len - 1);
-    vreg[i] = *reinterpret_cast<const float4 *>(
-        a.vcache + ((size_t)kvh * a.max_len + row) * kD + c4 * 4);
-  }
+  for (int j = 0; j < kPW; ++j)
+    vreg[j] = *reinterpret_cast<const float2 *>(
+        a.vcache + ((size_t)kvh * a.max_len + min(pw0 + j, a.max_len - 1)) * kD + lane * 2);
   const int pos_raw = *a.pos_ptr;
   const bool pos_ok = pos_raw >= 0 && pos_raw < a.max_len;
   const int pos = min(max(pos_raw, 0), a.max_len - 1);
   if (p0 > pos) { // nothing visible in this chunk: empty partials
-    for (int i = tid; i < (h_hi - h_lo) * kD; i += kWaves * 64) {
-      const int h = kvh * a.group + h_lo + i / kD;
-      a.part_acc[((size_t)h * a.nchunks + chunk) * kD + i % kD] = 0.f;
-    }
-    if (tid < h_hi - h_lo) {
-      const int h = kvh * a.group + h_lo + tid;
+    for (int i = tid; i < a.group * kD; i += kWaves * 64)
+      a.part_acc[((size_t)(kvh * a.group + i / kD) * a.nchunks + chunk) * kD + i % kD] = 0.f;
+    if (tid < a.group) {
+      const int h = kvh * a.group + tid;
       a.part_ml[((size_t)h * a.nchunks + chunk) * 2 + 0] = kSeedM;
       a.part_ml[((size_t)h * a.nchunks + chunk) * 2 + 1] = 0.f;
     }
@@ -375,12 +403,11 @@ __global__ void __launch_bounds__(kWaves * 64)
       if (!a.rope_table)
         sincosf(cs[u] * (float)pos, &sn[u], &cs[u]);
       const float rot = raw[u] * cs[u] + pair[u] * sn[u];
-      if (hh < a.group) {
-        q_s[hh][j] = rot;
-      } else if (has_new) {
+      q_s[hh][j] = hh < a.group ? rot : 0.f; // the row behind the queries: columns of no head
+      if (hh == a.group && has_new) {
         knew_s[j] = rot;
         vnew_s[j] = vraw[u];
-        if (pos_ok && hs == 0) { // one writer per cache row
+        if (pos_ok) {
           a.kcache[((size_t)kvh * a.max_len + pos) * kD + j] = rot;
           a.vcache[((size_t)kvh * a.max_len + pos) * kD + j] = vraw[u];
         }
@@ -388,87 +415,69 @@ __global__ void __launch_bounds__(kWaves * 64)
     }
   }
   __syncthreads();
-  // the token's own rows replace what the cache holds at its position
+  float qreg[kSets][kD / 16];
 #pragma unroll
-  for (int i = 0; i < kR; ++i)
-    if (pw0 + par + 2 * i == pos) {
-      kreg[i] = *reinterpret_cast<const float4 *>(knew_s + c4 * 4);
-      vreg[i] = *reinterpret_cast<const float4 *>(vnew_s + c4 * 4);
+  for (int g = 0; g < kSets; ++g)
+#pragma unroll
+    for (int i = 0; i < kD / 16; ++i)
+      qreg[g][i] = q_s[min(4 * g + (lane & 3), a.group)][16 * i + (lane >> 2)];
+  // the token's own rows replace what the cache holds at its position; rows beyond it may hold anything
+  const bool edge = pw0 + kPW > pos;
+  if (edge) {
+    if (pw0 + col == pos) {
+#pragma unroll
+      for (int i = 0; i < kD / 16; ++i)
+        kreg[i] = *reinterpret_cast<const float4 *>(knew_s + 16 * i + quarter * 4);
     }
-  // The launch is bound by its vector instructions at long contexts, and every
-  // chunk but the one the position lies in is visible whole: those run without the
-  // comparisons and selects of the mask.
-  auto heads_pass = [&](auto whole_chunk) {
-    constexpr bool kWhole = decltype(whole_chunk)::value;
-    for (int hh = h_lo; hh < h_hi; ++hh) {
-      const float4 q4 = *reinterpret_cast<const float4 *>(q_s[hh] + c4 * 4);
-      float d[kR];
 #pragma unroll
-      for (int i = 0; i < kR; ++i) {
-        const float4 k4 = kreg[i];
-        d[i] = fmaf(q4.x, k4.x, fmaf(q4.y, k4.y, fmaf(q4.z, k4.z, q4.w * k4.w)));
-      }
-      // The sums of eight keys over the 32 lanes of a half, halving the keys a lane still
-      // carries with each of three exchanges: lane l ends up with key key_of(l), so there is
-      // one exponential a lane and not eight (12000 positions: 11.4 -> 10.7 us).
-      static_assert(kR == 8, "three halvings");
-      const bool b3 = lane & 8, b2 = lane & 4, b1 = lane & 2;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        d[i] = (b3 ? d[2 * i + 1] : d[2 * i]) + dpp_f<0x140>(b3 ? d[2 * i] : d[2 * i + 1]); // lane ^ 15
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-        d[i] = (b2 ? d[2 * i + 1] : d[2 * i]) + dpp_f<0x141>(b2 ? d[2 * i] : d[2 * i + 1]); // lane ^ 7
-      float s = (b1 ? d[1] : d[0]) + dpp_f<0x4E>(b1 ? d[0] : d[1]);                         // lane ^ 2
-      s += dpp_f<0xB1>(s);                                                                  // lane ^ 1
-      s += __shfl_xor(s, 16, 64);
-      const int mine = pw0 + par + 2 * ((lane >> 3 & 1) + (lane >> 1 & 2) + (lane << 1 & 4));
-      s = kWhole || mine <= pos ? s * a.scale : -INFINITY;
-      // over the eight keys of the half, each once, and both halves
-      float m_w = fmaxf(s, dpp_f<0x140>(s));
-      m_w = fmaxf(m_w, dpp_f<0x141>(m_w));
-      m_w = fmaxf(m_w, dpp_f<0x4E>(m_w));
-      m_w = fmaxf(fmaxf(kSeedM, m_w), __shfl_xor(m_w, 32, 64));
-      s = fast_exp(s - m_w);
-      float l_w = s + dpp_f<0x140>(s);
-      l_w += dpp_f<0x141>(l_w);
-      l_w += dpp_f<0x4E>(l_w);
-      l_w += __shfl_xor(l_w, 32, 64);
-      // every lane of a row of 16 gets the weight of key i from lane 8 i0 + 4 i1 + 2 i2
-      float sc[kR] = {dpp_f<0x150>(s), dpp_f<0x158>(s), dpp_f<0x154>(s), dpp_f<0x15C>(s),
-                      dpp_f<0x152>(s), dpp_f<0x15A>(s), dpp_f<0x156>(s), dpp_f<0x15E>(s)};
-      float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-      for (int i = 0; i < kR; ++i) {
-        const int p = pw0 + par + 2 * i;
-        float4 v = vreg[i];
-        if (!kWhole && p > pos) // rows beyond the position may hold anything
-          v = make_float4(0.f, 0.f, 0.f, 0.f);
-        acc.x = fmaf(v.x, sc[i], acc.x);
-        acc.y = fmaf(v.y, sc[i], acc.y);
-        acc.z = fmaf(v.z, sc[i], acc.z);
-        acc.w = fmaf(v.w, sc[i], acc.w);
-      }
-      acc.x += __shfl_xor(acc.x, 32, 64);
-      acc.y += __shfl_xor(acc.y, 32, 64);
-      acc.z += __shfl_xor(acc.z, 32, 64);
-      acc.w += __shfl_xor(acc.w, 32, 64);
-      if (lane < 32)
-        *reinterpret_cast<float4 *>(&accw_s[((size_t)hh * kWaves + wave) * kD + c4 * 4]) = acc;
-      if (lane == 0) {
-        mw_s[hh][wave] = m_w;
-        lw_s[hh][wave] = l_w;
-      }
+    for (int j = 0; j < kPW; ++j) {
+      if (pw0 + j == pos)
+        vreg[j] = *reinterpret_cast<const float2 *>(vnew_s + lane * 2);
+      else if (pw0 + j > pos)
+        vreg[j] = make_float2(0.f, 0.f);
     }
-  };
-  if (p0 + kChunk - 1 <= pos)
-    heads_pass(std::true_type{});
-  else
-    heads_pass(std::false_type{});
+  }
+  // ---- scores: register r of a lane is key `col`'s with head r of the set, over the dims of its quarter ----
+  float w[kSets];
+  {
+    v4f s[kSets][2] = {};
+#pragma unroll
+    for (int i = 0; i < kD / 16; ++i)
+#pragma unroll
+      for (int g = 0; g < kSets; ++g)
+        add_scores(qreg[g][i], kreg[i], s[g]);
+#pragma unroll
+    for (int g = 0; g < kSets; ++g) {
+      const float d = quarters_sum(s[g][0] + s[g][1]); // now head `quarter` of the set
+      w[g] = !edge || pw0 + col <= pos ? d * a.scale : -INFINITY;
+    }
+  }
+  // ---- this wavefront's own max, exp and sum: sixteen keys in the lanes of a row ----
+#pragma unroll
+  for (int g = 0; g < kSets; ++g) {
+    const float m = row16_max(fmaxf(kSeedM, w[g])); // stays there when no position is visible
+    w[g] = fast_exp(w[g] - m);
+    const float l = row16_sum(w[g]);
+    if (col == 0 && 4 * g + quarter < a.group) {
+      mw_s[4 * g + quarter][wave] = m;
+      lw_s[4 * g + quarter][wave] = l;
+    }
+    // block k, the four lanes from 4 k on, takes the four heads' weights of key k
+    w[g] = __uint_as_float(__builtin_amdgcn_ds_bpermute(((lane & 3) * 16 + (lane >> 2)) * 4, __float_as_uint(w[g])));
+  }
+  v4f acc[kSets][2] = {};
+  add_values<0, kSets>(w, vreg, acc);
+#pragma unroll
+  for (int g = 0; g < kSets; ++g)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (4 * g + r < a.group)
+        *reinterpret_cast<float2 *>(&accw_s[((size_t)(4 * g + r) * kWaves + wave) * kD + lane * 2]) =
+            make_float2(acc[g][0][r], acc[g][1][r]);
   __syncthreads();
   // ---- the wavefronts meet, once for all heads: one partial per (head, chunk) --
-  for (int i = tid; i < (h_hi - h_lo) * kD; i += kWaves * 64) {
-    const int hh = h_lo + i / kD, d = i % kD, h = kvh * a.group + hh;
+  for (int i = tid; i < a.group * kD; i += kWaves * 64) {
+    const int hh = i / kD, d = i % kD, h = kvh * a.group + hh;
     float m = mw_s[hh][0];
 #pragma unroll
     for (int w = 1; w < kWaves; ++w)
@@ -513,32 +522,36 @@ __global__ void __launch_bounds__(kD) attn_decode_combine(AttnArgs a) {
 }
 
 // The same fold for a step far into a long cache, where one partial after the
-// other would take a trip to memory each: a workgroup of 32 x 32 threads per head,
-// thread (q, g) gathers d = 4 q .. 4 q + 3 of the chunks s = g, g + 32, ... with
+// other would take a trip to memory each: four workgroups of 64 x 8 threads per head, a quarter
+// of its dims each (one compute unit took more than a microsecond to take in a head's partials of
+// 12000 positions: 901 -> 866 us a step); thread (g, q) gathers four dims of the chunks s = g, g + 64, ... with
 // every load in flight at once, every wavefront works out the common maximum and
-// the weights exp(m_s - max m) for itself, and the 32 groups meet in LDS.  The
+// the weights exp(m_s - max m) for itself, and the 64 groups meet in registers and LDS.  The
 // sums are those of the chunk-by-chunk rule in another order.
 constexpr int kWideChunks = kAttnWideChunks; // partials per head it takes
+constexpr int kWideParts = 4, kWideThreads = 512;
 
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__(kWideThreads)
     attn_decode_combine_wide(const float *p_acc, const float *p_ml, float *p_out, int p_nchunks,
                              int p_used) { // (arguments preloaded into SGPRs)
-  constexpr int kPer = kWideChunks / 32; // chunks per thread at most
-  constexpr int kFast = 4;               // passes of 64 chunks whose (max, sum) pairs stay in registers
+  constexpr int kQuads = kD / 4 / kWideParts, kGroups = kWideThreads / kQuads, kWaves = kWideThreads / 64;
+  constexpr int kPer = kWideChunks / kGroups; // chunks per thread at most
+  constexpr int kFast = 4;                    // passes of 64 chunks whose (max, sum) pairs stay in registers
+  static_assert(kQuads == 8, "the exchanges below leave lanes equal modulo 8 with one sum");
   __shared__ float w_s[kWideChunks];
-  __shared__ __attribute__((aligned(16))) float4 red_s[32][32];
+  __shared__ __attribute__((aligned(16))) float4 red_s[kWaves][kQuads];
   const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
-  const int q = tid & 31, g = tid >> 5;
+  const int q = tid % kQuads, g = tid / kQuads, d0 = (blockIdx.y * kQuads + q) * 4;
   const int used = p_used;
   const float2 *ml = reinterpret_cast<const float2 *>(p_ml) + (size_t)h * p_nchunks;
-  const float *acc = p_acc + (size_t)h * p_nchunks * kD + q * 4;
+  const float *acc = p_acc + (size_t)h * p_nchunks * kD + d0;
   // the partial sums of this thread's first four chunks and the (max, sum) pairs
   // are requested together, before anything is known of the weights: one trip
   // (chunks past the last repeat it and are not added)
   float4 v[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
-    v[i] = *reinterpret_cast<const float4 *>(acc + (size_t)min(g + 32 * i, used - 1) * kD);
+    v[i] = *reinterpret_cast<const float4 *>(acc + (size_t)min(g + kGroups * i, used - 1) * kD);
   float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
   // the weights: every wavefront computes all of them (64 chunks per pass) and
   // wavefront 0 leaves them in LDS
@@ -550,39 +563,41 @@ __global__ void __launch_bounds__(1024)
       mine[p] = ml[min(64 * p + lane, used - 1)];
 #pragma unroll
     for (int p = 0; p < kFast; ++p)
-      m_all = fmaxf(m_all, wave_max(64 * p + lane < used ? mine[p].x : kSeedM));
+      m_all = fmaxf(m_all, 64 * p + lane < used ? mine[p].x : kSeedM);
+    m_all = wave_max(m_all);
 #pragma unroll
     for (int p = 0; p < kFast; ++p) {
       const bool in = 64 * p + lane < used;
       const float w = in ? fast_exp(mine[p].x - m_all) : 0.f;
-      l_all += wave_sum(mine[p].y * w);
+      l_all = fmaf(mine[p].y, w, l_all);
       if (tid < 64 && in)
         w_s[64 * p + lane] = w;
     }
   } else {
     for (int s0 = 0; s0 < used; s0 += 64)
-      m_all = fmaxf(m_all, wave_max(s0 + lane < used ? ml[s0 + lane].x : kSeedM));
+      m_all = fmaxf(m_all, s0 + lane < used ? ml[s0 + lane].x : kSeedM);
+    m_all = wave_max(m_all);
     for (int s0 = 0; s0 < used; s0 += 64) {
       const bool in = s0 + lane < used;
       const float2 mine = ml[min(s0 + lane, used - 1)];
       const float w = in ? fast_exp(mine.x - m_all) : 0.f;
-      l_all += wave_sum(mine.y * w);
+      l_all = fmaf(mine.y, w, l_all);
       if (tid < 64 && in)
         w_s[s0 + lane] = w;
     }
   }
   __syncthreads();
   for (int i0 = 0; i0 < kPer; i0 += 4) {
-    if (g + 32 * i0 >= used)
+    if (kGroups * i0 >= used)
       break;
     if (i0 > 0) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        v[i] = *reinterpret_cast<const float4 *>(acc + (size_t)min(g + 32 * (i0 + i), used - 1) * kD);
+        v[i] = *reinterpret_cast<const float4 *>(acc + (size_t)min(g + kGroups * (i0 + i), used - 1) * kD);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int c = g + 32 * (i0 + i);
+      const int c = g + kGroups * (i0 + i);
       if (c < used) {
         const float w = w_s[c];
         sum.x = fmaf(v[i].x, w, sum.x);
@@ -592,17 +607,26 @@ __global__ void __launch_bounds__(1024)
       }
     }
   }
-  red_s[g][q] = sum;
+  // the eight groups of a wavefront
+  auto meet = [](float x) {
+    x += dpp_f<0x128>(x); // lanes eight apart in a row of 16
+    x += __shfl_xor(x, 16, 64);
+    return x + __shfl_xor(x, 32, 64);
+  };
+  sum = make_float4(meet(sum.x), meet(sum.y), meet(sum.z), meet(sum.w));
+  l_all = wave_sum(l_all);
+  if (lane < kQuads)
+    red_s[tid >> 6][q] = sum;
   __syncthreads();
-  if (tid < 32) {
-    float4 o = red_s[0][tid];
-#pragma unroll 8
-    for (int gg = 1; gg < 32; ++gg) {
-      const float4 r = red_s[gg][tid];
+  if (tid < kQuads) {
+    float4 o = red_s[0][q];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) {
+      const float4 r = red_s[w][q];
       o.x += r.x; o.y += r.y; o.z += r.z; o.w += r.w;
     }
     const float inv = 1.0f / l_all;
-    *reinterpret_cast<float4 *>(p_out + (size_t)h * kD + tid * 4) =
+    *reinterpret_cast<float4 *>(p_out + (size_t)h * kD + d0) =
         make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
   }
 }
@@ -706,7 +730,6 @@ int launch_attn_decode(const AttnDecodeArgs &in, hipStream_t stream) {
   a.out = in.out;
   a.lse = in.lse;
   a.used = in.chunks_used > 0 ? std::min(in.chunks_used, a.nchunks) : a.nchunks;
-  a.head_split = 1;
   BH_REQUIRE(!in.combine || in.wide_combine || a.used == a.nchunks,
              "attn_decode: the combine pass needs a partial for every chunk");
   BH_REQUIRE(!in.wide_combine || (in.combine && !in.lse && a.used <= kWideChunks),
@@ -715,32 +738,27 @@ int launch_attn_decode(const AttnDecodeArgs &in, hipStream_t stream) {
   a.pairs_padded = (int)round_up((int64_t)a.used * in.kv_heads, 8);
   if (in.wide_combine) {
     // far into a long cache: one workgroup per (chunk, KV head) for all its heads
-    BH_REQUIRE(in.head_split == 1 || in.head_split == 2, "attn_decode: head_split %d",
-               in.head_split);
-    a.head_split = std::min(in.head_split, a.group); // a group of one head has nothing to share out
-    const dim3 grid(a.pairs_padded, a.head_split);
+    const dim3 grid(a.pairs_padded);
+    const int sets = a.group <= 4 ? 1 : 2;
     BH_REQUIRE(in.heads < 4096, "attn_decode: %d heads", in.heads);
     const int hp = pack_heads(a.heads, a.kv_heads, a.group);
     const size_t lds = sizeof(float) * (size_t)a.group * (in.chunk / kPW) * kD; // <= 64 KiB
     if (in.chunk == 64) {
-      hipLaunchKernelGGL(attn_decode_partial_group<4>, grid, dim3(4 * 64), lds, stream, a.qkv,
-                         a.kcache, a.vcache, a.rope_table, a.pos_ptr, a.used, a.max_len, hp,
-                         a.head_split, a);
+      hipLaunchKernelGGL((sets == 1 ? attn_decode_partial_group<4, 1> : attn_decode_partial_group<4, 2>), grid, dim3(4 * 64), lds, stream, a.qkv,
+                         a.kcache, a.vcache, a.rope_table, a.pos_ptr, a.used, a.max_len, hp, a);
     } else if (in.chunk == 128) {
-      hipLaunchKernelGGL(attn_decode_partial_group<8>, grid, dim3(8 * 64), lds, stream, a.qkv,
-                         a.kcache, a.vcache, a.rope_table, a.pos_ptr, a.used, a.max_len, hp,
-                         a.head_split, a);
+      hipLaunchKernelGGL((sets == 1 ? attn_decode_partial_group<8, 1> : attn_decode_partial_group<8, 2>), grid, dim3(8 * 64), lds, stream, a.qkv,
+                         a.kcache, a.vcache, a.rope_table, a.pos_ptr, a.used, a.max_len, hp, a);
     } else {
       // with 8 heads per KV head the 64 KiB of dynamic LDS come on top of 6 KiB
       static DynLdsOnce dyn_lds;
       BH_CHECK_HIP(ensure_dyn_lds(dyn_lds,
-                                  reinterpret_cast<const void *>(attn_decode_partial_group<16>),
+                                  reinterpret_cast<const void *>(attn_decode_partial_group<16, 2>),
                                   (int)(sizeof(float) * kMaxGroup * 16 * kD)));
-      hipLaunchKernelGGL(attn_decode_partial_group<16>, grid, dim3(16 * 64), lds, stream, a.qkv,
-                         a.kcache, a.vcache, a.rope_table, a.pos_ptr, a.used, a.max_len, hp,
-                         a.head_split, a);
+      hipLaunchKernelGGL((sets == 1 ? attn_decode_partial_group<16, 1> : attn_decode_partial_group<16, 2>), grid, dim3(16 * 64), lds, stream, a.qkv,
+                         a.kcache, a.vcache, a.rope_table, a.pos_ptr, a.used, a.max_len, hp, a);
     }
-    hipLaunchKernelGGL(attn_decode_combine_wide, dim3(in.heads), dim3(1024), 0, stream, a.part_acc,
+    hipLaunchKernelGGL(attn_decode_combine_wide, dim3(in.heads, kWideParts), dim3(kWideThreads), 0, stream, a.part_acc,
                        a.part_ml, a.out, a.nchunks, a.used);
     BH_CHECK_HIP(hipGetLastError());
     return BUDDY_HIP_OK;
@@ -758,7 +776,7 @@ int launch_attn_decode(const AttnDecodeArgs &in, hipStream_t stream) {
     hipLaunchKernelGGL(attn_decode_partial<16>, grid, dim3(16 * 64), 0, stream, a.qkv, a.kcache,
                        a.vcache, a.rope_table, a.pos_ptr, a.used, a.max_len, hp, 0, a);
   if (in.combine && in.wide_combine)
-    hipLaunchKernelGGL(attn_decode_combine_wide, dim3(in.heads), dim3(1024), 0, stream, a.part_acc,
+    hipLaunchKernelGGL(attn_decode_combine_wide, dim3(in.heads, kWideParts), dim3(kWideThreads), 0, stream, a.part_acc,
                        a.part_ml, a.out, a.nchunks, a.used);
   else if (in.combine)
     hipLaunchKernelGGL(attn_decode_combine, dim3(in.heads), dim3(kD), 0, stream, a);

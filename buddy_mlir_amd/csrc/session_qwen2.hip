@@ -182,7 +182,7 @@ struct Qwen2Session : Session {
   // into a long cache keeps the last few and lets the rest go.
   std::pair<int, int> step_key(int pos) const override {
     const AttnStepPlan plan = step_plan(pos);
-    return {plan.chunk * 4 + plan.head_split, plan.own_fold ? -plan.used : plan.used};
+    return {plan.chunk, plan.own_fold ? -plan.used : plan.used};
   }
 
   // Enqueues one decode step (reads token/pos from device state) with the cut
@@ -228,7 +228,6 @@ struct Qwen2Session : Session {
       a.wide_combine = own_fold;
       a.chunk = attn_chunk;
       a.chunks_used = attn_used;
-      a.head_split = plan.head_split;
       if ((rc = launch_attn_decode(a, stream)))
         return rc;
       if (own_fold) {

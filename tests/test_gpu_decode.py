@@ -466,6 +466,27 @@ def test_long_context_steps_for_every_size_of_head_group(oracle, heads, kv_heads
     sess.close()
 
 
+@pytest.mark.parametrize("heads,kv_heads,start", [(12, 2, 8186), (6, 1, 16378), (8, 1, 32762), (5, 1, 40000)])
+def test_cuts_of_long_contexts_with_two_sets_of_heads(oracle, heads, kv_heads, start):
+    """Groups of five to eight heads are multiplied as two sets of four: steps across the positions at which
+    their workgroups go from 4 to 8 and from 8 to 16 wavefronts, and behind them."""
+    shape = Shape(layers=1, hidden=256, heads=heads, kv_heads=kv_heads, head_dim=128, inter=256,
+                  vocab=512, max_len=start + 64, rms_eps=1e-6)
+    sess, host = synthetic.build_session(shape, context=start, keep_host=True, ln_jitter=0.1)
+    om = oracle_model(oracle, shape, host)
+    kv = [a.copy() for a in host["kv"]]
+    tok = 3
+    for step in range(10):
+        nxt, logits = sess.decode(tok, start + step)
+        otok, ologits = om.decode_step(tok, start + step, kv)
+        check_close(logits, ologits)
+        assert nxt == otok
+        tok = otok
+    for j in range(2):
+        check_close(sess.get_kv(j)[:, start:start + 10, :], kv[j][:, start:start + 10, :])
+    sess.close()
+
+
 @pytest.mark.parametrize("start", [17000, 66000])
 def test_fold_of_more_partials_than_one_pass_takes(oracle, start):
     """The launch that folds the partials far into a long cache takes 128 of them
