@@ -139,22 +139,28 @@ argmax_final_kernel(const float *__restrict__ pv, const int *__restrict__ pi,
 // its embedding row and the cos/sin table of its position (shared by every
 // layer's attention kernel).  One workgroup.
 // Table: f32 rows as they are, or bfloat16 rows times a scale or normed.
+// What bounds it is its chain of trips to memory: the state and the candidates in one, the row in one more (the
+// norm's weights come beside the first), and the wavefronts meet in the lanes of each.  1536 values: a row read
+// value after value by 256 threads, twice where it is normed, and wavefronts met one after the other took 5.8 us,
+// normed 7.6, with 9496 candidates 6.5; so 4.1, 5.4 and 4.8.
+constexpr int kFinishThreads = 1024, kFinishWaves = kFinishThreads / 64;
 template <typename Table>
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__(kFinishThreads)
 finish_step_kernel(const float *__restrict__ pv, const int *__restrict__ pi,
                    int nparts, int *__restrict__ state, int *__restrict__ token_log,
                    const Table *__restrict__ table, float table_scale, int64_t hidden,
                    int64_t vocab, float *__restrict__ x, const float *__restrict__ inv_freq,
                    int half, float *__restrict__ rope, int advance, int log_cap,
                    const float *__restrict__ norm_w, float eps, StepGiven given) {
-  __shared__ float sv[16];
-  __shared__ int si[16];
+  static_assert(kFinishWaves == 16, "the wavefronts meet in the lanes of a row");
+  __shared__ float sv[kFinishWaves], ssum[kFinishWaves];
+  __shared__ int si[kFinishWaves];
   __shared__ int s_tok, s_pos;
-  const int threads = blockDim.x; // 256, or 1024 for thousands of candidates
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // token, position and step count: asked for with the first loads, not behind
   // the pick (only thread 0 uses them)
   int st_tok = 0, st_pos = 0, st_step = 0;
-  if (threadIdx.x == 0) {
+  if (tid == 0) {
     if (given.token >= 0 || given.at) {
       state[0] = st_tok = given.at ? given.at[0] : given.token;
       state[1] = st_pos = given.at ? given.at[1] : given.pos;
@@ -165,47 +171,60 @@ finish_step_kernel(const float *__restrict__ pv, const int *__restrict__ pi,
       st_step = state[2];
     }
   }
+  constexpr int kRow = 4; // values of the row a thread has in flight
+  float nw[kRow];
+  if (norm_w) {
+#pragma unroll
+    for (int j = 0; j < kRow; ++j)
+      nw[j] = norm_w[min((int64_t)tid + j * kFinishThreads, hidden - 1)];
+  }
+  const float freq = tid < half ? inv_freq[tid] : 0.f;
   if (nparts > 0) {
     float v = -INFINITY;
     int idx = 0x7fffffff;
     // ten candidates per thread in flight at once: the 9496 group maxima of a
     // 151936-word vocabulary cost 1024 threads one trip to memory, not three
     constexpr int kInFlight = 10;
-    for (int i0 = threadIdx.x; i0 < nparts; i0 += kInFlight * threads) {
+    for (int i0 = tid; i0 < nparts; i0 += kInFlight * kFinishThreads) {
       float cv[kInFlight];
       int ci[kInFlight];
 #pragma unroll
       for (int j = 0; j < kInFlight; ++j) {
-        const int i = min(i0 + j * threads, nparts - 1);
+        const int i = min(i0 + j * kFinishThreads, nparts - 1);
         cv[j] = pv[i];
         ci[j] = pi[i];
       }
 #pragma unroll
       for (int j = 0; j < kInFlight; ++j)
-        if (i0 + j * threads < nparts)
+        if (i0 + j * kFinishThreads < nparts)
           amax_merge(v, idx, cv[j], ci[j]);
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1)
       amax_merge(v, idx, __shfl_xor(v, o, 64), __shfl_xor(idx, o, 64));
-    if ((threadIdx.x & 63) == 0) {
-      sv[threadIdx.x >> 6] = v;
-      si[threadIdx.x >> 6] = idx;
+    if (lane == 0) {
+      sv[wave] = v;
+      si[wave] = idx;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-      for (int w = 1; w < threads / 64; ++w)
-        amax_merge(v, idx, sv[w], si[w]);
+    if (wave == 0) {
+      v = sv[lane & 15];
+      idx = si[lane & 15];
+#pragma unroll
+      for (int o = 8; o > 0; o >>= 1)
+        amax_merge(v, idx, __shfl_xor(v, o, 64), __shfl_xor(idx, o, 64));
       if (idx == 0x7fffffff)
         idx = 0;
-      // the host bounds the step count; a counter outside the log writes nothing
-      if ((unsigned)st_step < (unsigned)log_cap)
-        token_log[st_step] = idx;
-      state[0] = idx;
-      st_tok = idx;
+      if (lane == 0) {
+        // the host bounds the step count; a counter outside the log writes nothing
+        if ((unsigned)st_step < (unsigned)log_cap)
+          token_log[st_step] = idx;
+        state[0] = idx;
+        st_tok = idx;
+      }
     }
   }
-  if (threadIdx.x == 0) {
+  if (tid == 0) {
     if (advance) {
       st_pos += 1;
       st_step += 1;
@@ -220,39 +239,49 @@ finish_step_kernel(const float *__restrict__ pv, const int *__restrict__ pi,
   if (t < 0 || t >= vocab)
     t = 0;
   const Table *row = table + t * hidden;
-  float gain = table_scale;
-  if constexpr (sizeof(Table) == 2) {
-    if (norm_w) {
-      float ss = 0.f;
-      for (int64_t i = threadIdx.x; i < hidden; i += threads) {
-        const float v = __uint_as_float((unsigned)row[i] << 16);
-        ss = fmaf(v, v, ss);
-      }
-      ss = wave_sum(ss);
-      __syncthreads(); // the candidates have been read
-      if ((threadIdx.x & 63) == 0)
-        sv[threadIdx.x >> 6] = ss;
-      __syncthreads();
-      ss = 0.f;
-      for (int w = 0; w < threads / 64; ++w)
-        ss += sv[w];
-      gain = 1.0f / sqrtf(ss / (float)hidden + eps);
-    }
-  }
-  for (int64_t i = threadIdx.x; i < hidden; i += threads) {
+  const auto value = [&](Table v) {
     if constexpr (sizeof(Table) == 4)
-      x[i] = row[i];
-    else if (norm_w)
-      x[i] = __uint_as_float((unsigned)row[i] << 16) * gain * norm_w[i];
+      return v;
     else
-      x[i] = __uint_as_float((unsigned)row[i] << 16) * table_scale;
-  }
-  if (threadIdx.x < half) {
+      return __uint_as_float((unsigned)v << 16);
+  };
+  Table rv[kRow];
+#pragma unroll
+  for (int j = 0; j < kRow; ++j)
+    rv[j] = row[min((int64_t)tid + j * kFinishThreads, hidden - 1)];
+  if (tid < half) { // while the row is on its way
     float sn, cs;
-    sincosf(inv_freq[threadIdx.x] * (float)s_pos, &sn, &cs);
-    rope[threadIdx.x] = cs;
-    rope[half + threadIdx.x] = sn;
+    sincosf(freq * (float)s_pos, &sn, &cs);
+    rope[tid] = cs;
+    rope[half + tid] = sn;
   }
+  float gain = sizeof(Table) == 4 ? 1.0f : table_scale;
+  if (norm_w) {
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < kRow; ++j) {
+      const float v = (int64_t)tid + j * kFinishThreads < hidden ? value(rv[j]) : 0.f;
+      ss = fmaf(v, v, ss);
+    }
+    for (int64_t i = tid + kRow * kFinishThreads; i < hidden; i += kFinishThreads) {
+      const float v = value(row[i]);
+      ss = fmaf(v, v, ss);
+    }
+    ss = wave_sum(ss);
+    if (lane == 0)
+      ssum[wave] = ss;
+    __syncthreads();
+    ss = row16_sum(ssum[lane & 15]);
+    gain = 1.0f / sqrtf(ss / (float)hidden + eps);
+  }
+#pragma unroll
+  for (int j = 0; j < kRow; ++j) {
+    const int64_t i = (int64_t)tid + j * kFinishThreads;
+    if (i < hidden)
+      x[i] = norm_w ? value(rv[j]) * gain * nw[j] : value(rv[j]) * gain;
+  }
+  for (int64_t i = tid + kRow * kFinishThreads; i < hidden; i += kFinishThreads)
+    x[i] = norm_w ? value(row[i]) * gain * norm_w[i] : value(row[i]) * gain;
 }
 
 } // namespace
@@ -264,7 +293,7 @@ int launch_finish_step(const float *cand_v, const int *cand_i, int nparts, int *
   BH_REQUIRE(state && table && x && inv_freq && rope && head_dim > 0 &&
                  head_dim / 2 <= 256 && (nparts == 0 || (cand_v && cand_i && token_log && !given.any())),
              "finish_step: bad argument");
-  hipLaunchKernelGGL(finish_step_kernel<float>, dim3(1), dim3(nparts > 1024 ? 1024 : 256), 0,
+  hipLaunchKernelGGL(finish_step_kernel<float>, dim3(1), dim3(kFinishThreads), 0,
                      stream, cand_v, cand_i, nparts, state, token_log, table, 1.0f, hidden, vocab,
                      x, inv_freq, head_dim / 2, rope, advance ? 1 : 0, token_log_cap,
                      (const float *)nullptr, 0.f, given);
@@ -278,7 +307,7 @@ int launch_finish_step_bf16(const float *cand_v, const int *cand_i, int nparts, 
                             bool advance, int token_log_cap, hipStream_t stream, StepGiven given) {
   BH_REQUIRE(state && table && x && (nparts == 0 || (cand_v && cand_i && token_log && !given.any())),
              "finish_step: bad argument");
-  hipLaunchKernelGGL(finish_step_kernel<uint16_t>, dim3(1), dim3(nparts > 1024 ? 1024 : 256), 0,
+  hipLaunchKernelGGL(finish_step_kernel<uint16_t>, dim3(1), dim3(kFinishThreads), 0,
                      stream, cand_v, cand_i, nparts, state, token_log, table, table_scale, hidden,
                      vocab, x, (const float *)nullptr, 0, (float *)nullptr, advance ? 1 : 0,
                      token_log_cap, norm_w, eps, given);
