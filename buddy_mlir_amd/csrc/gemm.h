@@ -14,6 +14,7 @@ struct PromptTerms {
 };
 struct RopeKv {
   const float *inv_freq = nullptr; // [64]
+  const float *turns = nullptr;    // [token][cos of 64 | sin of 64], or none
   float *kcache = nullptr, *vcache = nullptr;
   int heads = 0, kv_heads = 0, max_len = 0, start_pos = 0;
   PromptTerms terms;

@@ -309,6 +309,7 @@ struct GemmI8Args {
   int accumulate;
   int32_t *sums;      // one plane only: the int32 sums themselves, dense [M, N], or null
   int int_partials;   // one plane, K split: the slices leave their int32 sums as they are
+  RopeKv rope;        // of q | k | v that the product itself rotates
 };
 
 // The finished value of one output.  One plane is the w8a8 matmul, whose result
@@ -369,8 +370,100 @@ __device__ __forceinline__ float4 int_bits(const v16i32 &acc, int q) {
 constexpr int turn_floats(int span) { return span + 4; } // of a row of the epilogue's tile
 constexpr int turned_bytes(int span) { return kSlices * 32 * turn_floats(span) * 4; }
 
+// What follows q | k | v, for a tile whose finished values lie in LDS (32 rows of 4 x `kSpan` channels, whole
+// heads): sixteen lanes take a head's row, four channels and their partners each, rotate it by angles that
+// the prompt has as a table, and store queries to C, keys and values to the cache and, of a prompt alone, as
+// terms; a tile of terms is these 32 rows.  A launch for it was 5.6 us behind 512 tokens' product and 10.1
+// behind 1931's, most of which were its own and two more trips of the values; here 1 and 2.
+template <int GP>
+__device__ __forceinline__ void rotate_tile(const GemmI8Args &a, unsigned char *lds, int ctile, int m0) {
+  constexpr int kSpan = 32 * GP, kTurn = turn_floats(kSpan), kHalf = kAttnHeadDim / 2, kPasses = 2 * GP;
+  constexpr int kKeys = kTileKeys + 2; // of a channel in LDS: sixteen lanes' stores meet sixteen banks
+  static_assert(kAttnHeadDim == 4 * 32 && 2 * kAttnHeadDim * kKeys * 2 <= turned_bytes(32), "a head a channel tile");
+  const int tid = threadIdx.x, j = tid % 16 * 4;
+  const RopeKv &r = a.rope;
+  float lo[kPasses][4], hi[kPasses][4];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kPasses; ++i) { // pass i: rows 16 (i % 2) + 0..15 of head i / 2
+    const int row = i % 2 * 16 + tid / 16;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int ch = i / 2 * kAttnHeadDim + h * kHalf + j;
+      const float4 v = *reinterpret_cast<const float4 *>(
+          reinterpret_cast<const float *>(lds) + (ch / kSpan * 32 + row) * kTurn + ch % kSpan);
+      float *to = h ? hi[i] : lo[i];
+      to[0] = v.x; to[1] = v.y; to[2] = v.z; to[3] = v.w;
+    }
+  }
+  __syncthreads(); // the values have been read: LDS is free
+  auto store = [&](float *dst, const float (&l)[4], const float (&h)[4]) {
+    *reinterpret_cast<float4 *>(dst) = make_float4(l[0], l[1], l[2], l[3]);
+    *reinterpret_cast<float4 *>(dst + kHalf) = make_float4(h[0], h[1], h[2], h[3]);
+  };
+  unsigned short(*vt)[kAttnHeadDim][kKeys] = reinterpret_cast<unsigned short(*)[kAttnHeadDim][kKeys]>(lds);
+#pragma unroll
+  for (int i = 0; i < kPasses; ++i) {
+    const int head = ctile * GP + i / 2, row = i % 2 * 16 + tid / 16, m = m0 + row, pos = r.start_pos + m;
+    if (head * kAttnHeadDim >= a.N)
+      break;
+    const bool is = m < a.M;
+    if (head < r.heads + r.kv_heads) {
+      if (!is)
+        continue;
+      const float *turns = r.turns + (int64_t)m * kAttnHeadDim + j;
+      const float4 c4 = *reinterpret_cast<const float4 *>(turns), s4 = *reinterpret_cast<const float4 *>(turns + kHalf);
+      const float c[4] = {c4.x, c4.y, c4.z, c4.w}, s[4] = {s4.x, s4.y, s4.z, s4.w};
+      float nlo[4], nhi[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        nlo[e] = lo[i][e] * c[e] + (-hi[i][e]) * s[e];
+        nhi[e] = hi[i][e] * c[e] + lo[i][e] * s[e];
+      }
+      if (head < r.heads) {
+        store(a.C + (int64_t)m * a.ldc + head * kAttnHeadDim + j, nlo, nhi);
+      } else {
+        const int kvh = head - r.heads;
+        store(r.kcache + ((int64_t)kvh * r.max_len + pos) * kAttnHeadDim + j, nlo, nhi);
+        if (r.terms.tiles)
+          put_key_terms(r.terms, kvh, pos, j / 4, nlo, nhi);
+      }
+      continue;
+    }
+    const int kvh = head - r.heads - r.kv_heads;
+    if (is)
+      store(r.vcache + ((int64_t)kvh * r.max_len + pos) * kAttnHeadDim + j, lo[i], hi[i]);
+    if (!r.terms.tiles)
+      continue;
+    uint4 term[2] = {}; // of rows behind the prompt: numbers
+    if (is)
+      value_terms(r.terms, kvh, pos, j / 4, lo[i], hi[i], term);
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const unsigned w[4] = {term[p].x, term[p].y, term[p].z, term[p].w};
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        vt[p][kHalf * (e / 4) + j + e % 4][row] = (unsigned short)(e & 1 ? w[e / 2] >> 16 : w[e / 2]);
+    }
+    if (i % 2 == 0)
+      continue;
+    __syncthreads();
+    // sixteen bytes are keys 16 s + 4 half + 0..3 and the four 8 behind them, of a channel
+    unsigned char *tile = terms_tile(r.terms, kvh, r.start_pos + m0);
+#pragma unroll
+    for (int u = 0; u < 2 * 4 * kAttnHeadDim / 256; ++u) {
+      const int id = u * 256 + tid, c = id % kAttnHeadDim, key = id / kAttnHeadDim % 4 * 4, p = id / (4 * kAttnHeadDim);
+      const int first = key / 8 * 16 + key % 8;
+      const unsigned *from = reinterpret_cast<const unsigned *>(&vt[p][c][first]);
+      *reinterpret_cast<uint4 *>(value_term_at(tile, first, c, p)) = uint4{from[0], from[1], from[4], from[5]};
+    }
+    if (i + 1 < kPasses)
+      __syncthreads();
+  }
+}
+
 // The way of a tile's sums out, behind the last barrier of the loop over K (`lds` is free).
-template <int D, int RB, int GP, bool PAIR>
+template <int D, int RB, int GP, bool PAIR, bool ROPE = false>
 __device__ __forceinline__ void finish_tile(const GemmI8Args &a, const v16i32 (&acc)[GP][RB][D], unsigned char *lds,
                                             const float *scale_s, const float *bias_s, const float *step_s,
                                             int ctile, int rbk, int slice, int g0, int m0, int wave, int lane) {
@@ -446,6 +539,11 @@ __device__ __forceinline__ void finish_tile(const GemmI8Args &a, const v16i32 (&
         }
         turn_in(g, q, make_float4(o[0], o[1], o[2], o[3]));
       }
+    if constexpr (ROPE) {
+      static_assert(RB == 1 && !PAIR, "the rows of a tile of terms");
+      rotate_tile<GP>(a, lds, ctile, m0);
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < kQuads / 2; ++i) {
       const int idx = lane + 64 * i, row = idx / kQuads, c4 = idx % kQuads;
@@ -501,7 +599,7 @@ __device__ __forceinline__ void finish_tile(const GemmI8Args &a, const v16i32 (&
   }
 }
 
-template <int D, int RB, int GP, bool PAIR>
+template <int D, int RB, int GP, bool PAIR, bool ROPE = false>
 __device__ __forceinline__ void multiply_tile(const GemmI8Args &a, int unit, int rbk, int row0 = 0) {
   constexpr int kWidth = PAIR ? 16 : 32;    // channels of the result per tile
   constexpr int kSpan = kWidth * GP;        // ... and per wavefront
@@ -699,7 +797,7 @@ __device__ __forceinline__ void multiply_tile(const GemmI8Args &a, int unit, int
     }
   }
 
-  finish_tile<D, RB, GP, PAIR>(a, acc, lds, scale_s, bias_s, step_s, ctile, rbk, slice, g0, m0, wave, lane);
+  finish_tile<D, RB, GP, PAIR, ROPE>(a, acc, lds, scale_s, bias_s, step_s, ctile, rbk, slice, g0, m0, wave, lane);
 }
 
 // The same product for tiles of many sums, two workgroups to a compute unit: two wavefronts on a
@@ -888,21 +986,21 @@ __device__ __forceinline__ void multiply_block(const GemmI8Args &a, int unit, in
   a.panel = panel;
 
 // 32 rows x 128 channels per workgroup; 256 channels; the others of kTiles
-template <int D, bool PAIR>
+template <int D, bool PAIR, bool ROPE = false>
 __global__ void __launch_bounds__(kSlices *kWave) gemm_w8_i8_kernel(BH_I8_LEADING) {
   BH_I8_TAKE
   int unit, rbk;
   if (!place_tile(a.ncols * a.slices, a.row_tiles, a.panel, unit, rbk))
     return;
-  multiply_tile<D, 1, 1, PAIR>(a, unit, rbk);
+  multiply_tile<D, 1, 1, PAIR, ROPE>(a, unit, rbk);
 }
-template <int D, bool PAIR>
-__global__ void __launch_bounds__(kSlices *kWave) gemm_w8_i8_wide_kernel(BH_I8_LEADING) {
+template <int D, bool PAIR, bool ROPE = false>
+__global__ void __launch_bounds__(kSlices *kWave, ROPE ? 2 : 1) gemm_w8_i8_wide_kernel(BH_I8_LEADING) {
   BH_I8_TAKE
   int unit, rbk;
   if (!place_tile(a.ncols * a.slices, a.row_tiles, a.panel, unit, rbk))
     return;
-  multiply_tile<D, wide_blocks(D), 2, PAIR>(a, unit, rbk);
+  multiply_tile<D, wide_blocks(D), 2, PAIR, ROPE>(a, unit, rbk);
 }
 template <int D, int RB, int GP, bool PAIR>
 __global__ void __launch_bounds__(kSlices *kWave, tall_shares(D, GP) ? 2 : 1)
@@ -1316,6 +1414,7 @@ BH_VARIANT_FAMILY(NarrowFamily, "gemm_w8_i8_kernel");
 BH_TILE_FAMILY(NarrowPairFamily, "gemm_w8_i8_kernel pair");
 BH_TILE_FAMILY(TallFamily, "gemm_w8_i8_tall_kernel");
 BH_TILE_FAMILY(TailedFamily, "gemm_w8_i8_tailed_kernel");
+BH_TILE_FAMILY(RotatesFamily, "gemm_w8_i8 rotates"); // planes, channel tiles per wavefront
 
 template <class Kernel>
 int launch_tiles(Kernel kernel, const GemmI8Args &a, unsigned blocks, hipStream_t stream) {
@@ -1583,6 +1682,11 @@ TilePlan plan_tiles(int64_t M, int64_t channels, int chunks, bool may_split, dou
   return best;
 }
 
+// Whether the product rotates q | k | v itself: tiles of 32 rows and whole heads with K whole.
+bool rotates(const TilePlan &plan, const GemmI8Args &a) {
+  return a.rope.turns && plan.slices == 1 && !plan.tail && plan.rb == 1 && plan.gp <= 2;
+}
+
 // a.partial stays null where K was to be split and no workspace could be had: the caller
 // comes back with a plan that leaves K whole.
 template <int D, bool PAIR>
@@ -1610,6 +1714,16 @@ int launch_plan(const TilePlan &plan, GemmI8Args &a, hipStream_t stream) {
   const int64_t tiles = (a.panel ? units : round_up(units, 8)) * a.row_tiles;
   BH_REQUIRE(tiles < (1u << 31), "gemm_w8: %lld tiles", (long long)tiles);
   const unsigned blocks = (unsigned)tiles;
+  if constexpr (D > 1 && !PAIR) {
+    if (rotates(plan, a)) {
+      if (plan.gp == 1) {
+        BH_NOTE_VARIANT(RotatesFamily, D, 1);
+        return launch_tiles(gemm_w8_i8_kernel<D, false, true>, a, blocks, stream);
+      }
+      BH_NOTE_VARIANT(RotatesFamily, D, 2);
+      return launch_tiles(gemm_w8_i8_wide_kernel<D, false, true>, a, blocks, stream);
+    }
+  }
   if (plan.tail)
     return launch_tailed(a, blocks, stream);
   if (plan.gp == 1)
@@ -1740,13 +1854,21 @@ int launch_gemm_w8_digits_d(const GemmW8Args &in, const void *planes, hipStream_
     a.N = (int)(in.N / 2);
     return launch_plan<D, true>(plan_tiles<D, true>(in.M, a.N, a.chunks, false, 0.0, 0.0, 0), a, stream);
   }
+  if (in.then_rope && in.then_rope->turns && !in.accumulate && in.ldc % 4 == 0 &&
+      in.N == (int64_t)(in.then_rope->heads + 2 * in.then_rope->kv_heads) * kAttnHeadDim &&
+      ((reinterpret_cast<uintptr_t>(in.C) | reinterpret_cast<uintptr_t>(in.then_rope->turns) |
+        reinterpret_cast<uintptr_t>(in.then_rope->kcache) | reinterpret_cast<uintptr_t>(in.then_rope->vcache)) & 15) == 0)
+    a.rope = *in.then_rope;
   // A norm that is to follow (then_norm_w) costs a launch of its own, about
   // 5 us, unless the kernel that adds K slices writes its planes (it holds whole
   // rows, up to kRowCache columns).
   const bool slices_fuse_norm = gemm_staging_layout(in.M, in.N).cols_padded <= kRowCache;
   // The rotation behind q | k | v likewise: 4 us, in the kernel that adds slices 0.5 and what the
-  // angles take, which every head works out for itself there.
-  const double norm_us = in.then_norm_w ? 5.0 : in.then_rope ? 4.0 : 0.0;
+  // angles take, which every head works out for itself there.  In the product itself (see `rotates`) it
+  // takes one or two; what is said here is where prompts become shorter with K whole (three planes, 64 tokens
+  // 1771 and 1765 us, 128 2157 and 2120, 160 2321 and 2242; two, 128 2057 and 1985).
+  const double turn_us = !a.rope.turns ? 4.0 : D == 3 ? 2.9 : 3.3;
+  const double norm_us = in.then_norm_w ? 5.0 : in.then_rope ? turn_us : 0.0;
   const double split_norm_us = in.then_rope ? 0.5 + 0.004 * (double)in.M : slices_fuse_norm ? 0.0 : norm_us;
   TilePlan plan = plan_tiles<D, false>(in.M, in.N, a.chunks, true, norm_us, split_norm_us, 0);
   if (int rc = launch_plan<D, false>(plan, a, stream))
@@ -1757,7 +1879,7 @@ int launch_gemm_w8_digits_d(const GemmW8Args &in, const void *planes, hipStream_
       return rc;
   }
   if (plan.slices == 1)
-    return norm_behind(in, stream);
+    return rotates(plan, a) ? BUDDY_HIP_OK : norm_behind(in, stream);
   return add_slices(in, a, stream);
 }
 } // namespace

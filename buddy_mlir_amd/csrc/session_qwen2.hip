@@ -72,10 +72,11 @@ struct Layer {
   bool set = false;
 };
 
-// x[t, :] = table[token[t], :]
+// x[t, :] = table[token[t], :], and cos | sin of the token's angles for the layers' rotations
 __global__ void __launch_bounds__(256)
 embedding_rows_kernel(const float *__restrict__ table, const int *__restrict__ tokens,
-                      int64_t hidden, int64_t vocab, float *__restrict__ out) {
+                      int64_t hidden, int64_t vocab, float *__restrict__ out,
+                      const float *__restrict__ inv_freq, int half, int start_pos, float *__restrict__ turns) {
   int64_t t = tokens[blockIdx.x];
   if (t < 0 || t >= vocab)
     t = 0;
@@ -83,6 +84,10 @@ embedding_rows_kernel(const float *__restrict__ table, const int *__restrict__ t
   float *dst = out + (int64_t)blockIdx.x * hidden;
   for (int64_t i = threadIdx.x; i < hidden; i += 256)
     dst[i] = row[i];
+  for (int i = threadIdx.x; i < half; i += 256) {
+    float *turn = turns + (int64_t)blockIdx.x * 2 * half + i;
+    sincosf(inv_freq[i] * (float)(start_pos + (int)blockIdx.x), turn + half, turn);
+  }
 }
 
 } // namespace
@@ -108,6 +113,7 @@ struct Qwen2Session : Session {
   size_t kv_rows_cap = 0;
   unsigned short *pf_xn_bf = nullptr, *pf_g_bf = nullptr; // bf16 matmul inputs
   void *pf_attn_ws = nullptr;          // partial results of the attention
+  float *pf_turns = nullptr;           // angles of a prompt's rotation (RopeKv::turns)
   unsigned char *pf_terms = nullptr;   // keys and values of a prompt alone as terms
   unsigned short *pf_att_dg = nullptr; // digit planes or terms of the attention output (o_proj's input)
   int gemm_terms = 3; // bf16 terms per activation in the prefill matmuls (3 = exact)
@@ -310,7 +316,7 @@ struct Qwen2Session : Session {
       return BUDDY_HIP_OK;
     const auto &S = shape;
     const size_t QN = (size_t)S.heads * S.head_dim, KVN = (size_t)S.kv_heads * S.head_dim;
-    for (float **p : {&pf_x, &pf_xn, &pf_qkv, &pf_att, &pf_g})
+    for (float **p : {&pf_x, &pf_xn, &pf_qkv, &pf_att, &pf_g, &pf_turns})
       if (*p) {
         (void)hipFree(*p);
         *p = nullptr;
@@ -337,6 +343,7 @@ struct Qwen2Session : Session {
     BH_CHECK_HIP(hipMalloc((void **)&pf_xn, sizeof(float) * rows * S.hidden));
     BH_CHECK_HIP(hipMalloc((void **)&pf_qkv, sizeof(float) * rows * (QN + 2 * KVN)));
     BH_CHECK_HIP(hipMalloc((void **)&pf_att, sizeof(float) * rows * QN));
+    BH_CHECK_HIP(hipMalloc((void **)&pf_turns, sizeof(float) * rows * S.head_dim));
     // gate | up side by side: rows of 2 * inter floats
     BH_CHECK_HIP(hipMalloc((void **)&pf_g, sizeof(float) * rows * 2 * S.inter));
     pf_u = pf_g + S.inter;
@@ -481,7 +488,8 @@ struct Qwen2Session : Session {
     const int64_t QKV = (int64_t)(S.heads + 2 * S.kv_heads) * S.head_dim;
     const float scale = (float)(1.0 / std::sqrt((double)S.head_dim));
     hipLaunchKernelGGL(embedding_rows_kernel, dim3(n), dim3(256), 0, stream, embed,
-                       pf_tokens, (int64_t)S.hidden, (int64_t)S.vocab, pf_x);
+                       pf_tokens, (int64_t)S.hidden, (int64_t)S.vocab, pf_x, inv_freq, S.head_dim / 2,
+                       start_pos, pf_turns);
     BH_CHECK_HIP(hipGetLastError());
     int rc;
     const bool few = few_tokens(n);
@@ -501,6 +509,7 @@ struct Qwen2Session : Session {
       Layer &L = layers[(size_t)i];
       RopeKv rope;
       rope.inv_freq = inv_freq;
+      rope.turns = pf_turns;
       rope.kcache = L.kc;
       rope.vcache = L.vc;
       rope.heads = S.heads;
@@ -717,7 +726,7 @@ struct Qwen2Session : Session {
       (void)hipStreamSynchronize(stream);
     for (void *p : {(void *)pf_x, (void *)pf_xn, (void *)pf_qkv, (void *)pf_att, (void *)pf_g,
                     (void *)pf_tokens, (void *)kv_rows, (void *)pf_xn_bf, (void *)pf_g_bf,
-                    (void *)pf_att_dg, (void *)pf_terms, pf_attn_ws})
+                    (void *)pf_att_dg, (void *)pf_terms, (void *)pf_turns, pf_attn_ws})
       if (p)
         (void)hipFree(p);
     release_gemm_staging(stream);

@@ -575,6 +575,40 @@ def test_rotation_behind_qkv(bh, hidden, heads, kv_heads, before, n, trips, prec
     sess.close()
 
 
+# the rotation within q | k | v's product: tiles of one head and of two, of which one may be queries and one
+# keys, or keys and values, or the last alone; part of a tile of 32 rows, whole ones, one row more; alone,
+# where keys and values leave as terms too, and behind a context
+@pytest.mark.parametrize("precision", ["digits", "digits2"])
+@pytest.mark.parametrize("heads,kv_heads,before,n,gp", [
+    (12, 2, 0, 33, (1, 1)), (3, 3, 0, 17, (1, 1)), (8, 1, 9, 64, (1, 1)), (12, 2, 0, 901, (2, 1)),
+    (12, 2, 0, 1376, (2, 2)), (15, 5, 0, 800, (2, 0)), (15, 3, 3, 864, (2, 0))])
+def test_rotation_within_qkv(bh, heads, kv_heads, before, n, gp, precision):
+    shape = Shape(layers=2, hidden=256, heads=heads, kv_heads=kv_heads, head_dim=128, inter=64, vocab=320,
+                  max_len=before + n + 8)
+    toks = synthetic.first_tokens(shape, n, seed=n).astype(np.int32)
+    rows = []
+    for by_token in (False, True):
+        sess, _ = synthetic.build_session(shape, context=before, ln_jitter=0.1)
+        bh.buddy_hip_variant_reset()
+        if by_token:
+            for i, t in enumerate(toks):
+                sess.decode(int(t), before + i, want_logits=False)
+        else:
+            sess.prefill(toks, before, precision=precision)
+            D = 3 if precision == "digits" else 2  # (0: tiles that leave it to a launch behind them)
+            assert [tiles_run(bh)[f"gemm_w8_i8 rotates<{D}, {g}>"] for g in (1, 2)] == \
+                [shape.layers * (gp[precision == "digits2"] == g) for g in (1, 2)]
+        rows.append([sess.get_kv(j)[:, :before + n] for j in range(4)])
+        sess.close()
+    for got, want in zip(*rows):
+        np.testing.assert_array_equal(got[:, :before], want[:, :before])
+        got, want = got[:, before:], want[:, before:]
+        if precision == "digits":
+            check_close(got, want)
+        else:  # roundings of 2^-15 of a row's largest value, as in the test above
+            assert np.linalg.norm(got - want) < 2.0**-10 * np.linalg.norm(want)
+
+
 # bfloat16 modes: gate and up as one product whose result leaves as terms, on tiles of one and of
 # two channel tiles per wavefront, a result that ends inside 64 channels; the norm behind o and down
 # in the kernel that adds slices of K and as a launch of its own; the attention's fold as terms
