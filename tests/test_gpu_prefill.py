@@ -179,6 +179,25 @@ def test_digit_planes_are_the_rounded_fixed_point(M, K):
     assert (np.abs(got - xh) <= 0.5 * step + 2e-7 * np.abs(xh)).all()
 
 
+# rows that stay in registers, in each number of runs of four a thread, ending within one and at its end,
+# against rows one float into a buffer, which go through LDS: the same digits, so the same bits of the product
+@pytest.mark.parametrize("M,K", [(1, 4), (17, 1020), (33, 2048), (31, 2052), (40, 4100), (65, 6148), (18, 10240),
+                                 (16, 10244), (34, 14336)])
+@pytest.mark.parametrize("digits", [2, 3])
+def test_rows_become_digits_in_registers_as_in_lds(M, K, digits):
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    x = torch.randn((M, K), generator=g, device="cuda")
+    x[M // 2] *= 2.0 ** 90
+    x[M - 1, K - 1] = float("inf") if M > 1 else 2.0 ** -130
+    shifted = torch.empty(M * K + 1, device="cuda")[1:].reshape(M, K)
+    shifted.copy_(x)
+    q, s = synthetic.quantized_linear(K, 48, M)
+    packed = ops.pack_w8(q)
+    a, b = (ops.gemm_w8a32(t, packed, s, K, 48, digits=digits) for t in (x, shifted))
+    torch.cuda.synchronize()
+    assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+
+
 # gate and up in one launch with SiLU(gate) * up in its epilogue: the model's
 # shape, one shape for each of the four workgroup tiles, single-tile and ragged rows
 SILU_PAIR_SHAPES = [(512, 1536, 8960), (144, 256, 8192), (300, 256, 5120), (200, 192, 8192),
