@@ -1852,7 +1852,7 @@ int launch_plan(const TilePlan &plan, GemmI8Args &a, hipStream_t stream) {
   if (plan.tail)
     a.row_tiles = plan.tail;
   const int64_t units = (int64_t)a.ncols * a.slices;
-  a.panel = panel_for(units, a.row_tiles);
+  a.panel = panel_for(units, a.row_tiles, D > 1);
   const int64_t tiles = (a.panel ? units : round_up(units, 8)) * a.row_tiles;
   BH_REQUIRE(tiles < (1u << 31), "gemm_w8: %lld tiles", (long long)tiles);
   const unsigned blocks = (unsigned)tiles;

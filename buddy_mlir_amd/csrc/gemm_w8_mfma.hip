@@ -781,7 +781,7 @@ int launch_plan(const TilePlan &plan, GemmArgs &a, const GemmW8Args &in, hipStre
     a.partial = reinterpret_cast<float *>(ws);
   }
   const int64_t units = (int64_t)a.ncols * a.slices;
-  a.panel = panel_for(units, a.row_tiles);
+  a.panel = panel_for(units, a.row_tiles, false);
   const int64_t tiles = (a.panel ? units : round_up(units, 8)) * a.row_tiles;
   BH_REQUIRE(tiles < (1u << 31), "gemm_w8: %lld tiles", (long long)tiles);
   const unsigned blocks = (unsigned)tiles;
