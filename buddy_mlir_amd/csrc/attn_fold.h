@@ -46,7 +46,10 @@ struct PromptTerms;
 size_t attn_prompt_workspace_bytes(int q_len, int k_len, int heads, int kv_heads);
 int launch_attn_prompt(const AttnPrefillArgs &a, const PromptTerms &terms, void *workspace, PromptFold &fold,
                        hipStream_t stream);
-// the finished rows as the bf16 terms of the matmul behind the attention (gemm_w8_mfma.hip) ...
+// the finished rows in `out`, [tokens, heads * 128], which may be fold.out ...
+int launch_attn_fold_rows(const PromptFold &fold, int64_t o_stride, int heads, int tokens, float *out,
+                          hipStream_t stream);
+// ... as the bf16 terms of the matmul behind the attention (gemm_w8_mfma.hip) ...
 int launch_attn_fold_to_terms(const PromptFold &fold, int64_t o_stride, int heads, int tokens, int terms,
                               unsigned short *staged, hipStream_t stream);
 // ... or as its digit planes (gemm_w8_i8.hip)

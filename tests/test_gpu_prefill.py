@@ -1043,6 +1043,23 @@ def test_prompts_of_few_tokens(bh, hidden, heads, kv_heads, inter, before, n, pr
             assert np.linalg.norm(g - w) < bound * np.linalg.norm(w)
 
 
+# ... behind contexts whose attention leaves parts, fewer and more than are asked for at once: folded to f32 rows
+@pytest.mark.parametrize("precision", ["digits", "digits2", "bf16"])
+@pytest.mark.parametrize("heads,kv_heads,before,n", [(12, 2, 400, 8), (16, 2, 1500, 16), (12, 2, 3000, 2), (8, 4, 900, 5)])
+def test_few_tokens_behind_long_contexts(heads, kv_heads, before, n, precision):
+    shape = Shape(layers=2, hidden=384, heads=heads, kv_heads=kv_heads, head_dim=128, inter=336, vocab=320,
+                  max_len=before + n + 8)
+    toks = synthetic.first_tokens(shape, n, seed=n).astype(np.int32)
+    sess, _ = synthetic.build_session(shape, context=before, ln_jitter=0.1)
+    _, got = sess.prefill(toks, before, precision=precision)
+    sess.close()
+    sess, _ = synthetic.build_session(shape, context=before, ln_jitter=0.1)
+    for i, t in enumerate(toks):
+        _, want = sess.decode(int(t), before + i, want_logits=i + 1 == n)
+    sess.close()
+    check_close(got, want)
+
+
 # Where that ends: rows cast to bfloat16 in layers of 80, 128 and 250 million weights, and rows that are not
 # read 16 bytes at a time
 @pytest.mark.parametrize("precision,hidden,heads,kv_heads,inter,n,few", [
