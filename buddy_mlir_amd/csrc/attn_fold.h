@@ -60,9 +60,10 @@ int launch_attn_fold_to_digits(const PromptFold &fold, int64_t o_stride, int hea
 // The row of query head h at token t once more, in f32 sums, key after key: 32 lanes that
 // hold four values each from d on.  A row comes to this when its sum of weights is NaN:
 // because it is to be, or because the float16 terms of an operand do not exist (an
-// infinity) or leave none to the row's other values (one far above them), or a score's leave the range that the
-// score itself is in.  An infinite score of -inf has no weight, and an infinite value makes
-// its own channel infinite, as in the other attention kernels.  (1900 keys: some 0.4 ms.)
+// infinity) or leave none to the row's other values (one far above them), a row of values is far from
+// ordinary magnitudes (attn_terms.h), or a score's terms leave the range that the score itself is in.  An infinite
+// score of -inf has no weight, and an infinite value makes its own channel infinite, as in the other attention
+// kernels.  (1900 keys: some 0.4 ms.)
 __device__ __forceinline__ void f32_row(const PromptFold &f, int t, int h, int d, float (&v)[4]) {
 #pragma clang fp contract(off) // a score is rounded before the maximum is taken from it
   const int64_t head = (int64_t)(h / f.group) * f.kv_stride * kPromptD;
@@ -100,6 +101,9 @@ __device__ __forceinline__ void f32_row(const PromptFold &f, int t, int h, int d
   for (int e = 0; e < 4; ++e)
     v[e] *= inv;
 }
+
+// 1 / a row's sum of weights; NaN, so that the row is computed again, of one that is infinite
+__device__ __forceinline__ float inverse_of(float sum) { return fmaf(sum, 0.f, 1.0f / sum); }
 
 // Four values d .. d + 3 of query head h at token t, from where the launch left them; at most kMost parts
 // asked for at once.  Sixteen take registers that leave a compute unit one workgroup of 512 threads: for as
@@ -157,7 +161,7 @@ __device__ __forceinline__ void left4(const PromptFold &f, int64_t out_stride, i
   else
     for (int j = 0; j < b.parts; j += kMost)
       add(j, std::integral_constant<int, kMost>{});
-  const float inv = 1.0f / l;
+  const float inv = inverse_of(l);
 #pragma unroll
   for (int e = 0; e < 4; ++e)
     v[e] = s[e] * inv;

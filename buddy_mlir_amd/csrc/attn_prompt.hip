@@ -432,7 +432,7 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
       *reinterpret_cast<float2 *>(a.ml + (slot + col) * 2) = make_float2(rs.m, sum);
     // turned so that a store writes 128 bytes of each of eight rows (as they lie, 32 of each of 32: twice
     // as long)
-    const float f = whole ? 1.0f / sum : 1.0f;
+    const float f = whole ? inverse_of(sum) : 1.0f;
     const Base base = base_of(p.b);
     float *dst[4];
 #pragma unroll

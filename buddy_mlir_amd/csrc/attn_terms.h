@@ -1,9 +1,14 @@
 // attn_terms.h -- keys, values, queries and weights of a prompt's attention as float16 terms.
 //
 // A row of 128 values is brought to a largest magnitude of 2^14 .. 2^15 by a power of two of its own; an f32
-// value is then the sum of two float16 ones, rounded to nearest, 2^-24 off at most (a row's small values 2^-40
-// of its largest one).  Of the four products of two such sums the three of more than 2^-24 are taken,
-// each exact, all summed in f32.
+// value is then the sum of two float16 ones, rounded to nearest, 2^-23 of it off at most (a row's small values 2^-40
+// of its largest one).  Of the four products of two such sums the one of two second terms, 2^-22 at most, is left
+// out; the others are exact, all summed in f32.
+//
+// The rows of values whose keys share a sum must not be scaled too differently: a weight is held times its row's
+// scale, and the sum of the weights as those are (tile_weights).  Scales end at 2^50 and 2^-25, rows that
+// ask for more are computed again in f32 (value_scale).  A weight held is then at most 2^15, in the sum 2^65, and
+// 2^-43 of a row's largest weight is 2^-126 at least, as a weight held and as the factor between two parts of a row.
 //
 // 32 keys are a tile:  S^T[key, row] = K . Q^T and O^T[d, row] += V^T . P^T on v_mfma_f32_32x32x16_f16, a lane
 // with row lane % 32.  The registers of S^T are the operand P^T as they lie: a lane has keys
@@ -109,7 +114,9 @@ __device__ __forceinline__ unsigned key_scale(const float (&x)[8], float &undo) 
 // The same of a value's row.  A value that has no terms, or leaves none to the others, must not reach rows that
 // do not see its key, whose weight there is zero, nor other channels: it becomes zero, and the
 // row's log2, NaN, makes NaN of the rows that do see the key, which are computed again.  cleared(i): value i of this
-// lane became zero.
+// lane became zero.  So are rows that see one all below 2^-36 and not zero, or of 2^40 and more; a row of zeros, for
+// whose key there is a weight like any other's, has the scale of one of 2^-36.
+constexpr unsigned kLeastValue = 127 - 36, kMostValue = 127 + 39; // exponents of a row's largest magnitude
 template <class F>
 __device__ __forceinline__ unsigned value_scale(float (&x)[8], float &log2_of, F &&cleared) {
   bool bad = false;
@@ -129,7 +136,8 @@ __device__ __forceinline__ unsigned value_scale(float (&x)[8], float &log2_of, F
         cleared(i);
       }
   }
-  const unsigned e = scale_exponent(most);
+  const unsigned of = most >> 23, e = scale_exponent(max(of, kLeastValue) << 23);
+  bad |= (most != 0 && of < kLeastValue) || of > kMostValue;
   log2_of = bad ? __uint_as_float(0x7fc00000u) : 127.0f - (float)e;
   return e;
 }

@@ -178,7 +178,7 @@ attn_terms_kernel(const unsigned char *tiles, const float *q, int64_t q_stride, 
     }
     if (row > last) // of half a wavefront together
       continue;
-    const float inv = 1.0f / l;
+    const float inv = inverse_of(l);
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       v[e] *= inv;

@@ -826,6 +826,70 @@ def test_prompt_attention_over_magnitudes(which, powers):
         check_close(got, want)
 
 
+# Values that are zero, or so small beside others that their scales are far apart: their keys have weight all the
+# same.  The first tile of 32 keys a wavefront or a workgroup takes, tiles further on, all there are.
+@pytest.mark.parametrize("precision", ["digits", "exact"])
+@pytest.mark.parametrize("rows,power", [((0, 32), None), ((0, 64), None), ((96, 128), None), ((0, 600), None),
+                                        ((0, 32), -120), ((0, 600), -105), ((0, 600), -40), ((31, 600), None),
+                                        ((1, 600, 3), None), ((0, 600, 2), -60)])
+@pytest.mark.parametrize("beside", [0, 9, 30])
+def test_prompt_attention_of_values_without_magnitude(bh, rows, power, beside, precision):
+    """Behind a context, in one of two KV heads (in both a common factor of the sums of weights would be lost in the
+    norm that follows); the others' cached values times 2^beside: as the decode step has them."""
+    before, n = 600, 70
+    shape = Shape(layers=2, hidden=256, heads=6, kv_heads=2, head_dim=128, inter=256, vocab=320,
+                  max_len=before + n + 8)
+    toks = synthetic.first_tokens(shape, n, seed=6).astype(np.int32)
+    got = []
+    for by_token in (False, True):
+        sess, _ = synthetic.build_session(shape, context=before, ln_jitter=0.1)
+        t = sess.get_kv(1)
+        few = t[0, slice(*rows)] * np.float32(0.0 if power is None else 2.0**power)
+        t[:, :before] *= np.float32(2.0**beside)
+        t[0, slice(*rows)] = few
+        sess.set_kv(1, t)
+        if by_token:
+            for i, tok in enumerate(toks):
+                sess.decode(int(tok), before + i, want_logits=False)
+        else:
+            bh.buddy_hip_variant_reset()
+            sess.prefill(toks, before, precision=precision)
+            assert tiles_run(bh)["attn_prompt_kernel<256>"] == shape.layers
+        got.append([sess.get_kv(j)[:, before:before + n] for j in (2, 3)])
+        sess.close()
+    for a, b in zip(*got):
+        check_close(a, b)
+
+
+# ... of a prompt alone, whose tokens' embedding is zero, or so small that their values are, on all three kernels
+@pytest.mark.parametrize("heads,kv_heads,n,precision,kernel", [
+    (12, 2, 300, "digits", "attn_terms_kernel<32>"), (64, 8, 320, "digits", "attn_prompt_kernel<256>"),
+    (12, 2, 300, "exact", None)])
+@pytest.mark.parametrize("at", [(0, 32), (32, 33), (64, 65), (96, 160), (0, 257)])
+@pytest.mark.parametrize("size", [0.0, 2.0**-110])
+def test_prompt_alone_of_values_without_magnitude(bh, heads, kv_heads, n, precision, kernel, at, size):
+    shape = Shape(layers=2, hidden=256, heads=heads, kv_heads=kv_heads, head_dim=128, inter=256, vocab=320,
+                  max_len=n + 8)
+    toks = (synthetic.first_tokens(shape, n, seed=n) % 300).astype(np.int32)
+    toks[at[0]:at[1]] = 310
+    sess, g = DecoderSession(shape), synthetic.make_globals(shape)
+    g["embed"][310] *= size
+    sess.set_globals(g["embed"], g["inv_freq"], g["ln_f"], g["w_lm"], g["s_lm"])
+    for i in range(shape.layers):
+        sess.set_layer(i, synthetic.make_layer(shape, i, 0.1))
+    torch.cuda.synchronize()
+    bh.buddy_hip_variant_reset()
+    sess.prefill(toks, 0, precision=precision)
+    if kernel:
+        assert tiles_run(bh)[kernel] == shape.layers
+    got = [sess.get_kv(j)[:, :n] for j in range(4)]
+    for i, t in enumerate(toks):
+        sess.decode(int(t), i, want_logits=False)
+    for j in range(4):
+        check_close(got[j], sess.get_kv(j)[:, :n])
+    sess.close()
+
+
 @pytest.mark.parametrize("at", [0, 3, 4, 15, 16, 31, 63, 70])
 @pytest.mark.parametrize("size", [3.4e38, 8e38])  # above the largest bfloat16 value; infinite
 def test_prompt_attention_of_a_value_beyond_bfloat16(at, size):
