@@ -499,9 +499,12 @@ struct Qwen2Session : Session {
     if (folded && !pf_attn_ws) // for as many rows as the other buffers have, behind any context
       BH_CHECK_HIP(hipMalloc(&pf_attn_ws, attn_prompt_workspace_bytes(pf_rows, S.max_len, S.heads, S.kv_heads)));
     // a prompt alone: its attention reads terms that the rotation leaves (few tokens are done sooner from rows as
-    // they lie: 6 to 16 alone 1151 to 1256 us, 1160 to 1259 on terms)
+    // they lie: 6 to 16 alone 1151 to 1256 us, 1160 to 1259 on terms).  Where every f32 bit was asked for, only
+    // that of long ones: of few keys the terms' 23 bits show (27 tokens 1.5e-7 from 64 bits, f32 products 1.1e-7; 1931
+    // tokens 2.5e-7 and 2.3e-7).
     PromptTerms terms;
-    if (start_pos == 0 && !few && (folded || n <= kTermsMostKeys)) {
+    const bool every_bit = !gemm_digits && gemm_terms == 3;
+    if (start_pos == 0 && !few && (folded || (!every_bit && n <= kTermsMostKeys))) {
       terms.tiles = pf_terms;
       terms.per_head = (int)ceil_div(pf_rows, kTileKeys);
     }

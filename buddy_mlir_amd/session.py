@@ -236,7 +236,8 @@ class DecoderSession(_Session):
                 precision: str = "digits"):
         """precision: how the matmuls carry their f32 activations -- "digits" (three
         int8 digit planes on the int8 matrix cores), "digits2" (two planes), "exact"
-        (three bf16 terms) or "bf16" (cast)."""
+        (three bf16 terms; attention of all but long prompts and contexts in f32 products, too)
+        or "bf16" (cast)."""
         check(self._lib.buddy_hip_session_set_prefill_precision(
             self._h, self.PREFILL_PRECISION[precision]), "set_prefill_precision")
         return super().prefill(tokens, start_pos, want_logits)

@@ -762,7 +762,7 @@ def test_prompt_attention_of_a_key_beyond_bfloat16_in_long_rows(heads, kv_heads)
 # a prompt alone on the terms that the rotation leaves: part of a block of 32 rows, a tile of 32 keys and one more, a
 # tile to each wavefront and one more, groups that divide a block and that do not; the rotation in the
 # kernel that adds slices and as a launch of its own, q | k | v in f32
-@pytest.mark.parametrize("heads,kv_heads,n", [(6, 1, 1), (12, 2, 2), (12, 2, 27), (4, 4, 32), (6, 2, 33), (5, 1, 100),
+@pytest.mark.parametrize("heads,kv_heads,n", [(6, 1, 17), (12, 2, 18), (12, 2, 27), (4, 4, 32), (6, 2, 33), (5, 1, 100),
                                               (8, 1, 257), (12, 2, 300), (3, 3, 545)])
 @pytest.mark.parametrize("qkv_f32", [False, True])
 def test_prompt_attention_on_terms_of_the_rotation(bh, heads, kv_heads, n, qkv_f32):
@@ -782,12 +782,32 @@ def test_prompt_attention_on_terms_of_the_rotation(bh, heads, kv_heads, n, qkv_f
     torch.cuda.synchronize()
     sess.prefill(np.concatenate([toks[:1], [310], np.tile(toks, 40)[:n + 20]]).astype(np.int32), 0)
     bh.buddy_hip_variant_reset()
-    _, got = sess.prefill(toks, 0, precision="exact")
+    _, got = sess.prefill(toks, 0)
     assert tiles_run(bh)["attn_terms_kernel<32>"] == shape.layers
     rows = [sess.get_kv(j)[:, :n] for j in (2, 3)]
     for i, t in enumerate(toks):
         _, want = sess.decode(int(t), i, want_logits=i + 1 == n)
     check_close(got, want)
+    for j in (2, 3):
+        check_close(rows[j - 2], sess.get_kv(j)[:, :n])
+    sess.close()
+
+
+@pytest.mark.parametrize("heads,n,kernel", [(12, 1, None), (12, 27, None), (12, 300, None), (64, 320, "attn_prompt_kernel<256>")])
+def test_every_bit_of_a_prompt_alone(bh, heads, n, kernel):
+    """Where every f32 bit is asked for, a prompt's attention is on f32 instructions, that of long ones on terms."""
+    shape = Shape(layers=2, hidden=256, heads=heads, kv_heads=heads // 4, head_dim=128, inter=256, vocab=320,
+                  max_len=n + 8)
+    toks = synthetic.first_tokens(shape, n, seed=n).astype(np.int32)
+    sess, _ = synthetic.build_session(shape, context=0, ln_jitter=0.1)
+    bh.buddy_hip_variant_reset()
+    sess.prefill(toks, 0, precision="exact")
+    ran = tiles_run(bh)
+    for name in ("attn_terms_kernel<32>", "attn_prompt_kernel<256>"):
+        assert ran[name] == (shape.layers if name == kernel else 0)
+    rows = [sess.get_kv(j)[:, :n] for j in (2, 3)]
+    for i, t in enumerate(toks):
+        sess.decode(int(t), i, want_logits=False)
     for j in (2, 3):
         check_close(rows[j - 2], sess.get_kv(j)[:, :n])
     sess.close()
