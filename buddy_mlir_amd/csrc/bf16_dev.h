@@ -48,15 +48,24 @@ __device__ __forceinline__ float gated_act(GatedAct act, float g, float u, float
   return act == kActGeluTanh ? gelu_tanh_f(g) * u : expert_act(g, u, limit);
 }
 
-// The same with the one-instruction exponential and reciprocal (an ulp each), for results that leave as bfloat16:
-// the library's forms are some 25 instructions more a value, which a product's workgroups all spend at its end.
+// The same for results that leave as bfloat16, with one-instruction exponential and reciprocal (an ulp each; what the
+// exponential's argument loses in its product is put back): the library's forms are some 20 instructions more a value,
+// which a product's workgroups all spend at its end.  Against 64 bits, clamped form, g of -60 to 60: the
+// library's 4.8e-6 off at most and 8.0e-7 on average, these 2.3e-7 and 4.2e-8 (without `lost` 6.5e-6 and 9.9e-7);
+// results below 2^-126 are zero here.  gate | up of 16 experts, 2048 x 4 rows: 1 us of 110 for `lost`.
 __device__ __forceinline__ float gated_act_bf16(GatedAct act, float g, float u, float limit) {
-  auto sigmoid = [](float z) { return fast_rcp(1.0f + fast_exp(-z)); };
+  auto sigmoid_times = [](auto by, float z) { // sigmoid(by() * z)
+    constexpr double kBy = by() * -1.44269504088896340736;
+    constexpr float kHigh = (float)kBy, kLow = (float)(kBy - (double)kHigh);
+    z = __builtin_amdgcn_fmed3f(z, -256.f, 256.f); // beyond them 0 and 1
+    const float t = z * kHigh, lost = fmaf(z, kLow, fmaf(z, kHigh, -t));
+    return fast_rcp(1.0f + __builtin_amdgcn_exp2f(t) * fmaf(lost, 0.693147180559945309f, 1.0f));
+  };
   if (act == kActGeluTanh)
-    return g * sigmoid(1.59576912160573071f * fmaf(0.044715f * g * g, g, g)) * u;
+    return g * sigmoid_times([] { return 1.59576912160573071; }, fmaf(0.044715f * g * g, g, g)) * u;
   g = fminf(g, limit);
   u = fminf(fmaxf(u, -limit), limit);
-  return g * sigmoid(1.702f * g) * (u + 1.0f);
+  return g * sigmoid_times([] { return 1.702; }, g) * (u + 1.0f);
 }
 
 // an element of an activation buffer

@@ -317,7 +317,7 @@ rows_gemm_kernel(const uint4 *__restrict__ W, int ktiles, int steps, int columns
 // registers, one such tile to a compute unit and its loads between its products: gate | up of 16
 // experts, 2048 x 4 rows of 1536 -> 2 x 1792, 148 us, with rows by DMA 120; 777 x 1536 -> 2 x 8960
 // 68 and 58.  With the activation and the stores in cheaper forms (gated_act_bf16, the turn below)
-// 109 and 53.
+// 110 and 54.
 // (Rows past the registers for the tiles of 32 and 64 rows too: 8960 -> 1536 at 777 rows 47 us
 // whole, 56 so; 1536 -> 1536 of 400 rows 8.1 and 8.5.)  Against 16 x 16 tiles (us, rows x K x channels):
 //   bfloat16  2048 x 4096 x 4096   82.0 -> 75.2    f32   523 -> 216
