@@ -236,8 +236,10 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
       *reinterpret_cast<float *>(raw + 2048 + (lane >> 4) * 512 + g8 * 32 + i * 4) = 0.f;
       again = true;
     });
-    if (__any(again))
+    if (__any(again)) {
+      lds_turn();
       columns_of(y);
+    }
     if (g8 == 0) {
       sc.value[key] = log2_of;
       sc.undo[key] = pow2(e);
@@ -342,12 +344,14 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
           *reinterpret_cast<uint2 *>(turn + p * 2048 + r * 64 + (((lane & 7) >> 1) ^ (r >> 1 & 3)) * 16 +
                                      (lane & 1) * 8) = t[p];
       }
+      lds_turn();
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int p = 0; p < 2; ++p)
           qf[2 * c + i][p] = *reinterpret_cast<const uint4 *>(turn + p * 2048 + col * 64 +
                                                               ((2 * i + up) ^ (col >> 1 & 3)) * 16);
+      lds_turn();
       __builtin_amdgcn_sched_barrier(0);
     }
     if ((lane & 7) == 0) {
@@ -355,6 +359,7 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
       for (int j = 0; j < 4; ++j)
         *reinterpret_cast<float *>(turn + (8 * j + (lane >> 3)) * 4) = of_row[j];
     }
+    lds_turn();
     rs.q_scale = *reinterpret_cast<const float *>(turn + col * 4);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -452,6 +457,7 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
       for (int j = 0; j < 4; ++j)
         *reinterpret_cast<float4 *>(turn + col * 128 + ((2 * j + up) ^ (col & 7)) * 16) =
             float4{rs.o[dt][4 * j] * f, rs.o[dt][4 * j + 1] * f, rs.o[dt][4 * j + 2] * f, rs.o[dt][4 * j + 3] * f};
+      lds_turn();
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float4 x = *reinterpret_cast<const float4 *>(turn + (8 * i + (lane >> 3)) * 128 +
@@ -459,6 +465,7 @@ attn_prompt_kernel(const float *p_k, const float *p_v, int64_t p_kv_stride, int 
         if (8 * i + (lane >> 3) < left)
           *reinterpret_cast<float4 *>(dst[i] + dt * 32) = x;
       }
+      lds_turn();
     }
     if (tid == 0 && from_start) {
       // whoever has the block's first tile says where its parts are

@@ -751,6 +751,7 @@ rows_gemm_wide_kernel(const uint4 *W, int ktiles, int steps, int columns, int ro
           else
             *reinterpret_cast<uint2 *>(to) = uint2{pack_bf(v[0], v[1]), pack_bf(v[2], v[3])};
         }
+      lds_turn();
       constexpr int kPieces = kSegment / 16; // of a row
 #pragma unroll
       for (int i = 0; i < kPieces / 2; ++i) {
@@ -765,6 +766,7 @@ rows_gemm_wide_kernel(const uint4 *W, int ktiles, int steps, int columns, int ro
         unsigned char *to = static_cast<unsigned char *>(a.C) + ((int64_t)orow * a.ldc + ch0 * 16 + ch) * kOutSize;
         *reinterpret_cast<uint4 *>(to) = x;
       }
+      lds_turn();
     } else if (lr < rows) {
 #pragma unroll
       for (int g = 0; g < kTilesOut; ++g)

@@ -127,6 +127,14 @@ __device__ __forceinline__ float fast_exp(float x) {
 __device__ __forceinline__ float fast_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ __forceinline__ float fast_rsqrt(float x) { return __builtin_amdgcn_rsqf(x); }
 
+// A wavefront's LDS accesses ahead of this before those behind it, where lanes exchange values through a part of
+// LDS of the wavefront's own: the hardware completes them in order, the compiler is told to keep it.
+__device__ __forceinline__ void lds_turn() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Cross-lane reductions on DPP (data-parallel primitives: a VALU operand read
 // from another lane of the same row of 16, a few cycles) instead of
 // ds_bpermute round trips through the LDS crossbar.

@@ -583,6 +583,8 @@ __device__ __forceinline__ void finish_tile(const GemmI8Args &a, const v16i32 (&
     float *part = a.partial + at * kRows * kSpan;
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
+      if (rb > 0)
+        lds_turn();
 #pragma unroll
       for (int g = 0; g < GP; ++g)
 #pragma unroll
@@ -596,6 +598,7 @@ __device__ __forceinline__ void finish_tile(const GemmI8Args &a, const v16i32 (&
           }
           turn_in(g, q, o);
         }
+      lds_turn();
 #pragma unroll
       for (int i = 0; i < kQuads / 2; ++i) {
         const int idx = lane + 64 * i, row = idx / kQuads, c4 = idx % kQuads;
@@ -610,6 +613,8 @@ __device__ __forceinline__ void finish_tile(const GemmI8Args &a, const v16i32 (&
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
     const float row_step = step_s[rb * 32 + col];
+    if (rb > 0)
+      lds_turn();
 #pragma unroll
     for (int g = 0; g < GP; ++g)
 #pragma unroll
@@ -640,6 +645,7 @@ __device__ __forceinline__ void finish_tile(const GemmI8Args &a, const v16i32 (&
       rotate_tile<GP>(a, lds, ctile, m0);
       return;
     }
+    lds_turn();
 #pragma unroll
     for (int i = 0; i < kQuads / 2; ++i) {
       const int idx = lane + 64 * i, row = idx / kQuads, c4 = idx % kQuads;
@@ -665,11 +671,13 @@ __device__ __forceinline__ void finish_tile(const GemmI8Args &a, const v16i32 (&
     }
     if constexpr (D == 1) {
       if (a.sums) { // the same turn for the integer sums, carried as float bit patterns
+        lds_turn();
 #pragma unroll
         for (int g = 0; g < GP; ++g)
 #pragma unroll
           for (int q = 0; q < 4; ++q)
             turn_in(g, q, int_bits(acc[g][rb][0], q));
+        lds_turn();
         const bool ivec = (a.N & 3) == 0 && (reinterpret_cast<uintptr_t>(a.sums) & 15) == 0;
 #pragma unroll
         for (int i = 0; i < kQuads / 2; ++i) {
