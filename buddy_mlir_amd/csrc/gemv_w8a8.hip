@@ -26,6 +26,7 @@
 // that quantises.
 #include "common.h"
 #include <algorithm>
+#include <type_traits>
 #include "gemm.h"
 
 namespace bh {
@@ -408,6 +409,7 @@ w8a8_add_slices_kernel(const int32_t *partial, const float *part, int parts, int
     }
 }
 
+BH_TILE_FAMILY(RowsFamily, "w8a8_rows_kernel"); // channel tiles side by side; whether the rows are all there are
 struct RowsPlan {
   int ct = 0; // 0: another way
   int slices, per_slice, ncols, row_tiles;
@@ -473,10 +475,20 @@ int launch_rows(const float *A, const int4 *W, const RowsOut &to, int64_t M, int
     hipLaunchKernelGGL(kernel, grid, dim3(kRowsThreads), 0, st, A, W, part, parts, (int)M, (int)K, (int)N,
                        (int)ceil_div(N, kTileN), (int)ceil_div(K, kTileK), p.per_slice, p.ncols, p.slices, out);
   };
+  auto launch_ct = [&](auto ct) {
+    constexpr int kCt = decltype(ct)::value;
+    if (own) {
+      BH_NOTE_VARIANT(RowsFamily, kCt, 1);
+      launch(w8a8_rows_kernel<kCt, true>);
+    } else {
+      BH_NOTE_VARIANT(RowsFamily, kCt, 0);
+      launch(w8a8_rows_kernel<kCt, false>);
+    }
+  };
   if (p.ct == 2)
-    own ? launch(w8a8_rows_kernel<2, true>) : launch(w8a8_rows_kernel<2, false>);
+    launch_ct(std::integral_constant<int, 2>{});
   else
-    own ? launch(w8a8_rows_kernel<4, true>) : launch(w8a8_rows_kernel<4, false>);
+    launch_ct(std::integral_constant<int, 4>{});
   if (p.slices > 1)
     hipLaunchKernelGGL(w8a8_add_slices_kernel, dim3((unsigned)ceil_div(M * ceil_div(N, 4), 256)), dim3(256), 0, st,
                        out.partial, part, parts, (int)M, (int)N, columns, p.slices, out);

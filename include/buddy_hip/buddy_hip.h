@@ -679,7 +679,9 @@ int buddy_hip_gemv_f32_panels(const float *x, const float *packed, float *y,
  * A/s_a)), acc = A_q . W in int32 (exact), C = f32(acc) * (s_a * wscale[n]).
  * `packed` is the wave-tile copy of W; acc_out (int32 [M,N], dense) may be
  * NULL.  It runs on the int8 matrix cores (the i8 x i8 -> i32 branch of the BLIS kernel,
- * midend/lib/Conversion/MatMulOptimization/MatMulBlisVectorization.cpp:668-724);
+ * midend/lib/Conversion/MatMulOptimization/MatMulBlisVectorization.cpp:668-724); up to 16 rows as a GEMV on
+ * v_dot4_i32_i8 where they hold few values (2048, of more than 1536 k 5120), K is no multiple of 4 or above
+ * 131072, A is not 16-byte aligned or N is so large that the tiles outnumber the compute units;
  * more than 16 rows need K <= 131072.  A and C are dense ([M,K], [M,N]).
  * workspace: buddy_hip_w8a8_workspace_bytes, 16-byte aligned. */
 size_t buddy_hip_w8a8_workspace_bytes(int64_t M, int64_t K);

@@ -10,6 +10,7 @@ import torch
 import buddy_mlir_amd as bma
 from buddy_mlir_amd import ops, synthetic
 from parity import check_close
+from tile_report import tiles_run
 
 pytestmark = pytest.mark.gpu
 
@@ -154,14 +155,13 @@ def test_w8a8_many_rows_extremes(bh, oracle):
     assert abs(int(wacc[0, 0])) == K * 127 * 128
 
 
-# rows quantised by the workgroups that multiply them against the way of rows that cannot be read
-# 16 bytes at a time: (a tile's edges in rows, channels and k; K in slices; channels one by one)
-@pytest.mark.parametrize("M,K,N", [(2, 1536, 64), (5, 4, 7), (31, 68, 130), (32, 1536, 8960),
-                                   (33, 1536, 33), (64, 1540, 257), (256, 1000, 1111), (3, 3076, 70),
-                                   (16, 8960, 1536), (96, 8960, 1536), (17, 131072, 40),
-                                   (650, 1540, 1530)])
-@pytest.mark.parametrize("special", [False, True])
-def test_w8a8_rows_equal_the_general_path(bh, M, K, N, special):
+def w8a8_rows_launches(bh):
+    return {k: v for k, v in tiles_run(bh).items() if v and k.startswith("w8a8_rows_kernel")}
+
+
+def w8a8_rows(bh, M, K, N, special):
+    """The product of rows as they lie and of the same rows one float into a buffer, as bits, and the launches of
+    w8a8_rows_kernel for either."""
     q, s = synthetic.quantized_linear(K, N, M + K)
     packed = ops.pack_w8(q)
     x = torch.randn((M, K), generator=torch.Generator(device="cuda").manual_seed(N), device="cuda")
@@ -177,11 +177,38 @@ def test_w8a8_rows_equal_the_general_path(bh, M, K, N, special):
         C = torch.full((M, N), 7.0, device="cuda")
         acc = torch.full((M, N), 7, dtype=torch.int32, device="cuda")
         torch.cuda.synchronize()
+        bh.buddy_hip_variant_reset()
         sync_check(bh.buddy_hip_w8a8_matmul(A.data_ptr(), packed.data_ptr(), s.data_ptr(), C.data_ptr(),
                                             acc.data_ptr(), M, K, N, ws.data_ptr(), nb, None))
-        got.append((C.view(torch.int32), acc))
-    assert torch.equal(got[0][1], got[1][1])
-    assert torch.equal(got[0][0], got[1][0])
+        got.append((C.view(torch.int32), acc, w8a8_rows_launches(bh)))
+    return got
+
+
+# rows quantised by the workgroups that multiply them against the way of rows that cannot be read
+# 16 bytes at a time: (a tile's edges in rows, channels and k; K in slices; channels one by one; one chunk);
+# channel tiles side by side, whether a workgroup's rows are all there are
+@pytest.mark.parametrize("M,K,N,ct,own", [
+    (2, 1536, 64, 2, 1), (17, 4, 7, 2, 1), (31, 68, 130, 2, 1), (32, 1536, 8960, 2, 1), (5, 1536, 20000, 4, 1),
+    (33, 1536, 33, 2, 0), (64, 1540, 257, 2, 0), (256, 1000, 1111, 2, 0), (3, 3076, 70, 2, 0),
+    (16, 8960, 1536, 2, 0), (96, 8960, 1536, 4, 0), (17, 131072, 40, 2, 0), (650, 1536, 1530, 4, 0)])
+@pytest.mark.parametrize("special", [False, True])
+def test_w8a8_rows_equal_the_general_path(bh, M, K, N, ct, own, special):
+    a, b = w8a8_rows(bh, M, K, N, special)
+    assert a[2] == {f"w8a8_rows_kernel<{ct}, {own}>": 1} and not b[2]
+    assert torch.equal(a[1], b[1])
+    assert torch.equal(a[0], b[0])
+
+
+# ... and calls that go that way whatever the alignment: few values, more tiles than compute units, K of no
+# multiple of four or above 131072
+@pytest.mark.parametrize("M,K,N", [(5, 4, 7), (1, 1536, 64), (2, 2560, 40), (650, 1540, 1530), (20, 1538, 64),
+                                   (3, 131076, 20)])
+@pytest.mark.parametrize("special", [False, True])
+def test_w8a8_rows_of_the_general_path(bh, M, K, N, special):
+    a, b = w8a8_rows(bh, M, K, N, special)
+    assert not a[2] and not b[2]
+    assert torch.equal(a[1], b[1])
+    assert torch.equal(a[0], b[0])
 
 
 def test_buddy_matmul_f32_entry_point(bh):
