@@ -743,20 +743,21 @@ int launch_attn_decode(const AttnDecodeArgs &in, hipStream_t stream) {
     BH_REQUIRE(in.heads < 4096, "attn_decode: %d heads", in.heads);
     const int hp = pack_heads(a.heads, a.kv_heads, a.group);
     const size_t lds = sizeof(float) * (size_t)a.group * (in.chunk / kPW) * kD; // <= 64 KiB
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, dim3(in.chunk / kPW * 64), lds, stream, a.qkv, a.kcache, a.vcache, a.rope_table,
+                         a.pos_ptr, a.used, a.max_len, hp, a);
+    };
     if (in.chunk == 64) {
-      hipLaunchKernelGGL((sets == 1 ? attn_decode_partial_group<4, 1> : attn_decode_partial_group<4, 2>), grid, dim3(4 * 64), lds, stream, a.qkv,
-                         a.kcache, a.vcache, a.rope_table, a.pos_ptr, a.used, a.max_len, hp, a);
+      launch(sets == 1 ? attn_decode_partial_group<4, 1> : attn_decode_partial_group<4, 2>);
     } else if (in.chunk == 128) {
-      hipLaunchKernelGGL((sets == 1 ? attn_decode_partial_group<8, 1> : attn_decode_partial_group<8, 2>), grid, dim3(8 * 64), lds, stream, a.qkv,
-                         a.kcache, a.vcache, a.rope_table, a.pos_ptr, a.used, a.max_len, hp, a);
+      launch(sets == 1 ? attn_decode_partial_group<8, 1> : attn_decode_partial_group<8, 2>);
     } else {
-      // with 8 heads per KV head the 64 KiB of dynamic LDS come on top of 6 KiB
+      // with 8 heads per KV head the 64 KiB of dynamic LDS come on top of 7 KiB
       static DynLdsOnce dyn_lds;
       BH_CHECK_HIP(ensure_dyn_lds(dyn_lds,
                                   reinterpret_cast<const void *>(attn_decode_partial_group<16, 2>),
                                   (int)(sizeof(float) * kMaxGroup * 16 * kD)));
-      hipLaunchKernelGGL((sets == 1 ? attn_decode_partial_group<16, 1> : attn_decode_partial_group<16, 2>), grid, dim3(16 * 64), lds, stream, a.qkv,
-                         a.kcache, a.vcache, a.rope_table, a.pos_ptr, a.used, a.max_len, hp, a);
+      launch(sets == 1 ? attn_decode_partial_group<16, 1> : attn_decode_partial_group<16, 2>);
     }
     hipLaunchKernelGGL(attn_decode_combine_wide, dim3(in.heads, kWideParts), dim3(kWideThreads), 0, stream, a.part_acc,
                        a.part_ml, a.out, a.nchunks, a.used);
@@ -775,10 +776,7 @@ int launch_attn_decode(const AttnDecodeArgs &in, hipStream_t stream) {
   else
     hipLaunchKernelGGL(attn_decode_partial<16>, grid, dim3(16 * 64), 0, stream, a.qkv, a.kcache,
                        a.vcache, a.rope_table, a.pos_ptr, a.used, a.max_len, hp, 0, a);
-  if (in.combine && in.wide_combine)
-    hipLaunchKernelGGL(attn_decode_combine_wide, dim3(in.heads, kWideParts), dim3(kWideThreads), 0, stream, a.part_acc,
-                       a.part_ml, a.out, a.nchunks, a.used);
-  else if (in.combine)
+  if (in.combine)
     hipLaunchKernelGGL(attn_decode_combine, dim3(in.heads), dim3(kD), 0, stream, a);
   BH_CHECK_HIP(hipGetLastError());
   return BUDDY_HIP_OK;
