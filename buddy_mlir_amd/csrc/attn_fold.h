@@ -35,8 +35,9 @@ struct PromptFold {
 };
 
 // Whether launch_attn_prompt and the fold behind it are to be taken for a session's prompt, or
-// attn_prefill.hip and, if it `converts` its rows for the output product, the launch that does.
-bool attn_prompt_pays(int q_len, int q_offset, int heads, int kv_heads, bool converts);
+// attn_prefill.hip and, if it `converts` its rows for the output product, the launch that does; or, of a prompt
+// alone `on_terms`, attn_terms.hip.
+bool attn_prompt_pays(int q_len, int q_offset, int heads, int kv_heads, bool converts, bool on_terms);
 
 // Attention of a session's prompt tokens (no mask), on a workspace of
 // attn_prompt_workspace_bytes for at least as many tokens and positions; what it leaves is

@@ -11,8 +11,9 @@
 // head (tosa.py:4578-4579,4700); here the KV head is h / group, so the cache is
 // read in place.  The causal structure is exploited: key blocks that lie wholly
 // in a query block's future are skipped (they are exactly zero after softmax).
-// Arithmetic is f32 throughout, on the f32 matrix cores.  (A session takes it for prompts behind a context;
-// attn_terms.hip for a prompt alone, attn_prompt.hip for long ones.)
+// Arithmetic is f32 throughout, on the f32 matrix cores.  (A session takes it for prompts behind a context
+// that attn_prompt.hip does not pay for, and for prompts alone of few tokens or every f32 bit;
+// attn_terms.hip for other prompts alone, attn_prompt.hip for long ones.)
 #include "attn.h"
 #include "attn_terms.h"
 

@@ -596,12 +596,13 @@ PromptShare share_out(int q_len, int q_offset, int heads, int kv_heads) {
 }
 } // namespace
 
-// An estimate of both ways in microseconds, fitted to 1748 prompts of 12 layers: eight shapes of 1 to
-// 64 heads, 4 to 1000 tokens behind 0 to 1200, in three modes.  `converts`: behind the other way the
+// An estimate of both ways in microseconds, fitted to 1748 prompts of 12 layers (eight shapes of 1
+// to 64 heads, 4 to 1000 tokens behind 0 to 1200, in three modes) when this kernel took 5.1 us a tile, for 3 now, and
+// the fold one workgroup a token.  The line still lies where the two were equal then: prompts a little on the
+// other way's side of it may be faster this way by now.  `converts`: behind the other way the
 // rows take a launch of their own to become the output product's input, which the fold is here
-// (not up to 16 tokens as f32, nor up to 128 as digits, which that product makes itself).
-// The choice is up to 13 % of a layer slower than the better way and 0.25 % on average.  us a
-// layer with its products, the other way and this one, where the line lies:
+// (not up to 16 tokens as f32, nor up to 128 as digits, which that product makes itself).  us a
+// layer with its products, the other way and this one as it was, where the line lies:
 //   12 heads, 2 KV heads, digits: 4 behind 400 40.9, 42.3, behind 700 47.0, 43.9, 32 behind 256
 //     53.3, 54.9, behind 700 60.7, 58.0, 256 behind 400 70.1, 70.1, 500 alone 74.9, 75.6, behind
 //     128 79.5, 86.7, behind 400 93.0, 90.3, 730 alone 99.8, 102.0, 920 115.9, 113.7
@@ -611,12 +612,12 @@ PromptShare share_out(int q_len, int q_offset, int heads, int kv_heads) {
 // More than 32 tokens behind 400 and more go this way in doubt, up to 6 us, and more than 640 up to
 // 2.5: it asks for each key once for all heads of a KV head, and what is not finite stays with the
 // rows that see it.
-// A prompt alone has attn_terms.hip as the other way, whose workgroups read every key of their 32 rows for
+// `on_terms`: a prompt alone that has attn_terms.hip as the other way, whose workgroups read every key of their 32 rows for
 // themselves: us a layer, that way and this one, 12 heads, 2 KV heads, 400 tokens 126 and 133, 800 195 and 206, 1000
 // 226 and 235, 1500 320 and 323, 1931 405 and 401; 32 and 8, 400 tokens 156 and 165, 600 202 and 210, 800 256 and
 // 252, 1000 301 and 291, 1931 570 and 532.  One line for both: 890 tokens, of more than 22 heads fewer.
-bool attn_prompt_pays(int q_len, int q_offset, int heads, int kv_heads, bool converts) {
-  if (q_offset == 0)
+bool attn_prompt_pays(int q_len, int q_offset, int heads, int kv_heads, bool converts, bool on_terms) {
+  if (on_terms)
     return q_len > 890 || (int64_t)q_len * heads > 20000;
   const double kilo_rows = 1e-4 * q_len * heads; // tens of thousands of (token, head)
   // attn_prefill.hip: blocks of 16 queries, one to a workgroup of eight wavefronts, then two, while

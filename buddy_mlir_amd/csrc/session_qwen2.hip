@@ -495,16 +495,16 @@ struct Qwen2Session : Session {
     const bool few = few_tokens(n);
     // attention's rows go to their product as they are (few) or it makes their digits (gemm_digit_rows)
     const bool converts = !few && !(gemm_digits && gemm_w8_takes_rows(n, layers[0].o.K, S.hidden, layers[0].o.K));
-    const bool folded = attn_prompt_pays(n, start_pos, S.heads, S.kv_heads, converts);
-    if (folded && !pf_attn_ws) // for as many rows as the other buffers have, behind any context
-      BH_CHECK_HIP(hipMalloc(&pf_attn_ws, attn_prompt_workspace_bytes(pf_rows, S.max_len, S.heads, S.kv_heads)));
     // a prompt alone: its attention reads terms that the rotation leaves (few tokens are done sooner from rows as
     // they lie: 6 to 16 alone 1151 to 1256 us, 1160 to 1259 on terms).  Where every f32 bit was asked for, only
     // that of long ones: of few keys the terms' 23 bits show (27 tokens 1.5e-7 from 64 bits, f32 products 1.1e-7; 1931
     // tokens 2.5e-7 and 2.3e-7).
+    const bool every_bit = !gemm_digits && gemm_terms == 3, on_terms = start_pos == 0 && !few && !every_bit;
+    const bool folded = attn_prompt_pays(n, start_pos, S.heads, S.kv_heads, converts, on_terms);
+    if (folded && !pf_attn_ws) // for as many rows as the other buffers have, behind any context
+      BH_CHECK_HIP(hipMalloc(&pf_attn_ws, attn_prompt_workspace_bytes(pf_rows, S.max_len, S.heads, S.kv_heads)));
     PromptTerms terms;
-    const bool every_bit = !gemm_digits && gemm_terms == 3;
-    if (start_pos == 0 && !few && (folded || (!every_bit && n <= kTermsMostKeys))) {
+    if (folded ? start_pos == 0 && !few : on_terms && n <= kTermsMostKeys) {
       terms.tiles = pf_terms;
       terms.per_head = (int)ceil_div(pf_rows, kTileKeys);
     }

@@ -793,7 +793,7 @@ def test_prompt_attention_on_terms_of_the_rotation(bh, heads, kv_heads, n, qkv_f
     sess.close()
 
 
-@pytest.mark.parametrize("heads,n,kernel", [(12, 1, None), (12, 27, None), (12, 300, None), (64, 320, "attn_prompt_kernel<256>")])
+@pytest.mark.parametrize("heads,n,kernel", [(12, 1, None), (12, 27, None), (12, 300, None), (64, 600, "attn_prompt_kernel<256>")])
 def test_every_bit_of_a_prompt_alone(bh, heads, n, kernel):
     """Where every f32 bit is asked for, a prompt's attention is on f32 instructions, that of long ones on terms."""
     shape = Shape(layers=2, hidden=256, heads=heads, kv_heads=heads // 4, head_dim=128, inter=256, vocab=320,
