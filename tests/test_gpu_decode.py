@@ -408,15 +408,15 @@ def test_small_model_decodes_at_long_context(oracle):
     sess.close()
 
 
-@pytest.mark.parametrize("start", [100, 1140, 2296, 4596, 5110, 12535, 16375])
+@pytest.mark.parametrize("start", [100, 1140, 2296, 4596, 5110, 8182, 12535, 16375])
 def test_small_model_steps_across_the_attention_chunk_sizes(oracle, start):
     """A step far into a long cache takes attention chunks of 128 or 256 positions
     (from positions 1152 and 2304 on), covers only the chunks up to its position,
     and from position 5120 on folds the partials in a launch of its own instead of
     in the o_proj launch: greedy steps that cross each boundary, a short context
-    in a large cache, and the positions at which the launches that take the heads
-    of a KV head together change their cut (12544 and 16384 with two KV
-    heads), against the oracle -- every step's logits and the token fed back on
+    in a large cache, the positions at which the launches that take the heads
+    of a KV head together change their cut (8192 and 16384 with two KV
+    heads) and one between them, against the oracle -- every step's logits and the token fed back on
     the device."""
     shape = Shape(layers=2, hidden=256, heads=4, kv_heads=2, head_dim=128, inter=512,
                   vocab=1024, max_len=(start + 100 + 63) // 64 * 64 if start > 4400 else 4352,
@@ -445,9 +445,9 @@ def test_small_model_steps_across_the_attention_chunk_sizes(oracle, start):
 
 @pytest.mark.parametrize("heads,kv_heads", [(1, 1), (3, 1), (5, 1), (6, 1), (8, 1), (12, 2), (8, 4)])
 def test_long_context_steps_for_every_size_of_head_group(oracle, heads, kv_heads):
-    """From position 5120 on a workgroup takes all the query heads of a KV head, or,
-    where there are few KV heads, half of them (a group of 3 or 5 splits unevenly, a
-    group of one not at all): steps that cross that position against the oracle."""
+    """From position 5120 on a workgroup takes all the query heads of a KV head, four at a time (a group of 1 or 3
+    leaves columns of a set empty, one of 5 or 6 of its second): steps that cross that position against the
+    oracle."""
     start = 5114
     shape = Shape(layers=1, hidden=256, heads=heads, kv_heads=kv_heads, head_dim=128, inter=256,
                   vocab=512, max_len=5184, rms_eps=1e-6)
@@ -489,10 +489,10 @@ def test_cuts_of_long_contexts_with_two_sets_of_heads(oracle, heads, kv_heads, s
 
 @pytest.mark.parametrize("start", [17000, 66000])
 def test_fold_of_more_partials_than_one_pass_takes(oracle, start):
-    """The launch that folds the partials far into a long cache takes 128 of them
-    per head in its first pass and keeps the (max, sum) pairs of up to 256 in
+    """The launch that folds the partials far into a long cache takes 256 of them
+    per head in its first pass and keeps the (max, sum) pairs of as many in
     registers: with one KV head 17000 positions are 136 partials of 128
-    positions, 66000 are 260 of 256."""
+    positions, a part of that pass, 66000 are 260 of 256."""
     shape = Shape(layers=1, hidden=256, heads=2, kv_heads=1, head_dim=128, inter=256,
                   vocab=512, max_len=start + 64, rms_eps=1e-6)
     sess, host = synthetic.build_session(shape, context=start, keep_host=True, ln_jitter=0.1)
