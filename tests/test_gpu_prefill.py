@@ -851,7 +851,8 @@ def test_prompt_attention_over_magnitudes(which, powers):
 @pytest.mark.parametrize("precision", ["digits", "exact"])
 @pytest.mark.parametrize("rows,power", [((0, 32), None), ((0, 64), None), ((96, 128), None), ((0, 600), None),
                                         ((0, 32), -120), ((0, 600), -105), ((0, 600), -40), ((31, 600), None),
-                                        ((1, 600, 3), None), ((0, 600, 2), -60)])
+                                        ((1, 600, 3), None), ((0, 600, 2), -60), ((0, 600, 2), -38),
+                                        ((1, 600, 3), 38)])
 @pytest.mark.parametrize("beside", [0, 9, 30])
 def test_prompt_attention_of_values_without_magnitude(bh, rows, power, beside, precision):
     """Behind a context, in one of two KV heads (in both a common factor of the sums of weights would be lost in the
